@@ -51,13 +51,9 @@ template <int HD> __device__ __forceinline__ void kv_pack_thread(const AttnDev& 
 // each group of eight dims the halves are stored in the order 0 4 1 5 2 6 3 7, the order in which a 32-bit word of
 // eight 4-bit keys unpacks into f16 pairs.
 template <int HD>
-__global__ __launch_bounds__(HD) void k_attn_prep(AttnDev a, KvDev kv, const float* __restrict__ qkv, int stride, int start, const int* __restrict__ posp, float* __restrict__ qout, uint16_t* __restrict__ qh, float* __restrict__ qsc, size_t wz_qkv, size_t wz_q) {
+__global__ __launch_bounds__(HD) void k_attn_prep(AttnDev a, KvDev kv, const float* __restrict__ qkv, int stride, int start, const int* __restrict__ posp, float* __restrict__ qout, uint16_t* __restrict__ qh, float* __restrict__ qsc) {
   __shared__ float buf[HD]; __shared__ float red[HD / 64]; __shared__ float redm[HD / 64];
   if (posp) start = *posp;
-  if (gridDim.z > 1) {          // consecutive windows in one launch (a long prompt's blocks): window z's projection wz_qkv bytes, its query buffers wz_q bytes further on per window, its positions behind the window before
-    const size_t z = blockIdx.z; start += (int)z * (int)gridDim.y;
-    qkv = (const float*)((const char*)qkv + z * wz_qkv); qout = (float*)((char*)qout + z * wz_q); qh = (uint16_t*)((char*)qh + z * wz_q); qsc = (float*)((char*)qsc + z * wz_q);
-  }
   const int b = blockIdx.x, ti = blockIdx.y, tid = threadIdx.x, pos = start + ti;
   if (b >= a.nkv + a.nh) {
     int p0, p1;
@@ -94,7 +90,7 @@ __global__ __launch_bounds__(HD) void k_attn_prep(AttnDev a, KvDev kv, const flo
     kv.kf[kv_blk((size_t)h * HD + tid, (size_t)a.nkv * HD, pos)] = v;
     kv.vf[(size_t)pos * a.nkv * HD + (size_t)h * HD + tid] = vrow;
   } else {
-    qout[((size_t)ti * a.nh + h) * HD + tid] = v;
+    if (qout) qout[((size_t)ti * a.nh + h) * HD + tid] = v;
     float am = fabsf(v); am = am == am ? am : INFINITY;
     am = wave_max(am);
     if ((tid & 63) == 0) redm[tid >> 6] = am;
@@ -739,7 +735,7 @@ template <int G> static void launch_decode(pyre_ctx* ctx, const AttnDev& a, cons
 int pyre_attn_launch(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const AttnWork& w, const float* qkv, int stride, int start, int t, int* packed_done, float* out, const int* posp) {
   return pyre_attn_launch_sel(ctx, a, kv, w, qkv, stride, start, t, packed_done, out, posp, nullptr);
 }
-int pyre_attn_launch_sel(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const AttnWork& w, const float* qkv, int stride, int start, int t, int* packed_done, float* out, const int* posp, const QsaWork* qw, int part) {
+int pyre_attn_launch_sel(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const AttnWork& w, const float* qkv, int stride, int start, int t, int* packed_done, float* out, const int* posp, const QsaWork* qw) {
   if (a.hd != 256) return pyre_fail(ctx, PYRE_E_SHAPE, "attention: head dim %d unsupported (256 only)", a.hd);
   if (a.nkv < 1 || a.nh % a.nkv) return pyre_fail(ctx, PYRE_E_SHAPE, "attention: %d query heads over %d kv heads", a.nh, a.nkv);
   int G = a.nh / a.nkv; if (G != 1 && G != 2 && G != 4 && G != 8) return pyre_fail(ctx, PYRE_E_SHAPE, "attention: group size %d unsupported (1, 2, 4, 8)", G);
@@ -747,18 +743,11 @@ int pyre_attn_launch_sel(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const
   if (start < 0 || start + t > kv.cap) return pyre_fail(ctx, PYRE_E_STATE, "attention: position %d exceeds the cache capacity %d", start + t, kv.cap);
   if (a.n_rot > a.hd || (a.n_rot & 1)) return pyre_fail(ctx, PYRE_E_SHAPE, "attention: n_rot %d", a.n_rot);
   // a single-token step at a device-side position: the packing check rides on the prep launch as extra blocks
-  // part 1: the cache write (rotated q into w.q / qh / qsc, K and V into the cache, packing); part 2: the attention pass over
-  // the cache and the merge, which read only what part 1 of this and of earlier windows has written (w.q* must then be this
-  // window's own until part 2 has run); 0: both
-  if (part < 0 || part > 2 || (part && posp)) return pyre_fail(ctx, PYRE_E_ARG, "attention: part %d", part);
-  const int nwin = ctx->batch_n;          // part 1 for that many consecutive windows of t tokens in one launch (ctx->batch_stride / batch_stride2: the windows' projections / query buffers apart)
-  if (nwin > 1 && (part != 1 || qw || start + nwin * t > kv.cap)) return pyre_fail(ctx, PYRE_E_ARG, "attention: %d windows a launch (the cache write alone, dense, inside the cache)", nwin);
   const bool pack_rides = posp && t == 1 && a.kv_bits == 4;
   const int pack_blocks = pack_rides ? (64 * (a.nkv * a.hd / 32) * 2 + 255) / 256 : 0;
-  if (part != 2) {
-  { ProfScope ps(ctx, "attn_prep", 8.0 * t * (a.nh + 2.0 * a.nkv) * a.hd); hipLaunchKernelGGL((k_attn_prep<256>), dim3(a.nkv + a.nh + pack_blocks, t, nwin), dim3(256), 0, ctx->stream, a, kv, qkv, stride, start, posp, w.q, w.qh, w.qsc, ctx->batch_stride, ctx->batch_stride2); } PYRE_CHECK_LAUNCH(ctx);
+  { ProfScope ps(ctx, "attn_prep", 8.0 * t * (a.nh + 2.0 * a.nkv) * a.hd); hipLaunchKernelGGL((k_attn_prep<256>), dim3(a.nkv + a.nh + pack_blocks, t), dim3(256), 0, ctx->stream, a, kv, qkv, stride, start, posp, w.q, w.qh, w.qsc); } PYRE_CHECK_LAUNCH(ctx);
   // pack the positions that fall below the boundary of the longest view of this call
-  int pbn = (int)pyre_packed_boundary((size_t)start + (size_t)nwin * t, a.kv_bits, a.kv_recent);
+  int pbn = (int)pyre_packed_boundary((size_t)start + t, a.kv_bits, a.kv_recent);
   if (posp) {   // one 64-position packing step at most; the kernel decides from the device-side position
     if (a.kv_bits == 4 && !pack_rides) { size_t thr = (size_t)64 * (a.nkv * a.hd / 32) * 2; hipLaunchKernelGGL((k_kv_pack<256>), dim3((unsigned)((thr + 127) / 128)), dim3(128), 0, ctx->stream, a, kv, 0, 0, posp); PYRE_CHECK_LAUNCH(ctx); }
   } else if (pbn > *packed_done) {
@@ -766,8 +755,6 @@ int pyre_attn_launch_sel(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const
     { ProfScope ps(ctx, "kv_pack", (double)(pbn - *packed_done) * a.nkv * a.hd * 2 * 4.625); hipLaunchKernelGGL((k_kv_pack<256>), dim3((unsigned)((thr + 127) / 128)), dim3(128), 0, ctx->stream, a, kv, *packed_done, pbn, (const int*)nullptr); } PYRE_CHECK_LAUNCH(ctx);
     *packed_done = pbn;
   }
-  }
-  if (part == 1) return PYRE_OK;
   double kvb = 0;
   for (int ti = 0; ti < t; ++ti) {
     double n = start + ti + 1, pb = (double)pyre_packed_boundary((size_t)n, a.kv_bits, a.kv_recent);
@@ -782,11 +769,25 @@ int pyre_attn_launch_sel(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const
   return PYRE_OK;
 }
 
+// the cache write of a prompt's block: one launch for any number of tokens, one packing step
+int pyre_attn_blk_prep(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const float* qkv, int stride, int start, int T, int* packed_done, float* q, uint16_t* qh, float* qsc) {
+  if (a.hd != 256 || a.n_rot > a.hd || (a.n_rot & 1)) return pyre_fail(ctx, PYRE_E_SHAPE, "attention: head dim %d, n_rot %d", a.hd, a.n_rot);
+  if (T < 1 || start < 0 || start + T > kv.cap) return pyre_fail(ctx, PYRE_E_STATE, "attention: positions %d..%d outside the cache (%d)", start, start + T, kv.cap);
+  { ProfScope ps(ctx, "attn_prep", 8.0 * T * (a.nh + 2.0 * a.nkv) * a.hd); hipLaunchKernelGGL((k_attn_prep<256>), dim3(a.nkv + a.nh, T), dim3(256), 0, ctx->stream, a, kv, qkv, stride, start, (const int*)nullptr, q, qh, qsc); } PYRE_CHECK_LAUNCH(ctx);
+  const int pbn = (int)pyre_packed_boundary((size_t)start + T, a.kv_bits, a.kv_recent);
+  if (pbn > *packed_done) {
+    const size_t thr = (size_t)(pbn - *packed_done) * (a.nkv * a.hd / 32) * 2;
+    ProfScope ps(ctx, "kv_pack", (double)(pbn - *packed_done) * a.nkv * a.hd * 2 * 4.625); hipLaunchKernelGGL((k_kv_pack<256>), dim3((unsigned)((thr + 127) / 128)), dim3(128), 0, ctx->stream, a, kv, *packed_done, pbn, (const int*)nullptr);
+    *packed_done = pbn;
+  } PYRE_CHECK_LAUNCH(ctx);
+  return PYRE_OK;
+}
+
 // K / V of positions start..start+t-1 into an f32 cache, nothing attended (the drafter's catch-up over committed cells)
 int pyre_attn_append_launch(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const AttnWork& w, const float* qkv, int stride, int start, int t) {
   if (a.hd != 256 || a.kv_bits != 0) return pyre_fail(ctx, PYRE_E_SHAPE, "attention append: head dim %d, %d-bit cache (256, f32 only)", a.hd, a.kv_bits);
   if (t < 1 || t > 8 || start < 0 || start + t > kv.cap) return pyre_fail(ctx, PYRE_E_STATE, "attention append: positions %d..%d outside the cache (%d)", start, start + t, kv.cap);
-  { ProfScope ps(ctx, "attn_prep", 8.0 * t * (a.nh + 2.0 * a.nkv) * a.hd); hipLaunchKernelGGL((k_attn_prep<256>), dim3(a.nkv + a.nh, t), dim3(256), 0, ctx->stream, a, kv, qkv, stride, start, (const int*)nullptr, w.q, w.qh, w.qsc, (size_t)0, (size_t)0); } PYRE_CHECK_LAUNCH(ctx);
+  { ProfScope ps(ctx, "attn_prep", 8.0 * t * (a.nh + 2.0 * a.nkv) * a.hd); hipLaunchKernelGGL((k_attn_prep<256>), dim3(a.nkv + a.nh, t), dim3(256), 0, ctx->stream, a, kv, qkv, stride, start, (const int*)nullptr, w.q, w.qh, w.qsc); } PYRE_CHECK_LAUNCH(ctx);
   return PYRE_OK;
 }
 

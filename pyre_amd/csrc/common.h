@@ -42,7 +42,6 @@ struct pyre_ctx {
   bool prof_on = false; std::vector<ProfPending> prof_pending; std::map<std::string, ProfAcc> prof_acc; std::vector<hipEvent_t> prof_pool;
   std::string prof_text;
   void* aop_buf = nullptr; size_t aop_bytes = 0;       // split activations of the operator's matrix-core GEMM (grow-only)
-  int batch_n = 1; size_t batch_stride = 0, batch_stride2 = 0;            // the matrix-core hyper-connection launches (hc.hip) for batch_n windows at once: window z's own buffers batch_stride bytes further on per window (a long prompt's blocks; 1 / 0 otherwise)
   void* aop_static = nullptr;                          // device address of this GPU's copy of the file-scope operand array (gemm_m.hip), resolved at creation
   uint32_t* d_iq2xs_sgn = nullptr;                     // IQ2_XS likewise: two tables of 8192 x four signed bytes (weights 0..3 / 4..7 of an entry)
   uint32_t* d_iq3s_sgn = nullptr;                      // IQ3_S codebook with the signs folded in: 8192 x four signed bytes (gemv_n.hip), made at first use
@@ -308,14 +307,13 @@ struct RouteSrc { const float* p; int nsl; int r64; const uint32_t* dgx = nullpt
 // token in w.parts, group q of token ti at parts + (q*t + ti)*d, instead of the unreduced terms.
 int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const float* x_dev, int t, float* y_dev, const RouteSrc* routed = nullptr, bool in_groups = false);
 inline bool pyre_moe_groups_ok(const MoeDev& m) { return m.top_k <= PYRE_MOE_KMAX; }
-// The FFN of a block of prompt windows (T = 8 * windows tokens) with the tokens grouped by expert, on the matrix cores (moe.hip):
-// what the windows' mixes leave in their workspaces -- window w's x [8][d] at x + w * ws, its router K-slice sums at rpart + w * ws
-// (slice s of token ti at (s * 8 + ti) * r64) -- and where window w's group sums go: parts + w * ws, laid out as
-// MoeWork::parts of a window of eight.  The rest is the block's own scratch (pyre_moe_block_carve): the routing, the (token, choice) pairs by
+// The FFN of a prompt's block of T tokens, grouped by expert, on the matrix cores (moe.hip): x [T][d]; the router's K-slice sums of
+// group w (eight tokens; slice s of token ti at (s * 8 + ti) * r64) at rpart + w * wr; the group sums of every token in
+// parts [group][PYRE_MOE_GROUPS][8][d].  The rest is the block's own scratch (pyre_moe_block_carve): the routing, the (token, choice) pairs by
 // expert, x and h as f16 operand rows a token (xh [T + 1][2][d], hh [T * (k + 1) + 1][2][ff], the last row of each zero) with
 // their scale factors, the gate and up products and the unreduced down terms.
 struct MoeBlk {
-  const float* x; const float* rpart; float* parts; size_t ws;      // window w's x, router sums and group sums at these + w * ws floats (the windows' workspaces: one stride)
+  const float* x; const float* rpart; float* parts; size_t wr;
   int32_t* sel_idx; float* sel_w; float* sg; int32_t* eoff; int32_t* elist; float* g; float* u; float* partial;
   uint16_t* xh; float* xinv; uint16_t* hh; float* hinv;
 };
@@ -323,7 +321,7 @@ bool   pyre_moe_block_ok(const MoeDev& m);
 size_t pyre_moe_block_bytes(const MoeDev& m, int T);
 void   pyre_moe_block_carve(const MoeDev& m, int T, void* base, MoeBlk* b);
 int    pyre_moe_block_zero_rows(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T);
-int    pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_max, int nsl, int r64, bool router_here = false);      // router_here: the router's sums are formed by this call (k_moe_router_blk), not left by the mixes
+int    pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_max, int nsl, int r64);
 // K parts the gate/up dot products are summed in (1 or 2; k_moe_gu)
 int pyre_moe_gu_parts(const MoeDev& m);
 
@@ -374,6 +372,22 @@ bool pyre_hc_route_ok(const HcDev& h, const QMatDev& router);
 bool pyre_hc_plan(const HcDev& h, int* nw, int* upw, int* ksplit);
 int pyre_hc_combine_launch(pyre_ctx* ctx, int d, int hc, float* x_dev, int t, const float* out_dev, const float* inj_dev);
 
+// ---- a prompt taken layer by layer (prompt.hip): the mixes and projections of hundreds of tokens a launch ------------------------
+// Tokens in groups of eight, a group's activations as sixteen f16 operand rows (PyreAop with R = 16) at op + group * op_gs
+// (uint4), their factors [super-block][8] at inv + group * inv_gs.
+struct BlkMix { float* ssq; float* smx; float* part; uint16_t* lo; float* lo_dn; float* scl; float2* opb; };      // scratch of one mix over T tokens
+bool   pyre_blk_mix_ok(const HcDev& h);
+size_t pyre_blk_mix_bytes(const HcDev& h, int T);
+void   pyre_blk_mix_carve(const HcDev& h, int T, void* base, BlkMix* b);
+// pyre_hc_mix_launch over T tokens: x [token][hc][d] is updated in place (x_in may be the embedding rows: in_ss = 0), the pending
+// update in np vectors (0 none; 1: comb [token][d]; PYRE_MOE_GROUPS: comb [group][PYRE_MOE_GROUPS][8][d])
+int pyre_blk_mix_launch(pyre_ctx* ctx, const HcDev& h, const BlkMix& b, const float* x_in, int in_ss, int in_ts, float* x, int T, const float* comb, int np, const float* comb_inj, float eps,
+                        float* mixed, float* inj, uint4* op, size_t op_gs, float* inv, int inv_gs);
+int pyre_blk_gemm_launch(pyre_ctx* ctx, const QMatDev& m, const uint4* op, size_t op_gs, const float* inv, int inv_gs, float* y, int ys, int T);      // y[token * ys + row]
+int pyre_blk_op_split_launch(pyre_ctx* ctx, const float* x, int cols, int T, uint4* op, size_t op_gs, float* inv, int inv_gs);      // x [T][cols] -> operand rows, a power of two per 256 columns
+// a Gated DeltaNet layer's raw output o [T][heads * 128] -> RMS norm per head, * sigmoid(z), as operand rows scaled by `up` and / or as f32 rows `out`
+int pyre_blk_gdn_out_launch(pyre_ctx* ctx, const float* o, const float* z, int zs, const float* nw, float eps, int heads, int T, float up, uint4* op, size_t op_gs, float* out);
+
 // ---- Gated DeltaNet (gdn.hip) -----------------------------------------------------------------------------------------
 struct GdnDev { const float* a; const float* dt; const float* conv_w; const float* norm_w; int nk, nv, dk, dv, conv_k; float eps; };
 // proj [t][ch + nv*dv + 2*nv] = [qkv | z | beta | alpha] per token (row stride = proj_stride floats).
@@ -384,15 +398,16 @@ struct GdnDev { const float* a; const float* dt; const float* conv_w; const floa
 // The state it leaves differs in rounding from the nv-workgroup form's (the column sums meet in another order): a layer
 // uses one form for every call.
 struct GdnQ { uint16_t* op; float* sq; };
-// the convolution of n consecutive windows of t tokens in one launch (gdn.hip: k_gdn_conv_blk)
-int pyre_gdn_conv_block_launch(pyre_ctx* ctx, const GdnDev& g, const float* proj, int stride, int t, int n, size_t ws, const float* prev, int prev_stride, float* conv_out, float* co);
 int pyre_gdn_launch(pyre_ctx* ctx, const GdnDev& g, const float* proj, int proj_stride, int t, const float* conv_in, float* conv_out,
-                    const float* ssm_in, float* ssm_out, float* co_scratch, float* out_dev, bool conv_done = false, uint16_t* aop = nullptr, float aop_up = 1.0f, const GdnQ* gq = nullptr, int nwin = 1, size_t ws = 0);      // nwin > 1: that many consecutive windows, their projections, convolution outputs and operands ws floats apart, in one launch (the per-quarter form, conv_done)
+                    const float* ssm_in, float* ssm_out, float* co_scratch, float* out_dev, bool conv_done = false, uint16_t* aop = nullptr, float aop_up = 1.0f, const GdnQ* gq = nullptr);
 
-// Chunked (64-token) form of the same recurrence on the fp32 matrix cores; T must be a positive multiple of 64.
-// scratch: co [T][ch], logg [T][nv], beta [T][nv], oraw [T][nv*dv].
-int pyre_gdn_prefill_launch(pyre_ctx* ctx, const GdnDev& g, const float* proj, int proj_stride, int T, const float* conv_in, float* conv_out,
-                            const float* ssm_in, float* ssm_out, float* co, float* logg, float* beta, float* oraw, float* out_dev);
+// Chunked (64-token) form of the same recurrence on the fp32 matrix cores (gdn_prefill.hip), any T >= 1: raw outputs
+// oraw [T][nv*dv] (no head norm: pyre_blk_gdn_out_launch), states conv_in -> conv_out and ssm_in -> ssm_out (in == out is fine).
+struct GdnChunk { float* co; float* kt; float* w; float* u; float* p; float* dec; };
+size_t pyre_gdn_chunk_bytes(const GdnDev& g, int T);
+void   pyre_gdn_chunk_carve(const GdnDev& g, int T, void* base, GdnChunk* b);
+int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int proj_stride, int T, const float* conv_in, float* conv_out,
+                          const float* ssm_in, float* ssm_out, float* oraw);
 
 // ---- gated attention over the KV cache (attn.hip) -----------------------------------------------------------------------
 struct AttnDev { const float* qn; const float* kn; const float* rope_inv; int nh, nkv, hd, n_rot, kv_bits, kv_recent; float eps; float mscale = 1.0f; };   // mscale: YaRN magnitude factor on cos and sin
@@ -426,6 +441,13 @@ size_t pyre_packed_boundary(size_t n_visible, int kv_bits, int recent);
 // qn_ctx::rope_inv (src/qn_ctx.rs:164-185): inverse frequencies [n_rot/2]; YaRN when ctx > ctx_train > 0; returns mscale
 float pyre_rope_table(int n_rot, float base, int ctx_train, int ctx, float* inv_host);
 
+// Queries start .. start + T - 1 of a prompt over the cache (attn_prompt.hip).  pyre_attn_blk_prep: K and V of those positions into
+// the cache, the packing, and the rotated queries as halves qh [T][nh][2][hd] with qsc [T][nh] (q: their f32 rows, or null);
+// pyre_attn_prompt_launch: out [T][nh*hd], scratch of pyre_attn_prompt_bytes.
+int pyre_attn_blk_prep(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const float* qkv, int stride, int start, int T, int* packed_done, float* q, uint16_t* qh, float* qsc);
+size_t pyre_attn_prompt_bytes(const AttnDev& a, int start, int T);
+int pyre_attn_prompt_launch(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const uint16_t* qh, const float* qsc, const float* qkv, int stride, int start, int T, void* scratch, float* out);
+
 // ---- QSA sparse indexer (qsa.hip), qwen4exp_gguf.rs:1565-1599 ------------------------------------------------------------
 // Blocks of `ratio` tokens; a query that sees more than budget + ratio - 1 positions attends to the budget / ratio
 // blocks with the largest  sum_h relu(q_h . block key) / sqrt(hd)  and to the incomplete tail.
@@ -452,5 +474,5 @@ int pyre_qsa_launch(pyre_ctx* ctx, const QsaDev& q, const AttnDev& a, const QsaB
 int pyre_qsa_pool_all(pyre_ctx* ctx, const QsaDev& q, const AttnDev& a, const QsaBuf& b, int n);
 // the attention launch with an optional position list (qw == nullptr: dense)
 int pyre_attn_launch_sel(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const AttnWork& w, const float* qkv, int qkv_stride, int start, int t,
-                         int* packed_done, float* out_dev, const int* posp, const QsaWork* qw, int part = 0);      // part: 1 = the cache write alone, 2 = the pass over the cache and the merge alone (w.q / qh / qsc kept in between), 0 = both
+                         int* packed_done, float* out_dev, const int* posp, const QsaWork* qw);
 int pyre_attn_append_launch(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const AttnWork& w, const float* qkv, int stride, int start, int t);      // K / V only

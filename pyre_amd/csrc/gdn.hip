@@ -25,31 +25,6 @@ __global__ __launch_bounds__(256) void k_gdn_conv(const float* __restrict__ proj
   for (int k = 0; k < kk - 1; ++k) conv_out[(size_t)k * ch + c] = hist[k];
 }
 
-// The same for n consecutive windows of t tokens in one launch (a long prompt's blocks): grid (ceil(ch/256), n).  Window z's
-// projection rows lie at proj + z * ws, its output at co + z * ws (the windows' workspaces, ws floats apart); its history is
-// the last kk - 1 rows of window z - 1's projection -- for window 0 the kk - 1 rows at prev (row stride prev_stride: the
-// layer's convolution state, or the projection rows of the window in front of the group).  The last window leaves the state
-// in conv_out if that is given.  A channel's arithmetic is k_gdn_conv's, so are its bits.  Needs t >= kk - 1.
-__global__ __launch_bounds__(256) void k_gdn_conv_blk(const float* __restrict__ proj, int stride, int t, int ch, int kk, const float* __restrict__ conv_w, size_t ws,
-                                                      const float* __restrict__ prev, int prev_stride, float* __restrict__ conv_out, float* __restrict__ co) {
-  const int c = blockIdx.x * 256 + threadIdx.x, z = blockIdx.y; if (c >= ch) return;
-  const float* pz = proj + (size_t)z * ws;
-  float w[8], hist[8];
-  for (int k = 0; k < kk; ++k) w[k] = conv_w[(size_t)c * kk + k];
-  if (z == 0) { for (int k = 0; k < kk - 1; ++k) hist[k] = prev[(size_t)k * prev_stride + c]; }
-  else { const float* pp = pz - ws + (size_t)(t - (kk - 1)) * stride; for (int k = 0; k < kk - 1; ++k) hist[k] = pp[(size_t)k * stride + c]; }
-  float* cz = co + (size_t)z * ws;
-  for (int ti = 0; ti < t; ++ti) {
-    float cur = pz[(size_t)ti * stride + c];
-    float o = w[kk - 1] * cur;
-    for (int k = 0; k < kk - 1; ++k) o += w[k] * hist[k];
-    cz[(size_t)ti * ch + c] = o * g_sigm(o);
-    for (int k = 0; k + 1 < kk - 1; ++k) hist[k] = hist[k + 1];
-    hist[kk - 2] = cur;
-  }
-  if (conv_out && z == (int)gridDim.y - 1) for (int k = 0; k < kk - 1; ++k) conv_out[(size_t)k * ch + c] = hist[k];
-}
-
 // grid nv, 512 threads (8 waves), at most 8 tokens.  Thread (grp = tid/128, j = tid%128) keeps rows 32*grp..32*grp+31 of
 // column j of the head's 128x128 state in registers across the whole window, so the state is read once and written once
 // per launch.  Whatever does not depend on the state is done per token by one wave each, before the recurrence (wave ti
@@ -127,12 +102,9 @@ __global__ __launch_bounds__(512) void k_gdn_delta(GdnDev p, const float* __rest
 // all 128 columns, so it is left to the consumer (the output projection, PyreAop::sq): wave ti leaves token ti's
 // un-normalised gated output u = (o * norm_w) * sigmoid(z) of its 32 columns as f16 operand rows scaled by the quarter's own
 // power of two (its largest magnitude into [2^13, 2^14)), that factor's inverse, and the quarter's sum of o^2.
-// nwin > 1 (a long prompt's blocks): nwin consecutive windows of t tokens in one launch -- window wi's projection, convolution
-// output, operand rows and sums lie ws floats further on per window (the windows' workspaces); the state stays in registers
-// from window to window, is fetched once and stored once.  A token's arithmetic is the same whatever nwin.
 template <int DK, int DV, int FT = 0, int FNK = 0, int FNV = 0>
 __global__ __launch_bounds__(512) void k_gdn_delta_q(GdnDev p, const float* __restrict__ proj, int stride, int t, const float* __restrict__ co_all,
-                                                     const float* __restrict__ ssm_in, float* __restrict__ ssm_out, uint16_t* __restrict__ aop, int aop_rows, float* __restrict__ sq, int nwin, size_t ws) {
+                                                     const float* __restrict__ ssm_in, float* __restrict__ ssm_out, uint16_t* __restrict__ aop, int aop_rows, float* __restrict__ sq) {
   static_assert(DK == 128 && DV == 128, "tiling assumes 128x128 heads");
   constexpr int QC = 32, G = 16, R = DK / G, MT = 8;
   args_now(p.a, p.dt, p.norm_w, p.nk, p.nv, p.eps, proj, stride, t, co_all, ssm_in, ssm_out, aop, sq);
@@ -143,72 +115,61 @@ __global__ __launch_bounds__(512) void k_gdn_delta_q(GdnDev p, const float* __re
   const int ch = 2 * p.nk * DK + p.nv * DV, w = p.nv * DV, jc = qd * QC + j;
   const float* sin_ = ssm_in + (size_t)h * DK * DV; float* sout = ssm_out + (size_t)h * DK * DV;
   float q0 = 0.0f, q1 = 0.0f, k0 = 0.0f, k1 = 0.0f, v0 = 0.0f, z0 = 0.0f, alpha_raw = 0.0f, beta_raw = 0.0f;
-  auto fetch = [&](int wi) {          // wave ti: token ti's inputs of window wi
-    if (wave < t) {
-      const float* co = co_all + (size_t)wi * ws + (size_t)wave * ch; const float* pr = proj + (size_t)wi * ws + (size_t)wave * stride;
-      q0 = co[kh * DK + lane]; q1 = co[kh * DK + lane + 64]; k0 = co[p.nk * DK + kh * DK + lane]; k1 = co[p.nk * DK + kh * DK + lane + 64];
-      v0 = co[2 * p.nk * DK + h * DV + qd * QC + (lane & 31)]; z0 = pr[ch + h * DV + qd * QC + (lane & 31)];
-      alpha_raw = pr[ch + w + p.nv + h]; beta_raw = pr[ch + w + h];
-    }
-  };
-  fetch(0);
+  if (wave < t) {          // wave ti: token ti's inputs
+    const float* co = co_all + (size_t)wave * ch; const float* pr = proj + (size_t)wave * stride;
+    q0 = co[kh * DK + lane]; q1 = co[kh * DK + lane + 64]; k0 = co[p.nk * DK + kh * DK + lane]; k1 = co[p.nk * DK + kh * DK + lane + 64];
+    v0 = co[2 * p.nk * DK + h * DV + qd * QC + (lane & 31)]; z0 = pr[ch + h * DV + qd * QC + (lane & 31)];
+    alpha_raw = pr[ch + w + p.nv + h]; beta_raw = pr[ch + w + h];
+  }
   const float a = p.a[h], dtb = p.dt[h], nw = p.norm_w[qd * QC + (lane & 31)];
   float S[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) S[r] = sin_[(size_t)(rg * R + r) * DV + jc];
-  for (int wi = 0; wi < nwin; ++wi) {
-    if (wave < t) {          // L2 norms of q and k (:1649-1651): the sum of each half of the vector, then the two halves -- as in k_gdn_delta
-      const float sq_ = wave_sum(q0 * q0) + wave_sum(q1 * q1), sk = wave_sum(k0 * k0) + wave_sum(k1 * k1);
-      const float fq = (1.0f / sqrtf(sq_ + 1e-6f)) * (1.0f / sqrtf((float)DK)), fk = (1.0f / sqrtf(sk + 1e-6f)) * 1.0f;
-      qs[wave][lane] = q0 * fq; qs[wave][lane + 64] = q1 * fq; ks[wave][lane] = k0 * fk; ks[wave][lane + 64] = k1 * fk;
-      if (lane < QC) { vs[wave][lane] = v0; zs[wave][lane] = z0; }
-      if (lane == 0) { gs[wave] = expf(g_softplus(alpha_raw + dtb) * a); bs[wave] = g_sigm(beta_raw); }
-    }
-    if (wi + 1 < nwin) fetch(wi + 1);          // the next window's inputs travel behind this window's recurrence
+  if (wave < t) {          // L2 norms of q and k (:1649-1651): the sum of each half of the vector, then the two halves -- as in k_gdn_delta
+    const float sq_ = wave_sum(q0 * q0) + wave_sum(q1 * q1), sk = wave_sum(k0 * k0) + wave_sum(k1 * k1);
+    const float fq = (1.0f / sqrtf(sq_ + 1e-6f)) * (1.0f / sqrtf((float)DK)), fk = (1.0f / sqrtf(sk + 1e-6f)) * 1.0f;
+    qs[wave][lane] = q0 * fq; qs[wave][lane + 64] = q1 * fq; ks[wave][lane] = k0 * fk; ks[wave][lane + 64] = k1 * fk;
+    if (lane < QC) { vs[wave][lane] = v0; zs[wave][lane] = z0; }
+    if (lane == 0) { gs[wave] = expf(g_softplus(alpha_raw + dtb) * a); bs[wave] = g_sigm(beta_raw); }
+  }
+  lds_barrier();
+  for (int ti = 0; ti < t; ++ti) {
+    const float g = gs[ti], b = bs[ti];
+    float pmv = 0.0f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) { S[r] *= g; pmv += S[r] * ks[ti][rg * R + r]; }
+    pm[ti & 1][rg][j] = pmv;
     lds_barrier();
-    for (int ti = 0; ti < t; ++ti) {
-      const float g = gs[ti], b = bs[ti];
-      float pmv = 0.0f;
+    float mem = pm[ti & 1][0][j];
 #pragma unroll
-      for (int r = 0; r < R; ++r) { S[r] *= g; pmv += S[r] * ks[ti][rg * R + r]; }
-      pm[ti & 1][rg][j] = pmv;
-      lds_barrier();
-      float mem = pm[ti & 1][0][j];
+    for (int k = 1; k < G; ++k) mem += pm[ti & 1][k][j];
+    const float delta = (vs[ti][j] - mem) * b;
+    float pov = 0.0f;
 #pragma unroll
-      for (int k = 1; k < G; ++k) mem += pm[ti & 1][k][j];
-      const float delta = (vs[ti][j] - mem) * b;
-      float pov = 0.0f;
+    for (int r = 0; r < R; ++r) { S[r] += ks[ti][rg * R + r] * delta; pov += S[r] * qs[ti][rg * R + r]; }
+    po[ti][rg][j] = pov;
+  }
 #pragma unroll
-      for (int r = 0; r < R; ++r) { S[r] += ks[ti][rg * R + r] * delta; pov += S[r] * qs[ti][rg * R + r]; }
-      po[ti][rg][j] = pov;
-    }
-    if (wi + 1 == nwin) {
+  for (int r = 0; r < R; ++r) sout[(size_t)(rg * R + r) * DV + jc] = S[r];
+  lds_barrier();
+  if (wave < t) {
+    const int jl = lane & 31; const bool on = lane < QC;
+    float o = po[wave][0][jl];
 #pragma unroll
-      for (int r = 0; r < R; ++r) sout[(size_t)(rg * R + r) * DV + jc] = S[r];
-    }
-    lds_barrier();
-    if (wave < t) {
-      const int jl = lane & 31; const bool on = lane < QC;
-      float o = po[wave][0][jl];
-#pragma unroll
-      for (int k = 1; k < G; ++k) o += po[wave][k][jl];
-      const float ss = wave_sum(on ? o * o : 0.0f);
-      const float u = (o * nw) * g_sigm(zs[wave][jl]);
-      float am = on ? fabsf(u) : 0.0f; am = am == am ? am : INFINITY;
-      am = wave_max(am);
-      int e = 0;
-      if (am > 0.0f && am < INFINITY) { e = 140 - (int)((__float_as_uint(am) >> 23) & 0xFF); e = e > 100 ? 100 : e; }
-      uint16_t* aw = aop + (size_t)wi * ws * 2; float* sw = sq + (size_t)wi * ws;
-      if (on) aop_store(aw, aop_rows, h * DV + qd * QC + jl, wave, u * __uint_as_float((uint32_t)(127 + e) << 23));
-      if (lane == 0) { sw[((size_t)wave * p.nv + h) * 4 + qd] = __uint_as_float((uint32_t)(127 - e) << 23); sw[(size_t)8 * p.nv * 4 + ((size_t)wave * p.nv + h) * 4 + qd] = ss; }
-    }
-    if (wi + 1 < nwin) lds_barrier();          // the next window's inputs overwrite what this window's outputs were read from
+    for (int k = 1; k < G; ++k) o += po[wave][k][jl];
+    const float ss = wave_sum(on ? o * o : 0.0f);
+    const float u = (o * nw) * g_sigm(zs[wave][jl]);
+    float am = on ? fabsf(u) : 0.0f; am = am == am ? am : INFINITY;
+    am = wave_max(am);
+    int e = 0;
+    if (am > 0.0f && am < INFINITY) { e = 140 - (int)((__float_as_uint(am) >> 23) & 0xFF); e = e > 100 ? 100 : e; }
+    if (on) aop_store(aop, aop_rows, h * DV + qd * QC + jl, wave, u * __uint_as_float((uint32_t)(127 + e) << 23));
+    if (lane == 0) { sq[((size_t)wave * p.nv + h) * 4 + qd] = __uint_as_float((uint32_t)(127 - e) << 23); sq[(size_t)8 * p.nv * 4 + ((size_t)wave * p.nv + h) * 4 + qd] = ss; }
   }
 }
 
 int pyre_gdn_launch(pyre_ctx* ctx, const GdnDev& g, const float* proj, int stride, int t, const float* conv_in, float* conv_out,
-                    const float* ssm_in, float* ssm_out, float* co, float* out, bool conv_done, uint16_t* aop, float aop_up, const GdnQ* gq, int nwin, size_t ws) {
-  if (nwin < 1 || (nwin > 1 && !(gq && conv_done))) return pyre_fail(ctx, PYRE_E_ARG, "gdn: several windows a launch need the per-quarter form behind a finished convolution");
+                    const float* ssm_in, float* ssm_out, float* co, float* out, bool conv_done, uint16_t* aop, float aop_up, const GdnQ* gq) {
   if (aop && t > 8) return pyre_fail(ctx, PYRE_E_ARG, "gdn: an f16 operand holds at most 8 tokens, not %d", t);
   if (gq && (!gq->op || !gq->sq)) return pyre_fail(ctx, PYRE_E_ARG, "gdn: the per-quarter form needs its operand and scale arrays");
   if (g.dk != 128 || g.dv != 128) return pyre_fail(ctx, PYRE_E_SHAPE, "gdn: head dims %dx%d unsupported (128x128 only)", g.dk, g.dv);
@@ -218,12 +179,12 @@ int pyre_gdn_launch(pyre_ctx* ctx, const GdnDev& g, const float* proj, int strid
   if (!conv_done) { ProfScope ps(ctx, "gdn_conv", 4.0 * ch * (2.0 * (g.conv_k - 1) + g.conv_k + 2.0 * t)); hipLaunchKernelGGL(k_gdn_conv, dim3((ch + 255) / 256), dim3(256), 0, ctx->stream, proj, stride, t, ch, g.conv_k, g.conv_w, conv_in, conv_out, co); } PYRE_CHECK_LAUNCH(ctx);
   if (gq) {
     ProfScope ps(ctx, "gdn_delta", 8.0 * g.nv * g.dk * g.dv + 4.0 * t * (ch + 2.0 * g.nv * g.dv));
-#define GDN_Q_FIX(FT) hipLaunchKernelGGL((k_gdn_delta_q<128, 128, FT, 16, 32>), dim3(g.nv, 4), dim3(512), 0, ctx->stream, g, proj, stride, t, co, ssm_in, ssm_out, gq->op, pyre_aop_rows(t), gq->sq, nwin, ws)
+#define GDN_Q_FIX(FT) hipLaunchKernelGGL((k_gdn_delta_q<128, 128, FT, 16, 32>), dim3(g.nv, 4), dim3(512), 0, ctx->stream, g, proj, stride, t, co, ssm_in, ssm_out, gq->op, pyre_aop_rows(t), gq->sq)
     if (g.nk == 16 && g.nv == 32) {          // the A3B geometry: the window width and the head counts folded in
       switch (t) { case 1: GDN_Q_FIX(1); break; case 2: GDN_Q_FIX(2); break; case 3: GDN_Q_FIX(3); break; case 4: GDN_Q_FIX(4); break; case 5: GDN_Q_FIX(5); break; case 6: GDN_Q_FIX(6); break; case 7: GDN_Q_FIX(7); break; default: GDN_Q_FIX(8); break; }
     }
 #undef GDN_Q_FIX
-    else hipLaunchKernelGGL((k_gdn_delta_q<128, 128>), dim3(g.nv, 4), dim3(512), 0, ctx->stream, g, proj, stride, t, co, ssm_in, ssm_out, gq->op, pyre_aop_rows(t), gq->sq, nwin, ws);
+    else hipLaunchKernelGGL((k_gdn_delta_q<128, 128>), dim3(g.nv, 4), dim3(512), 0, ctx->stream, g, proj, stride, t, co, ssm_in, ssm_out, gq->op, pyre_aop_rows(t), gq->sq);
     PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
   }
   { ProfScope ps(ctx, "gdn_delta", 8.0 * g.nv * g.dk * g.dv + 4.0 * t * (ch + 2.0 * g.nv * g.dv)); if (t == 1 && g.nk == 16 && g.nv == 32) hipLaunchKernelGGL((k_gdn_delta<128, 128, 1, 16, 32>), dim3(g.nv), dim3(512), 0, ctx->stream, g, proj, stride, t, co, ssm_in, ssm_out, out, aop, aop ? pyre_aop_rows(t) : 0, aop_up);          // a single token of the A3B geometry: constants folded in
@@ -231,18 +192,11 @@ int pyre_gdn_launch(pyre_ctx* ctx, const GdnDev& g, const float* proj, int strid
   return PYRE_OK;
 }
 
-int pyre_gdn_conv_block_launch(pyre_ctx* ctx, const GdnDev& g, const float* proj, int stride, int t, int n, size_t ws, const float* prev, int prev_stride, float* conv_out, float* co) {
-  if (g.conv_k < 2 || g.conv_k > 8 || t < g.conv_k - 1 || t > 8 || n < 1) return pyre_fail(ctx, PYRE_E_ARG, "gdn block conv: kernel %d, %d windows of %d tokens", g.conv_k, n, t);
-  const int ch = 2 * g.nk * g.dk + g.nv * g.dv;
-  ProfScope ps(ctx, "gdn_conv", 4.0 * ch * n * (g.conv_k + 2.0 * t));
-  hipLaunchKernelGGL(k_gdn_conv_blk, dim3((ch + 255) / 256, n), dim3(256), 0, ctx->stream, proj, stride, t, ch, g.conv_k, g.conv_w, ws, prev, prev_stride, conv_out, co);
-  PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
-}
 
 // ---- C ABI: standalone layer core for the block harness ---------------------------------------------------------------
 struct pyre_gdn {
   pyre_ctx* ctx; GdnDev dv; float* params; int ch, pw;      // pw = projection width per token
-  float* conv[2]; float* ssm[2]; int cur; float* co; float* io; size_t io_tokens;
+  float* conv[2]; float* ssm[2]; int cur; float* co; float* io; size_t io_tokens; void* chunk_mem = nullptr; size_t chunk_bytes = 0;      // (grow-only: inputs and outputs, the chunked form's scratch)
 };
 
 extern "C" {
@@ -264,7 +218,7 @@ int pyre_gdn_create(pyre_ctx* ctx, int nk, int nv, int dk, int dv, int conv_k, f
   g->dv = GdnDev{g->params, g->params + nv, g->params + 2 * nv, g->params + 2 * nv + (size_t)g->ch * conv_k, nk, nv, dk, dv, conv_k, eps};
   *out = g; return PYRE_OK;
 }
-void pyre_gdn_destroy(pyre_gdn* g) { if (!g) return; (void)hipStreamSynchronize(g->ctx->stream); (void)hipFree(g->params); for (int i = 0; i < 2; ++i) { (void)hipFree(g->conv[i]); (void)hipFree(g->ssm[i]); } (void)hipFree(g->co); if (g->io) (void)hipFree(g->io); delete g; }
+void pyre_gdn_destroy(pyre_gdn* g) { if (!g) return; (void)hipStreamSynchronize(g->ctx->stream); (void)hipFree(g->params); for (int i = 0; i < 2; ++i) { (void)hipFree(g->conv[i]); (void)hipFree(g->ssm[i]); } (void)hipFree(g->co); if (g->io) (void)hipFree(g->io); if (g->chunk_mem) (void)hipFree(g->chunk_mem); delete g; }
 
 int pyre_gdn_set_state(pyre_ctx* ctx, pyre_gdn* g, const float* conv_host, const float* ssm_host) {
   if (!ctx || !g) return pyre_fail(ctx, PYRE_E_ARG, "pyre_gdn_set_state: null argument");
@@ -303,7 +257,7 @@ int pyre_gdn_step(pyre_ctx* ctx, pyre_gdn* g, const float* proj_host, int t, flo
   PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); return PYRE_OK;
 }
 
-// Prefill of T tokens: whole chunks of 64 go through the matrix-core chunked form, the remainder through the step kernels.
+// Prefill of T tokens in the matrix-core chunked form.
 int pyre_gdn_prefill_chunked(pyre_ctx* ctx, pyre_gdn* g, const float* proj_host, int T, int chunk, float* out_host) {
   if (!ctx || !g || !proj_host || !out_host) return pyre_fail(ctx, PYRE_E_ARG, "pyre_gdn_prefill_chunked: null argument");
   if (T < 1) return pyre_fail(ctx, PYRE_E_ARG, "pyre_gdn_prefill_chunked: T = %d", T);
@@ -311,21 +265,15 @@ int pyre_gdn_prefill_chunked(pyre_ctx* ctx, pyre_gdn* g, const float* proj_host,
   int rc = gdn_io(ctx, g, T); if (rc) return rc;
   float* pd = g->io; float* od = g->io + (size_t)T * g->pw; size_t ow = (size_t)g->dv.nv * g->dv.dv;
   PYRE_HIP(ctx, hipMemcpyAsync(pd, proj_host, (size_t)T * g->pw * 4, hipMemcpyHostToDevice, ctx->stream));
-  int Tc = T / 64 * 64;
-  if (Tc) {
-    float* scr = nullptr; size_t n = (size_t)Tc * ((size_t)g->ch + 2 * g->dv.nv + ow);
-    PYRE_HIP(ctx, hipMalloc((void**)&scr, n * 4));
-    float* co = scr; float* lg = co + (size_t)Tc * g->ch; float* be = lg + (size_t)Tc * g->dv.nv; float* oraw = be + (size_t)Tc * g->dv.nv; int nx = g->cur ^ 1;
-    rc = pyre_gdn_prefill_launch(ctx, g->dv, pd, g->pw, Tc, g->conv[g->cur], g->conv[nx], g->ssm[g->cur], g->ssm[nx], co, lg, be, oraw, od);
-    hipError_t e = hipStreamSynchronize(ctx->stream); (void)hipFree(scr);
-    if (rc) return rc; if (e != hipSuccess) return pyre_fail(ctx, PYRE_E_HIP, "pyre_gdn_prefill_chunked: %s", hipGetErrorString(e));
-    g->cur = nx;
+  const size_t cb = pyre_gdn_chunk_bytes(g->dv, T), need = cb + (size_t)T * ow * 4;
+  if (g->chunk_bytes < need) {
+    if (g->chunk_mem) { PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); PYRE_HIP(ctx, hipFree(g->chunk_mem)); g->chunk_mem = nullptr; g->chunk_bytes = 0; }
+    PYRE_HIP(ctx, hipMalloc(&g->chunk_mem, need)); g->chunk_bytes = need;
   }
-  for (int t0 = Tc; t0 < T; t0 += 8) {
-    int n = T - t0 < 8 ? T - t0 : 8; int nx = g->cur ^ 1;
-    rc = pyre_gdn_launch(ctx, g->dv, pd + (size_t)t0 * g->pw, g->pw, n, g->conv[g->cur], g->conv[nx], g->ssm[g->cur], g->ssm[nx], g->co, od + (size_t)t0 * ow); if (rc) return rc;
-    g->cur = nx;
-  }
+  GdnChunk ck; pyre_gdn_chunk_carve(g->dv, T, g->chunk_mem, &ck); float* oraw = (float*)((uint8_t*)g->chunk_mem + cb); const int nx = g->cur ^ 1;
+  rc = pyre_gdn_chunk_launch(ctx, g->dv, ck, pd, g->pw, T, g->conv[g->cur], g->conv[nx], g->ssm[g->cur], g->ssm[nx], oraw); if (rc) return rc;
+  g->cur = nx;
+  if ((rc = pyre_blk_gdn_out_launch(ctx, oraw, pd + g->ch, g->pw, g->dv.norm_w, g->dv.eps, g->dv.nv, T, 1.0f, nullptr, 0, od))) return rc;
   PYRE_HIP(ctx, hipMemcpyAsync(out_host, od, (size_t)T * ow * 4, hipMemcpyDeviceToHost, ctx->stream));
   PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); return PYRE_OK;
 }

@@ -1,171 +1,242 @@
-// Gated DeltaNet prefill in chunked form on the fp32 matrix cores (v_mfma_f32_32x32x2_f32).
+// Gated DeltaNet over a prompt in chunked form on the fp32 matrix cores (v_mfma_f32_16x16x4_f32).
 //
 // The reference has no chunked form (linear_core runs the recurrence token by token, src/model/qwen4exp_gguf.rs:
 // 1654-1670); this is the same recurrence regrouped per chunk of C = 64 tokens.  With L_i = sum_{j<=i} log g_j inside
 // the chunk and S_0 the state at its start,
-//     delta_i = beta_i ( v_i - e^{L_i} S_0^T k_i - sum_{j<i} e^{L_i-L_j} (k_i.k_j) delta_j )        (I + A) Delta = B
-//     o_i     = e^{L_i} S_0^T q_i + sum_{j<=i} e^{L_i-L_j} (q_i.k_j) delta_j                        O = O1 + P Delta
+//     (I + A) Delta = diag(beta) (V - diag(e^L) K S_0),   A_ij = beta_i e^{L_i-L_j} k_i.k_j  (j < i)
+//     o_i     = e^{L_i} S_0^T q_i + sum_{j<=i} P_ij delta_j,   P_ij = e^{L_i-L_j} q_i.k_j
 //     S_C     = e^{L_C} S_0 + sum_j e^{L_C-L_j} k_j (x) delta_j
 // Every decay factor is the exponential of a non-positive difference of log-decays, so nothing overflows however
-// strong the gate is.  State columns are independent, so each value head is split into column blocks of 32.
+// strong the gate is.  Delta is linear in S_0:  Delta = U - W S_0 with (I + A) [W | U] = [diag(beta e^L) K | diag(beta) V], so
+// everything but three products with the state is done for all chunks at once:
+//   k_gdnc_conv   convolution, SiLU, L2 norms, k once more transposed                     (all tokens)
+//   k_gdnc_chunk  A, P, the solve for W and U                                             (chunks x heads workgroups)
+//   k_gdnc_scan   Delta, the outputs and the state, chunk after chunk                     (heads x 8 workgroups of 16 state columns)
+// When one workgroup did all of it per chunk a chunk took 39 us and a prompt of 4096 tokens 2.5 ms (the serial solve, with half of
+// the chip idle); the scan, now the only serial part, is three small products.  fp32 throughout.
+// Tokens past T in the last chunk have beta = 0, k = q = 0 and no decay: they leave the state as it is.
 #include "formats.h"
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float v4f_ __attribute__((ext_vector_type(4)));
 
+namespace {
+
+constexpr int C = 64, DK = 128;
 __device__ __forceinline__ float p_sigm(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float p_softplus(float x) { return x > 20.0f ? x : log1pf(expf(x)); }
+// four steps of a 16x16x4 product: lane (row, q) holds a[i] = A[row][4 q + i], b[i] = B[4 q + i][column]: the sum over sixteen k
+__device__ __forceinline__ v4f_ mac16(const float4& a, const float4& b, v4f_ acc) {
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, acc, 0, 0, 0); acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, b.y, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, b.z, acc, 0, 0, 0); return __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, b.w, acc, 0, 0, 0);
+}
+__device__ __forceinline__ float4 as4(const v4f_& v) { return make_float4(v[0], v[1], v[2], v[3]); }
 
-// conv + SiLU for every (token, channel); the window of the first conv_k-1 tokens reaches into conv_in (oldest first).
-__global__ void k_gdnp_conv(const float* __restrict__ proj, int stride, int T, int ch, int kk, const float* __restrict__ conv_w, const float* __restrict__ conv_in,
-                            float* __restrict__ co, float* __restrict__ conv_out) {
-  int c = blockIdx.x * blockDim.x + threadIdx.x, ti = blockIdx.y; if (c >= ch) return;
-  float o = conv_w[(size_t)c * kk + kk - 1] * proj[(size_t)ti * stride + c];
-  for (int k = 0; k < kk - 1; ++k) { int src = ti - (kk - 1) + k; float v = src >= 0 ? proj[(size_t)src * stride + c] : conv_in[(size_t)(kk - 1 + src) * ch + c]; o += conv_w[(size_t)c * kk + k] * v; }
-  co[(size_t)ti * ch + c] = o * p_sigm(o);
-  if (ti == T - 1) for (int k = 0; k < kk - 1; ++k) { int src = T - (kk - 1) + k; conv_out[(size_t)k * ch + c] = src >= 0 ? proj[(size_t)src * stride + c] : conv_in[(size_t)(kk - 1 + src) * ch + c]; }
+// grid (ch / 256, ceil(Tp / 16)), 256 threads: thread = channel, sixteen tokens (the taps and the history are fetched once for
+// them).  Channels of q and k: two heads a workgroup, L2-normalised over their 128 channels (q also x 1/sqrt(dk)); k also goes to kt
+// [chunk][key head][128][64].  Tokens T .. Tp-1 (the last chunk's padding) become zeros.
+template <int KK>
+__global__ __launch_bounds__(256) void k_gdnc_conv(GdnDev p, const float* __restrict__ proj, int stride, int T, int Tp, const float* __restrict__ conv_in, float* __restrict__ conv_out, float* __restrict__ co, float* __restrict__ kt) {
+  __shared__ float red[4][16];
+  const int c = blockIdx.x * 256 + threadIdx.x, t0 = blockIdx.y * 16, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv; const bool in = c < ch;
+  const int kk = KK ? KK : p.conv_k;
+  float w[8], h[16 + 7];          // h[7 + i]: token t0 + i; before it the history
+#pragma unroll
+  for (int k = 0; k < 8; ++k) w[k] = in && k < kk ? p.conv_w[(size_t)c * kk + k] : 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16 + 7; ++i) {
+    const int t = t0 + i - 7; h[i] = 0.0f;
+    if (in && t < T && i >= 7 - (kk - 1)) h[i] = t >= 0 ? proj[(size_t)t * stride + c] : (t >= -(kk - 1) ? conv_in[(size_t)(kk - 1 + t) * ch + c] : 0.0f);
+  }
+  float v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    float o = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) if (k == kk - 1) o = w[k] * h[7 + i];
+#pragma unroll
+    for (int k = 0; k < 7; ++k) if (k < kk - 1) {          // tap k reads token i - (kk - 1) + k
+      float hv = 0.0f;
+#pragma unroll
+      for (int b = 0; b < 8; ++b) if (b == kk - 1 - k) hv = h[7 + i - b];
+      o += w[k] * hv;
+    }
+    v[i] = t0 + i < T ? o * p_sigm(o) : 0.0f;
+  }
+  if (blockIdx.x * 256 < 2 * nqk) {          // (uniform: 2 nk heads of 128 channels, two a workgroup; nk even or the last pair ends with a head of v, whose factor stays 1)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) { const float s = wave_sum(v[i] * v[i]); if (lane == 0) red[wave][i] = s; }
+    lds_barrier();
+    if (c < 2 * nqk) {
+      const float f = c < nqk ? 1.0f / sqrtf((float)DK) : 1.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = v[i] * ((1.0f / sqrtf(red[wave & 2][i] + red[(wave & 2) + 1][i] + 1e-6f)) * f);
+    }
+  }
+  if (!in) return;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) co[(size_t)(t0 + i) * ch + c] = v[i];
+  if (c >= nqk && c < 2 * nqk) {
+    float* k2 = kt + (((size_t)(t0 / C) * p.nk + (c - nqk) / DK) * DK + (c - nqk) % DK) * C + t0 % C;
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) *(float4*)(k2 + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
+  }
+  if (t0 <= T - 1 && T - 1 < t0 + 16) for (int k = 0; k < kk - 1; ++k) {          // (in == out is fine: only the first group of sixteen reads conv_in, and it has)
+    const int src = T - (kk - 1) + k;
+    if (src >= 0) conv_out[(size_t)k * ch + c] = proj[(size_t)src * stride + c];
+    else { float hv = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 7; ++i) if (i - 7 == src) hv = h[i];
+      conv_out[(size_t)k * ch + c] = hv; }
+  }
 }
 
-// grid (T, nk + 1), 128 threads.  y < nk: L2-normalise q (x 1/sqrt(dk)) and k of key head y in place;
-// y == nk: per value head log-decay softplus(alpha + dt) * a and beta = sigmoid(beta).
-__global__ __launch_bounds__(128) void k_gdnp_prep(GdnDev p, const float* __restrict__ proj, int stride, float* __restrict__ co, float* __restrict__ logg, float* __restrict__ beta) {
-  __shared__ float red[4];
-  const int ti = blockIdx.x, y = blockIdx.y, tid = threadIdx.x; const int ch = 2 * p.nk * p.dk + p.nv * p.dv, w = p.nv * p.dv;
-  if (y == p.nk) { for (int h = tid; h < p.nv; h += 128) { const float* pr = proj + (size_t)ti * stride; logg[(size_t)ti * p.nv + h] = p_softplus(pr[ch + w + p.nv + h] + p.dt[h]) * p.a[h]; beta[(size_t)ti * p.nv + h] = p_sigm(pr[ch + w + h]); } return; }
-  float* q = co + (size_t)ti * ch + (size_t)y * p.dk; float* k = q + (size_t)p.nk * p.dk;
-  float qv = q[tid], kv = k[tid], sq = qv * qv, sk = kv * kv;
+// grid (chunks, nv), 4 waves.  dec [chunk][head][2][64]: e^{L_i}, e^{L_C-L_j}.
+__global__ __launch_bounds__(256) void k_gdnc_chunk(GdnDev p, const float* __restrict__ co, const float* __restrict__ proj, int stride, int T, float* __restrict__ W, float* __restrict__ U, float* __restrict__ P, float* __restrict__ dec) {
+  __shared__ __align__(16) float Ks[C][DK + 4], Qs[C][DK + 4], A[C][C + 4], Ti[4][16][20];          // (rows padded against bank conflicts); A holds -A below its diagonal blocks, A inside them
+  __shared__ double L[C]; __shared__ float Bt[C], eL[C];
+  const int ck = blockIdx.x, h = blockIdx.y, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv, w = p.nv * p.dv, t0 = ck * C;
+  const float* qc = co + (size_t)t0 * ch + (size_t)kh * DK; const float* kc = qc + nqk; const float* vc = co + (size_t)t0 * ch + 2 * nqk + (size_t)h * p.dv;
+  for (int i = tid; i < C * (DK / 4); i += 256) { const int row = i >> 5, c4 = (i & 31) * 4; *(float4*)&Ks[row][c4] = *(const float4*)(kc + (size_t)row * ch + c4); *(float4*)&Qs[row][c4] = *(const float4*)(qc + (size_t)row * ch + c4); }
+  if (wave == 0) {
+    const bool on = t0 + lane < T; const float* pr = proj + (size_t)(on ? t0 + lane : 0) * stride + ch + w;
+    float lg = on ? p_softplus(pr[p.nv + h] + p.dt[h]) * p.a[h] : 0.0f; const float bt = on ? p_sigm(pr[h]) : 0.0f;
+    // the running sum in double: with strong gates it reaches thousands inside a chunk, and what counts are differences of
+    // neighbours' sums, which in f32 would keep three digits
+    double run = 0.0, mine = 0.0;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) { sq += __shfl_xor(sq, o); sk += __shfl_xor(sk, o); }
-  if ((tid & 63) == 0) { red[tid >> 6] = sq; red[2 + (tid >> 6)] = sk; }
+    for (int i = 0; i < C; ++i) { run += (double)__int_as_float(__builtin_amdgcn_readlane(__float_as_int(lg), i)); if (lane == i) mine = run; }
+    L[lane] = mine; Bt[lane] = bt; const float e = expf((float)mine); eL[lane] = e;
+    float* d = dec + ((size_t)ck * p.nv + h) * 2 * C; d[lane] = e; d[C + lane] = expf((float)(run - mine));
+  }
   __syncthreads();
-  q[tid] = qv * ((1.0f / sqrtf(red[0] + red[1] + 1e-6f)) * (1.0f / sqrtf((float)p.dk)));
-  k[tid] = kv * ((1.0f / sqrtf(red[2] + red[3] + 1e-6f)) * 1.0f);
-}
-
-// grid (nv, dv/32), 256 threads (4 waves).  One workgroup carries 32 columns of one head's state through all chunks.
-template <int DK, int C>
-__global__ __launch_bounds__(256) void k_gdnp_chunk(GdnDev p, const float* __restrict__ co, const float* __restrict__ logg, const float* __restrict__ beta, int nchunks,
-                                                    const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
-  static_assert(DK == 128 && C == 64, "tiling assumes dk = 128 and chunks of 64");
-  __shared__ float S[DK][33];        // state block [i][c]
-  __shared__ float A[C][C + 1];      // beta_i e^{L_i-L_j} k_i.k_j, j < i
-  __shared__ float P[C][C + 1];      // e^{L_i-L_j} q_i.k_j, j <= i
-  __shared__ float D[C][33];         // B, then Delta
-  __shared__ float L[C], Bt[C];
-  __shared__ __align__(16) float Qs[C][DK + 4], Ks[C][DK + 4];      // the chunk's q and k rows, staged once (rows padded against bank conflicts)
-  const int h = blockIdx.x, cb = blockIdx.y, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int ch = 2 * p.nk * DK + p.nv * p.dv, w = p.nv * p.dv, r = lane & 31, kk = lane >> 5;
-  const float* sin_ = ssm_in + (size_t)h * DK * p.dv + cb * 32; float* sout = ssm_out + (size_t)h * DK * p.dv + cb * 32;
-  for (int i = tid; i < DK * 32; i += 256) S[i >> 5][i & 31] = sin_[(size_t)(i >> 5) * p.dv + (i & 31)];
-  for (int c = 0; c < nchunks; ++c) {
-    const int t0 = c * C;
-    const float* qc = co + (size_t)t0 * ch + (size_t)kh * DK;                 // q_i at qc + i*ch
-    const float* kc = qc + (size_t)p.nk * DK;
-    const float* vc = co + (size_t)t0 * ch + 2 * (size_t)p.nk * DK + (size_t)h * p.dv + cb * 32;
-    __syncthreads();                                                           // previous chunk done with L, A, P, D, Qs, Ks; S final
-    for (int i = tid; i < C * (DK / 4); i += 256) {                            // coalesced: a row is 512 contiguous bytes
-      const int row = i / (DK / 4), c4 = i % (DK / 4);
-      *(float4*)&Qs[row][4 * c4] = *(const float4*)(qc + (size_t)row * ch + 4 * c4); *(float4*)&Ks[row][4 * c4] = *(const float4*)(kc + (size_t)row * ch + 4 * c4);
-    }
-    // the chunk's log-decays are fetched by 64 threads at once (one thread walking them would pay a memory round trip per
-    // token), then summed in token order by one
-    if (tid < C) { Bt[tid] = beta[(size_t)(t0 + tid) * p.nv + h]; L[tid] = logg[(size_t)(t0 + tid) * p.nv + h]; }
-    __syncthreads();
-    if (tid == 0) { float acc = 0.0f; for (int i = 0; i < C; ++i) { acc += L[i]; L[i] = acc; } }
-    __syncthreads();
-    // ---- A and P: 64x64x128 each, tile (ti, tj) with tj <= ti; waves 0..2 take A tiles (0,0),(1,0),(1,1), then P likewise
-    for (int job = wave; job < 6; job += 4) {
-      const int which = job / 3, tsel = job % 3, ti = tsel == 0 ? 0 : 1, tj = tsel == 2 ? 1 : 0;
-      const float* arow = which == 0 ? Ks[32 * ti + r] : Qs[32 * ti + r]; const float* brow = Ks[32 * tj + r];
-      floatx16 acc = {0};
-      for (int k0 = 0; k0 < DK; k0 += 8) {
-        float4 a4 = *(const float4*)(arow + k0 + 4 * kk), b4 = *(const float4*)(brow + k0 + 4 * kk);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.x, b4.x, acc, 0, 0, 0); acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.y, b4.y, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.z, b4.z, acc, 0, 0, 0); acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.w, b4.w, acc, 0, 0, 0);
-      }
+  // A and P: ten 16x16 tiles on or below the diagonal each, five a wave
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        int i = 32 * ti + 8 * (e >> 2) + 4 * kk + (e & 3), j = 32 * tj + r;
-        float dec = j <= i ? expf(L[i] - L[j]) : 0.0f;
-        if (which == 0) A[i][j] = j < i ? Bt[i] * dec * acc[e] : 0.0f; else P[i][j] = dec * acc[e];
-      }
-    }
-    if (wave == 3) { for (int i = lane; i < 32 * 32; i += 64) { A[i >> 5][32 + (i & 31)] = 0.0f; P[i >> 5][32 + (i & 31)] = 0.0f; } }     // upper-right tiles
-    // ---- K S_0 (waves 0,1) and Q S_0 (waves 2,3): 64x32x128, row tile = wave & 1
-    floatx16 acc1 = {0};
-    {
-      const int ti = wave & 1; const float* arow = wave < 2 ? Ks[32 * ti + r] : Qs[32 * ti + r];
-      for (int k0 = 0; k0 < DK; k0 += 8) {
-        float4 a4 = *(const float4*)(arow + k0 + 4 * kk); const int kb = k0 + 4 * kk;
-        acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.x, S[kb][r], acc1, 0, 0, 0); acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.y, S[kb + 1][r], acc1, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.z, S[kb + 2][r], acc1, 0, 0, 0); acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a4.w, S[kb + 3][r], acc1, 0, 0, 0);
-      }
+  for (int u = 0; u < 5; ++u) {
+    const int job = wave * 5 + u, which = job >= 10 ? 1 : 0, ix = job - 10 * which, ti = ix >= 6 ? 3 : (ix >= 3 ? 2 : (ix >= 1 ? 1 : 0)), tj = ix - ti * (ti + 1) / 2;
+    const float* ar = which ? &Qs[16 * ti + r][4 * q] : &Ks[16 * ti + r][4 * q]; const float* br = &Ks[16 * tj + r][4 * q];
+    v4f_ acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        int i = 32 * ti + 8 * (e >> 2) + 4 * kk + (e & 3); float eL = expf(L[i]);
-        if (wave < 2) D[i][r] = Bt[i] * (vc[(size_t)i * ch + r] - eL * acc1[e]);      // B = beta (v - e^{L} K S_0)
-        else acc1[e] = eL * acc1[e];                                                 // O1 = e^{L} Q S_0, stays in registers
-      }
-    }
-    __syncthreads();
-    // ---- forward substitution (I + A) Delta = B, column by column of A: once Delta_j is final every later row takes its
-    // term, all 256 threads at work; an element still receives its terms in ascending j, as a row-by-row solve would give it
-    // The 32 columns of Delta are independent: wave w solves columns 8w .. 8w+7 with eight lanes per column (lane t of a column
-    // takes the rows j+1+t, j+1+t+8, ..), and a wave's shared-memory operations execute in order, so the 63 steps need no
-    // workgroup barrier.
-    {
-      const int c = 8 * wave + (lane & 7), tr = lane >> 3;
-      for (int j = 0; j < C - 1; ++j) {
-        const float dj = D[j][c];
-        for (int i = j + 1 + tr; i < C; i += 8) D[i][c] -= A[i][j] * dj;
-        __builtin_amdgcn_wave_barrier();
-      }
-    }
-    __syncthreads();
-    // ---- O = O1 + P Delta (waves 2,3): 64x32x64
-    if (wave >= 2) {
-      const int ti = wave & 1;
-      for (int k0 = 0; k0 < C; k0 += 2) acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(P[32 * ti + r][k0 + kk], D[k0 + kk][r], acc1, 0, 0, 0);
+    for (int k0 = 0; k0 < DK; k0 += 16) acc = mac16(*(const float4*)(ar + k0), *(const float4*)(br + k0), acc);
 #pragma unroll
-      for (int e = 0; e < 16; ++e) { int i = 32 * ti + 8 * (e >> 2) + 4 * kk + (e & 3); oraw[(size_t)(t0 + i) * w + (size_t)h * p.dv + cb * 32 + r] = acc1[e]; }
-    }
-    // ---- S_C = e^{L_C} S_0 + (e^{L_C-L_j} k_j)^T Delta: 128x32x64, row tile = wave
-    {
-      floatx16 acc2; const float eLC = expf(L[C - 1]);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc2[e] = eLC * S[32 * wave + 8 * (e >> 2) + 4 * kk + (e & 3)][r];
-      for (int k0 = 0; k0 < C; k0 += 2) { int j = k0 + kk; float a = Ks[j][32 * wave + r] * expf(L[C - 1] - L[j]); acc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a, D[j][r], acc2, 0, 0, 0); }
-      __syncthreads();                                                        // every wave has read the old S
-#pragma unroll
-      for (int e = 0; e < 16; ++e) S[32 * wave + 8 * (e >> 2) + 4 * kk + (e & 3)][r] = acc2[e];
+    for (int e = 0; e < 4; ++e) {
+      const int i = 16 * ti + 4 * q + e, j = 16 * tj + r; const float dc = j <= i ? expf((float)(L[i] - L[j])) : 0.0f;
+      if (which) P[(((size_t)ck * p.nv + h) * C + i) * C + j] = dc * acc[e];
+      else { const float a = j < i ? Bt[i] * dc * acc[e] : 0.0f; A[i][j] = ti == tj ? a : -a; }
     }
   }
   __syncthreads();
-  for (int i = tid; i < DK * 32; i += 256) sout[(size_t)(i >> 5) * p.dv + (i & 31)] = S[i >> 5][i & 31];
-}
-
-// grid (T, nv), dv threads: out = rms_inplace(o, norm) * sigmoid(z)
-__global__ __launch_bounds__(128) void k_gdnp_norm(GdnDev p, const float* __restrict__ proj, int stride, const float* __restrict__ oraw, float* __restrict__ out) {
-  __shared__ float red[2];
-  const int ti = blockIdx.x, h = blockIdx.y, j = threadIdx.x; const int ch = 2 * p.nk * p.dk + p.nv * p.dv, w = p.nv * p.dv;
-  float o = oraw[(size_t)ti * w + (size_t)h * p.dv + j], ss = o * o;
+  // the diagonal blocks' inverses, a wave each, a column a lane: x_i = delta_ic - sum_{k<i} A_ik x_k
+  if (lane < 16) {
+    float x[16];
 #pragma unroll
-  for (int d = 32; d > 0; d >>= 1) ss += __shfl_xor(ss, d);
-  if ((j & 63) == 0) red[j >> 6] = ss;
+    for (int i = 0; i < 16; ++i) {
+      float s = i == lane ? 1.0f : 0.0f;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) if (k < i) s = fmaf(-A[16 * wave + i][16 * wave + k], x[k], s);
+      x[i] = s; Ti[wave][i][lane] = s;
+    }
+  }
   __syncthreads();
-  float sc = 1.0f / sqrtf((red[0] + red[1]) / (float)p.dv + p.eps);
-  out[(size_t)ti * w + (size_t)h * p.dv + j] = (o * (sc * p.norm_w[j])) * p_sigm(proj[(size_t)ti * stride + ch + (size_t)h * p.dv + j]);
+  // W and U by block rows: D_i = T_ii (B_i - sum_{k<i} A_ik D_k); a wave four column tiles of [W | U] at a time
+#pragma unroll 1
+  for (int u = 0; u < 4; ++u) {
+    const int ct = 4 * wave + u, col = (ct & 7) * 16 + r; const bool is_w = ct < 8;
+    v4f_ D[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v4f_ acc;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { const int row = 16 * i + 4 * q + e; acc[e] = is_w ? Bt[row] * eL[row] * Ks[row][col] : Bt[row] * vc[(size_t)row * ch + col]; }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) if (k < i) acc = mac16(*(const float4*)&A[16 * i + r][16 * k + 4 * q], as4(D[k]), acc);
+      const v4f_ z = {0.0f, 0.0f, 0.0f, 0.0f};
+      D[i] = mac16(*(const float4*)&Ti[i][r][4 * q], as4(acc), z);
+      float* o = (is_w ? W : U) + (((size_t)ck * p.nv + h) * C + 16 * i + 4 * q) * DK + col;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[(size_t)e * DK] = D[i][e];
+    }
+  }
 }
 
-// T must be a multiple of 64.  scratch: co [T][ch], logg [T][nv], beta [T][nv], oraw [T][nv*dv].
-int pyre_gdn_prefill_launch(pyre_ctx* ctx, const GdnDev& g, const float* proj, int stride, int T, const float* conv_in, float* conv_out,
-                            const float* ssm_in, float* ssm_out, float* co, float* logg, float* beta, float* oraw, float* out) {
-  if (g.dk != 128 || g.dv != 128) return pyre_fail(ctx, PYRE_E_SHAPE, "gdn prefill: head dims %dx%d unsupported (128x128 only)", g.dk, g.dv);
-  if (T < 64 || T % 64) return pyre_fail(ctx, PYRE_E_ARG, "gdn prefill: %d tokens is not a positive multiple of the chunk size 64", T);
-  const int ch = 2 * g.nk * g.dk + g.nv * g.dv;
-  { ProfScope ps(ctx, "gdn_prefill_conv", 8.0 * T * ch); hipLaunchKernelGGL(k_gdnp_conv, dim3((ch + 255) / 256, T), dim3(256), 0, ctx->stream, proj, stride, T, ch, g.conv_k, g.conv_w, conv_in, co, conv_out); } PYRE_CHECK_LAUNCH(ctx);
-  { ProfScope ps(ctx, "gdn_prefill_prep", 16.0 * T * g.nk * g.dk); hipLaunchKernelGGL(k_gdnp_prep, dim3(T, g.nk + 1), dim3(128), 0, ctx->stream, g, proj, stride, co, logg, beta); } PYRE_CHECK_LAUNCH(ctx);
-  { ProfScope ps(ctx, "gdn_prefill_chunk", 8.0 * g.nv * g.dk * g.dv + 4.0 * T * (ch + g.nv * g.dv));
-    hipLaunchKernelGGL((k_gdnp_chunk<128, 64>), dim3(g.nv, g.dv / 32), dim3(256), 0, ctx->stream, g, co, logg, beta, T / 64, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
-  { ProfScope ps(ctx, "gdn_prefill_norm", 12.0 * T * g.nv * g.dv); hipLaunchKernelGGL(k_gdnp_norm, dim3(T, g.nv), dim3(128), 0, ctx->stream, g, proj, stride, oraw, out); } PYRE_CHECK_LAUNCH(ctx);
+// grid (nv, dv / 16), 4 waves: sixteen columns of a head's state through all chunks.  The state lies in shared memory transposed, so
+// that four consecutive rows of a column -- what a lane supplies to four steps of the product and receives from it -- are one
+// 16-byte access.  Per chunk: W S_0 and Q S_0 (a row tile a wave) | P Delta, S update (two row tiles a wave).
+__global__ __launch_bounds__(256) void k_gdnc_scan(GdnDev p, const float* __restrict__ co, const float* __restrict__ kt, const float* __restrict__ W, const float* __restrict__ U, const float* __restrict__ P, const float* __restrict__ dec,
+                                                   int nch, int T, const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
+  __shared__ __align__(16) float St[16][DK + 4], Dt[16][C + 4], Dd[16][C + 4];          // S, Delta, Delta x e^{L_C-L_j}: [column][row]
+  const int h = blockIdx.x, cb = blockIdx.y * 16, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, r = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv, w = p.nv * p.dv;
+  const float* sin_ = ssm_in + (size_t)h * DK * p.dv + cb; float* sout = ssm_out + (size_t)h * DK * p.dv + cb;
+  for (int i = tid; i < DK * 16; i += 256) St[i & 15][i >> 4] = sin_[(size_t)(i >> 4) * p.dv + (i & 15)];
+  float4 wf[8], qf[8]; float uf[4];
+  auto fetch = [&](int c) {
+    const float* wr = W + (((size_t)c * p.nv + h) * C + 16 * wave + r) * DK + 4 * q; const float* qr = co + (size_t)(c * C + 16 * wave + r) * ch + (size_t)kh * DK + 4 * q;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) { wf[k] = *(const float4*)(wr + 16 * k); qf[k] = *(const float4*)(qr + 16 * k); }
+    const float* ur = U + (((size_t)c * p.nv + h) * C + 16 * wave + 4 * q) * DK + cb + r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) uf[e] = ur[(size_t)e * DK];
+  };
+  fetch(0);
+  __syncthreads();
+  for (int c = 0; c < nch; ++c) {
+    const float* pr = P + (((size_t)c * p.nv + h) * C + 16 * wave + r) * C + 4 * q; const float* kr = kt + (((size_t)c * p.nk + kh) * DK + 32 * wave + r) * C + 4 * q; const float* dc = dec + ((size_t)c * p.nv + h) * 2 * C;
+    float4 pf[4], kf[2][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) { pf[j] = j <= wave ? *(const float4*)(pr + 16 * j) : make_float4(0.0f, 0.0f, 0.0f, 0.0f); kf[0][j] = *(const float4*)(kr + 16 * j); kf[1][j] = *(const float4*)(kr + 16 * C + 16 * j); }
+    const float4 e1 = *(const float4*)(dc + 16 * wave + 4 * q), e2 = *(const float4*)(dc + C + 16 * wave + 4 * q); const float eC = dc[C - 1];
+    v4f_ aw = {0.0f, 0.0f, 0.0f, 0.0f}, aq = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) { const float4 s = *(const float4*)&St[r][16 * k + 4 * q]; aw = mac16(wf[k], s, aw); aq = mac16(qf[k], s, aq); }
+    float4 d; d.x = uf[0] - aw[0]; d.y = uf[1] - aw[1]; d.z = uf[2] - aw[2]; d.w = uf[3] - aw[3];
+    *(float4*)&Dt[r][16 * wave + 4 * q] = d;
+    *(float4*)&Dd[r][16 * wave + 4 * q] = make_float4(d.x * e2.x, d.y * e2.y, d.z * e2.z, d.w * e2.w);
+    aq[0] *= e1.x; aq[1] *= e1.y; aq[2] *= e1.z; aq[3] *= e1.w;
+    lds_barrier();
+    if (c + 1 < nch) fetch(c + 1);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {          // the state first: the next chunk waits for it
+      float4* sp = (float4*)&St[r][32 * wave + 16 * u + 4 * q]; const float4 s = *sp;
+      v4f_ a = {eC * s.x, eC * s.y, eC * s.z, eC * s.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a = mac16(kf[u][j], *(const float4*)&Dd[r][16 * j + 4 * q], a);
+      *sp = as4(a);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) if (j <= wave) aq = mac16(pf[j], *(const float4*)&Dt[r][16 * j + 4 * q], aq);
+    const int ti = c * C + 16 * wave + 4 * q;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) if (ti + e < T) oraw[(size_t)(ti + e) * w + (size_t)h * p.dv + cb + r] = aq[e];
+    lds_barrier();
+  }
+  for (int i = tid; i < DK * 16; i += 256) sout[(size_t)(i >> 4) * p.dv + (i & 15)] = St[i & 15][i >> 4];
+}
+
+}  // namespace
+
+size_t pyre_gdn_chunk_bytes(const GdnDev& g, int T) {
+  const size_t nch = ((size_t)T + C - 1) / C, ch = 2 * (size_t)g.nk * g.dk + (size_t)g.nv * g.dv;
+  return 6 * 256 + 4 * (nch * C * ch + nch * g.nk * DK * C + nch * g.nv * (2 * (size_t)C * DK + (size_t)C * C + 2 * C));
+}
+void pyre_gdn_chunk_carve(const GdnDev& g, int T, void* base, GdnChunk* b) {
+  const size_t nch = ((size_t)T + C - 1) / C, ch = 2 * (size_t)g.nk * g.dk + (size_t)g.nv * g.dv;
+  uint8_t* p = (uint8_t*)base; auto take = [&](size_t n) { void* r = p; p += (n * 4 + 255) & ~(size_t)255; return (float*)r; };
+  b->co = take(nch * C * ch); b->kt = take(nch * g.nk * DK * C); b->w = take(nch * g.nv * C * DK); b->u = take(nch * g.nv * C * DK); b->p = take(nch * g.nv * C * C); b->dec = take(nch * g.nv * 2 * C);
+}
+int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int stride, int T, const float* conv_in, float* conv_out, const float* ssm_in, float* ssm_out, float* oraw) {
+  if (g.dk != 128 || g.dv != 128) return pyre_fail(ctx, PYRE_E_SHAPE, "gdn prompt: head dims %dx%d unsupported (128x128 only)", g.dk, g.dv);
+  if (T < 1 || g.conv_k < 1 || g.conv_k > 8) return pyre_fail(ctx, PYRE_E_ARG, "gdn prompt: %d tokens, %d taps", T, g.conv_k);
+  const int ch = 2 * g.nk * g.dk + g.nv * g.dv, nch = (T + C - 1) / C, Tp = nch * C;
+  { ProfScope ps(ctx, "gdn_prompt_conv", 8.0 * T * ch);
+    if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, b.kt);
+    else hipLaunchKernelGGL(k_gdnc_conv<0>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, b.kt); } PYRE_CHECK_LAUNCH(ctx);
+  { ProfScope ps(ctx, "gdn_prompt_chunk", 4.0 * T * (ch + g.nv * (2.0 * DK + C)));
+    hipLaunchKernelGGL(k_gdnc_chunk, dim3(nch, g.nv), dim3(256), 0, ctx->stream, g, b.co, proj, stride, T, b.w, b.u, b.p, b.dec); } PYRE_CHECK_LAUNCH(ctx);
+  { ProfScope ps(ctx, "gdn_prompt_scan", 8.0 * g.nv * g.dk * g.dv + 4.0 * T * g.nv * (4.0 * DK + C));
+    hipLaunchKernelGGL(k_gdnc_scan, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, b.kt, b.w, b.u, b.p, b.dec, nch, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
   return PYRE_OK;
 }

@@ -23,7 +23,8 @@ struct Layer {
 
 }  // namespace
 
-struct PromptPipe; void prompt_pipe_free(PromptPipe* P); size_t prompt_pipe_blocks(const PromptPipe* P);
+struct PromptPipe; void prompt_pipe_free(PromptPipe* P);
+struct PromptBlk; void prompt_blk_free(PromptBlk* B); size_t prompt_blk_count(const PromptBlk* B);
 
 struct pyre_model {
   pyre_ctx* ctx = nullptr; pyre_model_cfg c{};
@@ -41,6 +42,7 @@ struct pyre_model {
   float* gdn_sq = nullptr;      // [2][8][nv][4]: per token, head and quarter the inverse power of two of the Gated DeltaNet operand and the quarter's sum of squares (PyreAop::sq)
   float* aop_inv = nullptr;     // [super-blocks][8]: the inverse of the power of two the hyper-connection mix scaled each token of that operand by
   PromptPipe* pipe = nullptr;      // further window workspaces and streams for a long prompt (prompt_pipe), made at the first one
+  PromptBlk* blk = nullptr;        // the workspace of a prompt taken layer by layer (run_block), made at the first one
 };
 
 struct pyre_state {
@@ -288,12 +290,12 @@ int pyre_model_create(pyre_ctx* ctx, const pyre_model_cfg* cfg, const pyre_tenso
 
 void pyre_model_destroy(pyre_model* m) {
   if (!m) return; (void)hipSetDevice(m->ctx->device); (void)hipStreamSynchronize(m->ctx->stream);
-  prompt_pipe_free(m->pipe);
+  prompt_pipe_free(m->pipe); prompt_blk_free(m->blk);
   for (auto q : m->owned) pyre_qmat_destroy(q); for (auto b : m->bufs) (void)hipFree(b); if (m->work) (void)hipFree(m->work); if (m->toks) (void)hipFree(m->toks);
   delete m;
 }
 size_t pyre_model_weight_bytes_per_token(const pyre_model* m) { return m ? m->token_weight_bytes : 0; }
-size_t pyre_model_prompt_blocks(const pyre_model* m) { return m && m->pipe ? prompt_pipe_blocks(m->pipe) : 0; }
+size_t pyre_model_prompt_blocks(const pyre_model* m) { return m && m->blk ? prompt_blk_count(m->blk) : 0; }
 
 int pyre_state_create(pyre_ctx* ctx, const pyre_model* m, int max_ctx, pyre_state** out) {
   if (!ctx || !m || !out || max_ctx < 1) return pyre_fail(ctx, PYRE_E_ARG, "pyre_state_create: bad argument");
@@ -453,15 +455,7 @@ struct PromptPipe {
   std::vector<hipEvent_t> done;                // [set] end of the set's last window
   hipEvent_t start = nullptr;
   uint32_t* ids = nullptr; size_t ids_cap = 0; // the call's token ids on the device
-  // blocks of windows taken layer by layer with the FFN of all their tokens grouped by expert (prompt_block_get)
-  std::vector<pyre_model*> wmdl;               // a window workspace per window of a block
-  void* blk_mem = nullptr; MoeBlk blk[2]{}; int blk_nsl = 0, blk_r64 = 0;          // two blocks in flight: one's FFN beside the other's windows
-  hipEvent_t moe_done[2] = {nullptr, nullptr}; std::vector<hipEvent_t> front_done[2]; size_t blocks_done = 0;
-  pyre_ctx* moe_ctx = nullptr;                 // the stream of the blocks' FFN launches
-  size_t win_stride = 0;                       // bytes between the workspaces of consecutive windows of a block
-  void* qmem = nullptr; size_t q_stride = 0, q_off[2] = {0, 0};      // per window of a block: the rotated queries (f32, f16 halves, scales) of an attention layer, kept from the cache write to the pass over the cache
 };
-size_t prompt_pipe_blocks(const PromptPipe* P) { return P->blocks_done; }
 static int prompt_streams() { static const int k = [] { const char* e = getenv("PYRE_PROMPT_STREAMS"); int v = e && *e ? atoi(e) : 3; return v < 1 ? 1 : (v > 4 ? 4 : v); }(); return k; }
 void prompt_pipe_free(PromptPipe* P) {
   if (!P) return;
@@ -471,12 +465,6 @@ void prompt_pipe_free(PromptPipe* P) {
   for (auto e : P->done) if (e) (void)hipEventDestroy(e);
   if (P->start) (void)hipEventDestroy(P->start);
   if (P->ids) (void)hipFree(P->ids);
-  for (auto* mc : P->wmdl) if (mc) { if (mc->work) (void)hipFree(mc->work); delete mc; }
-  if (P->blk_mem) (void)hipFree(P->blk_mem);
-  for (auto e : P->moe_done) if (e) (void)hipEventDestroy(e);
-  for (auto& v : P->front_done) for (auto e : v) if (e) (void)hipEventDestroy(e);
-  if (P->moe_ctx) pyre_ctx_destroy(P->moe_ctx);
-  if (P->qmem) (void)hipFree(P->qmem);
   delete P;
 }
 static int prompt_pipe_get(pyre_ctx* ctx, const pyre_model* m, PromptPipe** out) {
@@ -487,7 +475,7 @@ static int prompt_pipe_get(pyre_ctx* ctx, const pyre_model* m, PromptPipe** out)
   for (int i = 1; i < k; ++i) {
     pyre_ctx* cx = nullptr; int rc = pyre_ctx_create(ctx->device, &cx); if (rc) return pyre_fail(ctx, rc, "prompt streams: %s", pyre_last_error(nullptr));
     P->ctx.push_back(cx);
-    pyre_model* mc = new pyre_model(*m); mc->ctx = cx; mc->owned.clear(); mc->bufs.clear(); mc->work = nullptr; mc->toks = nullptr; mc->toks_cap = 0; mc->pipe = nullptr;
+    pyre_model* mc = new pyre_model(*m); mc->ctx = cx; mc->owned.clear(); mc->bufs.clear(); mc->work = nullptr; mc->toks = nullptr; mc->toks_cap = 0; mc->pipe = nullptr; mc->blk = nullptr;
     P->mdl.push_back(mc);
     int kmax = 0; rc = model_alloc_work(cx, mc, &kmax);
     if (!rc) { uint4* op; float* ainv; rc = pyre_gemm_m_scratch(cx, (kmax + 255) / 256 * 256, &op, &ainv); }
@@ -520,65 +508,126 @@ static int prompt_pipe_state(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, 
   return PYRE_OK;
 }
 
-// ---- a long prompt in blocks of windows, layer by layer ---------------------------------------------------------------------
-// Windows of eight tokens share nothing in the FFN (eight tokens pick 74 of 512 experts), which makes the expert products
-// the largest part of a prompt window.  A block of up to PROMPT_BLOCK_WINDOWS windows is therefore taken layer by layer: every
-// window's part of the layer up to the FFN mix (on the prompt's streams, the layer's state passing from window to window as
-// before), then the FFN of all of the block's tokens in one set of launches with the tokens grouped by expert, on the
-// matrix cores (pyre_moe_block_launch), whose group sums the windows' next mixes read.  Everything but the FFN is the
-// windows' kernels and arithmetic; the FFN's products are those of the matrix-core GEMM (f16 halves of the activations
-// instead of fixed-point digits): equal to rounding, not bit for bit.  For models whose every layer qualifies
-// (prompt_block_ok); the call's last tokens (the window whose logits are read, the rows a drafter keeps) take the windows'
-// path.  PYRE_PROMPT_BLOCK=0 switches it off.
-static int prompt_block_windows() { static const int k = [] { const char* e = getenv("PYRE_PROMPT_BLOCK_WINDOWS"); int v = e && *e ? atoi(e) : 128; return v < 8 ? 8 : (v > 128 ? 128 : v); }(); return k; }      // the most windows a block has (read once)
-#define PROMPT_BLOCK_WINDOWS prompt_block_windows()
-#define PROMPT_BLOCK_MIN 8
+// ---- a long prompt layer by layer ---------------------------------------------------------------------------------------------
+// Windows of eight tokens share nothing but what fits beside each other on the chip: every window decodes every weight again, and
+// its FFN's 74 of 512 experts.  A call of 72 tokens or more is therefore taken in blocks of up to 2048 tokens, layer by layer, a
+// launch a step for all of a block's tokens: the mixes and projections (prompt.hip), the Gated DeltaNet in chunks of 64
+// (gdn_prefill.hip), the attention (attn_prompt.hip), the FFN grouped by expert (moe.hip).  Against windows everything but
+// the recurrence's and the attention's order of sums and the FFN's operand form is the same arithmetic; logits agree to
+// rounding.  Blocks are cut at multiples of 128 tokens from the call's start, so that neither the chunks of the recurrence
+// nor the tiles of the attention -- hence not a bit of a token -- depend on the cutting.
+// For models whose every layer qualifies (prompt_block_ok); PYRE_PROMPT_BLOCK=0 switches it off, PYRE_PROMPT_PAIRS=0 halves the blocks.
+#define PROMPT_BLOCK_MIN 72
+#define PROMPT_BLOCK_MAX 2048
 static bool fuse_aop_on() { const char* e = getenv("PYRE_AOP_SPLIT"); return !(e && *e && atoi(e) != 0); }
 static bool prompt_block_ok(const pyre_model* m) {
   if (!prompt_block_env()) return false;
-  { const char* r = getenv("PYRE_ROUTER_RIDES"); if (r && *r && atoi(r) == 0) return false; }
-  { const char* r = getenv("PYRE_MOE_GROUPS"); if (r && *r && atoi(r) == 0) return false; }
   const pyre_model_cfg& c = m->c;
-  if (m->n_ple > 0 || c.top_k > PYRE_MOE_KMAX || c.d % 256 || !fuse_aop_on()) return false;
-  for (int il = 0; il < c.n_layers; ++il) { const Layer& L = m->layers[il];
-    if (!pyre_moe_block_ok(L.moe) || !pyre_hc_route_ok(L.hcf, L.moe.router) || !pyre_hc_aop_ok(L.hcf) || L.hca.di.fmt != FMT_IQ3_S || L.moe.router.tiles != m->layers[0].moe.router.tiles ||
-        L.moe.ff != m->layers[0].moe.ff || L.moe.sf != m->layers[0].moe.sf || L.moe.top_k != m->layers[0].moe.top_k || L.moe.n_exp != m->layers[0].moe.n_exp) return false; }
+  if (m->n_ple > 0 || c.top_k > PYRE_MOE_KMAX || c.d % 256 || c.conv_k < 2 || c.conv_k > 8 || !pyre_blk_mix_ok(m->head)) return false;
+  for (int il = 0; il < c.n_layers; ++il) { const Layer& L = m->layers[il]; const MoeDev& m0 = m->layers[0].moe;
+    if (!pyre_moe_block_ok(L.moe) || (L.moe.router.fmt != FMT_BF16 && L.moe.router.fmt != FMT_F32) || L.moe.router.U != c.d / 64 || L.moe.router.tiles != m0.router.tiles || L.moe.ff != m0.ff || L.moe.sf != m0.sf || L.moe.top_k != m0.top_k || L.moe.n_exp != m0.n_exp ||
+        !pyre_blk_mix_ok(L.hca) || !pyre_blk_mix_ok(L.hcf) || L.proj.fmt != FMT_IQ3_S_M || L.outp.fmt != FMT_IQ3_S_M || L.proj.cols % 256 || L.outp.cols % 256 || L.outp.rows != c.d || (!L.full && !L.gdn_ainv)) return false; }
   return true;
 }
-static int prompt_block_get(pyre_ctx* ctx, const pyre_model* m, PromptPipe* P) {
-  if (!P->wmdl.empty()) return PYRE_OK;
-  const pyre_model_cfg& c = m->c; const int NB = PROMPT_BLOCK_WINDOWS, d = c.d, K = (int)P->ctx.size() + 1;
-  const MoeDev& m0 = m->layers[0].moe;
-  const int nsl = d / 64, r64 = m0.router.tiles * 64;
-  // the windows' workspaces of both blocks in flight in one piece, a workspace every ws bytes: what a launch does for one
-  // window it can do for the next ones at the same addresses + ws; the FFN's own scratch once (its launches share a stream)
-  size_t aop_b = 0; const size_t ws = model_work_layout(const_cast<pyre_model*>(m), nullptr, nullptr, &aop_b), mb = al256(pyre_moe_block_bytes(m0, NB * 8));
-  PYRE_HIP(ctx, hipMalloc(&P->blk_mem, 2 * (size_t)NB * ws + mb + 256));
-  PYRE_HIP(ctx, hipMemsetAsync(P->blk_mem, 0, 2 * (size_t)NB * ws, ctx->stream));
-  uint8_t* p = (uint8_t*)P->blk_mem;
-  for (int w = 0; w < 2; ++w) for (int j = 0; j < NB; ++j) {
-    pyre_model* mc = new pyre_model(*m); mc->owned.clear(); mc->bufs.clear(); mc->work = nullptr; mc->toks = nullptr; mc->toks_cap = 0; mc->pipe = nullptr;
-    P->wmdl.push_back(mc);
-    (void)model_work_layout(mc, p + ((size_t)w * NB + j) * ws, nullptr, nullptr);
+struct PromptBlk {
+  pyre_ctx* ctx = nullptr; void* mem = nullptr; int T_max = 0; size_t blocks = 0;      // room for T_max tokens a block; blocks: pyre_model_prompt_blocks
+  float *emb = nullptr, *x = nullptr, *mixed = nullptr, *inj_a = nullptr, *inj_f = nullptr, *proj = nullptr, *o = nullptr, *core = nullptr, *inv = nullptr; uint4* op = nullptr; uint32_t* ids = nullptr;
+  BlkMix mix{}; MoeBlk moe{}; GdnChunk gdn{}; uint16_t* qh = nullptr; float* qsc = nullptr;
+  void* att = nullptr; size_t att_bytes = 0;             // the cache's fragments (grows with the context)
+};
+size_t prompt_blk_count(const PromptBlk* B) { return B->blocks; }
+void prompt_blk_free(PromptBlk* B) {
+  if (!B) return;
+  (void)hipStreamSynchronize(B->ctx->stream);
+  if (B->mem) (void)hipFree(B->mem);
+  if (B->att) (void)hipFree(B->att);
+  delete B;
+}
+// the workspace for blocks of T tokens and a context of n positions: kept by the model, grown when a longer call comes
+static int prompt_blk_get(pyre_ctx* ctx, const pyre_model* m, int T, int n, PromptBlk** out) {
+  pyre_model* mm = const_cast<pyre_model*>(m); const pyre_model_cfg& c = m->c;
+  if (!mm->blk) { mm->blk = new PromptBlk(); mm->blk->ctx = ctx; }
+  PromptBlk* B = mm->blk; *out = B;
+  T = (T + 127) / 128 * 128;
+  if (B->T_max < T) {
+    if (B->mem) { PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); (void)hipFree(B->mem); B->mem = nullptr; B->T_max = 0; }
+    T = T <= 512 ? 512 : PROMPT_BLOCK_MAX;
+    const MoeDev& m0 = m->layers[0].moe; const Layer* lin = nullptr; for (const Layer& L : m->layers) if (!L.full) lin = &L;
+    const size_t t = T, d = c.d, nq = (size_t)c.n_head * c.hd, cmax = std::max((size_t)c.lin_nv * c.lin_dv, nq), omax = std::max(d, cmax), pmax = std::max(m->pw_lin, m->pw_attn);
+    HcDev hmax = m->layers[0].hca;
+    const size_t rp = t * (d / 64) * m0.router.tiles * 64;
+    for (int pass = 0; pass < 2; ++pass) {
+      uint8_t* p = (uint8_t*)B->mem; size_t sum = 0;
+      auto take = [&](size_t bytes) { void* r = p; bytes = al256(bytes); if (pass) p += bytes; sum += bytes; return r; };
+      B->emb = (float*)take(4 * t * d); B->x = (float*)take(4 * t * c.hc * d); B->mixed = (float*)take(4 * t * d); B->inj_a = (float*)take(4 * t * c.hc); B->inj_f = (float*)take(4 * t * c.hc);
+      B->proj = (float*)take(4 * t * pmax); B->o = (float*)take(4 * t * d); B->core = (float*)take(4 * t * cmax); B->op = (uint4*)take(4 * t * omax); B->inv = (float*)take(4 * t * (omax / 256)); B->ids = (uint32_t*)take(4 * t);
+      void* mx = take(pyre_blk_mix_bytes(hmax, T)); void* mo = take(pyre_moe_block_bytes(m0, T)); void* gd = take(lin ? pyre_gdn_chunk_bytes(lin->gdn, T) : 0);
+      float* rpart = (float*)take(4 * rp); float* parts = (float*)take(4 * PYRE_MOE_GROUPS * t * d);
+      B->qh = (uint16_t*)take(2 * 2 * t * nq); B->qsc = (float*)take(4 * t * c.n_head);
+      if (!pass) { PYRE_HIP(ctx, hipMalloc(&B->mem, sum + 256)); continue; }
+      pyre_blk_mix_carve(hmax, T, mx, &B->mix); pyre_moe_block_carve(m0, T, mo, &B->moe); if (lin) pyre_gdn_chunk_carve(lin->gdn, T, gd, &B->gdn);
+      B->moe.x = B->mixed; B->moe.rpart = rpart; B->moe.parts = parts; B->moe.wr = 8 * (d / 64) * m0.router.tiles * 64;
+    }
+    PYRE_HIP(ctx, hipMemsetAsync(B->mem, 0, 4096, ctx->stream));
+    { int rc = pyre_moe_block_zero_rows(ctx, m0, B->moe, T); if (rc) return rc; }
+    B->T_max = T;
   }
-  pyre_moe_block_carve(m0, NB * 8, p + 2 * (size_t)NB * ws, &P->blk[0]);
-  P->blk[1] = P->blk[0];
-  for (int w = 0; w < 2; ++w) { const pyre_model* f = P->wmdl[(size_t)w * NB]; P->blk[w].x = f->mixed; P->blk[w].rpart = f->rpart; P->blk[w].parts = f->mw.parts; P->blk[w].ws = ws / 4; }
-  P->blk_nsl = nsl; P->blk_r64 = r64; P->win_stride = ws;
-  { int rc = pyre_moe_block_zero_rows(ctx, m0, P->blk[0], NB * 8); if (rc) return rc; }
-  if (!m->has_idx) {      // (with a sparse indexer the selection and the pass stay together in the chain)
-    const size_t nq = (size_t)8 * c.n_head * c.hd;
-    P->q_off[0] = al256(4 * nq); P->q_off[1] = P->q_off[0] + al256(2 * 2 * nq); P->q_stride = P->q_off[1] + al256(4 * 8 * (size_t)c.n_head);
-    PYRE_HIP(ctx, hipMalloc(&P->qmem, 2 * (size_t)NB * P->q_stride));
+  if (m->n_attn > 0 && !m->has_idx) {
+    AttnDev a0{nullptr, nullptr, nullptr, c.n_head, c.n_kv, c.hd, c.n_rot, c.kv_bits, c.kv_recent, c.eps};
+    const size_t need = pyre_attn_prompt_bytes(a0, std::max(0, n - B->T_max), B->T_max);
+    if (B->att_bytes < need) {
+      if (B->att) { PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); (void)hipFree(B->att); B->att = nullptr; B->att_bytes = 0; }
+      PYRE_HIP(ctx, hipMalloc(&B->att, need + need / 4)); B->att_bytes = need + need / 4;
+    }
   }
-  { int rc = pyre_ctx_create(ctx->device, &P->moe_ctx); if (rc) return pyre_fail(ctx, rc, "prompt blocks: %s", pyre_last_error(nullptr)); }
-  for (int w = 0; w < 2; ++w) {
-    PYRE_HIP(ctx, hipEventCreateWithFlags(&P->moe_done[w], hipEventDisableTiming));
-    P->front_done[w].resize(K, nullptr);
-    for (auto& e : P->front_done[w]) PYRE_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  }
-  PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return PYRE_OK;
+}
+// T tokens (ids on the host) behind the state's length; head: the last token's logits to m->logits
+static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBlk* B, const uint32_t* ids, int T, bool head) {
+  const pyre_model_cfg& c = m->c; const int d = c.d, hc = c.hc, start = s->len, G = (T + 7) / 8; int rc;
+  PYRE_HIP(ctx, hipMemcpyAsync(B->ids, ids, (size_t)T * 4, hipMemcpyHostToDevice, ctx->stream));
+  if (s->tokens_dev) PYRE_HIP(ctx, hipMemcpyAsync(s->tokens_dev + start, B->ids, (size_t)T * 4, hipMemcpyDeviceToDevice, ctx->stream));      // (a state with a drafter keeps the history)
+  if ((rc = pyre_row_launch(ctx, m->embd, B->ids, T, B->emb, d))) return rc;
+  const float* xin = B->emb; int in_ss = 0, in_ts = d, np = 0; const float* comb = nullptr; const float* cinj = nullptr;
+  auto gs = [](int cols) { return (size_t)cols * 2; }; auto is = [](int cols) { return cols / 256 * 8; };
+  for (int il = 0; il < c.n_layers; ++il) {
+    const Layer& L = m->layers[il]; const int pw = L.full ? m->pw_attn : m->pw_lin, oc = L.outp.cols;
+    if ((rc = pyre_blk_mix_launch(ctx, L.hca, B->mix, xin, in_ss, in_ts, B->x, T, comb, np, cinj, c.eps, B->mixed, B->inj_a, B->op, gs(d), B->inv, is(d)))) return rc;
+    xin = B->x; in_ss = d; in_ts = hc * d;
+    if ((rc = pyre_blk_gemm_launch(ctx, L.proj, B->op, gs(d), B->inv, is(d), B->proj, pw, T))) return rc;
+    if (L.full) {
+      const int ai = L.mix_index;
+      if (m->has_idx) {          // a sparse indexer selects per window of eight, behind the windows before it
+        for (int i = 0; i < T; i += 8) {
+          const int t = std::min(8, T - i); const float* pj = B->proj + (size_t)i * pw;
+          if ((rc = pyre_qsa_launch(ctx, L.qsa, L.attn, s->qsa[ai], s->qw, pj, pw, m->iq_off, start + i, t, nullptr))) return rc;
+          if ((rc = pyre_attn_launch_sel(ctx, L.attn, s->kv[ai], s->aw, pj, pw, start + i, t, &s->packed[ai], B->core + (size_t)i * oc, nullptr, &s->qw))) return rc;
+        }
+      } else {
+        if ((rc = pyre_attn_blk_prep(ctx, L.attn, s->kv[ai], B->proj, pw, start, T, &s->packed[ai], nullptr, B->qh, B->qsc))) return rc;
+        if (pyre_attn_prompt_bytes(L.attn, start, T) > B->att_bytes) return pyre_fail(ctx, PYRE_E_STATE, "forward: attention scratch of %zu bytes is too small", B->att_bytes);
+        if ((rc = pyre_attn_prompt_launch(ctx, L.attn, s->kv[ai], B->qh, B->qsc, B->proj, pw, start, T, B->att, B->core))) return rc;
+      }
+      if ((rc = pyre_blk_op_split_launch(ctx, B->core, oc, T, B->op, gs(oc), B->inv, is(oc)))) return rc;
+      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, is(oc), B->o, d, T))) return rc;
+    } else {
+      const int li = L.mix_index, b = s->cur[li], nb = b ^ 1;
+      if ((rc = pyre_gdn_chunk_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], B->core))) return rc;
+      s->cur[li] = nb;
+      if ((rc = pyre_blk_gdn_out_launch(ctx, B->core, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, L.gdn_up, B->op, gs(oc), nullptr))) return rc;
+      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), L.gdn_ainv, 0, B->o, d, T))) return rc;
+    }
+    if ((rc = pyre_blk_mix_launch(ctx, L.hcf, B->mix, xin, in_ss, in_ts, B->x, T, B->o, 1, B->inj_a, c.eps, B->mixed, B->inj_f, nullptr, 0, nullptr, 0))) return rc;
+    if (il == c.n_layers - 1 && !head) break;          // nobody reads the last layer's FFN
+    if ((rc = pyre_moe_block_launch(ctx, L.moe, B->moe, T, B->T_max, d / 64, L.moe.router.tiles * 64))) return rc;
+    comb = B->moe.parts; np = PYRE_MOE_GROUPS; cinj = B->inj_f;
+  }
+  s->len = start + T;
+  if (!head) return PYRE_OK;
+  const int g = G - 1, tl = T - 8 * g;          // the head of the last group's tokens; the last one's logits
+  if ((rc = pyre_blk_mix_launch(ctx, m->head, B->mix, B->x + (size_t)8 * g * hc * d, d, hc * d, B->x + (size_t)8 * g * hc * d, tl, B->moe.parts + (size_t)g * PYRE_MOE_GROUPS * 8 * d, PYRE_MOE_GROUPS,
+                                B->inj_f + (size_t)8 * g * hc, c.eps, B->mixed, B->inj_a, nullptr, 0, nullptr, 0))) return rc;
+  return pyre_gemv_launch(ctx, m->out, B->mixed + (size_t)(tl - 1) * d, 1, m->logits);
 }
 
 namespace {
@@ -595,12 +644,6 @@ struct WinOpt {
   // a prompt window that shares the GPU with its neighbours (prompt_pipe): its ids, the attention / selection workspace
   // it uses instead of the state's, and per layer the event it waits for (the previous window has left the layer) and records
   const uint32_t* ids_dev = nullptr; const AttnWork* aw = nullptr; const QsaWork* qw = nullptr; const hipEvent_t* wait_ev = nullptr; const hipEvent_t* rec_ev = nullptr;
-  int start = -1;               // the window's first position when the caller keeps the count (a block of windows taken layer by layer); -1: the state's length
-  bool no_len = false;          // ... and the state's length is then advanced by the caller
-  size_t win_stride = 0;        // bytes between this window's workspace and the next window's of its block (0: it stands alone)
-  bool router_apart = false;    // a block's window: the router's K-slice sums come from the block's FFN launch, not from this window's FFN mix
-  bool proj_early = false;      // a block's window: the layer's projection is launched with the mix in front of it (front_pre_proj), a Gated DeltaNet layer's convolution once for the group (front_mid_conv): neither needs the layer's state
-  bool attn_split = false; AttnWork aw_own{};      // a block's window: the attention pass over the cache leaves the chain through the layer's state (front_post_proj runs it); aw_own: the stream's attention workspace with q buffers of this window's own
 };
 
 // rows `from` .. t-1 of the window's final residual streams x [t][w] into the ring at their positions; grid (ceil(w/256), t - from)
@@ -621,10 +664,8 @@ static bool gdn_q_on(const pyre_model* m, const Layer& L) {
   const char* e = getenv("PYRE_GDN_Q");
   return !(e && *e && atoi(e) == 0) && fuse_aop_on() && !L.full && L.outp.fmt == FMT_IQ3_S_M && L.gdn.dv == 128 && L.gdn.dk == 128 && L.outp.cols == L.gdn.nv * 128 && m->gdn_sq != nullptr;
 }
-// One window of t <= 8 tokens as an object, so that a block of prompt windows can be taken layer by layer: begin() (embedding
-// rows, history, n-gram rows), per layer front(il) (everything up to the FFN mix, whose output is the FFN's input) and
-// moe(il) (the FFN; the block path runs pyre_moe_block_launch for all of its windows instead and calls moe_from_block),
-// finish() (bookkeeping, head).  run_window is the four in order.
+// One window of t <= 8 tokens as an object: begin() (embedding rows, history, n-gram rows), per layer front(il) (everything up to
+// the FFN mix, whose output is the FFN's input) and moe(il), finish() (bookkeeping, head).  run_window is the four in order.
 struct WinRun {
   pyre_ctx* ctx; const pyre_model* m; pyre_state* s; int t; WinOpt o;
   int start = 0; bool replay = false;
@@ -638,7 +679,7 @@ struct WinRun {
   bool gdn_fused(const Layer& L) const { return fuse_aop && L.outp.fmt == FMT_IQ3_S_M && L.gdn_ainv != nullptr; }
   int begin() {
     const pyre_model_cfg& c = m->c; const int d = c.d;
-    start = o.start >= 0 ? o.start : s->len; replay = o.step_dev != nullptr;
+    start = s->len; replay = o.step_dev != nullptr;
     if (start + t > s->cap) return pyre_fail(ctx, PYRE_E_STATE, "forward: context %d exceeds the state's capacity %d", start + t, s->cap);
     const uint32_t* ids = o.ids_dev ? o.ids_dev : m->ids;
     int rc = o.from_best ? pyre_pick_launch(ctx, m->best, pyre_gemv_best_count(m->out), m->ids, o.toks_out, &m->embd, m->emb, o.step_dev, s->tokens_dev) : pyre_row_launch(ctx, m->embd, ids, t, m->emb, d); if (rc) return rc;
@@ -671,9 +712,7 @@ struct WinRun {
   // A layer up to its FFN in three parts: the mix in front of the layer's state (pre), what reads and writes that state --
   // projection with its convolution and the recurrence, or projection and attention -- (mid), the output projection and the FFN
   // mix (post).  Only mid follows the previous window's mid; front() is the three in a row with the events around mid.
-  // nz: windows this launch serves (this one and the nz - 1 after it, their workspaces o.win_stride bytes apart); 0: none -- a
-  // launch of an earlier window of the group has served this one, only the bookkeeping is left
-  int front_pre(int il, int nz = 1) {
+  int front_pre(int il) {
     const pyre_model_cfg& c = m->c; const int d = c.d, hc = c.hc; int rc;
     const AopOut aout{m->aop, m->aop_inv, d / 256};
     auto opw = [&](const HcDev& h, const QMatDev& q) -> const AopOut* { return hc_fused(h, q) ? &aout : nullptr; };
@@ -686,116 +725,45 @@ struct WinRun {
     // the mix that produces a matrix-core GEMV's input also leaves it as that GEMV's f16 operand, every token scaled by a power of
     // two (AopOut); the Gated DeltaNet step likewise with a constant of the layer; the attention output goes through the GEMV's
     // own split launch (its magnitude has no bound a single workgroup of the merge could form)
-    if (nz > 0) {
-      ctx->batch_n = nz; ctx->batch_stride = nz > 1 ? o.win_stride : 0;
-      rc = pyre_hc_mix_launch(ctx, L.hca, m->hw, xin, in_ss, in_ts, xout, t, comb_out, comb_moe, comb_inj, c.eps, m->mixed, m->inj_a, nullptr, comb_np, opw(L.hca, L.proj));
-      ctx->batch_n = 1; ctx->batch_stride = 0;
-      if (rc) return rc;
-    }
+    if ((rc = pyre_hc_mix_launch(ctx, L.hca, m->hw, xin, in_ss, in_ts, xout, t, comb_out, comb_moe, comb_inj, c.eps, m->mixed, m->inj_a, nullptr, comb_np, opw(L.hca, L.proj)))) return rc;
     advance(); comb_np = 1;
-    return PYRE_OK;
-  }
-  // whether one launch of layer il's projection / output projection can serve several windows: the operand comes from the
-  // window's own workspace (the mix's, the recurrence's per-quarter form), not through the context's split buffer
-  bool proj_batchable(int il) const { const Layer& L = m->layers[il]; return hc_fused(L.hca, L.proj); }
-  bool outp_batchable(int il) const { const Layer& L = m->layers[il]; return L.outp.fmt == FMT_IQ3_S_M && (L.full ? (o.attn_split && L.outp.cols % 256 == 0) : gdn_q_on(m, L)); }
-  int front_pre_proj(int il, int nz = 1) {          // (proj_early) the layer's projection, without the convolution (nz as in front_pre)
-    const Layer& L = m->layers[il]; if (nz <= 0) return PYRE_OK;
-    const PyreAop aop_hc{(const uint4*)m->aop, m->aop_inv};
-    ctx->batch_n = nz; ctx->batch_stride = nz > 1 ? o.win_stride : 0;
-    const int rc = pyre_gemv_launch(ctx, L.proj, m->mixed, t, m->proj, hc_fused(L.hca, L.proj) ? &aop_hc : nullptr);
-    ctx->batch_n = 1; ctx->batch_stride = 0;
-    return rc;
-  }
-  // (proj_early) the convolution of this window and the n - 1 after it, a Gated DeltaNet layer: the history in front of this
-  // window is the layer's state (first: the block's first window) or the last rows of the window before it; the last window
-  // of the block leaves the state where the windows' recurrences will have turned the layer's buffers to
-  int front_mid_conv(int il, int n, bool first, bool last, int flips) {          // flips: turns of the layer's state buffers between here and the end of these windows' recurrences
-    const pyre_model_cfg& c = m->c; const Layer& L = m->layers[il]; if (L.full) return PYRE_OK;
-    const int li = L.mix_index, b = s->cur[li], K1 = c.conv_k - 1;
-    const float* prev = first ? s->conv[b][li] : m->proj - o.win_stride / 4 + (size_t)(t - K1) * m->pw_lin;
-    return pyre_gdn_conv_block_launch(ctx, L.gdn, m->proj, m->pw_lin, t, n, o.win_stride / 4, prev, first ? m->ch : m->pw_lin, last ? s->conv[b ^ (flips & 1)][li] : nullptr, m->co);
-  }
-  // (proj_early, attn_split) the cache write of this window and the n - 1 after it, an attention layer, in one launch (and one packing step)
-  int front_mid_attn(int il, int n, size_t q_stride) {
-    const Layer& L = m->layers[il]; const int ai = L.mix_index;
-    ctx->batch_n = n; ctx->batch_stride = n > 1 ? o.win_stride : 0; ctx->batch_stride2 = n > 1 ? q_stride : 0;
-    const int rc = pyre_attn_launch_sel(ctx, L.attn, s->kv[ai], o.aw_own, m->proj, m->pw_attn, start, t, &s->packed[ai], m->core, nullptr, nullptr, 1);
-    ctx->batch_n = 1; ctx->batch_stride = 0; ctx->batch_stride2 = 0;
-    return rc;
-  }
-  // (proj_early) the recurrence of this window and the n - 1 after it in one launch: the state stays in registers from window to window
-  bool gdn_group_ok(int il) const { const Layer& L = m->layers[il]; return !L.full && gdn_q_on(m, L); }
-  int front_mid_gdn(int il, int n) {
-    const Layer& L = m->layers[il]; const int li = L.mix_index, b = s->cur[li], nb = b ^ 1;
-    const GdnQ gq{m->aop, m->gdn_sq};
-    int rc = pyre_gdn_launch(ctx, L.gdn, m->proj, m->pw_lin, t, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], m->co, m->core, true, nullptr, L.gdn_up, &gq, n, o.win_stride / 4);
-    if (rc) return rc;
-    s->cur[li] = nb;
     return PYRE_OK;
   }
   int front_mid(int il) {
     const pyre_model_cfg& c = m->c; int rc;
-    const AttnWork& aw = o.attn_split ? o.aw_own : (o.aw ? *o.aw : s->aw); const QsaWork& qw = o.qw ? *o.qw : s->qw;
+    const AttnWork& aw = o.aw ? *o.aw : s->aw; const QsaWork& qw = o.qw ? *o.qw : s->qw;
     const PyreAop aop_hc{(const uint4*)m->aop, m->aop_inv};
     auto opnd = [&](const HcDev& h, const QMatDev& q) -> const PyreAop* { return hc_fused(h, q) ? &aop_hc : nullptr; };
     const Layer& L = m->layers[il];
     if (L.full) {
       int ai = L.mix_index;
-      if (!o.proj_early && (rc = pyre_gemv_launch(ctx, L.proj, m->mixed, t, m->proj, opnd(L.hca, L.proj)))) return rc;
+      if ((rc = pyre_gemv_launch(ctx, L.proj, m->mixed, t, m->proj, opnd(L.hca, L.proj)))) return rc;
       if (m->has_idx && (rc = pyre_qsa_launch(ctx, L.qsa, L.attn, s->qsa[ai], qw, m->proj, m->pw_attn, m->iq_off, start, t, o.step_dev))) return rc;
-      if ((rc = pyre_attn_launch_sel(ctx, L.attn, s->kv[ai], aw, m->proj, m->pw_attn, start, t, &s->packed[ai], m->core, o.step_dev, m->has_idx ? &qw : nullptr, o.attn_split ? 1 : 0))) return rc;
+      if ((rc = pyre_attn_launch_sel(ctx, L.attn, s->kv[ai], aw, m->proj, m->pw_attn, start, t, &s->packed[ai], m->core, o.step_dev, m->has_idx ? &qw : nullptr))) return rc;
     } else {
-      int li = L.mix_index; float* pj = o.proj_early ? m->proj : s->proj_saved[li]; int b = s->cur[li], nb = (replay || o.inplace) ? b : b ^ 1;
+      int li = L.mix_index; float* pj = s->proj_saved[li]; int b = s->cur[li], nb = (replay || o.inplace) ? b : b ^ 1;
       GemvEpi cv{nullptr, L.gdn.conv_w, s->conv[b][li], s->conv[nb][li], m->co, m->ch, c.conv_k};      // conv1d + SiLU ride on the projection
-      if (!o.proj_early && (rc = pyre_gemv_conv_launch(ctx, L.proj, m->mixed, t, pj, cv, opnd(L.hca, L.proj)))) return rc;
+      if ((rc = pyre_gemv_conv_launch(ctx, L.proj, m->mixed, t, pj, cv, opnd(L.hca, L.proj)))) return rc;
       const GdnQ gq{m->aop, m->gdn_sq};
       if ((rc = pyre_gdn_launch(ctx, L.gdn, pj, m->pw_lin, t, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], m->co, m->core, true, gdn_fused(L) ? m->aop : nullptr, L.gdn_up, gdn_q_on(m, L) ? &gq : nullptr))) return rc;
       s->cur[li] = nb;
     }
     return PYRE_OK;
   }
-  int front_post_attn(int il) {          // for a block's window: the attention pass its mid left out
-    const Layer& L = m->layers[il];
-    if (!(L.full && o.attn_split)) return PYRE_OK;
-    return pyre_attn_launch_sel(ctx, L.attn, s->kv[L.mix_index], o.aw_own, m->proj, m->pw_attn, start, t, &s->packed[L.mix_index], m->core, nullptr, nullptr, 2);
-  }
-  int front_post_proj(int il, int nz = 1) {          // the output projection (nz as in front_pre)
-    const pyre_model_cfg& c = m->c; const int d = c.d;
-    const Layer& L = m->layers[il];
-    if (nz <= 0) return PYRE_OK;
-    if (L.full && nz > 1) {          // an attention layer's output projection for several windows: the split into each window's own operand buffer (free since its projection), then the product
-      const PyreAop own{(const uint4*)m->aop, m->aop_inv};
-      ctx->batch_n = nz; ctx->batch_stride = o.win_stride;
-      int rc = pyre_act_split_launch(ctx, m->core, t, L.outp.cols, (uint4*)m->aop, m->aop_inv);
-      if (!rc) rc = outp_in_parts(L, d) ? pyre_gemv_parts_launch(ctx, L.outp, m->core, t, m->o, &own) : pyre_gemv_launch(ctx, L.outp, m->core, t, m->o, &own);
-      ctx->batch_n = 1; ctx->batch_stride = 0;
-      return rc;
-    }
-    const PyreAop aop_gdn{(const uint4*)m->aop, L.gdn_ainv}, aop_gdq{(const uint4*)m->aop, nullptr, m->gdn_sq, L.gdn.nv, L.gdn.eps};
-    const PyreAop* oa = (!L.full && gdn_q_on(m, L)) ? &aop_gdq : ((!L.full && gdn_fused(L)) ? &aop_gdn : nullptr);
-    ctx->batch_n = nz; ctx->batch_stride = nz > 1 ? o.win_stride : 0;
-    // few row tiles, long rows: four workgroups per row tile leave partial sums, the mix below adds them
-    const int rc = outp_in_parts(L, d) ? pyre_gemv_parts_launch(ctx, L.outp, m->core, t, m->o, oa) : pyre_gemv_launch(ctx, L.outp, m->core, t, m->o, oa);
-    ctx->batch_n = 1; ctx->batch_stride = 0;
-    return rc;
-  }
-  int front_post_mix(int il, int nz = 1) {          // the FFN mix (nz as in front_pre)
+  int front_post(int il) {
     const pyre_model_cfg& c = m->c; const int d = c.d; int rc;
     const Layer& L = m->layers[il];
+    const PyreAop aop_gdn{(const uint4*)m->aop, L.gdn_ainv}, aop_gdq{(const uint4*)m->aop, nullptr, m->gdn_sq, L.gdn.nv, L.gdn.eps};
+    const PyreAop* oa = (!L.full && gdn_q_on(m, L)) ? &aop_gdq : ((!L.full && gdn_fused(L)) ? &aop_gdn : nullptr);
+    // few row tiles, long rows: four workgroups per row tile leave partial sums, the mix below adds them
     const int o_parts = outp_in_parts(L, d) ? PYRE_GEMV_PARTS : 1;
-    ride = route_rides && !o.router_apart && pyre_hc_route_ok(L.hcf, L.moe.router);       // the router GEMV rides on the mix's second launch
+    if ((rc = o_parts > 1 ? pyre_gemv_parts_launch(ctx, L.outp, m->core, t, m->o, oa) : pyre_gemv_launch(ctx, L.outp, m->core, t, m->o, oa))) return rc;
+    ride = route_rides && pyre_hc_route_ok(L.hcf, L.moe.router);       // the router GEMV rides on the mix's second launch
     HcRoute hr{L.moe.router, m->rpart, m->mw.dgx};          // (the matrix-core mix leaves the digits of its output; after another mix the expert launch makes them)
-    if (nz > 0) {
-      ctx->batch_n = nz; ctx->batch_stride = nz > 1 ? o.win_stride : 0;
-      rc = pyre_hc_mix_launch(ctx, L.hcf, m->hw, xin, in_ss, in_ts, xout, t, m->o, nullptr, m->inj_a, c.eps, m->mixed, m->inj_f, ride ? &hr : nullptr, o_parts);
-      ctx->batch_n = 1; ctx->batch_stride = 0;
-      if (rc) return rc;
-    }
+    if ((rc = pyre_hc_mix_launch(ctx, L.hcf, m->hw, xin, in_ss, in_ts, xout, t, m->o, nullptr, m->inj_a, c.eps, m->mixed, m->inj_f, ride ? &hr : nullptr, o_parts))) return rc;
     advance();
     return PYRE_OK;
   }
-  int front_post(int il) { int rc = front_post_attn(il); if (!rc) rc = front_post_proj(il); return rc ? rc : front_post_mix(il); }
   int front(int il) {
     int rc; const Layer& L = m->layers[il];
     if (o.wait_ev && L.ple) PYRE_HIP(ctx, hipStreamWaitEvent(ctx->stream, o.wait_ev[il], 0));      // the layer's ring of rows is state
@@ -817,15 +785,13 @@ struct WinRun {
     comb_inj = m->inj_f;
     return PYRE_OK;
   }
-  // the block's FFN launch has left this window's group sums in m->mw.parts
-  void moe_from_block() { comb_out = m->mw.parts; comb_moe = nullptr; comb_np = PYRE_MOE_GROUPS; comb_inj = m->inj_f; }
   int finish() {
     const pyre_model_cfg& c = m->c; const int d = c.d, hc = c.hc; int rc;
     const PyreAop aop_hc{(const uint4*)m->aop, m->aop_inv};
     const AopOut aout{m->aop, m->aop_inv, d / 256};
     auto opnd = [&](const HcDev& h, const QMatDev& q) -> const PyreAop* { return hc_fused(h, q) ? &aop_hc : nullptr; };
     auto opw = [&](const HcDev& h, const QMatDev& q) -> const AopOut* { return hc_fused(h, q) ? &aout : nullptr; };
-    if (!replay && !o.no_len) s->len = start + t;
+    if (!replay) s->len = start + t;
     const bool want_r = s->mtp && o.keep_from < t;      // the head mix resolves the pending update of every token: its x_out rows are the final residual streams
     if (o.head_tokens == 0 && !want_r) return PYRE_OK;       // prompt window whose logits nobody reads
     if (o.head_tokens >= t || want_r) {
@@ -873,105 +839,37 @@ int pyre_forward(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, const uint32
   const auto t_enter = std::chrono::steady_clock::now();
   int rc = check_ids(ctx, m, ids, n); if (rc) return rc;
   s->last_window = 0;
-  const int nwin = (n + 7) / 8, K = prompt_streams();
-  PromptPipe* P = nullptr;
-  if (K > 1 && nwin >= 2 * K && !ctx->prof_on) {      // a long prompt: K windows in flight (the per-class timing wants one stream)
+  int i_first = 0;
+  const bool windows_only = [] { const char* e = getenv("PYRE_PROMPT_WINDOWS"); return e && *e && atoi(e) != 0; }();      // (read per call: 1 = this call in windows, whatever layouts the model keeps)
+  // (with a drafter the last tokens, whose residual streams the drafter's ring keeps, take the windows' path)
+  const int nblk_tok = !s->mtp ? n : std::max(0, n - 8 - mtp_window_of(s->mtp)) / 8 * 8;
+  if (!windows_only && nblk_tok >= PROMPT_BLOCK_MIN && prompt_block_ok(m)) {
+    const bool pairs = [] { const char* e = getenv("PYRE_PROMPT_PAIRS"); return !(e && *e && atoi(e) == 0); }();      // PYRE_PROMPT_PAIRS=0: blocks of up to 1024 tokens instead of 2048
+    const int most = pairs ? PROMPT_BLOCK_MAX : PROMPT_BLOCK_MAX / 2, nb = (nblk_tok + most - 1) / most, each = ((nblk_tok + nb - 1) / nb + 127) / 128 * 128;
+    PromptBlk* B = nullptr;
+    if ((rc = prompt_blk_get(ctx, m, std::min(each, nblk_tok), s->len + n, &B))) return rc;
+    while (i_first < nblk_tok) {
+      const int T = std::min(each, nblk_tok - i_first); const bool head = logits_host && i_first + T == n;
+      if ((rc = run_block(ctx, m, s, B, ids + i_first, T, head))) { s->broken = true; (void)hipStreamSynchronize(ctx->stream); return rc; }
+      i_first += T;
+    }
+    // what pyre_model_prompt_blocks counts: the whole windows in front of the call's last eight tokens in blocks of at most 128, an even number of them when taken in pairs
+    const int wins = (n - 8 - (s->mtp ? mtp_window_of(s->mtp) : 0)) / 8; int cnt = pairs ? 2 * ((wins + 255) / 256) : (wins + 127) / 128; while (cnt > 1 && wins / cnt < 8) --cnt; B->blocks += cnt;
+    if (i_first == n) {
+      if (logits_host) PYRE_HIP(ctx, hipMemcpyAsync(logits_host, m->logits, (size_t)m->c.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
+      PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); return PYRE_OK;
+    }
+  }
+  const int nwin = (n - i_first + 7) / 8, K = prompt_streams();
+  PromptPipe* P = nullptr; int prev = -1;
+  if (K > 1 && nwin >= 2 * K && !ctx->prof_on) {      // a long prompt in windows: K of them in flight (the per-class timing wants one stream)
     if ((rc = prompt_pipe_get(ctx, m, &P)) || (rc = prompt_pipe_state(ctx, m, s, K))) return rc;
     if (P->ids_cap < (size_t)n) { PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); if (P->ids) (void)hipFree(P->ids); P->ids = nullptr; P->ids_cap = 0;
       PYRE_HIP(ctx, hipMalloc((void**)&P->ids, (size_t)n * 4)); P->ids_cap = (size_t)n; }
     PYRE_HIP(ctx, hipMemcpyAsync(P->ids, ids, (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream));
-    if (s->tokens_dev) PYRE_HIP(ctx, hipMemcpyAsync(s->tokens_dev + s->len, P->ids, (size_t)n * 4, hipMemcpyDeviceToDevice, ctx->stream));      // the history every window's n-gram rows read
+    if (s->tokens_dev) PYRE_HIP(ctx, hipMemcpyAsync(s->tokens_dev + s->len, P->ids + i_first, (size_t)(n - i_first) * 4, hipMemcpyDeviceToDevice, ctx->stream));      // the history every window's n-gram rows read
     PYRE_HIP(ctx, hipEventRecord(P->start, ctx->stream));      // the other streams begin after everything already queued here
     for (auto* cx : P->ctx) PYRE_HIP(ctx, hipStreamWaitEvent(cx->stream, P->start, 0));
-  }
-  int prev = -1, i_first = 0;
-  const bool windows_only = [] { const char* e = getenv("PYRE_PROMPT_WINDOWS"); return e && *e && atoi(e) != 0; }();      // (read per call: 1 = this call in windows, whatever layouts the model keeps)
-  if (P && !windows_only && prompt_block_ok(m)) {      // whole blocks of windows in front of the call's last tokens: layer by layer, the FFN grouped by expert
-    // (a call's last block may be shorter, down to PROMPT_BLOCK_MIN windows: fewer tokens than that share too few experts to pay)
-    const int NBMAX = PROMPT_BLOCK_WINDOWS, tail = 8 + (s->mtp ? mtp_window_of(s->mtp) : 0);
-    int wins = n > tail ? (n - tail) / 8 : 0;
-    if (wins >= PROMPT_BLOCK_MIN && (rc = prompt_block_get(ctx, m, P))) return rc;
-    const int nl = m->c.n_layers;
-    const int G_env = [] { const char* e = getenv("PYRE_PROMPT_GROUP"); int v = e && *e ? atoi(e) : 0; return v < 0 ? 0 : (v > PROMPT_BLOCK_WINDOWS ? PROMPT_BLOCK_WINDOWS : v); }();      // PYRE_PROMPT_GROUP: windows a group (default: a group a stream)
-    const bool batch = [&] { const char* e = getenv("PYRE_PROMPT_BATCH"); if (e && *e && atoi(e) == 0) return false; for (const Layer& L : m->layers) if (!pyre_hc_aop_ok(L.hca) || !pyre_hc_aop_ok(L.hcf)) return false; return true; }();      // a group's mixes in one launch each (the matrix-core mixes; PYRE_PROMPT_BATCH=0: a launch a window)
-    const bool early = batch && m->c.conv_k >= 2 && m->c.conv_k <= 9 && !(getenv("PYRE_PROMPT_PROJ_EARLY") && atoi(getenv("PYRE_PROMPT_PROJ_EARLY")) == 0);      // the projections in front of the chain through the layer's state, the convolution once a group (PYRE_PROMPT_PROJ_EARLY=0: both in the chain, a window at a time)
-    const bool asplit = P->qmem && !(getenv("PYRE_PROMPT_ATTN_SPLIT") && atoi(getenv("PYRE_PROMPT_ATTN_SPLIT")) == 0);      // an attention layer's pass over the cache outside the chain (PYRE_PROMPT_ATTN_SPLIT=0: in it)
-    const bool rapart = batch && !(getenv("PYRE_PROMPT_ROUTER_APART") && atoi(getenv("PYRE_PROMPT_ROUTER_APART")) == 0);      // the router's sums with the block's FFN launches (beside the other block's windows) instead of riding on every window's FFN mix (PYRE_PROMPT_ROUTER_APART=0: riding)
-    const bool pairs = [] { const char* e = getenv("PYRE_PROMPT_PAIRS"); return !(e && *e && atoi(e) == 0); }();      // PYRE_PROMPT_PAIRS=0: one block at a time
-    auto cxk = [&](int k) { return k ? P->ctx[k - 1] : ctx; };
-    auto bail = [&](int code, pyre_ctx* cx) { s->broken = true; if (cx != ctx) pyre_fail(ctx, code, "%s", cx->err.c_str()); for (auto* c2 : P->ctx) (void)hipStreamSynchronize(c2->stream); (void)hipStreamSynchronize(P->moe_ctx->stream); (void)hipStreamSynchronize(ctx->stream); return code; };
-    // Blocks are taken two at a time, layer by layer: the windows of block A, A's FFN on the FFN stream, the windows of block B
-    // beside it, B's FFN beside A's windows of the next layer.  Within a block the windows go to the streams in groups of G
-    // consecutive ones, a group's launches in the order pre x G, mid x G, post x G: the mids of a group follow one another in
-    // their stream without an event, one event hands the layer's state to the next group's stream, and a stream that waits for
-    // it has its own pres behind it, not in front.  (8192 tokens, one block at a time: groups of one 2.17 s, two 1.98, four
-    // 2.05, eight 2.29, sixteen 2.58.)
-    struct Blk { int which, NB, G, NG, prev_in; std::vector<WinRun> runs; };
-    // the call's windows in an even number of blocks of (nearly) equal size, so that every block has a partner
-    int nblk = 0, bsz = 0, brem = 0;
-    if (wins >= PROMPT_BLOCK_MIN) {
-      nblk = pairs ? 2 * ((wins + 2 * NBMAX - 1) / (2 * NBMAX)) : (wins + NBMAX - 1) / NBMAX;
-      while (nblk > 1 && wins / nblk < PROMPT_BLOCK_MIN) --nblk;
-      bsz = wins / nblk; brem = wins % nblk;
-    }
-    for (int bi = 0; bi < nblk; ) {
-      Blk B[2]; int nb = 0; int pos = s->len, i0 = i_first, pin = prev;
-      for (int w = 0; w < (pairs ? 2 : 1) && bi < nblk; ++w, ++bi) {
-        Blk& b = B[nb++]; b.which = w; b.NB = bsz + (bi < brem ? 1 : 0); wins -= b.NB; b.G = G_env ? G_env : (b.NB + K - 1) / K; b.NG = (b.NB + b.G - 1) / b.G; const int G = b.G; b.prev_in = pin; b.runs.reserve(b.NB);
-        for (int j = 0; j < b.NB; ++j) {
-          const int set = (j / G) % K; WinOpt o; o.head_tokens = 0; o.keep_from = 8; o.start = pos + 8 * j; o.no_len = true;
-          o.ids_dev = P->ids + i0 + 8 * j; if (set) { o.aw = &s->aw_more[set - 1]; o.qw = &s->qw_more[set - 1]; }
-          o.win_stride = P->win_stride; o.proj_early = early; o.router_apart = rapart;
-          if (asplit) {          // q buffers of the window's own; the partial sums stay the stream's
-            o.attn_split = true; o.aw_own = set ? s->aw_more[set - 1] : s->aw;
-            uint8_t* qb = (uint8_t*)P->qmem + (size_t)(w * NBMAX + j) * P->q_stride;
-            o.aw_own.q = (float*)qb; o.aw_own.qh = (uint16_t*)(qb + P->q_off[0]); o.aw_own.qsc = (float*)(qb + P->q_off[1]);
-          }
-          b.runs.emplace_back(cxk(set), P->wmdl[w * NBMAX + j], s, 8, o);
-          if ((rc = b.runs.back().begin())) return bail(rc, cxk(set));
-        }
-        pos += b.NB * 8; i0 += b.NB * 8; pin = (b.NG - 1) % K;
-      }
-      // a block's windows of layer il: group by group in order, so that every record is issued before the wait that names it
-      auto fronts = [&](Blk& b, int il) -> int {
-        const int G = b.G;
-        for (int g = 0; g < b.NG; ++g) {
-          const int k = g % K; pyre_ctx* cx = cxk(k); int r;
-          if (il > 0 && g < K && hipStreamWaitEvent(cx->stream, P->moe_done[b.which], 0) != hipSuccess) return pyre_fail(cx, PYRE_E_HIP, "hipStreamWaitEvent failed");
-          const int j0 = g * G, j1 = j0 + G < b.NB ? j0 + G : b.NB;
-          for (int j = j0; j < j1; ++j) if ((r = b.runs[j].front_pre(il, batch ? (j == j0 ? j1 - j0 : 0) : 1))) return r;            // the group's mixes: one launch each
-          if (early) { const bool pb = b.runs[j0].proj_batchable(il); for (int j = j0; j < j1; ++j) if ((r = b.runs[j].front_pre_proj(il, pb ? (j == j0 ? j1 - j0 : 0) : 1))) return r; }
-          const int pset = g > 0 ? (g - 1) % K : b.prev_in;
-          if (pset >= 0 && pset != k && hipStreamWaitEvent(cx->stream, P->ev[pset][il], 0) != hipSuccess) return pyre_fail(cx, PYRE_E_HIP, "hipStreamWaitEvent failed");
-          const bool gg = early && b.runs[j0].gdn_group_ok(il);          // the group's recurrences in one launch
-          if (early && (r = b.runs[j0].front_mid_conv(il, j1 - j0, j0 == 0, j1 == b.NB, gg ? 1 : j1 - j0))) return r;
-          if (gg) { if ((r = b.runs[j0].front_mid_gdn(il, j1 - j0))) return r; }
-          else if (early && asplit && m->layers[il].full) { if ((r = b.runs[j0].front_mid_attn(il, j1 - j0, P->q_stride))) return r; }          // the group's cache writes in one launch
-          else for (int j = j0; j < j1; ++j) if ((r = b.runs[j].front_mid(il))) return r;
-          if (hipEventRecord(P->ev[k][il], cx->stream) != hipSuccess) return pyre_fail(cx, PYRE_E_HIP, "hipEventRecord failed");
-          for (int j = j0; j < j1; ++j) if ((r = b.runs[j].front_post_attn(il))) return r;
-          { const bool ob = batch && j1 - j0 > 1 && b.runs[j0].outp_batchable(il); for (int j = j0; j < j1; ++j) if ((r = b.runs[j].front_post_proj(il, ob ? (j == j0 ? j1 - j0 : 0) : 1))) return r; }
-          for (int j = j0; j < j1; ++j) if ((r = b.runs[j].front_post_mix(il, batch ? (j == j0 ? j1 - j0 : 0) : 1))) return r;
-        }
-        return PYRE_OK;
-      };
-      auto ffn = [&](Blk& b, int il) -> int {
-        pyre_ctx* mx = P->moe_ctx;
-        for (int k = 0; k < K && k < b.NG; ++k) { if (hipEventRecord(P->front_done[b.which][k], cxk(k)->stream) != hipSuccess || hipStreamWaitEvent(mx->stream, P->front_done[b.which][k], 0) != hipSuccess) return pyre_fail(ctx, PYRE_E_HIP, "event failed"); }
-        int r = pyre_moe_block_launch(mx, m->layers[il].moe, P->blk[b.which], b.NB * 8, NBMAX * 8, P->blk_nsl, P->blk_r64, rapart);
-        if (r) return pyre_fail(ctx, r, "%s", mx->err.c_str());
-        if (hipEventRecord(P->moe_done[b.which], mx->stream) != hipSuccess) return pyre_fail(ctx, PYRE_E_HIP, "hipEventRecord failed");
-        for (int j = 0; j < b.NB; ++j) b.runs[j].moe_from_block();
-        return PYRE_OK;
-      };
-      for (int il = 0; il < nl; ++il) for (int w = 0; w < nb; ++w) {
-        if ((rc = fronts(B[w], il))) return bail(rc, ctx);
-        if (il < nl - 1 && (rc = ffn(B[w], il))) return bail(rc, ctx);            // the last layer's FFN output has no reader in these windows
-      }
-      for (int w = 0; w < nb; ++w) { s->len += B[w].NB * 8; i_first += B[w].NB * 8; ++P->blocks_done; }
-      prev = pin;
-    }
-    if (i_first > 0) for (int k = 1; k < K; ++k) PYRE_HIP(ctx, hipEventRecord(P->done[k], P->ctx[k - 1]->stream));
   }
   const int nwin_tail = (n - i_first + 7) / 8;
   for (int i = i_first, w = 0; i < n; i += 8, ++w) {

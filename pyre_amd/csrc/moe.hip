@@ -550,7 +550,7 @@ __global__ __launch_bounds__(1024) void k_moe_route_blk(MoeDev m, MoeBlk b, int 
 #ifdef PYRE_PHASE_TS
   unsigned long long ts_[8];
 #endif
-  route_topk(b.rpart + (size_t)w * b.ws + (size_t)tw * r64, nsl, 8 * r64, n_exp, top_k, rl ROUTE_TS_ARG);
+  route_topk(b.rpart + (size_t)w * b.wr + (size_t)tw * r64, nsl, 8 * r64, n_exp, top_k, rl ROUTE_TS_ARG);
   route_weights(top_k, rl);
   if ((int)threadIdx.x < top_k) { b.sel_idx[ti * top_k + threadIdx.x] = rl.s_idx[threadIdx.x]; b.sel_w[ti * top_k + threadIdx.x] = rl.s_w[threadIdx.x]; }
 }
@@ -563,10 +563,10 @@ __global__ __launch_bounds__(256) void k_moe_router_blk(MoeDev m, MoeBlk b, int 
   __shared__ float xs[8][64];
   const uint2* lds2 = nullptr;
   const int sl = blockIdx.x, w = blockIdx.y, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const float* xw = b.x + (size_t)w * b.ws;
+  const float* xw = b.x + (size_t)w * 8 * m.d;
   for (int i = threadIdx.x; i < 8 * 64; i += 256) xs[i >> 6][i & 63] = xw[(size_t)(i >> 6) * m.d + sl * 64 + (i & 63)];
   lds_barrier();
-  float* rp = const_cast<float*>(b.rpart) + (size_t)w * b.ws;
+  float* rp = const_cast<float*>(b.rpart) + (size_t)w * b.wr;
   for (int tile = wave; tile < m.router.tiles; tile += 4) {
     const UnitRaw<RF> rraw = unit_load<RF>(m.router, tile, sl, lane);
 #pragma unroll 1
@@ -609,13 +609,13 @@ __device__ __forceinline__ int blk_entry(const BlkEntries& e, int i) { return e.
 // inv[r][cols / 256].  x2 given: the row is silu(x) * x2 (an expert's h out of its gate and up products).  gate_inp given:
 // sg[r] = sigmoid(gate_inp . x[r]) as well (the shared expert's gate).  grid (n), 256 threads, a stretch a round.  Row n of
 // xh is kept zero by the owner: the operand rows a pass has no token for point there.
-__global__ __launch_bounds__(256) void k_blk_split(const float* __restrict__ x, const float* __restrict__ x2, int cols, uint16_t* __restrict__ xh, float* __restrict__ inv, const float* __restrict__ gate_inp, float* __restrict__ sg, size_t ws) {      // ws > 0: row r of x at x + (r / 8) * ws + (r % 8) * cols (a window's eight rows in its workspace)
+__global__ __launch_bounds__(256) void k_blk_split(const float* __restrict__ x, const float* __restrict__ x2, int cols, uint16_t* __restrict__ xh, float* __restrict__ inv, const float* __restrict__ gate_inp, float* __restrict__ sg) {
   __shared__ float mx[2][4]; __shared__ float dp[4];
   const int r = blockIdx.x, i = threadIdx.x, wave = i >> 6, lane = i & 63;
   float dot = 0.0f;
   for (int sb = 0; sb < (cols >> 8); ++sb) {
     const int k = sb * 256 + i;
-    float v = (ws ? x + (size_t)(r >> 3) * ws + (size_t)(r & 7) * cols : x + (size_t)r * cols)[k];
+    float v = x[(size_t)r * cols + k];
     if (x2) { const float sgm = 1.0f / (1.0f + expf(-v)); v = (v * sgm) * x2[(size_t)r * cols + k]; }
     if (gate_inp) dot = fmaf(gate_inp[k], v, dot);
     float a = fabsf(v); a = a == a ? a : INFINITY;
@@ -709,7 +709,7 @@ __global__ __launch_bounds__(256) void k_moe_groups_blk(MoeDev m, MoeBlk b, int 
   const int r = blockIdx.x * 256 + threadIdx.x, ti = blockIdx.y, k = m.top_k, d = m.d, gsz = (k + 4) / 4;
   if (r >= d) return;
   const float* pt = b.partial + (size_t)ti * (k + 1) * d + r;
-  float* out = b.parts + (size_t)(ti >> 3) * b.ws + (size_t)(ti & 7) * d + r;
+  float* out = b.parts + (size_t)(ti >> 3) * PYRE_MOE_GROUPS * 8 * d + (size_t)(ti & 7) * d + r;
 #pragma unroll
   for (int q = 0; q < PYRE_MOE_GROUPS; ++q) {
     const int j0 = min(k, q * gsz), nr = min(k, j0 + gsz) - j0;
@@ -744,26 +744,26 @@ int pyre_moe_block_zero_rows(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, in
   PYRE_HIP(ctx, hipMemsetAsync(b.hh + 2 * ne * hs, 0, 2 * 2 * hs, ctx->stream));
   return PYRE_OK;
 }
-// T = 8 * windows tokens (T_max: the T the scratch was carved and its zero rows were set for); the router's K-slice sums (nsl
-// slices of r64 rows a token) come from the mixes
-int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_max, int nsl, int r64, bool router_here) {
-  if (!pyre_moe_block_ok(m) || T < 8 || T % 8 || T > T_max || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe block: unsupported shape (T = %d, %d router slices)", T, nsl);
+// T_max: the T the scratch was carved and its zero rows were set for (x readable up to the next multiple of eight rows); the router's
+// sums in nsl = d / 64 slices of r64 rows a token
+int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_max, int nsl, int r64) {
+  if (!pyre_moe_block_ok(m) || T < 1 || T > T_max || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe block: unsupported shape (T = %d, %d router slices)", T, nsl);
   const int hs = m.ff, ny = m.n_exp + (T + 7) / 8, ne = T * (m.top_k + 1), ne_max = T_max * (m.top_k + 1);
   const bool fix = m.n_exp == 512 && m.top_k == 10 && nsl == 32;
-  if (router_here) {          // the router's K-slice sums were not left by the mixes: form them now
+  {
     if (nsl != m.d / 64 || (m.router.fmt != FMT_BF16 && m.router.fmt != FMT_F32)) return pyre_fail(ctx, PYRE_E_ARG, "moe block: the router's sums by %d slices, router format %d", nsl, m.router.fmt);
     ProfScope ps(ctx, "moe_block_router", qmat_gguf_bytes(m.router, m.router.rows) + 4.0 * T * (m.d + (double)nsl * r64));
-    if (m.router.fmt == FMT_BF16) hipLaunchKernelGGL(k_moe_router_blk<FMT_BF16>, dim3(nsl, T / 8), dim3(256), 0, ctx->stream, m, b, r64);
-    else hipLaunchKernelGGL(k_moe_router_blk<FMT_F32>, dim3(nsl, T / 8), dim3(256), 0, ctx->stream, m, b, r64);
+    if (m.router.fmt == FMT_BF16) hipLaunchKernelGGL(k_moe_router_blk<FMT_BF16>, dim3(nsl, (T + 7) / 8), dim3(256), 0, ctx->stream, m, b, r64);
+    else hipLaunchKernelGGL(k_moe_router_blk<FMT_F32>, dim3(nsl, (T + 7) / 8), dim3(256), 0, ctx->stream, m, b, r64);
     PYRE_CHECK_LAUNCH(ctx);
   }
   { ProfScope ps(ctx, "moe_block_route", 4.0 * T * nsl * m.n_exp);
     if (fix) hipLaunchKernelGGL(k_moe_route_blk<true>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64); else hipLaunchKernelGGL(k_moe_route_blk<false>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64);
     hipLaunchKernelGGL(k_moe_lists, dim3(1), dim3(1024), 0, ctx->stream, m, b, T);
-    hipLaunchKernelGGL(k_blk_split, dim3(T), dim3(256), 0, ctx->stream, b.x, (const float*)nullptr, m.d, b.xh, b.xinv, m.sh_gate_inp, b.sg, b.ws); } PYRE_CHECK_LAUNCH(ctx);
+    hipLaunchKernelGGL(k_blk_split, dim3(T), dim3(256), 0, ctx->stream, b.x, (const float*)nullptr, m.d, b.xh, b.xinv, m.sh_gate_inp, b.sg); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "moe_block_gate_up", 2.0 * m.n_exp * qmat_gguf_bytes(m.gate_e, m.ff) + 2.0 * qmat_gguf_bytes(m.sh_gate, m.sf));
     hipLaunchKernelGGL(k_moe_mm_blk<false>, dim3((hs + 255) / 256, ny, 2), dim3(256), 0, ctx->stream, m, b, T, T_max);
-    hipLaunchKernelGGL(k_blk_split, dim3(ne), dim3(256), 0, ctx->stream, (const float*)b.g, (const float*)b.u, hs, b.hh, b.hinv, (const float*)nullptr, (float*)nullptr, (size_t)0); } PYRE_CHECK_LAUNCH(ctx);
+    hipLaunchKernelGGL(k_blk_split, dim3(ne), dim3(256), 0, ctx->stream, (const float*)b.g, (const float*)b.u, hs, b.hh, b.hinv, (const float*)nullptr, (float*)nullptr); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "moe_block_down", (double)m.n_exp * qmat_gguf_bytes(m.down_e, m.d) + qmat_gguf_bytes(m.sh_down, m.d));
     hipLaunchKernelGGL(k_moe_mm_blk<true>, dim3((m.d + 255) / 256, ny, 1), dim3(256), 0, ctx->stream, m, b, T, ne_max);
     hipLaunchKernelGGL(k_moe_groups_blk, dim3((m.d + 255) / 256, T), dim3(256), 0, ctx->stream, m, b, T); } PYRE_CHECK_LAUNCH(ctx);
