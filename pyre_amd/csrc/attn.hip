@@ -155,25 +155,23 @@ __device__ __forceinline__ h8v nib8_f16(uint32_t w) {
   for (int q = 0; q < 4; ++q) u.v[q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, ((x >> (4 * q)) & 0x000F000Fu) | 0x64006400u) - off);
   return __builtin_bit_cast(h8v, u);
 }
+// One pass: chunk `chunk` of KV head kvh for tokens tk0 .. tk0 + nk - 1 of the launch.
 // NC: columns the buffers hold -- G for launches of one token a pass (tp = 1), 16 otherwise.
+template <int NC> struct AttnSm {
+  float red[4 * PYRE_ATTN_CHUNK * NC];          // phase 1: [dq][position][column];  phase 3: [pw][column][dim]
+  __align__(16) float sc[NC][PYRE_ATTN_CHUNK + 4];          // [column][position]: eight consecutive positions of a column are two 16-byte reads
+  float wmax[PYRE_ATTN_NPW][NC], wsum[PYRE_ATTN_NPW][NC];
+};
 template <int HD, int G, int NC>
-__global__ __launch_bounds__(256 * PYRE_ATTN_NPW, 4) void k_attn_decode(AttnDev a, KvDev kv, const float* __restrict__ qbuf, const uint16_t* __restrict__ qh, const float* __restrict__ qsc, int start, const int* __restrict__ posp, float* __restrict__ part_o, float* __restrict__ part_ml, int max_chunks, int t, int tp) {
+__device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, const KvDev& kv, const float* __restrict__ qbuf, const uint16_t* __restrict__ qh, const float* __restrict__ qsc, int start, float* __restrict__ part_o, float* __restrict__ part_ml, int max_chunks, int chunk, int kvh, int tk0, int nk) {
   static_assert(HD == 256, "the wave layout assumes 4 x 64 head dims");
   constexpr int NPW = PYRE_ATTN_NPW, CH = PYRE_ATTN_CHUNK, NT = 256 * NPW;
   static_assert(4 * CH == NPW * HD, "the score and value partials share one buffer");
-  __shared__ float red[4 * CH * NC];          // phase 1: [dq][position][column];  phase 3: [pw][column][dim]
-  __shared__ __align__(16) float sc[NC][CH + 4];          // [column][position]: eight consecutive positions of a column are two 16-byte reads
-  __shared__ float wmax[NPW][NC], wsum[NPW][NC];
+  auto& red = sm.red; auto& sc = sm.sc; auto& wmax = sm.wmax; auto& wsum = sm.wsum;
   PYRE_TS_VARS PYRE_TS(0);
-  // Workgroups in dispatch order (x fastest): chunks descending, the KV heads of a chunk next to each other.  The
-  // workgroups past the view (a captured launch covers the whole cache) leave first; the chunks of the f32 window, which
-  // move eight times the bytes of a packed chunk, follow as neighbours in the order and so land on different compute
-  // units, where each later shares its unit with a packed chunk instead of another f32 one.
-  const int lin = (int)blockIdx.x + (int)gridDim.x * (int)blockIdx.y;
-  const int chunk = (int)gridDim.x - 1 - lin / (int)gridDim.y, kvh = lin % (int)gridDim.y, tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), pw = wave % NPW, dq = wave / NPW;
-  if (posp) start = *posp;
-  const int tk0 = blockIdx.z * tp, nk = min(tp, t - tk0), ncol = nk * G;          // tokens tk0 .. tk0+nk-1 in columns 0 .. ncol-1
+  const int ncol = nk * G;                                                         // tokens tk0 .. tk0+nk-1 in columns 0 .. ncol-1
   const int n = start + tk0 + nk;                                                  // the widest view of the pass
   if (chunk * CH >= n) return;
   const float scale = 1.0f / sqrtf((float)HD);
@@ -451,6 +449,33 @@ __global__ __launch_bounds__(256 * PYRE_ATTN_NPW, 4) void k_attn_decode(AttnDev 
 #endif
 }
 
+template <int HD, int G, int NC>
+__global__ __launch_bounds__(256 * PYRE_ATTN_NPW, 4) void k_attn_decode(AttnDev a, KvDev kv, const float* __restrict__ qbuf, const uint16_t* __restrict__ qh, const float* __restrict__ qsc, int start, const int* __restrict__ posp, float* __restrict__ part_o, float* __restrict__ part_ml, int max_chunks, int t, int tp) {
+  __shared__ AttnSm<NC> sm;
+  // Workgroups in dispatch order (x fastest): chunks descending, the KV heads of a chunk next to each other.  The
+  // workgroups past the view (a captured launch covers the whole cache) leave first; the chunks of the f32 window, which
+  // move eight times the bytes of a packed chunk, follow as neighbours in the order and so land on different compute
+  // units, where each later shares its unit with a packed chunk instead of another f32 one.
+  const int lin = (int)blockIdx.x + (int)gridDim.x * (int)blockIdx.y;
+  const int chunk = (int)gridDim.x - 1 - lin / (int)gridDim.y, kvh = lin % (int)gridDim.y;
+  if (posp) start = *posp;
+  const int tk0 = blockIdx.z * tp;
+  attn_pass<HD, G, NC>(sm, a, kv, qbuf, qh, qsc, start, part_o, part_ml, max_chunks, chunk, kvh, tk0, min(tp, t - tk0));
+}
+__device__ __forceinline__ int packed_boundary(const AttnDev& a, int n) { return (a.kv_bits == 4 && n > a.kv_recent + 64) ? ((n - a.kv_recent) / 64) * 64 : 0; }
+// The same passes for a prompt's block of T tokens: a launch a window of eight was 11000 launches at 8192 tokens, most of the
+// chip idle in each (19 us).  grid chunks * nkv * np, the passes of a chunk next to each other in the order, so that what
+// runs at a time shares a chunk's 40 .. 256 KB in the second-level caches.  Pass z holds tokens tp * z - off .. + tp - 1, off
+// chosen so that the 4-bit boundary moves between passes; where it still moves inside one, its tokens go one by one.
+template <int HD, int G>
+__global__ __launch_bounds__(256 * PYRE_ATTN_NPW, 4) void k_attn_blk(AttnDev a, KvDev kv, const float* __restrict__ qbuf, const uint16_t* __restrict__ qh, const float* __restrict__ qsc, int start, float* __restrict__ part_o, float* __restrict__ part_ml, int max_chunks, int t, int tp, int off, int np) {
+  __shared__ AttnSm<16> sm;
+  const int z = blockIdx.x % np, ck = blockIdx.x / np, kvh = ck % a.nkv, chunk = (int)(gridDim.x / np) / a.nkv - 1 - ck / a.nkv;
+  int t0 = tp * z - off; const int t1 = min(t, t0 + tp); t0 = max(t0, 0);
+  if (packed_boundary(a, start + t0 + 1) == packed_boundary(a, start + t1)) attn_pass<HD, G, 16>(sm, a, kv, qbuf, qh, qsc, start, part_o, part_ml, max_chunks, chunk, kvh, t0, t1 - t0);
+  else for (int k = t0; k < t1; ++k) { attn_pass<HD, G, 16>(sm, a, kv, qbuf, qh, qsc, start, part_o, part_ml, max_chunks, chunk, kvh, k, 1); __syncthreads(); }
+}
+
 // The same kernel over a position list: entry i of plist[ti] (pcount[ti] entries, ascending positions) takes the place of
 // position i; pcount[ti] < 0 means every visible position (the list is not read).  Listed positions are scattered over
 // the packed and the f32 part of the cache, so the choice between them is made per lane, not per wave.
@@ -699,6 +724,49 @@ __global__ __launch_bounds__(256) void k_attn_combine(AttnDev a, const float* __
   PYRE_TS(1); PYRE_TS(2); PYRE_TS(3); PYRE_TS(4); PYRE_TS(5); PYRE_TS(6); PYRE_TS(7); PYRE_TS_FLUSH(attn_ts, 16);
 }
 
+// The merge for a block's tokens: grid (nh, t), thread = dimension.  k_attn_combine spreads a head over sixteen workgroups because a
+// single token has only nh of them; with hundreds of tokens a workgroup takes a whole head, and a thread keeps all sixteen
+// groups' sums (chunks g, g + 16, .. in ascending order, the groups added in order: k_attn_combine's order, its bits).
+template <int HD>
+__global__ __launch_bounds__(HD) void k_attn_combine_blk(AttnDev a, const float* __restrict__ qkv, int stride, int start, const float* __restrict__ part_o, const float* __restrict__ part_ml, int max_chunks, float* __restrict__ out) {
+  constexpr int NG = 256 / PYRE_ATTN_CDIMS, CB = 64 * NG;
+  __shared__ float wmax[HD / 64], fs[CB], ls[CB], sl[NG];
+  const int h = blockIdx.x, ti = blockIdx.y, tid = threadIdx.x, n = start + ti + 1, nc = (n + PYRE_ATTN_CHUNK - 1) / PYRE_ATTN_CHUNK;
+  const float* ml = part_ml + ((size_t)ti * a.nh + h) * max_chunks * 2;
+  const float* po = part_o + ((size_t)ti * a.nh + h) * max_chunks * HD + tid;
+  const float gate = qkv[(size_t)ti * stride + (size_t)h * 2 * HD + HD + tid];
+  float M = -INFINITY; for (int c = tid; c < nc; c += HD) M = fmaxf(M, ml[2 * c]);
+  M = wave_max(M);
+  if ((tid & 63) == 0) wmax[tid >> 6] = M;
+  __syncthreads();
+  M = wmax[0];
+#pragma unroll
+  for (int i = 1; i < HD / 64; ++i) M = fmaxf(M, wmax[i]);
+  float o[NG], L = 0.0f;
+#pragma unroll
+  for (int g = 0; g < NG; ++g) o[g] = 0.0f;
+  for (int cb = 0; cb < nc; cb += CB) {
+    const int ce = min(CB, nc - cb);
+    if (cb > 0) __syncthreads();
+    for (int c = tid; c < ce; c += HD) { fs[c] = expf(ml[2 * (cb + c)] - M); ls[c] = ml[2 * (cb + c) + 1]; }
+    __syncthreads();
+    for (int c0 = 0; c0 < ce; c0 += NG) {
+      float pv[NG];
+#pragma unroll
+      for (int g = 0; g < NG; ++g) pv[g] = po[(size_t)min(cb + c0 + g, nc - 1) * HD];
+#pragma unroll
+      for (int g = 0; g < NG; ++g) if (c0 + g < ce) o[g] = fmaf(pv[g], fs[c0 + g], o[g]);
+    }
+    if (tid < NG) for (int c = tid; c < ce; c += NG) L = fmaf(ls[c], fs[c], L);
+  }
+  if (tid < NG) sl[tid] = L;
+  __syncthreads();
+  float ov = o[0]; L = sl[0];
+#pragma unroll
+  for (int g = 1; g < NG; ++g) { ov += o[g]; L += sl[g]; }
+  out[((size_t)ti * a.nh + h) * HD + tid] = (ov / L) * a_sigm(gate);
+}
+
 size_t pyre_kv_bytes(const AttnDev& a, int cap) {
   size_t row = (size_t)a.nkv * a.hd, c = cap;
   return 6 * 256 + c * row * 4 * 2 + c * row / 8 * 4 * 2 + c * row / 32 * 4 * 2;
@@ -780,6 +848,34 @@ int pyre_attn_blk_prep(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const f
     ProfScope ps(ctx, "kv_pack", (double)(pbn - *packed_done) * a.nkv * a.hd * 2 * 4.625); hipLaunchKernelGGL((k_kv_pack<256>), dim3((unsigned)((thr + 127) / 128)), dim3(128), 0, ctx->stream, a, kv, *packed_done, pbn, (const int*)nullptr);
     *packed_done = pbn;
   } PYRE_CHECK_LAUNCH(ctx);
+  return PYRE_OK;
+}
+
+// tokens a launch takes: the partial sums (1 KB a token, head and chunk) stay within about 128 MB, what the last-level cache holds beside the KV cache
+static int attn_blk_tokens(const AttnDev& a, int n, int T) {
+  const size_t per = (size_t)a.nh * ((n + PYRE_ATTN_CHUNK - 1) / PYRE_ATTN_CHUNK) * (a.hd + 2) * 4;
+  const int most = (int)(((size_t)128 << 20) / per) / 8 * 8;
+  return most < 8 ? 8 : (most < T ? most : T);
+}
+size_t pyre_attn_blk_bytes(const AttnDev& a, int n, int T) { return 512 + (size_t)attn_blk_tokens(a, n, T) * a.nh * ((n + PYRE_ATTN_CHUNK - 1) / PYRE_ATTN_CHUNK) * (a.hd + 2) * 4; }
+int pyre_attn_blk_launch(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const float* q, const uint16_t* qh, const float* qsc, const float* qkv, int stride, int start, int T, void* scratch, float* out) {
+  const int G = a.nkv > 0 ? a.nh / a.nkv : 0, n = start + T, sub = attn_blk_tokens(a, n, T);
+  if (a.hd != 256 || (G != 1 && G != 2 && G != 4 && G != 8) || a.nh % a.nkv) return pyre_fail(ctx, PYRE_E_SHAPE, "attention block: head dim %d, group size %d unsupported", a.hd, G);
+  if (T < 1 || start < 0 || n > kv.cap) return pyre_fail(ctx, PYRE_E_STATE, "attention block: positions %d..%d outside the cache (%d)", start, n, kv.cap);
+  const int mc = (n + PYRE_ATTN_CHUNK - 1) / PYRE_ATTN_CHUNK, tp = 16 / G > 8 ? 8 : 16 / G;
+  float* po = (float*)scratch; float* pml = po + (size_t)sub * a.nh * mc * a.hd;
+  for (int i = 0; i < T; i += sub) {
+    const int t = T - i < sub ? T - i : sub, s0 = start + i, nc = (s0 + t + PYRE_ATTN_CHUNK - 1) / PYRE_ATTN_CHUNK;
+    const int off = (((s0 + 1 - a.kv_recent) % tp) + tp) % tp, np = (t + off + tp - 1) / tp;          // the first pass is the shorter one: views of n = kv_recent (mod tp) begin a pass
+    const float* qi = q + (size_t)i * a.nh * a.hd; const uint16_t* hi = qh + (size_t)i * a.nh * 2 * a.hd; const float* ci = qsc + (size_t)i * a.nh;
+    { ProfScope ps(ctx, "attn_blk", 4.0 * t * a.nh * nc * a.hd);
+#define ATT_BLK(GG) hipLaunchKernelGGL((k_attn_blk<256, GG>), dim3((unsigned)(nc * a.nkv * np)), dim3(256 * PYRE_ATTN_NPW), 0, ctx->stream, a, kv, qi, hi, ci, s0, po, pml, mc, t, tp, off, np)
+      switch (G) { case 1: ATT_BLK(1); break; case 2: ATT_BLK(2); break; case 4: ATT_BLK(4); break; default: ATT_BLK(8); }
+#undef ATT_BLK
+    } PYRE_CHECK_LAUNCH(ctx);
+    { ProfScope ps(ctx, "attn_combine", 4.0 * t * a.nh * a.hd * (nc + 2));
+      hipLaunchKernelGGL((k_attn_combine_blk<256>), dim3(a.nh, t), dim3(256), 0, ctx->stream, a, qkv + (size_t)i * stride, stride, s0, po, pml, mc, out + (size_t)i * a.nh * a.hd); } PYRE_CHECK_LAUNCH(ctx);
+  }
   return PYRE_OK;
 }
 

@@ -302,7 +302,7 @@ void   pyre_moe_work_carve(const MoeDev& m, void* base, MoeWork* w);
 // (pyre_moe_out) for a consumer that evaluates moe_out_value itself.
 // Router logits that arrive as K-slice sums (left by the mix that produced x, see HcRoute): logit[t][e] = the slices
 // p[(s*T + t)*r64 + e], s = 0..nsl-1, added in slice order.
-struct RouteSrc { const float* p; int nsl; int r64; const uint32_t* dgx = nullptr; };          // dgx: the activations' digits (digits.h), left by the same mix, or null
+struct RouteSrc { const float* p; int nsl; int r64; const uint32_t* dgx = nullptr; int st = 0; };          // dgx: the activations' digits (digits.h), left by the same mix, or null; st: tokens a slice holds room for (0: T)
 // in_groups (t > 1, y == nullptr, pyre_moe_groups_ok): the down projection leaves the PYRE_MOE_GROUPS group sums of every
 // token in w.parts, group q of token ti at parts + (q*t + ti)*d, instead of the unreduced terms.
 int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const float* x_dev, int t, float* y_dev, const RouteSrc* routed = nullptr, bool in_groups = false);
@@ -321,7 +321,8 @@ bool   pyre_moe_block_ok(const MoeDev& m);
 size_t pyre_moe_block_bytes(const MoeDev& m, int T);
 void   pyre_moe_block_carve(const MoeDev& m, int T, void* base, MoeBlk* b);
 int    pyre_moe_block_zero_rows(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T);
-int    pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_max, int nsl, int r64);
+int    pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_router, int T_max, int nsl, int r64);
+int    pyre_moe_block_window(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const MoeBlk& b, int i0, int t, int nsl, int r64, bool raw);
 // K parts the gate/up dot products are summed in (1 or 2; k_moe_gu)
 int pyre_moe_gu_parts(const MoeDev& m);
 
@@ -383,10 +384,13 @@ void   pyre_blk_mix_carve(const HcDev& h, int T, void* base, BlkMix* b);
 // update in np vectors (0 none; 1: comb [token][d]; PYRE_MOE_GROUPS: comb [group][PYRE_MOE_GROUPS][8][d])
 int pyre_blk_mix_launch(pyre_ctx* ctx, const HcDev& h, const BlkMix& b, const float* x_in, int in_ss, int in_ts, float* x, int T, const float* comb, int np, const float* comb_inj, float eps,
                         float* mixed, float* inj, uint4* op, size_t op_gs, float* inv, int inv_gs);
-int pyre_blk_gemm_launch(pyre_ctx* ctx, const QMatDev& m, const uint4* op, size_t op_gs, const float* inv, int inv_gs, float* y, int ys, int T);      // y[token * ys + row]
+// y[token * ys + row]; parts = PYRE_GEMV_PARTS: y [group][parts][8][ys].  inv_chunks: eight factors a chunk of 128 columns instead of a super-block
+int pyre_blk_gemm_launch(pyre_ctx* ctx, const QMatDev& m, const uint4* op, size_t op_gs, const float* inv, int inv_gs, bool inv_chunks, float* y, int ys, int T, int parts);
 int pyre_blk_op_split_launch(pyre_ctx* ctx, const float* x, int cols, int T, uint4* op, size_t op_gs, float* inv, int inv_gs);      // x [T][cols] -> operand rows, a power of two per 256 columns
 // a Gated DeltaNet layer's raw output o [T][heads * 128] -> RMS norm per head, * sigmoid(z), as operand rows scaled by `up` and / or as f32 rows `out`
 int pyre_blk_gdn_out_launch(pyre_ctx* ctx, const float* o, const float* z, int zs, const float* nw, float eps, int heads, int T, float up, uint4* op, size_t op_gs, float* out);
+// ... and in the per-quarter form of GdnQ: operand rows at op, the factors of a chunk (a head's 128 columns) at inv
+int pyre_blk_gdn_out_q_launch(pyre_ctx* ctx, const float* o, const float* z, int zs, const float* nw, float eps, int heads, int T, uint4* op, size_t op_gs, float* inv, int inv_gs);
 
 // ---- Gated DeltaNet (gdn.hip) -----------------------------------------------------------------------------------------
 struct GdnDev { const float* a; const float* dt; const float* conv_w; const float* norm_w; int nk, nv, dk, dv, conv_k; float eps; };
@@ -408,6 +412,9 @@ size_t pyre_gdn_chunk_bytes(const GdnDev& g, int T);
 void   pyre_gdn_chunk_carve(const GdnDev& g, int T, void* base, GdnChunk* b);
 int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int proj_stride, int T, const float* conv_in, float* conv_out,
                           const float* ssm_in, float* ssm_out, float* oraw);
+// the recurrence token by token instead, the bits of pyre_gdn_launch's per-quarter form (conv_in != conv_out; b.co is all it needs)
+int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int proj_stride, int T, const float* conv_in, float* conv_out,
+                        const float* ssm_in, float* ssm_out, float* oraw);
 
 // ---- gated attention over the KV cache (attn.hip) -----------------------------------------------------------------------
 struct AttnDev { const float* qn; const float* kn; const float* rope_inv; int nh, nkv, hd, n_rot, kv_bits, kv_recent; float eps; float mscale = 1.0f; };   // mscale: YaRN magnitude factor on cos and sin
@@ -441,12 +448,12 @@ size_t pyre_packed_boundary(size_t n_visible, int kv_bits, int recent);
 // qn_ctx::rope_inv (src/qn_ctx.rs:164-185): inverse frequencies [n_rot/2]; YaRN when ctx > ctx_train > 0; returns mscale
 float pyre_rope_table(int n_rot, float base, int ctx_train, int ctx, float* inv_host);
 
-// Queries start .. start + T - 1 of a prompt over the cache (attn_prompt.hip).  pyre_attn_blk_prep: K and V of those positions into
-// the cache, the packing, and the rotated queries as halves qh [T][nh][2][hd] with qsc [T][nh] (q: their f32 rows, or null);
-// pyre_attn_prompt_launch: out [T][nh*hd], scratch of pyre_attn_prompt_bytes.
+// Queries start .. start + T - 1 of a prompt's block over the cache.  pyre_attn_blk_prep: K and V of those positions into the cache,
+// the packing, and the rotated queries q [T][nh][hd], as halves qh [T][nh][2][hd] with qsc [T][nh]; pyre_attn_blk_launch: out
+// [T][nh*hd], scratch of pyre_attn_blk_bytes(a, start + T, T) or more.  A token's bits are those of pyre_attn_launch.
 int pyre_attn_blk_prep(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const float* qkv, int stride, int start, int T, int* packed_done, float* q, uint16_t* qh, float* qsc);
-size_t pyre_attn_prompt_bytes(const AttnDev& a, int start, int T);
-int pyre_attn_prompt_launch(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const uint16_t* qh, const float* qsc, const float* qkv, int stride, int start, int T, void* scratch, float* out);
+size_t pyre_attn_blk_bytes(const AttnDev& a, int n, int T);
+int pyre_attn_blk_launch(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const float* q, const uint16_t* qh, const float* qsc, const float* qkv, int stride, int start, int T, void* scratch, float* out);
 
 // ---- QSA sparse indexer (qsa.hip), qwen4exp_gguf.rs:1565-1599 ------------------------------------------------------------
 // Blocks of `ratio` tokens; a query that sees more than budget + ratio - 1 positions attends to the budget / ratio

@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256) void k_gdnc_conv(GdnDev p, const float* __rest
   if (!in) return;
 #pragma unroll
   for (int i = 0; i < 16; ++i) co[(size_t)(t0 + i) * ch + c] = v[i];
-  if (c >= nqk && c < 2 * nqk) {
+  if (kt && c >= nqk && c < 2 * nqk) {
     float* k2 = kt + (((size_t)(t0 / C) * p.nk + (c - nqk) / DK) * DK + (c - nqk) % DK) * C + t0 % C;
 #pragma unroll
     for (int i = 0; i < 16; i += 4) *(float4*)(k2 + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
@@ -216,6 +216,82 @@ __global__ __launch_bounds__(256) void k_gdnc_scan(GdnDev p, const float* __rest
   for (int i = tid; i < DK * 16; i += 256) sout[(size_t)(i >> 4) * p.dv + (i & 15)] = St[i & 15][i >> 4];
 }
 
+// ---- the recurrence token by token, the bits of k_gdn_delta_q -------------------------------------------------------------------
+// A prompt of the model takes this one: its state and outputs are then those of decoding the tokens in windows, to the bit, so
+// that no token's expert choice tips with the path the prompt took.  k_gdn_delta_q keeps 32 columns a workgroup, eight rows a
+// thread, and adds the sixteen row groups' sums through shared memory behind a barrier: 0.9 us a token.  Here a wave keeps
+// four columns, a row of sixteen lanes (a lane: eight rows) each: the sums meet in the same order by DPP row shifts
+// (x <- p + x of the lane before, fifteen times: the last lane has ((p0 + p1) + p2) + ..), without a barrier, and the
+// output's sums of one token run in the wait slots of the next token's.  About 100 vector instructions a token, one wave a SIMD
+// for 32 heads (the recurrence is a chain, so further waves would only share the SIMD).
+// grid (nv, 8), 4 waves: workgroup (h, y) columns 16 y .. of head h.  The keys, queries (normalised, co of k_gdnc_conv), values and gate
+// inputs of sixteen tokens at a time go through shared memory, the next sixteen in registers meanwhile.
+__device__ __forceinline__ float row_shr1(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x111, 0xf, 0xf, true)); }
+__device__ __forceinline__ float row_last(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x15F, 0xf, 0xf, true)); }
+__global__ __launch_bounds__(256) void k_gdn_rec(GdnDev p, const float* __restrict__ co, const float* __restrict__ proj, int stride, int T, const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
+  constexpr int TB = 16, R = 8;
+  __shared__ __align__(16) float4 kq[2][TB][2][2][16];          // [buffer][token][k, q][rows 0-3, 4-7 of a row group][row group]
+  __shared__ float vs[2][TB][16], gs[2][TB], bs[2][TB], os[2][TB][16];
+  const int h = blockIdx.x, cb = blockIdx.y * 16, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, rg = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), jl = wave * 4 + (lane >> 4), col = cb + jl;
+  const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv, w = p.nv * p.dv;
+  const float dtb = p.dt[h], ah = p.a[h];
+  const size_t so = ((size_t)h * DK + rg * R) * p.dv + col;
+  float S[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) S[r] = ssm_in[so + (size_t)r * p.dv];
+  float4 f0, f1, f2, f3; float fv, fa = 0.0f, fb = 0.0f;
+  auto src = [&](int t0, int i) { const int e = tid + 256 * i, t = min(t0 + (e >> 6), T - 1), f = e & 63; return *(const float4*)(co + (size_t)t * ch + (f < 32 ? nqk : 0) + kh * DK + 4 * (f & 31)); };
+  auto fetch = [&](int t0) {          // token t0 + e / 64's float4 e % 64: 32 of k, 32 of q (past the end: the last token's again)
+    f0 = src(t0, 0); f1 = src(t0, 1); f2 = src(t0, 2); f3 = src(t0, 3);
+    fv = co[(size_t)min(t0 + (tid >> 4), T - 1) * ch + 2 * nqk + (size_t)h * p.dv + cb + (tid & 15)];
+    if (tid < TB) { const float* pr = proj + (size_t)min(t0 + tid, T - 1) * stride + ch + w; fa = pr[p.nv + h]; fb = pr[h]; }
+  };
+  auto put = [&](int buf, int i, const float4& f) { const int e = tid + 256 * i, c = e & 63; kq[buf][e >> 6][c >> 5][c & 1][(c & 31) >> 1] = f; };
+  auto store = [&](int buf) {
+    put(buf, 0, f0); put(buf, 1, f1); put(buf, 2, f2); put(buf, 3, f3);
+    vs[buf][tid >> 4][tid & 15] = fv;
+    if (tid < TB) { gs[buf][tid] = expf(p_softplus(fa + dtb) * ah); bs[buf][tid] = p_sigm(fb); }
+  };
+  struct Tok { float4 k0, k1, q0, q1; float g, b, v; };
+  auto get = [&](int buf, int t) { return Tok{kq[buf][t][0][0][rg], kq[buf][t][0][1][rg], kq[buf][t][1][0][rg], kq[buf][t][1][1][rg], gs[buf][t], bs[buf][t], vs[buf][t][jl]}; };
+  fetch(0); store(0);
+  lds_barrier();
+  for (int t0 = 0, buf = 0; t0 < T; t0 += TB, buf ^= 1) {
+    if (t0 + TB < T) fetch(t0 + TB);
+    const int n = min(TB, T - t0);
+    float po = 0.0f;          // the previous token's output terms
+    auto step = [&](const Tok& c, int t) {
+      const float k[R] = {c.k0.x, c.k0.y, c.k0.z, c.k0.w, c.k1.x, c.k1.y, c.k1.z, c.k1.w}, q[R] = {c.q0.x, c.q0.y, c.q0.z, c.q0.w, c.q1.x, c.q1.y, c.q1.z, c.q1.w};
+      float pm = 0.0f;
+#pragma unroll
+      for (int r = 0; r < R; ++r) { S[r] *= c.g; pm += S[r] * k[r]; }
+      float m = pm, o = po;
+#pragma unroll
+      for (int i = 0; i < 15; ++i) { m = pm + row_shr1(m); o = po + row_shr1(o); }
+      if (rg == 15) os[buf][max(t - 1, 0)][jl] = o;          // (the first token's writes nothing of use: the next one overwrites it)
+      const float delta = (c.v - row_last(m)) * c.b;
+      po = 0.0f;
+#pragma unroll
+      for (int r = 0; r < R; ++r) { S[r] += k[r] * delta; po += S[r] * q[r]; }
+    };
+    // a token ahead: the wave is alone on its SIMD, nothing else hides the reads; two sets of registers taking turns
+    Tok x0 = get(buf, 0), x1;
+    int t = 0;
+    for (; t + 1 < n; t += 2) { x1 = get(buf, t + 1); step(x0, t); x0 = get(buf, min(t + 2, n - 1)); step(x1, t + 1); }
+    if (t < n) step(x0, t);
+    { float o = po;
+#pragma unroll
+      for (int i = 0; i < 15; ++i) o = po + row_shr1(o);
+      if (rg == 15) os[buf][n - 1][jl] = o; }
+    if (t0 + TB < T) store(buf ^ 1);
+    lds_barrier();
+    if ((tid >> 4) < n) oraw[(size_t)(t0 + (tid >> 4)) * w + (size_t)h * p.dv + cb + (tid & 15)] = os[buf][tid >> 4][tid & 15];
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) ssm_out[so + (size_t)r * p.dv] = S[r];
+}
+
 }  // namespace
 
 size_t pyre_gdn_chunk_bytes(const GdnDev& g, int T) {
@@ -238,5 +314,18 @@ int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, con
     hipLaunchKernelGGL(k_gdnc_chunk, dim3(nch, g.nv), dim3(256), 0, ctx->stream, g, b.co, proj, stride, T, b.w, b.u, b.p, b.dec); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "gdn_prompt_scan", 8.0 * g.nv * g.dk * g.dv + 4.0 * T * g.nv * (4.0 * DK + C));
     hipLaunchKernelGGL(k_gdnc_scan, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, b.kt, b.w, b.u, b.p, b.dec, nch, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
+  return PYRE_OK;
+}
+
+// the same steps with the recurrence token by token, bit for bit that of the windows' kernels (pyre_gdn_launch with GdnQ); ssm_in == ssm_out is fine, conv_in == conv_out is not
+int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int stride, int T, const float* conv_in, float* conv_out, const float* ssm_in, float* ssm_out, float* oraw) {
+  if (g.dk != 128 || g.dv != 128) return pyre_fail(ctx, PYRE_E_SHAPE, "gdn prompt: head dims %dx%d unsupported (128x128 only)", g.dk, g.dv);
+  if (T < 1 || g.conv_k < 1 || g.conv_k > 8 || conv_in == conv_out) return pyre_fail(ctx, PYRE_E_ARG, "gdn prompt: %d tokens, %d taps", T, g.conv_k);
+  const int ch = 2 * g.nk * g.dk + g.nv * g.dv, Tp = (T + 15) / 16 * 16;
+  { ProfScope ps(ctx, "gdn_prompt_conv", 8.0 * T * ch);
+    if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr);
+    else hipLaunchKernelGGL(k_gdnc_conv<0>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr); } PYRE_CHECK_LAUNCH(ctx);
+  { ProfScope ps(ctx, "gdn_prompt_rec", 8.0 * g.nv * g.dk * g.dv + 4.0 * T * (ch + 2.0 * g.nv * g.dv));
+    hipLaunchKernelGGL(k_gdn_rec, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, proj, stride, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
   return PYRE_OK;
 }

@@ -111,3 +111,44 @@ template <int G> __device__ __forceinline__ void chunk_mac(const WBuf<G>& wb, co
   }
 }
 
+// ---- the same product with the decoding apart, for a weight that meets several groups of sixteen activation rows -----------------
+// sixteen bytes a lane from memory straight into shared memory: lane l's land at dst + 16 l (dst: the wave's own, uniform)
+__device__ __forceinline__ void lds_fetch16(const void* src, void* dst) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+// workgroup barrier behind lds_fetch16: a wave's own fetches have landed before it arrives
+__device__ __forceinline__ void lds_fetch_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// A wave's 128-column chunk of one row group, decoded: four matrix operands and the row's scale.
+struct WDec { v8h b[4]; float d; };
+__device__ __forceinline__ void decode_chunk(const uint4& w, const uint2& h, int c, const NibK& nk, WDec& o) {
+  const int sh = 8 * (c & 1);
+  const v2h four = {(_Float16)4.0f, (_Float16)4.0f}, m62 = {(_Float16)-62.0f, (_Float16)-62.0f}, m235 = {(_Float16)-23.5f, (_Float16)-23.5f};
+  const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
+  const uint32_t hs = h.y >> sh;
+  const uint32_t np0 = ((hs << 6) & nk.K) | nk.E, np1 = ((hs << 2) & nk.K) | nk.E;
+  v2h s2[2], s47[2];
+  s2[0] = __builtin_elementwise_fma(__builtin_bit_cast(v2h, np0), four, m62); s2[1] = __builtin_elementwise_fma(__builtin_bit_cast(v2h, np1), four, m62);
+  s47[0] = s2[0] * m235; s47[1] = s2[1] * m235;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const v2h vs2 = {s2[s >> 1][s & 1], s2[s >> 1][s & 1]}, vs47 = {s47[s >> 1][s & 1], s47[s >> 1][s & 1]};
+    struct U4 { uint32_t x[4]; } q; uint32_t p[4];
+    nib_f16(wd[s], nk, p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) q.x[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(v2h, p[i]), vs2, vs47));
+    o.b[s] = __builtin_bit_cast(v8h, q);
+  }
+  o.d = h2f_bits(h.x & 0xFFFFu);
+}
+// tot += the chunk's product, the two halves of the lane's two tokens apart, as chunk_mac forms them
+__device__ __forceinline__ void chunk_add(const WDec& w, const v8h (&a)[4], float ai0, float ai1, v4f& tot) {
+  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[s], w.b[s], acc, 0, 0, 0);
+  const float d0 = w.d * ai0, d1 = w.d * ai1;
+  tot[0] = fmaf(acc[0], d0, tot[0]); tot[1] = fmaf(acc[1], d0, tot[1]); tot[2] = fmaf(acc[2], d1, tot[2]); tot[3] = fmaf(acc[3], d1, tot[3]);
+}
+__device__ __forceinline__ float halves0(const v4f& t) { return t[0] + t[1] * (1.0f / 2048.0f); }
+__device__ __forceinline__ float halves1(const v4f& t) { return t[2] + t[3] * (1.0f / 2048.0f); }

@@ -511,29 +511,37 @@ static int prompt_pipe_state(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, 
 // ---- a long prompt layer by layer ---------------------------------------------------------------------------------------------
 // Windows of eight tokens share nothing but what fits beside each other on the chip: every window decodes every weight again, and
 // its FFN's 74 of 512 experts.  A call of 72 tokens or more is therefore taken in blocks of up to 2048 tokens, layer by layer, a
-// launch a step for all of a block's tokens: the mixes and projections (prompt.hip), the Gated DeltaNet in chunks of 64
-// (gdn_prefill.hip), the attention (attn_prompt.hip), the FFN grouped by expert (moe.hip).  Against windows everything but
-// the recurrence's and the attention's order of sums and the FFN's operand form is the same arithmetic; logits agree to
-// rounding.  Blocks are cut at multiples of 128 tokens from the call's start, so that neither the chunks of the recurrence
-// nor the tiles of the attention -- hence not a bit of a token -- depend on the cutting.
+// launch a step for all of a block's tokens: the mixes and projections (prompt.hip), the Gated DeltaNet's recurrence
+// (gdn_prefill.hip), the attention (k_attn_blk), the FFN grouped by expert (moe.hip).  Every sum is formed in the order of the
+// windows' launches, so a token has a window's bits and the cutting never shows; the one exception is the grouped FFN, whose
+// operands are f16 halves instead of fixed-point digits: it takes the whole groups of eight in front of the call's last eight
+// tokens, the last 8 .. 15 tokens' FFN goes through the windows' launches.
 // For models whose every layer qualifies (prompt_block_ok); PYRE_PROMPT_BLOCK=0 switches it off, PYRE_PROMPT_PAIRS=0 halves the blocks.
-#define PROMPT_BLOCK_MIN 72
+#define PROMPT_BLOCK_MIN 64
 #define PROMPT_BLOCK_MAX 2048
 static bool fuse_aop_on() { const char* e = getenv("PYRE_AOP_SPLIT"); return !(e && *e && atoi(e) != 0); }
+static bool outp_in_parts(const Layer& L, int d) { return pyre_gemv_parts_ok(L.outp) && (int)L.outp.rows == d && L.hcf.di.fmt == FMT_IQ3_S; }
+// A Gated DeltaNet layer whose output projection is on the matrix cores runs its recurrence on nv x 4 workgroups and leaves
+// the head norm to that projection (GdnQ / PyreAop::sq) -- in every call that touches the layer's state, the re-run of
+// pyre_spec_keep included: the two forms of the kernel round the state differently.  PYRE_GDN_Q=0: nv workgroups.
+static bool gdn_q_on(const pyre_model* m, const Layer& L) {
+  const char* e = getenv("PYRE_GDN_Q");
+  return !(e && *e && atoi(e) == 0) && fuse_aop_on() && !L.full && L.outp.fmt == FMT_IQ3_S_M && L.gdn.dv == 128 && L.gdn.dk == 128 && L.outp.cols == L.gdn.nv * 128 && m->gdn_sq != nullptr;
+}
 static bool prompt_block_ok(const pyre_model* m) {
   if (!prompt_block_env()) return false;
   const pyre_model_cfg& c = m->c;
   if (m->n_ple > 0 || c.top_k > PYRE_MOE_KMAX || c.d % 256 || c.conv_k < 2 || c.conv_k > 8 || !pyre_blk_mix_ok(m->head)) return false;
   for (int il = 0; il < c.n_layers; ++il) { const Layer& L = m->layers[il]; const MoeDev& m0 = m->layers[0].moe;
     if (!pyre_moe_block_ok(L.moe) || (L.moe.router.fmt != FMT_BF16 && L.moe.router.fmt != FMT_F32) || L.moe.router.U != c.d / 64 || L.moe.router.tiles != m0.router.tiles || L.moe.ff != m0.ff || L.moe.sf != m0.sf || L.moe.top_k != m0.top_k || L.moe.n_exp != m0.n_exp ||
-        !pyre_blk_mix_ok(L.hca) || !pyre_blk_mix_ok(L.hcf) || L.proj.fmt != FMT_IQ3_S_M || L.outp.fmt != FMT_IQ3_S_M || L.proj.cols % 256 || L.outp.cols % 256 || L.outp.rows != c.d || (!L.full && !L.gdn_ainv)) return false; }
+        !pyre_blk_mix_ok(L.hca) || !pyre_blk_mix_ok(L.hcf) || L.proj.fmt != FMT_IQ3_S_M || L.outp.fmt != FMT_IQ3_S_M || L.proj.cols % 256 || L.outp.cols % 256 || L.outp.rows != c.d || !outp_in_parts(L, c.d) || (!L.full && !gdn_q_on(m, L))) return false; }
   return true;
 }
 struct PromptBlk {
   pyre_ctx* ctx = nullptr; void* mem = nullptr; int T_max = 0; size_t blocks = 0;      // room for T_max tokens a block; blocks: pyre_model_prompt_blocks
   float *emb = nullptr, *x = nullptr, *mixed = nullptr, *inj_a = nullptr, *inj_f = nullptr, *proj = nullptr, *o = nullptr, *core = nullptr, *inv = nullptr; uint4* op = nullptr; uint32_t* ids = nullptr;
-  BlkMix mix{}; MoeBlk moe{}; GdnChunk gdn{}; uint16_t* qh = nullptr; float* qsc = nullptr;
-  void* att = nullptr; size_t att_bytes = 0;             // the cache's fragments (grows with the context)
+  BlkMix mix{}; MoeBlk moe{}; GdnChunk gdn{}; float* q = nullptr; uint16_t* qh = nullptr; float* qsc = nullptr;
+  void* att = nullptr; size_t att_bytes = 0;             // the attention's partial sums (grows with the context)
 };
 size_t prompt_blk_count(const PromptBlk* B) { return B->blocks; }
 void prompt_blk_free(PromptBlk* B) {
@@ -548,10 +556,9 @@ static int prompt_blk_get(pyre_ctx* ctx, const pyre_model* m, int T, int n, Prom
   pyre_model* mm = const_cast<pyre_model*>(m); const pyre_model_cfg& c = m->c;
   if (!mm->blk) { mm->blk = new PromptBlk(); mm->blk->ctx = ctx; }
   PromptBlk* B = mm->blk; *out = B;
-  T = (T + 127) / 128 * 128;
   if (B->T_max < T) {
     if (B->mem) { PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); (void)hipFree(B->mem); B->mem = nullptr; B->T_max = 0; }
-    T = T <= 512 ? 512 : PROMPT_BLOCK_MAX;
+    T = T <= 512 ? 512 : PROMPT_BLOCK_MAX + 16;
     const MoeDev& m0 = m->layers[0].moe; const Layer* lin = nullptr; for (const Layer& L : m->layers) if (!L.full) lin = &L;
     const size_t t = T, d = c.d, nq = (size_t)c.n_head * c.hd, cmax = std::max((size_t)c.lin_nv * c.lin_dv, nq), omax = std::max(d, cmax), pmax = std::max(m->pw_lin, m->pw_attn);
     HcDev hmax = m->layers[0].hca;
@@ -560,10 +567,10 @@ static int prompt_blk_get(pyre_ctx* ctx, const pyre_model* m, int T, int n, Prom
       uint8_t* p = (uint8_t*)B->mem; size_t sum = 0;
       auto take = [&](size_t bytes) { void* r = p; bytes = al256(bytes); if (pass) p += bytes; sum += bytes; return r; };
       B->emb = (float*)take(4 * t * d); B->x = (float*)take(4 * t * c.hc * d); B->mixed = (float*)take(4 * t * d); B->inj_a = (float*)take(4 * t * c.hc); B->inj_f = (float*)take(4 * t * c.hc);
-      B->proj = (float*)take(4 * t * pmax); B->o = (float*)take(4 * t * d); B->core = (float*)take(4 * t * cmax); B->op = (uint4*)take(4 * t * omax); B->inv = (float*)take(4 * t * (omax / 256)); B->ids = (uint32_t*)take(4 * t);
+      B->proj = (float*)take(4 * t * pmax); B->o = (float*)take(4 * PYRE_GEMV_PARTS * t * d); B->core = (float*)take(4 * t * cmax); B->op = (uint4*)take(4 * t * omax); B->inv = (float*)take(4 * t * (omax / 128)); B->ids = (uint32_t*)take(4 * t);
       void* mx = take(pyre_blk_mix_bytes(hmax, T)); void* mo = take(pyre_moe_block_bytes(m0, T)); void* gd = take(lin ? pyre_gdn_chunk_bytes(lin->gdn, T) : 0);
       float* rpart = (float*)take(4 * rp); float* parts = (float*)take(4 * PYRE_MOE_GROUPS * t * d);
-      B->qh = (uint16_t*)take(2 * 2 * t * nq); B->qsc = (float*)take(4 * t * c.n_head);
+      B->q = (float*)take(4 * t * nq); B->qh = (uint16_t*)take(2 * 2 * t * nq); B->qsc = (float*)take(4 * t * c.n_head);
       if (!pass) { PYRE_HIP(ctx, hipMalloc(&B->mem, sum + 256)); continue; }
       pyre_blk_mix_carve(hmax, T, mx, &B->mix); pyre_moe_block_carve(m0, T, mo, &B->moe); if (lin) pyre_gdn_chunk_carve(lin->gdn, T, gd, &B->gdn);
       B->moe.x = B->mixed; B->moe.rpart = rpart; B->moe.parts = parts; B->moe.wr = 8 * (d / 64) * m0.router.tiles * 64;
@@ -574,7 +581,7 @@ static int prompt_blk_get(pyre_ctx* ctx, const pyre_model* m, int T, int n, Prom
   }
   if (m->n_attn > 0 && !m->has_idx) {
     AttnDev a0{nullptr, nullptr, nullptr, c.n_head, c.n_kv, c.hd, c.n_rot, c.kv_bits, c.kv_recent, c.eps};
-    const size_t need = pyre_attn_prompt_bytes(a0, std::max(0, n - B->T_max), B->T_max);
+    const size_t need = pyre_attn_blk_bytes(a0, n, std::min(n, B->T_max));
     if (B->att_bytes < need) {
       if (B->att) { PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); (void)hipFree(B->att); B->att = nullptr; B->att_bytes = 0; }
       PYRE_HIP(ctx, hipMalloc(&B->att, need + need / 4)); B->att_bytes = need + need / 4;
@@ -582,19 +589,21 @@ static int prompt_blk_get(pyre_ctx* ctx, const pyre_model* m, int T, int n, Prom
   }
   return PYRE_OK;
 }
-// T tokens (ids on the host) behind the state's length; head: the last token's logits to m->logits
-static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBlk* B, const uint32_t* ids, int T, bool head) {
-  const pyre_model_cfg& c = m->c; const int d = c.d, hc = c.hc, start = s->len, G = (T + 7) / 8; int rc;
+// T tokens (ids on the host) behind the state's length; tail: the last of them whose FFN takes the windows' launches (0: none;
+// T - tail is a multiple of eight); head: the last token's logits to m->logits
+static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBlk* B, const uint32_t* ids, int T, int tail, bool head) {
+  const pyre_model_cfg& c = m->c; const int d = c.d, hc = c.hc, start = s->len, Tb = T - tail; int rc;
   PYRE_HIP(ctx, hipMemcpyAsync(B->ids, ids, (size_t)T * 4, hipMemcpyHostToDevice, ctx->stream));
   if (s->tokens_dev) PYRE_HIP(ctx, hipMemcpyAsync(s->tokens_dev + start, B->ids, (size_t)T * 4, hipMemcpyDeviceToDevice, ctx->stream));      // (a state with a drafter keeps the history)
   if ((rc = pyre_row_launch(ctx, m->embd, B->ids, T, B->emb, d))) return rc;
   const float* xin = B->emb; int in_ss = 0, in_ts = d, np = 0; const float* comb = nullptr; const float* cinj = nullptr;
   auto gs = [](int cols) { return (size_t)cols * 2; }; auto is = [](int cols) { return cols / 256 * 8; };
+  const int r64 = m->layers[0].moe.router.tiles * 64;
   for (int il = 0; il < c.n_layers; ++il) {
     const Layer& L = m->layers[il]; const int pw = L.full ? m->pw_attn : m->pw_lin, oc = L.outp.cols;
     if ((rc = pyre_blk_mix_launch(ctx, L.hca, B->mix, xin, in_ss, in_ts, B->x, T, comb, np, cinj, c.eps, B->mixed, B->inj_a, B->op, gs(d), B->inv, is(d)))) return rc;
     xin = B->x; in_ss = d; in_ts = hc * d;
-    if ((rc = pyre_blk_gemm_launch(ctx, L.proj, B->op, gs(d), B->inv, is(d), B->proj, pw, T))) return rc;
+    if ((rc = pyre_blk_gemm_launch(ctx, L.proj, B->op, gs(d), B->inv, is(d), false, B->proj, pw, T, 1))) return rc;
     if (L.full) {
       const int ai = L.mix_index;
       if (m->has_idx) {          // a sparse indexer selects per window of eight, behind the windows before it
@@ -604,30 +613,34 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
           if ((rc = pyre_attn_launch_sel(ctx, L.attn, s->kv[ai], s->aw, pj, pw, start + i, t, &s->packed[ai], B->core + (size_t)i * oc, nullptr, &s->qw))) return rc;
         }
       } else {
-        if ((rc = pyre_attn_blk_prep(ctx, L.attn, s->kv[ai], B->proj, pw, start, T, &s->packed[ai], nullptr, B->qh, B->qsc))) return rc;
-        if (pyre_attn_prompt_bytes(L.attn, start, T) > B->att_bytes) return pyre_fail(ctx, PYRE_E_STATE, "forward: attention scratch of %zu bytes is too small", B->att_bytes);
-        if ((rc = pyre_attn_prompt_launch(ctx, L.attn, s->kv[ai], B->qh, B->qsc, B->proj, pw, start, T, B->att, B->core))) return rc;
+        if ((rc = pyre_attn_blk_prep(ctx, L.attn, s->kv[ai], B->proj, pw, start, T, &s->packed[ai], B->q, B->qh, B->qsc))) return rc;
+        if (pyre_attn_blk_bytes(L.attn, start + T, T) > B->att_bytes) return pyre_fail(ctx, PYRE_E_STATE, "forward: attention scratch of %zu bytes is too small", B->att_bytes);
+        if ((rc = pyre_attn_blk_launch(ctx, L.attn, s->kv[ai], B->q, B->qh, B->qsc, B->proj, pw, start, T, B->att, B->core))) return rc;
       }
       if ((rc = pyre_blk_op_split_launch(ctx, B->core, oc, T, B->op, gs(oc), B->inv, is(oc)))) return rc;
-      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, is(oc), B->o, d, T))) return rc;
+      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, is(oc), false, B->o, d, T, PYRE_GEMV_PARTS))) return rc;
     } else {
       const int li = L.mix_index, b = s->cur[li], nb = b ^ 1;
-      if ((rc = pyre_gdn_chunk_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], B->core))) return rc;
+      if ((rc = pyre_gdn_rec_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], B->core))) return rc;
       s->cur[li] = nb;
-      if ((rc = pyre_blk_gdn_out_launch(ctx, B->core, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, L.gdn_up, B->op, gs(oc), nullptr))) return rc;
-      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), L.gdn_ainv, 0, B->o, d, T))) return rc;
+      if ((rc = pyre_blk_gdn_out_q_launch(ctx, B->core, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, B->op, gs(oc), B->inv, oc / 16))) return rc;
+      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, oc / 16, true, B->o, d, T, PYRE_GEMV_PARTS))) return rc;
     }
-    if ((rc = pyre_blk_mix_launch(ctx, L.hcf, B->mix, xin, in_ss, in_ts, B->x, T, B->o, 1, B->inj_a, c.eps, B->mixed, B->inj_f, nullptr, 0, nullptr, 0))) return rc;
-    if (il == c.n_layers - 1 && !head) break;          // nobody reads the last layer's FFN
-    if ((rc = pyre_moe_block_launch(ctx, L.moe, B->moe, T, B->T_max, d / 64, L.moe.router.tiles * 64))) return rc;
+    if ((rc = pyre_blk_mix_launch(ctx, L.hcf, B->mix, xin, in_ss, in_ts, B->x, T, B->o, PYRE_GEMV_PARTS, B->inj_a, c.eps, B->mixed, B->inj_f, nullptr, 0, nullptr, 0))) return rc;
+    const bool end = il == c.n_layers - 1;
+    if (end && !head) break;          // nobody reads the last layer's FFN
+    if ((rc = pyre_moe_block_launch(ctx, L.moe, B->moe, end ? 0 : Tb, T, B->T_max, d / 64, r64))) return rc;
+    for (int i = end ? (T - 1) / 8 * 8 : Tb; i < T; i += 8) if ((rc = pyre_moe_block_window(ctx, L.moe, m->mw, B->moe, i, std::min(8, T - i), d / 64, r64, end))) return rc;
     comb = B->moe.parts; np = PYRE_MOE_GROUPS; cinj = B->inj_f;
   }
   s->len = start + T;
   if (!head) return PYRE_OK;
-  const int g = G - 1, tl = T - 8 * g;          // the head of the last group's tokens; the last one's logits
-  if ((rc = pyre_blk_mix_launch(ctx, m->head, B->mix, B->x + (size_t)8 * g * hc * d, d, hc * d, B->x + (size_t)8 * g * hc * d, tl, B->moe.parts + (size_t)g * PYRE_MOE_GROUPS * 8 * d, PYRE_MOE_GROUPS,
-                                B->inj_f + (size_t)8 * g * hc, c.eps, B->mixed, B->inj_a, nullptr, 0, nullptr, 0))) return rc;
-  return pyre_gemv_launch(ctx, m->out, B->mixed + (size_t)(tl - 1) * d, 1, m->logits);
+  // the last token alone: its pending update and the head, as a window's finish()
+  const MoeOut mol = pyre_moe_out(m->layers.back().moe, m->mw, (T - 1) % 8); const size_t last = (size_t)(T - 1) * hc * d;
+  const bool fused = fuse_aop_on() && m->out.fmt == FMT_IQ3_S_M && m->out.cols == d && pyre_hc_aop_ok(m->head);
+  const AopOut aout{m->aop, m->aop_inv, d / 256}; const PyreAop aop{(const uint4*)m->aop, m->aop_inv};
+  if ((rc = pyre_hc_mix_launch(ctx, m->head, m->hw, B->x + last, d, hc * d, m->x, 1, nullptr, &mol, B->inj_f + (size_t)(T - 1) * hc, c.eps, m->hbuf, m->inj_a, nullptr, 1, fused ? &aout : nullptr))) return rc;
+  return pyre_gemv_launch(ctx, m->out, m->hbuf, 1, m->logits, fused ? &aop : nullptr);
 }
 
 namespace {
@@ -654,16 +667,8 @@ __global__ __launch_bounds__(256) void k_ring_store(const float* __restrict__ x,
 }
 int mtp_window_of(const pyre_mtp* m);
 
-bool outp_in_parts(const Layer& L, int d) { return pyre_gemv_parts_ok(L.outp) && (int)L.outp.rows == d && L.hcf.di.fmt == FMT_IQ3_S; }
 
 // One window of t <= 8 tokens (ids in m->ids unless from_best).
-// A Gated DeltaNet layer whose output projection is on the matrix cores runs its recurrence on nv x 4 workgroups and leaves
-// the head norm to that projection (GdnQ / PyreAop::sq) -- in every call that touches the layer's state, the re-run of
-// pyre_spec_keep included: the two forms of the kernel round the state differently.  PYRE_GDN_Q=0: nv workgroups.
-static bool gdn_q_on(const pyre_model* m, const Layer& L) {
-  const char* e = getenv("PYRE_GDN_Q");
-  return !(e && *e && atoi(e) == 0) && fuse_aop_on() && !L.full && L.outp.fmt == FMT_IQ3_S_M && L.gdn.dv == 128 && L.gdn.dk == 128 && L.outp.cols == L.gdn.nv * 128 && m->gdn_sq != nullptr;
-}
 // One window of t <= 8 tokens as an object: begin() (embedding rows, history, n-gram rows), per layer front(il) (everything up to
 // the FFN mix, whose output is the FFN's input) and moe(il), finish() (bookkeeping, head).  run_window is the four in order.
 struct WinRun {
@@ -841,16 +846,16 @@ int pyre_forward(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, const uint32
   s->last_window = 0;
   int i_first = 0;
   const bool windows_only = [] { const char* e = getenv("PYRE_PROMPT_WINDOWS"); return e && *e && atoi(e) != 0; }();      // (read per call: 1 = this call in windows, whatever layouts the model keeps)
-  // (with a drafter the last tokens, whose residual streams the drafter's ring keeps, take the windows' path)
-  const int nblk_tok = !s->mtp ? n : std::max(0, n - 8 - mtp_window_of(s->mtp)) / 8 * 8;
-  if (!windows_only && nblk_tok >= PROMPT_BLOCK_MIN && prompt_block_ok(m)) {
+  // whole groups of eight in front of the call's last tokens; those follow in the last block, with a drafter, whose ring keeps their residual streams, in windows
+  const int nblk_ffn = std::max(0, n - 8 - (s->mtp ? mtp_window_of(s->mtp) : 0)) / 8 * 8, nblk_tok = s->mtp ? nblk_ffn : n;
+  if (!windows_only && nblk_ffn >= PROMPT_BLOCK_MIN && prompt_block_ok(m)) {
     const bool pairs = [] { const char* e = getenv("PYRE_PROMPT_PAIRS"); return !(e && *e && atoi(e) == 0); }();      // PYRE_PROMPT_PAIRS=0: blocks of up to 1024 tokens instead of 2048
-    const int most = pairs ? PROMPT_BLOCK_MAX : PROMPT_BLOCK_MAX / 2, nb = (nblk_tok + most - 1) / most, each = ((nblk_tok + nb - 1) / nb + 127) / 128 * 128;
+    const int most = pairs ? PROMPT_BLOCK_MAX : PROMPT_BLOCK_MAX / 2, nb = (nblk_ffn + most - 1) / most, groups = nblk_ffn / 8;      // blocks of (nearly) equal size, the last with up to fifteen tokens more
     PromptBlk* B = nullptr;
-    if ((rc = prompt_blk_get(ctx, m, std::min(each, nblk_tok), s->len + n, &B))) return rc;
-    while (i_first < nblk_tok) {
-      const int T = std::min(each, nblk_tok - i_first); const bool head = logits_host && i_first + T == n;
-      if ((rc = run_block(ctx, m, s, B, ids + i_first, T, head))) { s->broken = true; (void)hipStreamSynchronize(ctx->stream); return rc; }
+    if ((rc = prompt_blk_get(ctx, m, (groups + nb - 1) / nb * 8 + nblk_tok - nblk_ffn, s->len + n, &B))) return rc;
+    for (int k = 0; k < nb; ++k) {
+      const int tail = k + 1 == nb ? nblk_tok - nblk_ffn : 0, T = 8 * (int)((int64_t)groups * (k + 1) / nb - (int64_t)groups * k / nb) + tail; const bool head = logits_host && i_first + T == n;
+      if ((rc = run_block(ctx, m, s, B, ids + i_first, T, tail, head))) { s->broken = true; (void)hipStreamSynchronize(ctx->stream); return rc; }
       i_first += T;
     }
     // what pyre_model_prompt_blocks counts: the whole windows in front of the call's last eight tokens in blocks of at most 128, an even number of them when taken in pairs

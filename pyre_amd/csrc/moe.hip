@@ -474,7 +474,7 @@ int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const floa
   if (routed && (routed->nsl < 1 || routed->nsl > 64 || routed->r64 < m.n_exp)) return pyre_fail(ctx, PYRE_E_ARG, "moe_ffn: %d router slices of %d rows", routed->nsl, routed->r64);
   if (t > 1 && getenv("PYRE_DEBUG_SKIP_MOE")) return PYRE_OK;
   if (!routed) { int rc = pyre_gemv_launch(ctx, m.router, x, t, w.logits); if (rc) return rc; }
-  const float* lg = routed ? routed->p : w.logits; const int nsl = routed ? routed->nsl : 1, sstride = routed ? t * routed->r64 : 0, tstride = routed ? routed->r64 : m.n_exp;
+  const float* lg = routed ? routed->p : w.logits; const int nsl = routed ? routed->nsl : 1, sstride = routed ? (routed->st ? routed->st : t) * routed->r64 : 0, tstride = routed ? routed->r64 : m.n_exp;
   auto mat_bytes = [](const QMatDev& q, double rows) { return qmat_gguf_bytes(q, rows); };
   const int hs = m.ff > m.sf ? m.ff : m.sf, entries = t * (m.top_k + 1);
   const uint2* g2 = (const uint2*)ctx->d_iq2xs;
@@ -703,6 +703,73 @@ __global__ __launch_bounds__(256, 3) void k_moe_mm_blk(MoeDev m, MoeBlk b, int T
     }
   }
 }
+// The same products where an expert has many tokens: the workgroup takes up to TG groups of eight entries through together, so
+// that a weight is decoded once for all of them (k_moe_mm_blk decodes it again every eight entries: at 2048 tokens, forty
+// entries an expert, 710 us a layer for gate and up).  A chunk of the groups' operand rows (16 rows x 256 bytes a group) goes
+// from memory straight into shared memory once for the four waves, a row's sixteen pieces in the order piece ^ row, so that
+// neither the gather (whole rows) nor the reads (sixteen rows, one piece each) meet on a bank.  Same sums in the same order.
+template <bool DOWN, int TG>
+__global__ __launch_bounds__(256, 2) void k_moe_mm_many(MoeDev m, MoeBlk b, int T, int zrow) {
+  __shared__ __align__(16) uint4 la[2][TG][256];
+  extern __shared__ __align__(16) float li[];          // [TG][super-blocks][8]
+  const int ye = blockIdx.y, k1 = m.top_k + 1; const bool shared = ye >= m.n_exp;
+  BlkEntries E;
+  if (!shared) { const int e0 = b.eoff[ye]; E.n = b.eoff[ye + 1] - e0; E.list = b.elist + e0; E.first = 0; E.step = 0; }
+  else { const int t0 = (ye - m.n_exp) * 8 * TG; E.n = min(8 * TG, T - t0); E.list = nullptr; E.first = t0 * k1 + m.top_k; E.step = k1; }
+  if (E.n <= 0) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
+  const QMatDev& W = DOWN ? (shared ? m.sh_down_m : m.down_m) : (blockIdx.z ? (shared ? m.sh_up_m : m.up_m) : (shared ? m.sh_gate_m : m.gate_m));
+  const int rows = DOWN ? m.d : m.ff, kc = DOWN ? m.ff : m.d, rt = blockIdx.x * 4 + wave;          // (rows % 256 == 0: every wave has a tile)
+  const uint16_t* opnd = DOWN ? b.hh : b.xh; const float* inv = DOWN ? b.hinv : b.xinv;
+  float* out = DOWN ? b.partial : (blockIdx.z ? b.u : b.g);
+  const int tile = (shared ? 0 : ye * (rows >> 6)) + rt, K128 = kc >> 7, nsb = kc >> 8;
+  const NibK nk = nib_consts();
+  const int fr = 4 * wave + (lane >> 4), fcg = (lane & 15) ^ fr;          // the operand row and piece this lane fetches
+  for (int i0 = 0; i0 < E.n; i0 += 8 * TG) {
+    const int np = min(8 * TG, E.n - i0), ng = (np + 7) >> 3;
+    auto row_of = [&](int sl) { const int en = blk_entry(E, i0 + sl); return DOWN ? en : en / k1; };
+    const uint16_t* so[TG];
+#pragma unroll
+    for (int u = 0; u < TG; ++u) { const int sl = u * 8 + (fr >> 1); so[u] = opnd + ((size_t)(sl < np ? row_of(sl) : zrow) * 2 + (fr & 1)) * kc + fcg * 8; }
+    if (i0 > 0) __syncthreads();
+    for (int i = threadIdx.x; i < ng * 8 * nsb; i += 256) { const int sl = i / nsb, sb = i - sl * nsb; li[((sl >> 3) * nsb + sb) * 8 + (sl & 7)] = sl < np ? inv[(size_t)row_of(sl) * nsb + sb] : 0.0f; }
+    auto fetch = [&](int c, int buf) {
+#pragma unroll
+      for (int u = 0; u < TG; ++u) if (u < ng) lds_fetch16(so[u] + c * 128, &la[buf][u][wave * 64]);
+    };
+    v4f tot[TG][4];
+#pragma unroll
+    for (int u = 0; u < TG; ++u)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) tot[u][g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    WBuf<4> wb; fetch(0, 0); load_w<4>(W, tile * 4, 0, lane, K128, wb);
+    lds_fetch_barrier();
+    for (int c = 0; c < K128; ++c) {
+      WDec wd[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) decode_chunk(wb.w[g], wb.h[g], c, nk, wd[g]);
+      if (c + 1 < K128) { fetch(c + 1, (c + 1) & 1); load_w<4>(W, tile * 4, c + 1, lane, K128, wb); }
+#pragma unroll
+      for (int u = 0; u < TG; ++u) if (u < ng) {
+        v8h a[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) a[s] = __builtin_bit_cast(v8h, la[c & 1][u][r * 16 + ((s * 4 + q) ^ r)]);
+        const float2 ai = *(const float2*)&li[(u * nsb + (c >> 1)) * 8 + 2 * q];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) chunk_add(wd[g], a, ai.x, ai.y, tot[u][g]);
+      }
+      lds_fetch_barrier();
+    }
+#pragma unroll
+    for (int u = 0; u < TG; ++u) if (u < ng) {
+      const int s0 = u * 8 + 2 * q;
+      float* o0 = s0 < np ? out + (size_t)blk_entry(E, i0 + s0) * rows + rt * 64 + r : nullptr;
+      float* o1 = s0 + 1 < np ? out + (size_t)blk_entry(E, i0 + s0 + 1) * rows + rt * 64 + r : nullptr;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) { if (o0) o0[g * 16] = halves0(tot[u][g]); if (o1) o1[g * 16] = halves1(tot[u][g]); }
+    }
+  }
+}
 // the four group sums of every token (moe_out_value's groups, folded as k_moe_down_groups folds them) into the token's
 // window: grid (d / 256, T), thread = row
 __global__ __launch_bounds__(256) void k_moe_groups_blk(MoeDev m, MoeBlk b, int T) {
@@ -744,30 +811,52 @@ int pyre_moe_block_zero_rows(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, in
   PYRE_HIP(ctx, hipMemsetAsync(b.hh + 2 * ne * hs, 0, 2 * 2 * hs, ctx->stream));
   return PYRE_OK;
 }
-// T_max: the T the scratch was carved and its zero rows were set for (x readable up to the next multiple of eight rows); the router's
+// The first T of T_router tokens (the router's sums are formed for all of them); T_max: the T the scratch was carved and its zero rows were set for (x readable up to the next multiple of eight rows); the router's
 // sums in nsl = d / 64 slices of r64 rows a token
-int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_max, int nsl, int r64) {
-  if (!pyre_moe_block_ok(m) || T < 1 || T > T_max || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe block: unsupported shape (T = %d, %d router slices)", T, nsl);
+int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_router, int T_max, int nsl, int r64) {
+  if (!pyre_moe_block_ok(m) || T < 0 || T > T_router || T_router < 1 || T_router > T_max || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe block: unsupported shape (T = %d, %d router slices)", T, nsl);
   const int hs = m.ff, ny = m.n_exp + (T + 7) / 8, ne = T * (m.top_k + 1), ne_max = T_max * (m.top_k + 1);
   const bool fix = m.n_exp == 512 && m.top_k == 10 && nsl == 32;
+  // entries an expert: eight or fewer go through in one pass of k_moe_mm_blk, more share the decoding
+  static const int force = [] { const char* e = getenv("PYRE_MM_TG"); return e ? atoi(e) : 0; }();
+  const int mean = T * m.top_k / m.n_exp, tg = force ? force : (mean <= 6 ? 1 : (mean <= 12 ? 2 : (mean <= 26 ? 4 : 8)));
+#define MM_MANY(DN, TG, GX, GZ, ZR, KC) hipLaunchKernelGGL((k_moe_mm_many<DN, TG>), dim3(GX, m.n_exp + (T + 8 * TG - 1) / (8 * TG), GZ), dim3(256), (size_t)TG * 8 * (KC / 256) * 4, ctx->stream, m, b, T, ZR)
+#define MM_GO(DN, GX, GZ, ZR, KC) do { if (tg == 1) hipLaunchKernelGGL(k_moe_mm_blk<DN>, dim3(GX, ny, GZ), dim3(256), 0, ctx->stream, m, b, T, ZR); else if (tg == 2) MM_MANY(DN, 2, GX, GZ, ZR, KC); else if (tg == 4) MM_MANY(DN, 4, GX, GZ, ZR, KC); else MM_MANY(DN, 8, GX, GZ, ZR, KC); } while (0)
   {
     if (nsl != m.d / 64 || (m.router.fmt != FMT_BF16 && m.router.fmt != FMT_F32)) return pyre_fail(ctx, PYRE_E_ARG, "moe block: the router's sums by %d slices, router format %d", nsl, m.router.fmt);
     ProfScope ps(ctx, "moe_block_router", qmat_gguf_bytes(m.router, m.router.rows) + 4.0 * T * (m.d + (double)nsl * r64));
-    if (m.router.fmt == FMT_BF16) hipLaunchKernelGGL(k_moe_router_blk<FMT_BF16>, dim3(nsl, (T + 7) / 8), dim3(256), 0, ctx->stream, m, b, r64);
-    else hipLaunchKernelGGL(k_moe_router_blk<FMT_F32>, dim3(nsl, (T + 7) / 8), dim3(256), 0, ctx->stream, m, b, r64);
+    if (m.router.fmt == FMT_BF16) hipLaunchKernelGGL(k_moe_router_blk<FMT_BF16>, dim3(nsl, (T_router + 7) / 8), dim3(256), 0, ctx->stream, m, b, r64);
+    else hipLaunchKernelGGL(k_moe_router_blk<FMT_F32>, dim3(nsl, (T_router + 7) / 8), dim3(256), 0, ctx->stream, m, b, r64);
     PYRE_CHECK_LAUNCH(ctx);
   }
+  if (T == 0) return PYRE_OK;
   { ProfScope ps(ctx, "moe_block_route", 4.0 * T * nsl * m.n_exp);
     if (fix) hipLaunchKernelGGL(k_moe_route_blk<true>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64); else hipLaunchKernelGGL(k_moe_route_blk<false>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64);
     hipLaunchKernelGGL(k_moe_lists, dim3(1), dim3(1024), 0, ctx->stream, m, b, T);
     hipLaunchKernelGGL(k_blk_split, dim3(T), dim3(256), 0, ctx->stream, b.x, (const float*)nullptr, m.d, b.xh, b.xinv, m.sh_gate_inp, b.sg); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "moe_block_gate_up", 2.0 * m.n_exp * qmat_gguf_bytes(m.gate_e, m.ff) + 2.0 * qmat_gguf_bytes(m.sh_gate, m.sf));
-    hipLaunchKernelGGL(k_moe_mm_blk<false>, dim3((hs + 255) / 256, ny, 2), dim3(256), 0, ctx->stream, m, b, T, T_max);
+    MM_GO(false, (hs + 255) / 256, 2, T_max, m.d);
     hipLaunchKernelGGL(k_blk_split, dim3(ne), dim3(256), 0, ctx->stream, (const float*)b.g, (const float*)b.u, hs, b.hh, b.hinv, (const float*)nullptr, (float*)nullptr); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "moe_block_down", (double)m.n_exp * qmat_gguf_bytes(m.down_e, m.d) + qmat_gguf_bytes(m.sh_down, m.d));
-    hipLaunchKernelGGL(k_moe_mm_blk<true>, dim3((m.d + 255) / 256, ny, 1), dim3(256), 0, ctx->stream, m, b, T, ne_max);
+    MM_GO(true, (m.d + 255) / 256, 1, ne_max, hs);
+#undef MM_GO
     hipLaunchKernelGGL(k_moe_groups_blk, dim3((m.d + 255) / 256, T), dim3(256), 0, ctx->stream, m, b, T); } PYRE_CHECK_LAUNCH(ctx);
   return PYRE_OK;
+}
+
+// Tokens i0 .. i0 + t - 1 (t <= 8, one group) of a block through the windows' launches instead: their bits are a window's (the digits
+// form of the experts).  The router's sums are there (pyre_moe_block_launch has been called for the block).
+// raw: the unreduced terms stay in w (pyre_moe_out), no group sums.
+int pyre_moe_block_window(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const MoeBlk& b, int i0, int t, int nsl, int r64, bool raw) {
+  if (i0 % 8 || t < 1 || t > 8) return pyre_fail(ctx, PYRE_E_ARG, "moe block: a window of %d tokens at %d", t, i0);
+  const RouteSrc rs{b.rpart + (size_t)(i0 / 8) * b.wr, nsl, r64, nullptr, 8};
+  float* parts = b.parts + (size_t)(i0 / 8) * PYRE_MOE_GROUPS * 8 * m.d;
+  MoeWork w2 = w; if (t == 8) w2.parts = parts;
+  int rc = pyre_moe_launch(ctx, m, w2, b.x + (size_t)i0 * m.d, t, nullptr, &rs, t == 8 && !raw); if (rc || t == 8 || raw) return rc;
+  MoeBlk o = b; o.partial = w.partial; o.sel_w = w.sel_w; o.sg = w.sg; o.parts = parts;          // fewer than eight: the terms first, then their groups
+  ProfScope ps(ctx, "moe_block_groups", 4.0 * t * m.d * (m.top_k + 5));
+  hipLaunchKernelGGL(k_moe_groups_blk, dim3((m.d + 255) / 256, t), dim3(256), 0, ctx->stream, m, o, t);
+  PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
 
 // ---- C ABI -------------------------------------------------------------------------------------------------------------

@@ -24,98 +24,76 @@ __device__ __forceinline__ void b_split(float xs, uint16_t* h1, uint16_t* h2) {
   const _Float16 a = (_Float16)xs, b = (_Float16)((xs - (float)a) * 2048.0f);
   *h1 = __builtin_bit_cast(unsigned short, a); *h2 = __builtin_bit_cast(unsigned short, b);
 }
-// sixteen bytes a lane from memory straight into shared memory: lane l's land at dst + 16 l (dst: the wave's own, uniform)
-__device__ __forceinline__ void lds_fetch(const void* src, void* dst) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-}
-
-// workgroup barrier behind lds_fetch: a wave's own fetches have landed before it arrives
-__device__ __forceinline__ void fetch_barrier() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// A wave's 128-column chunk of one row group, decoded: four matrix operands and the row's scale.
-struct WDec { v8h b[4]; float d; };
-__device__ __forceinline__ void decode_chunk(const uint4& w, const uint2& h, int c, const NibK& nk, WDec& o) {
-  const int sh = 8 * (c & 1);
-  const v2h four = {(_Float16)4.0f, (_Float16)4.0f}, m62 = {(_Float16)-62.0f, (_Float16)-62.0f}, m235 = {(_Float16)-23.5f, (_Float16)-23.5f};
-  const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
-  const uint32_t hs = h.y >> sh;
-  const uint32_t np0 = ((hs << 6) & nk.K) | nk.E, np1 = ((hs << 2) & nk.K) | nk.E;
-  v2h s2[2], s47[2];
-  s2[0] = __builtin_elementwise_fma(__builtin_bit_cast(v2h, np0), four, m62); s2[1] = __builtin_elementwise_fma(__builtin_bit_cast(v2h, np1), four, m62);
-  s47[0] = s2[0] * m235; s47[1] = s2[1] * m235;
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    const v2h vs2 = {s2[s >> 1][s & 1], s2[s >> 1][s & 1]}, vs47 = {s47[s >> 1][s & 1], s47[s >> 1][s & 1]};
-    struct U4 { uint32_t x[4]; } q; uint32_t p[4];
-    nib_f16(wd[s], nk, p);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) q.x[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(v2h, p[i]), vs2, vs47));
-    o.b[s] = __builtin_bit_cast(v8h, q);
-  }
-  o.d = h2f_bits(h.x & 0xFFFFu);
-}
-// s0 / s1 += the chunk's product for the two tokens the lane holds: the halves of a token meet first (h1 + h2 * 2^-11), then the scales
-__device__ __forceinline__ void chunk_add(const WDec& w, const v8h (&a)[4], float ai0, float ai1, float& s0, float& s1) {
-  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[s], w.b[s], acc, 0, 0, 0);
-  s0 = fmaf(fmaf(acc[1], 1.0f / 2048.0f, acc[0]), w.d * ai0, s0);
-  s1 = fmaf(fmaf(acc[3], 1.0f / 2048.0f, acc[2]), w.d * ai1, s1);
-}
-
 // ---- the product with a matrix of row tiles of 64 ------------------------------------------------------------------------------
-// grid (row tiles / 4, groups / TG), 4 waves: wave w owns row tile 4 x + w and TG groups of eight tokens.  The groups' operand
+// grid (row tiles / 4, groups / TG, K slices), 4 waves: wave w owns row tile 4 x + w and TG groups of eight tokens.  The groups' operand
 // rows of a chunk (4 KB a group) go through shared memory once for the four waves, straight from memory, the next chunk's
 // while this one's products run; a wave's codes and headers are in registers one chunk ahead.
-// op: group g's operand at op + g * op_gs uint4 ([column / 8][16 rows] x 16 B); inv: [super-block][8] factors at inv + g * inv_gs.
-// y[token * ys + row].
-template <int TG>
-__global__ __launch_bounds__(256, 2) void k_blk_gemm(QMatDev m, const uint4* __restrict__ op, size_t op_gs, const float* __restrict__ inv, int inv_gs, float* __restrict__ y, int ys, int T) {
+// op: group g's operand at op + g * op_gs uint4 ([column / 8][16 rows] x 16 B); inv: eight factors a super-block (ish = 1) or a
+// chunk (ish = 0) at inv + g * inv_gs.  One slice: y[token * ys + row]; several: slice z of group g's token t in
+// y + ((g * slices + z) * 8 + t) * ys, for a mix that adds them in order.
+// A window's launch (k_gemm_m) gives cw chunks of a slice to each of its waves and adds the waves' sums in order; the sums
+// here fall in the same order, cw chunks at a time, so a token's bits are a window's.  CW1: cw = 1 (no running sum to keep).
+template <int TG, bool CW1>
+__global__ __launch_bounds__(256, 2) void k_blk_gemm(QMatDev m, const uint4* __restrict__ op, size_t op_gs, const float* __restrict__ inv, int inv_gs, int ish, int cw, float* __restrict__ y, int ys, int T) {
   __shared__ __align__(16) uint4 la[2][TG][256];
-  extern __shared__ __align__(16) float li[];            // [TG][super-blocks][8]
+  extern __shared__ __align__(16) float li[];            // [TG][the slice's super-blocks or chunks][8]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, q = lane >> 4;
-  const int K128 = m.cols >> 7, nsb = m.cols >> 8, G = (T + 7) >> 3, g0 = blockIdx.y * TG;
+  const int K128 = m.cols >> 7, G = (T + 7) >> 3, g0 = blockIdx.y * TG, nz = gridDim.z, per = (K128 + nz - 1) / nz, c0 = blockIdx.z * per, c1 = min(K128, c0 + per);
+  const int f0 = c0 >> ish, nf = ((c1 - 1) >> ish) - f0 + 1;
   const int tile = min((int)blockIdx.x * 4 + wave, m.tiles - 1);
   auto fetch = [&](int c, int buf) {
 #pragma unroll
     for (int u = 0; u < TG; ++u) {          // 4 TG KB: a wave one KB of every group
       const uint4* src = op + (size_t)min(g0 + u, G - 1) * op_gs + (size_t)c * 256 + wave * 64 + lane;
-      lds_fetch(src, &la[buf][u][wave * 64]);
+      lds_fetch16(src, &la[buf][u][wave * 64]);
     }
   };
-  for (int i = threadIdx.x; i < TG * nsb * 8; i += 256) { const int u = i / (nsb * 8), r = i - u * nsb * 8; li[i] = inv[(size_t)min(g0 + u, G - 1) * inv_gs + r]; }
-  float s0[TG][4], s1[TG][4];
+  for (int i = threadIdx.x; i < TG * nf * 8; i += 256) { const int u = i / (nf * 8), r = i - u * nf * 8; li[i] = inv[(size_t)min(g0 + u, G - 1) * inv_gs + f0 * 8 + r]; }
+  float s0[TG][4], s1[TG][4]; v4f tot[CW1 ? 1 : TG][4];
 #pragma unroll
   for (int u = 0; u < TG; ++u)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) { s0[u][g] = 0.0f; s1[u][g] = 0.0f; }
+    for (int g = 0; g < 4; ++g) { s0[u][g] = 0.0f; s1[u][g] = 0.0f; if constexpr (!CW1) tot[u][g] = v4f{0.0f, 0.0f, 0.0f, 0.0f}; }
   const NibK nk = nib_consts();
-  WBuf<4> wb; fetch(0, 0); load_w<4>(m, tile * 4, 0, lane, K128, wb);
-  fetch_barrier();
-  for (int c = 0; c < K128; ++c) {
+  WBuf<4> wb; fetch(c0, 0); load_w<4>(m, tile * 4, c0, lane, K128, wb);
+  lds_fetch_barrier();
+  int left = cw;          // chunks until the running sums join
+  for (int c = c0; c < c1; ++c) {
+    const int buf = (c - c0) & 1;
     WDec wd[4];
 #pragma unroll
     for (int g = 0; g < 4; ++g) decode_chunk(wb.w[g], wb.h[g], c, nk, wd[g]);
-    if (c + 1 < K128) { fetch(c + 1, (c + 1) & 1); load_w<4>(m, tile * 4, c + 1, lane, K128, wb); }
+    if (c + 1 < c1) { fetch(c + 1, buf ^ 1); load_w<4>(m, tile * 4, c + 1, lane, K128, wb); }
 #pragma unroll
     for (int u = 0; u < TG; ++u) {
       v8h a[4];
 #pragma unroll
-      for (int s = 0; s < 4; ++s) a[s] = __builtin_bit_cast(v8h, la[c & 1][u][(s * 4 + q) * 16 + (lane & 15)]);
-      const float2 ai = *(const float2*)&li[((size_t)u * nsb + (c >> 1)) * 8 + 2 * q];
+      for (int s = 0; s < 4; ++s) a[s] = __builtin_bit_cast(v8h, la[buf][u][(s * 4 + q) * 16 + (lane & 15)]);
+      const float2 ai = *(const float2*)&li[((size_t)u * nf + (c >> ish) - f0) * 8 + 2 * q];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) chunk_add(wd[g], a, ai.x, ai.y, s0[u][g], s1[u][g]);
+      for (int g = 0; g < 4; ++g) {
+        if constexpr (CW1) { v4f r = {0.0f, 0.0f, 0.0f, 0.0f}; chunk_add(wd[g], a, ai.x, ai.y, r); s0[u][g] += halves0(r); s1[u][g] += halves1(r); }
+        else chunk_add(wd[g], a, ai.x, ai.y, tot[u][g]);
+      }
     }
-    fetch_barrier();
+    if constexpr (!CW1) if (--left == 0 || c + 1 == c1) {
+      left = cw;
+#pragma unroll
+      for (int u = 0; u < TG; ++u)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) { s0[u][g] += halves0(tot[u][g]); s1[u][g] += halves1(tot[u][g]); tot[u][g] = v4f{0.0f, 0.0f, 0.0f, 0.0f}; }
+    }
+    lds_fetch_barrier();
   }
   if ((int)blockIdx.x * 4 + wave >= m.tiles) return;
 #pragma unroll
   for (int u = 0; u < TG; ++u) {
     const int t0 = (g0 + u) * 8 + 2 * q; if (g0 + u >= G) break;
+    float* y0 = nz > 1 ? y + (((size_t)(g0 + u) * nz + blockIdx.z) * 8 + 2 * q) * ys : y + (size_t)t0 * ys;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int row = tile * 64 + g * 16 + (lane & 15);
-      if (row < m.rows) { if (t0 < T) y[(size_t)t0 * ys + row] = s0[u][g]; if (t0 + 1 < T) y[(size_t)(t0 + 1) * ys + row] = s1[u][g]; }
+      if (row < m.rows) { if (t0 < T) y0[row] = s0[u][g]; if (t0 + 1 < T) y0[ys + row] = s1[u][g]; }
     }
   }
 }
@@ -209,8 +187,9 @@ __global__ __launch_bounds__(256 * CS) void k_blk_mix_down(QMatDev m, const floa
   for (int tile = 0; tile < m.tiles; ++tile) {
     WDec d0, d1; decode_chunk(w0.w[0], w0.h[0], ch0, nk, d0); decode_chunk(w1.w[0], w1.h[0], ch0 + 1, nk, d1);
     if (tile + 1 < m.tiles) { load_w<1>(m, (tile + 1) * 4 + g, ch0, lane, K128, w0); load_w<1>(m, (tile + 1) * 4 + g, ch0 + 1, lane, K128, w1); }
-    float r0 = 0.0f, r1 = 0.0f;
-    chunk_add(d0, a0, dn0, dn1, r0, r1); chunk_add(d1, a1, dn0, dn1, r0, r1);
+    v4f tot = {0.0f, 0.0f, 0.0f, 0.0f};
+    chunk_add(d0, a0, dn0, dn1, tot); chunk_add(d1, a1, dn0, dn1, tot);
+    const float r0 = halves0(tot), r1 = halves1(tot);
     const size_t row = (size_t)tile * 64 + g * 16 + (lane & 15);
     if constexpr (CS == 2) { if (p == 1) { float* h = hsum + (((size_t)tile * 4 + g) * 2) * 64 + lane; h[0] = r0; h[64] = r1; } else { pg[(2 * q) * r64 + row] = r0; pg[(2 * q + 1) * r64 + row] = r1; } }
     else { pg[(2 * q) * r64 + row] = r0; pg[(2 * q + 1) * r64 + row] = r1; }
@@ -296,14 +275,14 @@ __global__ __launch_bounds__(1024) void k_blk_mix_up(QMatDev up, const uint4* __
   { const NibK nk = nib_consts(); WBuf<1> w;
 #pragma unroll
     for (int c = 0; c < KC; ++c) { load_w<1>(up, ((s * d + col0) >> 4) + g, c, lane, KC, w); decode_chunk(w.w[0], w.h[0], c, nk, wd[c]); } }
-  auto fetch = [&](int grp, int buf) { for (int j = wave; j < KC * 4; j += nw) lds_fetch(lo + (size_t)grp * KC * 256 + j * 64 + lane, &la[buf][j * 64]); };
+  auto fetch = [&](int grp, int buf) { for (int j = wave; j < KC * 4; j += nw) lds_fetch16(lo + (size_t)grp * KC * 256 + j * 64 + lane, &la[buf][j * 64]); };
   // thread = (token, column) of the epilogue; with fewer than 512 threads in rounds
   const int l = tid & 63;
   float nr[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) nr[k] = k < hc ? norm[(size_t)k * d + col0 + l] : 0.0f;
   fetch(b0, 0);
-  fetch_barrier();
+  lds_fetch_barrier();
   for (int b = b0; b < b1; ++b) {
     const int buf = (b - b0) & 1, t0 = b * 8;
     float xv[4];          // the first round's stream values, in flight beside the products
@@ -311,16 +290,16 @@ __global__ __launch_bounds__(1024) void k_blk_mix_up(QMatDev up, const uint4* __
 #pragma unroll
       for (int k = 0; k < 4; ++k) xv[k] = k < hc && t < 8 ? x[((size_t)ti * hc + k) * d + col0 + l] : 0.0f; }
     if (b + 1 < b1) fetch(b + 1, buf ^ 1);
-    float r0 = 0.0f, r1 = 0.0f;
+    v4f tot = {0.0f, 0.0f, 0.0f, 0.0f};
     { const float dn0 = lo_dn[min(t0 + 2 * q, T - 1)], dn1 = lo_dn[min(t0 + 2 * q + 1, T - 1)];
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
         v8h a[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) a[j] = __builtin_bit_cast(v8h, la[buf][((c * 4 + j) * 4 + q) * 16 + (lane & 15)]);
-        chunk_add(wd[c], a, dn0, dn1, r0, r1);
+        chunk_add(wd[c], a, dn0, dn1, tot);
       } }
-    red[s][2 * q][g * 16 + (lane & 15)] = r0; red[s][2 * q + 1][g * 16 + (lane & 15)] = r1;
+    red[s][2 * q][g * 16 + (lane & 15)] = halves0(tot); red[s][2 * q + 1][g * 16 + (lane & 15)] = halves1(tot);
     lds_barrier();
     for (int t = tid >> 6; t < 8; t += nw) {
       const int ti = t0 + t; const bool on = ti < T;
@@ -340,7 +319,7 @@ __global__ __launch_bounds__(1024) void k_blk_mix_up(QMatDev up, const uint4* __
         if (on && blockIdx.x == 0 && l < (d >> 8)) inv[(size_t)b * inv_gs + l * 8 + t] = ob.y;
       }
     }
-    fetch_barrier();          // (also: the next group's operand has arrived)
+    lds_fetch_barrier();          // (also: the next group's operand has arrived)
     if (op && tid < 128) op[(size_t)b * op_gs + (size_t)(col0 >> 3) * 16 + tid] = ((const uint4*)st[buf])[tid];
   }
 }
@@ -373,16 +352,56 @@ __global__ __launch_bounds__(256) void k_blk_gdn_out(const float* __restrict__ o
   }
 }
 
+// The same in the per-quarter form of k_gdn_delta_q and its reader load_a_sq (the bits of a window): a quarter of a head, 32 columns,
+// is split into halves on its own power of two, brought to the head's largest power by exponent arithmetic, and the head's
+// 1 / RMS goes into the chunk's factor, inv + group * inv_gs + head * 8 + token.
+__global__ __launch_bounds__(256) void k_blk_gdn_out_q(const float* __restrict__ o, const float* __restrict__ z, int zs, const float* __restrict__ nw, float eps, int heads, int T, uint4* __restrict__ op, size_t op_gs, float* __restrict__ inv, int inv_gs) {
+  const size_t gi = (size_t)blockIdx.x * 256 + threadIdx.x; const int j = (int)(gi & 15), h = (int)((gi >> 4) % heads); const int ti = (int)((gi >> 4) / heads);
+  if (ti >= T) return;          // (whole rows of sixteen lanes)
+  const float* po = o + ((size_t)ti * heads + h) * 128 + 8 * j; const float* pz = z + (size_t)ti * zs + h * 128 + 8 * j;
+  float v[8], u[8];
+#pragma unroll
+  for (int k = 0; k < 8; k += 4) { const float4 a = *(const float4*)(po + k), b = *(const float4*)(pz + k), c = *(const float4*)(nw + 8 * j + k);
+    v[k] = a.x; v[k + 1] = a.y; v[k + 2] = a.z; v[k + 3] = a.w;
+    u[k] = (a.x * c.x) * b_sigm(b.x); u[k + 1] = (a.y * c.y) * b_sigm(b.y); u[k + 2] = (a.z * c.z) * b_sigm(b.z); u[k + 3] = (a.w * c.w) * b_sigm(b.w); }
+  // the order of a wave's sum over the quarter's 32 columns: a tree of neighbours
+  float ss = ((v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3])) + ((v[4] * v[4] + v[5] * v[5]) + (v[6] * v[6] + v[7] * v[7]));
+  ss += wave_dpp<0xB1, 0xf>(0.0f, ss); ss += wave_dpp<0x4E, 0xf>(0.0f, ss);
+  float am = b_nan_abs(u[0]);
+#pragma unroll
+  for (int k = 1; k < 8; ++k) am = fmaxf(am, b_nan_abs(u[k]));
+  am = fmaxf(am, wave_dpp<0xB1, 0xf>(0.0f, am)); am = fmaxf(am, wave_dpp<0x4E, 0xf>(0.0f, am));
+  float up, dn; b_scale_of(am, &up, &dn);
+  float mr = fmaxf(dn, wave_dpp<0x141, 0xf>(0.0f, dn)); mr = fmaxf(mr, wave_dpp<0x140, 0xf>(0.0f, mr));
+  const _Float16 f = (_Float16)__uint_as_float(__float_as_uint(dn) - (__float_as_uint(mr) - 0x3F800000u));
+  struct H8 { uint16_t v[8]; } a, b;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    b_split(u[k] * up, &a.v[k], &b.v[k]);
+    a.v[k] = __builtin_bit_cast(unsigned short, (_Float16)(__builtin_bit_cast(_Float16, a.v[k]) * f)); b.v[k] = __builtin_bit_cast(unsigned short, (_Float16)(__builtin_bit_cast(_Float16, b.v[k]) * f));
+  }
+  uint4* dst = op + (size_t)(ti >> 3) * op_gs + (size_t)(h * 16 + j) * 16 + 2 * (ti & 7);
+  dst[0] = __builtin_bit_cast(uint4, a); dst[1] = __builtin_bit_cast(uint4, b);
+  const float q0 = wave_dpp<0x150, 0xf>(0.0f, ss), q1 = wave_dpp<0x154, 0xf>(0.0f, ss), q2 = wave_dpp<0x158, 0xf>(0.0f, ss), q3 = wave_dpp<0x15C, 0xf>(0.0f, ss);
+  if (j == 0) inv[(size_t)(ti >> 3) * inv_gs + h * 8 + (ti & 7)] = mr * __builtin_amdgcn_rsqf((((q0 + q1) + q2) + q3) * (1.0f / 128.0f) + eps);
+}
+
 }  // namespace
 
-int pyre_blk_gemm_launch(pyre_ctx* ctx, const QMatDev& m, const uint4* op, size_t op_gs, const float* inv, int inv_gs, float* y, int ys, int T) {
+// parts: K slices left apart for the mix that follows (PYRE_GEMV_PARTS, as pyre_gemv_parts_launch cuts them), or 1
+int pyre_blk_gemm_launch(pyre_ctx* ctx, const QMatDev& m, const uint4* op, size_t op_gs, const float* inv, int inv_gs, bool inv_chunks, float* y, int ys, int T, int parts) {
   if (m.fmt != FMT_IQ3_S_M || !m.mq || m.cols % 256) return pyre_fail(ctx, PYRE_E_TYPE, "blk_gemm: the matrix is not held in the matrix-core layout");
-  const int G = (T + 7) / 8, bx = (m.tiles + 3) / 4, nsb = m.cols / 256;
+  int nw, cw; pyre_gemm_m_plan(m, parts, &nw, &cw);
+  const int K128 = m.cols / 128, per = (K128 + parts - 1) / parts;
+  if (parts > 1) { nw = 4; cw = (per + 3) / 4; }          // (GemvEpi::four_waves)
+  if (K128 % parts || nw * cw < per) return pyre_fail(ctx, PYRE_E_SHAPE, "blk_gemm: %d columns in %d slices", m.cols, parts);
+  const int G = (T + 7) / 8, bx = (m.tiles + 3) / 4, ish = inv_chunks ? 0 : 1;
   ProfScope ps(ctx, "blk_gemm", qmat_gguf_bytes(m, m.rows) + 4.0 * T * ((double)m.cols + m.rows));
-  // eight groups a wave amortise the decoding best; with too few workgroups for the chip, fewer groups and more workgroups
-  const int tg = bx * ((G + 7) / 8) >= 512 ? 8 : (bx * ((G + 3) / 4) >= 512 ? 4 : (bx * ((G + 1) / 2) >= 192 ? 2 : 1));
-#define BLK_GO(TG) hipLaunchKernelGGL((k_blk_gemm<TG>), dim3(bx, (G + TG - 1) / TG), dim3(256), (size_t)TG * nsb * 8 * 4, ctx->stream, m, op, op_gs, inv, inv_gs, y, ys, T)
-  if (tg == 8) BLK_GO(8); else if (tg == 4) BLK_GO(4); else if (tg == 2) BLK_GO(2); else BLK_GO(1);
+  // many groups a wave amortise the decoding (eight, with running sums to keep four); with too few workgroups for the chip, fewer groups and more workgroups
+  const int b2 = bx * parts, tg = cw == 1 && b2 * ((G + 7) / 8) >= 512 ? 8 : (b2 * ((G + 3) / 4) >= 512 ? 4 : (b2 * ((G + 1) / 2) >= 192 ? 2 : 1));
+#define BLK_GO(TG, CW1) hipLaunchKernelGGL((k_blk_gemm<TG, CW1>), dim3(bx, (G + TG - 1) / TG, parts), dim3(256), (size_t)TG * (per / (ish + 1) + 1) * 8 * 4, ctx->stream, m, op, op_gs, inv, inv_gs, ish, cw, y, ys, T)
+  if (cw == 1) { if (tg == 8) BLK_GO(8, true); else if (tg == 4) BLK_GO(4, true); else if (tg == 2) BLK_GO(2, true); else BLK_GO(1, true); }
+  else { if (tg == 4) BLK_GO(4, false); else if (tg == 2) BLK_GO(2, false); else BLK_GO(1, false); }
 #undef BLK_GO
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
@@ -394,6 +413,12 @@ int pyre_blk_op_split_launch(pyre_ctx* ctx, const float* x, int cols, int T, uin
 int pyre_blk_gdn_out_launch(pyre_ctx* ctx, const float* o, const float* z, int zs, const float* nw, float eps, int heads, int T, float up, uint4* op, size_t op_gs, float* out) {
   ProfScope ps(ctx, "blk_gdn_out", 4.0 * T * heads * 128 * 3);
   hipLaunchKernelGGL(k_blk_gdn_out, dim3((unsigned)(((size_t)T * heads * 16 + 255) / 256)), dim3(256), 0, ctx->stream, o, z, zs, nw, eps, heads, T, up, op, op_gs, out);
+  PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
+}
+
+int pyre_blk_gdn_out_q_launch(pyre_ctx* ctx, const float* o, const float* z, int zs, const float* nw, float eps, int heads, int T, uint4* op, size_t op_gs, float* inv, int inv_gs) {
+  ProfScope ps(ctx, "blk_gdn_out", 4.0 * T * heads * 128 * 3);
+  hipLaunchKernelGGL(k_blk_gdn_out_q, dim3((unsigned)(((size_t)T * heads * 16 + 255) / 256)), dim3(256), 0, ctx->stream, o, z, zs, nw, eps, heads, T, op, op_gs, inv, inv_gs);
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
 
