@@ -142,13 +142,20 @@ __device__ __forceinline__ void decode_chunk(const uint4& w, const uint2& h, int
   }
   o.d = h2f_bits(h.x & 0xFFFFu);
 }
-// tot += the chunk's product, the two halves of the lane's two tokens apart, as chunk_mac forms them
-__device__ __forceinline__ void chunk_add(const WDec& w, const v8h (&a)[4], float ai0, float ai1, v4f& tot) {
-  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[s], w.b[s], acc, 0, 0, 0);
-  const float d0 = w.d * ai0, d1 = w.d * ai1;
-  tot[0] = fmaf(acc[0], d0, tot[0]); tot[1] = fmaf(acc[1], d0, tot[1]); tot[2] = fmaf(acc[2], d1, tot[2]); tot[3] = fmaf(acc[3], d1, tot[3]);
-}
+// a token's two halves meet (h1 + h2 * 2^-11)
 __device__ __forceinline__ float halves0(const v4f& t) { return t[0] + t[1] * (1.0f / 2048.0f); }
 __device__ __forceinline__ float halves1(const v4f& t) { return t[2] + t[3] * (1.0f / 2048.0f); }
+// N chunks (or row groups) at once, N independent chains of matrix instructions in turn: four in a row on one accumulator leave the
+// matrix cores idle for the latency of three
+template <int N> __device__ __forceinline__ void multi_mfma(const WDec (&w)[N], const v8h (&a)[4], v4f (&acc)[N]) {
+#pragma unroll
+  for (int g = 0; g < N; ++g) acc[g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int g = 0; g < N; ++g) acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[s], w[g].b[s], acc[g], 0, 0, 0);
+}
+__device__ __forceinline__ void scale_add(const v4f& acc, float d, float ai0, float ai1, v4f& tot) {
+  const float d0 = d * ai0, d1 = d * ai1;
+  tot[0] = fmaf(acc[0], d0, tot[0]); tot[1] = fmaf(acc[1], d0, tot[1]); tot[2] = fmaf(acc[2], d1, tot[2]); tot[3] = fmaf(acc[3], d1, tot[3]);
+}

@@ -728,14 +728,14 @@ __global__ __launch_bounds__(256, 2) void k_moe_mm_many(MoeDev m, MoeBlk b, int 
   for (int i0 = 0; i0 < E.n; i0 += 8 * TG) {
     const int np = min(8 * TG, E.n - i0), ng = (np + 7) >> 3;
     auto row_of = [&](int sl) { const int en = blk_entry(E, i0 + sl); return DOWN ? en : en / k1; };
-    const uint16_t* so[TG];
+    uint32_t so[TG];          // byte offsets (the operand stays below 4 GB: pyre_moe_block_launch)
 #pragma unroll
-    for (int u = 0; u < TG; ++u) { const int sl = u * 8 + (fr >> 1); so[u] = opnd + ((size_t)(sl < np ? row_of(sl) : zrow) * 2 + (fr & 1)) * kc + fcg * 8; }
+    for (int u = 0; u < TG; ++u) { const int sl = u * 8 + (fr >> 1); so[u] = (((uint32_t)(sl < np ? row_of(sl) : zrow) * 2 + (fr & 1)) * (uint32_t)kc + fcg * 8) * 2; }
     if (i0 > 0) __syncthreads();
     for (int i = threadIdx.x; i < ng * 8 * nsb; i += 256) { const int sl = i / nsb, sb = i - sl * nsb; li[((sl >> 3) * nsb + sb) * 8 + (sl & 7)] = sl < np ? inv[(size_t)row_of(sl) * nsb + sb] : 0.0f; }
     auto fetch = [&](int c, int buf) {
 #pragma unroll
-      for (int u = 0; u < TG; ++u) if (u < ng) lds_fetch16(so[u] + c * 128, &la[buf][u][wave * 64]);
+      for (int u = 0; u < TG; ++u) if (u < ng) lds_fetch16((const uint8_t*)opnd + so[u] + c * 256, &la[buf][u][wave * 64]);
     };
     v4f tot[TG][4];
 #pragma unroll
@@ -745,18 +745,25 @@ __global__ __launch_bounds__(256, 2) void k_moe_mm_many(MoeDev m, MoeBlk b, int 
     WBuf<4> wb; fetch(0, 0); load_w<4>(W, tile * 4, 0, lane, K128, wb);
     lds_fetch_barrier();
     for (int c = 0; c < K128; ++c) {
+      v8h a[4];
+      auto read_a = [&](int u) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) a[s] = __builtin_bit_cast(v8h, la[c & 1][u][r * 16 + ((s * 4 + q) ^ r)]);
+      };
+      read_a(0);
       WDec wd[4];
 #pragma unroll
       for (int g = 0; g < 4; ++g) decode_chunk(wb.w[g], wb.h[g], c, nk, wd[g]);
       if (c + 1 < K128) { fetch(c + 1, (c + 1) & 1); load_w<4>(W, tile * 4, c + 1, lane, K128, wb); }
 #pragma unroll
       for (int u = 0; u < TG; ++u) if (u < ng) {
-        v8h a[4];
+        v4f acc[4]; const float2 ai = *(const float2*)&li[(u * nsb + (c >> 1)) * 8 + 2 * q];
+        multi_mfma<4>(wd, a, acc);
+        __builtin_amdgcn_sched_barrier(0);
+        if (u + 1 < TG) read_a(u + 1);          // (behind the instructions that read the registers, in flight beside the scaling)
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < 4; ++s) a[s] = __builtin_bit_cast(v8h, la[c & 1][u][r * 16 + ((s * 4 + q) ^ r)]);
-        const float2 ai = *(const float2*)&li[(u * nsb + (c >> 1)) * 8 + 2 * q];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) chunk_add(wd[g], a, ai.x, ai.y, tot[u][g]);
+        for (int g = 0; g < 4; ++g) scale_add(acc[g], wd[g].d, ai.x, ai.y, tot[u][g]);
       }
       lds_fetch_barrier();
     }
@@ -814,14 +821,14 @@ int pyre_moe_block_zero_rows(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, in
 // The first T of T_router tokens (the router's sums are formed for all of them); T_max: the T the scratch was carved and its zero rows were set for (x readable up to the next multiple of eight rows); the router's
 // sums in nsl = d / 64 slices of r64 rows a token
 int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_router, int T_max, int nsl, int r64) {
-  if (!pyre_moe_block_ok(m) || T < 0 || T > T_router || T_router < 1 || T_router > T_max || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe block: unsupported shape (T = %d, %d router slices)", T, nsl);
+  if (!pyre_moe_block_ok(m) || T < 0 || T > T_router || T_router < 1 || T_router > T_max || (size_t)T_max * (m.top_k + 1) * m.ff * 4 >= (1ull << 32) || (size_t)T_max * m.d * 4 >= (1ull << 32) || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe block: unsupported shape (T = %d, %d router slices)", T, nsl);
   const int hs = m.ff, ny = m.n_exp + (T + 7) / 8, ne = T * (m.top_k + 1), ne_max = T_max * (m.top_k + 1);
   const bool fix = m.n_exp == 512 && m.top_k == 10 && nsl == 32;
   // entries an expert: eight or fewer go through in one pass of k_moe_mm_blk, more share the decoding
   static const int force = [] { const char* e = getenv("PYRE_MM_TG"); return e ? atoi(e) : 0; }();
   const int mean = T * m.top_k / m.n_exp, tg = force ? force : (mean <= 6 ? 1 : (mean <= 12 ? 2 : (mean <= 26 ? 4 : 8)));
 #define MM_MANY(DN, TG, GX, GZ, ZR, KC) hipLaunchKernelGGL((k_moe_mm_many<DN, TG>), dim3(GX, m.n_exp + (T + 8 * TG - 1) / (8 * TG), GZ), dim3(256), (size_t)TG * 8 * (KC / 256) * 4, ctx->stream, m, b, T, ZR)
-#define MM_GO(DN, GX, GZ, ZR, KC) do { if (tg == 1) hipLaunchKernelGGL(k_moe_mm_blk<DN>, dim3(GX, ny, GZ), dim3(256), 0, ctx->stream, m, b, T, ZR); else if (tg == 2) MM_MANY(DN, 2, GX, GZ, ZR, KC); else if (tg == 4) MM_MANY(DN, 4, GX, GZ, ZR, KC); else MM_MANY(DN, 8, GX, GZ, ZR, KC); } while (0)
+#define MM_GO(DN, GX, GZ, ZR, KC) do { if (tg == 1) hipLaunchKernelGGL(k_moe_mm_blk<DN>, dim3(GX, ny, GZ), dim3(256), 0, ctx->stream, m, b, T, ZR); else if (tg == 2) MM_MANY(DN, 2, GX, GZ, ZR, KC); else if (tg == 4) MM_MANY(DN, 4, GX, GZ, ZR, KC); else MM_MANY(DN, 6, GX, GZ, ZR, KC); } while (0)
   {
     if (nsl != m.d / 64 || (m.router.fmt != FMT_BF16 && m.router.fmt != FMT_F32)) return pyre_fail(ctx, PYRE_E_ARG, "moe block: the router's sums by %d slices, router format %d", nsl, m.router.fmt);
     ProfScope ps(ctx, "moe_block_router", qmat_gguf_bytes(m.router, m.router.rows) + 4.0 * T * (m.d + (double)nsl * r64));

@@ -60,20 +60,27 @@ __global__ __launch_bounds__(256, 2) void k_blk_gemm(QMatDev m, const uint4* __r
   int left = cw;          // chunks until the running sums join
   for (int c = c0; c < c1; ++c) {
     const int buf = (c - c0) & 1;
+    v8h a[4];
+    auto read_a = [&](int u) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) a[s] = __builtin_bit_cast(v8h, la[buf][u][(s * 4 + q) * 16 + (lane & 15)]);
+    };
+    read_a(0);
     WDec wd[4];
 #pragma unroll
     for (int g = 0; g < 4; ++g) decode_chunk(wb.w[g], wb.h[g], c, nk, wd[g]);
     if (c + 1 < c1) { fetch(c + 1, buf ^ 1); load_w<4>(m, tile * 4, c + 1, lane, K128, wb); }
 #pragma unroll
     for (int u = 0; u < TG; ++u) {
-      v8h a[4];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) a[s] = __builtin_bit_cast(v8h, la[buf][u][(s * 4 + q) * 16 + (lane & 15)]);
-      const float2 ai = *(const float2*)&li[((size_t)u * nf + (c >> ish) - f0) * 8 + 2 * q];
+      v4f acc[4]; const float2 ai = *(const float2*)&li[((size_t)u * nf + (c >> ish) - f0) * 8 + 2 * q];
+      multi_mfma<4>(wd, a, acc);
+      __builtin_amdgcn_sched_barrier(0);
+      if (u + 1 < TG) read_a(u + 1);          // (behind the instructions that read the registers, in flight beside the scaling)
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        if constexpr (CW1) { v4f r = {0.0f, 0.0f, 0.0f, 0.0f}; chunk_add(wd[g], a, ai.x, ai.y, r); s0[u][g] += halves0(r); s1[u][g] += halves1(r); }
-        else chunk_add(wd[g], a, ai.x, ai.y, tot[u][g]);
+        if constexpr (CW1) { v4f r = {0.0f, 0.0f, 0.0f, 0.0f}; scale_add(acc[g], wd[g].d, ai.x, ai.y, r); s0[u][g] += halves0(r); s1[u][g] += halves1(r); }
+        else scale_add(acc[g], wd[g].d, ai.x, ai.y, tot[u][g]);
       }
     }
     if constexpr (!CW1) if (--left == 0 || c + 1 == c1) {
@@ -185,10 +192,13 @@ __global__ __launch_bounds__(256 * CS) void k_blk_mix_down(QMatDev m, const floa
   const size_t r64 = (size_t)m.tiles * 64;
   float* pg = part + ((size_t)grp * nks + ks) * 8 * r64;
   for (int tile = 0; tile < m.tiles; ++tile) {
+    if (tile * 64 + g * 16 >= m.rows) break;          // (the last tile's padding; nobody reads those rows)
     WDec d0, d1; decode_chunk(w0.w[0], w0.h[0], ch0, nk, d0); decode_chunk(w1.w[0], w1.h[0], ch0 + 1, nk, d1);
     if (tile + 1 < m.tiles) { load_w<1>(m, (tile + 1) * 4 + g, ch0, lane, K128, w0); load_w<1>(m, (tile + 1) * 4 + g, ch0 + 1, lane, K128, w1); }
-    v4f tot = {0.0f, 0.0f, 0.0f, 0.0f};
-    chunk_add(d0, a0, dn0, dn1, tot); chunk_add(d1, a1, dn0, dn1, tot);
+    v4f c0 = {0.0f, 0.0f, 0.0f, 0.0f}, c1 = c0, tot = c0;
+#pragma unroll
+    for (int st = 0; st < 4; ++st) { c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0[st], d0.b[st], c0, 0, 0, 0); c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1[st], d1.b[st], c1, 0, 0, 0); }
+    scale_add(c0, d0.d, dn0, dn1, tot); scale_add(c1, d1.d, dn0, dn1, tot);
     const float r0 = halves0(tot), r1 = halves1(tot);
     const size_t row = (size_t)tile * 64 + g * 16 + (lane & 15);
     if constexpr (CS == 2) { if (p == 1) { float* h = hsum + (((size_t)tile * 4 + g) * 2) * 64 + lane; h[0] = r0; h[64] = r1; } else { pg[(2 * q) * r64 + row] = r0; pg[(2 * q + 1) * r64 + row] = r1; } }
@@ -196,7 +206,7 @@ __global__ __launch_bounds__(256 * CS) void k_blk_mix_down(QMatDev m, const floa
   }
   if constexpr (CS == 2) {          // the second chunk pair's sums join the first's (the lane that wrote them adds to its own words)
     lds_barrier();
-    if (p == 0) for (int tile = 0; tile < m.tiles; ++tile) {
+    if (p == 0) for (int tile = 0; tile < m.tiles && tile * 64 + g * 16 < m.rows; ++tile) {
       const float* h = hsum + (((size_t)tile * 4 + g) * 2) * 64 + lane; const size_t row = (size_t)tile * 64 + g * 16 + (lane & 15);
       pg[(2 * q) * r64 + row] += h[0]; pg[(2 * q + 1) * r64 + row] += h[64];
     }
@@ -292,13 +302,16 @@ __global__ __launch_bounds__(1024) void k_blk_mix_up(QMatDev up, const uint4* __
     if (b + 1 < b1) fetch(b + 1, buf ^ 1);
     v4f tot = {0.0f, 0.0f, 0.0f, 0.0f};
     { const float dn0 = lo_dn[min(t0 + 2 * q, T - 1)], dn1 = lo_dn[min(t0 + 2 * q + 1, T - 1)];
+      v4f acc[KC];
 #pragma unroll
-      for (int c = 0; c < KC; ++c) {
-        v8h a[4];
+      for (int c = 0; c < KC; ++c) acc[c] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) a[j] = __builtin_bit_cast(v8h, la[buf][((c * 4 + j) * 4 + q) * 16 + (lane & 15)]);
-        chunk_add(wd[c], a, dn0, dn1, tot);
-      } }
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int c = 0; c < KC; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, la[buf][((c * 4 + j) * 4 + q) * 16 + (lane & 15)]), wd[c].b[j], acc[c], 0, 0, 0);
+#pragma unroll
+      for (int c = 0; c < KC; ++c) scale_add(acc[c], wd[c].d, dn0, dn1, tot);
+    }
     red[s][2 * q][g * 16 + (lane & 15)] = halves0(tot); red[s][2 * q + 1][g * 16 + (lane & 15)] = halves1(tot);
     lds_barrier();
     for (int t = tid >> 6; t < 8; t += nw) {
