@@ -158,7 +158,7 @@ __device__ __forceinline__ h8v nib8_f16(uint32_t w) {
 // One pass: chunk `chunk` of KV head kvh for tokens tk0 .. tk0 + nk - 1 of the launch.
 // NC: columns the buffers hold -- G for launches of one token a pass (tp = 1), 16 otherwise.
 template <int NC> struct AttnSm {
-  float red[4 * PYRE_ATTN_CHUNK * NC];          // phase 1: [dq][position][column];  phase 3: [pw][column][dim]
+  __align__(16) float red[4 * NC * (PYRE_ATTN_CHUNK + 4)];          // phase 1: [dq][column][position] (a lane's four positions are one 16-byte write, the reads of 64 neighbouring positions meet no bank twice);  phase 3: [pw][column][dim]
   __align__(16) float sc[NC][PYRE_ATTN_CHUNK + 4];          // [column][position]: eight consecutive positions of a column are two 16-byte reads
   float wmax[PYRE_ATTN_NPW][NC], wsum[PYRE_ATTN_NPW][NC];
 };
@@ -166,7 +166,8 @@ template <int HD, int G, int NC>
 __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, const KvDev& kv, const float* __restrict__ qbuf, const uint16_t* __restrict__ qh, const float* __restrict__ qsc, int start, float* __restrict__ part_o, float* __restrict__ part_ml, int max_chunks, int chunk, int kvh, int tk0, int nk) {
   static_assert(HD == 256, "the wave layout assumes 4 x 64 head dims");
   constexpr int NPW = PYRE_ATTN_NPW, CH = PYRE_ATTN_CHUNK, NT = 256 * NPW;
-  static_assert(4 * CH == NPW * HD, "the score and value partials share one buffer");
+  constexpr int RS = CH + 4;
+  static_assert(4 * RS >= NPW * HD, "the score and value partials share one buffer");
   auto& red = sm.red; auto& sc = sm.sc; auto& wmax = sm.wmax; auto& wsum = sm.wsum;
   PYRE_TS_VARS PYRE_TS(0);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -198,7 +199,7 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
       const int c = dq + 4 * gi; sv[gi] = -INFINITY;
       if (c < ncol) {
         const bool valid = p < start + tk0 + c / G + 1;          // the column's token sees positions below its own + 1
-        float v = ((red[((size_t)0 * CH + pos) * NC + c] + red[((size_t)1 * CH + pos) * NC + c]) + red[((size_t)2 * CH + pos) * NC + c]) + red[((size_t)3 * CH + pos) * NC + c];
+        float v = ((red[(0 * NC + c) * RS + pos] + red[(1 * NC + c) * RS + pos]) + red[(2 * NC + c) * RS + pos]) + red[(3 * NC + c) * RS + pos];
         sv[gi] = valid ? v * scale : -INFINITY;
         const float m = wave_max(sv[gi]);
         if (lane == 0) wmax[pw][c] = m;
@@ -292,7 +293,7 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
 #pragma unroll
       for (int pt = 0; pt < 4; ++pt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) if (4 * lg + r < ncol) red[((size_t)dq * CH + pw * 64 + 16 * pt + li) * NC + 4 * lg + r] = D[pt][r] * qinv[r];
+        for (int r = 0; r < 4; ++r) if (4 * lg + r < ncol) red[(dq * NC + 4 * lg + r) * RS + pw * 64 + 16 * pt + li] = D[pt][r] * qinv[r];
     }
     PYRE_TS(2);
     __syncthreads(); PYRE_TS(3);
@@ -377,15 +378,11 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
           for (int pt = 0; pt < 4; ++pt) D[pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[pt][s], B[s], D[pt], 0, 0, 0);
         if (li < ncol) {
 #pragma unroll
-          for (int pt = 0; pt < 4; ++pt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) red[((size_t)dq * CH + pw * 64 + 16 * pt + 4 * lg + r) * NC + li] = D[pt][r];
+          for (int pt = 0; pt < 4; ++pt) *(float4*)&red[(dq * NC + li) * RS + pw * 64 + 16 * pt + 4 * lg] = make_float4(D[pt][0], D[pt][1], D[pt][2], D[pt][3]);
         }
       } else if (li < ncol) {          // a wave past the view: its positions carry no weight, their scores are read all the same
 #pragma unroll
-        for (int pt = 0; pt < 4; ++pt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) red[((size_t)dq * CH + pw * 64 + 16 * pt + 4 * lg + r) * NC + li] = 0.0f;
+        for (int pt = 0; pt < 4; ++pt) *(float4*)&red[(dq * NC + li) * RS + pw * 64 + 16 * pt + 4 * lg] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       }
     }
     // f32 values: requested now, while the scores are being normalised (the keys' registers are free again; __syncthreads

@@ -384,8 +384,10 @@ void   pyre_blk_mix_carve(const HcDev& h, int T, void* base, BlkMix* b);
 // update in np vectors (0 none; 1: comb [token][d]; PYRE_MOE_GROUPS: comb [group][PYRE_MOE_GROUPS][8][d])
 int pyre_blk_mix_launch(pyre_ctx* ctx, const HcDev& h, const BlkMix& b, const float* x_in, int in_ss, int in_ts, float* x, int T, const float* comb, int np, const float* comb_inj, float eps,
                         float* mixed, float* inj, uint4* op, size_t op_gs, float* inv, int inv_gs);
-// y[token * ys + row]; parts = PYRE_GEMV_PARTS: y [group][parts][8][ys].  inv_chunks: eight factors a chunk of 128 columns instead of a super-block
-int pyre_blk_gemm_launch(pyre_ctx* ctx, const QMatDev& m, const uint4* op, size_t op_gs, const float* inv, int inv_gs, bool inv_chunks, float* y, int ys, int T, int parts);
+// y[token * ys + row]; parts = PYRE_GEMV_PARTS: y [group][parts][8][ys].  inv_kind: eight factors a super-block, a chunk of 128
+// columns, or a super-block all of them the token's one power of two
+enum { PYRE_INV_BLOCK = 0, PYRE_INV_CHUNK = 1, PYRE_INV_TOKEN = 2 };
+int pyre_blk_gemm_launch(pyre_ctx* ctx, const QMatDev& m, const uint4* op, size_t op_gs, const float* inv, int inv_gs, int inv_kind, float* y, int ys, int T, int parts);
 int pyre_blk_op_split_launch(pyre_ctx* ctx, const float* x, int cols, int T, uint4* op, size_t op_gs, float* inv, int inv_gs);      // x [T][cols] -> operand rows, a power of two per 256 columns
 // a Gated DeltaNet layer's raw output o [T][heads * 128] -> RMS norm per head, * sigmoid(z), as operand rows scaled by `up` and / or as f32 rows `out`
 int pyre_blk_gdn_out_launch(pyre_ctx* ctx, const float* o, const float* z, int zs, const float* nw, float eps, int heads, int T, float up, uint4* op, size_t op_gs, float* out);

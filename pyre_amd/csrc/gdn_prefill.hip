@@ -35,10 +35,14 @@ __device__ __forceinline__ float4 as4(const v4f_& v) { return make_float4(v[0], 
 // them).  Channels of q and k: two heads a workgroup, L2-normalised over their 128 channels (q also x 1/sqrt(dk)); k also goes to kt
 // [chunk][key head][128][64].  Tokens T .. Tp-1 (the last chunk's padding) become zeros.
 template <int KK>
-__global__ __launch_bounds__(256) void k_gdnc_conv(GdnDev p, const float* __restrict__ proj, int stride, int T, int Tp, const float* __restrict__ conv_in, float* __restrict__ conv_out, float* __restrict__ co, float* __restrict__ kt) {
+__global__ __launch_bounds__(256) void k_gdnc_conv(GdnDev p, const float* __restrict__ proj, int stride, int T, int Tp, const float* __restrict__ conv_in, float* __restrict__ conv_out, float* __restrict__ co, float* __restrict__ kt, float2* __restrict__ gates) {
   __shared__ float red[4][16];
   const int c = blockIdx.x * 256 + threadIdx.x, t0 = blockIdx.y * 16, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv; const bool in = c < ch;
+  if (gates && (int)blockIdx.x == (ch + 255) / 256) {          // one more workgroup a group of tokens: decay and beta of every head, gates [token][head]
+    for (int i = tid; i < 16 * p.nv; i += 256) { const int t = t0 + i / p.nv, h = i % p.nv; if (t < T) { const float* pr = proj + (size_t)t * stride + ch + p.nv * p.dv; gates[(size_t)t * p.nv + h] = make_float2(expf(p_softplus(pr[p.nv + h] + p.dt[h]) * p.a[h]), p_sigm(pr[h])); } }
+    return;
+  }
   const int kk = KK ? KK : p.conv_k;
   float w[8], h[16 + 7];          // h[7 + i]: token t0 + i; before it the history
 #pragma unroll
@@ -228,62 +232,75 @@ __global__ __launch_bounds__(256) void k_gdnc_scan(GdnDev p, const float* __rest
 // inputs of sixteen tokens at a time go through shared memory, the next sixteen in registers meanwhile.
 __device__ __forceinline__ float row_shr1(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x111, 0xf, 0xf, true)); }
 __device__ __forceinline__ float row_last(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x15F, 0xf, 0xf, true)); }
-__global__ __launch_bounds__(256) void k_gdn_rec(GdnDev p, const float* __restrict__ co, const float* __restrict__ proj, int stride, int T, const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
+__global__ __launch_bounds__(256) void k_gdn_rec(GdnDev p, const float* __restrict__ co, const float2* __restrict__ gates, int T, const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
   constexpr int TB = 16, R = 8;
   __shared__ __align__(16) float4 kq[2][TB][2][2][16];          // [buffer][token][k, q][rows 0-3, 4-7 of a row group][row group]
-  __shared__ float vs[2][TB][16], gs[2][TB], bs[2][TB], os[2][TB][16];
+  __shared__ float vs[2][TB][16], os[2][TB][16]; __shared__ float2 gb[2][TB];
   const int h = blockIdx.x, cb = blockIdx.y * 16, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, rg = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), jl = wave * 4 + (lane >> 4), col = cb + jl;
   const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv, w = p.nv * p.dv;
-  const float dtb = p.dt[h], ah = p.a[h];
   const size_t so = ((size_t)h * DK + rg * R) * p.dv + col;
   float S[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) S[r] = ssm_in[so + (size_t)r * p.dv];
-  float4 f0, f1, f2, f3; float fv, fa = 0.0f, fb = 0.0f;
+  float4 f0, f1, f2, f3; float fv; float2 fg = make_float2(0.0f, 0.0f);
   auto src = [&](int t0, int i) { const int e = tid + 256 * i, t = min(t0 + (e >> 6), T - 1), f = e & 63; return *(const float4*)(co + (size_t)t * ch + (f < 32 ? nqk : 0) + kh * DK + 4 * (f & 31)); };
   auto fetch = [&](int t0) {          // token t0 + e / 64's float4 e % 64: 32 of k, 32 of q (past the end: the last token's again)
     f0 = src(t0, 0); f1 = src(t0, 1); f2 = src(t0, 2); f3 = src(t0, 3);
     fv = co[(size_t)min(t0 + (tid >> 4), T - 1) * ch + 2 * nqk + (size_t)h * p.dv + cb + (tid & 15)];
-    if (tid < TB) { const float* pr = proj + (size_t)min(t0 + tid, T - 1) * stride + ch + w; fa = pr[p.nv + h]; fb = pr[h]; }
+    if (tid < TB) fg = gates[(size_t)min(t0 + tid, T - 1) * p.nv + h];
   };
   auto put = [&](int buf, int i, const float4& f) { const int e = tid + 256 * i, c = e & 63; kq[buf][e >> 6][c >> 5][c & 1][(c & 31) >> 1] = f; };
   auto store = [&](int buf) {
     put(buf, 0, f0); put(buf, 1, f1); put(buf, 2, f2); put(buf, 3, f3);
     vs[buf][tid >> 4][tid & 15] = fv;
-    if (tid < TB) { gs[buf][tid] = expf(p_softplus(fa + dtb) * ah); bs[buf][tid] = p_sigm(fb); }
+    if (tid < TB) gb[buf][tid] = fg;
   };
-  struct Tok { float4 k0, k1, q0, q1; float g, b, v; };
-  auto get = [&](int buf, int t) { return Tok{kq[buf][t][0][0][rg], kq[buf][t][0][1][rg], kq[buf][t][1][0][rg], kq[buf][t][1][1][rg], gs[buf][t], bs[buf][t], vs[buf][t][jl]}; };
+  struct Tok { float4 k0, k1, q0, q1; float2 g; float v; };
+  auto get = [&](int buf, int t) { return Tok{kq[buf][t][0][0][rg], kq[buf][t][0][1][rg], kq[buf][t][1][0][rg], kq[buf][t][1][1][rg], gb[buf][t], vs[buf][t][jl]}; };
   fetch(0); store(0);
   lds_barrier();
   for (int t0 = 0, buf = 0; t0 < T; t0 += TB, buf ^= 1) {
     if (t0 + TB < T) fetch(t0 + TB);
     const int n = min(TB, T - t0);
-    float po = 0.0f;          // the previous token's output terms
+    // In the wait slots of token t's chain: the output terms of token t - 1 (its state is still there: the decayed one goes to
+    // other registers) and the output chain of token t - 2.
+    float po2 = 0.0f, po1 = 0.0f; float4 qa = make_float4(0.0f, 0.0f, 0.0f, 0.0f), qb = qa;          // chain input of token t - 2; the query of token t - 1
+    auto terms = [&]() { const float q[R] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w}; float o = S[0] * q[0];
+#pragma unroll
+      for (int r = 1; r < R; ++r) o += S[r] * q[r];
+      return o; };
     auto step = [&](const Tok& c, int t) {
-      const float k[R] = {c.k0.x, c.k0.y, c.k0.z, c.k0.w, c.k1.x, c.k1.y, c.k1.z, c.k1.w}, q[R] = {c.q0.x, c.q0.y, c.q0.z, c.q0.w, c.q1.x, c.q1.y, c.q1.z, c.q1.w};
-      float pm = 0.0f;
+      const float k[R] = {c.k0.x, c.k0.y, c.k0.z, c.k0.w, c.k1.x, c.k1.y, c.k1.z, c.k1.w};
+      float D[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) { S[r] *= c.g; pm += S[r] * k[r]; }
-      float m = pm, o = po;
+      for (int r = 0; r < R; ++r) D[r] = S[r] * c.g.x;
+      float pm = D[0] * k[0];
 #pragma unroll
-      for (int i = 0; i < 15; ++i) { m = pm + row_shr1(m); o = po + row_shr1(o); }
-      if (rg == 15) os[buf][max(t - 1, 0)][jl] = o;          // (the first token's writes nothing of use: the next one overwrites it)
-      const float delta = (c.v - row_last(m)) * c.b;
-      po = 0.0f;
+      for (int r = 1; r < R; ++r) pm += D[r] * k[r];
+      const float q[R] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+      float m = pm, o = po2, pt = S[0] * q[0];
 #pragma unroll
-      for (int r = 0; r < R; ++r) { S[r] += k[r] * delta; po += S[r] * q[r]; }
+      for (int i = 0; i < 15; ++i) {
+        m = pm + row_shr1(m); o = po2 + row_shr1(o);
+        if (i & 1) { if (i / 2 + 1 < R) pt += S[i / 2 + 1] * q[i / 2 + 1]; }
+      }
+      if (rg == 15) os[buf][max(t - 2, 0)][jl] = o;          // (the first two tokens' write nothing of use: the next one overwrites it)
+      const float delta = (c.v - row_last(m)) * c.g.y;
+#pragma unroll
+      for (int r = 0; r < R; ++r) S[r] = D[r] + k[r] * delta;
+      po2 = pt; qa = c.q0; qb = c.q1;
     };
     // a token ahead: the wave is alone on its SIMD, nothing else hides the reads; two sets of registers taking turns
     Tok x0 = get(buf, 0), x1;
     int t = 0;
     for (; t + 1 < n; t += 2) { x1 = get(buf, t + 1); step(x0, t); x0 = get(buf, min(t + 2, n - 1)); step(x1, t + 1); }
     if (t < n) step(x0, t);
-    { float o = po;
+    po1 = terms();
+    { float o = po2, o1 = po1;
 #pragma unroll
-      for (int i = 0; i < 15; ++i) o = po + row_shr1(o);
-      if (rg == 15) os[buf][n - 1][jl] = o; }
+      for (int i = 0; i < 15; ++i) { o = po2 + row_shr1(o); o1 = po1 + row_shr1(o1); }
+      if (rg == 15) { if (n > 1) os[buf][n - 2][jl] = o; os[buf][n - 1][jl] = o1; } }
     if (t0 + TB < T) store(buf ^ 1);
     lds_barrier();
     if ((tid >> 4) < n) oraw[(size_t)(t0 + (tid >> 4)) * w + (size_t)h * p.dv + cb + (tid & 15)] = os[buf][tid >> 4][tid & 15];
@@ -308,8 +325,8 @@ int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, con
   if (T < 1 || g.conv_k < 1 || g.conv_k > 8) return pyre_fail(ctx, PYRE_E_ARG, "gdn prompt: %d tokens, %d taps", T, g.conv_k);
   const int ch = 2 * g.nk * g.dk + g.nv * g.dv, nch = (T + C - 1) / C, Tp = nch * C;
   { ProfScope ps(ctx, "gdn_prompt_conv", 8.0 * T * ch);
-    if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, b.kt);
-    else hipLaunchKernelGGL(k_gdnc_conv<0>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, b.kt); } PYRE_CHECK_LAUNCH(ctx);
+    if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, b.kt, (float2*)nullptr);
+    else hipLaunchKernelGGL(k_gdnc_conv<0>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, b.kt, (float2*)nullptr); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "gdn_prompt_chunk", 4.0 * T * (ch + g.nv * (2.0 * DK + C)));
     hipLaunchKernelGGL(k_gdnc_chunk, dim3(nch, g.nv), dim3(256), 0, ctx->stream, g, b.co, proj, stride, T, b.w, b.u, b.p, b.dec); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "gdn_prompt_scan", 8.0 * g.nv * g.dk * g.dv + 4.0 * T * g.nv * (4.0 * DK + C));
@@ -323,9 +340,9 @@ int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const
   if (T < 1 || g.conv_k < 1 || g.conv_k > 8 || conv_in == conv_out) return pyre_fail(ctx, PYRE_E_ARG, "gdn prompt: %d tokens, %d taps", T, g.conv_k);
   const int ch = 2 * g.nk * g.dk + g.nv * g.dv, Tp = (T + 15) / 16 * 16;
   { ProfScope ps(ctx, "gdn_prompt_conv", 8.0 * T * ch);
-    if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr);
-    else hipLaunchKernelGGL(k_gdnc_conv<0>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr); } PYRE_CHECK_LAUNCH(ctx);
+    if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256 + 1, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr, (float2*)b.dec);
+    else hipLaunchKernelGGL(k_gdnc_conv<0>, dim3((ch + 255) / 256 + 1, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr, (float2*)b.dec); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "gdn_prompt_rec", 8.0 * g.nv * g.dk * g.dv + 4.0 * T * (ch + 2.0 * g.nv * g.dv));
-    hipLaunchKernelGGL(k_gdn_rec, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, proj, stride, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
+    hipLaunchKernelGGL(k_gdn_rec, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
   return PYRE_OK;
 }

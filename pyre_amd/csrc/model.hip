@@ -603,7 +603,7 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
     const Layer& L = m->layers[il]; const int pw = L.full ? m->pw_attn : m->pw_lin, oc = L.outp.cols;
     if ((rc = pyre_blk_mix_launch(ctx, L.hca, B->mix, xin, in_ss, in_ts, B->x, T, comb, np, cinj, c.eps, B->mixed, B->inj_a, B->op, gs(d), B->inv, is(d)))) return rc;
     xin = B->x; in_ss = d; in_ts = hc * d;
-    if ((rc = pyre_blk_gemm_launch(ctx, L.proj, B->op, gs(d), B->inv, is(d), false, B->proj, pw, T, 1))) return rc;
+    if ((rc = pyre_blk_gemm_launch(ctx, L.proj, B->op, gs(d), B->inv, is(d), PYRE_INV_TOKEN, B->proj, pw, T, 1))) return rc;
     if (L.full) {
       const int ai = L.mix_index;
       if (m->has_idx) {          // a sparse indexer selects per window of eight, behind the windows before it
@@ -618,13 +618,13 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
         if ((rc = pyre_attn_blk_launch(ctx, L.attn, s->kv[ai], B->q, B->qh, B->qsc, B->proj, pw, start, T, B->att, B->core))) return rc;
       }
       if ((rc = pyre_blk_op_split_launch(ctx, B->core, oc, T, B->op, gs(oc), B->inv, is(oc)))) return rc;
-      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, is(oc), false, B->o, d, T, PYRE_GEMV_PARTS))) return rc;
+      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, is(oc), PYRE_INV_BLOCK, B->o, d, T, PYRE_GEMV_PARTS))) return rc;
     } else {
       const int li = L.mix_index, b = s->cur[li], nb = b ^ 1;
       if ((rc = pyre_gdn_rec_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], B->core))) return rc;
       s->cur[li] = nb;
       if ((rc = pyre_blk_gdn_out_q_launch(ctx, B->core, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, B->op, gs(oc), B->inv, oc / 16))) return rc;
-      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, oc / 16, true, B->o, d, T, PYRE_GEMV_PARTS))) return rc;
+      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, oc / 16, PYRE_INV_CHUNK, B->o, d, T, PYRE_GEMV_PARTS))) return rc;
     }
     if ((rc = pyre_blk_mix_launch(ctx, L.hcf, B->mix, xin, in_ss, in_ts, B->x, T, B->o, PYRE_GEMV_PARTS, B->inj_a, c.eps, B->mixed, B->inj_f, nullptr, 0, nullptr, 0))) return rc;
     const bool end = il == c.n_layers - 1;

@@ -826,7 +826,7 @@ int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T
   const bool fix = m.n_exp == 512 && m.top_k == 10 && nsl == 32;
   // entries an expert: eight or fewer go through in one pass of k_moe_mm_blk, more share the decoding
   static const int force = [] { const char* e = getenv("PYRE_MM_TG"); return e ? atoi(e) : 0; }();
-  const int mean = T * m.top_k / m.n_exp, tg = force ? force : (mean <= 6 ? 1 : (mean <= 12 ? 2 : (mean <= 26 ? 4 : 8)));
+  const int mean = T * m.top_k / m.n_exp, tg = force ? force : (mean <= 3 ? 1 : (mean <= 8 ? 2 : (mean <= 32 ? 4 : 6)));
 #define MM_MANY(DN, TG, GX, GZ, ZR, KC) hipLaunchKernelGGL((k_moe_mm_many<DN, TG>), dim3(GX, m.n_exp + (T + 8 * TG - 1) / (8 * TG), GZ), dim3(256), (size_t)TG * 8 * (KC / 256) * 4, ctx->stream, m, b, T, ZR)
 #define MM_GO(DN, GX, GZ, ZR, KC) do { if (tg == 1) hipLaunchKernelGGL(k_moe_mm_blk<DN>, dim3(GX, ny, GZ), dim3(256), 0, ctx->stream, m, b, T, ZR); else if (tg == 2) MM_MANY(DN, 2, GX, GZ, ZR, KC); else if (tg == 4) MM_MANY(DN, 4, GX, GZ, ZR, KC); else MM_MANY(DN, 6, GX, GZ, ZR, KC); } while (0)
   {

@@ -33,7 +33,8 @@ __device__ __forceinline__ void b_split(float xs, uint16_t* h1, uint16_t* h2) {
 // y + ((g * slices + z) * 8 + t) * ys, for a mix that adds them in order.
 // A window's launch (k_gemm_m) gives cw chunks of a slice to each of its waves and adds the waves' sums in order; the sums
 // here fall in the same order, cw chunks at a time, so a token's bits are a window's.  CW1: cw = 1 (no running sum to keep).
-template <int TG, bool CW1>
+// UNI: a token's factor is one power of two for all its columns (the mixes' operands) and meets the finished sum.
+template <int TG, bool CW1, bool UNI>
 __global__ __launch_bounds__(256, 2) void k_blk_gemm(QMatDev m, const uint4* __restrict__ op, size_t op_gs, const float* __restrict__ inv, int inv_gs, int ish, int cw, float* __restrict__ y, int ys, int T) {
   __shared__ __align__(16) uint4 la[2][TG][256];
   extern __shared__ __align__(16) float li[];            // [TG][the slice's super-blocks or chunks][8]
@@ -72,14 +73,14 @@ __global__ __launch_bounds__(256, 2) void k_blk_gemm(QMatDev m, const uint4* __r
     if (c + 1 < c1) { fetch(c + 1, buf ^ 1); load_w<4>(m, tile * 4, c + 1, lane, K128, wb); }
 #pragma unroll
     for (int u = 0; u < TG; ++u) {
-      v4f acc[4]; const float2 ai = *(const float2*)&li[((size_t)u * nf + (c >> ish) - f0) * 8 + 2 * q];
+      v4f acc[4]; float2 ai = make_float2(1.0f, 1.0f); if constexpr (!UNI) ai = *(const float2*)&li[((size_t)u * nf + (c >> ish) - f0) * 8 + 2 * q];
       multi_mfma<4>(wd, a, acc);
       __builtin_amdgcn_sched_barrier(0);
       if (u + 1 < TG) read_a(u + 1);          // (behind the instructions that read the registers, in flight beside the scaling)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        if constexpr (CW1) { v4f r = {0.0f, 0.0f, 0.0f, 0.0f}; scale_add(acc[g], wd[g].d, ai.x, ai.y, r); s0[u][g] += halves0(r); s1[u][g] += halves1(r); }
+        if constexpr (CW1) { const float d0 = UNI ? wd[g].d : wd[g].d * ai.x, d1 = UNI ? wd[g].d : wd[g].d * ai.y; s0[u][g] += fmaf(acc[g][1] * d0, 1.0f / 2048.0f, acc[g][0] * d0); s1[u][g] += fmaf(acc[g][3] * d1, 1.0f / 2048.0f, acc[g][2] * d1); }
         else scale_add(acc[g], wd[g].d, ai.x, ai.y, tot[u][g]);
       }
     }
@@ -96,11 +97,12 @@ __global__ __launch_bounds__(256, 2) void k_blk_gemm(QMatDev m, const uint4* __r
 #pragma unroll
   for (int u = 0; u < TG; ++u) {
     const int t0 = (g0 + u) * 8 + 2 * q; if (g0 + u >= G) break;
+    float2 fu = make_float2(1.0f, 1.0f); if constexpr (UNI) fu = *(const float2*)&li[(size_t)u * nf * 8 + 2 * q];
     float* y0 = nz > 1 ? y + (((size_t)(g0 + u) * nz + blockIdx.z) * 8 + 2 * q) * ys : y + (size_t)t0 * ys;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int row = tile * 64 + g * 16 + (lane & 15);
-      if (row < m.rows) { if (t0 < T) y0[row] = s0[u][g]; if (t0 + 1 < T) y0[ys + row] = s1[u][g]; }
+      if (row < m.rows) { if (t0 < T) y0[row] = UNI ? s0[u][g] * fu.x : s0[u][g]; if (t0 + 1 < T) y0[ys + row] = UNI ? s1[u][g] * fu.y : s1[u][g]; }
     }
   }
 }
@@ -144,13 +146,21 @@ __global__ __launch_bounds__(256 * CS) void k_blk_mix_down(QMatDev m, const floa
   const int c0 = ks * 256 * CS, s = c0 / d, i0 = c0 - s * d, K128 = m.cols >> 7, t0 = grp * 8, nt = min(8, T - t0);
   const float nv = norm[(size_t)s * d + i0 + tid];
   float v[8];
+  if constexpr (NP > 0) {          // the tokens' weights of the pending update, once for the workgroup
+    if (tid < 8) wsum[0][tid] = 2.0f * b_sigm(inj[(t0 + min(tid, nt - 1)) * hc + s]);
+    lds_barrier();
+  }
+  float wt[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) wt[t] = NP > 0 ? wsum[0][t] : 0.0f;
+  if constexpr (NP > 0) lds_barrier();
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
     v[t] = 0.0f;
     if (t < nt) {
       v[t] = x_in[(size_t)(t0 + t) * in_ts + (size_t)s * in_ss + i0 + tid];
       if constexpr (NP > 0) {
-        const float w = 2.0f * b_sigm(inj[(t0 + t) * hc + s]); float o;
+        const float w = wt[t]; float o;
         if constexpr (NP == 1) o = comb[(size_t)(t0 + t) * d + i0 + tid];
         else {
           const float* pc = comb + ((size_t)grp * NP * 8 + t) * d + i0 + tid;
@@ -402,19 +412,20 @@ __global__ __launch_bounds__(256) void k_blk_gdn_out_q(const float* __restrict__
 }  // namespace
 
 // parts: K slices left apart for the mix that follows (PYRE_GEMV_PARTS, as pyre_gemv_parts_launch cuts them), or 1
-int pyre_blk_gemm_launch(pyre_ctx* ctx, const QMatDev& m, const uint4* op, size_t op_gs, const float* inv, int inv_gs, bool inv_chunks, float* y, int ys, int T, int parts) {
+int pyre_blk_gemm_launch(pyre_ctx* ctx, const QMatDev& m, const uint4* op, size_t op_gs, const float* inv, int inv_gs, int inv_kind, float* y, int ys, int T, int parts) {
   if (m.fmt != FMT_IQ3_S_M || !m.mq || m.cols % 256) return pyre_fail(ctx, PYRE_E_TYPE, "blk_gemm: the matrix is not held in the matrix-core layout");
   int nw, cw; pyre_gemm_m_plan(m, parts, &nw, &cw);
   const int K128 = m.cols / 128, per = (K128 + parts - 1) / parts;
   if (parts > 1) { nw = 4; cw = (per + 3) / 4; }          // (GemvEpi::four_waves)
   if (K128 % parts || nw * cw < per) return pyre_fail(ctx, PYRE_E_SHAPE, "blk_gemm: %d columns in %d slices", m.cols, parts);
-  const int G = (T + 7) / 8, bx = (m.tiles + 3) / 4, ish = inv_chunks ? 0 : 1;
+  const int G = (T + 7) / 8, bx = (m.tiles + 3) / 4, ish = inv_kind == PYRE_INV_CHUNK ? 0 : 1; const bool uni = inv_kind == PYRE_INV_TOKEN;
   ProfScope ps(ctx, "blk_gemm", qmat_gguf_bytes(m, m.rows) + 4.0 * T * ((double)m.cols + m.rows));
   // many groups a wave amortise the decoding (eight, with running sums to keep four); with too few workgroups for the chip, fewer groups and more workgroups
   const int b2 = bx * parts, tg = cw == 1 && b2 * ((G + 7) / 8) >= 512 ? 8 : (b2 * ((G + 3) / 4) >= 512 ? 4 : (b2 * ((G + 1) / 2) >= 192 ? 2 : 1));
-#define BLK_GO(TG, CW1) hipLaunchKernelGGL((k_blk_gemm<TG, CW1>), dim3(bx, (G + TG - 1) / TG, parts), dim3(256), (size_t)TG * (per / (ish + 1) + 1) * 8 * 4, ctx->stream, m, op, op_gs, inv, inv_gs, ish, cw, y, ys, T)
-  if (cw == 1) { if (tg == 8) BLK_GO(8, true); else if (tg == 4) BLK_GO(4, true); else if (tg == 2) BLK_GO(2, true); else BLK_GO(1, true); }
-  else { if (tg == 4) BLK_GO(4, false); else if (tg == 2) BLK_GO(2, false); else BLK_GO(1, false); }
+#define BLK_GO(TG, CW1, UNI) hipLaunchKernelGGL((k_blk_gemm<TG, CW1, UNI>), dim3(bx, (G + TG - 1) / TG, parts), dim3(256), (size_t)TG * (per / (ish + 1) + 1) * 8 * 4, ctx->stream, m, op, op_gs, inv, inv_gs, ish, cw, y, ys, T)
+  if (cw == 1 && uni) { if (tg == 8) BLK_GO(8, true, true); else if (tg == 4) BLK_GO(4, true, true); else if (tg == 2) BLK_GO(2, true, true); else BLK_GO(1, true, true); }
+  else if (cw == 1) { if (tg == 8) BLK_GO(8, true, false); else if (tg == 4) BLK_GO(4, true, false); else if (tg == 2) BLK_GO(2, true, false); else BLK_GO(1, true, false); }
+  else { if (tg == 4) BLK_GO(4, false, false); else if (tg == 2) BLK_GO(2, false, false); else BLK_GO(1, false, false); }
 #undef BLK_GO
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
