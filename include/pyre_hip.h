@@ -146,9 +146,12 @@ int  pyre_gdn_get_state(pyre_ctx* ctx, pyre_gdn* g, float* conv_host, float* ssm
 /* proj [t][ch + nv*dv + 2*nv] = per token [qkv | z | beta | alpha] -> out [t][nv*dv]; tokens run in time order. */
 int  pyre_gdn_step(pyre_ctx* ctx, pyre_gdn* g, const float* proj_host, int t, float* out_host);
 /* The same recurrence for a prompt of T tokens in chunked form (chunk = 64) on the fp32 matrix cores; the reference has
- * only the sequential form (linear_core above), which is therefore the oracle.  A remainder T % 64 runs through the
- * step kernels. */
+ * only the sequential form (linear_core above), which is therefore the oracle.  pyre_gdn_prefill_parts takes the four
+ * projections from arrays of their own ([T][ch], [T][nv*dv], [T][nv], [T][nv], row strides in floats), so that the caller
+ * need not join them. */
 int  pyre_gdn_prefill_chunked(pyre_ctx* ctx, pyre_gdn* g, const float* proj_host, int T, int chunk, float* out_host);
+int  pyre_gdn_prefill_parts(pyre_ctx* ctx, pyre_gdn* g, const float* qkv, size_t qkv_stride, const float* z, size_t z_stride, const float* beta, size_t beta_stride, const float* alpha, size_t alpha_stride,
+                            int T, int chunk, float* out_host);
 
 /* ---- gated attention layer core over a 4-bit KV cache --------------------------------------------------------------
  * attn_core, dense branch (qwen4exp_gguf.rs:1558-1615): k RMSNorm + RoPE, append; per head q RMSNorm + RoPE,

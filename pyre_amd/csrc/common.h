@@ -28,7 +28,16 @@
 #define PYRE_WAVE 64
 #define PYRE_UNIT 64            // weights per decode unit (one lane decodes one unit at a time)
 
+// Pinned staging for host arrays that are too large to leave to the runtime's pageable copies (pyre_host_pipe, ctx.hip): each of WORKERS
+// threads owns two buffers of SEG bytes a direction, a stream a direction carries the copies.  Made at the first use, given back with the context.
+struct HostPipe {
+  static constexpr int WORKERS = 12; static constexpr size_t SEG = (size_t)2 << 20;
+  hipStream_t up = nullptr, down = nullptr; uint8_t* mem = nullptr;
+  hipEvent_t ev[WORKERS][2][2] = {};          // [worker][direction][buffer]: its last copy
+  uint8_t* buf(int w, int dir, int i) const { return mem + ((size_t)(w * 2 + dir) * 2 + i) * SEG; }
+};
 struct pyre_ctx {
+  HostPipe* pipe = nullptr;
   int device = 0;
   hipStream_t stream = nullptr;
   std::string err;
@@ -94,6 +103,7 @@ int pyre_fail(pyre_ctx* ctx, int code, const char* fmt, ...);
 #define PYRE_CHECK_LAUNCH(ctx) PYRE_HIP(ctx, hipGetLastError())
 
 int pyre_stage(pyre_ctx* ctx, size_t nbytes, void** out);          // grow-only device staging buffer
+int pyre_host_pipe(pyre_ctx* ctx, HostPipe** out);
 
 // ---- device-side matrix view --------------------------------------------------------------------------------------
 // Weights live in "lane = row" planes: rows are grouped in tiles of 64, and for every (tile, unit) the 64 rows'

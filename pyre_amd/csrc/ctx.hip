@@ -21,6 +21,26 @@ int pyre_stage(pyre_ctx* ctx, size_t nbytes, void** out) {
   *out = ctx->stage; return PYRE_OK;
 }
 
+static void host_pipe_free(HostPipe* P) {
+  if (!P) return;
+  if (P->up) { (void)hipStreamSynchronize(P->up); (void)hipStreamDestroy(P->up); }
+  if (P->down) { (void)hipStreamSynchronize(P->down); (void)hipStreamDestroy(P->down); }
+  for (auto& a : P->ev) for (auto& b : a) for (auto e : b) if (e) (void)hipEventDestroy(e);
+  if (P->mem) (void)hipHostFree(P->mem);
+  delete P;
+}
+int pyre_host_pipe(pyre_ctx* ctx, HostPipe** out) {
+  if (!ctx->pipe) {
+    HostPipe* P = new HostPipe(); hipError_t e = hipStreamCreateWithFlags(&P->up, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&P->down, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&P->mem, (size_t)HostPipe::WORKERS * 4 * HostPipe::SEG, hipHostMallocDefault);
+    for (auto& a : P->ev) for (auto& b : a) for (auto& v : b) if (e == hipSuccess) e = hipEventCreateWithFlags(&v, hipEventDisableTiming);
+    if (e != hipSuccess) { host_pipe_free(P); return pyre_fail(ctx, PYRE_E_HIP, "host staging: %s", hipGetErrorString(e)); }
+    ctx->pipe = P;
+  }
+  *out = ctx->pipe; return PYRE_OK;
+}
+
 // ---- synthetic blocks: pyre_amd/synth.py:blocks() on the device -----------------------------------------------------
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {
   z ^= z >> 30; z *= 0xBF58476D1CE4E5B9ull; z ^= z >> 27; z *= 0x94D049BB133111EBull; z ^= z >> 31; return z;
@@ -86,6 +106,7 @@ void pyre_ctx_destroy(pyre_ctx* ctx) {
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   if (ctx->stage) (void)hipFree(ctx->stage);
+  host_pipe_free(ctx->pipe);
   if (ctx->d_iq3s) (void)hipFree(ctx->d_iq3s);
   if (ctx->d_cb) (void)hipFree(ctx->d_cb);
   if (ctx->aop_buf) (void)hipFree(ctx->aop_buf);

@@ -86,6 +86,7 @@ def _declare(L):
         "pyre_gdn_get_state": (i32, [vp, vp, vp, vp]),
         "pyre_gdn_step": (i32, [vp, vp, vp, i32, vp]),
         "pyre_gdn_prefill_chunked": (i32, [vp, vp, vp, i32, i32, vp]),
+        "pyre_gdn_prefill_parts": (i32, [vp, vp, vp, sz, vp, sz, vp, sz, vp, sz, i32, i32, vp]),
         "pyre_attn_create": (i32, [vp, i32, i32, i32, i32, f32, f32, vp, vp, i32, i32, i32, C.POINTER(vp)]),
         "pyre_attn_destroy": (None, [vp]),
         "pyre_attn_len": (i32, [vp]),
@@ -427,10 +428,12 @@ class Gdn:
         return out
 
     def prefill_chunked(self, qkv, z, beta, alpha, chunk=64):
-        proj = np.ascontiguousarray(np.concatenate([qkv, z, beta, alpha], axis=1), dtype=np.float32)
-        t = proj.shape[0]
+        parts = [np.ascontiguousarray(v, dtype=np.float32) for v in (qkv, z, beta, alpha)]
+        t = parts[0].shape[0]
+        assert [p.shape for p in parts] == [(t, self.ch), (t, self.nv * self.dv), (t, self.nv), (t, self.nv)]
         out = np.empty((t, self.nv * self.dv), dtype=np.float32)
-        self.ctx.check(self.ctx.L.pyre_gdn_prefill_chunked(self.ctx.h, self.h, _ptr(proj), t, chunk, _ptr(out)), "gdn_prefill_chunked")
+        args = [a for p in parts for a in (_ptr(p), p.shape[1])]
+        self.ctx.check(self.ctx.L.pyre_gdn_prefill_parts(self.ctx.h, self.h, *args, t, chunk, _ptr(out)), "gdn_prefill_chunked")
         return out
 
     def close(self):
