@@ -164,12 +164,14 @@ int pyre_gemv_n_launch(pyre_ctx* ctx, const void* nq, size_t rows, size_t cols, 
 //   co:   rows < ch are the channels of a causal depthwise conv1d (kernel kk, weights conv_w[ch][kk]); the lane that
 //         owns a row runs the window's tokens in order, o = w[kk-1]*cur + sum_j w[j]*state[j], co[t][row] = silu(o),
 //         and slides the row's state conv_in -> conv_out ([kk-1][ch], oldest first; in == out is fine).
-struct GemvEpi { uint32_t* best; const float* conv_w; const float* conv_in; float* conv_out; float* co; int ch, kk; int four_waves; int sq_heads = 0; float sq_eps = 0.0f; };          // sq_*: PyreAop::sq travels to the kernel here
+struct GemvEpi { uint32_t* best; const float* conv_w; const float* conv_in; float* conv_out; float* co; int ch, kk; int four_waves; int sq_heads = 0; float sq_eps = 0.0f; int nz = 0; };          // sq_*: PyreAop::sq travels to the kernel here
 // launchers implemented in qmat.hip, used by the block / model code
 // Matrices in the matrix-core layout (FMT_IQ3_S_M) take their activations as the f16 operand `a` when the caller has one (a
 // producer kernel wrote it); otherwise x_dev is split into the context's operand buffer by one more launch.
 struct PyreAop;
 int pyre_gemv_launch(pyre_ctx* ctx, const QMatDev& m, const float* x_dev, int t, float* y_dev, const PyreAop* a = nullptr);
+// the product of a lane = row matrix for groups of eight tokens in one launch: x [groups * 8][cols] -> y [groups * 8][rows]
+int pyre_gemv_rows_launch(pyre_ctx* ctx, const QMatDev& m, const float* x_dev, int groups, float* y_dev);
 // waves per workgroup and units per wave the (unsplit) GEMV uses for this matrix
 void pyre_gemv_plan(const QMatDev& m, int* nw, int* upw);
 // K range split over `ksplit` workgroups per row tile; partial[(ks*t_count + t)*tiles*64 + row] holds the slice sums and
@@ -312,7 +314,7 @@ void   pyre_moe_work_carve(const MoeDev& m, void* base, MoeWork* w);
 // (pyre_moe_out) for a consumer that evaluates moe_out_value itself.
 // Router logits that arrive as K-slice sums (left by the mix that produced x, see HcRoute): logit[t][e] = the slices
 // p[(s*T + t)*r64 + e], s = 0..nsl-1, added in slice order.
-struct RouteSrc { const float* p; int nsl; int r64; const uint32_t* dgx = nullptr; int st = 0; };          // dgx: the activations' digits (digits.h), left by the same mix, or null; st: tokens a slice holds room for (0: T)
+struct RouteSrc { const float* p; int nsl; int r64; const uint32_t* dgx = nullptr; };          // dgx: the activations' digits (digits.h), left by the same mix, or null
 // in_groups (t > 1, y == nullptr, pyre_moe_groups_ok): the down projection leaves the PYRE_MOE_GROUPS group sums of every
 // token in w.parts, group q of token ti at parts + (q*t + ti)*d, instead of the unreduced terms.
 int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const float* x_dev, int t, float* y_dev, const RouteSrc* routed = nullptr, bool in_groups = false);
@@ -332,7 +334,13 @@ size_t pyre_moe_block_bytes(const MoeDev& m, int T);
 void   pyre_moe_block_carve(const MoeDev& m, int T, void* base, MoeBlk* b);
 int    pyre_moe_block_zero_rows(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T);
 int    pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_router, int T_max, int nsl, int r64);
-int    pyre_moe_block_window(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const MoeBlk& b, int i0, int t, int nsl, int r64, bool raw);
+// any number of tokens with the windows' arithmetic: moe.hip
+struct MoeRows { int32_t* sel_idx; float* sel_w; int32_t* elist; float* sg; int32_t* eoff; float* h; float* partial; uint32_t* dgx; uint32_t* dgh; };
+size_t pyre_moe_rows_bytes(const MoeDev& m, int T);
+void   pyre_moe_rows_carve(const MoeDev& m, int T, void* base, MoeRows* w);
+bool   pyre_moe_rows_ok(const MoeDev& m);
+int    pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const float* x, int T, const float* rpart, size_t wr, int nsl, int r64, float* parts);
+inline MoeOut pyre_moe_rows_out(const MoeDev& m, const MoeRows& w, int first_token) { return MoeOut{w.partial + (size_t)first_token * (m.top_k + 1) * m.d, w.sel_w + (size_t)first_token * m.top_k, w.sg + first_token, m.d, m.top_k}; }
 // K parts the gate/up dot products are summed in (1 or 2; k_moe_gu)
 int pyre_moe_gu_parts(const MoeDev& m);
 
@@ -383,6 +391,14 @@ bool pyre_hc_route_ok(const HcDev& h, const QMatDev& router);
 bool pyre_hc_plan(const HcDev& h, int* nw, int* upw, int* ksplit);
 int pyre_hc_combine_launch(pyre_ctx* ctx, int d, int hc, float* x_dev, int t, const float* out_dev, const float* inj_dev);
 
+// the lane = row mix for `groups` groups of eight tokens in one launch a step (rows of the last group past the prompt hold anything
+// finite): w's buffers hold pyre_hc_rows_bytes; route.part [group][slice][8][rows]
+size_t pyre_hc_rows_bytes(const HcDev& h, int groups);
+void   pyre_hc_rows_carve(const HcDev& h, int groups, void* base, HcWork* w);
+bool   pyre_hc_rows_ok(const HcDev& h);
+int pyre_hc_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const float* x_in, int in_ss, int in_ts, float* x_out, int groups, const float* comb_out, const MoeOut* comb_moe, const float* comb_inj,
+                            float eps, float* mixed_dev, float* inj_dev, const HcRoute* route);
+
 // ---- a prompt taken layer by layer (prompt.hip): the mixes and projections of hundreds of tokens a launch ------------------------
 // Tokens in groups of eight, a group's activations as sixteen f16 operand rows (PyreAop with R = 16) at op + group * op_gs
 // (uint4), their factors [super-block][8] at inv + group * inv_gs.
@@ -403,6 +419,8 @@ int pyre_blk_op_split_launch(pyre_ctx* ctx, const float* x, int cols, int T, uin
 int pyre_blk_gdn_out_launch(pyre_ctx* ctx, const float* o, const float* z, int zs, const float* nw, float eps, int heads, int T, float up, uint4* op, size_t op_gs, float* out);
 // ... and in the per-quarter form of GdnQ: operand rows at op, the factors of a chunk (a head's 128 columns) at inv
 int pyre_blk_gdn_out_q_launch(pyre_ctx* ctx, const float* o, const float* z, int zs, const float* nw, float eps, int heads, int T, uint4* op, size_t op_gs, float* inv, int inv_gs);
+// ... and as f32 rows with the head norm of k_gdn_delta (its order of sums)
+int pyre_blk_gdn_out_w_launch(pyre_ctx* ctx, const float* o, const float* z, int zs, const float* nw, float eps, int heads, int T, float* out);
 
 // ---- Gated DeltaNet (gdn.hip) -----------------------------------------------------------------------------------------
 struct GdnDev { const float* a; const float* dt; const float* conv_w; const float* norm_w; int nk, nv, dk, dv, conv_k; float eps; };
@@ -424,9 +442,10 @@ size_t pyre_gdn_chunk_bytes(const GdnDev& g, int T);
 void   pyre_gdn_chunk_carve(const GdnDev& g, int T, void* base, GdnChunk* b);
 int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int proj_stride, int T, const float* conv_in, float* conv_out,
                           const float* ssm_in, float* ssm_out, float* oraw);
-// the recurrence token by token instead, the bits of pyre_gdn_launch's per-quarter form (conv_in != conv_out; b.co is all it needs)
+// the recurrence token by token instead, the bits of pyre_gdn_launch's per-quarter form (quarters) or of its head-a-workgroup form
+// (conv_in != conv_out; b.co and b.dec are all it needs)
 int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int proj_stride, int T, const float* conv_in, float* conv_out,
-                        const float* ssm_in, float* ssm_out, float* oraw);
+                        const float* ssm_in, float* ssm_out, float* oraw, bool quarters = true);
 
 // ---- gated attention over the KV cache (attn.hip) -----------------------------------------------------------------------
 struct AttnDev { const float* qn; const float* kn; const float* rope_inv; int nh, nkv, hd, n_rot, kv_bits, kv_recent; float eps; float mscale = 1.0f; };   // mscale: YaRN magnitude factor on cos and sin

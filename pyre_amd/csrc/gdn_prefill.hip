@@ -309,6 +309,49 @@ __global__ __launch_bounds__(256) void k_gdn_rec(GdnDev p, const float* __restri
   for (int r = 0; r < R; ++r) ssm_out[so + (size_t)r * p.dv] = S[r];
 }
 
+// The same for layers in the head-a-workgroup form (k_gdn_delta: four groups of 32 rows a column): a quad of lanes a column, a lane its
+// group's 32 rows, the four sums by quad broadcasts in order.  grid (nv, 2), 4 waves: 64 columns a workgroup.
+template <int I> __device__ __forceinline__ float quad_lane(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), I * 0x55, 0xf, 0xf, true)); }
+__device__ __forceinline__ float quad_sum(float x) { return ((quad_lane<0>(x) + quad_lane<1>(x)) + quad_lane<2>(x)) + quad_lane<3>(x); }
+__global__ __launch_bounds__(256) void k_gdn_rec4(GdnDev p, const float* __restrict__ co, const float2* __restrict__ gates, int T, const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
+  constexpr int TB = 8, R = 32;
+  __shared__ __align__(16) float ks[2][TB][4][R + 4], qs[2][TB][4][R + 4];          // (a group's row padded: four groups, four banks)
+  __shared__ float vs[2][TB][64]; __shared__ float2 gb[2][TB];
+  const int h = blockIdx.x, cb = blockIdx.y * 64, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, g = lane & 3;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), jl = wave * 16 + (lane >> 2);
+  const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv, w = p.nv * p.dv;
+  const size_t so = ((size_t)h * DK + g * R) * p.dv + cb + jl;
+  float S[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) S[r] = ssm_in[so + (size_t)r * p.dv];
+  auto load = [&](int t0, int buf) {          // eight tokens: 128 k, 128 q, 64 v each
+    for (int i = tid; i < TB * DK; i += 256) { const int t = min(t0 + i / DK, T - 1), c = i % DK; const float* r = co + (size_t)t * ch + kh * DK + c; ks[buf][i / DK][c >> 5][c & 31] = r[nqk]; qs[buf][i / DK][c >> 5][c & 31] = r[0]; }
+    for (int i = tid; i < TB * 64; i += 256) vs[buf][i >> 6][i & 63] = co[(size_t)min(t0 + (i >> 6), T - 1) * ch + 2 * nqk + (size_t)h * p.dv + cb + (i & 63)];
+    if (tid < TB) gb[buf][tid] = gates[(size_t)min(t0 + tid, T - 1) * p.nv + h];
+  };
+  load(0, 0);
+  lds_barrier();
+  for (int t0 = 0, buf = 0; t0 < T; t0 += TB, buf ^= 1) {
+    if (t0 + TB < T) load(t0 + TB, buf ^ 1);
+    const int n = min(TB, T - t0);
+    for (int t = 0; t < n; ++t) {
+      const float2 gt = gb[buf][t]; const float* k = ks[buf][t][g]; const float* q = qs[buf][t][g];
+      float pm = 0.0f;
+#pragma unroll
+      for (int r = 0; r < R; ++r) { S[r] *= gt.x; pm += S[r] * k[r]; }
+      const float delta = (vs[buf][t][jl] - quad_sum(pm)) * gt.y;
+      float po = 0.0f;
+#pragma unroll
+      for (int r = 0; r < R; ++r) { S[r] += k[r] * delta; po += S[r] * q[r]; }
+      const float o = quad_sum(po);
+      if (g == 0) oraw[(size_t)(t0 + t) * w + (size_t)h * p.dv + cb + jl] = o;
+    }
+    lds_barrier();
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) ssm_out[so + (size_t)r * p.dv] = S[r];
+}
+
 }  // namespace
 
 size_t pyre_gdn_chunk_bytes(const GdnDev& g, int T) {
@@ -335,7 +378,7 @@ int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, con
 }
 
 // the same steps with the recurrence token by token, bit for bit that of the windows' kernels (pyre_gdn_launch with GdnQ); ssm_in == ssm_out is fine, conv_in == conv_out is not
-int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int stride, int T, const float* conv_in, float* conv_out, const float* ssm_in, float* ssm_out, float* oraw) {
+int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int stride, int T, const float* conv_in, float* conv_out, const float* ssm_in, float* ssm_out, float* oraw, bool quarters) {
   if (g.dk != 128 || g.dv != 128) return pyre_fail(ctx, PYRE_E_SHAPE, "gdn prompt: head dims %dx%d unsupported (128x128 only)", g.dk, g.dv);
   if (T < 1 || g.conv_k < 1 || g.conv_k > 8 || conv_in == conv_out) return pyre_fail(ctx, PYRE_E_ARG, "gdn prompt: %d tokens, %d taps", T, g.conv_k);
   const int ch = 2 * g.nk * g.dk + g.nv * g.dv, Tp = (T + 15) / 16 * 16;
@@ -343,6 +386,7 @@ int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const
     if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256 + 1, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr, (float2*)b.dec);
     else hipLaunchKernelGGL(k_gdnc_conv<0>, dim3((ch + 255) / 256 + 1, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr, (float2*)b.dec); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "gdn_prompt_rec", 8.0 * g.nv * g.dk * g.dv + 4.0 * T * (ch + 2.0 * g.nv * g.dv));
-    hipLaunchKernelGGL(k_gdn_rec, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
+    if (!quarters) hipLaunchKernelGGL(k_gdn_rec4, dim3(g.nv, g.dv / 64), dim3(256), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw);
+    else hipLaunchKernelGGL(k_gdn_rec, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
   return PYRE_OK;
 }

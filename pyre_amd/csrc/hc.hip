@@ -67,8 +67,13 @@ template <int T> __device__ __forceinline__ void hc_load_slices(float (&pv)[32],
 //      updated stream (x_out, never the buffer x_in points into)
 //   2. each wave takes upw units of the slice; partial sums -> part[(ks*T + t)*tiles*64 + row]
 template <int FMT, int T, int NP> __global__ __launch_bounds__(512) void k_hc_norm_down(QMatDev m, const float* __restrict__ x_in, int in_ss, int in_ts, float* __restrict__ x_out,
-    const float* __restrict__ comb_out, MoeOut mo, const float* __restrict__ comb_inj, const float* __restrict__ norm, int d, int hc, float* __restrict__ ssq,
+    const float* __restrict__ comb_out, MoeOut mo_in, const float* __restrict__ comb_inj, const float* __restrict__ norm, int d, int hc, float* __restrict__ ssq,
     float* __restrict__ part, int upw, const uint2* __restrict__ g2) {
+  const size_t zt = (size_t)blockIdx.z * T;          // a further group of T tokens (pyre_hc_mix_rows_launch)
+  const MoeOut mo{mo_in.partial ? mo_in.partial + zt * (mo_in.k + 1) * mo_in.d : nullptr, mo_in.sel_w + zt * mo_in.k, mo_in.sg + zt, mo_in.d, mo_in.k};
+  x_in += zt * in_ts; x_out += zt * hc * d; ssq += zt * gridDim.y; part += zt * gridDim.y * ((size_t)m.tiles * 64);
+  if (comb_out) comb_out += zt * d;
+  if (comb_inj) comb_inj += zt * hc;
   const uint2* lds2 = nullptr;          // no format needs a codebook in shared memory any more
   PYRE_TS_VARS PYRE_TS(0);
   qmat_args_now(m); args_now(x_in, in_ss, in_ts, x_out, comb_out, mo.partial, mo.sel_w, mo.sg, mo.d, mo.k, comb_inj, norm, d, hc, ssq, part, upw);
@@ -149,6 +154,10 @@ template <int FMT, int T, int RF> __global__ __launch_bounds__(1024) void k_hc_u
     const float* __restrict__ xnew, const float* __restrict__ norm, float eps, int d, float* __restrict__ mixed, float* __restrict__ inj, const uint2* __restrict__ g2,
     QMatDev router, float* __restrict__ rpart) {
   constexpr bool ROUTE = RF >= 0; constexpr int RFX = ROUTE ? RF : FMT_F32;
+  if (blockIdx.z) {          // a further group of T tokens (pyre_hc_mix_rows_launch)
+    const size_t z = blockIdx.z; part += z * ksplit * T * r64; ssq += z * ksplit * T; xnew += z * T * hc * d; mixed += z * T * d; inj += z * T * hc;
+    if (ROUTE) rpart += z * (d / 64) * T * router.tiles * 64;
+  }
   const uint2* lds2 = nullptr;          // no format needs a codebook in shared memory any more
   PYRE_TS_VARS PYRE_TS(0);
   qmat_args_now(up); args_now(part, ssq, ksplit, r64, lr, hc, has_inject, xnew, norm, eps, d, mixed, inj);
@@ -526,21 +535,21 @@ DownPlan down_plan(const HcDev& h) {
 }
 
 template <int FMT, int T> int norm_down_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const DownPlan& p, const float* x_in, int in_ss, int in_ts, float* x_out,
-                                               const float* comb_out, int comb_parts, const MoeOut& mo, const float* comb_inj, float eps) {
+                                               const float* comb_out, int comb_parts, const MoeOut& mo, const float* comb_inj, float eps, int nz = 1) {
   const int L = p.nw * p.upw * 64; size_t lds = 4 * ((size_t)T * L + (size_t)p.nw * T * 64 + (size_t)p.nw * T);
   ProfScope ps(ctx, "hc_norm_down", qmat_gguf_bytes(h.di, h.di.rows) + 4.0 * T * h.hc * h.d * 4);
-#define NORM_DOWN_GO(NP) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, NP>), dim3(h.di.tiles, p.ksplit), dim3(p.nw * 64), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
+#define NORM_DOWN_GO(NP) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, NP>), dim3(h.di.tiles, p.ksplit, nz), dim3(p.nw * 64), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
                      w.ssq, w.o, p.upw, (const uint2*)ctx->d_iq2xs)
   if constexpr (FMT == FMT_IQ3_S) { if (comb_parts > 1) NORM_DOWN_GO(PYRE_GEMV_PARTS); else NORM_DOWN_GO(1); } else NORM_DOWN_GO(1);
 #undef NORM_DOWN_GO
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
-template <int FMT, int T> int up_mix_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, const float* xnew, float eps, float* mixed, float* inj, const HcRoute* rt) {
+template <int FMT, int T> int up_mix_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, const float* xnew, float eps, float* mixed, float* inj, const HcRoute* rt, int nz = 1) {
   const int nw = h.hc * h.up.U; size_t lds = 4 * ((size_t)T * h.lr + (size_t)nw * T * 64 + (size_t)T * 32 + (size_t)T * h.hc * 64);
   const QMatDev rq = rt ? rt->router : QMatDev{}; float* rp = rt ? rt->part : nullptr;
   ProfScope ps(ctx, rt ? "hc_up_mix_router" : "hc_up_mix", qmat_gguf_bytes(h.up, h.up.rows) + 4.0 * T * (h.hc * h.d + h.d + (double)ksplit * (h.lr + h.hc)) +
                (rt ? qmat_gguf_bytes(rq, rq.rows) + 4.0 * T * (h.d / 64) * rq.tiles * 64 : 0.0));
-#define UP_MIX_GO(RF) hipLaunchKernelGGL((k_hc_up_mix<FMT, T, RF>), dim3(h.d / 64), dim3(nw * 64), lds, ctx->stream, h.up, w.o, w.ssq, ksplit, h.di.tiles * 64, h.lr, h.hc, h.has_inject ? 1 : 0, xnew, h.norm, eps, \
+#define UP_MIX_GO(RF) hipLaunchKernelGGL((k_hc_up_mix<FMT, T, RF>), dim3(h.d / 64, 1, nz), dim3(nw * 64), lds, ctx->stream, h.up, w.o, w.ssq, ksplit, h.di.tiles * 64, h.lr, h.hc, h.has_inject ? 1 : 0, xnew, h.norm, eps, \
                      h.d, mixed, inj, (const uint2*)ctx->d_iq2xs, rq, rp)
   if constexpr (FMT == FMT_IQ3_S || FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {
     if (rt && rq.fmt == FMT_BF16) UP_MIX_GO(FMT_BF16); else if (rt && rq.fmt == FMT_F32) UP_MIX_GO(FMT_F32); else UP_MIX_GO(-1);
@@ -637,6 +646,19 @@ size_t pyre_hc_work_bytes(const HcDev& h) { return 256 * 4 + 2 * 4 * 8 * 32 + 4 
 void pyre_hc_work_carve(const HcDev& h, void* base, HcWork* w) {
   uint8_t* p = (uint8_t*)base; auto take = [&](size_t n) { void* r = p; p += (n + 255) & ~(size_t)255; return r; };
   w->ssq = (float*)take(4 * 8 * 32); w->smx = (float*)take(4 * 8 * 32); w->o = (float*)take(4 * 8 * 32 * ((size_t)h.lr + h.hc + 64));
+}
+
+// groups of eight tokens, the lane = row kernels (a window's launches with a group index in the grid)
+static int hc_rows_split(const HcDev& h) { return down_plan(h).ksplit; }
+bool pyre_hc_rows_ok(const HcDev& h) { int nw, upw, ks; return !hc_on_matrix_cores(h) && pyre_hc_plan(h, &nw, &upw, &ks); }
+size_t pyre_hc_rows_bytes(const HcDev& h, int groups) { return 3 * 256 + 4 * (size_t)groups * hc_rows_split(h) * 8 * (1 + (size_t)h.di.tiles * 64); }
+void pyre_hc_rows_carve(const HcDev& h, int groups, void* base, HcWork* w) { w->ssq = (float*)base; w->smx = nullptr; w->o = (float*)((uint8_t*)base + ((4 * (size_t)groups * hc_rows_split(h) * 8 + 255) & ~(size_t)255)); }
+int pyre_hc_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const float* x_in, int in_ss, int in_ts, float* x_out, int groups, const float* comb_out, const MoeOut* comb_moe, const float* comb_inj,
+                            float eps, float* mixed, float* inj, const HcRoute* rt) {
+  if (!pyre_hc_rows_ok(h) || groups < 1 || groups > 65535 || x_in == x_out || (rt && !pyre_hc_route_ok(h, rt->router))) return pyre_fail(ctx, PYRE_E_ARG, "hc_mix_rows: unsupported shape");
+  const DownPlan p = down_plan(h); const MoeOut mo = comb_moe ? *comb_moe : MoeOut{nullptr, nullptr, nullptr, 0, 0};
+  int rc = [&]() -> int { HC_FMT_SWITCH(h.di.fmt, return (norm_down_launch<F, 8>(ctx, h, w, p, x_in, in_ss, in_ts, x_out, comb_out, 1, mo, comb_inj, eps, groups));) }(); if (rc) return rc;
+  return [&]() -> int { HC_FMT_SWITCH(h.up.fmt, return (up_mix_launch<F, 8>(ctx, h, w, p.ksplit, x_out, eps, mixed, inj, rt, groups));) }();
 }
 
 int pyre_hc_mix_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const float* x_in, int in_ss, int in_ts, float* x_out, int t, const float* comb_out, const MoeOut* comb_moe, const float* comb_inj,

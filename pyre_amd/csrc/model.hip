@@ -511,14 +511,16 @@ static int prompt_pipe_state(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, 
 // ---- a long prompt layer by layer ---------------------------------------------------------------------------------------------
 // Windows of eight tokens share nothing but what fits beside each other on the chip: every window decodes every weight again, and
 // its FFN's 74 of 512 experts.  A call of 72 tokens or more is therefore taken in blocks of up to 2048 tokens, layer by layer, a
-// launch a step for all of a block's tokens: the mixes and projections (prompt.hip), the Gated DeltaNet's recurrence
+// launch a step for all of a block's tokens (shorter calls of more than eight likewise): the mixes and projections (prompt.hip), the Gated DeltaNet's recurrence
 // (gdn_prefill.hip), the attention (k_attn_blk), the FFN grouped by expert (moe.hip).  Every sum is formed in the order of the
 // windows' launches, so a token has a window's bits and the cutting never shows; the one exception is the grouped FFN, whose
 // operands are f16 halves instead of fixed-point digits: it takes the whole groups of eight in front of the call's last eight
-// tokens, the last 8 .. 15 tokens' FFN goes through the windows' launches.
+// tokens, the last 8 .. 15 tokens' FFN (all of it in a call of fewer than 72 tokens) is formed as the windows form it (pyre_moe_rows_launch).
 // For models whose every layer qualifies (prompt_block_ok); PYRE_PROMPT_BLOCK=0 switches it off, PYRE_PROMPT_PAIRS=0 halves the blocks.
 #define PROMPT_BLOCK_MIN 64
 #define PROMPT_BLOCK_MAX 2048
+#define PROMPT_TAIL_MAX 96          // tokens whose FFN a block can take in the windows' form: a call of fewer than 72, or the last ones
+#define PROMPT_ROWS_MAX 512         // tokens of a block of a model in other formats (run_rows)
 static bool fuse_aop_on() { const char* e = getenv("PYRE_AOP_SPLIT"); return !(e && *e && atoi(e) != 0); }
 static bool outp_in_parts(const Layer& L, int d) { return pyre_gemv_parts_ok(L.outp) && (int)L.outp.rows == d && L.hcf.di.fmt == FMT_IQ3_S; }
 // A Gated DeltaNet layer whose output projection is on the matrix cores runs its recurrence on nv x 4 workgroups and leaves
@@ -540,7 +542,7 @@ static bool prompt_block_ok(const pyre_model* m) {
 struct PromptBlk {
   pyre_ctx* ctx = nullptr; void* mem = nullptr; int T_max = 0; size_t blocks = 0;      // room for T_max tokens a block; blocks: pyre_model_prompt_blocks
   float *emb = nullptr, *x = nullptr, *mixed = nullptr, *inj_a = nullptr, *inj_f = nullptr, *proj = nullptr, *o = nullptr, *core = nullptr, *inv = nullptr; uint4* op = nullptr; uint32_t* ids = nullptr;
-  BlkMix mix{}; MoeBlk moe{}; GdnChunk gdn{}; float* q = nullptr; uint16_t* qh = nullptr; float* qsc = nullptr;
+  BlkMix mix{}; MoeBlk moe{}; MoeRows rows{}; HcWork hw{}; GdnChunk gdn{}; float* x2 = nullptr; float* rpart = nullptr; float* q = nullptr; uint16_t* qh = nullptr; float* qsc = nullptr;
   void* att = nullptr; size_t att_bytes = 0;             // the attention's partial sums (grows with the context)
 };
 size_t prompt_blk_count(const PromptBlk* B) { return B->blocks; }
@@ -550,6 +552,24 @@ void prompt_blk_free(PromptBlk* B) {
   if (B->mem) (void)hipFree(B->mem);
   if (B->att) (void)hipFree(B->att);
   delete B;
+}
+// the last of T tokens alone: its pending update and the head, as a window's finish(); x: its streams
+static int prompt_head(pyre_ctx* ctx, const pyre_model* m, PromptBlk* B, const float* x, int T) {
+  const pyre_model_cfg& c = m->c; const int d = c.d; int rc;
+  const MoeOut mol = pyre_moe_rows_out(m->layers.back().moe, B->rows, (T - 1) % 8);
+  const bool fused = fuse_aop_on() && m->out.fmt == FMT_IQ3_S_M && m->out.cols == d && d % 256 == 0 && pyre_hc_aop_ok(m->head);
+  const AopOut aout{m->aop, m->aop_inv, d / 256}; const PyreAop aop{(const uint4*)m->aop, m->aop_inv};
+  if ((rc = pyre_hc_mix_launch(ctx, m->head, m->hw, x, d, c.hc * d, m->x, 1, nullptr, &mol, B->inj_f + (size_t)(T - 1) * c.hc, c.eps, m->hbuf, m->inj_a, nullptr, 1, fused ? &aout : nullptr))) return rc;
+  return pyre_gemv_launch(ctx, m->out, m->hbuf, 1, m->logits, fused ? &aop : nullptr);
+}
+// the attention's partial sums for n positions
+static int prompt_att_get(pyre_ctx* ctx, const pyre_model* m, PromptBlk* B, int n) {
+  if (m->n_attn == 0 || m->has_idx) return PYRE_OK;
+  const pyre_model_cfg& c = m->c; AttnDev a0{nullptr, nullptr, nullptr, c.n_head, c.n_kv, c.hd, c.n_rot, c.kv_bits, c.kv_recent, c.eps};
+  const size_t need = pyre_attn_blk_bytes(a0, n, std::min(n, B->T_max));
+  if (B->att_bytes >= need) return PYRE_OK;
+  if (B->att) { PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); (void)hipFree(B->att); B->att = nullptr; B->att_bytes = 0; }
+  PYRE_HIP(ctx, hipMalloc(&B->att, need + need / 4)); B->att_bytes = need + need / 4; return PYRE_OK;
 }
 // the workspace for blocks of T tokens and a context of n positions: kept by the model, grown when a longer call comes
 static int prompt_blk_get(pyre_ctx* ctx, const pyre_model* m, int T, int n, PromptBlk** out) {
@@ -568,26 +588,106 @@ static int prompt_blk_get(pyre_ctx* ctx, const pyre_model* m, int T, int n, Prom
       auto take = [&](size_t bytes) { void* r = p; bytes = al256(bytes); if (pass) p += bytes; sum += bytes; return r; };
       B->emb = (float*)take(4 * t * d); B->x = (float*)take(4 * t * c.hc * d); B->mixed = (float*)take(4 * t * d); B->inj_a = (float*)take(4 * t * c.hc); B->inj_f = (float*)take(4 * t * c.hc);
       B->proj = (float*)take(4 * t * pmax); B->o = (float*)take(4 * PYRE_GEMV_PARTS * t * d); B->core = (float*)take(4 * t * cmax); B->op = (uint4*)take(4 * t * omax); B->inv = (float*)take(4 * t * (omax / 128)); B->ids = (uint32_t*)take(4 * t);
-      void* mx = take(pyre_blk_mix_bytes(hmax, T)); void* mo = take(pyre_moe_block_bytes(m0, T)); void* gd = take(lin ? pyre_gdn_chunk_bytes(lin->gdn, T) : 0);
+      void* mx = take(pyre_blk_mix_bytes(hmax, T)); void* mo = take(pyre_moe_block_bytes(m0, T)); void* rw = take(pyre_moe_rows_bytes(m0, PROMPT_TAIL_MAX)); void* gd = take(lin ? pyre_gdn_chunk_bytes(lin->gdn, T) : 0);
       float* rpart = (float*)take(4 * rp); float* parts = (float*)take(4 * PYRE_MOE_GROUPS * t * d);
       B->q = (float*)take(4 * t * nq); B->qh = (uint16_t*)take(2 * 2 * t * nq); B->qsc = (float*)take(4 * t * c.n_head);
       if (!pass) { PYRE_HIP(ctx, hipMalloc(&B->mem, sum + 256)); continue; }
-      pyre_blk_mix_carve(hmax, T, mx, &B->mix); pyre_moe_block_carve(m0, T, mo, &B->moe); if (lin) pyre_gdn_chunk_carve(lin->gdn, T, gd, &B->gdn);
+      pyre_blk_mix_carve(hmax, T, mx, &B->mix); pyre_moe_block_carve(m0, T, mo, &B->moe); pyre_moe_rows_carve(m0, PROMPT_TAIL_MAX, rw, &B->rows); if (lin) pyre_gdn_chunk_carve(lin->gdn, T, gd, &B->gdn);
       B->moe.x = B->mixed; B->moe.rpart = rpart; B->moe.parts = parts; B->moe.wr = 8 * (d / 64) * m0.router.tiles * 64;
     }
     PYRE_HIP(ctx, hipMemsetAsync(B->mem, 0, 4096, ctx->stream));
     { int rc = pyre_moe_block_zero_rows(ctx, m0, B->moe, T); if (rc) return rc; }
     B->T_max = T;
   }
-  if (m->n_attn > 0 && !m->has_idx) {
-    AttnDev a0{nullptr, nullptr, nullptr, c.n_head, c.n_kv, c.hd, c.n_rot, c.kv_bits, c.kv_recent, c.eps};
-    const size_t need = pyre_attn_blk_bytes(a0, n, std::min(n, B->T_max));
-    if (B->att_bytes < need) {
-      if (B->att) { PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); (void)hipFree(B->att); B->att = nullptr; B->att_bytes = 0; }
-      PYRE_HIP(ctx, hipMalloc(&B->att, need + need / 4)); B->att_bytes = need + need / 4;
+  return prompt_att_get(ctx, m, B, n);
+}
+// ---- the same for models in other formats -----------------------------------------------------------------------------------------
+// Hyper-connection matrices in bf16 (as files store them) or matrices other than IQ3_S have lane = row kernels for windows of eight:
+// a launch of one window fills a fraction of the chip, and three windows in flight still left a 200-token prompt of a Q4_K
+// model at 110 ms.  run_rows launches every step once for all of a block's windows (a group index in the grid; the
+// recurrence, the attention and the expert products over all tokens): the windows' kernels, the windows' bits.
+// Rows of the last group past the prompt are computed on whatever finite values they hold; nobody reads them.
+static bool prompt_rows_ok(const pyre_model* m) {
+  if (!prompt_block_env()) return false;
+  const pyre_model_cfg& c = m->c;
+  if (m->n_ple > 0 || m->has_idx || c.top_k > PYRE_MOE_KMAX || c.d % 256 || c.conv_k < 2 || c.conv_k > 8 || c.hd != 256) return false;
+  { const char* e = getenv("PYRE_ROUTER_RIDES"); if (e && *e && atoi(e) == 0) return false; }
+  for (int il = 0; il < c.n_layers; ++il) { const Layer& L = m->layers[il]; const MoeDev& m0 = m->layers[0].moe;
+    if (!pyre_moe_rows_ok(L.moe) || L.moe.router.tiles != m0.router.tiles || L.moe.ff != m0.ff || L.moe.sf != m0.sf || L.moe.top_k != m0.top_k || L.moe.n_exp != m0.n_exp || !pyre_hc_rows_ok(L.hca) || !pyre_hc_rows_ok(L.hcf) ||
+        !pyre_hc_route_ok(L.hcf, L.moe.router) || outp_in_parts(L, c.d) || L.proj.cols % 256 || L.outp.cols % 256 || (int)L.outp.rows != c.d || (!L.full && (L.gdn.dk != 128 || L.gdn.dv != 128 || (L.outp.fmt == FMT_IQ3_S_M) != gdn_q_on(m, L)))) return false; }
+  return true;
+}
+static int prompt_rows_get(pyre_ctx* ctx, const pyre_model* m, int T, int n, PromptBlk** out) {
+  pyre_model* mm = const_cast<pyre_model*>(m); const pyre_model_cfg& c = m->c;
+  if (!mm->blk) { mm->blk = new PromptBlk(); mm->blk->ctx = ctx; }
+  PromptBlk* B = mm->blk; *out = B;
+  if (B->T_max < T) {
+    if (B->mem) { PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); (void)hipFree(B->mem); B->mem = nullptr; B->T_max = 0; }
+    T = T <= 128 ? 128 : PROMPT_ROWS_MAX;
+    const MoeDev& m0 = m->layers[0].moe; const Layer* lin = nullptr; for (const Layer& L : m->layers) if (!L.full) lin = &L;
+    const size_t t = T, d = c.d, nq = (size_t)c.n_head * c.hd, cmax = std::max((size_t)c.lin_nv * c.lin_dv, nq), omax = std::max(d, cmax), pmax = std::max(m->pw_lin, m->pw_attn); size_t total = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+      uint8_t* p = (uint8_t*)B->mem; size_t sum = 0;
+      auto take = [&](size_t bytes) { void* r = p; bytes = al256(bytes); if (pass) p += bytes; sum += bytes; return r; };
+      B->emb = (float*)take(4 * t * d); B->x = (float*)take(4 * t * c.hc * d); B->x2 = (float*)take(4 * t * c.hc * d); B->mixed = (float*)take(4 * t * d); B->inj_a = (float*)take(4 * t * c.hc); B->inj_f = (float*)take(4 * t * c.hc);
+      B->proj = (float*)take(4 * t * pmax); B->o = (float*)take(4 * t * d); B->core = (float*)take(4 * t * cmax); B->op = (uint4*)take(4 * t * omax); B->inv = (float*)take(4 * t * (omax / 128)); B->ids = (uint32_t*)take(4 * t);
+      void* hw = take(pyre_hc_rows_bytes(m->layers[0].hca, T / 8)); void* rw = take(pyre_moe_rows_bytes(m0, T)); void* gd = take(lin ? pyre_gdn_chunk_bytes(lin->gdn, T) : 0);
+      B->rpart = (float*)take(4 * t * (d / 64) * m0.router.tiles * 64); B->q = (float*)take(4 * t * nq); B->qh = (uint16_t*)take(2 * 2 * t * nq); B->qsc = (float*)take(4 * t * c.n_head);
+      if (!pass) { PYRE_HIP(ctx, hipMalloc(&B->mem, sum + 256)); total = sum; continue; }
+      pyre_hc_rows_carve(m->layers[0].hca, T / 8, hw, &B->hw); pyre_moe_rows_carve(m0, T, rw, &B->rows); if (lin) pyre_gdn_chunk_carve(lin->gdn, T, gd, &B->gdn);
     }
+    PYRE_HIP(ctx, hipMemsetAsync(B->mem, 0, total, ctx->stream));          // (the rows past a prompt start finite)
+    B->T_max = T;
   }
-  return PYRE_OK;
+  return prompt_att_get(ctx, m, B, n);
+}
+static int run_rows(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBlk* B, const uint32_t* ids, int T, bool head) {
+  const pyre_model_cfg& c = m->c; const int d = c.d, hc = c.hc, start = s->len, G = (T + 7) / 8; int rc;
+  PYRE_HIP(ctx, hipMemcpyAsync(B->ids, ids, (size_t)T * 4, hipMemcpyHostToDevice, ctx->stream));
+  if (s->tokens_dev) PYRE_HIP(ctx, hipMemcpyAsync(s->tokens_dev + start, B->ids, (size_t)T * 4, hipMemcpyDeviceToDevice, ctx->stream));
+  if ((rc = pyre_row_launch(ctx, m->embd, B->ids, T, B->emb, d))) return rc;
+  const float* xin = B->emb; int in_ss = 0, in_ts = d; float* xout = B->x; float* xother = B->x2; const MoeOut* comb = nullptr; const float* cinj = nullptr;
+  const int r64 = m->layers[0].moe.router.tiles * 64; const size_t wr = (size_t)8 * (d / 64) * r64; const MoeOut all = pyre_moe_rows_out(m->layers[0].moe, B->rows, 0);
+  auto advance = [&]() { xin = xout; in_ss = d; in_ts = hc * d; std::swap(xout, xother); };
+  // a matrix over all tokens: the lane = row product in groups of eight, or the matrix cores behind a split
+  auto mul = [&](const QMatDev& q, const float* x, float* y) -> int {
+    if (q.fmt != FMT_IQ3_S_M) return pyre_gemv_rows_launch(ctx, q, x, G, y);
+    int r = pyre_blk_op_split_launch(ctx, x, q.cols, T, B->op, (size_t)q.cols * 2, B->inv, q.cols / 32); if (r) return r;
+    return pyre_blk_gemm_launch(ctx, q, B->op, (size_t)q.cols * 2, B->inv, q.cols / 32, PYRE_INV_BLOCK, y, (int)q.rows, T, 1);
+  };
+  for (int il = 0; il < c.n_layers; ++il) {
+    const Layer& L = m->layers[il]; const int oc = L.outp.cols, pw = (int)L.proj.rows;
+    if ((rc = pyre_hc_mix_rows_launch(ctx, L.hca, B->hw, xin, in_ss, in_ts, xout, G, nullptr, comb, cinj, c.eps, B->mixed, B->inj_a, nullptr))) return rc;
+    advance();
+    if ((rc = mul(L.proj, B->mixed, B->proj))) return rc;
+    if (L.full) {
+      const int ai = L.mix_index;
+      if ((rc = pyre_attn_blk_prep(ctx, L.attn, s->kv[ai], B->proj, pw, start, T, &s->packed[ai], B->q, B->qh, B->qsc))) return rc;
+      if (pyre_attn_blk_bytes(L.attn, start + T, T) > B->att_bytes) return pyre_fail(ctx, PYRE_E_STATE, "forward: attention scratch of %zu bytes is too small", B->att_bytes);
+      if ((rc = pyre_attn_blk_launch(ctx, L.attn, s->kv[ai], B->q, B->qh, B->qsc, B->proj, pw, start, T, B->att, B->core))) return rc;
+      if ((rc = mul(L.outp, B->core, B->o))) return rc;
+    } else {
+      const int li = L.mix_index, b = s->cur[li], nb = b ^ 1; const bool q = gdn_q_on(m, L);
+      if ((rc = pyre_gdn_rec_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], q ? B->core : (float*)B->op, q))) return rc;
+      s->cur[li] = nb;
+      if (q) {
+        if ((rc = pyre_blk_gdn_out_q_launch(ctx, B->core, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, B->op, (size_t)oc * 2, B->inv, oc / 16))) return rc;
+        if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, (size_t)oc * 2, B->inv, oc / 16, PYRE_INV_CHUNK, B->o, d, T, 1))) return rc;
+      } else {
+        if ((rc = pyre_blk_gdn_out_w_launch(ctx, (float*)B->op, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, B->core))) return rc;
+        if ((rc = mul(L.outp, B->core, B->o))) return rc;
+      }
+    }
+    const HcRoute hr{L.moe.router, B->rpart, nullptr};
+    if ((rc = pyre_hc_mix_rows_launch(ctx, L.hcf, B->hw, xin, in_ss, in_ts, xout, G, B->o, nullptr, B->inj_a, c.eps, B->mixed, B->inj_f, &hr))) return rc;
+    advance();
+    const bool end = il == c.n_layers - 1; const int i0 = end ? (T - 1) / 8 * 8 : 0;
+    if (end && !head) break;          // nobody reads the last layer's FFN
+    if ((rc = pyre_moe_rows_launch(ctx, L.moe, B->rows, B->mixed + (size_t)i0 * d, T - i0, B->rpart + (size_t)(i0 / 8) * wr, wr, d / 64, r64, nullptr))) return rc;
+    comb = &all; cinj = B->inj_f;
+  }
+  s->len = start + T;
+  return head ? prompt_head(ctx, m, B, xin + (size_t)(T - 1) * hc * d, T) : PYRE_OK;
 }
 // T tokens (ids on the host) behind the state's length; tail: the last of them whose FFN takes the windows' launches (0: none;
 // T - tail is a multiple of eight); head: the last token's logits to m->logits
@@ -630,17 +730,13 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
     const bool end = il == c.n_layers - 1;
     if (end && !head) break;          // nobody reads the last layer's FFN
     if ((rc = pyre_moe_block_launch(ctx, L.moe, B->moe, end ? 0 : Tb, T, B->T_max, d / 64, r64))) return rc;
-    for (int i = end ? (T - 1) / 8 * 8 : Tb; i < T; i += 8) if ((rc = pyre_moe_block_window(ctx, L.moe, m->mw, B->moe, i, std::min(8, T - i), d / 64, r64, end))) return rc;
+    const int i0 = end ? (T - 1) / 8 * 8 : Tb;          // (the last layer: the last group's terms, for the head)
+    if (i0 < T && (rc = pyre_moe_rows_launch(ctx, L.moe, B->rows, B->mixed + (size_t)i0 * d, T - i0, B->moe.rpart + (size_t)(i0 / 8) * B->moe.wr, B->moe.wr, d / 64, r64, end ? nullptr : B->moe.parts + (size_t)(i0 / 8) * PYRE_MOE_GROUPS * 8 * d))) return rc;
     comb = B->moe.parts; np = PYRE_MOE_GROUPS; cinj = B->inj_f;
   }
   s->len = start + T;
   if (!head) return PYRE_OK;
-  // the last token alone: its pending update and the head, as a window's finish()
-  const MoeOut mol = pyre_moe_out(m->layers.back().moe, m->mw, (T - 1) % 8); const size_t last = (size_t)(T - 1) * hc * d;
-  const bool fused = fuse_aop_on() && m->out.fmt == FMT_IQ3_S_M && m->out.cols == d && pyre_hc_aop_ok(m->head);
-  const AopOut aout{m->aop, m->aop_inv, d / 256}; const PyreAop aop{(const uint4*)m->aop, m->aop_inv};
-  if ((rc = pyre_hc_mix_launch(ctx, m->head, m->hw, B->x + last, d, hc * d, m->x, 1, nullptr, &mol, B->inj_f + (size_t)(T - 1) * hc, c.eps, m->hbuf, m->inj_a, nullptr, 1, fused ? &aout : nullptr))) return rc;
-  return pyre_gemv_launch(ctx, m->out, m->hbuf, 1, m->logits, fused ? &aop : nullptr);
+  return prompt_head(ctx, m, B, B->x + (size_t)(T - 1) * hc * d, T);
 }
 
 namespace {
@@ -848,18 +944,33 @@ int pyre_forward(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, const uint32
   const bool windows_only = [] { const char* e = getenv("PYRE_PROMPT_WINDOWS"); return e && *e && atoi(e) != 0; }();      // (read per call: 1 = this call in windows, whatever layouts the model keeps)
   // whole groups of eight in front of the call's last tokens; those follow in the last block, with a drafter, whose ring keeps their residual streams, in windows
   const int nblk_ffn = std::max(0, n - 8 - (s->mtp ? mtp_window_of(s->mtp) : 0)) / 8 * 8, nblk_tok = s->mtp ? nblk_ffn : n;
-  if (!windows_only && nblk_ffn >= PROMPT_BLOCK_MIN && prompt_block_ok(m)) {
+  const bool small = nblk_ffn < PROMPT_BLOCK_MIN;          // too few tokens to group by expert: all of the FFN in the windows' form, one block
+  if (!windows_only && n > 8 && !(small && s->mtp) && prompt_block_ok(m)) {
     const bool pairs = [] { const char* e = getenv("PYRE_PROMPT_PAIRS"); return !(e && *e && atoi(e) == 0); }();      // PYRE_PROMPT_PAIRS=0: blocks of up to 1024 tokens instead of 2048
-    const int most = pairs ? PROMPT_BLOCK_MAX : PROMPT_BLOCK_MAX / 2, nb = (nblk_ffn + most - 1) / most, groups = nblk_ffn / 8;      // blocks of (nearly) equal size, the last with up to fifteen tokens more
+    const int most = pairs ? PROMPT_BLOCK_MAX : PROMPT_BLOCK_MAX / 2, ffn = small ? 0 : nblk_ffn, nb = std::max(1, (ffn + most - 1) / most), groups = ffn / 8;      // blocks of (nearly) equal size, the last with up to fifteen tokens more
     PromptBlk* B = nullptr;
-    if ((rc = prompt_blk_get(ctx, m, (groups + nb - 1) / nb * 8 + nblk_tok - nblk_ffn, s->len + n, &B))) return rc;
+    if ((rc = prompt_blk_get(ctx, m, (groups + nb - 1) / nb * 8 + nblk_tok - ffn, s->len + n, &B))) return rc;
     for (int k = 0; k < nb; ++k) {
-      const int tail = k + 1 == nb ? nblk_tok - nblk_ffn : 0, T = 8 * (int)((int64_t)groups * (k + 1) / nb - (int64_t)groups * k / nb) + tail; const bool head = logits_host && i_first + T == n;
+      const int tail = k + 1 == nb ? nblk_tok - ffn : 0, T = 8 * (int)((int64_t)groups * (k + 1) / nb - (int64_t)groups * k / nb) + tail; const bool head = logits_host && i_first + T == n;
       if ((rc = run_block(ctx, m, s, B, ids + i_first, T, tail, head))) { s->broken = true; (void)hipStreamSynchronize(ctx->stream); return rc; }
       i_first += T;
     }
     // what pyre_model_prompt_blocks counts: the whole windows in front of the call's last eight tokens in blocks of at most 128, an even number of them when taken in pairs
-    const int wins = (n - 8 - (s->mtp ? mtp_window_of(s->mtp) : 0)) / 8; int cnt = pairs ? 2 * ((wins + 255) / 256) : (wins + 127) / 128; while (cnt > 1 && wins / cnt < 8) --cnt; B->blocks += cnt;
+    const int wins = (n - 8 - (s->mtp ? mtp_window_of(s->mtp) : 0)) / 8; int cnt = pairs ? 2 * ((wins + 255) / 256) : (wins + 127) / 128; while (cnt > 1 && wins / cnt < 8) --cnt; if (!small) B->blocks += cnt;
+    if (i_first == n) {
+      if (logits_host) PYRE_HIP(ctx, hipMemcpyAsync(logits_host, m->logits, (size_t)m->c.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
+      PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); return PYRE_OK;
+    }
+  }
+  const int nrow = s->mtp ? nblk_ffn : n;
+  if (i_first == 0 && !windows_only && nrow > 8 && prompt_rows_ok(m)) {
+    PromptBlk* B = nullptr;
+    if ((rc = prompt_rows_get(ctx, m, std::min(nrow, PROMPT_ROWS_MAX), s->len + n, &B))) return rc;
+    while (i_first < nrow) {
+      const int T = std::min(nrow - i_first, PROMPT_ROWS_MAX);
+      if ((rc = run_rows(ctx, m, s, B, ids + i_first, T, logits_host && i_first + T == n))) { s->broken = true; (void)hipStreamSynchronize(ctx->stream); return rc; }
+      i_first += T;
+    }
     if (i_first == n) {
       if (logits_host) PYRE_HIP(ctx, hipMemcpyAsync(logits_host, m->logits, (size_t)m->c.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
       PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); return PYRE_OK;

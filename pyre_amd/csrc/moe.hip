@@ -139,10 +139,13 @@ __device__ __forceinline__ void route_weights(int k, RouteLds& L) {
 // time (the launcher checks them) -- same arithmetic.
 // ID (IQ3_S): the dot products in the integer form of digits.h -- 1.4 vector instructions a weight where byte -> float and
 // multiply-add take 3; dgx holds the digits of the window's activations, token ti at dgx + ti * (d / 64) * DGX_STRIDE.
+// perm (a launch for hundreds of tokens): workgroup y takes entry perm[y], the routed entries by expert, so that an expert's
+// weights are in the second-level caches for all of its tokens; the shared expert's entries follow
+__device__ __forceinline__ int entry_of(const int32_t* __restrict__ perm, int y, int T, int top_k) { return __builtin_amdgcn_readfirstlane(y < T * top_k ? perm[y] : (y - T * top_k) * (top_k + 1) + top_k); }
 template <int FMT, int NW, int P, bool PRE, bool FIX = false, bool ID = false>
 __global__ __launch_bounds__(NW * 64, (PRE && P == 2 && FMT >= 5 && FMT <= 7) ? 8 : 1) void k_moe_gu(MoeDev m, const float* __restrict__ logits, int32_t* __restrict__ sel_idx, float* __restrict__ sel_w, float* __restrict__ sg,
                                                    const float* __restrict__ x, float* __restrict__ h, int hstride, const uint2* __restrict__ g2, int nsl, int sstride, int tstride, const uint32_t* __restrict__ dgx,
-                                                   uint32_t* __restrict__ dgh) {
+                                                   uint32_t* __restrict__ dgh, const int32_t* __restrict__ perm) {
   static_assert(!ID || FMT == FMT_IQ3_S, "the integer form is IQ3_S's");
   const uint2* lds2 = nullptr;          // no format needs a codebook in shared memory any more
   PYRE_TS_VARS PYRE_TS(0);
@@ -152,7 +155,9 @@ __global__ __launch_bounds__(NW * 64, (PRE && P == 2 && FMT >= 5 && FMT <= 7) ? 
   __shared__ float red[2][P][NW][64];
   __shared__ RouteLds rl;
   __shared__ uint8_t hsm[ID ? 3 : 1][64];
-  const int entry = blockIdx.y, k1 = top_k + 1, ti = entry / k1, j = entry % k1;
+  const int k1 = top_k + 1; int entry = blockIdx.y;
+  if constexpr (PRE) if (perm) entry = entry_of(perm, entry, (int)gridDim.y / k1, top_k);
+  const int ti = entry / k1, j = entry % k1;
   const bool shared = j == top_k;
   const int nrows = shared ? m.sf : ff;
   if ((int)blockIdx.x * 64 >= nrows) return;
@@ -271,7 +276,7 @@ __global__ __launch_bounds__(1024) void k_moe_route(MoeDev m, const float* __res
 // the wave that forms the unit's values (NZ > 1); the same digits either way, so a token's bits do not depend on the form.
 template <int FMT, int NW, int NZ, bool FIX = false, bool ID = false>
 __global__ __launch_bounds__(NW * 64) void k_moe_down(MoeDev m, const int32_t* __restrict__ sel_idx, const float* __restrict__ h, int hstride, float* __restrict__ partial,
-                                                     const uint2* __restrict__ g2, const uint32_t* __restrict__ dgh) {
+                                                     const uint2* __restrict__ g2, const uint32_t* __restrict__ dgh, const int32_t* __restrict__ perm) {
   static_assert(!ID || FMT == FMT_IQ3_S, "the integer form is IQ3_S's");
   const uint2* lds2 = nullptr;          // no format needs a codebook in shared memory any more
   PYRE_TS_VARS PYRE_TS(0);
@@ -281,7 +286,9 @@ __global__ __launch_bounds__(NW * 64) void k_moe_down(MoeDev m, const int32_t* _
   __shared__ float hx[(NZ > 1 && !ID) ? NW : 1][64];
   __shared__ __align__(16) uint32_t hdg[(NZ > 1 && ID) ? NW : 1][DGX_STRIDE];
   __shared__ uint8_t hsm[(NZ > 1 && ID) ? NW : 1][3][64];
-  const int entry = blockIdx.y, k1 = top_k + 1, ti = entry / k1, j = entry % k1;
+  const int k1 = top_k + 1; int entry = blockIdx.y;
+  if constexpr (NZ == 1) if (perm) entry = entry_of(perm, entry, (int)gridDim.y / k1, top_k);
+  const int ti = entry / k1, j = entry % k1;
   const bool shared = j == top_k;
   const QMatDev& D = shared ? m.sh_down : m.down_e;
   const int tile = (shared ? 0 : sel_idx[ti * top_k + j] * (d >> 6)) + blockIdx.x;
@@ -460,6 +467,8 @@ void pyre_moe_work_carve(const MoeDev& m, void* base, MoeWork* w) {
     case FMT_C4: { constexpr int F = FMT_C4; CALL; } break; case FMT_C8: { constexpr int F = FMT_C8; CALL; } break; \
     default: { constexpr int F = FMT_IQ3_S; CALL; } break; }
 
+static bool moe_idot() { static const bool on = !(getenv("PYRE_MOE_IDOT") && atoi(getenv("PYRE_MOE_IDOT")) == 0); return on; }
+static bool moe_idot_gu_only() { static const bool on = getenv("PYRE_MOE_IDOT") && atoi(getenv("PYRE_MOE_IDOT")) == 1; return on; }
 // K parts of the gate/up dot products (a property of the matrices, so that every window length gives a token the
 // same bits) and whether a window of t tokens launches one workgroup per part: only a single token does, whose
 // tiles x (k+1) workgroups would leave most of the chip idle.
@@ -474,26 +483,24 @@ int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const floa
   if (routed && (routed->nsl < 1 || routed->nsl > 64 || routed->r64 < m.n_exp)) return pyre_fail(ctx, PYRE_E_ARG, "moe_ffn: %d router slices of %d rows", routed->nsl, routed->r64);
   if (t > 1 && getenv("PYRE_DEBUG_SKIP_MOE")) return PYRE_OK;
   if (!routed) { int rc = pyre_gemv_launch(ctx, m.router, x, t, w.logits); if (rc) return rc; }
-  const float* lg = routed ? routed->p : w.logits; const int nsl = routed ? routed->nsl : 1, sstride = routed ? (routed->st ? routed->st : t) * routed->r64 : 0, tstride = routed ? routed->r64 : m.n_exp;
+  const float* lg = routed ? routed->p : w.logits; const int nsl = routed ? routed->nsl : 1, sstride = routed ? t * routed->r64 : 0, tstride = routed ? routed->r64 : m.n_exp;
   auto mat_bytes = [](const QMatDev& q, double rows) { return qmat_gguf_bytes(q, rows); };
   const int hs = m.ff > m.sf ? m.ff : m.sf, entries = t * (m.top_k + 1);
   const uint2* g2 = (const uint2*)ctx->d_iq2xs;
   const int P = pyre_moe_gu_parts(m), nz = (P > 1 && t == 1) ? P : 1;
   // IQ3_S experts: gate/up in the integer form, on the digits the mix left beside the activations or on a launch of their own
-  static const bool idot_on = !(getenv("PYRE_MOE_IDOT") && atoi(getenv("PYRE_MOE_IDOT")) == 0);
-  const bool idot = idot_on && m.gate_e.fmt == FMT_IQ3_S && m.sh_gate.fmt == FMT_IQ3_S;
+  const bool idot = moe_idot() && m.gate_e.fmt == FMT_IQ3_S && m.sh_gate.fmt == FMT_IQ3_S;
   const uint32_t* dgx = nullptr;
   if (idot) {
     if (routed && routed->dgx) dgx = routed->dgx;
     else { ProfScope ps(ctx, "moe_digits", 4.0 * t * m.d * 2); hipLaunchKernelGGL(k_act_digits_eo, dim3(m.d / 64, t), dim3(64), 0, ctx->stream, x, m.d, w.dgx); PYRE_CHECK_LAUNCH(ctx); dgx = w.dgx; }
   }
   // ... and the down products on the digits of h, which a window's gate/up launch leaves and a single token's down launch forms
-  static const bool idot_gu_only = getenv("PYRE_MOE_IDOT") && atoi(getenv("PYRE_MOE_IDOT")) == 1;
-  const bool idot_dn = idot && !idot_gu_only && m.down_e.fmt == FMT_IQ3_S && m.sh_down.fmt == FMT_IQ3_S;
+  const bool idot_dn = idot && !moe_idot_gu_only() && m.down_e.fmt == FMT_IQ3_S && m.sh_down.fmt == FMT_IQ3_S;
   uint32_t* dgh = idot_dn ? w.dgh : nullptr;
   const bool a3b = t == 1 && m.gate_e.fmt == FMT_IQ3_S && m.down_e.fmt == FMT_IQ3_S && m.n_exp == 512 && m.top_k == 10 && m.d == 2048 && m.ff == 512 && m.sf == 512;          // the instances with these constants folded in
   { ProfScope ps(ctx, "moe_route_gate_up", t * (2.0 * m.top_k * mat_bytes(m.gate_e, m.ff) + 2.0 * mat_bytes(m.sh_gate, m.sf)) + 4.0 * t * (m.n_exp + 2.0 * m.d));
-#define GU_ARGS(NZ) dim3(hs / 64, entries, NZ), dim3(16 * 64), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, w.sg, x, w.h, hs, g2, nsl, sstride, tstride, dgx, dgh
+#define GU_ARGS(NZ) dim3(hs / 64, entries, NZ), dim3(16 * 64), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, w.sg, x, w.h, hs, g2, nsl, sstride, tstride, dgx, dgh, (const int32_t*)nullptr
 #define GU_GO(PP, NZ, PRE) do { if (idot) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, PP, PRE, false, true>), GU_ARGS(NZ)); else MOE_FMT_DISPATCH(m.gate_e.fmt, hipLaunchKernelGGL((k_moe_gu<F, 16, PP, PRE>), GU_ARGS(NZ))); } while (0)
   if (t == 1 && a3b && nsl == 32 && nz == 2) { if (idot) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 1, false, true, true>), GU_ARGS(2)); else hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 1, false, true>), GU_ARGS(2)); }
   else if (t == 1) { GU_GO(1, nz, false); }          // the selection inside the launch; one workgroup per K part
@@ -519,7 +526,7 @@ int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const floa
 #undef DOWN_G_ARGS
 #undef DOWN_G_GO
   }
-#define DOWN_ARGS dim3(m.d / 64, entries), dim3(8 * 64), 0, ctx->stream, m, w.sel_idx, w.h, hs, w.partial, g2, dgh
+#define DOWN_ARGS dim3(m.d / 64, entries), dim3(8 * 64), 0, ctx->stream, m, w.sel_idx, w.h, hs, w.partial, g2, dgh, (const int32_t*)nullptr
   else if (a3b && nz == 2) { if (idot_dn) hipLaunchKernelGGL((k_moe_down<FMT_IQ3_S, 8, 2, true, true>), DOWN_ARGS); else hipLaunchKernelGGL((k_moe_down<FMT_IQ3_S, 8, 2, true>), DOWN_ARGS); }
   else if (idot_dn) { if (nz == 1) hipLaunchKernelGGL((k_moe_down<FMT_IQ3_S, 8, 1, false, true>), DOWN_ARGS); else hipLaunchKernelGGL((k_moe_down<FMT_IQ3_S, 8, 2, false, true>), DOWN_ARGS); }
   else if (nz == 1) { MOE_FMT_DISPATCH(m.down_e.fmt, hipLaunchKernelGGL((k_moe_down<F, 8, 1>), DOWN_ARGS)); }
@@ -851,19 +858,47 @@ int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T
   return PYRE_OK;
 }
 
-// Tokens i0 .. i0 + t - 1 (t <= 8, one group) of a block through the windows' launches instead: their bits are a window's (the digits
-// form of the experts).  The router's sums are there (pyre_moe_block_launch has been called for the block).
-// raw: the unreduced terms stay in w (pyre_moe_out), no group sums.
-int pyre_moe_block_window(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const MoeBlk& b, int i0, int t, int nsl, int r64, bool raw) {
-  if (i0 % 8 || t < 1 || t > 8) return pyre_fail(ctx, PYRE_E_ARG, "moe block: a window of %d tokens at %d", t, i0);
-  const RouteSrc rs{b.rpart + (size_t)(i0 / 8) * b.wr, nsl, r64, nullptr, 8};
-  float* parts = b.parts + (size_t)(i0 / 8) * PYRE_MOE_GROUPS * 8 * m.d;
-  MoeWork w2 = w; if (t == 8) w2.parts = parts;
-  int rc = pyre_moe_launch(ctx, m, w2, b.x + (size_t)i0 * m.d, t, nullptr, &rs, t == 8 && !raw); if (rc || t == 8 || raw) return rc;
-  MoeBlk o = b; o.partial = w.partial; o.sel_w = w.sel_w; o.sg = w.sg; o.parts = parts;          // fewer than eight: the terms first, then their groups
-  ProfScope ps(ctx, "moe_block_groups", 4.0 * t * m.d * (m.top_k + 5));
-  hipLaunchKernelGGL(k_moe_groups_blk, dim3((m.d + 255) / 256, t), dim3(256), 0, ctx->stream, m, o, t);
-  PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
+// The windows' arithmetic (k_moe_gu / k_moe_down, the digits form for IQ3_S experts) for any number of tokens in one set of launches,
+// entry by entry in the order of the experts: a prompt of a model whose experts have no matrix-core layout, and the last tokens of
+// one whose experts have.  Router sums as in MoeBlk (rpart + group * wr).  parts: the group sums [group][PYRE_MOE_GROUPS][8][d], or
+// null: the unreduced terms stay in w (pyre_moe_out).
+size_t pyre_moe_rows_bytes(const MoeDev& m, int T) {
+  const size_t hs = (size_t)(m.ff > m.sf ? m.ff : m.sf), k1 = m.top_k + 1, n = T;
+  return 256 * 12 + 4 * (3 * n * m.top_k + n + 1024 + n * k1 * (hs + m.d) + n * (m.d / 64) * DGX_STRIDE + n * k1 * (hs / 64) * DGX_STRIDE);
+}
+void pyre_moe_rows_carve(const MoeDev& m, int T, void* base, MoeRows* w) {
+  uint8_t* p = (uint8_t*)base; auto take = [&](size_t n) { void* r = p; p += (4 * n + 255) & ~(size_t)255; return r; };
+  const size_t hs = (size_t)(m.ff > m.sf ? m.ff : m.sf), k1 = m.top_k + 1, n = T;
+  w->sel_idx = (int32_t*)take(n * m.top_k); w->sel_w = (float*)take(n * m.top_k); w->elist = (int32_t*)take(n * m.top_k); w->sg = (float*)take(n); w->eoff = (int32_t*)take(1024);
+  w->h = (float*)take(n * k1 * hs); w->partial = (float*)take(n * k1 * m.d); w->dgx = (uint32_t*)take(n * (m.d / 64) * DGX_STRIDE); w->dgh = (uint32_t*)take(n * k1 * (hs / 64) * DGX_STRIDE);
+}
+bool pyre_moe_rows_ok(const MoeDev& m) { return m.top_k <= PYRE_MOE_KMAX && m.n_exp <= 1023 && m.d % 64 == 0; }
+int pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const float* x, int T, const float* rpart, size_t wr, int nsl, int r64, float* parts) {
+  if (!pyre_moe_rows_ok(m) || T < 1 || T * (m.top_k + 1) > 65535 || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe rows: unsupported shape (T = %d, %d router slices)", T, nsl);
+  MoeBlk b{}; b.rpart = rpart; b.wr = wr; b.parts = parts; b.sel_idx = w.sel_idx; b.sel_w = w.sel_w; b.eoff = w.eoff; b.elist = w.elist; b.partial = w.partial; b.sg = w.sg;
+  const int hs = m.ff > m.sf ? m.ff : m.sf, entries = T * (m.top_k + 1), P = pyre_moe_gu_parts(m);
+  const uint2* g2 = (const uint2*)ctx->d_iq2xs;
+  const bool idot = moe_idot() && m.gate_e.fmt == FMT_IQ3_S && m.sh_gate.fmt == FMT_IQ3_S, idot_dn = idot && !moe_idot_gu_only() && m.down_e.fmt == FMT_IQ3_S && m.sh_down.fmt == FMT_IQ3_S;
+  uint32_t* dgh = idot_dn ? w.dgh : nullptr;
+  { ProfScope ps(ctx, "moe_rows_route", 4.0 * T * nsl * m.n_exp);
+    if (m.n_exp == 512 && m.top_k == 10 && nsl == 32) hipLaunchKernelGGL(k_moe_route_blk<true>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64); else hipLaunchKernelGGL(k_moe_route_blk<false>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64);
+    hipLaunchKernelGGL(k_moe_lists, dim3(1), dim3(1024), 0, ctx->stream, m, b, T);
+    if (idot) hipLaunchKernelGGL(k_act_digits_eo, dim3(m.d / 64, T), dim3(64), 0, ctx->stream, x, m.d, w.dgx); } PYRE_CHECK_LAUNCH(ctx);
+  { ProfScope ps(ctx, "moe_rows_gate_up", T * (2.0 * m.top_k * qmat_gguf_bytes(m.gate_e, m.ff) + 2.0 * qmat_gguf_bytes(m.sh_gate, m.sf)));
+#define ROWS_GU dim3(hs / 64, entries, 1), dim3(16 * 64), 0, ctx->stream, m, (const float*)nullptr, w.sel_idx, w.sel_w, w.sg, x, w.h, hs, g2, nsl, 0, 0, w.dgx, dgh, w.elist
+    const bool fix = m.gate_e.fmt == FMT_IQ3_S && m.down_e.fmt == FMT_IQ3_S && m.n_exp == 512 && m.top_k == 10 && m.d == 2048 && m.ff == 512 && m.sf == 512 && nsl == 32;
+    if (idot && fix && P == 2) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, true, true>), ROWS_GU);
+    else if (idot) { if (P == 2) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, false, true>), ROWS_GU); else hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 1, true, false, true>), ROWS_GU); }
+    else { MOE_FMT_DISPATCH(m.gate_e.fmt, if (P == 2) hipLaunchKernelGGL((k_moe_gu<F, 16, 2, true>), ROWS_GU); else hipLaunchKernelGGL((k_moe_gu<F, 16, 1, true>), ROWS_GU)); }
+#undef ROWS_GU
+  } PYRE_CHECK_LAUNCH(ctx);
+  { ProfScope ps(ctx, "moe_rows_down", T * (m.top_k * qmat_gguf_bytes(m.down_e, m.d) + qmat_gguf_bytes(m.sh_down, m.d)));
+#define ROWS_DN dim3(m.d / 64, entries), dim3(8 * 64), 0, ctx->stream, m, w.sel_idx, w.h, hs, w.partial, g2, dgh, w.elist
+    if (idot_dn) hipLaunchKernelGGL((k_moe_down<FMT_IQ3_S, 8, 1, false, true>), ROWS_DN);
+    else { MOE_FMT_DISPATCH(m.down_e.fmt, hipLaunchKernelGGL((k_moe_down<F, 8, 1>), ROWS_DN)); }
+#undef ROWS_DN
+    if (parts) hipLaunchKernelGGL(k_moe_groups_blk, dim3((m.d + 255) / 256, T), dim3(256), 0, ctx->stream, m, b, T); } PYRE_CHECK_LAUNCH(ctx);
+  return PYRE_OK;
 }
 
 // ---- C ABI -------------------------------------------------------------------------------------------------------------

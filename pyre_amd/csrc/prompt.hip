@@ -409,6 +409,21 @@ __global__ __launch_bounds__(256) void k_blk_gdn_out_q(const float* __restrict__
   if (j == 0) inv[(size_t)(ti >> 3) * inv_gs + h * 8 + (ti & 7)] = mr * __builtin_amdgcn_rsqf((((q0 + q1) + q2) + q3) * (1.0f / 128.0f) + eps);
 }
 
+// ... and as f32 rows in k_gdn_delta's order: the sum of squares of each half of the head as a tree of neighbours, then the two halves
+__global__ __launch_bounds__(256) void k_blk_gdn_out_w(const float* __restrict__ o, const float* __restrict__ z, int zs, const float* __restrict__ nw, float eps, int heads, int T, float* __restrict__ out) {
+  const size_t gi = (size_t)blockIdx.x * 256 + threadIdx.x; const int j = (int)(gi & 15), h = (int)((gi >> 4) % heads); const int ti = (int)((gi >> 4) / heads);
+  if (ti >= T) return;
+  const float* po = o + ((size_t)ti * heads + h) * 128 + 8 * j; const float* pz = z + (size_t)ti * zs + h * 128 + 8 * j; float* pr = out + ((size_t)ti * heads + h) * 128 + 8 * j;
+  float v[8];
+#pragma unroll
+  for (int k = 0; k < 8; k += 4) { const float4 a = *(const float4*)(po + k); v[k] = a.x; v[k + 1] = a.y; v[k + 2] = a.z; v[k + 3] = a.w; }
+  float ss = ((v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3])) + ((v[4] * v[4] + v[5] * v[5]) + (v[6] * v[6] + v[7] * v[7]));
+  ss += wave_dpp<0xB1, 0xf>(0.0f, ss); ss += wave_dpp<0x4E, 0xf>(0.0f, ss); ss += wave_dpp<0x141, 0xf>(0.0f, ss); ss += wave_dpp<0x140, 0xf>(0.0f, ss);
+  const float sc = 1.0f / sqrtf(ss / 128.0f + eps);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) pr[k] = (v[k] * (sc * nw[8 * j + k])) * b_sigm(pz[k]);
+}
+
 }  // namespace
 
 // parts: K slices left apart for the mix that follows (PYRE_GEMV_PARTS, as pyre_gemv_parts_launch cuts them), or 1
@@ -446,6 +461,11 @@ int pyre_blk_gdn_out_q_launch(pyre_ctx* ctx, const float* o, const float* z, int
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
 
+int pyre_blk_gdn_out_w_launch(pyre_ctx* ctx, const float* o, const float* z, int zs, const float* nw, float eps, int heads, int T, float* out) {
+  ProfScope ps(ctx, "blk_gdn_out", 4.0 * T * heads * 128 * 3);
+  hipLaunchKernelGGL(k_blk_gdn_out_w, dim3((unsigned)(((size_t)T * heads * 16 + 255) / 256)), dim3(256), 0, ctx->stream, o, z, zs, nw, eps, heads, T, out);
+  PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
+}
 static int blk_mix_cs(const HcDev& h) { return h.d % 512 == 0 ? 2 : 1; }
 static int blk_mix_slices(const HcDev& h) { return h.hc * h.d / (256 * blk_mix_cs(h)); }
 bool pyre_blk_mix_ok(const HcDev& h) { return pyre_hc_aop_ok(h) && (h.lr == 256 || h.lr == 512) && blk_mix_slices(h) <= 16 && h.d / 256 <= 64; }

@@ -229,6 +229,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemv(QMatDev m, const float* __rest
 #pragma unroll
     for (int k = 0; k < 8; ++k) { cw[k] = k < ep.kk ? ep.conv_w[row * ep.kk + k] : 0.0f; chist[k] = k < ep.kk - 1 ? ep.conv_in[(size_t)k * ep.ch + row] : 0.0f; }
   }
+  if (blockIdx.z) { x += (size_t)blockIdx.z * T * m.cols; y += (size_t)blockIdx.z * T * m.rows; }          // (a further group of T tokens: pyre_gemv_rows_launch)
   const int k0 = (ks * NW + wave) * upw; const int k1 = min(m.U, k0 + upw);
   float acc[T];
 #pragma unroll
@@ -322,7 +323,7 @@ template <int FMT, int T, int NW> int gemv_launch_nw(pyre_ctx* ctx, const QMatDe
   static const char* fn[FMT_COUNT] = {"f32", "f16", "bf16", "q8_0", "q4_k", "iq2_xs", "iq3_s", "c4", "c8", "iq3_s", "q4_k", "iq2_xs", "q8_0"};
   static const std::string name = std::string("gemv_") + fn[FMT] + "_t" + std::to_string(T);
   ProfScope ps(ctx, name.c_str(), qmat_gguf_bytes(m, m.rows) + 4.0 * T * ((double)m.cols + m.rows));
-  hipLaunchKernelGGL((k_gemv<FMT, T, NW>), dim3(m.tiles, ksplit), dim3(NW * 64), T > 1 ? (size_t)NW * 2 * 64 * T * 4 : 0, ctx->stream, m, x, y, upw, ep, (const uint2*)ctx->d_iq2xs);
+  hipLaunchKernelGGL((k_gemv<FMT, T, NW>), dim3(m.tiles, ksplit, ep.nz > 1 ? ep.nz : 1), dim3(NW * 64), T > 1 ? (size_t)NW * 2 * 64 * T * 4 : 0, ctx->stream, m, x, y, upw, ep, (const uint2*)ctx->d_iq2xs);
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
 // Waves per workgroup: enough that a row tile's whole K range is covered by one workgroup with few units per wave,
@@ -367,6 +368,12 @@ int pyre_gemv_launch(pyre_ctx* ctx, const QMatDev& m, const float* x, int t, flo
   if (m.fmt == FMT_IQ3_S_M) return gemm_m_from_f32(ctx, m, x, t, y, 1, GemvEpi{}, a);
   int rc = PYRE_OK;
   FMT_DISPATCH(m.fmt, rc = gemv_f<F>(ctx, m, x, t, y, 1, GemvEpi{}));
+  return rc;
+}
+int pyre_gemv_rows_launch(pyre_ctx* ctx, const QMatDev& m, const float* x, int groups, float* y) {
+  if (m.fmt == FMT_IQ3_S_M || groups < 1 || groups > 65535) return pyre_fail(ctx, PYRE_E_ARG, "gemv: %d groups of rows", groups);
+  GemvEpi ep{}; ep.nz = groups; int rc = PYRE_OK;
+  FMT_DISPATCH(m.fmt, rc = (gemv_t<F, 8>(ctx, m, x, y, 1, ep)));
   return rc;
 }
 int pyre_gemv_split_launch(pyre_ctx* ctx, const QMatDev& m, const float* x, int t, float* partial, int ksplit, const PyreAop* a) {
