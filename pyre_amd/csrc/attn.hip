@@ -854,7 +854,11 @@ static int attn_blk_tokens(const AttnDev& a, int n, int T) {
   const int most = (int)(((size_t)128 << 20) / per) / 8 * 8;
   return most < 8 ? 8 : (most < T ? most : T);
 }
-size_t pyre_attn_blk_bytes(const AttnDev& a, int n, int T) { return 512 + (size_t)attn_blk_tokens(a, n, T) * a.nh * ((n + PYRE_ATTN_CHUNK - 1) / PYRE_ATTN_CHUNK) * (a.hd + 2) * 4; }
+// (never less for more positions: a call's earlier blocks take more tokens a launch)
+size_t pyre_attn_blk_bytes(const AttnDev& a, int n, int T) {
+  const size_t per = (size_t)a.nh * ((n + PYRE_ATTN_CHUNK - 1) / PYRE_ATTN_CHUNK) * (a.hd + 2) * 4, all = per * (T < 8 ? 8 : T), most = (size_t)128 << 20;
+  return 512 + (all < most ? all : (8 * per > most ? 8 * per : most));
+}
 int pyre_attn_blk_launch(pyre_ctx* ctx, const AttnDev& a, const KvDev& kv, const float* q, const uint16_t* qh, const float* qsc, const float* qkv, int stride, int start, int T, void* scratch, float* out) {
   const int G = a.nkv > 0 ? a.nh / a.nkv : 0, n = start + T, sub = attn_blk_tokens(a, n, T);
   if (a.hd != 256 || (G != 1 && G != 2 && G != 4 && G != 8) || a.nh % a.nkv) return pyre_fail(ctx, PYRE_E_SHAPE, "attention block: head dim %d, group size %d unsupported", a.hd, G);

@@ -339,7 +339,7 @@ struct MoeRows { int32_t* sel_idx; float* sel_w; int32_t* elist; float* sg; int3
 size_t pyre_moe_rows_bytes(const MoeDev& m, int T);
 void   pyre_moe_rows_carve(const MoeDev& m, int T, void* base, MoeRows* w);
 bool   pyre_moe_rows_ok(const MoeDev& m);
-int    pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const float* x, int T, const float* rpart, size_t wr, int nsl, int r64, float* parts);
+int    pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const float* x, int T, const float* rpart, size_t wr, int nsl, int r64, float* parts, float* y);
 inline MoeOut pyre_moe_rows_out(const MoeDev& m, const MoeRows& w, int first_token) { return MoeOut{w.partial + (size_t)first_token * (m.top_k + 1) * m.d, w.sel_w + (size_t)first_token * m.top_k, w.sg + first_token, m.d, m.top_k}; }
 // K parts the gate/up dot products are summed in (1 or 2; k_moe_gu)
 int pyre_moe_gu_parts(const MoeDev& m);

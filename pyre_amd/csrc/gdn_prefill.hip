@@ -334,15 +334,26 @@ __global__ __launch_bounds__(256) void k_gdn_rec4(GdnDev p, const float* __restr
   for (int t0 = 0, buf = 0; t0 < T; t0 += TB, buf ^= 1) {
     if (t0 + TB < T) load(t0 + TB, buf ^ 1);
     const int n = min(TB, T - t0);
-    for (int t = 0; t < n; ++t) {
-      const float2 gt = gb[buf][t]; const float* k = ks[buf][t][g]; const float* q = qs[buf][t][g];
+    struct Row { float4 v[8]; };
+    auto row = [&](const float* x) { Row r;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) r.v[i] = *(const float4*)(x + 4 * i);
+      return r; };
+    Row k = row(ks[buf][0][g]);
+    for (int t = 0; t < n; ++t) {          // (the query is read behind the keys' sums, the next token's keys behind the query's)
+      const float2 gt = gb[buf][t]; const float vt = vs[buf][t][jl];
+      const Row q = row(qs[buf][t][g]);
+      const float* kk = (const float*)&k; const float* qq = (const float*)&q;
       float pm = 0.0f;
 #pragma unroll
-      for (int r = 0; r < R; ++r) { S[r] *= gt.x; pm += S[r] * k[r]; }
-      const float delta = (vs[buf][t][jl] - quad_sum(pm)) * gt.y;
+      for (int r = 0; r < R; ++r) { S[r] *= gt.x; pm += S[r] * kk[r]; }
+      const float delta = (vt - quad_sum(pm)) * gt.y;
+#pragma unroll
+      for (int r = 0; r < R; ++r) S[r] += kk[r] * delta;
+      k = row(ks[buf][min(t + 1, n - 1)][g]);
       float po = 0.0f;
 #pragma unroll
-      for (int r = 0; r < R; ++r) { S[r] += k[r] * delta; po += S[r] * q[r]; }
+      for (int r = 0; r < R; ++r) po += S[r] * qq[r];
       const float o = quad_sum(po);
       if (g == 0) oraw[(size_t)(t0 + t) * w + (size_t)h * p.dv + cb + jl] = o;
     }

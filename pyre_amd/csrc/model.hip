@@ -646,8 +646,8 @@ static int run_rows(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBlk
   PYRE_HIP(ctx, hipMemcpyAsync(B->ids, ids, (size_t)T * 4, hipMemcpyHostToDevice, ctx->stream));
   if (s->tokens_dev) PYRE_HIP(ctx, hipMemcpyAsync(s->tokens_dev + start, B->ids, (size_t)T * 4, hipMemcpyDeviceToDevice, ctx->stream));
   if ((rc = pyre_row_launch(ctx, m->embd, B->ids, T, B->emb, d))) return rc;
-  const float* xin = B->emb; int in_ss = 0, in_ts = d; float* xout = B->x; float* xother = B->x2; const MoeOut* comb = nullptr; const float* cinj = nullptr;
-  const int r64 = m->layers[0].moe.router.tiles * 64; const size_t wr = (size_t)8 * (d / 64) * r64; const MoeOut all = pyre_moe_rows_out(m->layers[0].moe, B->rows, 0);
+  const float* xin = B->emb; int in_ss = 0, in_ts = d; float* xout = B->x; float* xother = B->x2; const float* comb = nullptr; const float* cinj = nullptr;
+  const int r64 = m->layers[0].moe.router.tiles * 64; const size_t wr = (size_t)8 * (d / 64) * r64;
   auto advance = [&]() { xin = xout; in_ss = d; in_ts = hc * d; std::swap(xout, xother); };
   // a matrix over all tokens: the lane = row product in groups of eight, or the matrix cores behind a split
   auto mul = [&](const QMatDev& q, const float* x, float* y) -> int {
@@ -657,7 +657,7 @@ static int run_rows(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBlk
   };
   for (int il = 0; il < c.n_layers; ++il) {
     const Layer& L = m->layers[il]; const int oc = L.outp.cols, pw = (int)L.proj.rows;
-    if ((rc = pyre_hc_mix_rows_launch(ctx, L.hca, B->hw, xin, in_ss, in_ts, xout, G, nullptr, comb, cinj, c.eps, B->mixed, B->inj_a, nullptr))) return rc;
+    if ((rc = pyre_hc_mix_rows_launch(ctx, L.hca, B->hw, xin, in_ss, in_ts, xout, G, comb, nullptr, cinj, c.eps, B->mixed, B->inj_a, nullptr))) return rc;
     advance();
     if ((rc = mul(L.proj, B->mixed, B->proj))) return rc;
     if (L.full) {
@@ -683,8 +683,8 @@ static int run_rows(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBlk
     advance();
     const bool end = il == c.n_layers - 1; const int i0 = end ? (T - 1) / 8 * 8 : 0;
     if (end && !head) break;          // nobody reads the last layer's FFN
-    if ((rc = pyre_moe_rows_launch(ctx, L.moe, B->rows, B->mixed + (size_t)i0 * d, T - i0, B->rpart + (size_t)(i0 / 8) * wr, wr, d / 64, r64, nullptr))) return rc;
-    comb = &all; cinj = B->inj_f;
+    if ((rc = pyre_moe_rows_launch(ctx, L.moe, B->rows, B->mixed + (size_t)i0 * d, T - i0, B->rpart + (size_t)(i0 / 8) * wr, wr, d / 64, r64, nullptr, end ? nullptr : B->o))) return rc;          // (summed once: five row tiles of the next mix would each gather the terms)
+    comb = B->o; cinj = B->inj_f;
   }
   s->len = start + T;
   return head ? prompt_head(ctx, m, B, xin + (size_t)(T - 1) * hc * d, T) : PYRE_OK;
@@ -731,7 +731,7 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
     if (end && !head) break;          // nobody reads the last layer's FFN
     if ((rc = pyre_moe_block_launch(ctx, L.moe, B->moe, end ? 0 : Tb, T, B->T_max, d / 64, r64))) return rc;
     const int i0 = end ? (T - 1) / 8 * 8 : Tb;          // (the last layer: the last group's terms, for the head)
-    if (i0 < T && (rc = pyre_moe_rows_launch(ctx, L.moe, B->rows, B->mixed + (size_t)i0 * d, T - i0, B->moe.rpart + (size_t)(i0 / 8) * B->moe.wr, B->moe.wr, d / 64, r64, end ? nullptr : B->moe.parts + (size_t)(i0 / 8) * PYRE_MOE_GROUPS * 8 * d))) return rc;
+    if (i0 < T && (rc = pyre_moe_rows_launch(ctx, L.moe, B->rows, B->mixed + (size_t)i0 * d, T - i0, B->moe.rpart + (size_t)(i0 / 8) * B->moe.wr, B->moe.wr, d / 64, r64, end ? nullptr : B->moe.parts + (size_t)(i0 / 8) * PYRE_MOE_GROUPS * 8 * d, nullptr))) return rc;
     comb = B->moe.parts; np = PYRE_MOE_GROUPS; cinj = B->inj_f;
   }
   s->len = start + T;

@@ -858,22 +858,154 @@ int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T
   return PYRE_OK;
 }
 
+// k_moe_gu<.., PRE> (both K parts in the workgroup) and k_moe_down with up to four of an expert's tokens through together: a weight is decoded once for
+// them (3.5 of a Q4_K weight's 4.5 vector instructions; 200 tokens, four an expert: 607 us an entry at a time).  grid (row tiles,
+// experts + groups of the shared expert, gate and up), NW waves, raw sums in w.h [gate, up][entry]; a wave stages the four times 64 activations of its unit in its own slice of shared
+// memory.  A token's operations are k_moe_gu's, in its order.
+// one pass of TG entries (elist + i, or i-th of the shared expert's): products of row tile `tile` of Q with x rows by token, raw sums to out [entry]
+template <int FMT, int NW, int TG>
+__device__ __forceinline__ void gu_pass(const QMatDev& Q, int tile, const float* __restrict__ x, int d, const int32_t* __restrict__ list, int first, int step, int k1, int np, float* __restrict__ out, int hstride, float* red, float* xs) {
+  const uint2* lds2 = nullptr;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, QU = Q.U, upw = (QU + NW * np - 1) / (NW * np);
+  float* xw = xs + (size_t)wave * TG * 64;
+  int en[TG];
+#pragma unroll
+  for (int t = 0; t < TG; ++t) en[t] = __builtin_amdgcn_readfirstlane(list ? list[t] : first + t * step);
+#pragma unroll 1
+  for (int p = 0; p < np; ++p) {
+    float acc[TG];
+#pragma unroll
+    for (int t = 0; t < TG; ++t) acc[t] = 0.0f;
+    const int k0 = min(QU, (wave * np + p) * upw), kend = min(QU, k0 + upw);
+    for (int ku = k0; ku < kend; ++ku) {
+      const UnitRaw<FMT> r = unit_load<FMT>(Q, tile, ku, lane);
+      float xv[TG];
+#pragma unroll
+      for (int t = 0; t < TG; ++t) xv[t] = x[(size_t)(en[t] / k1) * d + ku * 64 + lane];
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int t = 0; t < TG; ++t) xw[t * 64 + lane] = xv[t];
+      __builtin_amdgcn_wave_barrier();
+      unit_fma<FMT, TG>(Q, r, ku, lds2, lane, xw, 64, acc);
+      __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int t = 0; t < TG; ++t) red[((p * NW + wave) * TG + t) * 64 + lane] = acc[t];
+  }
+  __syncthreads();
+  for (int i = tid; i < TG * 64; i += NW * 64) {
+    const int t = i >> 6; float sum = 0.0f;
+    for (int p = 0; p < np; ++p) {
+      float part = red[((p * NW) * TG + t) * 64 + lane];
+#pragma unroll
+      for (int q = 1; q < NW; ++q) part += red[((p * NW + q) * TG + t) * 64 + lane];
+      sum = p == 0 ? part : sum + part;
+    }
+    int e = en[0];
+#pragma unroll
+    for (int q = 1; q < TG; ++q) if (q == t) e = en[q];
+    out[(size_t)e * hstride + blockIdx.x * 64 + lane] = sum;
+  }
+  __syncthreads();
+}
+template <int FMT, int NW>
+__global__ __launch_bounds__(NW * 64) void k_moe_gu_rows(MoeDev m, MoeRows w, const float* __restrict__ x, int hstride, int T, int np) {
+  constexpr int TG = 4;
+  __shared__ float red[2 * NW * TG * 64];
+  __shared__ __align__(16) float xs[NW * TG * 64];
+  const int ye = blockIdx.y, k1 = m.top_k + 1; const bool shared = ye >= m.n_exp;
+  if ((int)blockIdx.x * 64 >= (shared ? m.sf : m.ff)) return;
+  const int t0 = (ye - m.n_exp) * TG, e0 = shared ? 0 : w.eoff[ye], n = shared ? min(TG, T - t0) : w.eoff[ye + 1] - e0;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const QMatDev& Q = blockIdx.z ? (shared ? m.sh_up : m.up_e) : (shared ? m.sh_gate : m.gate_e);
+  float* out = w.h + (size_t)blockIdx.z * T * k1 * hstride;
+  const int tile = (shared ? 0 : ye * (m.ff >> 6)) + blockIdx.x;
+  for (int i0 = 0; i0 < n; ) {          // four entries at a time, the rest two and one
+    const int32_t* list = shared ? nullptr : w.elist + e0 + i0; const int first = (t0 + i0) * k1 + m.top_k;
+    if (n - i0 >= 4) { gu_pass<FMT, NW, 4>(Q, tile, x, m.d, list, first, k1, k1, np, out, hstride, red, xs); i0 += 4; }
+    else if (n - i0 >= 2) { gu_pass<FMT, NW, 2>(Q, tile, x, m.d, list, first, k1, k1, np, out, hstride, red, xs); i0 += 2; }
+    else { gu_pass<FMT, NW, 1>(Q, tile, x, m.d, list, first, k1, k1, np, out, hstride, red, xs); i0 += 1; }
+  }
+  if (!shared || blockIdx.x || blockIdx.z) return;
+  for (int t = 0; t < n; ++t) {          // the shared expert's gate of the group's tokens
+    const float* xt = x + (size_t)(t0 + t) * m.d; float p = 0.0f;
+    for (int ib = tid; ib < m.d; ib += NW * 64) p = fmaf(m.sh_gate_inp[ib], xt[ib], p);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) p += __shfl_xor(p, o);
+    if (lane == 0) red[wave] = p;
+    __syncthreads();
+    if (tid == 0) { float tot = 0.0f; for (int q = 0; q < NW; ++q) tot += red[q]; w.sg[t0 + t] = 1.0f / (1.0f + expf(-tot)); }
+    __syncthreads();
+  }
+}
+// ... and k_moe_down likewise, forming silu(gate) * up of the two sums on the way
+template <int FMT, int NW, int TG>
+__device__ __forceinline__ void down_pass(const QMatDev& D, int tile, const MoeRows& w, int d, const int32_t* __restrict__ list, int first, int step, size_t up, int hstride, float* red, float* xs) {
+  const uint2* lds2 = nullptr;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, upw = (D.U + NW - 1) / NW, k0 = wave * upw, kend = min((int)D.U, k0 + upw);
+  float* xw = xs + (size_t)wave * TG * 64;
+  int en[TG]; float acc[TG];
+#pragma unroll
+  for (int t = 0; t < TG; ++t) { en[t] = __builtin_amdgcn_readfirstlane(list ? list[t] : first + t * step); acc[t] = 0.0f; }
+  for (int ku = k0; ku < kend; ++ku) {
+    const UnitRaw<FMT> r = unit_load<FMT>(D, tile, ku, lane);
+    float xv[TG];
+#pragma unroll
+    for (int t = 0; t < TG; ++t) { const float* h = w.h + (size_t)en[t] * hstride + ku * 64 + lane; const float g = h[0], u = h[up], s = 1.0f / (1.0f + expf(-g)); xv[t] = (g * s) * u; }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < TG; ++t) xw[t * 64 + lane] = xv[t];
+    __builtin_amdgcn_wave_barrier();
+    unit_fma<FMT, TG>(D, r, ku, lds2, lane, xw, 64, acc);
+    __builtin_amdgcn_wave_barrier();
+  }
+#pragma unroll
+  for (int t = 0; t < TG; ++t) red[(wave * TG + t) * 64 + lane] = acc[t];
+  __syncthreads();
+  for (int i = tid; i < TG * 64; i += NW * 64) {
+    const int t = i >> 6; float sum = red[t * 64 + lane];
+#pragma unroll
+    for (int q = 1; q < NW; ++q) sum += red[(q * TG + t) * 64 + lane];
+    int e = en[0];
+#pragma unroll
+    for (int q = 1; q < TG; ++q) if (q == t) e = en[q];
+    w.partial[(size_t)e * d + blockIdx.x * 64 + lane] = sum;
+  }
+  __syncthreads();
+}
+template <int FMT, int NW>
+__global__ __launch_bounds__(NW * 64) void k_moe_down_rows(MoeDev m, MoeRows w, int hstride, int T) {
+  constexpr int TG = 4;
+  __shared__ float red[NW * TG * 64];
+  __shared__ __align__(16) float xs[NW * TG * 64];
+  const int ye = blockIdx.y, k1 = m.top_k + 1; const bool shared = ye >= m.n_exp;
+  const int t0 = (ye - m.n_exp) * TG, e0 = shared ? 0 : w.eoff[ye], n = shared ? min(TG, T - t0) : w.eoff[ye + 1] - e0;
+  const QMatDev& D = shared ? m.sh_down : m.down_e;
+  const int tile = (shared ? 0 : ye * (m.d >> 6)) + blockIdx.x; const size_t up = (size_t)T * k1 * hstride;
+  for (int i0 = 0; i0 < n; ) {
+    const int32_t* list = shared ? nullptr : w.elist + e0 + i0; const int first = (t0 + i0) * k1 + m.top_k;
+    if (n - i0 >= 4) { down_pass<FMT, NW, 4>(D, tile, w, m.d, list, first, k1, up, hstride, red, xs); i0 += 4; }
+    else if (n - i0 >= 2) { down_pass<FMT, NW, 2>(D, tile, w, m.d, list, first, k1, up, hstride, red, xs); i0 += 2; }
+    else { down_pass<FMT, NW, 1>(D, tile, w, m.d, list, first, k1, up, hstride, red, xs); i0 += 1; }
+  }
+}
+
 // The windows' arithmetic (k_moe_gu / k_moe_down, the digits form for IQ3_S experts) for any number of tokens in one set of launches,
 // entry by entry in the order of the experts: a prompt of a model whose experts have no matrix-core layout, and the last tokens of
 // one whose experts have.  Router sums as in MoeBlk (rpart + group * wr).  parts: the group sums [group][PYRE_MOE_GROUPS][8][d], or
-// null: the unreduced terms stay in w (pyre_moe_out).
+// null; y: their sum [token][d], or null; the unreduced terms stay in w (pyre_moe_rows_out).
 size_t pyre_moe_rows_bytes(const MoeDev& m, int T) {
   const size_t hs = (size_t)(m.ff > m.sf ? m.ff : m.sf), k1 = m.top_k + 1, n = T;
-  return 256 * 12 + 4 * (3 * n * m.top_k + n + 1024 + n * k1 * (hs + m.d) + n * (m.d / 64) * DGX_STRIDE + n * k1 * (hs / 64) * DGX_STRIDE);
+  return 256 * 12 + 4 * (3 * n * m.top_k + n + 1024 + n * k1 * (2 * hs + m.d) + n * (m.d / 64) * DGX_STRIDE + n * k1 * (hs / 64) * DGX_STRIDE);
 }
 void pyre_moe_rows_carve(const MoeDev& m, int T, void* base, MoeRows* w) {
   uint8_t* p = (uint8_t*)base; auto take = [&](size_t n) { void* r = p; p += (4 * n + 255) & ~(size_t)255; return r; };
   const size_t hs = (size_t)(m.ff > m.sf ? m.ff : m.sf), k1 = m.top_k + 1, n = T;
   w->sel_idx = (int32_t*)take(n * m.top_k); w->sel_w = (float*)take(n * m.top_k); w->elist = (int32_t*)take(n * m.top_k); w->sg = (float*)take(n); w->eoff = (int32_t*)take(1024);
-  w->h = (float*)take(n * k1 * hs); w->partial = (float*)take(n * k1 * m.d); w->dgx = (uint32_t*)take(n * (m.d / 64) * DGX_STRIDE); w->dgh = (uint32_t*)take(n * k1 * (hs / 64) * DGX_STRIDE);
+  w->h = (float*)take(2 * n * k1 * hs); w->partial = (float*)take(n * k1 * m.d); w->dgx = (uint32_t*)take(n * (m.d / 64) * DGX_STRIDE); w->dgh = (uint32_t*)take(n * k1 * (hs / 64) * DGX_STRIDE);
 }
 bool pyre_moe_rows_ok(const MoeDev& m) { return m.top_k <= PYRE_MOE_KMAX && m.n_exp <= 1023 && m.d % 64 == 0; }
-int pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const float* x, int T, const float* rpart, size_t wr, int nsl, int r64, float* parts) {
+int pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const float* x, int T, const float* rpart, size_t wr, int nsl, int r64, float* parts, float* y) {
   if (!pyre_moe_rows_ok(m) || T < 1 || T * (m.top_k + 1) > 65535 || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe rows: unsupported shape (T = %d, %d router slices)", T, nsl);
   MoeBlk b{}; b.rpart = rpart; b.wr = wr; b.parts = parts; b.sel_idx = w.sel_idx; b.sel_w = w.sel_w; b.eoff = w.eoff; b.elist = w.elist; b.partial = w.partial; b.sg = w.sg;
   const int hs = m.ff > m.sf ? m.ff : m.sf, entries = T * (m.top_k + 1), P = pyre_moe_gu_parts(m);
@@ -889,15 +1021,17 @@ int pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const
     const bool fix = m.gate_e.fmt == FMT_IQ3_S && m.down_e.fmt == FMT_IQ3_S && m.n_exp == 512 && m.top_k == 10 && m.d == 2048 && m.ff == 512 && m.sf == 512 && nsl == 32;
     if (idot && fix && P == 2) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, true, true>), ROWS_GU);
     else if (idot) { if (P == 2) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, false, true>), ROWS_GU); else hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 1, true, false, true>), ROWS_GU); }
-    else { MOE_FMT_DISPATCH(m.gate_e.fmt, if (P == 2) hipLaunchKernelGGL((k_moe_gu<F, 16, 2, true>), ROWS_GU); else hipLaunchKernelGGL((k_moe_gu<F, 16, 1, true>), ROWS_GU)); }
+    else { MOE_FMT_DISPATCH(m.gate_e.fmt, hipLaunchKernelGGL((k_moe_gu_rows<F, 16>), dim3(hs / 64, m.n_exp + (T + 3) / 4, 2), dim3(16 * 64), 0, ctx->stream, m, w, x, hs, T, P)); }
 #undef ROWS_GU
   } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "moe_rows_down", T * (m.top_k * qmat_gguf_bytes(m.down_e, m.d) + qmat_gguf_bytes(m.sh_down, m.d)));
 #define ROWS_DN dim3(m.d / 64, entries), dim3(8 * 64), 0, ctx->stream, m, w.sel_idx, w.h, hs, w.partial, g2, dgh, w.elist
     if (idot_dn) hipLaunchKernelGGL((k_moe_down<FMT_IQ3_S, 8, 1, false, true>), ROWS_DN);
-    else { MOE_FMT_DISPATCH(m.down_e.fmt, hipLaunchKernelGGL((k_moe_down<F, 8, 1>), ROWS_DN)); }
+    else if (idot) { MOE_FMT_DISPATCH(m.down_e.fmt, hipLaunchKernelGGL((k_moe_down<F, 8, 1>), ROWS_DN)); }          // (behind the digits form h is finished)
+    else { MOE_FMT_DISPATCH(m.down_e.fmt, hipLaunchKernelGGL((k_moe_down_rows<F, 8>), dim3(m.d / 64, m.n_exp + (T + 3) / 4), dim3(8 * 64), 0, ctx->stream, m, w, hs, T)); }
 #undef ROWS_DN
-    if (parts) hipLaunchKernelGGL(k_moe_groups_blk, dim3((m.d + 255) / 256, T), dim3(256), 0, ctx->stream, m, b, T); } PYRE_CHECK_LAUNCH(ctx);
+    if (parts) hipLaunchKernelGGL(k_moe_groups_blk, dim3((m.d + 255) / 256, T), dim3(256), 0, ctx->stream, m, b, T);
+    if (y) hipLaunchKernelGGL(k_moe_sum, dim3((m.d + 255) / 256, T), dim3(256), 0, ctx->stream, w.partial, w.sel_w, w.sg, m.d, m.top_k, y); } PYRE_CHECK_LAUNCH(ctx);
   return PYRE_OK;
 }
 
