@@ -536,7 +536,7 @@ static bool prompt_block_ok(const pyre_model* m) {
   if (m->n_ple > 0 || c.top_k > PYRE_MOE_KMAX || c.d % 256 || c.conv_k < 2 || c.conv_k > 8 || !pyre_blk_mix_ok(m->head)) return false;
   for (int il = 0; il < c.n_layers; ++il) { const Layer& L = m->layers[il]; const MoeDev& m0 = m->layers[0].moe;
     if (!pyre_moe_block_ok(L.moe) || (L.moe.router.fmt != FMT_BF16 && L.moe.router.fmt != FMT_F32) || L.moe.router.U != c.d / 64 || L.moe.router.tiles != m0.router.tiles || L.moe.ff != m0.ff || L.moe.sf != m0.sf || L.moe.top_k != m0.top_k || L.moe.n_exp != m0.n_exp ||
-        !pyre_blk_mix_ok(L.hca) || !pyre_blk_mix_ok(L.hcf) || L.proj.fmt != FMT_IQ3_S_M || L.outp.fmt != FMT_IQ3_S_M || L.proj.cols % 256 || L.outp.cols % 256 || L.outp.rows != c.d || !outp_in_parts(L, c.d) || (!L.full && !gdn_q_on(m, L))) return false; }
+        !pyre_blk_mix_ok(L.hca) || !pyre_blk_mix_ok(L.hcf) || L.proj.fmt != FMT_IQ3_S_M || L.outp.fmt != FMT_IQ3_S_M || L.proj.cols % 256 || L.outp.cols % 256 || L.outp.rows != c.d || (!L.full && !gdn_q_on(m, L))) return false; }
   return true;
 }
 struct PromptBlk {
@@ -700,7 +700,7 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
   auto gs = [](int cols) { return (size_t)cols * 2; }; auto is = [](int cols) { return cols / 256 * 8; };
   const int r64 = m->layers[0].moe.router.tiles * 64;
   for (int il = 0; il < c.n_layers; ++il) {
-    const Layer& L = m->layers[il]; const int pw = L.full ? m->pw_attn : m->pw_lin, oc = L.outp.cols;
+    const Layer& L = m->layers[il]; const int pw = L.full ? m->pw_attn : m->pw_lin, oc = L.outp.cols, o_parts = outp_in_parts(L, d) ? PYRE_GEMV_PARTS : 1;
     if ((rc = pyre_blk_mix_launch(ctx, L.hca, B->mix, xin, in_ss, in_ts, B->x, T, comb, np, cinj, c.eps, B->mixed, B->inj_a, B->op, gs(d), B->inv, is(d)))) return rc;
     xin = B->x; in_ss = d; in_ts = hc * d;
     if ((rc = pyre_blk_gemm_launch(ctx, L.proj, B->op, gs(d), B->inv, is(d), PYRE_INV_TOKEN, B->proj, pw, T, 1))) return rc;
@@ -718,15 +718,15 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
         if ((rc = pyre_attn_blk_launch(ctx, L.attn, s->kv[ai], B->q, B->qh, B->qsc, B->proj, pw, start, T, B->att, B->core))) return rc;
       }
       if ((rc = pyre_blk_op_split_launch(ctx, B->core, oc, T, B->op, gs(oc), B->inv, is(oc)))) return rc;
-      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, is(oc), PYRE_INV_BLOCK, B->o, d, T, PYRE_GEMV_PARTS))) return rc;
+      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, is(oc), PYRE_INV_BLOCK, B->o, d, T, o_parts))) return rc;
     } else {
       const int li = L.mix_index, b = s->cur[li], nb = b ^ 1;
       if ((rc = pyre_gdn_rec_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], B->core))) return rc;
       s->cur[li] = nb;
       if ((rc = pyre_blk_gdn_out_q_launch(ctx, B->core, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, B->op, gs(oc), B->inv, oc / 16))) return rc;
-      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, oc / 16, PYRE_INV_CHUNK, B->o, d, T, PYRE_GEMV_PARTS))) return rc;
+      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, oc / 16, PYRE_INV_CHUNK, B->o, d, T, o_parts))) return rc;
     }
-    if ((rc = pyre_blk_mix_launch(ctx, L.hcf, B->mix, xin, in_ss, in_ts, B->x, T, B->o, PYRE_GEMV_PARTS, B->inj_a, c.eps, B->mixed, B->inj_f, nullptr, 0, nullptr, 0))) return rc;
+    if ((rc = pyre_blk_mix_launch(ctx, L.hcf, B->mix, xin, in_ss, in_ts, B->x, T, B->o, o_parts, B->inj_a, c.eps, B->mixed, B->inj_f, nullptr, 0, nullptr, 0))) return rc;
     const bool end = il == c.n_layers - 1;
     if (end && !head) break;          // nobody reads the last layer's FFN
     if ((rc = pyre_moe_block_launch(ctx, L.moe, B->moe, end ? 0 : Tb, T, B->T_max, d / 64, r64))) return rc;
