@@ -235,6 +235,8 @@ int pyre_gemm_m_launch(pyre_ctx* ctx, const QMatDev& m, const PyreAop& a, int t,
 bool pyre_gemm_m_x_ok(const QMatDev& m, int t, const GemvEpi& ep);
 // K parts / waves per workgroup the kernel uses for this matrix (ksplit parts)
 void pyre_gemm_m_plan(const QMatDev& m, int ksplit, int* nw, int* hb_per_wave);
+// waves per workgroup of the operator's windows (m16: IQ3_S; 0 = as planned)
+int pyre_gemm_op_nw(const QMatDev& m, bool m16);
 // the operator's own scratch for the split operand (grow-only, per context), and the fixed per-GPU array of the entry point
 // that allocates nothing (resolved at context creation)
 int pyre_gemm_m_scratch(pyre_ctx* ctx, int cols, uint4** op, float** ainv);
@@ -259,7 +261,7 @@ struct MoeDev {
   QMatDev gate_m{}, up_m{}, down_m{}, sh_gate_m{}, sh_up_m{}, sh_down_m{};      // the expert matrices once more in the matrix-core layout (FMT_IQ3_S_M), when the model keeps it: a long prompt's blocks (pyre_moe_block_launch)
 };
 struct MoeWork {            // scratch for up to 8 tokens, owned by whoever launches the block
-  float* logits;            // [8][n_exp]
+  float* logits;            // [8][n_exp], or the shares of them (pyre_moe_launch without routed)
   int32_t* sel_idx;         // [8][top_k] ascending expert id
   float* sel_w;             // [8][top_k]
   float* sg;                // [8] sigmoid(sh_gate_inp . x)

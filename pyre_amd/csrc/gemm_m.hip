@@ -26,42 +26,40 @@ PYRE_TS_DECL(gemm_ts) PYRE_TS_EXPORT(gemm_ts, pyre_debug_ts_gemm)
 int pyre_aop_rows(int t) { return t <= 1 ? 2 : (t == 2 ? 4 : (t <= 4 ? 8 : 16)); }
 size_t pyre_aop_bytes(int cols, int t) { return (size_t)(cols / 8) * pyre_aop_rows(t) * 16; }
 
-// ---- the activation operand from f32 rows: grid = super-blocks (256 columns), 256 threads, thread = column ---------------------
+// ---- the activation operand from f32 rows: grid (super-blocks of 256 columns, 8), 256 threads, thread = column, a workgroup a token ----
 // Each 256-column stretch of a token is scaled by its own power of two so that its largest magnitude lands in [2^13, 2^14):
 // the f16 halves then keep 22 bits of every value that matters to the sum, whatever the magnitudes of x.
+// (The launch is latency: a load, a maximum, a store.  All eight tokens a workgroup, by six shuffles each: 4.8 us; a token a
+// workgroup and the maximum by lane moves inside the vector unit: 2.6 us.)
 __global__ __launch_bounds__(256) void k_act_split(const float* __restrict__ x, int T, int R, int cols, uint16_t* __restrict__ op, float* __restrict__ ainv) {
-  __shared__ float mx[4][8];
+  __shared__ float mx[4];
   PYRE_TS_VARS PYRE_TS(0);
-  const int sb = blockIdx.x, i = threadIdx.x, k = sb * 256 + i, wave = i >> 6, lane = i & 63;
-  float v[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) v[t] = t < T ? x[(size_t)t * cols + k] : 0.0f;
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    float a = fabsf(v[t]); a = a == a ? a : INFINITY;         // a NaN anywhere makes the stretch non-finite
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) a = fmaxf(a, __shfl_xor(a, o));
-    if (lane == 0) mx[wave][t] = a;
+  const int sb = blockIdx.x, t = blockIdx.y, i = threadIdx.x, k = sb * 256 + i, wave = i >> 6, lane = i & 63;
+  if (t >= T) {          // rows no token of the window owns (the operand has R rows, the factors eight)
+    if (2 * t < R) { uint16_t* o = op + ((size_t)(k >> 3) * R + 2 * t) * 8 + (k & 7); o[0] = 0; o[8] = 0; }
+    if (i == 0) ainv[sb * 8 + t] = 0.0f;
+    return;
   }
+  const float v = x[(size_t)t * cols + k];
+  float a = fabsf(v); a = a == a ? a : INFINITY;         // a NaN anywhere makes the stretch non-finite
+  a = wave_max(a);
+  if (lane == 0) mx[wave] = a;
   __syncthreads();
-  uint16_t* o = op + (size_t)(k >> 3) * R * 8 + (k & 7);
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const float m = fmaxf(fmaxf(mx[0][t], mx[1][t]), fmaxf(mx[2][t], mx[3][t]));
-    int e = 0;                                                // m * 2^e in [2^13, 2^14); zero and non-finite stretches stay as they are
-    if (m > 0.0f && m < INFINITY) { e = 140 - (int)((__float_as_uint(m) >> 23) & 0xFF); e = e > 100 ? 100 : e; }
-    const float up = __uint_as_float((uint32_t)(127 + e) << 23), dn = __uint_as_float((uint32_t)(127 - e) << 23);
-    const float xs = v[t] * up;
-    const _Float16 h1 = (_Float16)xs, h2 = (_Float16)((xs - (float)h1) * 2048.0f);
-    if (2 * t < R) { o[(2 * t) * 8] = __builtin_bit_cast(unsigned short, h1); o[(2 * t + 1) * 8] = __builtin_bit_cast(unsigned short, h2); }
-    if (i == 0) ainv[sb * 8 + t] = t < T ? dn : 0.0f;
-  }
+  const float m = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
+  int e = 0;                                                // m * 2^e in [2^13, 2^14); zero and non-finite stretches stay as they are
+  if (m > 0.0f && m < INFINITY) { e = 140 - (int)((__float_as_uint(m) >> 23) & 0xFF); e = e > 100 ? 100 : e; }
+  const float up = __uint_as_float((uint32_t)(127 + e) << 23), dn = __uint_as_float((uint32_t)(127 - e) << 23);
+  const float xs = v * up;
+  const _Float16 h1 = (_Float16)xs, h2 = (_Float16)((xs - (float)h1) * 2048.0f);
+  uint16_t* o = op + ((size_t)(k >> 3) * R + 2 * t) * 8 + (k & 7);
+  o[0] = __builtin_bit_cast(unsigned short, h1); o[8] = __builtin_bit_cast(unsigned short, h2);
+  if (i == 0) ainv[sb * 8 + t] = dn;
   PYRE_TS(1); PYRE_TS_FLUSH(gemm_ts, 24);
 }
 
 int pyre_act_split_launch(pyre_ctx* ctx, const float* x_dev, int t, int cols, uint4* op, float* ainv) {
   ProfScope ps(ctx, "act_split_f16", 4.0 * t * cols + (double)pyre_aop_bytes(cols, t));
-  hipLaunchKernelGGL(k_act_split, dim3(cols / 256), dim3(256), 0, ctx->stream, x_dev, t, pyre_aop_rows(t), cols, (uint16_t*)op, ainv);
+  hipLaunchKernelGGL(k_act_split, dim3(cols / 256, 8), dim3(256), 0, ctx->stream, x_dev, t, pyre_aop_rows(t), cols, (uint16_t*)op, ainv);
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
 
@@ -235,6 +233,19 @@ void pyre_gemm_m_plan(const QMatDev& m, int ksplit, int* nw, int* cpw) {
   const int per_wg = ((m.cols >> 7) + ksplit - 1) / ksplit; *cpw = (per_wg + *nw - 1) / *nw; if (*cpw < 1) *cpw = 1;
 }
 
+// Waves per workgroup of the operator's windows (the kernels of Q4_K, Q8_0 and IQ2_XS, and with `m16` of IQ3_S, where 0 means the plan
+// above).  A row tile's waves end together, so a workgroup of many waves leaves the last round of the chip emptier, and sixteen of the
+// 64-row accumulators do not fit the registers: four waves, but eight where there are few tiles (under 256) and rows long enough for
+// eight shares.  Q4_K 40525 x 2048, five tokens: 8 waves 20.9 us, 4 waves 17.4; 12000 x 1536: 16 waves 18.2, 4 waves 8.6; 8448 x 6144:
+// 16 waves 51, 8 waves 17.0, 4 waves 18.0.  IQ3_S (fewer registers) gains from four only from 256 tiles on with rows of at most 3072
+// columns (60000 x 1024, eight tokens 15.0 -> 11.9; 16384 x 4096 12.1 -> 12.7).
+int pyre_gemm_op_nw(const QMatDev& m, bool m16) {
+  static const int force = env_i("PYRE_GEMM_M_NW", 0);
+  if (force == 4 || force == 8 || (m16 && force == 16)) return m16 ? (force == 4 ? 4 : 0) : force;
+  if (m16) return m.tiles >= 256 && m.cols <= 3072 ? 4 : 0;
+  return m.tiles < 256 && m.cols > 4096 ? 8 : 4;
+}
+
 int pyre_gemm_m_best_count(const QMatDev& m) { return m.tiles; }
 
 bool pyre_gemm_m_x_ok(const QMatDev& m, int t, const GemvEpi& ep) {
@@ -295,5 +306,6 @@ int pyre_gemm_m_static(pyre_ctx* ctx, const QMatDev& m, const float* x_dev, int 
   if (!ctx->aop_static) return pyre_fail(ctx, PYRE_E_HIP, "pyre_qmatmul_static_dev: the device array was not resolved at context creation");
   uint4* op = (uint4*)ctx->aop_static; float* ainv = (float*)((uint8_t*)ctx->aop_static + STATIC_OP_BYTES);
   int rc = pyre_act_split_launch(ctx, x_dev, t, m.cols, op, ainv); if (rc) return rc;
-  return pyre_gemm_m_launch(ctx, m, PyreAop{op, ainv}, t, y_dev, 1, GemvEpi{});
+  GemvEpi ep{}; ep.four_waves = pyre_gemm_op_nw(m, true) == 4;
+  return pyre_gemm_m_launch(ctx, m, PyreAop{op, ainv}, t, y_dev, 1, ep);
 }

@@ -162,11 +162,10 @@ int pyre_gemm_q2_launch(pyre_ctx* ctx, const QMatDev& m, const float* x_dev, int
   ainv = (float*)((uint8_t*)op + ((pyre_aop_bytes(m.cols, 8) + 255) & ~(size_t)255));
   int rc = pyre_act_split_launch(ctx, x_dev, t, m.cols, op, ainv); if (rc) return rc;
   const int R = pyre_aop_rows(t);
-  int nw, cpw; pyre_gemm_m_plan(m, 1, &nw, &cpw);
+  const int nw = pyre_gemm_op_nw(m, false), cpw = ((m.cols >> 7) + nw - 1) / nw;
   static const std::string names[9] = {"", "gemm_iq2xs_t1", "gemm_iq2xs_t2", "gemm_iq2xs_t3", "gemm_iq2xs_t4", "gemm_iq2xs_t5", "gemm_iq2xs_t6", "gemm_iq2xs_t7", "gemm_iq2xs_t8"};
   ProfScope ps(ctx, names[t].c_str(), qmat_gguf_bytes(m, m.rows) + 4.0 * t * ((double)m.cols + m.rows));
   if (nw == 4) hipLaunchKernelGGL((k_gemm_q2<4>), dim3(m.tiles), dim3(256), 0, ctx->stream, m, op, ainv, y_dev, t, R, cpw);
-  else if (nw == 8) hipLaunchKernelGGL((k_gemm_q2<8>), dim3(m.tiles), dim3(512), 0, ctx->stream, m, op, ainv, y_dev, t, R, cpw);
-  else hipLaunchKernelGGL((k_gemm_q2<16>), dim3(m.tiles), dim3(1024), 0, ctx->stream, m, op, ainv, y_dev, t, R, cpw);
+  else hipLaunchKernelGGL((k_gemm_q2<8>), dim3(m.tiles), dim3(512), 0, ctx->stream, m, op, ainv, y_dev, t, R, cpw);
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }

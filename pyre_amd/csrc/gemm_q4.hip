@@ -45,39 +45,36 @@ __global__ __launch_bounds__(256) void k_repack_q4m(int rows, int rows_pad, int 
   mh[mh_slot(rg, sb, SB) + j] = hd;
 }
 
-// ---- the activation operand and the sub-block sums: grid = super-blocks (256 columns), 256 threads, thread = column ------------
+// ---- the activation operand and the sub-block sums: grid (super-blocks of 256 columns, 8), 256 threads, thread = column, a workgroup a token ----
 // The operand rows as k_act_split leaves them (each 256-column stretch of a token on its own power of two); asum[(k / 32) * 8 + t]
 // = the f32 sum of token t's columns 32 (k / 32) .. + 31, added in a fixed tree.
 __global__ __launch_bounds__(256) void k_act_split_q4(const float* __restrict__ x, int T, int R, int cols, uint16_t* __restrict__ op, float* __restrict__ ainv, float* __restrict__ asum) {
-  __shared__ float mx[4][8];
-  const int sb = blockIdx.x, i = threadIdx.x, k = sb * 256 + i, wave = i >> 6, lane = i & 63;
-  float v[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) v[t] = t < T ? x[(size_t)t * cols + k] : 0.0f;
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    float a = fabsf(v[t]); a = a == a ? a : INFINITY;         // a NaN anywhere makes the stretch non-finite
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) a = fmaxf(a, __shfl_xor(a, o));
-    if (lane == 0) mx[wave][t] = a;
-    float s = v[t];
-#pragma unroll
-    for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if ((lane & 31) == 0) asum[(size_t)(k >> 5) * 8 + t] = s;
+  __shared__ float mx[4];
+  const int sb = blockIdx.x, t = blockIdx.y, i = threadIdx.x, k = sb * 256 + i, wave = i >> 6, lane = i & 63;
+  if (t >= T) {
+    if (2 * t < R) { uint16_t* o = op + ((size_t)(k >> 3) * R + 2 * t) * 8 + (k & 7); o[0] = 0; o[8] = 0; }
+    if (i == 0) ainv[sb * 8 + t] = 0.0f;
+    if ((lane & 31) == 0) asum[(size_t)(k >> 5) * 8 + t] = 0.0f;
+    return;
   }
+  const float v = x[(size_t)t * cols + k];
+  float a = fabsf(v); a = a == a ? a : INFINITY;         // a NaN anywhere makes the stretch non-finite
+  a = wave_max(a);
+  if (lane == 0) mx[wave] = a;
+  float s = v;
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  if ((lane & 31) == 0) asum[(size_t)(k >> 5) * 8 + t] = s;
   __syncthreads();
-  uint16_t* o = op + (size_t)(k >> 3) * R * 8 + (k & 7);
-#pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    const float m = fmaxf(fmaxf(mx[0][t], mx[1][t]), fmaxf(mx[2][t], mx[3][t]));
-    int e = 0;                                                // m * 2^e in [2^13, 2^14); zero and non-finite stretches stay as they are
-    if (m > 0.0f && m < INFINITY) { e = 140 - (int)((__float_as_uint(m) >> 23) & 0xFF); e = e > 100 ? 100 : e; }
-    const float up = __uint_as_float((uint32_t)(127 + e) << 23), dn = __uint_as_float((uint32_t)(127 - e) << 23);
-    const float xs = v[t] * up;
-    const _Float16 h1 = (_Float16)xs, h2 = (_Float16)((xs - (float)h1) * 2048.0f);
-    if (2 * t < R) { o[(2 * t) * 8] = __builtin_bit_cast(unsigned short, h1); o[(2 * t + 1) * 8] = __builtin_bit_cast(unsigned short, h2); }
-    if (i == 0) ainv[sb * 8 + t] = t < T ? dn : 0.0f;
-  }
+  const float m = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
+  int e = 0;                                                // m * 2^e in [2^13, 2^14); zero and non-finite stretches stay as they are
+  if (m > 0.0f && m < INFINITY) { e = 140 - (int)((__float_as_uint(m) >> 23) & 0xFF); e = e > 100 ? 100 : e; }
+  const float up = __uint_as_float((uint32_t)(127 + e) << 23), dn = __uint_as_float((uint32_t)(127 - e) << 23);
+  const float xs = v * up;
+  const _Float16 h1 = (_Float16)xs, h2 = (_Float16)((xs - (float)h1) * 2048.0f);
+  uint16_t* o = op + ((size_t)(k >> 3) * R + 2 * t) * 8 + (k & 7);
+  o[0] = __builtin_bit_cast(unsigned short, h1); o[8] = __builtin_bit_cast(unsigned short, h2);
+  if (i == 0) ainv[sb * 8 + t] = dn;
 }
 
 // ---- the product -----------------------------------------------------------------------------------------------------------------
@@ -190,12 +187,11 @@ int pyre_gemm_q4_launch(pyre_ctx* ctx, const QMatDev& m, const float* x_dev, int
   ainv = (float*)((uint8_t*)op + ob); float* asum = ainv + (size_t)(m.cols / 256) * 8 + 64;
   const int R = pyre_aop_rows(t);
   { ProfScope ps(ctx, "act_split_f16", 4.0 * t * m.cols + (double)pyre_aop_bytes(m.cols, t));
-    hipLaunchKernelGGL(k_act_split_q4, dim3(m.cols / 256), dim3(256), 0, ctx->stream, x_dev, t, R, m.cols, (uint16_t*)op, ainv, asum); } PYRE_CHECK_LAUNCH(ctx);
-  int nw, cpw; pyre_gemm_m_plan(m, 1, &nw, &cpw);
+    hipLaunchKernelGGL(k_act_split_q4, dim3(m.cols / 256, 8), dim3(256), 0, ctx->stream, x_dev, t, R, m.cols, (uint16_t*)op, ainv, asum); } PYRE_CHECK_LAUNCH(ctx);
+  const int nw = pyre_gemm_op_nw(m, false), cpw = ((m.cols >> 7) + nw - 1) / nw;
   static const std::string names[9] = {"", "gemm_q4k_t1", "gemm_q4k_t2", "gemm_q4k_t3", "gemm_q4k_t4", "gemm_q4k_t5", "gemm_q4k_t6", "gemm_q4k_t7", "gemm_q4k_t8"};
   ProfScope ps(ctx, names[t].c_str(), qmat_gguf_bytes(m, m.rows) + 4.0 * t * ((double)m.cols + m.rows));
   if (nw == 4) hipLaunchKernelGGL((k_gemm_q4<4>), dim3(m.tiles), dim3(256), 0, ctx->stream, m, op, ainv, asum, y_dev, t, R, cpw);
-  else if (nw == 8) hipLaunchKernelGGL((k_gemm_q4<8>), dim3(m.tiles), dim3(512), 0, ctx->stream, m, op, ainv, asum, y_dev, t, R, cpw);
-  else hipLaunchKernelGGL((k_gemm_q4<16>), dim3(m.tiles), dim3(1024), 0, ctx->stream, m, op, ainv, asum, y_dev, t, R, cpw);
+  else hipLaunchKernelGGL((k_gemm_q4<8>), dim3(m.tiles), dim3(512), 0, ctx->stream, m, op, ainv, asum, y_dev, t, R, cpw);
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }

@@ -620,7 +620,7 @@ static int qmatmul_launch(pyre_ctx* ctx, const pyre_qmat* m, const float* x_dev,
   // a window of a large IQ2_XS matrix likewise (PYRE_QMATMUL_Q2M=0: the lane = row GEMV)
   if (t >= 2 && env_int("PYRE_QMATMUL_Q2M", 1) && m->dvm.fmt == FMT_IQ2_XS_M && m->dvm.mq && !f32_path && !f32_only && !(m->dv.tiles <= 128 && env_int("PYRE_QMATMUL_SMALL", 1))) return pyre_gemm_q2_launch(ctx, m->dvm, x_dev, t, y_dev);
   const bool has_m = m->dvm.fmt == FMT_IQ3_S_M && m->dvm.mq, has_rows = m->base != nullptr;
-  if (has_m && (!has_rows || (!f32_path && !f32_only))) return pyre_gemv_launch(ctx, m->dvm, x_dev, t, y_dev);
+  if (has_m && (!has_rows || (!f32_path && !f32_only))) { GemvEpi ep{}; ep.four_waves = pyre_gemm_op_nw(m->dvm, true) == 4; return gemm_m_from_f32(ctx, m->dvm, x_dev, t, y_dev, 1, ep, nullptr); }
   return pyre_gemv_launch(ctx, m->dv, x_dev, t, y_dev);
 }
 static int qmatmul_dev(pyre_ctx* ctx, const pyre_qmat* m, const float* x_dev, int t, float* y_dev, bool f32_path) {
