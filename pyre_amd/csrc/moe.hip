@@ -254,12 +254,13 @@ __global__ __launch_bounds__(NW * 64, (PRE && P == 2 && FMT >= 5 && FMT <= 7) ? 
 }
 
 // ---- routing alone (windows of several tokens): grid t, 1024 threads; ids ascending and softmax weights of token ti ------
-template <bool FIX = false>
+// NSL > 0: 512 experts, top 10 and NSL router slices folded in at compile time (checked by the launcher)
+template <int NSL = 0>
 __global__ __launch_bounds__(1024) void k_moe_route(MoeDev m, const float* __restrict__ logits, int32_t* __restrict__ sel_idx, float* __restrict__ sel_w, int nsl, int sstride, int tstride) {
   __shared__ RouteLds rl;
   const int ti = blockIdx.x;
-  const int n_exp = FIX ? 512 : m.n_exp, top_k = FIX ? 10 : m.top_k;          // FIX: the A3B configuration (and 32 router slices), checked by the launcher
-  if constexpr (FIX) nsl = 32;
+  const int n_exp = NSL ? 512 : m.n_exp, top_k = NSL ? 10 : m.top_k;
+  if constexpr (NSL > 0) nsl = NSL;
 #ifdef PYRE_PHASE_TS
   unsigned long long ts_[8];
 #endif
@@ -446,15 +447,35 @@ __global__ __launch_bounds__(64) void k_act_digits_eo(const float* __restrict__ 
   digits_eo_wave(x[(size_t)ti * d + ku * 64 + lane], lane, sm, dgx + ((size_t)ti * (d >> 6) + ku) * DGX_STRIDE);
 }
 
+// The router's product by the shares of its GEMV's waves, and (further workgroups, one wave each) the digits of the activations: grid
+// tiles * nw + (d / 64) * t, one wave.  Share w of row tile b: units [w * upw, + upw) of every token, part[(w * t + ti) * tiles * 64 + row].
+// A share is what wave w of k_gemv forms; added in wave order they are its sum, bit for bit.
+template <int RF>
+__global__ __launch_bounds__(64) void k_moe_router_shares(QMatDev q, const float* __restrict__ x, int t, int d, int nw, int upw, float* __restrict__ part, uint32_t* __restrict__ dgx) {
+  __shared__ uint8_t sm[3][64];
+  const uint2* lds2 = nullptr;
+  const int lane = threadIdx.x, ns = q.tiles * nw, b = blockIdx.x;
+  if (b >= ns) { const int ku = (b - ns) % (d >> 6), ti = (b - ns) / (d >> 6); digits_eo_wave(x[(size_t)ti * d + ku * 64 + lane], lane, sm, dgx + ((size_t)ti * (d >> 6) + ku) * DGX_STRIDE); return; }
+  const int tile = b / nw, w = b - tile * nw, k0 = w * upw, k1 = min((int)q.U, k0 + upw);
+  const size_t r64 = (size_t)q.tiles * 64;
+  for (int ti = 0; ti < t; ++ti) {
+    float acc[1] = {0.0f};
+    for (int ku = k0; ku < k1; ++ku) { const UnitRaw<RF> r = unit_load<RF>(q, tile, ku, lane); unit_fma<RF, 1>(q, r, ku, lds2, lane, x + (size_t)ti * d + ku * 64, 0, acc); }
+    part[((size_t)w * t + ti) * r64 + (size_t)tile * 64 + lane] = acc[0];
+  }
+}
+
 #define PYRE_MOE_GU_NZMAX 2
+static bool router_shares_ok(const MoeDev& m) { int nw, upw; pyre_gemv_plan(m.router, &nw, &upw); return (m.router.fmt == FMT_BF16 || m.router.fmt == FMT_F32) && nw <= 16; }
+static size_t router_floats(const MoeDev& m) { int nw, upw; pyre_gemv_plan(m.router, &nw, &upw); const size_t sh = (size_t)nw * m.router.tiles * 64; return 8 * (sh > (size_t)m.n_exp ? sh : (size_t)m.n_exp); }      // logits, or the shares of them
 size_t pyre_moe_work_bytes(const MoeDev& m) {
   size_t hs = (size_t)(m.ff > m.sf ? m.ff : m.sf), k1 = m.top_k + 1;
-  return 256 * 11 + sizeof(float) * (8 * (size_t)m.n_exp + 8 * (size_t)m.top_k * 2 + 8 + 8 * k1 * hs * 2 * PYRE_MOE_GU_NZMAX + 8 * k1 * (size_t)m.d + 8 * PYRE_MOE_GROUPS * (size_t)m.d + 8 * (size_t)(m.d / 64) * DGX_STRIDE + 8 * k1 * (hs / 64) * DGX_STRIDE);
+  return 256 * 11 + sizeof(float) * (router_floats(m) + 8 * (size_t)m.top_k * 2 + 8 + 8 * k1 * hs * 2 * PYRE_MOE_GU_NZMAX + 8 * k1 * (size_t)m.d + 8 * PYRE_MOE_GROUPS * (size_t)m.d + 8 * (size_t)(m.d / 64) * DGX_STRIDE + 8 * k1 * (hs / 64) * DGX_STRIDE);
 }
 void pyre_moe_work_carve(const MoeDev& m, void* base, MoeWork* w) {
   uint8_t* p = (uint8_t*)base; auto take = [&](size_t n) { void* r = p; p += (n + 255) & ~(size_t)255; return r; };
   size_t hs = (size_t)(m.ff > m.sf ? m.ff : m.sf), k1 = m.top_k + 1;
-  w->logits = (float*)take(4 * 8 * (size_t)m.n_exp); w->sel_idx = (int32_t*)take(4 * 8 * (size_t)m.top_k); w->sel_w = (float*)take(4 * 8 * (size_t)m.top_k);
+  w->logits = (float*)take(4 * router_floats(m)); w->sel_idx = (int32_t*)take(4 * 8 * (size_t)m.top_k); w->sel_w = (float*)take(4 * 8 * (size_t)m.top_k);
   w->sg = (float*)take(4 * 8); w->h = (float*)take(4 * 8 * k1 * hs * 2 * PYRE_MOE_GU_NZMAX); w->partial = (float*)take(4 * 8 * k1 * (size_t)m.d);
   w->parts = (float*)take(4 * 8 * PYRE_MOE_GROUPS * (size_t)m.d);
   w->dgx = (uint32_t*)take(4 * 8 * (size_t)(m.d / 64) * DGX_STRIDE);
@@ -482,8 +503,6 @@ int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const floa
   if (!y && m.top_k > PYRE_MOE_KMAX) return pyre_fail(ctx, PYRE_E_SHAPE, "moe_ffn: an unreduced output needs top_k <= %d", PYRE_MOE_KMAX);
   if (routed && (routed->nsl < 1 || routed->nsl > 64 || routed->r64 < m.n_exp)) return pyre_fail(ctx, PYRE_E_ARG, "moe_ffn: %d router slices of %d rows", routed->nsl, routed->r64);
   if (t > 1 && getenv("PYRE_DEBUG_SKIP_MOE")) return PYRE_OK;
-  if (!routed) { int rc = pyre_gemv_launch(ctx, m.router, x, t, w.logits); if (rc) return rc; }
-  const float* lg = routed ? routed->p : w.logits; const int nsl = routed ? routed->nsl : 1, sstride = routed ? t * routed->r64 : 0, tstride = routed ? routed->r64 : m.n_exp;
   auto mat_bytes = [](const QMatDev& q, double rows) { return qmat_gguf_bytes(q, rows); };
   const int hs = m.ff > m.sf ? m.ff : m.sf, entries = t * (m.top_k + 1);
   const uint2* g2 = (const uint2*)ctx->d_iq2xs;
@@ -491,13 +510,25 @@ int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const floa
   // IQ3_S experts: gate/up in the integer form, on the digits the mix left beside the activations or on a launch of their own
   const bool idot = moe_idot() && m.gate_e.fmt == FMT_IQ3_S && m.sh_gate.fmt == FMT_IQ3_S;
   const uint32_t* dgx = nullptr;
-  if (idot) {
-    if (routed && routed->dgx) dgx = routed->dgx;
-    else { ProfScope ps(ctx, "moe_digits", 4.0 * t * m.d * 2); hipLaunchKernelGGL(k_act_digits_eo, dim3(m.d / 64, t), dim3(64), 0, ctx->stream, x, m.d, w.dgx); PYRE_CHECK_LAUNCH(ctx); dgx = w.dgx; }
-  }
   // ... and the down products on the digits of h, which a window's gate/up launch leaves and a single token's down launch forms
   const bool idot_dn = idot && !moe_idot_gu_only() && m.down_e.fmt == FMT_IQ3_S && m.sh_down.fmt == FMT_IQ3_S;
   uint32_t* dgh = idot_dn ? w.dgh : nullptr;
+  // the router's sums: given (a mix left them), or the shares of its GEMV's waves, which the selection adds in wave order -- a
+  // workgroup a share and row tile instead of one a row tile (eight of them at 512 experts: 8.5 us) -- with the digits in the same launch
+  const float* lg = w.logits; int nsl = 1, sstride = 0, tstride = m.n_exp;
+  if (routed) { lg = routed->p; nsl = routed->nsl; sstride = t * routed->r64; tstride = routed->r64; }
+  else if (router_shares_ok(m)) {
+    int nw, upw; pyre_gemv_plan(m.router, &nw, &upw); nsl = nw; tstride = m.router.tiles * 64; sstride = t * tstride;
+    const bool dig = idot; const int nd = dig ? (m.d / 64) * t : 0;
+    ProfScope ps(ctx, "moe_router", qmat_gguf_bytes(m.router, m.router.rows) + 4.0 * t * (m.d + (double)nw * tstride));
+    if (m.router.fmt == FMT_BF16) hipLaunchKernelGGL(k_moe_router_shares<FMT_BF16>, dim3(m.router.tiles * nw + nd), dim3(64), 0, ctx->stream, m.router, x, t, m.d, nw, upw, w.logits, w.dgx);
+    else hipLaunchKernelGGL(k_moe_router_shares<FMT_F32>, dim3(m.router.tiles * nw + nd), dim3(64), 0, ctx->stream, m.router, x, t, m.d, nw, upw, w.logits, w.dgx);
+    PYRE_CHECK_LAUNCH(ctx); dgx = dig ? w.dgx : nullptr;
+  } else { int rc = pyre_gemv_launch(ctx, m.router, x, t, w.logits); if (rc) return rc; }
+  if (idot && !dgx) {
+    if (routed && routed->dgx) dgx = routed->dgx;
+    else { ProfScope ps(ctx, "moe_digits", 4.0 * t * m.d * 2); hipLaunchKernelGGL(k_act_digits_eo, dim3(m.d / 64, t), dim3(64), 0, ctx->stream, x, m.d, w.dgx); PYRE_CHECK_LAUNCH(ctx); dgx = w.dgx; }
+  }
   const bool a3b = t == 1 && m.gate_e.fmt == FMT_IQ3_S && m.down_e.fmt == FMT_IQ3_S && m.n_exp == 512 && m.top_k == 10 && m.d == 2048 && m.ff == 512 && m.sf == 512;          // the instances with these constants folded in
   { ProfScope ps(ctx, "moe_route_gate_up", t * (2.0 * m.top_k * mat_bytes(m.gate_e, m.ff) + 2.0 * mat_bytes(m.sh_gate, m.sf)) + 4.0 * t * (m.n_exp + 2.0 * m.d));
 #define GU_ARGS(NZ) dim3(hs / 64, entries, NZ), dim3(16 * 64), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, w.sg, x, w.h, hs, g2, nsl, sstride, tstride, dgx, dgh, (const int32_t*)nullptr
@@ -505,9 +536,11 @@ int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const floa
   if (t == 1 && a3b && nsl == 32 && nz == 2) { if (idot) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 1, false, true, true>), GU_ARGS(2)); else hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 1, false, true>), GU_ARGS(2)); }
   else if (t == 1) { GU_GO(1, nz, false); }          // the selection inside the launch; one workgroup per K part
   else {
-    const bool a3bw = m.gate_e.fmt == FMT_IQ3_S && m.down_e.fmt == FMT_IQ3_S && m.n_exp == 512 && m.top_k == 10 && m.d == 2048 && m.ff == 512 && m.sf == 512 && nsl == 32;          // a window of the A3B configuration: constants folded in
-    if (a3bw) hipLaunchKernelGGL(k_moe_route<true>, dim3(t), dim3(1024), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, nsl, sstride, tstride);
-    else hipLaunchKernelGGL(k_moe_route<false>, dim3(t), dim3(1024), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, nsl, sstride, tstride);
+    const bool a3bw = m.gate_e.fmt == FMT_IQ3_S && m.down_e.fmt == FMT_IQ3_S && m.n_exp == 512 && m.top_k == 10 && m.d == 2048 && m.ff == 512 && m.sf == 512;          // a window of the A3B configuration: constants folded in
+    const bool r10 = m.n_exp == 512 && m.top_k == 10;
+    if (r10 && nsl == 32) hipLaunchKernelGGL(k_moe_route<32>, dim3(t), dim3(1024), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, nsl, sstride, tstride);
+    else if (r10 && nsl == 16) hipLaunchKernelGGL(k_moe_route<16>, dim3(t), dim3(1024), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, nsl, sstride, tstride);
+    else hipLaunchKernelGGL(k_moe_route<0>, dim3(t), dim3(1024), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, nsl, sstride, tstride);
     if (a3bw && P == 2) { if (idot) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, true, true>), GU_ARGS(1)); else hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, true>), GU_ARGS(1)); }
     else if (P == 2) { GU_GO(2, 1, true); } else { GU_GO(1, 1, true); }
   } }
