@@ -105,9 +105,9 @@ __device__ __forceinline__ void load_a_x(const float* __restrict__ x, int c, int
   b.ai0 = kg == 0 ? dn : 0.0f; b.ai1 = 0.0f;
 }
 //   SQ: the operand of a Gated DeltaNet output projection with per-sub-block scales and the head norm (load_a_sq).
-template <int NW, bool SC, bool CONV, int FT = 0, bool XF = false, bool SQ = false>
+template <int NW, bool SC, bool CONV, int FT = 0, bool XF = false, bool SQ = false, int RG = 4>
 __global__ __launch_bounds__(NW * 64) void k_gemm_m(QMatDev m, const uint4* __restrict__ aop, const float* __restrict__ ainv, float* __restrict__ y, int T, int R, int cpw, GemvEpi ep) {
-  __shared__ float red[NW][4][2][64];
+  __shared__ float red[NW][RG][2][64];
   PYRE_TS_VARS PYRE_TS(0);
   qmat_args_now(m); args_now(aop, ainv, y, T, R, cpw, ep.best, ep.conv_w, ep.conv_in, ep.conv_out, ep.co, ep.ch, ep.kk);
   constexpr bool ONE = FT == 1;
@@ -117,16 +117,18 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_m(QMatDev m, const uint4* __re
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int K128 = m.cols >> 7;
   const int c0 = (ks * NW + wave) * cpw, c1 = min(K128, c0 + cpw);
-  v4f tot[4];
+  v4f tot[RG];
 #pragma unroll
-  for (int g = 0; g < 4; ++g) tot[g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int g = 0; g < RG; ++g) tot[g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   const NibK nk = nib_consts();
   static_assert(!XF || (ONE && !CONV), "f32 activations: the single-token instance without the conv epilogue");
   const AopRsrc ar = aop_rsrc(aop, m.cols, R, lane);
   const float* xf = (const float*)aop;
   auto get_a = [&](int c, ABuf& b) { if constexpr (XF) load_a_x(xf, c, lane, b); else if constexpr (SQ) load_a_sq(ar, ainv, ep.sq_heads, ep.sq_eps, R, c, lane, b); else load_a<SC>(ar, ainv, R, c, lane, b); };
-  WBuf<4> w0; ABuf a0;
-  if (c0 < c1) { get_a(c0, a0); load_w<4>(m, tile * 4, c0, lane, K128, w0); }
+  static_assert(RG == 4 || !CONV, "the conv epilogue's rows are a whole tile's");
+  constexpr bool ONE_LOOP = NW == 16 && !CONV;          // (nothing to overlap with the first fetch: one copy of its code)
+  WBuf<RG> w0; ABuf a0;
+  if (!ONE_LOOP && c0 < c1) { get_a(c0, a0); load_w<RG>(m, tile * RG, c0, lane, K128, w0); }
   // conv epilogue: wave 0 fetches its rows' taps and state now, behind the weights, so the loads overlap the products
   float cw[CONV ? 8 : 1], chist[CONV ? 8 : 1]; const bool conv_row = CONV && wave == 0 && tile * 64 + lane < ep.ch;
   if constexpr (CONV) if (conv_row) {
@@ -137,38 +139,38 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_m(QMatDev m, const uint4* __re
   PYRE_TS(1);
   if constexpr (NW == 16) {                   // sixteen waves: one or two chunks a wave and 128 registers a lane: one buffer, no look-ahead
     for (int c = c0; c < c1; ++c) {
-      if (c > c0) { get_a(c, a0); load_w<4>(m, tile * 4, c, lane, K128, w0); }
-      chunk_mac<4>(w0, a0, c, nk, tot);
+      if (ONE_LOOP || c > c0) { get_a(c, a0); load_w<RG>(m, tile * RG, c, lane, K128, w0); }
+      chunk_mac<RG>(w0, a0, c, nk, tot);
     }
   } else {                                    // two buffers taking turns (a copy from one to the other would wait for the loads just issued)
-    WBuf<4> w1; ABuf a1;
+    WBuf<RG> w1; ABuf a1;
     for (int c = c0; c < c1; c += 2) {
-      if (c + 1 < c1) { get_a(c + 1, a1); load_w<4>(m, tile * 4, c + 1, lane, K128, w1); }
+      if (c + 1 < c1) { get_a(c + 1, a1); load_w<RG>(m, tile * RG, c + 1, lane, K128, w1); }
       __builtin_amdgcn_sched_barrier(0);      // (keeps the compiler from sinking the loads down to their first use)
-      chunk_mac<4>(w0, a0, c, nk, tot);
+      chunk_mac<RG>(w0, a0, c, nk, tot);
       __builtin_amdgcn_sched_barrier(0);
-      if (c + 2 < c1) { get_a(c + 2, a0); load_w<4>(m, tile * 4, c + 2, lane, K128, w0); }
+      if (c + 2 < c1) { get_a(c + 2, a0); load_w<RG>(m, tile * RG, c + 2, lane, K128, w0); }
       __builtin_amdgcn_sched_barrier(0);
-      if (c + 1 < c1) chunk_mac<4>(w1, a1, c + 1, nk, tot);
+      if (c + 1 < c1) chunk_mac<RG>(w1, a1, c + 1, nk, tot);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
   PYRE_TS(2);
   // lane (q, j) holds, for row group g, token 2q (rows 0, 1 of its four) and token 2q + 1 (rows 2, 3): halves h1, h2 * 2^11
 #pragma unroll
-  for (int g = 0; g < 4; ++g) { red[wave][g][0][lane] = tot[g][0] + tot[g][1] * (1.0f / 2048.0f); red[wave][g][1][lane] = tot[g][2] + tot[g][3] * (1.0f / 2048.0f); }
+  for (int g = 0; g < RG; ++g) { red[wave][g][0][lane] = tot[g][0] + tot[g][1] * (1.0f / 2048.0f); red[wave][g][1][lane] = tot[g][2] + tot[g][3] * (1.0f / 2048.0f); }
   lds_barrier(); PYRE_TS(3);
   auto rsum = [&](int t, int rl) { const int l = (t >> 1) * 16 + (rl & 15), g = rl >> 4, h = t & 1; float s = red[0][g][h][l];
 #pragma unroll
     for (int w = 1; w < NW; ++w) s += red[w][g][h][l];
     return s; };
   const size_t r64 = (size_t)m.tiles * 64;
-  for (int i = threadIdx.x; i < T * 64; i += NW * 64) {
-    const int t = i >> 6, l = i & 63; const float s = rsum(t, l);
-    const size_t row = (size_t)tile * 64 + l;
+  for (int i = threadIdx.x; i < T * RG * 16; i += NW * 64) {
+    const int t = i / (RG * 16), l = i & (RG * 16 - 1); const float s = rsum(t, l);
+    const size_t row = (size_t)tile * (RG * 16) + l;
     if (ksplit == 1) { if (row < (size_t)m.rows) y[(size_t)t * m.rows + row] = s; }
     else y[((size_t)ks * T + t) * r64 + row] = s;
-    if (T == 1 && ep.best != nullptr) {       // threads 0..63 = wave 0: first maximum of the tile (sampler::argmax order)
+    if (RG == 4 && T == 1 && ep.best != nullptr) {       // threads 0..63 = wave 0: first maximum of the tile (sampler::argmax order)
       float bv = row < (size_t)m.rows ? s : -INFINITY; uint32_t bi = (uint32_t)row;
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) { float ov = __shfl_xor(bv, o); uint32_t oi = __shfl_xor(bi, o); if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; } }
@@ -208,22 +210,29 @@ int gemm_m_nw(const QMatDev& m, int ksplit) {
   return nw;
 }
 template <int NW> void gemm_m_go(pyre_ctx* ctx, const QMatDev& m, const PyreAop& a, int t, float* y, int ksplit, int cpw, const GemvEpi& ep, const float* xf = nullptr) {
-  if (xf) { hipLaunchKernelGGL((k_gemm_m<NW, true, false, 1, true>), dim3(m.tiles, ksplit), dim3(NW * 64), 0, ctx->stream, m, (const uint4*)xf, (const float*)nullptr, y, 1, 2, cpw, ep); return; }
+  // few row tiles (2048 and 4096 rows): a workgroup a row group of sixteen instead of one a tile of four, so that 128 compute units work
+  // instead of 32, each on a quarter of the instructions; the same sums.  2048 x 4096, sixteen waves, one token: 9.3 -> 7.3 us, f32
+  // activations 12.9 -> 9.9; in four parts 5.2 -> 4.7.  From 65 tiles on the chip is covered and the operand would be read four times as often.
+  const bool rg1 = !ep.co && !ep.best && m.tiles <= 64;
+#define GEMM_M_RG(FT, XF, SQ, AOP, SCL, RR, EP) do { if (rg1) hipLaunchKernelGGL((k_gemm_m<NW, true, false, FT, XF, SQ, 1>), dim3(m.tiles * 4, ksplit), dim3(NW * 64), 0, ctx->stream, m, AOP, SCL, y, t, RR, cpw, EP); \
+    else hipLaunchKernelGGL((k_gemm_m<NW, true, false, FT, XF, SQ>), dim3(m.tiles, ksplit), dim3(NW * 64), 0, ctx->stream, m, AOP, SCL, y, t, RR, cpw, EP); } while (0)
+  if (xf) { GEMM_M_RG(1, true, false, (const uint4*)xf, (const float*)nullptr, 2, ep); return; }
 #define GEMM_M_T(CALL) switch (t) { case 1: { constexpr int FT = 1; CALL; } break; case 2: { constexpr int FT = 2; CALL; } break; case 3: { constexpr int FT = 3; CALL; } break; case 4: { constexpr int FT = 4; CALL; } break; \
     case 5: { constexpr int FT = 5; CALL; } break; case 6: { constexpr int FT = 6; CALL; } break; case 7: { constexpr int FT = 7; CALL; } break; default: { constexpr int FT = 8; CALL; } break; }
   if (a.sq) {          // (the launcher has checked: no conv epilogue, chunks = heads)
     GemvEpi e2 = ep; e2.sq_heads = a.sq_heads; e2.sq_eps = a.sq_eps;
-    GEMM_M_T(hipLaunchKernelGGL((k_gemm_m<NW, true, false, FT, false, true>), dim3(m.tiles, ksplit), dim3(NW * 64), 0, ctx->stream, m, a.op, a.sq, y, t, pyre_aop_rows(t), cpw, e2));
+    GEMM_M_T(GEMM_M_RG(FT, false, true, a.op, a.sq, pyre_aop_rows(t), e2));
     return;
   }
 #define GEMM_M_GO(SC, CONV) hipLaunchKernelGGL((k_gemm_m<NW, SC, CONV, 0>), dim3(m.tiles, ksplit), dim3(NW * 64), 0, ctx->stream, m, a.op, a.ainv, y, t, pyre_aop_rows(t), cpw, ep)
   if (a.ainv && (!ep.co || ep.kk == 4)) {          // scaled operand rows (every launch of the model and of the operator): the instance with the window width folded in
     if (ep.co) { GEMM_M_T(hipLaunchKernelGGL((k_gemm_m<NW, true, true, FT>), dim3(m.tiles, ksplit), dim3(NW * 64), 0, ctx->stream, m, a.op, a.ainv, y, t, pyre_aop_rows(t), cpw, ep)); }
-    else { GEMM_M_T(hipLaunchKernelGGL((k_gemm_m<NW, true, false, FT>), dim3(m.tiles, ksplit), dim3(NW * 64), 0, ctx->stream, m, a.op, a.ainv, y, t, pyre_aop_rows(t), cpw, ep)); }
+    else { GEMM_M_T(GEMM_M_RG(FT, false, false, a.op, a.ainv, pyre_aop_rows(t), ep)); }
   }
   else if (ep.co) { if (a.ainv) GEMM_M_GO(true, true); else GEMM_M_GO(false, true); }
   else { if (a.ainv) GEMM_M_GO(true, false); else GEMM_M_GO(false, false); }
 #undef GEMM_M_T
+#undef GEMM_M_RG
 #undef GEMM_M_GO
 }
 }  // namespace
