@@ -316,6 +316,10 @@ void   pyre_moe_work_carve(const MoeDev& m, void* base, MoeWork* w);
 // (pyre_moe_out) for a consumer that evaluates moe_out_value itself.
 // Router logits that arrive as K-slice sums (left by the mix that produced x, see HcRoute): logit[t][e] = the slices
 // p[(s*T + t)*r64 + e], s = 0..nsl-1, added in slice order.
+// the router's product by K shares (share w: units [w * upw, + upw) of every token, part[(w * t + token) * tiles * 64 + row]) and, unless dgx is
+// null, the digits of x; whether a block's expert products take digits
+int pyre_moe_router_shares_launch(pyre_ctx* ctx, const char* name, const QMatDev& router, const float* x, int t, int nw, int upw, float* part, uint32_t* dgx);
+bool pyre_moe_takes_digits(const MoeDev& m);
 struct RouteSrc { const float* p; int nsl; int r64; const uint32_t* dgx = nullptr; };          // dgx: the activations' digits (digits.h), left by the same mix, or null
 // in_groups (t > 1, y == nullptr, pyre_moe_groups_ok): the down projection leaves the PYRE_MOE_GROUPS group sums of every
 // token in w.parts, group q of token ti at parts + (q*t + ti)*d, instead of the unreduced terms.
@@ -386,6 +390,7 @@ struct HcRoute { QMatDev router; float* part; uint32_t* dgx = nullptr; };       
 //     layer (pyre_gdn_launch takes the factor, the model keeps the matching ainv)
 struct AopOut { uint16_t* op; float* ainv; int nsb; };
 bool pyre_hc_aop_ok(const HcDev& h);
+bool pyre_hc_leaves_digits(const HcDev& h);          // with a riding router: whether HcRoute::dgx is filled
 int pyre_hc_mix_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const float* x_in, int in_ss, int in_ts, float* x_out, int t, const float* comb_out, const MoeOut* comb_moe, const float* comb_inj,
                        float eps, float* mixed_dev, float* inj_dev, const HcRoute* route = nullptr, int comb_parts = 1, const AopOut* aop = nullptr);
 bool pyre_hc_route_ok(const HcDev& h, const QMatDev& router);

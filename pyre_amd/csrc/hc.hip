@@ -66,7 +66,8 @@ template <int T> __device__ __forceinline__ void hc_load_slices(float (&pv)[32],
 //      squares of x_new are summed over the slice -> ssq[ks*T + t]; the tile-0 workgroup of the slice also publishes the
 //      updated stream (x_out, never the buffer x_in points into)
 //   2. each wave takes upw units of the slice; partial sums -> part[(ks*T + t)*tiles*64 + row]
-template <int FMT, int T, int NP> __global__ __launch_bounds__(512) void k_hc_norm_down(QMatDev m, const float* __restrict__ x_in, int in_ss, int in_ts, float* __restrict__ x_out,
+// FD, FK > 0: the model width (and eight waves of one unit each) and the routed experts per token as compile-time constants, as k_hc_norm_down_m.
+template <int FMT, int T, int NP, int FD = 0, int FK = 0> __global__ __launch_bounds__(512) void k_hc_norm_down(QMatDev m, const float* __restrict__ x_in, int in_ss, int in_ts, float* __restrict__ x_out,
     const float* __restrict__ comb_out, MoeOut mo_in, const float* __restrict__ comb_inj, const float* __restrict__ norm, int d, int hc, float* __restrict__ ssq,
     float* __restrict__ part, int upw, const uint2* __restrict__ g2) {
   const size_t zt = (size_t)blockIdx.z * T;          // a further group of T tokens (pyre_hc_mix_rows_launch)
@@ -77,8 +78,9 @@ template <int FMT, int T, int NP> __global__ __launch_bounds__(512) void k_hc_no
   const uint2* lds2 = nullptr;          // no format needs a codebook in shared memory any more
   PYRE_TS_VARS PYRE_TS(0);
   qmat_args_now(m); args_now(x_in, in_ss, in_ts, x_out, comb_out, mo.partial, mo.sel_w, mo.sg, mo.d, mo.k, comb_inj, norm, d, hc, ssq, part, upw);
+  if constexpr (FD > 0) { d = FD; upw = 1; }
   extern __shared__ __align__(16) float sm[];
-  const int nthr = blockDim.x, nw = nthr >> 6, tid = threadIdx.x, L = nw * upw * 64;
+  const int nthr = FD > 0 ? 512 : blockDim.x, nw = nthr >> 6, tid = threadIdx.x, L = nw * upw * 64;
   float* xs = sm;                         // [T][L]
   float* red = sm + (size_t)T * L;        // [nw][T][64]
   float* wsum = red + (size_t)nw * T * 64;   // [nw][T]
@@ -94,7 +96,7 @@ template <int FMT, int T, int NP> __global__ __launch_bounds__(512) void k_hc_no
   if (tid < L) {
     nv0 = norm[(size_t)s * d + i0 + tid];
 #pragma unroll
-    for (int t = 0; t < T; ++t) v0[t] = hc_x_new<T, NP>(x_in, in_ss, in_ts, comb_out, mo, w[t], d, t, s, i0 + tid);
+    for (int t = 0; t < T; ++t) v0[t] = hc_x_new<T, NP, FK>(x_in, in_ss, in_ts, comb_out, mo, w[t], d, t, s, i0 + tid);
   }
   UnitRaw<FMT> raw = unit_load<FMT>(m, tile, ks * nw * upw + wave * upw, lane);
   if (tid < L) {
@@ -110,7 +112,7 @@ template <int FMT, int T, int NP> __global__ __launch_bounds__(512) void k_hc_no
     const float nv = norm[(size_t)s * d + i0 + j];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      float v = hc_x_new<T, NP>(x_in, in_ss, in_ts, comb_out, mo, w[t], d, t, s, i0 + j);
+      float v = hc_x_new<T, NP, FK>(x_in, in_ss, in_ts, comb_out, mo, w[t], d, t, s, i0 + j);
       ss[t] += v * v;
       xs[(size_t)t * L + j] = v * nv;
       if (tile == 0) x_out[((size_t)t * hc + s) * d + i0 + j] = v;
@@ -253,6 +255,104 @@ template <int FMT, int T, int RF> __global__ __launch_bounds__(1024) void k_hc_u
     }
   }
   PYRE_TS(7); PYRE_TS_FLUSH(hc_ts, ROUTE ? 16 : 24);
+}
+
+// The same launch for a window alone (at most eight tokens) and the formats of up_by_columns: grid (d / 16), sixteen columns a workgroup, a lane a (stream, unit, column)
+// item of the up GEMV and TS sets of them sharing the tokens (set k: tokens k, k + TS, ..), on d / 16 compute units instead of d / 64; the
+// router is a launch of its own behind it.  The launch is latency, and half of that was fetching instructions: 18 KB of straight code
+// with run-time stream and slice counts, 6 KB with them folded in (FHC, FLR, FKS; the launcher checks them).  A3B shape, bf16, one token:
+// 8.2 us as k_hc_up_mix (13.9 with the router, and 2.5 for the digits behind it), 8.4 here with run-time counts, 6.8 with the folded ones
+// (and 3.2 for router and digits).  A lane's terms, and every order of adding, are those of k_hc_up_mix, bit for bit.  A unit's row of lo
+// is PAD floats behind the last one: the four units of a wave read four different banks.
+#define PYRE_UP_PAD 68
+template <int FMT, int T, int FHC = 0, int FLR = 0, int FKS = 0> __global__ __launch_bounds__(512) void k_hc_up_mix_c(QMatDev up, const float* __restrict__ part, const float* __restrict__ ssq, int ksplit, int r64, int lr, int hc, int has_inject,
+    const float* __restrict__ xnew, const float* __restrict__ norm, float eps, int d, float* __restrict__ mixed, float* __restrict__ inj) {
+  constexpr int TS = T > 1 ? 2 : 1, TT = (T + TS - 1) / TS, KS = FKS > 0 ? FKS : 32, QS = FHC > 0 ? FHC : 8;
+  const uint2* lds2 = nullptr;
+  qmat_args_now(up); args_now(part, ssq, ksplit, r64, lr, hc, has_inject, xnew, norm, eps, d, mixed, inj);
+  if constexpr (FHC > 0) { hc = FHC; lr = FLR; ksplit = FKS; }
+  extern __shared__ __align__(16) float sm[];
+  const int nthr = blockDim.x, tid = threadIdx.x, U = lr >> 6, kps = ksplit / hc, items = hc * U * 16;
+  float* lo = sm;                                          // [T][U][PAD]
+  float* red = lo + (size_t)T * U * PYRE_UP_PAD;           // [hc * U][T][16]
+  float* sls = red + (size_t)hc * U * T * 16;              // [T][32]: the RMS scale of the stream each slice belongs to
+  const int ts = tid / items, it = tid - ts * items, su = it >> 4, r = it & 15, s = su / U, ku = su - s * U, col0 = blockIdx.x * 16;
+  const bool work = ts < TS;
+  float ssv[32];
+  const int stt = tid / hc, sq = tid - stt * hc;
+  const bool own = tid < T * hc;                           // thread (token stt, stream sq): the stream's scale, and in the first workgroup its inject row
+  if constexpr (FKS > 0) {
+#pragma unroll
+    for (int k = 0; k < FKS / FHC; ++k) ssv[k] = own ? (ssq + (size_t)(sq * kps) * T + stt)[k * T] : 0.0f;
+  } else {
+#pragma unroll
+    for (int k = 0; k < 32; ++k) ssv[k] = 0.0f;
+    if (own) hc_load_run(ssv, ssq + (size_t)(sq * kps) * T + stt, kps, T);
+  }
+  auto slices = [&](float (&v)[32], bool want, int tk, int row) {
+    if constexpr (FKS > 0) {
+#pragma unroll
+      for (int ks = 0; ks < FKS; ++ks) v[ks] = want ? (part + (size_t)ks * T * r64)[(unsigned)(tk * r64 + row)] : 0.0f;
+    } else hc_load_slices<T>(v, part, want, ksplit, tk, r64, row); };
+  float pv[32], pvi[32];
+  int idx = tid, t = idx / lr, i = idx - t * lr;
+  slices(pv, idx < T * lr, t, i);
+  slices(pvi, own && has_inject && blockIdx.x == 0, stt, lr + sq);
+  const UnitRaw<FMT> raw = unit_load<FMT>(up, s * (d >> 6) + (col0 >> 6), work ? ku : 0, (col0 & 63) + r);
+  // the epilogue's operands: thread (token tid / 16, column tid % 16) adds the streams of its column
+  float xpre[QS], npre[QS];
+  const int et = tid >> 4, el = tid & 15;
+#pragma unroll
+  for (int q = 0; q < QS; ++q) if (tid < T * 16 && q < hc) { xpre[q] = xnew[((size_t)et * hc + q) * d + col0 + el]; npre[q] = norm[(size_t)q * d + col0 + el]; } else { xpre[q] = 0.0f; npre[q] = 0.0f; }
+  if (own) {
+    float tot = ssv[0];
+#pragma unroll
+    for (int k = 1; k < (FKS > 0 ? FKS / FHC : 32); ++k) if (k < kps) tot += ssv[k];
+    const float sc = 1.0f / sqrtf(tot / (float)d + eps);
+    for (int k = 0; k < kps; ++k) sls[stt * 32 + sq * kps + k] = sc;
+  }
+  lds_barrier();
+  auto slice_sum = [&](const float (&v)[32], int tk) {      // slices in order, each times its stream's scale
+    float o = 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) if (ks < ksplit) { const float tm = v[ks] * sls[tk * 32 + ks]; o = ks == 0 ? tm : o + tm; }
+    return o; };
+  while (idx < T * lr) {
+    const float v = slice_sum(pv, t) / (float)hc;
+    lo[((size_t)t * U + (i >> 6)) * PYRE_UP_PAD + (i & 63)] = v * sigm(v);
+    idx += nthr;
+    if (idx < T * lr) { t = idx / lr; i = idx - t * lr; slices(pv, true, t, i); }
+  }
+  if (own && blockIdx.x == 0) inj[stt * hc + sq] = has_inject ? slice_sum(pvi, stt) / (float)hc : 0.0f;
+  lds_barrier();
+  if (work) {
+    float acc[TT];
+#pragma unroll
+    for (int k = 0; k < TT; ++k) acc[k] = 0.0f;
+    if constexpr (T % TS == 0) unit_fma<FMT, TT>(up, raw, ku, lds2, tid & 63, lo + ((size_t)ts * U + ku) * PYRE_UP_PAD, TS * U * PYRE_UP_PAD, acc);
+    else {          // an odd width: the second set has a token less
+      if (ts == 0) unit_fma<FMT, TT>(up, raw, ku, lds2, tid & 63, lo + ku * PYRE_UP_PAD, TS * U * PYRE_UP_PAD, acc);
+      else { float a1[TT - 1]; 
+#pragma unroll
+        for (int k = 0; k + 1 < TT; ++k) a1[k] = 0.0f;
+        unit_fma<FMT, TT - 1>(up, raw, ku, lds2, tid & 63, lo + ((size_t)ts * U + ku) * PYRE_UP_PAD, TS * U * PYRE_UP_PAD, a1);
+#pragma unroll
+        for (int k = 0; k + 1 < TT; ++k) acc[k] = a1[k]; }
+    }
+#pragma unroll
+    for (int k = 0; k < TT; ++k) { const int t2 = ts + k * TS; if (t2 < T) red[((size_t)su * T + t2) * 16 + r] = acc[k]; }
+  }
+  lds_barrier();
+  if (tid < T * 16) {
+    float mx = 0.0f;
+#pragma unroll
+    for (int q = 0; q < QS; ++q) if (q < hc) {          // streams ascending from zero (:1380)
+      float g = red[((size_t)(q * U) * T + et) * 16 + el];
+      for (int k = 1; k < U; ++k) g += red[((size_t)(q * U + k) * T + et) * 16 + el];
+      mx += xpre[q] * sls[et * 32 + q * kps] * npre[q] * sigm(g);            // rms, :209: (x * s) * w
+    }
+    mixed[(size_t)et * d + col0 + el] = mx / (float)hc;
+  }
 }
 
 // ---- the same two launches with both GEMVs on the f16 matrix cores -------------------------------------------------------
@@ -540,11 +640,17 @@ template <int FMT, int T> int norm_down_launch(pyre_ctx* ctx, const HcDev& h, co
   ProfScope ps(ctx, "hc_norm_down", qmat_gguf_bytes(h.di, h.di.rows) + 4.0 * T * h.hc * h.d * 4);
 #define NORM_DOWN_GO(NP) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, NP>), dim3(h.di.tiles, p.ksplit, nz), dim3(p.nw * 64), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
                      w.ssq, w.o, p.upw, (const uint2*)ctx->d_iq2xs)
-  if constexpr (FMT == FMT_IQ3_S) { if (comb_parts > 1) NORM_DOWN_GO(PYRE_GEMV_PARTS); else NORM_DOWN_GO(1); } else NORM_DOWN_GO(1);
+#define NORM_DOWN_FIX hipLaunchKernelGGL((k_hc_norm_down<FMT, T, 1, 2048, 10>), dim3(h.di.tiles, p.ksplit, nz), dim3(512), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
+                     w.ssq, w.o, p.upw, (const uint2*)ctx->d_iq2xs)
+  if constexpr (FMT == FMT_IQ3_S) { if (comb_parts > 1) NORM_DOWN_GO(PYRE_GEMV_PARTS); else NORM_DOWN_GO(1); }
+  else if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {          // the A3B width as files store it: constants folded in (6.1 -> 5.0 us a token)
+    if (h.d == 2048 && p.nw == 8 && p.upw == 1 && (!mo.partial || mo.k == 10)) NORM_DOWN_FIX; else NORM_DOWN_GO(1);
+  } else NORM_DOWN_GO(1);
+#undef NORM_DOWN_FIX
 #undef NORM_DOWN_GO
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
-template <int FMT, int T> int up_mix_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, const float* xnew, float eps, float* mixed, float* inj, const HcRoute* rt, int nz = 1) {
+template <int FMT, int T> int up_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, const float* xnew, float eps, float* mixed, float* inj, const HcRoute* rt, int nz) {
   const int nw = h.hc * h.up.U; size_t lds = 4 * ((size_t)T * h.lr + (size_t)nw * T * 64 + (size_t)T * 32 + (size_t)T * h.hc * 64);
   const QMatDev rq = rt ? rt->router : QMatDev{}; float* rp = rt ? rt->part : nullptr;
   ProfScope ps(ctx, rt ? "hc_up_mix_router" : "hc_up_mix", qmat_gguf_bytes(h.up, h.up.rows) + 4.0 * T * (h.hc * h.d + h.d + (double)ksplit * (h.lr + h.hc)) +
@@ -556,6 +662,25 @@ template <int FMT, int T> int up_mix_launch(pyre_ctx* ctx, const HcDev& h, const
   } else UP_MIX_GO(-1);
 #undef UP_MIX_GO
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
+}
+// The formats whose products a lane forms alone; the others take sums of the activations across the wave, which then has to hold one unit.
+constexpr bool up_by_columns(int fmt) { return fmt == FMT_F32 || fmt == FMT_F16 || fmt == FMT_BF16 || fmt == FMT_Q8_0 || fmt == FMT_Q4_K; }
+template <int FMT, int T> int up_mix_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, const float* xnew, float eps, float* mixed, float* inj, const HcRoute* rt) {
+  if constexpr (!up_by_columns(FMT)) return up_mix_rows_launch<FMT, T>(ctx, h, w, ksplit, xnew, eps, mixed, inj, rt, 1);
+  else {
+  constexpr int TS = T > 1 ? 2 : 1;
+  const int items = h.hc * h.up.U * 16, nthr = std::max((TS * items + 63) / 64 * 64, (T * 16 + 63) / 64 * 64); const size_t lds = 4 * ((size_t)T * h.up.U * PYRE_UP_PAD + (size_t)items * T + (size_t)T * 32);
+  { ProfScope ps(ctx, "hc_up_mix", qmat_gguf_bytes(h.up, h.up.rows) + 4.0 * T * (h.hc * h.d + h.d + (double)ksplit * (h.lr + h.hc)));
+#define UP_MIX_C_GO(...) hipLaunchKernelGGL((k_hc_up_mix_c<FMT, T __VA_ARGS__>), dim3(h.d / 16), dim3(nthr), lds, ctx->stream, h.up, w.o, w.ssq, ksplit, h.di.tiles * 64, h.lr, h.hc, h.has_inject ? 1 : 0, xnew, h.norm, eps, h.d, mixed, inj)
+#define UP_MIX_C_A3B , 4, 256, 16
+    bool done = false;
+    if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) { if (h.hc == 4 && h.lr == 256 && ksplit == 16) { UP_MIX_C_GO(UP_MIX_C_A3B); done = true; } }          // the A3B configuration as files store it: constants folded in
+    if (!done) UP_MIX_C_GO();
+#undef UP_MIX_C_A3B
+#undef UP_MIX_C_GO
+  } PYRE_CHECK_LAUNCH(ctx);
+  return rt ? pyre_moe_router_shares_launch(ctx, "hc_up_mix_router", rt->router, mixed, T, h.d / 64, 1, rt->part, rt->dgx) : PYRE_OK;
+  }
 }
 int hc_m_cs(const HcDev& h) { return h.d % 512 == 0 ? 2 : 1; }      // columns a thread of k_hc_norm_down_m prepares
 int hc_m_slices(const HcDev& h) { return h.hc * h.d / (256 * hc_m_cs(h)); }
@@ -632,6 +757,7 @@ int up_mix(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, int t, co
 }
 }  // namespace
 
+bool pyre_hc_leaves_digits(const HcDev& h) { return hc_on_matrix_cores(h) || up_by_columns(h.up.fmt); }
 bool pyre_hc_aop_ok(const HcDev& h) { return hc_on_matrix_cores(h) && h.hc <= 4; }
 bool pyre_hc_route_ok(const HcDev& h, const QMatDev& router) {
   const int f = h.up.fmt;
@@ -658,7 +784,7 @@ int pyre_hc_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, cons
   if (!pyre_hc_rows_ok(h) || groups < 1 || groups > 65535 || x_in == x_out || (rt && !pyre_hc_route_ok(h, rt->router))) return pyre_fail(ctx, PYRE_E_ARG, "hc_mix_rows: unsupported shape");
   const DownPlan p = down_plan(h); const MoeOut mo = comb_moe ? *comb_moe : MoeOut{nullptr, nullptr, nullptr, 0, 0};
   int rc = [&]() -> int { HC_FMT_SWITCH(h.di.fmt, return (norm_down_launch<F, 8>(ctx, h, w, p, x_in, in_ss, in_ts, x_out, comb_out, 1, mo, comb_inj, eps, groups));) }(); if (rc) return rc;
-  return [&]() -> int { HC_FMT_SWITCH(h.up.fmt, return (up_mix_launch<F, 8>(ctx, h, w, p.ksplit, x_out, eps, mixed, inj, rt, groups));) }();
+  return [&]() -> int { HC_FMT_SWITCH(h.up.fmt, return (up_mix_rows_launch<F, 8>(ctx, h, w, p.ksplit, x_out, eps, mixed, inj, rt, groups));) }();
 }
 
 int pyre_hc_mix_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const float* x_in, int in_ss, int in_ts, float* x_out, int t, const float* comb_out, const MoeOut* comb_moe, const float* comb_inj,

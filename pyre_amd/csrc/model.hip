@@ -860,7 +860,7 @@ struct WinRun {
     const int o_parts = outp_in_parts(L, d) ? PYRE_GEMV_PARTS : 1;
     if ((rc = o_parts > 1 ? pyre_gemv_parts_launch(ctx, L.outp, m->core, t, m->o, oa) : pyre_gemv_launch(ctx, L.outp, m->core, t, m->o, oa))) return rc;
     ride = route_rides && pyre_hc_route_ok(L.hcf, L.moe.router);       // the router GEMV rides on the mix's second launch
-    HcRoute hr{L.moe.router, m->rpart, m->mw.dgx};          // (the matrix-core mix leaves the digits of its output; after another mix the expert launch makes them)
+    HcRoute hr{L.moe.router, m->rpart, pyre_moe_takes_digits(L.moe) ? m->mw.dgx : nullptr};          // (where the mix leaves the digits of its output, it does so with the router's sums)
     if ((rc = pyre_hc_mix_launch(ctx, L.hcf, m->hw, xin, in_ss, in_ts, xout, t, m->o, nullptr, m->inj_a, c.eps, m->mixed, m->inj_f, ride ? &hr : nullptr, o_parts))) return rc;
     advance();
     return PYRE_OK;
@@ -878,7 +878,7 @@ struct WinRun {
 
   int moe(int il) {
     const pyre_model_cfg& c = m->c; const Layer& L = m->layers[il]; int rc;
-    RouteSrc rs{m->rpart, c.d / 64, L.moe.router.tiles * 64, pyre_hc_aop_ok(L.hcf) ? m->mw.dgx : nullptr};
+    RouteSrc rs{m->rpart, c.d / 64, L.moe.router.tiles * 64, pyre_moe_takes_digits(L.moe) && pyre_hc_leaves_digits(L.hcf) ? m->mw.dgx : nullptr};
     const bool groups = groups_at(il);
     if ((rc = pyre_moe_launch(ctx, L.moe, m->mw, m->mixed, t, raw_moe ? nullptr : m->y, ride ? &rs : nullptr, groups))) return rc;
     if (groups) { comb_out = m->mw.parts; comb_moe = nullptr; comb_np = PYRE_MOE_GROUPS; }

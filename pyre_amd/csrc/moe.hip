@@ -466,6 +466,16 @@ __global__ __launch_bounds__(64) void k_moe_router_shares(QMatDev q, const float
 }
 
 #define PYRE_MOE_GU_NZMAX 2
+static bool moe_idot() { static const bool on = !(getenv("PYRE_MOE_IDOT") && atoi(getenv("PYRE_MOE_IDOT")) == 0); return on; }
+bool pyre_moe_takes_digits(const MoeDev& m) { return moe_idot() && m.gate_e.fmt == FMT_IQ3_S && m.sh_gate.fmt == FMT_IQ3_S; }
+int pyre_moe_router_shares_launch(pyre_ctx* ctx, const char* name, const QMatDev& router, const float* x, int t, int nw, int upw, float* part, uint32_t* dgx) {
+  const int d = (int)router.cols; const dim3 grid(router.tiles * nw + (dgx ? (d / 64) * t : 0));
+  ProfScope ps(ctx, name, qmat_gguf_bytes(router, router.rows) + 4.0 * t * (d + (double)nw * router.tiles * 64));
+  if (router.fmt == FMT_BF16) hipLaunchKernelGGL(k_moe_router_shares<FMT_BF16>, grid, dim3(64), 0, ctx->stream, router, x, t, d, nw, upw, part, dgx);
+  else if (router.fmt == FMT_F32) hipLaunchKernelGGL(k_moe_router_shares<FMT_F32>, grid, dim3(64), 0, ctx->stream, router, x, t, d, nw, upw, part, dgx);
+  else return pyre_fail(ctx, PYRE_E_TYPE, "moe: the router's shares are for f32 and bf16 matrices");
+  PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
+}
 static bool router_shares_ok(const MoeDev& m) { int nw, upw; pyre_gemv_plan(m.router, &nw, &upw); return (m.router.fmt == FMT_BF16 || m.router.fmt == FMT_F32) && nw <= 16; }
 static size_t router_floats(const MoeDev& m) { int nw, upw; pyre_gemv_plan(m.router, &nw, &upw); const size_t sh = (size_t)nw * m.router.tiles * 64; return 8 * (sh > (size_t)m.n_exp ? sh : (size_t)m.n_exp); }      // logits, or the shares of them
 size_t pyre_moe_work_bytes(const MoeDev& m) {
@@ -488,7 +498,6 @@ void pyre_moe_work_carve(const MoeDev& m, void* base, MoeWork* w) {
     case FMT_C4: { constexpr int F = FMT_C4; CALL; } break; case FMT_C8: { constexpr int F = FMT_C8; CALL; } break; \
     default: { constexpr int F = FMT_IQ3_S; CALL; } break; }
 
-static bool moe_idot() { static const bool on = !(getenv("PYRE_MOE_IDOT") && atoi(getenv("PYRE_MOE_IDOT")) == 0); return on; }
 static bool moe_idot_gu_only() { static const bool on = getenv("PYRE_MOE_IDOT") && atoi(getenv("PYRE_MOE_IDOT")) == 1; return on; }
 // K parts of the gate/up dot products (a property of the matrices, so that every window length gives a token the
 // same bits) and whether a window of t tokens launches one workgroup per part: only a single token does, whose
@@ -508,7 +517,7 @@ int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const floa
   const uint2* g2 = (const uint2*)ctx->d_iq2xs;
   const int P = pyre_moe_gu_parts(m), nz = (P > 1 && t == 1) ? P : 1;
   // IQ3_S experts: gate/up in the integer form, on the digits the mix left beside the activations or on a launch of their own
-  const bool idot = moe_idot() && m.gate_e.fmt == FMT_IQ3_S && m.sh_gate.fmt == FMT_IQ3_S;
+  const bool idot = pyre_moe_takes_digits(m);
   const uint32_t* dgx = nullptr;
   // ... and the down products on the digits of h, which a window's gate/up launch leaves and a single token's down launch forms
   const bool idot_dn = idot && !moe_idot_gu_only() && m.down_e.fmt == FMT_IQ3_S && m.sh_down.fmt == FMT_IQ3_S;
@@ -519,11 +528,8 @@ int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const floa
   if (routed) { lg = routed->p; nsl = routed->nsl; sstride = t * routed->r64; tstride = routed->r64; }
   else if (router_shares_ok(m)) {
     int nw, upw; pyre_gemv_plan(m.router, &nw, &upw); nsl = nw; tstride = m.router.tiles * 64; sstride = t * tstride;
-    const bool dig = idot; const int nd = dig ? (m.d / 64) * t : 0;
-    ProfScope ps(ctx, "moe_router", qmat_gguf_bytes(m.router, m.router.rows) + 4.0 * t * (m.d + (double)nw * tstride));
-    if (m.router.fmt == FMT_BF16) hipLaunchKernelGGL(k_moe_router_shares<FMT_BF16>, dim3(m.router.tiles * nw + nd), dim3(64), 0, ctx->stream, m.router, x, t, m.d, nw, upw, w.logits, w.dgx);
-    else hipLaunchKernelGGL(k_moe_router_shares<FMT_F32>, dim3(m.router.tiles * nw + nd), dim3(64), 0, ctx->stream, m.router, x, t, m.d, nw, upw, w.logits, w.dgx);
-    PYRE_CHECK_LAUNCH(ctx); dgx = dig ? w.dgx : nullptr;
+    int rc = pyre_moe_router_shares_launch(ctx, "moe_router", m.router, x, t, nw, upw, w.logits, idot ? w.dgx : nullptr); if (rc) return rc;
+    dgx = idot ? w.dgx : nullptr;
   } else { int rc = pyre_gemv_launch(ctx, m.router, x, t, w.logits); if (rc) return rc; }
   if (idot && !dgx) {
     if (routed && routed->dgx) dgx = routed->dgx;
@@ -1043,7 +1049,7 @@ int pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const
   MoeBlk b{}; b.rpart = rpart; b.wr = wr; b.parts = parts; b.sel_idx = w.sel_idx; b.sel_w = w.sel_w; b.eoff = w.eoff; b.elist = w.elist; b.partial = w.partial; b.sg = w.sg;
   const int hs = m.ff > m.sf ? m.ff : m.sf, entries = T * (m.top_k + 1), P = pyre_moe_gu_parts(m);
   const uint2* g2 = (const uint2*)ctx->d_iq2xs;
-  const bool idot = moe_idot() && m.gate_e.fmt == FMT_IQ3_S && m.sh_gate.fmt == FMT_IQ3_S, idot_dn = idot && !moe_idot_gu_only() && m.down_e.fmt == FMT_IQ3_S && m.sh_down.fmt == FMT_IQ3_S;
+  const bool idot = pyre_moe_takes_digits(m), idot_dn = idot && !moe_idot_gu_only() && m.down_e.fmt == FMT_IQ3_S && m.sh_down.fmt == FMT_IQ3_S;
   uint32_t* dgh = idot_dn ? w.dgh : nullptr;
   { ProfScope ps(ctx, "moe_rows_route", 4.0 * T * nsl * m.n_exp);
     if (m.n_exp == 512 && m.top_k == 10 && nsl == 32) hipLaunchKernelGGL(k_moe_route_blk<true>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64); else hipLaunchKernelGGL(k_moe_route_blk<false>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64);
