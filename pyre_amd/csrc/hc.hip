@@ -152,10 +152,12 @@ template <int FMT, int T, int NP, int FD = 0, int FK = 0> __global__ __launch_bo
 // from zero (:1380).
 // RF >= 0: the launch also leaves its K slice of the router GEMV over the mixed vector (format RF; HcRoute): wave w
 // takes router tile w, w + nw, .. at unit blockIdx.x, the first tile's weights fetched ahead of the up GEMV.
-template <int FMT, int T, int RF> __global__ __launch_bounds__(1024) void k_hc_up_mix(QMatDev up, const float* __restrict__ part, const float* __restrict__ ssq, int ksplit, int r64, int lr, int hc, int has_inject,
+// FHC, FLR, FKS > 0: the stream count, the low rank and the slice count as compile-time constants (the launcher checks them).
+template <int FMT, int T, int RF, int FHC = 0, int FLR = 0, int FKS = 0> __global__ __launch_bounds__(1024) void k_hc_up_mix(QMatDev up, const float* __restrict__ part, const float* __restrict__ ssq, int ksplit, int r64, int lr, int hc, int has_inject,
     const float* __restrict__ xnew, const float* __restrict__ norm, float eps, int d, float* __restrict__ mixed, float* __restrict__ inj, const uint2* __restrict__ g2,
     QMatDev router, float* __restrict__ rpart) {
   constexpr bool ROUTE = RF >= 0; constexpr int RFX = ROUTE ? RF : FMT_F32;
+  if constexpr (FHC > 0) { hc = FHC; lr = FLR; ksplit = FKS; }
   if (blockIdx.z) {          // a further group of T tokens (pyre_hc_mix_rows_launch)
     const size_t z = blockIdx.z; part += z * ksplit * T * r64; ssq += z * ksplit * T; xnew += z * T * hc * d; mixed += z * T * d; inj += z * T * hc;
     if (ROUTE) rpart += z * (d / 64) * T * router.tiles * 64;
@@ -165,7 +167,7 @@ template <int FMT, int T, int RF> __global__ __launch_bounds__(1024) void k_hc_u
   qmat_args_now(up); args_now(part, ssq, ksplit, r64, lr, hc, has_inject, xnew, norm, eps, d, mixed, inj);
 
   extern __shared__ __align__(16) float sm[];
-  const int nthr = blockDim.x, tid = threadIdx.x, U = lr >> 6, kps = ksplit / hc, nw = nthr >> 6;
+  const int nthr = FHC > 0 ? FHC * FLR : blockDim.x, tid = threadIdx.x, U = lr >> 6, kps = ksplit / hc, nw = nthr >> 6;
   float* lo = sm;                         // [T][lr]
   float* red = sm + (size_t)T * lr;       // [nw][T][64]
   float* sls = red + (size_t)nw * T * 64;   // [T][32]: the RMS scale of the stream each slice belongs to
@@ -655,9 +657,17 @@ template <int FMT, int T> int up_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, 
   const QMatDev rq = rt ? rt->router : QMatDev{}; float* rp = rt ? rt->part : nullptr;
   ProfScope ps(ctx, rt ? "hc_up_mix_router" : "hc_up_mix", qmat_gguf_bytes(h.up, h.up.rows) + 4.0 * T * (h.hc * h.d + h.d + (double)ksplit * (h.lr + h.hc)) +
                (rt ? qmat_gguf_bytes(rq, rq.rows) + 4.0 * T * (h.d / 64) * rq.tiles * 64 : 0.0));
-#define UP_MIX_GO(RF) hipLaunchKernelGGL((k_hc_up_mix<FMT, T, RF>), dim3(h.d / 64, 1, nz), dim3(nw * 64), lds, ctx->stream, h.up, w.o, w.ssq, ksplit, h.di.tiles * 64, h.lr, h.hc, h.has_inject ? 1 : 0, xnew, h.norm, eps, \
+#define UP_MIX_GO(...) hipLaunchKernelGGL((k_hc_up_mix<FMT, T, __VA_ARGS__>), dim3(h.d / 64, 1, nz), dim3(nw * 64), lds, ctx->stream, h.up, w.o, w.ssq, ksplit, h.di.tiles * 64, h.lr, h.hc, h.has_inject ? 1 : 0, xnew, h.norm, eps, \
                      h.d, mixed, inj, (const uint2*)ctx->d_iq2xs, rq, rp)
-  if constexpr (FMT == FMT_IQ3_S || FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {
+  bool done = false;
+  if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {          // the A3B configuration as files store it: constants folded in
+    if (h.hc == 4 && h.lr == 256 && ksplit == 16) {
+      if (rt && rq.fmt == FMT_BF16) UP_MIX_GO(FMT_BF16, 4, 256, 16); else if (rt && rq.fmt == FMT_F32) UP_MIX_GO(FMT_F32, 4, 256, 16); else UP_MIX_GO(-1, 4, 256, 16);
+      done = true;
+    }
+  }
+  if (done) {}
+  else if constexpr (FMT == FMT_IQ3_S || FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {
     if (rt && rq.fmt == FMT_BF16) UP_MIX_GO(FMT_BF16); else if (rt && rq.fmt == FMT_F32) UP_MIX_GO(FMT_F32); else UP_MIX_GO(-1);
   } else UP_MIX_GO(-1);
 #undef UP_MIX_GO
