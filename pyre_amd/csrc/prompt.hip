@@ -132,7 +132,9 @@ __global__ __launch_bounds__(256) void k_blk_op_split(const float* __restrict__ 
 // ---- hyper-connection mix, first part: the pending update, sums of squares, [down ; inject] ---------------------------------------
 // grid (slices of 256 CS columns, groups), 4 CS waves, a thread prepares one column of the slice for the group's tokens once
 // and the waves walk every row tile with it (the launch for a window repeats the gather in each of its row tiles: at 43
-// windows 72 us, here the streams are read once).  x is updated in place: an element has one reader.  Outputs per group: ssq, smx [slice][8], part [slice][8][tiles * 64].
+// windows 72 us, here the streams are read once).  A workgroup is a chain of latencies, so its loads are all issued before the first
+// barrier, and its sums leave through shared memory (adding the second pair's to what the first had stored waited for the stores):
+// 301 tokens 34 -> 25 us, 2000 tokens 161 -> 112 us.  x is updated in place: an element has one reader.  Outputs per group: ssq, smx [slice][8], part [slice][8][tiles * 64].
 // NP: vectors the pending update comes in -- 0 none, 1 = comb[token][d], 4 = comb[group][4][8][d], added in order.
 template <int NP, int CS>
 __global__ __launch_bounds__(256 * CS) void k_blk_mix_down(QMatDev m, const float* __restrict__ x_in, int in_ss, int in_ts, float* __restrict__ x_out, const float* __restrict__ comb, const float* __restrict__ inj,
@@ -140,41 +142,45 @@ __global__ __launch_bounds__(256 * CS) void k_blk_mix_down(QMatDev m, const floa
   constexpr int NW = 4 * CS;
   __shared__ __align__(16) uint16_t ah[CS * 32 * 16 * 8];
   __shared__ float wsum[NW][8], wmax[NW][8];
-  extern __shared__ __align__(16) float hsum[];          // [tiles][4][2][64] (CS == 2)
+  extern __shared__ __align__(16) float hsum[];          // [2][tiles][4][2][64] (CS == 2)
   const int ks = blockIdx.x, grp = blockIdx.y, tid = threadIdx.x, nks = gridDim.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = wave & 3, p = wave >> 2, q = lane >> 4;
   const int c0 = ks * 256 * CS, s = c0 / d, i0 = c0 - s * d, K128 = m.cols >> 7, t0 = grp * 8, nt = min(8, T - t0);
   const float nv = norm[(size_t)s * d + i0 + tid];
-  float v[8];
-  if constexpr (NP > 0) {          // the tokens' weights of the pending update, once for the workgroup
-    if (tid < 8) wsum[0][tid] = 2.0f * b_sigm(inj[(t0 + min(tid, nt - 1)) * hc + s]);
-    lds_barrier();
-  }
-  float wt[8];
-#pragma unroll
-  for (int t = 0; t < 8; ++t) wt[t] = NP > 0 ? wsum[0][t] : 0.0f;
-  if constexpr (NP > 0) lds_barrier();
+  // every load the workgroup needs before its first barrier is issued at once: the tokens' weights of the pending update, the streams,
+  // the update's vectors (tokens past the end repeat the last one and are dropped), the first row tile's weights
+  float v[8], o[8][NP > 0 ? NP : 1];
+  const float iv = NP > 0 && tid < 8 ? inj[(t0 + min(tid, nt - 1)) * hc + s] : 0.0f;
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
-    v[t] = 0.0f;
-    if (t < nt) {
-      v[t] = x_in[(size_t)(t0 + t) * in_ts + (size_t)s * in_ss + i0 + tid];
-      if constexpr (NP > 0) {
-        const float w = wt[t]; float o;
-        if constexpr (NP == 1) o = comb[(size_t)(t0 + t) * d + i0 + tid];
-        else {
-          const float* pc = comb + ((size_t)grp * NP * 8 + t) * d + i0 + tid;
-          o = pc[0];
+    const int tt = min(t, nt - 1);
+    v[t] = x_in[(size_t)(t0 + tt) * in_ts + (size_t)s * in_ss + i0 + tid];
+    if constexpr (NP == 1) o[t][0] = comb[(size_t)(t0 + tt) * d + i0 + tid];
+    else if constexpr (NP > 1) {
 #pragma unroll
-          for (int k = 1; k < NP; ++k) o += pc[(size_t)k * 8 * d];
-        }
-        v[t] = v[t] + o * w;
-      }
+      for (int k = 0; k < NP; ++k) o[t][k] = (comb + ((size_t)grp * NP * 8 + tt) * d + i0 + tid)[(size_t)k * 8 * d];
     }
   }
   const int ch0 = ks * 2 * CS + 2 * p;
   WBuf<1> w0, w1; load_w<1>(m, g, ch0, lane, K128, w0); load_w<1>(m, g, ch0 + 1, lane, K128, w1);
   const NibK nk = nib_consts();
+  if constexpr (NP > 0) {          // the tokens' weights, once for the workgroup
+    if (tid < 8) wmax[0][tid] = 2.0f * b_sigm(iv);
+    lds_barrier();
+    float wt[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) wt[t] = wmax[0][t];
+    lds_barrier();
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      float ov = o[t][0];
+#pragma unroll
+      for (int k = 1; k < NP; ++k) ov += o[t][k];
+      v[t] = v[t] + ov * wt[t];
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 8; ++t) v[t] = t < nt ? v[t] : 0.0f;
   float xs[8];
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
@@ -210,15 +216,16 @@ __global__ __launch_bounds__(256 * CS) void k_blk_mix_down(QMatDev m, const floa
     for (int st = 0; st < 4; ++st) { c0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0[st], d0.b[st], c0, 0, 0, 0); c1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1[st], d1.b[st], c1, 0, 0, 0); }
     scale_add(c0, d0.d, dn0, dn1, tot); scale_add(c1, d1.d, dn0, dn1, tot);
     const float r0 = halves0(tot), r1 = halves1(tot);
-    const size_t row = (size_t)tile * 64 + g * 16 + (lane & 15);
-    if constexpr (CS == 2) { if (p == 1) { float* h = hsum + (((size_t)tile * 4 + g) * 2) * 64 + lane; h[0] = r0; h[64] = r1; } else { pg[(2 * q) * r64 + row] = r0; pg[(2 * q + 1) * r64 + row] = r1; } }
-    else { pg[(2 * q) * r64 + row] = r0; pg[(2 * q + 1) * r64 + row] = r1; }
+    if constexpr (CS == 2) { float* h = hsum + ((((size_t)p * m.tiles + tile) * 4 + g) * 2) * 64 + lane; h[0] = r0; h[64] = r1; }
+    else { const size_t row = (size_t)tile * 64 + g * 16 + (lane & 15); pg[(2 * q) * r64 + row] = r0; pg[(2 * q + 1) * r64 + row] = r1; }
   }
-  if constexpr (CS == 2) {          // the second chunk pair's sums join the first's (the lane that wrote them adds to its own words)
+  if constexpr (CS == 2) {          // the two chunk pairs' sums meet in shared memory and leave as rows
     lds_barrier();
-    if (p == 0) for (int tile = 0; tile < m.tiles && tile * 64 + g * 16 < m.rows; ++tile) {
-      const float* h = hsum + (((size_t)tile * 4 + g) * 2) * 64 + lane; const size_t row = (size_t)tile * 64 + g * 16 + (lane & 15);
-      pg[(2 * q) * r64 + row] += h[0]; pg[(2 * q + 1) * r64 + row] += h[64];
+    for (int i = tid; i < m.tiles * 512; i += 64 * NW) {
+      const int tile = i >> 9, t = (i >> 6) & 7, rl = i & 63;
+      if (tile * 64 + (rl & 48) >= m.rows) continue;
+      const float* h = hsum + (((size_t)tile * 4 + (rl >> 4)) * 2 + (t & 1)) * 64 + (t >> 1) * 16 + (rl & 15);
+      pg[t * r64 + tile * 64 + rl] = h[0] + h[(size_t)m.tiles * 512];
     }
   }
 }
@@ -485,7 +492,7 @@ int pyre_blk_mix_launch(pyre_ctx* ctx, const HcDev& h, const BlkMix& b, const fl
   if (!pyre_blk_mix_ok(h) || (np != 0 && np != 1 && np != PYRE_MOE_GROUPS)) return pyre_fail(ctx, PYRE_E_ARG, "blk_mix: unsupported shape or %d partial vectors", np);
   const int G = (T + 7) / 8, ks = blk_mix_slices(h), cs = blk_mix_cs(h);
   { ProfScope ps(ctx, "blk_mix_down", qmat_gguf_bytes(h.di, h.di.rows) + 4.0 * T * h.hc * h.d * 2);
-    const size_t lds = cs == 2 ? (size_t)h.di_m.tiles * 2048 : 0;
+    const size_t lds = cs == 2 ? (size_t)h.di_m.tiles * 4096 : 0;
 #define MIX_GO(NP, CS) hipLaunchKernelGGL((k_blk_mix_down<NP, CS>), dim3(ks, G), dim3(256 * CS), lds, ctx->stream, h.di_m, x_in, in_ss, in_ts, x, comb, comb_inj, h.norm, h.d, h.hc, T, b.ssq, b.smx, b.part)
     if (cs == 2) { if (np == 0) MIX_GO(0, 2); else if (np == 1) MIX_GO(1, 2); else MIX_GO(PYRE_MOE_GROUPS, 2); }
     else { if (np == 0) MIX_GO(0, 1); else if (np == 1) MIX_GO(1, 1); else MIX_GO(PYRE_MOE_GROUPS, 1); }
