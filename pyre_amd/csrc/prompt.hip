@@ -286,40 +286,50 @@ __global__ __launch_bounds__(256) void k_blk_mix_lo(const float* __restrict__ pa
   if (tid < hc) inj[(size_t)ti * hc + tid] = has_inject ? slice_sum(iv) / (float)hc : 0.0f;
 }
 // ---- third part: up, the gates and the mean of the streams -----------------------------------------------------------------------
-// grid (d / 64, cuts of the groups), 4 hc waves: wave (s, g) keeps row group g of the workgroup's 64 rows of stream s of `up`,
+// grid (d / 32, cuts of the groups), 2 hc waves: wave (s, g) keeps row group g of the workgroup's 32 rows of stream s of `up`,
 // decoded (low rank 256: two chunks, 32 registers), and walks the groups with it; the launch for a window decoded them again
-// for every window and redid the whole prologue in each of its workgroups (212 us at 43 windows).  Outputs: mixed [token][d] (f32) and, with op and inv given, the same as operand rows.
+// for every window and redid the whole prologue in each of its workgroups (212 us at 43 windows).  A turn is products, then the
+// epilogue's vector instructions, with a barrier between: with 64 columns one workgroup fitted a compute unit and its phases took turns
+// (20 us at 301 tokens, 85 at 2000); two of 32 columns overlap theirs, and what a turn reads is asked for a turn ahead (15.9, 70).  Outputs: mixed [token][d] (f32) and, with op and inv given, the same as operand rows.
 template <int KC>
-__global__ __launch_bounds__(1024) void k_blk_mix_up(QMatDev up, const uint4* __restrict__ lo, const float* __restrict__ lo_dn, const float* __restrict__ scl, const float2* __restrict__ opb, const float* __restrict__ x,
+__global__ __launch_bounds__(512) void k_blk_mix_up(QMatDev up, const uint4* __restrict__ lo, const float* __restrict__ lo_dn, const float* __restrict__ scl, const float2* __restrict__ opb, const float* __restrict__ x,
                                                      const float* __restrict__ norm, int hc, int d, int T, int per, float* __restrict__ mixed, uint4* __restrict__ op, size_t op_gs, float* __restrict__ inv, int inv_gs) {
   __shared__ __align__(16) uint4 la[2][KC * 256];
-  __shared__ float red[4][8][64];
-  __shared__ __align__(16) uint16_t st[2][8 * 16 * 8];
+  __shared__ float red[4][8][32];
+  __shared__ __align__(16) uint16_t st[2][4 * 16 * 8];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = lane >> 4, nw = blockDim.x >> 6;
-  const int s = wave >> 2, g = wave & 3, G = (T + 7) >> 3, b0 = blockIdx.y * per, b1 = min(G, b0 + per), col0 = blockIdx.x * 64;
+  const int s = wave >> 1, g = wave & 1, G = (T + 7) >> 3, b0 = blockIdx.y * per, b1 = min(G, b0 + per), col0 = blockIdx.x * 32, nt = blockDim.x >> 5;
   if (b0 >= b1) return;
   WDec wd[KC];
   { const NibK nk = nib_consts(); WBuf<1> w;
 #pragma unroll
     for (int c = 0; c < KC; ++c) { load_w<1>(up, ((s * d + col0) >> 4) + g, c, lane, KC, w); decode_chunk(w.w[0], w.h[0], c, nk, wd[c]); } }
   auto fetch = [&](int grp, int buf) { for (int j = wave; j < KC * 4; j += nw) lds_fetch16(lo + (size_t)grp * KC * 256 + j * 64 + lane, &la[buf][j * 64]); };
-  // thread = (token, column) of the epilogue; with fewer than 512 threads in rounds
-  const int l = tid & 63;
+  // thread = (token, column) of the epilogue; with fewer than 256 threads in rounds
+  const int l = tid & 31;
   float nr[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) nr[k] = k < hc ? norm[(size_t)k * d + col0 + l] : 0.0f;
-  fetch(b0, 0);
+  // what a group's epilogue reads of memory (thread = token tid / 32, column l; the token's factors) and the wave's two tokens' scales
+  const int et = tid >> 5;
+  float xn[4], sn[4], dn0n, dn1n; float2 obn;
+  auto ahead = [&](int grp) {
+    const int t0 = grp * 8; const size_t tc = min(t0 + et, T - 1);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { const bool w = k < hc && et < 8; xn[k] = w ? x[(tc * hc + k) * d + col0 + l] : 0.0f; sn[k] = w ? scl[tc * hc + k] : 0.0f; }
+    obn = op && et < 8 ? opb[tc] : make_float2(0.0f, 0.0f);
+    dn0n = lo_dn[min(t0 + 2 * q, T - 1)]; dn1n = lo_dn[min(t0 + 2 * q + 1, T - 1)]; };
+  fetch(b0, 0); ahead(b0);
   lds_fetch_barrier();
   for (int b = b0; b < b1; ++b) {
     const int buf = (b - b0) & 1, t0 = b * 8;
-    float xv[4];          // the first round's stream values, in flight beside the products
-    { const int t = tid >> 6, ti = min(t0 + t, T - 1);
+    const float dn0 = dn0n, dn1 = dn1n; float xv[4], sv[4]; float2 ob = obn;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) xv[k] = k < hc && t < 8 ? x[((size_t)ti * hc + k) * d + col0 + l] : 0.0f; }
-    if (b + 1 < b1) fetch(b + 1, buf ^ 1);
+    for (int k = 0; k < 4; ++k) { xv[k] = xn[k]; sv[k] = sn[k]; }
+    if (b + 1 < b1) { fetch(b + 1, buf ^ 1); ahead(b + 1); }          // a whole group ahead: a group's own loads would be waited for twice
+    __builtin_amdgcn_sched_barrier(0);
     v4f tot = {0.0f, 0.0f, 0.0f, 0.0f};
-    { const float dn0 = lo_dn[min(t0 + 2 * q, T - 1)], dn1 = lo_dn[min(t0 + 2 * q + 1, T - 1)];
-      v4f acc[KC];
+    { v4f acc[KC];
 #pragma unroll
       for (int c = 0; c < KC; ++c) acc[c] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -330,27 +340,30 @@ __global__ __launch_bounds__(1024) void k_blk_mix_up(QMatDev up, const uint4* __
       for (int c = 0; c < KC; ++c) scale_add(acc[c], wd[c].d, dn0, dn1, tot);
     }
     red[s][2 * q][g * 16 + (lane & 15)] = halves0(tot); red[s][2 * q + 1][g * 16 + (lane & 15)] = halves1(tot);
+    // the next group's operand and values have arrived behind the products; waiting here and not at the end leaves this group's stores
+    // a whole turn to complete
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     lds_barrier();
-    for (int t = tid >> 6; t < 8; t += nw) {
+    for (int t = et; t < 8; t += nt) {
       const int ti = t0 + t; const bool on = ti < T;
       const size_t tc = min(ti, T - 1);
-      if (t >= nw) {
+      if (t >= nt) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) xv[k] = k < hc ? x[(tc * hc + k) * d + col0 + l] : 0.0f;
+        for (int k = 0; k < 4; ++k) { xv[k] = k < hc ? x[(tc * hc + k) * d + col0 + l] : 0.0f; sv[k] = k < hc ? scl[tc * hc + k] : 0.0f; }
+        if (op) ob = opb[tc];
       }
       float mx = 0.0f;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) if (k < hc) mx += xv[k] * scl[tc * hc + k] * nr[k] * b_sigm(red[k][t][l]);            // rms: (x * s) * w
+      for (int k = 0; k < 4; ++k) if (k < hc) mx += xv[k] * sv[k] * nr[k] * b_sigm(red[k][t][l]);            // rms: (x * s) * w
       const float mv = mx / (float)hc;
       if (on) mixed[tc * d + col0 + l] = mv;
       if (op) {
-        const float2 ob = opb[tc];
         uint16_t* o = st[buf] + ((l >> 3) * 16 + 2 * t) * 8 + (l & 7); b_split(mv * ob.x, o, o + 8);
-        if (on && blockIdx.x == 0 && l < (d >> 8)) inv[(size_t)b * inv_gs + l * 8 + t] = ob.y;
+        if (on && blockIdx.x == 0) for (int sb = l; sb < (d >> 8); sb += 32) inv[(size_t)b * inv_gs + sb * 8 + t] = ob.y;
       }
     }
-    lds_fetch_barrier();          // (also: the next group's operand has arrived)
-    if (op && tid < 128) op[(size_t)b * op_gs + (size_t)(col0 >> 3) * 16 + tid] = ((const uint4*)st[buf])[tid];
+    lds_barrier();
+    if (op && tid < 64) op[(size_t)b * op_gs + (size_t)(col0 >> 3) * 16 + tid] = ((const uint4*)st[buf])[tid];
   }
 }
 
@@ -501,8 +514,8 @@ int pyre_blk_mix_launch(pyre_ctx* ctx, const HcDev& h, const BlkMix& b, const fl
   { ProfScope ps(ctx, "blk_mix_lo", 4.0 * T * ks * h.lr);
     hipLaunchKernelGGL(k_blk_mix_lo, dim3(8, G), dim3(256), 0, ctx->stream, b.part, b.ssq, b.smx, ks, h.di_m.tiles * 64, h.lr, h.hc, h.has_inject ? 1 : 0, eps, h.d, T, b.lo, b.lo_dn, b.scl, b.opb, inj); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "blk_mix_up", qmat_gguf_bytes(h.up, h.up.rows) + 4.0 * T * (h.hc * h.d + 2.0 * h.d));
-    const int bx = h.d / 64; int per = (int)std::max<int64_t>(1, (int64_t)bx * G / 512); per = std::min(per, 16);          // about two workgroups a compute unit, a decoded row group used up to sixteen times
-    const dim3 grid(bx, (G + per - 1) / per), blk(h.hc * 256);
+    const int bx = h.d / 32; int per = (int)std::max<int64_t>(1, (int64_t)bx * G / 1024); per = std::min(per, 16);          // about four workgroups a compute unit, a decoded row group used up to sixteen times
+    const dim3 grid(bx, (G + per - 1) / per), blk(h.hc * 128);
     if (h.lr == 256) hipLaunchKernelGGL((k_blk_mix_up<2>), grid, blk, 0, ctx->stream, h.up_m, (const uint4*)b.lo, b.lo_dn, b.scl, b.opb, x, h.norm, h.hc, h.d, T, per, mixed, op, op_gs, inv, inv_gs);
     else hipLaunchKernelGGL((k_blk_mix_up<4>), grid, blk, 0, ctx->stream, h.up_m, (const uint4*)b.lo, b.lo_dn, b.scl, b.opb, x, h.norm, h.hc, h.d, T, per, mixed, op, op_gs, inv, inv_gs); } PYRE_CHECK_LAUNCH(ctx);
   return PYRE_OK;
