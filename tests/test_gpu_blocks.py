@@ -388,6 +388,20 @@ def test_gdn_chunked_prefill_matches_sequential_oracle(ctx, nk, nv, T):
     assert relerr(o1, r1) <= TOL
 
 
+@pytest.mark.parametrize("T", [1, 1023, 1024, 1025, 2049])
+def test_gdn_prefill_from_host_arrays_at_the_edges_of_its_calls(ctx, T):
+    # the host entry cuts a prompt into device calls of 1024 tokens and pinned segments copied by several threads
+    nk, nv = 2, 4
+    p, ch = gdn_params(nk, nv, 820); p["dt"] = np.zeros(nv, np.float32)
+    ga, gb = (lib.Gdn(ctx, nk, nv, 128, 128, 4, 1e-6, p["a"], p["dt"], p["conv_w"], p["norm_w"]) for _ in range(2))
+    S0 = synth.normal((nv, 128, 128), 84, 0.01); cs0 = synth.normal((3, ch), 85, 0.3)
+    ga.set_state(cs0, S0); gb.set_state(cs0, S0)
+    x = gdn_inputs(nv, ch, T, 9600)
+    a, b = ga.prefill_chunked(*x), gb.step(*x)
+    assert relerr(a, b) <= TOL
+    assert relerr(ga.get_state()[1], gb.get_state()[1]) <= TOL and np.array_equal(ga.get_state()[0], gb.get_state()[0])
+
+
 def test_gdn_chunked_prefill_benchmark_length_against_the_step_kernels(ctx):
     # 4096 tokens, 16 QK / 32 V heads, chunk 64: the sequential device kernels (themselves pinned against the oracle)
     # are the reference at this length

@@ -274,6 +274,40 @@ def test_long_prompt_in_blocks_matches_the_oracle(ctx, kind):
     assert np.array_equal(tg, to)
 
 
+@pytest.mark.parametrize("n", [9, 16, 23, 71, 72, 80, 87, 519, 1101])
+@pytest.mark.parametrize("qtype,hc_type", [(synth.IQ3_S, synth.IQ3_S), (synth.IQ3_S, synth.BF16), (synth.Q4_K, synth.BF16), (synth.IQ2_XS, synth.F16)])
+def test_prompt_layer_by_layer_equals_the_windows(ctx, qtype, hc_type, n, monkeypatch):
+    # whole groups, ragged ends, the fewest tokens of a block's grouped experts (72), more than one block of rows (512) and the caches'
+    # 4-bit boundary; bit for bit, and to rounding where the block's experts take the f16 form (IQ3_S mixes, 72 tokens and more)
+    c = small_cfg(qtype=qtype, hc_type=hc_type, hc_lr=256 if hc_type == synth.IQ3_S else 64, n_exp=16, top_k=10)
+    hw = mg.build_host(c, seed=51); gm = lib.Model(ctx, c, hw.layers, hw.globals_)
+    ids = np.random.Generator(np.random.PCG64(n)).integers(0, c.vocab, n + 5, dtype=np.uint32)
+    out = []
+    for windows in ("1", "0"):
+        monkeypatch.setenv("PYRE_PROMPT_WINDOWS", windows)
+        st = gm.new_state(n + 64)
+        out.append((gm.forward(ids[:n], st), gm.forward_multi(ids[n:], st)))
+    for a, b in zip(*out):
+        if hc_type == synth.IQ3_S and n >= 72: assert relerr(a, b) <= 1e-4
+        else: assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("hc_type,router_type", [(synth.BF16, synth.BF16), (synth.F32, synth.F32), (synth.F16, synth.BF16)])
+def test_full_width_mixes_in_file_formats_window_equals_single_steps(ctx, hc_type, router_type):
+    # the launches with the A3B counts folded in (d 2048, four streams, low rank 256), every window width, the router's shares behind
+    # the mix: a window's logits are those of single steps, bit for bit, and the oracle's
+    c = mg.a3b_config(n_layers=1, vocab=512, n_exp=32, ff_exp=256, hc_type=hc_type, router_type=router_type)
+    hw, gm, om = pair(ctx, c, 53)
+    sa, sb, so = gm.new_state(64), gm.new_state(64), om.new_state()
+    g = np.random.Generator(np.random.PCG64(54))
+    for t in range(1, 9):
+        toks = g.integers(0, c.vocab, t, dtype=np.uint32)
+        lv = gm.forward_multi(toks, sa)
+        singles = np.array([gm.forward(toks[i:i + 1], sb) for i in range(t)])
+        assert np.array_equal(lv.view(np.uint32), singles.view(np.uint32)), t
+        assert relerr(lv[-1], om.forward(toks, so)) <= 1e-3, t
+
+
 @pytest.mark.parametrize("n_exp,top_k,ff_sh,qtype", [(32, 13, 512, synth.IQ3_S), (16, 3, 0, synth.IQ3_S), (16, 2, 0, synth.IQ3_S), (16, 10, 0, synth.Q4_K), (16, 11, 512, synth.Q8_0)])
 def test_window_ffn_output_as_group_sums_equals_single_steps_and_the_oracle(ctx, n_exp, top_k, ff_sh, qtype):
     # With IQ3_S hyper-connection matrices a window's FFN output reaches the next mix as four group sums a token (groups of

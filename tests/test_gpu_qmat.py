@@ -393,3 +393,17 @@ def test_q4k_window_on_the_matrix_cores(ctx, rows, cols, ty, switch, monkeypatch
     ctx.prof_enable(False)
     monkeypatch.setenv(switch, "0")
     assert relerr(m.matmul(x), truth) <= TOL                     # (the lane = row window path stays available)
+
+
+# ---- where the operator's windows change their launch: 128 / 129 row tiles (one f32 GEMV / matrix cores), under 256 tiles with rows
+# ---- of up to / over 4096 columns (four / eight waves), 64 / 65 tiles of IQ3_S (a workgroup a row group / a row tile), 256 tiles and
+# ---- 3072 columns of IQ3_S (four waves) -----------------------------------------------------------------------------------------
+@pytest.mark.parametrize("ty,rows,cols", [(ty, r, c) for ty in (lib.Q4_K, lib.Q8_0, lib.IQ2_XS) for r, c in ((8192, 256), (8193, 4096), (8255, 4352), (16320, 512), (16385, 768))] +
+                         [(lib.IQ3_S, r, c) for r, c in ((4095, 512), (4097, 512), (2048, 4096), (16385, 3072), (16385, 3328))])
+def test_window_launch_rules_at_their_edges(ctx, ty, rows, cols):
+    m = lib.QMat(ctx, ty, rows, cols, raw_matrix(ty, rows, cols, 41))
+    x = synth.normal((8, cols), 42)
+    y = m.matmul(x)
+    assert relerr(y, m.matmul_f32(x)) <= TOL
+    for t in (2, 5):          # a token's bits do not depend on the window's width
+        assert np.array_equal(bits(m.matmul(x[:t])), bits(y[:t])), t
