@@ -266,9 +266,10 @@ int   pyre_model_create(pyre_ctx* ctx, const pyre_model_cfg* cfg, const pyre_ten
 void  pyre_model_destroy(pyre_model* m);
 /* GGUF bytes of the weights one decode step reads (dense matrices, router, top_k + 1 experts, head, one embedding row). */
 size_t pyre_model_weight_bytes_per_token(const pyre_model* m);
-/* Blocks of up to 1024 prompt tokens this model's pyre_forward calls have taken layer by layer, a launch a step for all of a block's
- * tokens, since it was created (the prompt path at t >= 16: QMat::matmul's switch to a GEMM, src/model/gguf_q.rs:219-232, and
- * the chunk loop of src/engine_qn.rs:117-138); two such blocks share their launches.  A call of 72 tokens or more takes that path
+/* Blocks of prompt tokens this model's pyre_forward calls have run layer by layer, a launch a step for all of a block's tokens and
+ * the FFN grouped by expert, since it was created: up to 2048 tokens a block (1024 with PYRE_PROMPT_PAIRS=0) and the call's last
+ * tokens with the last one; a call's tokens are cut into as few blocks as that allows, of nearly equal size (the prompt path at t >= 16: QMat::matmul's switch to a GEMM, src/model/gguf_q.rs:219-232, and
+ * the chunk loop of src/engine_qn.rs:117-138).  A call of 72 tokens or more takes that path
  * when every layer's matrices are IQ3_S (router bf16 or f32) with experts of equal widths that are multiples of 256; PYRE_PROMPT_BLOCK=0
  * at model creation keeps the experts in one layout only and every prompt in windows of eight, PYRE_PROMPT_WINDOWS=1 does the
  * latter for the calls made while it is set. */

@@ -540,7 +540,7 @@ static bool prompt_block_ok(const pyre_model* m) {
   return true;
 }
 struct PromptBlk {
-  pyre_ctx* ctx = nullptr; void* mem = nullptr; int T_max = 0; size_t blocks = 0;      // room for T_max tokens a block; blocks: pyre_model_prompt_blocks
+  pyre_ctx* ctx = nullptr; void* mem = nullptr; int T_max = 0; size_t blocks = 0;      // room for T_max tokens a block; blocks whose FFN went by expert (pyre_model_prompt_blocks)
   float *emb = nullptr, *x = nullptr, *mixed = nullptr, *inj_a = nullptr, *inj_f = nullptr, *proj = nullptr, *o = nullptr, *core = nullptr, *inv = nullptr; uint4* op = nullptr; uint32_t* ids = nullptr;
   BlkMix mix{}; MoeBlk moe{}; MoeRows rows{}; HcWork hw{}; GdnChunk gdn{}; float* x2 = nullptr; float* rpart = nullptr; float* q = nullptr; uint16_t* qh = nullptr; float* qsc = nullptr;
   void* att = nullptr; size_t att_bytes = 0;             // the attention's partial sums (grows with the context)
@@ -735,6 +735,7 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
     comb = B->moe.parts; np = PYRE_MOE_GROUPS; cinj = B->inj_f;
   }
   s->len = start + T;
+  if (Tb > 0) ++B->blocks;
   if (!head) return PYRE_OK;
   return prompt_head(ctx, m, B, B->x + (size_t)(T - 1) * hc * d, T);
 }
@@ -955,8 +956,6 @@ int pyre_forward(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, const uint32
       if ((rc = run_block(ctx, m, s, B, ids + i_first, T, tail, head))) { s->broken = true; (void)hipStreamSynchronize(ctx->stream); return rc; }
       i_first += T;
     }
-    // what pyre_model_prompt_blocks counts: the whole windows in front of the call's last eight tokens in blocks of at most 128, an even number of them when taken in pairs
-    const int wins = (n - 8 - (s->mtp ? mtp_window_of(s->mtp) : 0)) / 8; int cnt = pairs ? 2 * ((wins + 255) / 256) : (wins + 127) / 128; while (cnt > 1 && wins / cnt < 8) --cnt; if (!small) B->blocks += cnt;
     if (i_first == n) {
       if (logits_host) PYRE_HIP(ctx, hipMemcpyAsync(logits_host, m->logits, (size_t)m->c.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
       PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); return PYRE_OK;

@@ -258,7 +258,7 @@ def test_long_prompt_in_blocks_matches_the_oracle(ctx, kind):
     prompt = g.integers(0, c.vocab, 250, dtype=np.uint32)
     gs, os_ = gm.new_state(480), om.new_state()
     lg = gm.forward(prompt, gs); lo = om.forward(prompt, os_)
-    assert gm.prompt_blocks() == 2                                     # 30 whole windows: a pair of blocks
+    assert gm.prompt_blocks() == 1
     assert relerr(lg, lo) <= 1e-3 and int(np.argmax(lg)) == int(np.argmax(lo))
     n_lin = sum(1 for il in range(c.n_layers) if not c.full(il))
     for li in range(n_lin):
@@ -268,10 +268,20 @@ def test_long_prompt_in_blocks_matches_the_oracle(ctx, kind):
     assert np.array_equal(tg, to)
     more = g.integers(0, c.vocab, 131, dtype=np.uint32)
     lg = gm.forward(more, gs); lo = om.forward(more, os_)
-    assert gm.prompt_blocks() == 3 and len(gs) == 250 + 5 + 131     # 15 whole windows: one block (the sixth generated token has not been fed)
+    assert gm.prompt_blocks() == 2 and len(gs) == 250 + 5 + 131     # (the sixth generated token has not been fed)
     assert relerr(lg, lo) <= 1e-3 and int(np.argmax(lg)) == int(np.argmax(lo))
     tg, _ = gm.generate_greedy(gs, lg, 6); to, _ = om.generate_greedy(os_, lo, 6)
     assert np.array_equal(tg, to)
+
+
+@pytest.mark.parametrize("pairs,n,want", [("1", 71, 0), ("1", 72, 1), ("1", 2063, 1), ("1", 2064, 2), ("0", 1039, 1), ("0", 1040, 2), ("0", 2064, 3)])
+def test_prompt_blocks_counts_the_blocks_that_ran(ctx, pairs, n, want, monkeypatch):
+    # grouped by expert: the whole groups of eight in front of the call's last eight tokens, 2048 (1024) a block; fewer than 64 are not
+    monkeypatch.setenv("PYRE_PROMPT_PAIRS", pairs)
+    c = small_cfg(qtype=synth.IQ3_S, hc_type=synth.IQ3_S, hc_lr=256, n_layers=2, full_every=2)
+    hw = mg.build_host(c, seed=47); gm = lib.Model(ctx, c, hw.layers, hw.globals_)
+    gm.forward(np.random.Generator(np.random.PCG64(n)).integers(0, c.vocab, n, dtype=np.uint32), gm.new_state(n + 8))
+    assert gm.prompt_blocks() == want
 
 
 @pytest.mark.parametrize("n", [9, 16, 23, 71, 72, 80, 87, 519, 1101])
