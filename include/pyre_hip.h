@@ -268,11 +268,11 @@ void  pyre_model_destroy(pyre_model* m);
 size_t pyre_model_weight_bytes_per_token(const pyre_model* m);
 /* Blocks of prompt tokens this model's pyre_forward calls have run layer by layer, a launch a step for all of a block's tokens and
  * the FFN grouped by expert, since it was created: up to 2048 tokens a block (1024 with PYRE_PROMPT_PAIRS=0) and the call's last
- * tokens with the last one; a call's tokens are cut into as few blocks as that allows, of nearly equal size (the prompt path at t >= 16: QMat::matmul's switch to a GEMM, src/model/gguf_q.rs:219-232, and
- * the chunk loop of src/engine_qn.rs:117-138).  A call of 72 tokens or more takes that path
- * when every layer's matrices are IQ3_S (router bf16 or f32) with experts of equal widths that are multiples of 256; PYRE_PROMPT_BLOCK=0
- * at model creation keeps the experts in one layout only and every prompt in windows of eight, PYRE_PROMPT_WINDOWS=1 does the
- * latter for the calls made while it is set. */
+ * tokens with the last one; a call's tokens are cut into as few blocks as that allows, of nearly equal size (the prompt path at
+ * t >= 16: QMat::matmul's switch to a GEMM, src/model/gguf_q.rs:219-232, and the chunk loop of src/engine_qn.rs:117-138).  A call
+ * of 72 tokens or more takes that path when every layer's mixes and experts are IQ3_S (router bf16 or f32; the other matrices in
+ * any format) with experts of equal widths that are multiples of 256; PYRE_PROMPT_BLOCK=0 at model creation keeps the experts in
+ * one layout only and every prompt in windows of eight, PYRE_PROMPT_WINDOWS=1 does the latter for the calls made while it is set. */
 size_t pyre_model_prompt_blocks(const pyre_model* m);
 /* new_state: empty token list, zero recurrent state, KV room for max_ctx positions. */
 int   pyre_state_create(pyre_ctx* ctx, const pyre_model* m, int max_ctx, pyre_state** out);

@@ -170,8 +170,9 @@ struct GemvEpi { uint32_t* best; const float* conv_w; const float* conv_in; floa
 // producer kernel wrote it); otherwise x_dev is split into the context's operand buffer by one more launch.
 struct PyreAop;
 int pyre_gemv_launch(pyre_ctx* ctx, const QMatDev& m, const float* x_dev, int t, float* y_dev, const PyreAop* a = nullptr);
-// the product of a lane = row matrix for groups of eight tokens in one launch: x [groups * 8][cols] -> y [groups * 8][rows]
-int pyre_gemv_rows_launch(pyre_ctx* ctx, const QMatDev& m, const float* x_dev, int groups, float* y_dev);
+// the product of a lane = row matrix for groups of eight tokens in one launch: x [groups * 8][cols] -> y [groups * 8][rows], or with
+// parts = PYRE_GEMV_PARTS (pyre_gemv_parts_ok) y [groups][parts][8][rows], the sums pyre_gemv_parts_launch leaves for a window
+int pyre_gemv_rows_launch(pyre_ctx* ctx, const QMatDev& m, const float* x_dev, int groups, float* y_dev, int parts = 1);
 // waves per workgroup and units per wave the (unsplit) GEMV uses for this matrix
 void pyre_gemv_plan(const QMatDev& m, int* nw, int* upw);
 // K range split over `ksplit` workgroups per row tile; partial[(ks*t_count + t)*tiles*64 + row] holds the slice sums and

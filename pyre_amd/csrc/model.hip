@@ -516,7 +516,8 @@ static int prompt_pipe_state(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, 
 // windows' launches, so a token has a window's bits and the cutting never shows; the one exception is the grouped FFN, whose
 // operands are f16 halves instead of fixed-point digits: it takes the whole groups of eight in front of the call's last eight
 // tokens, the last 8 .. 15 tokens' FFN (all of it in a call of fewer than 72 tokens) is formed as the windows form it (pyre_moe_rows_launch).
-// For models whose every layer qualifies (prompt_block_ok); PYRE_PROMPT_BLOCK=0 switches it off, PYRE_PROMPT_PAIRS=0 halves the blocks.
+// For models whose every layer qualifies (prompt_block_ok: mixes and experts in IQ3_S; projections in other formats take their windows'
+// lane = row product, eight tokens a group); PYRE_PROMPT_BLOCK=0 switches it off, PYRE_PROMPT_PAIRS=0 halves the blocks.
 #define PROMPT_BLOCK_MIN 64
 #define PROMPT_BLOCK_MAX 2048
 #define PROMPT_TAIL_MAX 96          // tokens whose FFN a block can take in the windows' form: a call of fewer than 72, or the last ones
@@ -533,10 +534,10 @@ static bool gdn_q_on(const pyre_model* m, const Layer& L) {
 static bool prompt_block_ok(const pyre_model* m) {
   if (!prompt_block_env()) return false;
   const pyre_model_cfg& c = m->c;
-  if (m->n_ple > 0 || c.top_k > PYRE_MOE_KMAX || c.d % 256 || c.conv_k < 2 || c.conv_k > 8 || !pyre_blk_mix_ok(m->head)) return false;
+  if (m->n_ple > 0 || c.top_k > PYRE_MOE_KMAX || c.d % 256 || c.conv_k < 2 || c.conv_k > 8) return false;
   for (int il = 0; il < c.n_layers; ++il) { const Layer& L = m->layers[il]; const MoeDev& m0 = m->layers[0].moe;
     if (!pyre_moe_block_ok(L.moe) || (L.moe.router.fmt != FMT_BF16 && L.moe.router.fmt != FMT_F32) || L.moe.router.U != c.d / 64 || L.moe.router.tiles != m0.router.tiles || L.moe.ff != m0.ff || L.moe.sf != m0.sf || L.moe.top_k != m0.top_k || L.moe.n_exp != m0.n_exp ||
-        !pyre_blk_mix_ok(L.hca) || !pyre_blk_mix_ok(L.hcf) || L.proj.fmt != FMT_IQ3_S_M || L.outp.fmt != FMT_IQ3_S_M || L.proj.cols % 256 || L.outp.cols % 256 || L.outp.rows != c.d || (!L.full && !gdn_q_on(m, L))) return false; }
+        !pyre_blk_mix_ok(L.hca) || !pyre_blk_mix_ok(L.hcf) || (int)L.outp.rows != c.d || (!L.full && (L.gdn.dk != 128 || L.gdn.dv != 128 || (L.outp.fmt == FMT_IQ3_S_M) != gdn_q_on(m, L)))) return false; }
   return true;
 }
 struct PromptBlk {
@@ -698,12 +699,14 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
   if ((rc = pyre_row_launch(ctx, m->embd, B->ids, T, B->emb, d))) return rc;
   const float* xin = B->emb; int in_ss = 0, in_ts = d, np = 0; const float* comb = nullptr; const float* cinj = nullptr;
   auto gs = [](int cols) { return (size_t)cols * 2; }; auto is = [](int cols) { return cols / 256 * 8; };
-  const int r64 = m->layers[0].moe.router.tiles * 64;
+  const int r64 = m->layers[0].moe.router.tiles * 64, G = (T + 7) / 8;
   for (int il = 0; il < c.n_layers; ++il) {
     const Layer& L = m->layers[il]; const int pw = L.full ? m->pw_attn : m->pw_lin, oc = L.outp.cols, o_parts = outp_in_parts(L, d) ? PYRE_GEMV_PARTS : 1;
-    if ((rc = pyre_blk_mix_launch(ctx, L.hca, B->mix, xin, in_ss, in_ts, B->x, T, comb, np, cinj, c.eps, B->mixed, B->inj_a, B->op, gs(d), B->inv, is(d)))) return rc;
+    const bool pm = L.proj.fmt == FMT_IQ3_S_M, om = L.outp.fmt == FMT_IQ3_S_M;
+    if ((rc = pyre_blk_mix_launch(ctx, L.hca, B->mix, xin, in_ss, in_ts, B->x, T, comb, np, cinj, c.eps, B->mixed, B->inj_a, pm ? B->op : nullptr, gs(d), B->inv, is(d)))) return rc;
     xin = B->x; in_ss = d; in_ts = hc * d;
-    if ((rc = pyre_blk_gemm_launch(ctx, L.proj, B->op, gs(d), B->inv, is(d), PYRE_INV_TOKEN, B->proj, pw, T, 1))) return rc;
+    if (!pm) { if ((rc = pyre_gemv_rows_launch(ctx, L.proj, B->mixed, G, B->proj))) return rc; }
+    else if ((rc = pyre_blk_gemm_launch(ctx, L.proj, B->op, gs(d), B->inv, is(d), PYRE_INV_TOKEN, B->proj, pw, T, 1))) return rc;
     if (L.full) {
       const int ai = L.mix_index;
       if (m->has_idx) {          // a sparse indexer selects per window of eight, behind the windows before it
@@ -717,15 +720,20 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
         if (pyre_attn_blk_bytes(L.attn, start + T, T) > B->att_bytes) return pyre_fail(ctx, PYRE_E_STATE, "forward: attention scratch of %zu bytes is too small", B->att_bytes);
         if ((rc = pyre_attn_blk_launch(ctx, L.attn, s->kv[ai], B->q, B->qh, B->qsc, B->proj, pw, start, T, B->att, B->core))) return rc;
       }
-      if ((rc = pyre_blk_op_split_launch(ctx, B->core, oc, T, B->op, gs(oc), B->inv, is(oc)))) return rc;
-      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, is(oc), PYRE_INV_BLOCK, B->o, d, T, o_parts))) return rc;
+      if (om) {
+        if ((rc = pyre_blk_op_split_launch(ctx, B->core, oc, T, B->op, gs(oc), B->inv, is(oc)))) return rc;
+        if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, is(oc), PYRE_INV_BLOCK, B->o, d, T, o_parts))) return rc;
+      }
     } else {
       const int li = L.mix_index, b = s->cur[li], nb = b ^ 1;
-      if ((rc = pyre_gdn_rec_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], B->core))) return rc;
+      if ((rc = pyre_gdn_rec_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], om ? B->core : (float*)B->op, om))) return rc;
       s->cur[li] = nb;
-      if ((rc = pyre_blk_gdn_out_q_launch(ctx, B->core, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, B->op, gs(oc), B->inv, oc / 16))) return rc;
-      if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, oc / 16, PYRE_INV_CHUNK, B->o, d, T, o_parts))) return rc;
+      if (om) {
+        if ((rc = pyre_blk_gdn_out_q_launch(ctx, B->core, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, B->op, gs(oc), B->inv, oc / 16))) return rc;
+        if ((rc = pyre_blk_gemm_launch(ctx, L.outp, B->op, gs(oc), B->inv, oc / 16, PYRE_INV_CHUNK, B->o, d, T, o_parts))) return rc;
+      } else if ((rc = pyre_blk_gdn_out_w_launch(ctx, (float*)B->op, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, B->core))) return rc;
     }
+    if (!om && (rc = pyre_gemv_rows_launch(ctx, L.outp, B->core, G, B->o, o_parts))) return rc;
     if ((rc = pyre_blk_mix_launch(ctx, L.hcf, B->mix, xin, in_ss, in_ts, B->x, T, B->o, o_parts, B->inj_a, c.eps, B->mixed, B->inj_f, nullptr, 0, nullptr, 0))) return rc;
     const bool end = il == c.n_layers - 1;
     if (end && !head) break;          // nobody reads the last layer's FFN

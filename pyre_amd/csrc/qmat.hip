@@ -229,7 +229,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemv(QMatDev m, const float* __rest
 #pragma unroll
     for (int k = 0; k < 8; ++k) { cw[k] = k < ep.kk ? ep.conv_w[row * ep.kk + k] : 0.0f; chist[k] = k < ep.kk - 1 ? ep.conv_in[(size_t)k * ep.ch + row] : 0.0f; }
   }
-  if (blockIdx.z) { x += (size_t)blockIdx.z * T * m.cols; y += (size_t)blockIdx.z * T * m.rows; }          // (a further group of T tokens: pyre_gemv_rows_launch)
+  if (blockIdx.z) { x += (size_t)blockIdx.z * T * m.cols; y += (size_t)blockIdx.z * T * (ksplit == 1 ? (size_t)m.rows : (size_t)ksplit * m.tiles * 64); }          // (a further group of T tokens: pyre_gemv_rows_launch)
   const int k0 = (ks * NW + wave) * upw; const int k1 = min(m.U, k0 + upw);
   float acc[T];
 #pragma unroll
@@ -370,10 +370,10 @@ int pyre_gemv_launch(pyre_ctx* ctx, const QMatDev& m, const float* x, int t, flo
   FMT_DISPATCH(m.fmt, rc = gemv_f<F>(ctx, m, x, t, y, 1, GemvEpi{}));
   return rc;
 }
-int pyre_gemv_rows_launch(pyre_ctx* ctx, const QMatDev& m, const float* x, int groups, float* y) {
-  if (m.fmt == FMT_IQ3_S_M || groups < 1 || groups > 65535) return pyre_fail(ctx, PYRE_E_ARG, "gemv: %d groups of rows", groups);
-  GemvEpi ep{}; ep.nz = groups; int rc = PYRE_OK;
-  FMT_DISPATCH(m.fmt, rc = (gemv_t<F, 8>(ctx, m, x, y, 1, ep)));
+int pyre_gemv_rows_launch(pyre_ctx* ctx, const QMatDev& m, const float* x, int groups, float* y, int parts) {
+  if (m.fmt == FMT_IQ3_S_M || groups < 1 || groups > 65535 || !(parts == 1 || (parts == PYRE_GEMV_PARTS && pyre_gemv_parts_ok(m)))) return pyre_fail(ctx, PYRE_E_ARG, "gemv: %d groups of rows in %d parts", groups, parts);
+  GemvEpi ep{}; ep.nz = groups; ep.four_waves = parts > 1; int rc = PYRE_OK;
+  FMT_DISPATCH(m.fmt, rc = (gemv_t<F, 8>(ctx, m, x, y, parts, ep)));
   return rc;
 }
 int pyre_gemv_split_launch(pyre_ctx* ctx, const QMatDev& m, const float* x, int t, float* partial, int ksplit, const PyreAop* a) {

@@ -302,6 +302,34 @@ def test_prompt_layer_by_layer_equals_the_windows(ctx, qtype, hc_type, n, monkey
         else: assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+PROJ = (mg.ATTN_Q, mg.ATTN_K, mg.ATTN_V, mg.LIN_QKV, mg.LIN_Z, mg.LIN_BETA, mg.LIN_ALPHA)
+OUTP = (mg.ATTN_O, mg.LIN_OUT)
+HEAD = (mg.G_HEAD_DOWN, mg.G_HEAD_UP)
+WIDE = dict(d=512, n_head=8, lin_nv=16)          # output projections of 2048 columns, which the windows leave in four parts
+
+
+@pytest.mark.parametrize("other,slots,geom", [(synth.Q6_K, PROJ + OUTP, {}), (synth.Q6_K, PROJ + OUTP, WIDE), (synth.Q4_K, OUTP, WIDE), (synth.Q8_0, PROJ, WIDE),
+                                              (synth.BF16, (mg.ATTN_O,), {}), (synth.BF16, HEAD, {})])
+def test_prompt_blocks_of_models_with_other_formats_beside_iq3s_experts(ctx, other, slots, geom, monkeypatch):
+    # What a block asks for is IQ3_S experts and mixes; projections and the head's mix are any.  Bits of the windows below 72 tokens,
+    # rounding (the f16 form of the experts) above.
+    c = small_cfg(**{**dict(qtype=synth.IQ3_S, hc_type=synth.IQ3_S, hc_lr=256, n_exp=16, top_k=10), **geom})
+    hw = mg.build_host(c, seed=61)
+    o = mg.build_host(small_cfg(**{**dict(qtype=other, hc_type=other if slots is HEAD else synth.IQ3_S, hc_lr=256, n_exp=16, top_k=10), **geom}), seed=62)
+    for a, b in [(hw.globals_, o.globals_)] if slots is HEAD else zip(hw.layers, o.layers):
+        a.update({s: b[s] for s in slots if s in b})
+    gm = lib.Model(ctx, c, hw.layers, hw.globals_)
+    for n, blocks in ((9, 0), (71, 0), (80, 1), (519, 1)):
+        ids = np.random.Generator(np.random.PCG64(n)).integers(0, c.vocab, n + 5, dtype=np.uint32); out = []
+        for windows in ("1", "0"):
+            monkeypatch.setenv("PYRE_PROMPT_WINDOWS", windows)
+            st = gm.new_state(n + 64); n0 = gm.prompt_blocks()
+            out.append((gm.forward(ids[:n], st), gm.forward_multi(ids[n:], st)))
+            assert gm.prompt_blocks() - n0 == (blocks if windows == "0" else 0), n
+        for a, b in zip(*out):
+            assert relerr(a, b) <= 1e-4 if n >= 72 else np.array_equal(a.view(np.uint32), b.view(np.uint32)), n
+
+
 @pytest.mark.parametrize("hc_type,router_type", [(synth.BF16, synth.BF16), (synth.F32, synth.F32), (synth.F16, synth.BF16)])
 def test_full_width_mixes_in_file_formats_window_equals_single_steps(ctx, hc_type, router_type):
     # the launches with the A3B counts folded in (d 2048, four streams, low rank 256), every window width, the router's shares behind
