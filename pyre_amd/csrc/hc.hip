@@ -696,7 +696,7 @@ int hc_m_cs(const HcDev& h) { return h.d % 512 == 0 ? 2 : 1; }      // columns a
 int hc_m_slices(const HcDev& h) { return h.hc * h.d / (256 * hc_m_cs(h)); }
 bool hc_on_matrix_cores(const HcDev& h) {
   static const bool off = [] { const char* e = getenv("PYRE_HC_ROWS"); return e && *e && atoi(e) != 0; }();      // 1: the lane = row kernels for every window width
-  return !off && h.di_m.fmt == FMT_IQ3_S_M && h.up_m.fmt == FMT_IQ3_S_M && h.d % 256 == 0 && hc_m_slices(h) <= 16 && h.lr % 256 == 0 && h.hc * 4 <= 16 && h.di_m.tiles == h.di.tiles;
+  return !off && h.di_m.fmt == FMT_IQ3_S_M && h.up_m.fmt == FMT_IQ3_S_M && h.d % 256 == 0 && hc_m_slices(h) <= 16 && h.lr % 256 == 0 && h.hc >= 2 && h.hc * 4 <= 16 && h.di_m.tiles == h.di.tiles;          // (a single stream's second launch has 256 threads for the 512 values of eight tokens)
 }
 template <int T> int norm_down_m_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const float* x_in, int in_ss, int in_ts, float* x_out, const float* comb_out, int comb_parts, const MoeOut& mo, const float* comb_inj) {
   ProfScope ps(ctx, "hc_norm_down", qmat_gguf_bytes(h.di, h.di.rows) + 4.0 * T * h.hc * h.d * 4);

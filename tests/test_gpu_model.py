@@ -302,6 +302,18 @@ def test_prompt_layer_by_layer_equals_the_windows(ctx, qtype, hc_type, n, monkey
         else: assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("geom", [dict(hc_lr=256), dict(hc_lr=768), dict(hc_lr=1024, d=512), dict(hc_lr=256, d=4608, n_layers=2, full_every=2)])
+def test_single_stream_models_match_the_oracle(ctx, geom):
+    # one residual stream with IQ3_S mixes: windows of up to eight tokens, single steps, a prompt past the grouped experts' fewest tokens
+    c = small_cfg(**{**dict(hc=1, qtype=synth.IQ3_S, hc_type=synth.IQ3_S, n_exp=16, top_k=10), **geom})
+    hw, gm, om = pair(ctx, c, 71)
+    ids = np.random.Generator(np.random.PCG64(72)).integers(0, c.vocab, 90, dtype=np.uint32)
+    gs, os_ = gm.new_state(128), om.new_state()
+    assert relerr(gm.forward(ids[:80], gs), om.forward(ids[:80], os_)) <= 1e-3
+    assert relerr(gm.forward_multi(ids[80:88], gs), om.forward_multi(ids[80:88], os_)) <= 1e-3
+    assert relerr(gm.forward(ids[88:89], gs), om.forward(ids[88:89], os_)) <= 1e-3
+
+
 PROJ = (mg.ATTN_Q, mg.ATTN_K, mg.ATTN_V, mg.LIN_QKV, mg.LIN_Z, mg.LIN_BETA, mg.LIN_ALPHA)
 OUTP = (mg.ATTN_O, mg.LIN_OUT)
 HEAD = (mg.G_HEAD_DOWN, mg.G_HEAD_UP)
