@@ -1,10 +1,10 @@
 // Gated DeltaNet recurrent step: causal depthwise conv1d + SiLU, L2-normalised q/k, gated delta rule on the fp32
 // state kept resident in HBM, gated RMSNorm.  Follows linear_core, src/model/qwen4exp_gguf.rs:1624-1673.
 #include "formats.h"
+#include "workers.h"
 #include <algorithm>
 #include <condition_variable>
 #include <mutex>
-#include <thread>
 PYRE_TS_DECL(gdn_ts) PYRE_TS_EXPORT(gdn_ts, pyre_debug_ts_gdn)
 
 __device__ __forceinline__ float g_sigm(float x) { return 1.0f / (1.0f + expf(-x)); }
@@ -306,7 +306,8 @@ int pyre_gdn_prefill_parts(pyre_ctx* ctx, pyre_gdn* g, const float* qkv, size_t 
     memcpy(out_host, P->buf(0, 1, 0), (size_t)T * ow * 4); return PYRE_OK;
   }
   // segments of SEG bytes of input; a segment's rows are interleaved on the way into its pinned buffer
-  PrefillJob J; J.seg = (int)std::min((size_t)64, HostPipe::SEG / (pw * 4)); J.n = (T + J.seg - 1) / J.seg; J.in_done.assign(J.n, 0);
+  PrefillJob J; J.seg = (int)std::min((size_t)64, HostPipe::SEG / (pw * 4)); J.n = (T + J.seg - 1) / J.seg;
+  try { J.in_done.assign(J.n, 0); } catch (...) { return pyre_fail(ctx, PYRE_E_NOMEM, "pyre_gdn_prefill_chunked: %d segments", J.n); }
   auto put = [&](int w, int i) -> hipError_t {          // segment i up, through worker w's buffers
     const int b = J.used[w][0]++ & 1, t0 = i * J.seg, t1 = std::min(T, t0 + J.seg);
     hipError_t e = hipEventSynchronize(P->ev[w][0][b]); if (e != hipSuccess) return e;
@@ -334,9 +335,10 @@ int pyre_gdn_prefill_parts(pyre_ctx* ctx, pyre_gdn* g, const float* qkv, size_t 
       J.cv.wait(lk);
     }
   };
-  std::vector<std::thread> th; const int nth = std::min(HostPipe::WORKERS - 1, J.n / 4);          // (a short prompt: the caller alone)
-  const int dev = ctx->device;
-  for (int w = 1; w <= nth; ++w) th.emplace_back([&, w] { (void)hipSetDevice(dev); while (work(w, true)) {} });
+  std::vector<std::thread> th; const int dev = ctx->device;
+  auto helper = [&](int w) { (void)hipSetDevice(dev); while (work(w, true)) {} };
+  start_helpers(th, helper_count(std::min(HostPipe::WORKERS - 1, J.n / 4)), helper);          // (a short prompt, or no thread to be had: the caller alone)
+  const int nth = (int)th.size();
   bool bad = false;
   for (int t0 = 0; t0 < T && !rc && !bad; t0 += PC) {
     const int t = std::min(PC, T - t0), last = (t0 + t - 1) / J.seg;

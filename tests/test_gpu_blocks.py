@@ -1,5 +1,7 @@
 """GPU parity of the block-level entry points (MoE FFN, Gated DeltaNet step, gated attention over the 4-bit cache)
 against the CPU oracle, through the C ABI.  Tolerance 1e-5 on max|d| / max|ref| unless stated."""
+import os
+
 import numpy as np
 import pytest
 
@@ -400,6 +402,22 @@ def test_gdn_prefill_from_host_arrays_at_the_edges_of_its_calls(ctx, T):
     a, b = ga.prefill_chunked(*x), gb.step(*x)
     assert relerr(a, b) <= TOL
     assert relerr(ga.get_state()[1], gb.get_state()[1]) <= TOL and np.array_equal(ga.get_state()[0], gb.get_state()[0])
+
+
+def test_gdn_prefill_from_host_arrays_without_helper_threads(ctx):
+    # a caller bound to one core stages all 33 segments itself: the bits of the call with helpers
+    nk, nv, T = 2, 4, 2049
+    p, ch = gdn_params(nk, nv, 821); x = gdn_inputs(nv, ch, T, 9700); out = []
+    cores = os.sched_getaffinity(0)
+    for use in (cores, {min(cores)}):
+        os.sched_setaffinity(0, use)
+        try:
+            g = lib.Gdn(ctx, nk, nv, 128, 128, 4, 1e-6, p["a"], p["dt"], p["conv_w"], p["norm_w"])
+            out.append((g.prefill_chunked(*x),) + g.get_state())
+        finally:
+            os.sched_setaffinity(0, cores)
+    for a, b in zip(*out):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
 def test_gdn_chunked_prefill_benchmark_length_against_the_step_kernels(ctx):
