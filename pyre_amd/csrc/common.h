@@ -444,14 +444,15 @@ int pyre_gdn_launch(pyre_ctx* ctx, const GdnDev& g, const float* proj, int proj_
                     const float* ssm_in, float* ssm_out, float* co_scratch, float* out_dev, bool conv_done = false, uint16_t* aop = nullptr, float aop_up = 1.0f, const GdnQ* gq = nullptr);
 
 // Chunked (64-token) form of the same recurrence on the fp32 matrix cores (gdn_prefill.hip), any T >= 1: raw outputs
-// oraw [T][nv*dv] (no head norm: pyre_blk_gdn_out_launch), states conv_in -> conv_out and ssm_in -> ssm_out (in == out is fine).
+// oraw [T][nv*dv] (no head norm: pyre_blk_gdn_out_launch), states conv_in -> conv_out (two buffers; the same one is refused) and
+// ssm_in -> ssm_out (in == out is fine).
 struct GdnChunk { float* co; float* kt; float* w; float* u; float* p; float* dec; };
 size_t pyre_gdn_chunk_bytes(const GdnDev& g, int T);
 void   pyre_gdn_chunk_carve(const GdnDev& g, int T, void* base, GdnChunk* b);
 int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int proj_stride, int T, const float* conv_in, float* conv_out,
                           const float* ssm_in, float* ssm_out, float* oraw);
 // the recurrence token by token instead, the bits of pyre_gdn_launch's per-quarter form (quarters) or of its head-a-workgroup form
-// (conv_in != conv_out; b.co and b.dec are all it needs)
+// (b.co and b.dec are all it needs)
 int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int proj_stride, int T, const float* conv_in, float* conv_out,
                         const float* ssm_in, float* ssm_out, float* oraw, bool quarters = true);
 

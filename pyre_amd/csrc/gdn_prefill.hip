@@ -85,7 +85,7 @@ __global__ __launch_bounds__(256) void k_gdnc_conv(GdnDev p, const float* __rest
 #pragma unroll
     for (int i = 0; i < 16; i += 4) *(float4*)(k2 + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
   }
-  if (t0 <= T - 1 && T - 1 < t0 + 16) for (int k = 0; k < kk - 1; ++k) {          // (in == out is fine: only the first group of sixteen reads conv_in, and it has)
+  if (t0 <= T - 1 && T - 1 < t0 + 16) for (int k = 0; k < kk - 1; ++k) {          // (the last group of sixteen writes conv_out, the first reads conv_in, in no order: never the same buffer)
     const int src = T - (kk - 1) + k;
     if (src >= 0) conv_out[(size_t)k * ch + c] = proj[(size_t)src * stride + c];
     else { float hv = 0.0f;
@@ -376,7 +376,7 @@ void pyre_gdn_chunk_carve(const GdnDev& g, int T, void* base, GdnChunk* b) {
 }
 int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int stride, int T, const float* conv_in, float* conv_out, const float* ssm_in, float* ssm_out, float* oraw) {
   if (g.dk != 128 || g.dv != 128) return pyre_fail(ctx, PYRE_E_SHAPE, "gdn prompt: head dims %dx%d unsupported (128x128 only)", g.dk, g.dv);
-  if (T < 1 || g.conv_k < 1 || g.conv_k > 8) return pyre_fail(ctx, PYRE_E_ARG, "gdn prompt: %d tokens, %d taps", T, g.conv_k);
+  if (T < 1 || g.conv_k < 1 || g.conv_k > 8 || conv_in == conv_out) return pyre_fail(ctx, PYRE_E_ARG, "gdn prompt: %d tokens, %d taps%s", T, g.conv_k, conv_in == conv_out ? ", the history in place" : "");
   const int ch = 2 * g.nk * g.dk + g.nv * g.dv, nch = (T + C - 1) / C, Tp = nch * C;
   { ProfScope ps(ctx, "gdn_prompt_conv", 8.0 * T * ch);
     if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, b.kt, (float2*)nullptr);
@@ -391,7 +391,7 @@ int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, con
 // the same steps with the recurrence token by token, bit for bit that of the windows' kernels (pyre_gdn_launch with GdnQ); ssm_in == ssm_out is fine, conv_in == conv_out is not
 int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int stride, int T, const float* conv_in, float* conv_out, const float* ssm_in, float* ssm_out, float* oraw, bool quarters) {
   if (g.dk != 128 || g.dv != 128) return pyre_fail(ctx, PYRE_E_SHAPE, "gdn prompt: head dims %dx%d unsupported (128x128 only)", g.dk, g.dv);
-  if (T < 1 || g.conv_k < 1 || g.conv_k > 8 || conv_in == conv_out) return pyre_fail(ctx, PYRE_E_ARG, "gdn prompt: %d tokens, %d taps", T, g.conv_k);
+  if (T < 1 || g.conv_k < 1 || g.conv_k > 8 || conv_in == conv_out) return pyre_fail(ctx, PYRE_E_ARG, "gdn prompt: %d tokens, %d taps%s", T, g.conv_k, conv_in == conv_out ? ", the history in place" : "");
   const int ch = 2 * g.nk * g.dk + g.nv * g.dv, Tp = (T + 15) / 16 * 16;
   { ProfScope ps(ctx, "gdn_prompt_conv", 8.0 * T * ch);
     if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256 + 1, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr, (float2*)b.dec);

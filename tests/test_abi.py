@@ -1,6 +1,8 @@
 """No-GPU checks of the C-ABI library: it loads, and it exports every symbol include/pyre_hip.h declares."""
 import ctypes as C
 import os
+import subprocess
+import sys
 
 import pytest
 
@@ -15,6 +17,24 @@ def test_library_is_built_and_exports_every_declared_symbol():
     assert len(names) >= 20
     missing = [n for n in names if not hasattr(L, n)]
     assert not missing, missing
+
+
+def test_prompt_recurrence_launches_refuse_the_convolution_history_in_place():
+    # the workgroups that read the old history and those that write the new one are not ordered: refused before anything is launched
+    # (the two launchers by their C++ names, in a process of its own)
+    code = '''
+import ctypes as C, re, subprocess, sys
+so = sys.argv[1]; L = C.CDLL(so); syms = subprocess.run(["nm", "-D", "--defined-only", so], capture_output=True, text=True, check=True).stdout
+class Gdn(C.Structure): _fields_ = [("p", C.c_void_p * 4), ("nk", C.c_int), ("nv", C.c_int), ("dk", C.c_int), ("dv", C.c_int), ("conv_k", C.c_int), ("eps", C.c_float)]
+g = Gdn(nk=2, nv=4, dk=128, dv=128, conv_k=4); b = (C.c_void_p * 6)(); h = C.c_void_p(4096); n = C.c_void_p()
+L.pyre_last_error.restype = C.c_char_p; L.pyre_last_error.argtypes = [C.c_void_p]
+for name in ("pyre_gdn_chunk_launch", "pyre_gdn_rec_launch"):
+    f = getattr(L, re.search(r" (_Z\\d+%s\\w+)" % name, syms).group(1))
+    rc = f(n, C.byref(g), C.byref(b), n, C.c_int(0), C.c_int(40), h, h, n, n, n, C.c_bool(True))
+    assert rc == -1 and b"in place" in L.pyre_last_error(None), (name, rc, L.pyre_last_error(None))
+'''
+    r = subprocess.run([sys.executable, "-c", code, lib.LIB_PATH], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, (r.returncode, r.stderr[-800:])
 
 
 def test_python_binding_declares_every_header_symbol():
