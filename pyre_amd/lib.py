@@ -168,8 +168,15 @@ def ngram_draft(history, k, min_n, max_n):
 
 def adapt_plan(n, ts, tv, p, td):
     """spec::adapt_plan through the library (host only, needs no GPU); tv: ten verify times, 0 = unmeasured."""
-    t = np.ascontiguousarray(tv, dtype=np.float64); assert t.size == 10
+    t = np.ascontiguousarray(tv, dtype=np.float64)
+    _expect(t.size == 10, "tv", "ten verify times", t.shape)
     return int(load().pyre_adapt_plan(n, ts, t.ctypes.data_as(C.c_void_p), p, td))
+
+
+def _expect(ok, what, wanted, got):
+    """The library takes pointers: what it would read is checked here, under python -O too."""
+    if not ok:
+        raise ValueError("%s: expected %s, got %s" % (what, wanted, got))
 
 
 class Safetensors:
@@ -422,7 +429,7 @@ class Gdn:
     def step(self, qkv, z, beta, alpha):
         proj = np.ascontiguousarray(np.concatenate([qkv, z, beta, alpha], axis=1), dtype=np.float32)
         t = proj.shape[0]
-        assert proj.shape[1] == self.pw
+        _expect(proj.shape[1] == self.pw, "qkv, z, beta, alpha", "%d columns in all" % self.pw, proj.shape[1])
         out = np.empty((t, self.nv * self.dv), dtype=np.float32)
         self.ctx.check(self.ctx.L.pyre_gdn_step(self.ctx.h, self.h, _ptr(proj), t, _ptr(out)), "gdn_step")
         return out
@@ -430,7 +437,8 @@ class Gdn:
     def prefill_chunked(self, qkv, z, beta, alpha, chunk=64):
         parts = [np.ascontiguousarray(v, dtype=np.float32) for v in (qkv, z, beta, alpha)]
         t = parts[0].shape[0]
-        assert [p.shape for p in parts] == [(t, self.ch), (t, self.nv * self.dv), (t, self.nv), (t, self.nv)]
+        want = [(t, self.ch), (t, self.nv * self.dv), (t, self.nv), (t, self.nv)]
+        _expect([p.shape for p in parts] == want, "qkv, z, beta, alpha", want, [p.shape for p in parts])
         out = np.empty((t, self.nv * self.dv), dtype=np.float32)
         args = [a for p in parts for a in (_ptr(p), p.shape[1])]
         self.ctx.check(self.ctx.L.pyre_gdn_prefill_parts(self.ctx.h, self.h, *args, t, chunk, _ptr(out)), "gdn_prefill_chunked")
@@ -485,7 +493,8 @@ class Attn:
         self.ctx.check(self.ctx.L.pyre_attn_set_context(self.ctx.h, self.h, ctx_train, ctx_tokens), "attn_set_context")
 
     def load_index(self, ik):
-        ik = np.ascontiguousarray(ik, dtype=np.float32); assert ik.shape[0] == len(self)
+        ik = np.ascontiguousarray(ik, dtype=np.float32)
+        _expect(ik.shape[0] == len(self), "ik", "%d rows" % len(self), ik.shape)
         self.ctx.check(self.ctx.L.pyre_attn_load_index(self.ctx.h, self.h, _ptr(ik)), "attn_load_index")
 
     def read_index(self):
@@ -718,7 +727,7 @@ class Model:
         ds = None
         if draft_stream is not None:
             ds = np.ascontiguousarray(draft_stream, dtype=np.uint32)
-            assert ds.size >= n_out + 8
+            _expect(ds.size >= n_out + 8, "draft_stream", "%d ids or more" % (n_out + 8), ds.shape)
         rounds = C.c_int(0)
         self.ctx.check(self.ctx.L.pyre_generate_greedy(self.ctx.h, self.h, st.h, _ptr(fl), n_out, _ptr(out), n_draft, _ptr(ds), C.byref(rounds)), "generate_greedy")
         return out, rounds.value
@@ -818,7 +827,7 @@ class Mtp:
     def generate_greedy_forced(self, st, first_logits, n_out, forced_stream, k=3):
         """The same loop with the drafter's ids replaced (after it ran) by forced_stream: the accepted path end to end."""
         fl = np.ascontiguousarray(first_logits, dtype=np.float32); fs = np.ascontiguousarray(forced_stream, dtype=np.uint32)
-        assert fs.size >= n_out + 8
+        _expect(fs.size >= n_out + 8, "forced_stream", "%d ids or more" % (n_out + 8), fs.shape)
         out = np.empty(n_out, dtype=np.uint32); r, d, a = C.c_int(0), C.c_int(0), C.c_int(0)
         self.m.ctx.check(self.m.ctx.L.pyre_generate_greedy_mtp_forced(self.m.ctx.h, self.m.h, self.h, st.h, _ptr(fl), n_out, _ptr(out), k, _ptr(fs),
                                                                       C.byref(r), C.byref(d), C.byref(a)), "generate_greedy_mtp_forced")

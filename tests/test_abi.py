@@ -37,6 +37,30 @@ for name in ("pyre_gdn_chunk_launch", "pyre_gdn_rec_launch"):
     assert r.returncode == 0, (r.returncode, r.stderr[-800:])
 
 
+def test_shape_checks_hold_without_assertions():
+    # python -O drops assert statements; a short array would be read past its end behind the C ABI
+    code = '''
+import numpy as np
+from pyre_amd import lib
+z = lambda *s: np.zeros(s, np.float32)
+g = object.__new__(lib.Gdn); g.h = None; g.ch, g.nv, g.dv, g.pw = 1024, 4, 128, 1544
+m = object.__new__(lib.Model); m.h = None; d = object.__new__(lib.Mtp); d.h = None
+class A(lib.Attn):
+    def __len__(self): return 5
+a = object.__new__(A); a.h = None
+calls = [lambda: lib.adapt_plan(1, 1.0, z(9), 0.5, 0.0), lambda: g.step(z(3, 1024), z(3, 512), z(3, 4), z(3, 3)), lambda: g.prefill_chunked(z(3, 1024), z(2, 512), z(3, 4), z(3, 4)),
+         lambda: g.prefill_chunked(z(3, 1000), z(3, 512), z(3, 4), z(3, 4)), lambda: a.load_index(z(4, 64)), lambda: m.generate_greedy(None, z(8), 4, 2, np.zeros(11, np.uint32)),
+         lambda: d.generate_greedy_forced(None, z(8), 4, np.zeros(11, np.uint32))]
+for i, c in enumerate(calls):
+    try: c()
+    except ValueError as e:
+        if "expected" in str(e): continue
+    raise SystemExit("call %d was not refused" % i)
+'''
+    r = subprocess.run([sys.executable, "-O", "-c", code], capture_output=True, text=True, timeout=120, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert r.returncode == 0, (r.returncode, r.stderr[-800:])
+
+
 def test_python_binding_declares_every_header_symbol():
     L = C.CDLL(lib.LIB_PATH)
     declared = set(lib._declare(L))
