@@ -15,7 +15,7 @@ PYRE_TS_DECL(moe_ts) PYRE_TS_EXPORT(moe_ts, pyre_debug_ts_moe)
 // -- the lowest index -- from a ballot, that lane retires its key), the waves' candidates meet in shared memory, each
 // candidate counts the candidates that beat it (larger key, or equal key and lower index) and the k that are beaten by
 // fewer than k others are the choice.  Leaves the chosen ids (ascending) in s_idx[0..k) and their logits in s_val[0..k).
-struct RouteLds { float lv[1024]; float r_val[32]; float s_val[32]; int s_idx[32]; float s_w[32]; uint64_t cand[512]; uint64_t win[32]; };
+struct RouteLds { float lv[1024]; float r_val[32]; float s_val[32]; int s_idx[32]; float s_w[32]; uint64_t cand[512 + 96]; uint64_t win[32]; };          // (cand: read in runs of 96)
 #ifdef PYRE_PHASE_TS
 #define ROUTE_TS_PARAM , unsigned long long* rts_
 #define ROUTE_TS_ARG , ts_
@@ -39,7 +39,8 @@ __device__ __forceinline__ uint32_t route_wave_max(uint32_t m) {          // ide
   m = max(m, route_dpp<0x142>(m)); m = max(m, route_dpp<0x143>(m));          // row_bcast 15, 31: lane 63 holds the wave's
   return (uint32_t)__builtin_amdgcn_readlane((int)m, 63);
 }
-// called by the whole workgroup (at least n_exp threads, a multiple of 64), after lv[] is complete
+// called by the whole workgroup of NT threads (at least n_exp, a multiple of 64), after lv[] is complete
+template <int NT>
 __device__ __forceinline__ void route_select(int n_exp, int k, RouteLds& L) {
   const int e = threadIdx.x, lane = e & 63, wave = e >> 6, nwv = (n_exp + 63) >> 6;
   if (wave < nwv) {
@@ -47,7 +48,7 @@ __device__ __forceinline__ void route_select(int n_exp, int k, RouteLds& L) {
     uint32_t ck = 0u, cl = 0u;          // lane r keeps the wave's r-th candidate
     for (int round = 0; round < k; ++round) {
       const uint32_t wm = route_wave_max(key);
-      const int ol = __ffsll((unsigned long long)__ballot(key == wm)) - 1;          // the lowest lane that holds it = the lowest index
+      const int ol = __builtin_ctzll((unsigned long long)__ballot(key == wm));          // the lowest lane that holds it = the lowest index
       ck = lane == round ? wm : ck; cl = lane == round ? (uint32_t)ol : cl;
       key = lane == ol ? 0u : key;
     }
@@ -57,14 +58,15 @@ __device__ __forceinline__ void route_select(int n_exp, int k, RouteLds& L) {
   // eight neighbouring lanes share a candidate and split the others among them; larger 64-bit word = larger key, or the
   // same key at a lower index: a strict order, so the k winners hold the ranks 0 .. k-1
   const int nc = nwv * k, sub = e & 7;
-  for (int i = e >> 3; i < nc; i += (int)(blockDim.x >> 3)) {
+  for (int i = e >> 3; i < nc; i += NT / 8) {
     const uint64_t ci = L.cand[i];
     int beaten = 0;
+    for (int jb = 0; jb < nc; jb += 96) {          // (twelve reads in flight before the first comparison: one round for eight waves' twelve candidates)
+      uint64_t cj[12];
 #pragma unroll
-    for (int jb = 0; jb < 512; jb += 32) if (jb < nc) {          // (uniform branches: with nc known at compile time every read is issued before the first comparison)
-      const int j = jb + sub;
-      const uint64_t c0 = L.cand[min(j, 511)], c1 = L.cand[min(j + 8, 511)], c2 = L.cand[min(j + 16, 511)], c3 = L.cand[min(j + 24, 511)];
-      beaten += ((j < nc && c0 > ci) ? 1 : 0) + ((j + 8 < nc && c1 > ci) ? 1 : 0) + ((j + 16 < nc && c2 > ci) ? 1 : 0) + ((j + 24 < nc && c3 > ci) ? 1 : 0);
+      for (int r = 0; r < 12; ++r) cj[r] = L.cand[jb + sub + 8 * r];
+#pragma unroll
+      for (int r = 0; r < 12; ++r) beaten += (jb + sub + 8 * r < nc && cj[r] > ci) ? 1 : 0;
     }
     beaten += __builtin_amdgcn_mov_dpp(beaten, 0xB1, 0xf, 0xf, true);          // quad_perm [1,0,3,2]
     beaten += __builtin_amdgcn_mov_dpp(beaten, 0x4E, 0xf, 0xf, true);          // quad_perm [2,3,0,1]
@@ -81,27 +83,37 @@ __device__ __forceinline__ void route_select(int n_exp, int k, RouteLds& L) {
   }
 }
 // The logits are given as nsl (<= 64) K-slice sums `sstride` floats apart, added in slice order (nsl == 1: the logits
-// themselves); all slices are fetched before the first add, in groups of eight behind launch-uniform branches.
+// themselves); all slices are fetched before the first add, in groups of eight behind launch-uniform branches.  NT: the threads of the
+// workgroup; NSM: a bound of nsl.
+template <int NT, int NSM = 64>
 __device__ __forceinline__ void route_topk(const float* __restrict__ logits, int nsl, int sstride, int n_exp, int k, RouteLds& L ROUTE_TS_PARAM) {
   const int e = threadIdx.x;
   if (e < n_exp) {
-    float sv[64];
+    float sv[NSM];
 #pragma unroll
-    for (int q = 0; q < 64; ++q) sv[q] = 0.0f;
+    for (int q = 0; q < NSM; ++q) sv[q] = 0.0f;
 #pragma unroll
-    for (int g = 0; g < 8; ++g) if (g * 8 < nsl) {
+    for (int g = 0; g < NSM / 8; ++g) if (g * 8 < nsl) {
 #pragma unroll
       for (int q = 0; q < 8; ++q) sv[g * 8 + q] = (logits + (size_t)min(g * 8 + q, nsl - 1) * sstride)[e];
     }
     float v = sv[0];
 #pragma unroll
-    for (int q = 1; q < 64; ++q) if (q < nsl) v += sv[q];
+    for (int g = 0; g < NSM / 8; ++g) {
+      if (g * 8 + 8 <= nsl) {          // (a whole group carries no predicates)
+#pragma unroll
+        for (int q = g ? 0 : 1; q < 8; ++q) v += sv[g * 8 + q];
+      } else {
+#pragma unroll
+        for (int q = g ? 0 : 1; q < 8; ++q) if (g * 8 + q < nsl) v += sv[g * 8 + q];
+      }
+    }
     if (isnan(v)) v = -INFINITY;      // nan_clean
     L.lv[e] = v;
   }
   ROUTE_TS(5);
   lds_barrier(); ROUTE_TS(6);
-  route_select(n_exp, k, L);
+  route_select<NT>(n_exp, k, L);
   ROUTE_TS(7);
   lds_barrier();
 }
@@ -109,12 +121,22 @@ __device__ __forceinline__ void route_topk(const float* __restrict__ logits, int
 __device__ __forceinline__ void route_weights(int k, RouteLds& L) {
   const int e = threadIdx.x;
   float mx = -INFINITY, ex = 1.0f;
-  if (e < k) { for (int i = 0; i < k; ++i) mx = fmaxf(mx, L.s_val[i]); ex = isfinite(mx) ? expf(L.s_val[e] - mx) : 1.0f; L.r_val[e] = ex; }
+  // the k (<= 32) values in order, eight in flight at a time
+  auto walk = [&](const float (&p)[32], auto&& f) {
+#pragma unroll
+    for (int g = 0; g < 32; g += 8) if (g < k) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = p[g + i];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) if (g + i < k) f(v[i]);
+    } };
+  if (e < k) { walk(L.s_val, [&](float v) { mx = fmaxf(mx, v); }); ex = isfinite(mx) ? expf(L.s_val[e] - mx) : 1.0f; L.r_val[e] = ex; }
   lds_barrier();
   if (e < k) {
     float w;
     if (!isfinite(mx)) w = 1.0f / (float)k;
-    else { float sum = 0.0f; for (int i = 0; i < k; ++i) sum += L.r_val[i]; w = ex / sum; }
+    else { float sum = 0.0f; walk(L.r_val, [&](float v) { sum += v; }); w = ex / sum; }
     L.s_w[e] = w;
   }
 }
@@ -166,7 +188,7 @@ __global__ __launch_bounds__(NW * 64, (PRE && P == 2 && FMT >= 5 && FMT <= 7) ? 
   int expert = 0;
   if (!shared) {
     if constexpr (PRE) expert = __builtin_amdgcn_readfirstlane(sel_idx[ti * top_k + j]);
-    else { route_topk(logits + (size_t)ti * tstride, nsl, sstride, n_exp, top_k, rl ROUTE_TS_ARG); expert = __builtin_amdgcn_readfirstlane(rl.s_idx[j]); }
+    else { route_topk<NW * 64>(logits + (size_t)ti * tstride, nsl, sstride, n_exp, top_k, rl ROUTE_TS_ARG); expert = __builtin_amdgcn_readfirstlane(rl.s_idx[j]); }
   } else if (blockIdx.x == 0) {
     float p = 0.0f;
     for (int ib = threadIdx.x; ib < d; ib += 4 * NW * 64) {          // four elements per pass, loads first (elements past d: weight zero)
@@ -254,17 +276,18 @@ __global__ __launch_bounds__(NW * 64, (PRE && P == 2 && FMT >= 5 && FMT <= 7) ? 
 }
 
 // ---- routing alone (windows of several tokens): grid t, 1024 threads; ids ascending and softmax weights of token ti ------
-// NSL > 0: 512 experts, top 10 and NSL router slices folded in at compile time (checked by the launcher)
-template <int NSL = 0>
+// K > 0: the experts a token (m.top_k) at compile time: the selection's loops are a chain of some forty steps a count (512 experts, top
+// 10, sixteen slices: 4.5 us with the count at run time, 3.8 with it folded).  NSM: a bound of the router slices, whose sums' registers
+// and predicates the compiler lays out for it.
+template <int K, int NSM>
 __global__ __launch_bounds__(1024) void k_moe_route(MoeDev m, const float* __restrict__ logits, int32_t* __restrict__ sel_idx, float* __restrict__ sel_w, int nsl, int sstride, int tstride) {
   __shared__ RouteLds rl;
-  const int ti = blockIdx.x;
-  const int n_exp = NSL ? 512 : m.n_exp, top_k = NSL ? 10 : m.top_k;
-  if constexpr (NSL > 0) nsl = NSL;
+  const int ti = blockIdx.x, n_exp = m.n_exp, top_k = K ? K : m.top_k;
+  args_now(n_exp, top_k, logits, sel_idx, sel_w, nsl, sstride, tstride);
 #ifdef PYRE_PHASE_TS
   unsigned long long ts_[8];
 #endif
-  route_topk(logits + (size_t)ti * tstride, nsl, sstride, n_exp, top_k, rl ROUTE_TS_ARG);
+  route_topk<1024, NSM>(logits + (size_t)ti * tstride, nsl, sstride, n_exp, top_k, rl ROUTE_TS_ARG);
   route_weights(top_k, rl);
   if ((int)threadIdx.x < top_k) { sel_idx[ti * top_k + threadIdx.x] = rl.s_idx[threadIdx.x]; sel_w[ti * top_k + threadIdx.x] = rl.s_w[threadIdx.x]; }
 }
@@ -506,6 +529,13 @@ int pyre_moe_gu_parts(const MoeDev& m) {
   static const bool off = getenv("PYRE_MOE_GU_PARTS") && atoi(getenv("PYRE_MOE_GU_PARTS")) == 0;
   return (!off && m.gate_e.U % 32 == 0 && m.sh_gate.U == m.gate_e.U) ? 2 : 1;
 }
+// every count of experts a token up to PYRE_MOE_KMAX has its instance, larger ones the one with the count at run time
+template <int K = PYRE_MOE_KMAX> static void moe_route_launch(int k, const MoeDev& m, dim3 grid, hipStream_t st, const float* lg, int32_t* sel_idx, float* sel_w, int nsl, int sstride, int tstride) {
+  if constexpr (K > 0) { if (k != K) return moe_route_launch<K - 1>(k, m, grid, st, lg, sel_idx, sel_w, nsl, sstride, tstride); }
+  if (nsl <= 16) hipLaunchKernelGGL((k_moe_route<K, 16>), grid, dim3(1024), 0, st, m, lg, sel_idx, sel_w, nsl, sstride, tstride);
+  else if (nsl <= 32) hipLaunchKernelGGL((k_moe_route<K, 32>), grid, dim3(1024), 0, st, m, lg, sel_idx, sel_w, nsl, sstride, tstride);
+  else hipLaunchKernelGGL((k_moe_route<K, 64>), grid, dim3(1024), 0, st, m, lg, sel_idx, sel_w, nsl, sstride, tstride);
+}
 int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const float* x, int t, float* y, const RouteSrc* routed, bool in_groups) {
   if (in_groups && (y || t < 2 || !pyre_moe_groups_ok(m))) return pyre_fail(ctx, PYRE_E_ARG, "moe_ffn: group sums are for unreduced windows of 2..8 tokens with top_k <= %d", PYRE_MOE_KMAX);
   if (t < 1 || t > 8) return pyre_fail(ctx, PYRE_E_ARG, "moe_ffn: t = %d outside 1..8", t);
@@ -543,10 +573,7 @@ int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const floa
   else if (t == 1) { GU_GO(1, nz, false); }          // the selection inside the launch; one workgroup per K part
   else {
     const bool a3bw = m.gate_e.fmt == FMT_IQ3_S && m.down_e.fmt == FMT_IQ3_S && m.n_exp == 512 && m.top_k == 10 && m.d == 2048 && m.ff == 512 && m.sf == 512;          // a window of the A3B configuration: constants folded in
-    const bool r10 = m.n_exp == 512 && m.top_k == 10;
-    if (r10 && nsl == 32) hipLaunchKernelGGL(k_moe_route<32>, dim3(t), dim3(1024), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, nsl, sstride, tstride);
-    else if (r10 && nsl == 16) hipLaunchKernelGGL(k_moe_route<16>, dim3(t), dim3(1024), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, nsl, sstride, tstride);
-    else hipLaunchKernelGGL(k_moe_route<0>, dim3(t), dim3(1024), 0, ctx->stream, m, lg, w.sel_idx, w.sel_w, nsl, sstride, tstride);
+    moe_route_launch(m.top_k <= PYRE_MOE_KMAX ? m.top_k : 0, m, dim3(t), ctx->stream, lg, w.sel_idx, w.sel_w, nsl, sstride, tstride);
     if (a3bw && P == 2) { if (idot) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, true, true>), GU_ARGS(1)); else hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, true>), GU_ARGS(1)); }
     else if (P == 2) { GU_GO(2, 1, true); } else { GU_GO(1, 1, true); }
   } }
@@ -596,7 +623,7 @@ __global__ __launch_bounds__(1024) void k_moe_route_blk(MoeDev m, MoeBlk b, int 
 #ifdef PYRE_PHASE_TS
   unsigned long long ts_[8];
 #endif
-  route_topk(b.rpart + (size_t)w * b.wr + (size_t)tw * r64, nsl, 8 * r64, n_exp, top_k, rl ROUTE_TS_ARG);
+  route_topk<1024>(b.rpart + (size_t)w * b.wr + (size_t)tw * r64, nsl, 8 * r64, n_exp, top_k, rl ROUTE_TS_ARG);
   route_weights(top_k, rl);
   if ((int)threadIdx.x < top_k) { b.sel_idx[ti * top_k + threadIdx.x] = rl.s_idx[threadIdx.x]; b.sel_w[ti * top_k + threadIdx.x] = rl.s_w[threadIdx.x]; }
 }

@@ -46,6 +46,33 @@ def test_moe_ffn_small(ctx, qtype, t):
     assert relerr(y, yo) <= TOL
 
 
+@pytest.fixture(scope="module")
+def zero_experts(ctx):
+    return lambda n_exp, d: [lib.QMat(ctx, synth.Q4_0, r, c, np.zeros(r * c // 32 * 18, np.uint8)) for r, c in ((n_exp * 64, d), (n_exp * 64, d), (n_exp * d, 64), (64, d), (64, d), (d, 64))]
+
+
+@pytest.mark.parametrize("n_exp,d", [(40, 512), (512, 1024), (1000, 256)])
+def test_moe_route_for_every_count_of_experts_a_token(ctx, zero_experts, n_exp, d):
+    # the selection of a window has its loops laid out for the count and a bound of the router's slices; the choice and its weights
+    # against numpy, every fifth expert with its neighbour's router row: ties go to the lower id
+    g = np.random.Generator(np.random.PCG64(n_exp))
+    R = g.integers(-4, 5, (n_exp, d)).astype(np.float32) / 64; R[4::5] = R[3::5][:len(R[4::5])]
+    bf = (np.ascontiguousarray(R).view(np.uint32) >> 16).astype(np.uint16).view(np.uint8).reshape(-1)
+    router = lib.QMat(ctx, lib.BF16, n_exp, d, bf); ge, ue, de, sg, su, sd = zero_experts(n_exp, d)
+    x = g.integers(-4, 5, (4, d)).astype(np.float32)          # (products and sums of small integers over 64: exact in any order)
+    lg = x.astype(np.float64) @ R.T.astype(np.float64)
+    for top_k in (1, 2, 3, 5, 8, 11, 15, 16, 17, 31, 32):
+        _, idx, w = lib.Moe(ctx, top_k, router, ge, ue, de, np.zeros(d, np.float32), sg, su, sd).ffn(x)
+        check_choice(lg, idx, w, top_k)
+
+
+def check_choice(lg, idx, w, top_k):
+    n_exp = lg.shape[1]
+    for t in range(4):
+        want = np.sort(np.lexsort((np.arange(n_exp), -lg[t]))[:top_k]); e = np.exp(lg[t, want] - lg[t, want].max())
+        assert np.array_equal(idx[t], want) and np.abs(w[t] - e / e.sum()).max() < 1e-6, top_k
+
+
 @pytest.mark.parametrize("qtype,d", [(synth.Q4_K, 2048), (synth.Q8_0, 2048), (synth.IQ2_XS, 2048), (synth.IQ4_NL, 2048), (synth.IQ3_S, 4096)])
 def test_moe_gate_up_in_two_k_parts(ctx, qtype, d):
     # rows of a multiple of 32 units: the gate/up dot products are summed in two K parts -- one workgroup per part for a
