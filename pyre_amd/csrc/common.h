@@ -286,16 +286,17 @@ static_assert(PYRE_MOE_GROUPS == PYRE_GEMV_PARTS, "the mix adds the group sums a
 #ifdef __HIPCC__
 // All loads are issued before the first add, so the value costs one memory round trip, not k + 1.
 // FK > 0: the number of routed experts as a compile-time constant (the caller guarantees mo.k == FK): the loads and the
-// grouping carry no predicates; the arithmetic is the same.
-template <int FK = 0> __device__ __forceinline__ float moe_out_value(const MoeOut& mo, int ti, int r) {
+// grouping carry no predicates; FG > 0: the experts a group, (k + 4) / 4, likewise: the terms of a group are known
+// registers; the arithmetic is the same.
+template <int FK = 0, int FG = 0> __device__ __forceinline__ float moe_out_value(const MoeOut& mo, int ti, int r) {
   const int k = FK ? FK : mo.k;
   const float* p = mo.partial + (size_t)ti * (k + 1) * mo.d + r; const float* w = mo.sel_w + ti * k;
-  constexpr int KM = FK ? FK : PYRE_MOE_KMAX;
+  constexpr int KM = FK ? FK : (FG && 4 * FG < PYRE_MOE_KMAX ? 4 * FG - 1 : PYRE_MOE_KMAX);          // (k <= 4 FG - 1)
   float pv[KM], wv[KM];
 #pragma unroll
   for (int j = 0; j < KM; ++j) { pv[j] = j < k ? p[(size_t)j * mo.d] : 0.0f; wv[j] = j < k ? w[j] : 0.0f; }
   float sh = p[(size_t)k * mo.d], g = mo.sg[ti];
-  const int gsz = (k + 4) / 4;
+  const int gsz = FG ? FG : (k + 4) / 4;
   float P[PYRE_MOE_GROUPS];
 #pragma unroll
   for (int q = 0; q < PYRE_MOE_GROUPS; ++q) {

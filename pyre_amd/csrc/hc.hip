@@ -17,7 +17,7 @@ __device__ __forceinline__ float sigm(float x) { return 1.0f / (1.0f + expf(-x))
 // `out` is a plain [t][d] vector (comb_out) or the unreduced FFN output (mo.partial != nullptr).
 // NP > 1: `out` comes as NP partial vectors, part q of token ti at comb_out + (q*T + ti)*d, added in order from the first
 // (pyre_gemv_parts_launch); all parts are fetched before the first add.
-template <int T, int NP, int FK = 0> __device__ __forceinline__ float hc_x_new(const float* __restrict__ x_in, int in_ss, int in_ts, const float* __restrict__ comb_out, const MoeOut& mo, float w, int d, int ti, int s, int i) {
+template <int T, int NP, int FK = 0, int FG = 0> __device__ __forceinline__ float hc_x_new(const float* __restrict__ x_in, int in_ss, int in_ts, const float* __restrict__ comb_out, const MoeOut& mo, float w, int d, int ti, int s, int i) {
   float v = x_in[(size_t)ti * in_ts + (size_t)s * in_ss + i];
   if constexpr (NP > 1) {
     float sv[NP];
@@ -28,65 +28,111 @@ template <int T, int NP, int FK = 0> __device__ __forceinline__ float hc_x_new(c
     for (int q = 1; q < NP; ++q) o += sv[q];
     v = v + o * w;
   } else {
-    if (mo.partial) v = v + moe_out_value<FK>(mo, ti, i) * w;
+    if (mo.partial) v = v + moe_out_value<FK, FG>(mo, ti, i) * w;
     else if (comb_out) v = v + comb_out[(size_t)ti * d + i] * w;
   }
   return v;
 }
 
+// x / n for 0 <= x < 2^16, n <= 2^12 with r = 1 / n within two units in the last place: (x + 1/2) / n lies 1 / (2 n) or more off an
+// integer, the product's error is below x / n * 2^-21
+__device__ __forceinline__ int hc_div(int x, float r) { return (int)(((float)x + 0.5f) * r); }
+__device__ __forceinline__ float hc_recip(int n) { return __builtin_amdgcn_rcpf((float)n); }
+// v / hc; a power of two by multiplication, the same bits
+__device__ __forceinline__ float hc_mean(float v, int hc) { return (hc & (hc - 1)) == 0 ? v * __uint_as_float((uint32_t)(127 - (31 - __builtin_clz(hc))) << 23) : v / (float)hc; }
+
 // The slices of one output row, all loads in flight together: groups of eight behind a branch the whole launch agrees on
 // (ksplit is a kernel argument), so that unused groups cost neither loads nor instruction fetch; inside a group slices
 // past ksplit repeat the last one and are never added.  `want` is the thread's own condition (one execution mask).
-__device__ __forceinline__ void hc_load_run(float (&sv)[32], const float* __restrict__ p, int n, int stride) {      // n (<= 32) values at p, p + stride, ..
+template <int KSM> __device__ __forceinline__ void hc_load_run(float (&sv)[KSM], const float* __restrict__ p, int n, int stride) {      // n (<= KSM) values at p, p + stride, ..
 #pragma unroll
-  for (int k = 0; k < 32; ++k) sv[k] = 0.0f;
+  for (int k = 0; k < KSM; ++k) sv[k] = 0.0f;
 #pragma unroll
-  for (int g = 0; g < 8; ++g) if (g * 4 < n) {
+  for (int g = 0; g < KSM / 4; ++g) if (g * 4 < n) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) sv[g * 4 + j] = p[(size_t)min(g * 4 + j, n - 1) * stride];
   }
 }
-template <int T> __device__ __forceinline__ void hc_load_slices(float (&pv)[32], const float* __restrict__ part, bool want, int ksplit, int t, int r64, int i) {
+template <int T, int KSM> __device__ __forceinline__ void hc_load_slices(float (&pv)[KSM], const float* __restrict__ part, bool want, int ksplit, int t, int r64, int i) {
 #pragma unroll
-  for (int ks = 0; ks < 32; ++ks) pv[ks] = 0.0f;
+  for (int ks = 0; ks < KSM; ++ks) pv[ks] = 0.0f;
   const unsigned off = (unsigned)(t * r64 + i);
   if (want) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) if (g * 8 < ksplit) {
+    for (int g = 0; g < KSM / 8; ++g) if (g * 8 < ksplit) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) pv[g * 8 + j] = (part + (size_t)min(g * 8 + j, ksplit - 1) * T * r64)[off];      // launch-uniform base + the thread's 32-bit offset
     }
   }
 }
 
-// grid (row tiles of [down ; inject], K slices), nw waves.  A workgroup owns L = nw*upw*64 columns of one stream s.
+// the slices of one row in order, each times its stream's scale (sls: at least KSM floats); whole groups of four carry no predicates
+template <int KSM> __device__ __forceinline__ float hc_slice_sum(const float (&pv)[KSM], const float* sls, int ksplit) {
+  float o = 0.0f;
+#pragma unroll
+  for (int g = 0; g < KSM; g += 4) if (g < ksplit) {
+    float sc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sc[j] = sls[g + j];
+    if (g + 4 <= ksplit) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) { const float tm = pv[g + j] * sc[j]; o = g + j == 0 ? tm : o + tm; }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 3; ++j) if (g + j < ksplit) { const float tm = pv[g + j] * sc[j]; o = g + j == 0 ? tm : o + tm; }
+    }
+  }
+  return o;
+}
+// the gate logit: U (<= 16) sums `stride` floats apart in order, four in flight at a time
+__device__ __forceinline__ float hc_unit_sum(const float* red, int U, int stride) {
+  float g = red[0];
+#pragma unroll
+  for (int k = 1; k < 16; k += 3) if (k < U) {
+    float v[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) v[j] = red[min(k + j, U - 1) * stride];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) if (k + j < U) g += v[j];
+  }
+  return g;
+}
+
+// grid (row tiles of [down ; inject], K slices of a stream, streams x groups of tokens), nw waves.  A workgroup owns L = nw*upw*64 columns
+// of one stream s.
 // The RMS scale of a stream multiplies every term of a row's dot product, so it is applied after the dot (by
 // k_hc_up_mix, which also sums the slices): a workgroup never needs the sum of squares of the whole stream.
 //   1. its L columns of x_new (the pending residual update applied) times the norm weight go to shared memory; the
 //      squares of x_new are summed over the slice -> ssq[ks*T + t]; the tile-0 workgroup of the slice also publishes the
 //      updated stream (x_out, never the buffer x_in points into)
 //   2. each wave takes upw units of the slice; partial sums -> part[(ks*T + t)*tiles*64 + row]
-// FD, FK > 0: the model width (and eight waves of one unit each) and the routed experts per token as compile-time constants, as k_hc_norm_down_m.
-template <int FMT, int T, int NP, int FD = 0, int FK = 0> __global__ __launch_bounds__(512) void k_hc_norm_down(QMatDev m, const float* __restrict__ x_in, int in_ss, int in_ts, float* __restrict__ x_out,
-    const float* __restrict__ comb_out, MoeOut mo_in, const float* __restrict__ comb_inj, const float* __restrict__ norm, int d, int hc, float* __restrict__ ssq,
+// ONE: eight waves of one unit each (every width in multiples of 512 with at most 32 slices): a thread prepares one column and a wave
+// forms one unit's sums, without loops.  FG > 0: the experts a group of the unreduced FFN output (moe_out_value).  One token, bf16,
+// 2048 columns, 6.1 us with the loops and the groups at run time, 5.0 with neither; 500 tokens' groups of eight 218 and 113 us.
+template <int FMT, int T, int NP, bool ONE = false, int FG = 0> __global__ __launch_bounds__(512) void k_hc_norm_down(QMatDev m, const float* __restrict__ x_in, int in_ss, int in_ts, float* __restrict__ x_out,
+    const float* __restrict__ comb_out, MoeOut mo, const float* __restrict__ comb_inj, const float* __restrict__ norm, int d, int hc, float* __restrict__ ssq,
     float* __restrict__ part, int upw, const uint2* __restrict__ g2) {
-  const size_t zt = (size_t)blockIdx.z * T;          // a further group of T tokens (pyre_hc_mix_rows_launch)
-  const MoeOut mo{mo_in.partial ? mo_in.partial + zt * (mo_in.k + 1) * mo_in.d : nullptr, mo_in.sel_w + zt * mo_in.k, mo_in.sg + zt, mo_in.d, mo_in.k};
-  x_in += zt * in_ts; x_out += zt * hc * d; ssq += zt * gridDim.y; part += zt * gridDim.y * ((size_t)m.tiles * 64);
-  if (comb_out) comb_out += zt * d;
-  if (comb_inj) comb_inj += zt * hc;
+  int s = blockIdx.z;
+  if (s >= hc) {          // a further group of T tokens (pyre_hc_mix_rows_launch)
+    const int grp = s / hc, ksplit = gridDim.y * hc; s -= grp * hc;
+    const size_t zt = (size_t)grp * T;
+    if (mo.partial) { mo.partial += zt * (mo.k + 1) * mo.d; mo.sel_w += zt * mo.k; mo.sg += zt; }
+    x_in += zt * in_ts; x_out += zt * hc * d; ssq += zt * ksplit; part += zt * ksplit * ((size_t)m.tiles * 64);
+    if (comb_out) comb_out += zt * d;
+    if (comb_inj) comb_inj += zt * hc;
+  }
   const uint2* lds2 = nullptr;          // no format needs a codebook in shared memory any more
   PYRE_TS_VARS PYRE_TS(0);
   qmat_args_now(m); args_now(x_in, in_ss, in_ts, x_out, comb_out, mo.partial, mo.sel_w, mo.sg, mo.d, mo.k, comb_inj, norm, d, hc, ssq, part, upw);
-  if constexpr (FD > 0) { d = FD; upw = 1; }
+  if constexpr (ONE) upw = 1;
   extern __shared__ __align__(16) float sm[];
-  const int nthr = FD > 0 ? 512 : blockDim.x, nw = nthr >> 6, tid = threadIdx.x, L = nw * upw * 64;
+  const int nthr = ONE ? 512 : blockDim.x, nw = nthr >> 6, tid = threadIdx.x, L = nw * upw * 64;
   float* xs = sm;                         // [T][L]
   float* red = sm + (size_t)T * L;        // [nw][T][64]
   float* wsum = red + (size_t)nw * T * 64;   // [nw][T]
-  const int tile = blockIdx.x, ks = blockIdx.y;
+  const int tile = blockIdx.x, ks = s * gridDim.y + blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int c0 = ks * L, s = c0 / d, i0 = c0 - s * d;
+  const int i0 = blockIdx.y * L;
   // Loads return in the order they were issued: the streams (and the pending update's terms) first, since the copy into
   // shared memory waits for them, then the first unit's weights, which stay in flight across the barrier.
   float w[T], ss[T];
@@ -96,7 +142,7 @@ template <int FMT, int T, int NP, int FD = 0, int FK = 0> __global__ __launch_bo
   if (tid < L) {
     nv0 = norm[(size_t)s * d + i0 + tid];
 #pragma unroll
-    for (int t = 0; t < T; ++t) v0[t] = hc_x_new<T, NP, FK>(x_in, in_ss, in_ts, comb_out, mo, w[t], d, t, s, i0 + tid);
+    for (int t = 0; t < T; ++t) v0[t] = hc_x_new<T, NP, 0, FG>(x_in, in_ss, in_ts, comb_out, mo, w[t], d, t, s, i0 + tid);
   }
   UnitRaw<FMT> raw = unit_load<FMT>(m, tile, ks * nw * upw + wave * upw, lane);
   if (tid < L) {
@@ -108,11 +154,11 @@ template <int FMT, int T, int NP, int FD = 0, int FK = 0> __global__ __launch_bo
       if (tile == 0) x_out[((size_t)t * hc + s) * d + i0 + tid] = v;
     }
   }
-  for (int j = tid + nthr; j < L; j += nthr) {
+  if constexpr (!ONE) for (int j = tid + nthr; j < L; j += nthr) {
     const float nv = norm[(size_t)s * d + i0 + j];
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      float v = hc_x_new<T, NP, FK>(x_in, in_ss, in_ts, comb_out, mo, w[t], d, t, s, i0 + j);
+      float v = hc_x_new<T, NP>(x_in, in_ss, in_ts, comb_out, mo, w[t], d, t, s, i0 + j);
       ss[t] += v * v;
       xs[(size_t)t * L + j] = v * nv;
       if (tile == 0) x_out[((size_t)t * hc + s) * d + i0 + j] = v;
@@ -152,12 +198,13 @@ template <int FMT, int T, int NP, int FD = 0, int FK = 0> __global__ __launch_bo
 // from zero (:1380).
 // RF >= 0: the launch also leaves its K slice of the router GEMV over the mixed vector (format RF; HcRoute): wave w
 // takes router tile w, w + nw, .. at unit blockIdx.x, the first tile's weights fetched ahead of the up GEMV.
-// FHC, FLR, FKS > 0: the stream count, the low rank and the slice count as compile-time constants (the launcher checks them).
-template <int FMT, int T, int RF, int FHC = 0, int FLR = 0, int FKS = 0> __global__ __launch_bounds__(1024) void k_hc_up_mix(QMatDev up, const float* __restrict__ part, const float* __restrict__ ssq, int ksplit, int r64, int lr, int hc, int has_inject,
+// KSM, HM: bounds of the slice and stream counts, which size the straight code (the launcher takes the smallest that holds the mix).
+// FLR > 0: a low rank of FLR and exactly KSM slices, at compile time.
+template <int FMT, int T, int RF, int KSM, int HM, int FLR = 0> __global__ __launch_bounds__(1024) void k_hc_up_mix(QMatDev up, const float* __restrict__ part, const float* __restrict__ ssq, int ksplit, int r64, int lr, int hc, int has_inject,
     const float* __restrict__ xnew, const float* __restrict__ norm, float eps, int d, float* __restrict__ mixed, float* __restrict__ inj, const uint2* __restrict__ g2,
     QMatDev router, float* __restrict__ rpart) {
   constexpr bool ROUTE = RF >= 0; constexpr int RFX = ROUTE ? RF : FMT_F32;
-  if constexpr (FHC > 0) { hc = FHC; lr = FLR; ksplit = FKS; }
+  if constexpr (FLR > 0) { lr = FLR; ksplit = KSM; }
   if (blockIdx.z) {          // a further group of T tokens (pyre_hc_mix_rows_launch)
     const size_t z = blockIdx.z; part += z * ksplit * T * r64; ssq += z * ksplit * T; xnew += z * T * hc * d; mixed += z * T * d; inj += z * T * hc;
     if (ROUTE) rpart += z * (d / 64) * T * router.tiles * 64;
@@ -167,53 +214,65 @@ template <int FMT, int T, int RF, int FHC = 0, int FLR = 0, int FKS = 0> __globa
   qmat_args_now(up); args_now(part, ssq, ksplit, r64, lr, hc, has_inject, xnew, norm, eps, d, mixed, inj);
 
   extern __shared__ __align__(16) float sm[];
-  const int nthr = FHC > 0 ? FHC * FLR : blockDim.x, tid = threadIdx.x, U = lr >> 6, kps = ksplit / hc, nw = nthr >> 6;
+  const int tid = threadIdx.x, U = lr >> 6, nthr = hc * lr, nw = hc * U;
+  const float rhc = hc_recip(hc); const int kps = __builtin_amdgcn_readfirstlane(hc_div(ksplit, rhc));
   float* lo = sm;                         // [T][lr]
   float* red = sm + (size_t)T * lr;       // [nw][T][64]
   float* sls = red + (size_t)nw * T * 64;   // [T][32]: the RMS scale of the stream each slice belongs to
   float* term = sls + (size_t)T * 32;     // [T*hc][64]: the streams' gated, normalized values before they are added
-  const int n_o = lr + hc;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int s = wave / U, ku = wave - s * U;
+  const int s = __builtin_amdgcn_readfirstlane(hc_div(wave, hc_recip(U))), ku = wave - s * U;
   // Loads return in the order they were issued, so they are issued in the order they are needed: the slice sums of
   // squares and of [down ; inject] first (the prologue waits for nothing else), then the up weights, the epilogue's
   // operands and the router tile, all of which stay in flight across the barriers below (which exchange through shared
   // memory only).
-  float ssv[32];
+  float ssv[KSM];
 #pragma unroll
-  for (int k = 0; k < 32; ++k) ssv[k] = 0.0f;
-  const int stt = tid / hc, sq = tid - stt * hc;
-  if (tid < T * hc) hc_load_run(ssv, ssq + (size_t)(sq * kps) * T + stt, kps, T);          // all of the stream's slices before the first add: one round trip
-  float pv[32]; int idx = tid; int t = idx / n_o, i = idx - t * n_o;
-  bool have = idx < T * n_o;
-  hc_load_slices<T>(pv, part, have && (i < lr || has_inject), ksplit, t, r64, i);
-  UnitRaw<FMT> raw = unit_load<FMT>(up, s * (d >> 6) + blockIdx.x, ku, lane);
+  for (int k = 0; k < KSM; ++k) ssv[k] = 0.0f;
+  const int stt = hc_div(tid, rhc), sq = tid - stt * hc;
+  if (tid < T * hc) hc_load_run<KSM>(ssv, ssq + (size_t)(sq * kps) * T + stt, kps, T);          // all of the stream's slices before the first add: one round trip
+  // the slices of rows of lo, with few slices two rounds of a row a thread ahead (T / hc rounds)
+  constexpr bool AHEAD = KSM <= 16 && T > 1;
+  const float rlr = hc_recip(lr); const int n_lo = T * lr;
+  float pv[KSM], pn[AHEAD ? KSM : 1];
+  auto slices = [&](float (&v)[KSM], int idx) { const int t = hc_div(idx, rlr); hc_load_slices<T, KSM>(v, part, idx < n_lo, ksplit, t, r64, idx - t * lr); };
+  slices(pv, tid);
+  if constexpr (AHEAD) { if (n_lo > nthr) slices(pn, tid + nthr); }
+  constexpr bool U_EARLY = FMT != FMT_F32 || T == 1;      // an f32 unit is 64 registers: with several tokens' it waits for the slice sums'
+  UnitRaw<FMT> raw;
+  if constexpr (U_EARLY) raw = unit_load<FMT>(up, s * (d >> 6) + blockIdx.x, ku, lane);
   // the epilogue's stream value and norm weight of this wave's first (token, stream) item
   float xpre = 0.0f, npre = 0.0f;
-  if (wave < T * hc) { const int t0 = wave / hc, q0 = wave - t0 * hc; xpre = (xnew + ((size_t)t0 * hc + q0) * d + blockIdx.x * 64)[lane]; npre = (norm + (size_t)q0 * d + blockIdx.x * 64)[lane]; }
+  if (wave < T * hc) { const int t0 = __builtin_amdgcn_readfirstlane(hc_div(wave, rhc)), q0 = wave - t0 * hc; xpre = (xnew + ((size_t)t0 * hc + q0) * d + blockIdx.x * 64)[lane]; npre = (norm + (size_t)q0 * d + blockIdx.x * 64)[lane]; }
   UnitRaw<RFX> rraw;
-  constexpr bool R_EARLY = RFX != FMT_F32;      // an f32 tile is 64 registers: fetched once the up GEMV has freed them
+  constexpr bool R_EARLY = RFX != FMT_F32 && U_EARLY && (T == 1 || KSM <= 16);      // an f32 tile is 64 registers: fetched once the up GEMV has freed them, and so are others beside too many of its own or of slices
   if (ROUTE && R_EARLY && wave < router.tiles) rraw = unit_load<RFX>(router, wave, blockIdx.x, lane);
   if (tid < T * hc) {
     float tot = ssv[0];
 #pragma unroll
-    for (int k = 1; k < 32; ++k) if (k < kps) tot += ssv[k];
+    for (int k = 1; k < KSM; ++k) if (k < kps) tot += ssv[k];
     const float sc = 1.0f / sqrtf(tot / (float)d + eps);
     for (int k = 0; k < kps; ++k) sls[stt * 32 + sq * kps + k] = sc;
   }
   lds_barrier(); PYRE_TS(1);
-  while (have) {
-    float o = 0.0f;                 // slices in order, each times its stream's scale
-    if (i < lr || has_inject) {
+  for (int i0 = 0; i0 < n_lo; i0 += nthr) {          // (a launch-uniform count of rounds)
+    const int idx = i0 + tid, t = min(hc_div(idx, rlr), T - 1);
+    const float v = hc_mean(hc_slice_sum<KSM>(pv, sls + t * 32, ksplit), hc);          // slices in order, each times its stream's scale
+    if (idx < n_lo) lo[idx] = v * sigm(v);
+    if (i0 + nthr < n_lo) {
+      if constexpr (AHEAD) {
 #pragma unroll
-      for (int ks = 0; ks < 32; ++ks) if (ks < ksplit) { const float tm = pv[ks] * sls[t * 32 + ks]; o = ks == 0 ? tm : o + tm; }
+        for (int k = 0; k < KSM; ++k) pv[k] = pn[k];
+        if (i0 + 2 * nthr < n_lo) slices(pn, idx + 2 * nthr);
+      } else slices(pv, idx + nthr);
     }
-    const float v = o / (float)hc;
-    if (i < lr) lo[t * lr + i] = v * sigm(v);
-    else if (blockIdx.x == 0) inj[t * hc + (i - lr)] = has_inject ? v : 0.0f;
-    idx += nthr; have = idx < T * n_o;
-    if (have) { t = idx / n_o; i = idx - t * n_o; hc_load_slices<T>(pv, part, i < lr || has_inject, ksplit, t, r64, i); }
   }
+  if (blockIdx.x == 0 && tid < T * hc) {          // one workgroup leaves the inject rows
+    float v = 0.0f;
+    if (has_inject) { hc_load_slices<T, KSM>(pv, part, true, ksplit, stt, r64, lr + sq); v = hc_mean(hc_slice_sum<KSM>(pv, sls + stt * 32, ksplit), hc); }
+    inj[stt * hc + sq] = v;
+  }
+  if constexpr (!U_EARLY) raw = unit_load<FMT>(up, s * (d >> 6) + blockIdx.x, ku, lane);
   lds_barrier(); PYRE_TS(2);
   float acc[T];
 #pragma unroll
@@ -226,9 +285,8 @@ template <int FMT, int T, int RF, int FHC = 0, int FLR = 0, int FKS = 0> __globa
   lds_barrier(); PYRE_TS(4);
   // one wave per (token, stream): the gate logit is the sum of the stream's waves in unit order; xn * sigm(gate) -> term
   for (int w = wave; w < T * hc; w += nw) {
-    const int t2 = w / hc, q = w - t2 * hc, col = blockIdx.x * 64 + lane;
-    float g = red[((size_t)(q * U) * T + t2) * 64 + lane];
-    for (int k = 1; k < U; ++k) g += red[((size_t)(q * U + k) * T + t2) * 64 + lane];
+    const int t2 = __builtin_amdgcn_readfirstlane(hc_div(w, rhc)), q = w - t2 * hc, col = blockIdx.x * 64 + lane;
+    const float g = hc_unit_sum(red + ((size_t)(q * U) * T + t2) * 64 + lane, U, T * 64);
     const float xv = w == wave ? xpre : xnew[((size_t)t2 * hc + q) * d + col];
     const float nv = w == wave ? npre : norm[(size_t)q * d + col];
     term[(size_t)w * 64 + lane] = xv * sls[t2 * 32 + q * kps] * nv * sigm(g);            // rms, :209: (x * s) * w
@@ -237,8 +295,8 @@ template <int FMT, int T, int RF, int FHC = 0, int FLR = 0, int FKS = 0> __globa
   for (int i2 = tid; i2 < T * 64; i2 += nthr) {
     const int t2 = i2 >> 6, l = i2 & 63, col = blockIdx.x * 64 + l; float mx = 0.0f;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) if (q < hc) mx += term[(size_t)(t2 * hc + q) * 64 + l];          // streams ascending from zero (:1380)
-    const float mv = mx / (float)hc;
+    for (int q = 0; q < HM; ++q) if (q < hc) mx += term[(size_t)(t2 * hc + q) * 64 + l];          // streams ascending from zero (:1380)
+    const float mv = hc_mean(mx, hc);
     mixed[(size_t)t2 * d + col] = mv;
     if (ROUTE) lo[t2 * 64 + l] = mv;          // lo is free after the barrier above
   }
@@ -261,71 +319,56 @@ template <int FMT, int T, int RF, int FHC = 0, int FLR = 0, int FKS = 0> __globa
 
 // The same launch for a window alone (at most eight tokens) and the formats of up_by_columns: grid (d / 16), sixteen columns a workgroup, a lane a (stream, unit, column)
 // item of the up GEMV and TS sets of them sharing the tokens (set k: tokens k, k + TS, ..), on d / 16 compute units instead of d / 64; the
-// router is a launch of its own behind it.  The launch is latency, and half of that was fetching instructions: 18 KB of straight code
-// with run-time stream and slice counts, 6 KB with them folded in (FHC, FLR, FKS; the launcher checks them).  A3B shape, bf16, one token:
-// 8.2 us as k_hc_up_mix (13.9 with the router, and 2.5 for the digits behind it), 8.4 here with run-time counts, 6.8 with the folded ones
-// (and 3.2 for router and digits).  A lane's terms, and every order of adding, are those of k_hc_up_mix, bit for bit.  A unit's row of lo
+// router is a launch of its own behind it.  The launch is latency, and half of that was fetching instructions and dividing: with room for
+// 32 slices and eight streams it is 18 KB of straight code, with room for sixteen and four (KSM, HM, as k_hc_up_mix) 10 KB, indices by
+// hc_div, whole groups of slices without predicates.  A3B shape, bf16, one token: 8.2 us as k_hc_up_mix (13.9 with the router, and 2.5
+// for the digits behind it), 8.4 here with the larger code, 6.9 with the smaller (and 3.2 for router and digits).  A lane's terms, and every order of adding, are those of k_hc_up_mix, bit for bit.  A unit's row of lo
 // is PAD floats behind the last one: the four units of a wave read four different banks.
 #define PYRE_UP_PAD 68
-template <int FMT, int T, int FHC = 0, int FLR = 0, int FKS = 0> __global__ __launch_bounds__(512) void k_hc_up_mix_c(QMatDev up, const float* __restrict__ part, const float* __restrict__ ssq, int ksplit, int r64, int lr, int hc, int has_inject,
+template <int FMT, int T, int KSM, int HM> __global__ __launch_bounds__(512) void k_hc_up_mix_c(QMatDev up, const float* __restrict__ part, const float* __restrict__ ssq, int ksplit, int r64, int lr, int hc, int has_inject,
     const float* __restrict__ xnew, const float* __restrict__ norm, float eps, int d, float* __restrict__ mixed, float* __restrict__ inj) {
-  constexpr int TS = T > 1 ? 2 : 1, TT = (T + TS - 1) / TS, KS = FKS > 0 ? FKS : 32, QS = FHC > 0 ? FHC : 8;
+  constexpr int TS = T > 1 ? 2 : 1, TT = (T + TS - 1) / TS;
   const uint2* lds2 = nullptr;
   qmat_args_now(up); args_now(part, ssq, ksplit, r64, lr, hc, has_inject, xnew, norm, eps, d, mixed, inj);
-  if constexpr (FHC > 0) { hc = FHC; lr = FLR; ksplit = FKS; }
   extern __shared__ __align__(16) float sm[];
-  const int nthr = blockDim.x, tid = threadIdx.x, U = lr >> 6, kps = ksplit / hc, items = hc * U * 16;
+  const int nthr = blockDim.x, tid = threadIdx.x, U = lr >> 6, items = hc * U * 16;
+  const float rhc = hc_recip(hc), rlr = hc_recip(lr); const int kps = __builtin_amdgcn_readfirstlane(hc_div(ksplit, rhc));
   float* lo = sm;                                          // [T][U][PAD]
   float* red = lo + (size_t)T * U * PYRE_UP_PAD;           // [hc * U][T][16]
   float* sls = red + (size_t)hc * U * T * 16;              // [T][32]: the RMS scale of the stream each slice belongs to
-  const int ts = tid / items, it = tid - ts * items, su = it >> 4, r = it & 15, s = su / U, ku = su - s * U, col0 = blockIdx.x * 16;
+  const int ts = tid >= items ? (tid >= 2 * items ? 2 : 1) : 0, it = ts < TS ? tid - ts * items : 0, su = it >> 4, r = it & 15, s = hc_div(su, hc_recip(U)), ku = su - s * U, col0 = blockIdx.x * 16;
   const bool work = ts < TS;
-  float ssv[32];
-  const int stt = tid / hc, sq = tid - stt * hc;
+  float ssv[KSM];
+  const int stt = hc_div(tid, rhc), sq = tid - stt * hc;
   const bool own = tid < T * hc;                           // thread (token stt, stream sq): the stream's scale, and in the first workgroup its inject row
-  if constexpr (FKS > 0) {
 #pragma unroll
-    for (int k = 0; k < FKS / FHC; ++k) ssv[k] = own ? (ssq + (size_t)(sq * kps) * T + stt)[k * T] : 0.0f;
-  } else {
-#pragma unroll
-    for (int k = 0; k < 32; ++k) ssv[k] = 0.0f;
-    if (own) hc_load_run(ssv, ssq + (size_t)(sq * kps) * T + stt, kps, T);
-  }
-  auto slices = [&](float (&v)[32], bool want, int tk, int row) {
-    if constexpr (FKS > 0) {
-#pragma unroll
-      for (int ks = 0; ks < FKS; ++ks) v[ks] = want ? (part + (size_t)ks * T * r64)[(unsigned)(tk * r64 + row)] : 0.0f;
-    } else hc_load_slices<T>(v, part, want, ksplit, tk, r64, row); };
-  float pv[32], pvi[32];
-  int idx = tid, t = idx / lr, i = idx - t * lr;
-  slices(pv, idx < T * lr, t, i);
-  slices(pvi, own && has_inject && blockIdx.x == 0, stt, lr + sq);
+  for (int k = 0; k < KSM; ++k) ssv[k] = 0.0f;
+  if (own) hc_load_run<KSM>(ssv, ssq + (size_t)(sq * kps) * T + stt, kps, T);
+  float pv[KSM], pvi[KSM];
+  int idx = tid, t = hc_div(idx, rlr), i = idx - t * lr;
+  hc_load_slices<T, KSM>(pv, part, idx < T * lr, ksplit, t, r64, i);
+  hc_load_slices<T, KSM>(pvi, part, own && has_inject && blockIdx.x == 0, ksplit, stt, r64, lr + sq);
   const UnitRaw<FMT> raw = unit_load<FMT>(up, s * (d >> 6) + (col0 >> 6), work ? ku : 0, (col0 & 63) + r);
   // the epilogue's operands: thread (token tid / 16, column tid % 16) adds the streams of its column
-  float xpre[QS], npre[QS];
+  float xpre[HM], npre[HM];
   const int et = tid >> 4, el = tid & 15;
 #pragma unroll
-  for (int q = 0; q < QS; ++q) if (tid < T * 16 && q < hc) { xpre[q] = xnew[((size_t)et * hc + q) * d + col0 + el]; npre[q] = norm[(size_t)q * d + col0 + el]; } else { xpre[q] = 0.0f; npre[q] = 0.0f; }
+  for (int q = 0; q < HM; ++q) if (tid < T * 16 && q < hc) { xpre[q] = xnew[((size_t)et * hc + q) * d + col0 + el]; npre[q] = norm[(size_t)q * d + col0 + el]; } else { xpre[q] = 0.0f; npre[q] = 0.0f; }
   if (own) {
     float tot = ssv[0];
 #pragma unroll
-    for (int k = 1; k < (FKS > 0 ? FKS / FHC : 32); ++k) if (k < kps) tot += ssv[k];
+    for (int k = 1; k < KSM; ++k) if (k < kps) tot += ssv[k];
     const float sc = 1.0f / sqrtf(tot / (float)d + eps);
     for (int k = 0; k < kps; ++k) sls[stt * 32 + sq * kps + k] = sc;
   }
   lds_barrier();
-  auto slice_sum = [&](const float (&v)[32], int tk) {      // slices in order, each times its stream's scale
-    float o = 0.0f;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) if (ks < ksplit) { const float tm = v[ks] * sls[tk * 32 + ks]; o = ks == 0 ? tm : o + tm; }
-    return o; };
   while (idx < T * lr) {
-    const float v = slice_sum(pv, t) / (float)hc;
+    const float v = hc_mean(hc_slice_sum<KSM>(pv, sls + t * 32, ksplit), hc);
     lo[((size_t)t * U + (i >> 6)) * PYRE_UP_PAD + (i & 63)] = v * sigm(v);
     idx += nthr;
-    if (idx < T * lr) { t = idx / lr; i = idx - t * lr; slices(pv, true, t, i); }
+    if (idx < T * lr) { t = hc_div(idx, rlr); i = idx - t * lr; hc_load_slices<T, KSM>(pv, part, true, ksplit, t, r64, i); }
   }
-  if (own && blockIdx.x == 0) inj[stt * hc + sq] = has_inject ? slice_sum(pvi, stt) / (float)hc : 0.0f;
+  if (own && blockIdx.x == 0) inj[stt * hc + sq] = has_inject ? hc_mean(hc_slice_sum<KSM>(pvi, sls + stt * 32, ksplit), hc) : 0.0f;
   lds_barrier();
   if (work) {
     float acc[TT];
@@ -348,12 +391,11 @@ template <int FMT, int T, int FHC = 0, int FLR = 0, int FKS = 0> __global__ __la
   if (tid < T * 16) {
     float mx = 0.0f;
 #pragma unroll
-    for (int q = 0; q < QS; ++q) if (q < hc) {          // streams ascending from zero (:1380)
-      float g = red[((size_t)(q * U) * T + et) * 16 + el];
-      for (int k = 1; k < U; ++k) g += red[((size_t)(q * U + k) * T + et) * 16 + el];
+    for (int q = 0; q < HM; ++q) if (q < hc) {          // streams ascending from zero (:1380)
+      const float g = hc_unit_sum(red + ((size_t)(q * U) * T + et) * 16 + el, U, T * 16);
       mx += xpre[q] * sls[et * 32 + q * kps] * npre[q] * sigm(g);            // rms, :209: (x * s) * w
     }
-    mixed[(size_t)et * d + col0 + el] = mx / (float)hc;
+    mixed[(size_t)et * d + col0 + el] = hc_mean(mx, hc);
   }
 }
 
@@ -640,18 +682,23 @@ template <int FMT, int T> int norm_down_launch(pyre_ctx* ctx, const HcDev& h, co
                                                const float* comb_out, int comb_parts, const MoeOut& mo, const float* comb_inj, float eps, int nz = 1) {
   const int L = p.nw * p.upw * 64; size_t lds = 4 * ((size_t)T * L + (size_t)p.nw * T * 64 + (size_t)p.nw * T);
   ProfScope ps(ctx, "hc_norm_down", qmat_gguf_bytes(h.di, h.di.rows) + 4.0 * T * h.hc * h.d * 4);
-#define NORM_DOWN_GO(NP) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, NP>), dim3(h.di.tiles, p.ksplit, nz), dim3(p.nw * 64), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
+#define NORM_DOWN_GO(NP) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, NP>), dim3(h.di.tiles, p.ksplit / h.hc, nz * h.hc), dim3(p.nw * 64), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
                      w.ssq, w.o, p.upw, (const uint2*)ctx->d_iq2xs)
-#define NORM_DOWN_FIX hipLaunchKernelGGL((k_hc_norm_down<FMT, T, 1, 2048, 10>), dim3(h.di.tiles, p.ksplit, nz), dim3(512), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
+#define NORM_DOWN_ONE(FG) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, 1, true, FG>), dim3(h.di.tiles, p.ksplit / h.hc, nz * h.hc), dim3(512), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
                      w.ssq, w.o, p.upw, (const uint2*)ctx->d_iq2xs)
   if constexpr (FMT == FMT_IQ3_S) { if (comb_parts > 1) NORM_DOWN_GO(PYRE_GEMV_PARTS); else NORM_DOWN_GO(1); }
-  else if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {          // the A3B width as files store it: constants folded in (6.1 -> 5.0 us a token)
-    if (h.d == 2048 && p.nw == 8 && p.upw == 1 && (!mo.partial || mo.k == 10)) NORM_DOWN_FIX; else NORM_DOWN_GO(1);
-  } else NORM_DOWN_GO(1);
-#undef NORM_DOWN_FIX
+  else if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {
+    if (p.nw != 8 || p.upw != 1) NORM_DOWN_GO(1);
+    else if constexpr (T == 1) { switch (mo.partial ? (mo.k + 4) / 4 : 0) { case 1: NORM_DOWN_ONE(1); break; case 2: NORM_DOWN_ONE(2); break; case 3: NORM_DOWN_ONE(3); break; case 4: NORM_DOWN_ONE(4); break; case 5: NORM_DOWN_ONE(5); break; default: NORM_DOWN_ONE(0); } }          // (a token's gather is the launch's longest chain)
+    else NORM_DOWN_ONE(0);
+  }
+  else NORM_DOWN_GO(1);
+#undef NORM_DOWN_ONE
 #undef NORM_DOWN_GO
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
+// the mixes whose straight code the smaller bounds hold: up to four streams of up to sixteen slices in all
+bool hc_few(const HcDev& h, int ksplit) { return h.hc <= 4 && ksplit <= 16; }
 template <int FMT, int T> int up_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, const float* xnew, float eps, float* mixed, float* inj, const HcRoute* rt, int nz) {
   const int nw = h.hc * h.up.U; size_t lds = 4 * ((size_t)T * h.lr + (size_t)nw * T * 64 + (size_t)T * 32 + (size_t)T * h.hc * 64);
   const QMatDev rq = rt ? rt->router : QMatDev{}; float* rp = rt ? rt->part : nullptr;
@@ -659,17 +706,25 @@ template <int FMT, int T> int up_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, 
                (rt ? qmat_gguf_bytes(rq, rq.rows) + 4.0 * T * (h.d / 64) * rq.tiles * 64 : 0.0));
 #define UP_MIX_GO(...) hipLaunchKernelGGL((k_hc_up_mix<FMT, T, __VA_ARGS__>), dim3(h.d / 64, 1, nz), dim3(nw * 64), lds, ctx->stream, h.up, w.o, w.ssq, ksplit, h.di.tiles * 64, h.lr, h.hc, h.has_inject ? 1 : 0, xnew, h.norm, eps, \
                      h.d, mixed, inj, (const uint2*)ctx->d_iq2xs, rq, rp)
+#define UP_MIX_R(KSM, HM) do { if (rt && rq.fmt == FMT_BF16) UP_MIX_GO(FMT_BF16, KSM, HM); else if (rt && rq.fmt == FMT_F32) UP_MIX_GO(FMT_F32, KSM, HM); else UP_MIX_GO(-1, KSM, HM); } while (0)
+  // Mixes as files store them in groups of eight: the common low ranks and slice counts (widths in powers of two) have instances of their
+  // own.  A launch is its instruction count -- low rank and slices at run time cost index arithmetic and a predicate a slice: A3B's
+  // shape (four streams, 256, sixteen slices), 200 tokens, 58 us and with the router 82 against 39 and 60.
+  constexpr bool OWN = FMT == FMT_BF16 && T == 8;
+#define UP_MIX_LR(KSM) do { if (h.lr == 64) UP_MIX_F(KSM, 64); else if (h.lr == 128) UP_MIX_F(KSM, 128); else if (h.lr == 256) UP_MIX_F(KSM, 256); else UP_MIX_F(KSM, 512); } while (0)
+#define UP_MIX_F(KSM, LR) do { if (rt && rq.fmt == FMT_BF16) UP_MIX_GO(FMT_BF16, KSM, 4, LR); else if (rt && rq.fmt == FMT_F32) UP_MIX_GO(FMT_F32, KSM, 4, LR); else UP_MIX_GO(-1, KSM, 4, LR); } while (0)
   bool done = false;
-  if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {          // the A3B configuration as files store it: constants folded in
-    if (h.hc == 4 && h.lr == 256 && ksplit == 16) {
-      if (rt && rq.fmt == FMT_BF16) UP_MIX_GO(FMT_BF16, 4, 256, 16); else if (rt && rq.fmt == FMT_F32) UP_MIX_GO(FMT_F32, 4, 256, 16); else UP_MIX_GO(-1, 4, 256, 16);
-      done = true;
-    }
+  if constexpr (OWN) {
+    done = h.hc <= 4 && (ksplit == 8 || ksplit == 16) && (h.lr == 64 || h.lr == 128 || h.lr == 256 || h.lr == 512);
+    if (done && ksplit == 16) UP_MIX_LR(16); else if (done) UP_MIX_LR(8);
   }
+#undef UP_MIX_F
+#undef UP_MIX_LR
   if (done) {}
-  else if constexpr (FMT == FMT_IQ3_S || FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {
-    if (rt && rq.fmt == FMT_BF16) UP_MIX_GO(FMT_BF16); else if (rt && rq.fmt == FMT_F32) UP_MIX_GO(FMT_F32); else UP_MIX_GO(-1);
-  } else UP_MIX_GO(-1);
+  else if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) { if (hc_few(h, ksplit)) UP_MIX_R(16, 4); else UP_MIX_R(32, 8); }
+  else if constexpr (FMT == FMT_IQ3_S) UP_MIX_R(32, 8);
+  else UP_MIX_GO(-1, 32, 8);
+#undef UP_MIX_R
 #undef UP_MIX_GO
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
@@ -681,12 +736,8 @@ template <int FMT, int T> int up_mix_launch(pyre_ctx* ctx, const HcDev& h, const
   constexpr int TS = T > 1 ? 2 : 1;
   const int items = h.hc * h.up.U * 16, nthr = std::max((TS * items + 63) / 64 * 64, (T * 16 + 63) / 64 * 64); const size_t lds = 4 * ((size_t)T * h.up.U * PYRE_UP_PAD + (size_t)items * T + (size_t)T * 32);
   { ProfScope ps(ctx, "hc_up_mix", qmat_gguf_bytes(h.up, h.up.rows) + 4.0 * T * (h.hc * h.d + h.d + (double)ksplit * (h.lr + h.hc)));
-#define UP_MIX_C_GO(...) hipLaunchKernelGGL((k_hc_up_mix_c<FMT, T __VA_ARGS__>), dim3(h.d / 16), dim3(nthr), lds, ctx->stream, h.up, w.o, w.ssq, ksplit, h.di.tiles * 64, h.lr, h.hc, h.has_inject ? 1 : 0, xnew, h.norm, eps, h.d, mixed, inj)
-#define UP_MIX_C_A3B , 4, 256, 16
-    bool done = false;
-    if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) { if (h.hc == 4 && h.lr == 256 && ksplit == 16) { UP_MIX_C_GO(UP_MIX_C_A3B); done = true; } }          // the A3B configuration as files store it: constants folded in
-    if (!done) UP_MIX_C_GO();
-#undef UP_MIX_C_A3B
+#define UP_MIX_C_GO(KSM, HM) hipLaunchKernelGGL((k_hc_up_mix_c<FMT, T, KSM, HM>), dim3(h.d / 16), dim3(nthr), lds, ctx->stream, h.up, w.o, w.ssq, ksplit, h.di.tiles * 64, h.lr, h.hc, h.has_inject ? 1 : 0, xnew, h.norm, eps, h.d, mixed, inj)
+    if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) { if (hc_few(h, ksplit)) UP_MIX_C_GO(16, 4); else UP_MIX_C_GO(32, 8); } else UP_MIX_C_GO(32, 8);
 #undef UP_MIX_C_GO
   } PYRE_CHECK_LAUNCH(ctx);
   return rt ? pyre_moe_router_shares_launch(ctx, "hc_up_mix_router", rt->router, mixed, T, h.d / 64, 1, rt->part, rt->dgx) : PYRE_OK;
@@ -791,7 +842,7 @@ size_t pyre_hc_rows_bytes(const HcDev& h, int groups) { return 3 * 256 + 4 * (si
 void pyre_hc_rows_carve(const HcDev& h, int groups, void* base, HcWork* w) { w->ssq = (float*)base; w->smx = nullptr; w->o = (float*)((uint8_t*)base + ((4 * (size_t)groups * hc_rows_split(h) * 8 + 255) & ~(size_t)255)); }
 int pyre_hc_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const float* x_in, int in_ss, int in_ts, float* x_out, int groups, const float* comb_out, const MoeOut* comb_moe, const float* comb_inj,
                             float eps, float* mixed, float* inj, const HcRoute* rt) {
-  if (!pyre_hc_rows_ok(h) || groups < 1 || groups > 65535 || x_in == x_out || (rt && !pyre_hc_route_ok(h, rt->router))) return pyre_fail(ctx, PYRE_E_ARG, "hc_mix_rows: unsupported shape");
+  if (!pyre_hc_rows_ok(h) || groups < 1 || groups * h.hc > 65535 || x_in == x_out || (rt && !pyre_hc_route_ok(h, rt->router))) return pyre_fail(ctx, PYRE_E_ARG, "hc_mix_rows: unsupported shape");
   const DownPlan p = down_plan(h); const MoeOut mo = comb_moe ? *comb_moe : MoeOut{nullptr, nullptr, nullptr, 0, 0};
   int rc = [&]() -> int { HC_FMT_SWITCH(h.di.fmt, return (norm_down_launch<F, 8>(ctx, h, w, p, x_in, in_ss, in_ts, x_out, comb_out, 1, mo, comb_inj, eps, groups));) }(); if (rc) return rc;
   return [&]() -> int { HC_FMT_SWITCH(h.up.fmt, return (up_mix_rows_launch<F, 8>(ctx, h, w, p.ksplit, x_out, eps, mixed, inj, rt, groups));) }();

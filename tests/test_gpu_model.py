@@ -342,6 +342,25 @@ def test_prompt_blocks_of_models_with_other_formats_beside_iq3s_experts(ctx, oth
             assert relerr(a, b) <= 1e-4 if n >= 72 else np.array_equal(a.view(np.uint32), b.view(np.uint32)), n
 
 
+@pytest.mark.parametrize("hc,hc_lr,d,top_k,hc_type,router_type", [
+    (3, 192, 512, 1, synth.BF16, synth.BF16), (4, 64, 1024, 4, synth.BF16, synth.F32), (4, 128, 1024, 7, synth.BF16, synth.BF16), (2, 512, 2048, 12, synth.BF16, synth.F16),
+    (4, 256, 2048, 16, synth.BF16, synth.BF16), (4, 256, 1024, 3, synth.F32, synth.BF16), (2, 64, 256, 5, synth.F32, synth.F32), (8, 128, 512, 2, synth.F16, synth.BF16), (2, 256, 4096, 9, synth.BF16, synth.F32),
+    (5, 192, 1024, 8, synth.BF16, synth.BF16), (4, 256, 4096, 10, synth.BF16, synth.BF16), (1, 1024, 512, 6, synth.F32, synth.BF16), (3, 128, 320, 13, synth.Q8_0, synth.F32)])
+def test_mixes_of_other_counts(ctx, hc, hc_lr, d, top_k, hc_type, router_type):
+    # streams, low ranks and slices on both sides of the bounds the mixes' launches are chosen by, every group size of the experts: a window is its
+    # single steps, a prompt layer by layer its windows, bit for bit, and the oracle's
+    c = small_cfg(hc=hc, hc_lr=hc_lr, d=d, top_k=top_k, n_exp=24, ff_exp=64, n_layers=2, full_every=2, hc_type=hc_type, router_type=router_type, qtype=synth.Q8_0)
+    hw, gm, om = pair(ctx, c, 57)
+    ids = np.random.Generator(np.random.PCG64(58)).integers(0, c.vocab, 27, dtype=np.uint32)
+    sa, sb, so = gm.new_state(64), gm.new_state(64), om.new_state()
+    la = gm.forward(ids[:19], sa)
+    for i in range(0, 19, 8): lb = gm.forward(ids[i:min(i + 8, 19)], sb)
+    assert np.array_equal(la.view(np.uint32), lb.view(np.uint32)) and relerr(la, om.forward(ids[:19], so)) <= 1e-4
+    lw = gm.forward_multi(ids[19:], sa)
+    for i in range(8): assert np.array_equal(gm.forward(ids[19 + i:20 + i], sb).view(np.uint32), lw[i].view(np.uint32)), i
+    assert relerr(lw, om.forward_multi(ids[19:], so)) <= 1e-4
+
+
 @pytest.mark.parametrize("hc_type,router_type", [(synth.BF16, synth.BF16), (synth.F32, synth.F32), (synth.F16, synth.BF16)])
 def test_full_width_mixes_in_file_formats_window_equals_single_steps(ctx, hc_type, router_type):
     # the launches with the A3B counts folded in (d 2048, four streams, low rank 256), every window width, the router's shares behind
