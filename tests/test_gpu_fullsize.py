@@ -111,35 +111,33 @@ def test_drafter_matches_the_oracle_at_full_width(ctx):
 
 
 def test_prompt_in_blocks_with_the_ffn_grouped_by_expert_agrees_with_the_windows_path(ctx, model4, monkeypatch):
-    """A long prompt takes blocks of up to 128 windows layer by layer, the FFN of a block's tokens grouped by expert on the
+    """A long prompt takes blocks of up to 2048 tokens layer by layer, the FFN of a block's tokens grouped by expert on the
     matrix cores: logits agree with the windows' path (PYRE_PROMPT_WINDOWS=1 at run time) to rounding, the tokens that follow
     and the state's length are the same, for a call that is whole blocks plus a ragged tail, and for a state that continues
-    with a second long call."""
+    with a second long call; the cutting into blocks (PYRE_PROMPT_PAIRS=0: 1024 tokens) and the per-class timing do not show in a bit."""
     cfg, gm = model4
     g = np.random.Generator(np.random.PCG64(21))
-    prompt = g.integers(0, cfg.vocab, 2 * 256 + 45, dtype=np.uint32)
-    more = g.integers(0, cfg.vocab, 256 + 100 + 9, dtype=np.uint32)          # a full block and a shorter one
+    prompt = g.integers(0, cfg.vocab, 2048 + 61, dtype=np.uint32)
+    more = g.integers(0, cfg.vocab, 1024 + 85, dtype=np.uint32)
     out = {}
-    modes = ("0", "1", "1 one block at a time", "1 groups of 5", "1 a launch a window", "1 projection in the chain", "1 attention in the chain", "1 router riding")
-    for mode in modes:
-        monkeypatch.setenv("PYRE_PROMPT_WINDOWS", "1" if mode == "0" else "0")
-        monkeypatch.setenv("PYRE_PROMPT_PAIRS", "0" if mode == "1 one block at a time" else "1")     # two blocks in flight, one's FFN beside the other's windows
-        monkeypatch.setenv("PYRE_PROMPT_GROUP", "5" if mode == "1 groups of 5" else "0")              # consecutive windows a stream takes together
-        monkeypatch.setenv("PYRE_PROMPT_BATCH", "0" if mode == "1 a launch a window" else "1")        # a group's mixes, projections, convolution and recurrences in one launch each
-        monkeypatch.setenv("PYRE_PROMPT_PROJ_EARLY", "0" if mode == "1 projection in the chain" else "1")     # projection (and convolution) outside the chain through the layer's state
-        monkeypatch.setenv("PYRE_PROMPT_ATTN_SPLIT", "0" if mode == "1 attention in the chain" else "1")      # the pass over the cache outside it
-        monkeypatch.setenv("PYRE_PROMPT_ROUTER_APART", "0" if mode == "1 router riding" else "1")           # the router's sums with the block's FFN launches, not on every window's FFN mix
-        st = gm.new_state(1024)
-        n0 = gm.prompt_blocks()
-        lg = gm.forward(prompt, st)
-        assert gm.prompt_blocks() - n0 == (0 if mode == "0" else 1)          # the path under test is the one that ran
-        toks = gm.decode_greedy_dev(st, int(np.argmax(lg)), 6)
-        lg2 = gm.forward(more, st)                                           # (starts at a position that is no multiple of eight)
-        toks2 = gm.decode_greedy_dev(st, int(np.argmax(lg2)), 4)
+    modes = {"windows": (0, 0), "blocks": (2, 1), "blocks of 1024": (3, 2), "blocks, timed": (2, 1)}          # and the blocks either call takes
+    for mode, want in modes.items():
+        monkeypatch.setenv("PYRE_PROMPT_WINDOWS", "1" if mode == "windows" else "0")
+        monkeypatch.setenv("PYRE_PROMPT_PAIRS", "0" if mode == "blocks of 1024" else "1")
+        ctx.prof_enable(mode == "blocks, timed")
+        try:
+            st = gm.new_state(4096)
+            n0 = gm.prompt_blocks(); lg = gm.forward(prompt, st); n1 = gm.prompt_blocks()
+            toks = gm.decode_greedy_dev(st, int(np.argmax(lg)), 6)
+            n2 = gm.prompt_blocks(); lg2 = gm.forward(more, st)                      # (starts at a position that is no multiple of eight)
+            assert (n1 - n0, gm.prompt_blocks() - n2) == want, mode                  # the path under test is the one that ran
+            toks2 = gm.decode_greedy_dev(st, int(np.argmax(lg2)), 4)
+        finally:
+            ctx.prof_enable(False)
         out[mode] = (lg.copy(), toks.copy(), lg2.copy(), toks2.copy(), len(st))
         st.close()
-    a, b = out["0"], out["1"]
-    for other in modes[2:]:          # the order and the grouping of the launches do not change a bit
+    a, b = out["windows"], out["blocks"]
+    for other in ("blocks of 1024", "blocks, timed"):
         for i in range(4):
             assert np.array_equal(np.asarray(b[i]).view(np.uint32), np.asarray(out[other][i]).view(np.uint32)), (other, i)
     assert a[4] == b[4] == prompt.size + 6 + more.size + 4
