@@ -946,7 +946,6 @@ int pyre_forward(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, const uint32
   if (s->m != m) return pyre_fail(ctx, PYRE_E_STATE, "pyre_forward: state belongs to another model");
   if (s->broken) return pyre_fail(ctx, PYRE_E_STATE, "%s: an earlier call failed half way through this state; pyre_state_reset or pyre_state_restore first", "pyre_forward");
   if (s->len + n > s->cap) return pyre_fail(ctx, PYRE_E_STATE, "pyre_forward: %d + %d tokens exceed the state's capacity %d", s->len, n, s->cap);
-  const auto t_enter = std::chrono::steady_clock::now();
   int rc = check_ids(ctx, m, ids, n); if (rc) return rc;
   s->last_window = 0;
   int i_first = 0;
@@ -1013,7 +1012,6 @@ int pyre_forward(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, const uint32
     if (rc) { s->broken = true; if (cx != ctx) pyre_fail(ctx, rc, "%s", cx->err.c_str()); for (auto* c2 : P->ctx) (void)hipStreamSynchronize(c2->stream); (void)hipStreamSynchronize(ctx->stream); return rc; }      // windows already issued have advanced the bookkeeping and part of the state
     prev = set;
   }
-  if (getenv("PYRE_DEBUG_ENQ")) { static auto t_prev = std::chrono::steady_clock::now(); auto t1 = std::chrono::steady_clock::now(); fprintf(stderr, "enq %d tokens (%d in blocks): %.3f ms since entry\n", n, i_first, std::chrono::duration<double>(t1 - t_enter).count() * 1e3); (void)t_prev; }
   if (P) for (int k = 1; k < K; ++k) PYRE_HIP(ctx, hipStreamWaitEvent(ctx->stream, P->done[k], 0));      // everything the other streams did precedes what follows here
   if (logits_host) PYRE_HIP(ctx, hipMemcpyAsync(logits_host, m->logits, (size_t)m->c.vocab * 4, hipMemcpyDeviceToHost, ctx->stream));
   PYRE_HIP(ctx, hipStreamSynchronize(ctx->stream)); return PYRE_OK;
