@@ -896,11 +896,13 @@ int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T
   if (!pyre_moe_block_ok(m) || T < 0 || T > T_router || T_router < 1 || T_router > T_max || (size_t)T_max * (m.top_k + 1) * m.ff * 4 >= (1ull << 32) || (size_t)T_max * m.d * 4 >= (1ull << 32) || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe block: unsupported shape (T = %d, %d router slices)", T, nsl);
   const int hs = m.ff, ny = m.n_exp + (T + 7) / 8, ne = T * (m.top_k + 1), ne_max = T_max * (m.top_k + 1);
   const bool fix = m.n_exp == 512 && m.top_k == 10 && nsl == 32;
-  // entries an expert: eight or fewer go through in one pass of k_moe_mm_blk, more share the decoding
-  static const int force = [] { const char* e = getenv("PYRE_MM_TG"); return e ? atoi(e) : 0; }();
-  const int mean = T * m.top_k / m.n_exp, tg = force ? force : (mean <= 3 ? 1 : (mean <= 8 ? 2 : (mean <= 32 ? 4 : 6)));
+  // Groups of eight entries that share an expert's decoding, by the mean entries an expert.  Gate / up + down, us, 512 experts top 10 of
+  // width 512: 64 tokens (mean 1.2) 168 with one, 172 with two; 104 (2.0) 199, 189; 208 (4.1) 225 with two, 230 with four; 312 (6.1)
+  // 262, 255; 520 (10) 320, 294; 2040 (40) 738 with four, 769 with six.  128 experts top 8: 104 (6.5) 92 with two, 101 with four; 160
+  // (10) 119, 109; 1648 (103) 535 with four, 585 with six.
+  const int mean = T * m.top_k / m.n_exp, tg = mean <= 1 ? 1 : (mean <= 6 ? 2 : 4);
 #define MM_MANY(DN, TG, GX, GZ, ZR, KC) hipLaunchKernelGGL((k_moe_mm_many<DN, TG>), dim3(GX, m.n_exp + (T + 8 * TG - 1) / (8 * TG), GZ), dim3(256), (size_t)TG * 8 * (KC / 256) * 4, ctx->stream, m, b, T, ZR)
-#define MM_GO(DN, GX, GZ, ZR, KC) do { if (tg == 1) hipLaunchKernelGGL(k_moe_mm_blk<DN>, dim3(GX, ny, GZ), dim3(256), 0, ctx->stream, m, b, T, ZR); else if (tg == 2) MM_MANY(DN, 2, GX, GZ, ZR, KC); else if (tg == 4) MM_MANY(DN, 4, GX, GZ, ZR, KC); else MM_MANY(DN, 6, GX, GZ, ZR, KC); } while (0)
+#define MM_GO(DN, GX, GZ, ZR, KC) do { if (tg == 1) hipLaunchKernelGGL(k_moe_mm_blk<DN>, dim3(GX, ny, GZ), dim3(256), 0, ctx->stream, m, b, T, ZR); else if (tg == 2) MM_MANY(DN, 2, GX, GZ, ZR, KC); else MM_MANY(DN, 4, GX, GZ, ZR, KC); } while (0)
   {
     if (nsl != m.d / 64 || (m.router.fmt != FMT_BF16 && m.router.fmt != FMT_F32)) return pyre_fail(ctx, PYRE_E_ARG, "moe block: the router's sums by %d slices, router format %d", nsl, m.router.fmt);
     ProfScope ps(ctx, "moe_block_router", qmat_gguf_bytes(m.router, m.router.rows) + 4.0 * T * (m.d + (double)nsl * r64));

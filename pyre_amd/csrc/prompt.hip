@@ -455,8 +455,13 @@ int pyre_blk_gemm_launch(pyre_ctx* ctx, const QMatDev& m, const uint4* op, size_
   if (K128 % parts || nw * cw < per) return pyre_fail(ctx, PYRE_E_SHAPE, "blk_gemm: %d columns in %d slices", m.cols, parts);
   const int G = (T + 7) / 8, bx = (m.tiles + 3) / 4, ish = inv_kind == PYRE_INV_CHUNK ? 0 : 1; const bool uni = inv_kind == PYRE_INV_TOKEN;
   ProfScope ps(ctx, "blk_gemm", qmat_gguf_bytes(m, m.rows) + 4.0 * T * ((double)m.cols + m.rows));
-  // many groups a wave amortise the decoding (eight, with running sums to keep four); with too few workgroups for the chip, fewer groups and more workgroups
-  const int b2 = bx * parts, tg = cw == 1 && b2 * ((G + 7) / 8) >= 512 ? 8 : (b2 * ((G + 3) / 4) >= 512 ? 4 : (b2 * ((G + 1) / 2) >= 192 ? 2 : 1));
+  // Groups a wave meets with a decoded chunk (eight, with running sums to keep four): as few as leave at most a workgroup a compute unit
+  // (256), with four K parts, whose workgroups are a quarter as long, two; four until there are 640.  us a launch, 2048 columns:
+  // 12352 rows (49 workgroups a group) 32 tokens 21.0 with one, 23.1 with two; 48: 28.0, 23.3; 72: 24.8 with two, 31.3 with four; 104:
+  // 33.8, 31.9; 264: 58.5, 46.1; 392: 67.1 with four, 66.9 with eight; 520: 84.2, 70.8; 2048: 258, 228.  9216 rows (36): 72 tokens 28.0
+  // with one, 23.6 with two; 136: 32.7 with two, 31.7 with four; 520: 65.6 with four, 66.8 with eight; 776: 85.5, 72.0.  2048 rows of 4096
+  // columns in four parts (32): 72 tokens 17.4 with one, 16.4 with two; 200: 21.4 with two, 22.3 with four; 264: 29.9, 27.8.
+  const int b2 = bx * parts, tg = b2 * G <= 256 ? 1 : (b2 * ((G + 1) / 2) <= (parts > 1 ? 512 : 256) ? 2 : (cw != 1 || b2 * ((G + 3) / 4) <= 640 ? 4 : 8));
 #define BLK_GO(TG, CW1, UNI) hipLaunchKernelGGL((k_blk_gemm<TG, CW1, UNI>), dim3(bx, (G + TG - 1) / TG, parts), dim3(256), (size_t)TG * (per / (ish + 1) + 1) * 8 * 4, ctx->stream, m, op, op_gs, inv, inv_gs, ish, cw, y, ys, T)
   if (cw == 1 && uni) { if (tg == 8) BLK_GO(8, true, true); else if (tg == 4) BLK_GO(4, true, true); else if (tg == 2) BLK_GO(2, true, true); else BLK_GO(1, true, true); }
   else if (cw == 1) { if (tg == 8) BLK_GO(8, true, false); else if (tg == 4) BLK_GO(4, true, false); else if (tg == 2) BLK_GO(2, true, false); else BLK_GO(1, true, false); }
