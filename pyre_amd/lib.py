@@ -947,6 +947,7 @@ class Session:
     def generate_greedy(self, first_logits, n_out, n_draft=0, draft_stream=None):
         fl = np.ascontiguousarray(first_logits, dtype=np.float32); out = np.empty(n_out, dtype=np.uint32); rounds = C.c_int32()
         ds = np.ascontiguousarray(draft_stream, dtype=np.uint32) if draft_stream is not None else None
+        _expect(ds is None or ds.size >= n_out + 8, "draft_stream", "%d ids or more" % (n_out + 8), ds is not None and ds.shape)
         self.ctx.check(self.ctx.L.pyre_session_generate_greedy(self.ctx.h, self.h, _ptr(fl), n_out, _ptr(out), n_draft, _ptr(ds) if ds is not None else None, C.byref(rounds)), "session_generate_greedy")
         return out, rounds.value
 

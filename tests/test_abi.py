@@ -44,13 +44,13 @@ import numpy as np
 from pyre_amd import lib
 z = lambda *s: np.zeros(s, np.float32)
 g = object.__new__(lib.Gdn); g.h = None; g.ch, g.nv, g.dv, g.pw = 1024, 4, 128, 1544
-m = object.__new__(lib.Model); m.h = None; d = object.__new__(lib.Mtp); d.h = None
+m = object.__new__(lib.Model); m.h = None; d = object.__new__(lib.Mtp); d.h = None; s = object.__new__(lib.Session); s.h = None
 class A(lib.Attn):
     def __len__(self): return 5
 a = object.__new__(A); a.h = None
 calls = [lambda: lib.adapt_plan(1, 1.0, z(9), 0.5, 0.0), lambda: g.step(z(3, 1024), z(3, 512), z(3, 4), z(3, 3)), lambda: g.prefill_chunked(z(3, 1024), z(2, 512), z(3, 4), z(3, 4)),
          lambda: g.prefill_chunked(z(3, 1000), z(3, 512), z(3, 4), z(3, 4)), lambda: a.load_index(z(4, 64)), lambda: m.generate_greedy(None, z(8), 4, 2, np.zeros(11, np.uint32)),
-         lambda: d.generate_greedy_forced(None, z(8), 4, np.zeros(11, np.uint32))]
+         lambda: d.generate_greedy_forced(None, z(8), 4, np.zeros(11, np.uint32)), lambda: s.generate_greedy(z(8), 4, 2, np.zeros(11, np.uint32))]
 for i, c in enumerate(calls):
     try: c()
     except ValueError as e:
