@@ -396,6 +396,8 @@ bool pyre_hc_leaves_digits(const HcDev& h);          // with a riding router: wh
 int pyre_hc_mix_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const float* x_in, int in_ss, int in_ts, float* x_out, int t, const float* comb_out, const MoeOut* comb_moe, const float* comb_inj,
                        float eps, float* mixed_dev, float* inj_dev, const HcRoute* route = nullptr, int comb_parts = 1, const AopOut* aop = nullptr);
 bool pyre_hc_route_ok(const HcDev& h, const QMatDev& router);
+// whether the mix of a window of t tokens adds a pending update that comes as PYRE_GEMV_PARTS partial vectors (comb_parts)
+bool pyre_hc_takes_parts(const HcDev& h, int t);
 // waves per workgroup, units per wave and K slices of the norm + [down ; inject] kernel; false if the shape is unsupported
 bool pyre_hc_plan(const HcDev& h, int* nw, int* upw, int* ksplit);
 int pyre_hc_combine_launch(pyre_ctx* ctx, int d, int hc, float* x_dev, int t, const float* out_dev, const float* inj_dev);

@@ -7,16 +7,16 @@
 // reduces the gated, normalized streams to their mean.
 #include "gemm_m.h"
 #include "digits.h"
+#include "hc.h"
 #include <stdlib.h>
 #include <algorithm>
 
 PYRE_TS_DECL(hc_ts) PYRE_TS_EXPORT(hc_ts, pyre_debug_ts_hc)
-__device__ __forceinline__ float sigm(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 // Stream element i of token ti with the pending residual update applied: x + out * w  (:1384-1387), w = 2*sigm(inj).
 // `out` is a plain [t][d] vector (comb_out) or the unreduced FFN output (mo.partial != nullptr).
 // NP > 1: `out` comes as NP partial vectors, part q of token ti at comb_out + (q*T + ti)*d, added in order from the first
-// (pyre_gemv_parts_launch); all parts are fetched before the first add.
+// (pyre_gemv_parts_launch); all parts are fetched before the first add.  NP = 0: never unreduced.
 template <int T, int NP, int FK = 0, int FG = 0> __device__ __forceinline__ float hc_x_new(const float* __restrict__ x_in, int in_ss, int in_ts, const float* __restrict__ comb_out, const MoeOut& mo, float w, int d, int ti, int s, int i) {
   float v = x_in[(size_t)ti * in_ts + (size_t)s * in_ss + i];
   if constexpr (NP > 1) {
@@ -28,74 +28,10 @@ template <int T, int NP, int FK = 0, int FG = 0> __device__ __forceinline__ floa
     for (int q = 1; q < NP; ++q) o += sv[q];
     v = v + o * w;
   } else {
-    if (mo.partial) v = v + moe_out_value<FK, FG>(mo, ti, i) * w;
+    if (NP == 1 && mo.partial) v = v + moe_out_value<FK, FG>(mo, ti, i) * w;
     else if (comb_out) v = v + comb_out[(size_t)ti * d + i] * w;
   }
   return v;
-}
-
-// x / n for 0 <= x < 2^16, n <= 2^12 with r = 1 / n within two units in the last place: (x + 1/2) / n lies 1 / (2 n) or more off an
-// integer, the product's error is below x / n * 2^-21
-__device__ __forceinline__ int hc_div(int x, float r) { return (int)(((float)x + 0.5f) * r); }
-__device__ __forceinline__ float hc_recip(int n) { return __builtin_amdgcn_rcpf((float)n); }
-// v / hc; a power of two by multiplication, the same bits
-__device__ __forceinline__ float hc_mean(float v, int hc) { return (hc & (hc - 1)) == 0 ? v * __uint_as_float((uint32_t)(127 - (31 - __builtin_clz(hc))) << 23) : v / (float)hc; }
-
-// The slices of one output row, all loads in flight together: groups of eight behind a branch the whole launch agrees on
-// (ksplit is a kernel argument), so that unused groups cost neither loads nor instruction fetch; inside a group slices
-// past ksplit repeat the last one and are never added.  `want` is the thread's own condition (one execution mask).
-template <int KSM> __device__ __forceinline__ void hc_load_run(float (&sv)[KSM], const float* __restrict__ p, int n, int stride) {      // n (<= KSM) values at p, p + stride, ..
-#pragma unroll
-  for (int k = 0; k < KSM; ++k) sv[k] = 0.0f;
-#pragma unroll
-  for (int g = 0; g < KSM / 4; ++g) if (g * 4 < n) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) sv[g * 4 + j] = p[(size_t)min(g * 4 + j, n - 1) * stride];
-  }
-}
-template <int T, int KSM> __device__ __forceinline__ void hc_load_slices(float (&pv)[KSM], const float* __restrict__ part, bool want, int ksplit, int t, int r64, int i) {
-#pragma unroll
-  for (int ks = 0; ks < KSM; ++ks) pv[ks] = 0.0f;
-  const unsigned off = (unsigned)(t * r64 + i);
-  if (want) {
-#pragma unroll
-    for (int g = 0; g < KSM / 8; ++g) if (g * 8 < ksplit) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) pv[g * 8 + j] = (part + (size_t)min(g * 8 + j, ksplit - 1) * T * r64)[off];      // launch-uniform base + the thread's 32-bit offset
-    }
-  }
-}
-
-// the slices of one row in order, each times its stream's scale (sls: at least KSM floats); whole groups of four carry no predicates
-template <int KSM> __device__ __forceinline__ float hc_slice_sum(const float (&pv)[KSM], const float* sls, int ksplit) {
-  float o = 0.0f;
-#pragma unroll
-  for (int g = 0; g < KSM; g += 4) if (g < ksplit) {
-    float sc[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) sc[j] = sls[g + j];
-    if (g + 4 <= ksplit) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) { const float tm = pv[g + j] * sc[j]; o = g + j == 0 ? tm : o + tm; }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 3; ++j) if (g + j < ksplit) { const float tm = pv[g + j] * sc[j]; o = g + j == 0 ? tm : o + tm; }
-    }
-  }
-  return o;
-}
-// the gate logit: U (<= 16) sums `stride` floats apart in order, four in flight at a time
-__device__ __forceinline__ float hc_unit_sum(const float* red, int U, int stride) {
-  float g = red[0];
-#pragma unroll
-  for (int k = 1; k < 16; k += 3) if (k < U) {
-    float v[3];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) v[j] = red[min(k + j, U - 1) * stride];
-#pragma unroll
-    for (int j = 0; j < 3; ++j) if (k + j < U) g += v[j];
-  }
-  return g;
 }
 
 // grid (row tiles of [down ; inject], K slices of a stream, streams x groups of tokens), nw waves.  A workgroup owns L = nw*upw*64 columns
@@ -315,88 +251,6 @@ template <int FMT, int T, int RF, int KSM, int HM, int FLR = 0> __global__ __lau
     }
   }
   PYRE_TS(7); PYRE_TS_FLUSH(hc_ts, ROUTE ? 16 : 24);
-}
-
-// The same launch for a window alone (at most eight tokens) and the formats of up_by_columns: grid (d / 16), sixteen columns a workgroup, a lane a (stream, unit, column)
-// item of the up GEMV and TS sets of them sharing the tokens (set k: tokens k, k + TS, ..), on d / 16 compute units instead of d / 64; the
-// router is a launch of its own behind it.  The launch is latency, and half of that was fetching instructions and dividing: with room for
-// 32 slices and eight streams it is 18 KB of straight code, with room for sixteen and four (KSM, HM, as k_hc_up_mix) 10 KB, indices by
-// hc_div, whole groups of slices without predicates.  A3B shape, bf16, one token: 8.2 us as k_hc_up_mix (13.9 with the router, and 2.5
-// for the digits behind it), 8.4 here with the larger code, 6.9 with the smaller (and 3.2 for router and digits).  A lane's terms, and every order of adding, are those of k_hc_up_mix, bit for bit.  A unit's row of lo
-// is PAD floats behind the last one: the four units of a wave read four different banks.
-#define PYRE_UP_PAD 68
-template <int FMT, int T, int KSM, int HM> __global__ __launch_bounds__(512) void k_hc_up_mix_c(QMatDev up, const float* __restrict__ part, const float* __restrict__ ssq, int ksplit, int r64, int lr, int hc, int has_inject,
-    const float* __restrict__ xnew, const float* __restrict__ norm, float eps, int d, float* __restrict__ mixed, float* __restrict__ inj) {
-  constexpr int TS = T > 1 ? 2 : 1, TT = (T + TS - 1) / TS;
-  const uint2* lds2 = nullptr;
-  qmat_args_now(up); args_now(part, ssq, ksplit, r64, lr, hc, has_inject, xnew, norm, eps, d, mixed, inj);
-  extern __shared__ __align__(16) float sm[];
-  const int nthr = blockDim.x, tid = threadIdx.x, U = lr >> 6, items = hc * U * 16;
-  const float rhc = hc_recip(hc), rlr = hc_recip(lr); const int kps = __builtin_amdgcn_readfirstlane(hc_div(ksplit, rhc));
-  float* lo = sm;                                          // [T][U][PAD]
-  float* red = lo + (size_t)T * U * PYRE_UP_PAD;           // [hc * U][T][16]
-  float* sls = red + (size_t)hc * U * T * 16;              // [T][32]: the RMS scale of the stream each slice belongs to
-  const int ts = tid >= items ? (tid >= 2 * items ? 2 : 1) : 0, it = ts < TS ? tid - ts * items : 0, su = it >> 4, r = it & 15, s = hc_div(su, hc_recip(U)), ku = su - s * U, col0 = blockIdx.x * 16;
-  const bool work = ts < TS;
-  float ssv[KSM];
-  const int stt = hc_div(tid, rhc), sq = tid - stt * hc;
-  const bool own = tid < T * hc;                           // thread (token stt, stream sq): the stream's scale, and in the first workgroup its inject row
-#pragma unroll
-  for (int k = 0; k < KSM; ++k) ssv[k] = 0.0f;
-  if (own) hc_load_run<KSM>(ssv, ssq + (size_t)(sq * kps) * T + stt, kps, T);
-  float pv[KSM], pvi[KSM];
-  int idx = tid, t = hc_div(idx, rlr), i = idx - t * lr;
-  hc_load_slices<T, KSM>(pv, part, idx < T * lr, ksplit, t, r64, i);
-  hc_load_slices<T, KSM>(pvi, part, own && has_inject && blockIdx.x == 0, ksplit, stt, r64, lr + sq);
-  const UnitRaw<FMT> raw = unit_load<FMT>(up, s * (d >> 6) + (col0 >> 6), work ? ku : 0, (col0 & 63) + r);
-  // the epilogue's operands: thread (token tid / 16, column tid % 16) adds the streams of its column
-  float xpre[HM], npre[HM];
-  const int et = tid >> 4, el = tid & 15;
-#pragma unroll
-  for (int q = 0; q < HM; ++q) if (tid < T * 16 && q < hc) { xpre[q] = xnew[((size_t)et * hc + q) * d + col0 + el]; npre[q] = norm[(size_t)q * d + col0 + el]; } else { xpre[q] = 0.0f; npre[q] = 0.0f; }
-  if (own) {
-    float tot = ssv[0];
-#pragma unroll
-    for (int k = 1; k < KSM; ++k) if (k < kps) tot += ssv[k];
-    const float sc = 1.0f / sqrtf(tot / (float)d + eps);
-    for (int k = 0; k < kps; ++k) sls[stt * 32 + sq * kps + k] = sc;
-  }
-  lds_barrier();
-  while (idx < T * lr) {
-    const float v = hc_mean(hc_slice_sum<KSM>(pv, sls + t * 32, ksplit), hc);
-    lo[((size_t)t * U + (i >> 6)) * PYRE_UP_PAD + (i & 63)] = v * sigm(v);
-    idx += nthr;
-    if (idx < T * lr) { t = hc_div(idx, rlr); i = idx - t * lr; hc_load_slices<T, KSM>(pv, part, true, ksplit, t, r64, i); }
-  }
-  if (own && blockIdx.x == 0) inj[stt * hc + sq] = has_inject ? hc_mean(hc_slice_sum<KSM>(pvi, sls + stt * 32, ksplit), hc) : 0.0f;
-  lds_barrier();
-  if (work) {
-    float acc[TT];
-#pragma unroll
-    for (int k = 0; k < TT; ++k) acc[k] = 0.0f;
-    if constexpr (T % TS == 0) unit_fma<FMT, TT>(up, raw, ku, lds2, tid & 63, lo + ((size_t)ts * U + ku) * PYRE_UP_PAD, TS * U * PYRE_UP_PAD, acc);
-    else {          // an odd width: the second set has a token less
-      if (ts == 0) unit_fma<FMT, TT>(up, raw, ku, lds2, tid & 63, lo + ku * PYRE_UP_PAD, TS * U * PYRE_UP_PAD, acc);
-      else { float a1[TT - 1]; 
-#pragma unroll
-        for (int k = 0; k + 1 < TT; ++k) a1[k] = 0.0f;
-        unit_fma<FMT, TT - 1>(up, raw, ku, lds2, tid & 63, lo + ((size_t)ts * U + ku) * PYRE_UP_PAD, TS * U * PYRE_UP_PAD, a1);
-#pragma unroll
-        for (int k = 0; k + 1 < TT; ++k) acc[k] = a1[k]; }
-    }
-#pragma unroll
-    for (int k = 0; k < TT; ++k) { const int t2 = ts + k * TS; if (t2 < T) red[((size_t)su * T + t2) * 16 + r] = acc[k]; }
-  }
-  lds_barrier();
-  if (tid < T * 16) {
-    float mx = 0.0f;
-#pragma unroll
-    for (int q = 0; q < HM; ++q) if (q < hc) {          // streams ascending from zero (:1380)
-      const float g = hc_unit_sum(red + ((size_t)(q * U) * T + et) * 16 + el, U, T * 16);
-      mx += xpre[q] * sls[et * 32 + q * kps] * npre[q] * sigm(g);            // rms, :209: (x * s) * w
-    }
-    mixed[(size_t)et * d + col0 + el] = hc_mean(mx, hc);
-  }
 }
 
 // ---- the same two launches with both GEMVs on the f16 matrix cores -------------------------------------------------------
@@ -684,21 +538,24 @@ template <int FMT, int T> int norm_down_launch(pyre_ctx* ctx, const HcDev& h, co
   ProfScope ps(ctx, "hc_norm_down", qmat_gguf_bytes(h.di, h.di.rows) + 4.0 * T * h.hc * h.d * 4);
 #define NORM_DOWN_GO(NP) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, NP>), dim3(h.di.tiles, p.ksplit / h.hc, nz * h.hc), dim3(p.nw * 64), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
                      w.ssq, w.o, p.upw, (const uint2*)ctx->d_iq2xs)
-#define NORM_DOWN_ONE(FG) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, 1, true, FG>), dim3(h.di.tiles, p.ksplit / h.hc, nz * h.hc), dim3(512), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
+  // a window's pending update as four partial vectors (pyre_hc_takes_parts); a prompt's groups of eight, whose update is summed, in an
+  // instance without the gather: its instructions cost 2.7 us of 49 at 200 tokens of A3B's shape, bf16
+  [[maybe_unused]] constexpr int NPT = T > 1 ? PYRE_GEMV_PARTS : 1, NPR = T == 8 ? 0 : 1;
+#define NORM_DOWN_ONE(NP, FG) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, NP, true, FG>), dim3(h.di.tiles, p.ksplit / h.hc, nz * h.hc), dim3(512), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
                      w.ssq, w.o, p.upw, (const uint2*)ctx->d_iq2xs)
   if constexpr (FMT == FMT_IQ3_S) { if (comb_parts > 1) NORM_DOWN_GO(PYRE_GEMV_PARTS); else NORM_DOWN_GO(1); }
   else if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {
     if (p.nw != 8 || p.upw != 1) NORM_DOWN_GO(1);
-    else if constexpr (T == 1) { switch (mo.partial ? (mo.k + 4) / 4 : 0) { case 1: NORM_DOWN_ONE(1); break; case 2: NORM_DOWN_ONE(2); break; case 3: NORM_DOWN_ONE(3); break; case 4: NORM_DOWN_ONE(4); break; case 5: NORM_DOWN_ONE(5); break; default: NORM_DOWN_ONE(0); } }          // (a token's gather is the launch's longest chain)
-    else NORM_DOWN_ONE(0);
+    else if (comb_parts > 1) NORM_DOWN_ONE(NPT, 0);
+    else if (T == 8 && nz > 1 && !mo.partial) NORM_DOWN_ONE(NPR, 0);
+    else if constexpr (T == 1) { switch (mo.partial ? (mo.k + 4) / 4 : 0) { case 1: NORM_DOWN_ONE(1, 1); break; case 2: NORM_DOWN_ONE(1, 2); break; case 3: NORM_DOWN_ONE(1, 3); break; case 4: NORM_DOWN_ONE(1, 4); break; case 5: NORM_DOWN_ONE(1, 5); break; default: NORM_DOWN_ONE(1, 0); } }          // (a token's gather is the launch's longest chain)
+    else NORM_DOWN_ONE(1, 0);
   }
   else NORM_DOWN_GO(1);
 #undef NORM_DOWN_ONE
 #undef NORM_DOWN_GO
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
-// the mixes whose straight code the smaller bounds hold: up to four streams of up to sixteen slices in all
-bool hc_few(const HcDev& h, int ksplit) { return h.hc <= 4 && ksplit <= 16; }
 template <int FMT, int T> int up_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, const float* xnew, float eps, float* mixed, float* inj, const HcRoute* rt, int nz) {
   const int nw = h.hc * h.up.U; size_t lds = 4 * ((size_t)T * h.lr + (size_t)nw * T * 64 + (size_t)T * 32 + (size_t)T * h.hc * 64);
   const QMatDev rq = rt ? rt->router : QMatDev{}; float* rp = rt ? rt->part : nullptr;
@@ -721,7 +578,7 @@ template <int FMT, int T> int up_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, 
 #undef UP_MIX_F
 #undef UP_MIX_LR
   if (done) {}
-  else if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) { if (hc_few(h, ksplit)) UP_MIX_R(16, 4); else UP_MIX_R(32, 8); }
+  else if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) { if (pyre_hc_few(h, ksplit)) UP_MIX_R(16, 4); else UP_MIX_R(32, 8); }
   else if constexpr (FMT == FMT_IQ3_S) UP_MIX_R(32, 8);
   else UP_MIX_GO(-1, 32, 8);
 #undef UP_MIX_R
@@ -733,13 +590,7 @@ constexpr bool up_by_columns(int fmt) { return fmt == FMT_F32 || fmt == FMT_F16 
 template <int FMT, int T> int up_mix_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, const float* xnew, float eps, float* mixed, float* inj, const HcRoute* rt) {
   if constexpr (!up_by_columns(FMT)) return up_mix_rows_launch<FMT, T>(ctx, h, w, ksplit, xnew, eps, mixed, inj, rt, 1);
   else {
-  constexpr int TS = T > 1 ? 2 : 1;
-  const int items = h.hc * h.up.U * 16, nthr = std::max((TS * items + 63) / 64 * 64, (T * 16 + 63) / 64 * 64); const size_t lds = 4 * ((size_t)T * h.up.U * PYRE_UP_PAD + (size_t)items * T + (size_t)T * 32);
-  { ProfScope ps(ctx, "hc_up_mix", qmat_gguf_bytes(h.up, h.up.rows) + 4.0 * T * (h.hc * h.d + h.d + (double)ksplit * (h.lr + h.hc)));
-#define UP_MIX_C_GO(KSM, HM) hipLaunchKernelGGL((k_hc_up_mix_c<FMT, T, KSM, HM>), dim3(h.d / 16), dim3(nthr), lds, ctx->stream, h.up, w.o, w.ssq, ksplit, h.di.tiles * 64, h.lr, h.hc, h.has_inject ? 1 : 0, xnew, h.norm, eps, h.d, mixed, inj)
-    if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) { if (hc_few(h, ksplit)) UP_MIX_C_GO(16, 4); else UP_MIX_C_GO(32, 8); } else UP_MIX_C_GO(32, 8);
-#undef UP_MIX_C_GO
-  } PYRE_CHECK_LAUNCH(ctx);
+  const int rc = pyre_hc_up_cols_launch(ctx, h, w, ksplit, T, xnew, eps, mixed, inj); if (rc) return rc;
   return rt ? pyre_moe_router_shares_launch(ctx, "hc_up_mix_router", rt->router, mixed, T, h.d / 64, 1, rt->part, rt->dgx) : PYRE_OK;
   }
 }
@@ -820,6 +671,10 @@ int up_mix(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, int t, co
 
 bool pyre_hc_leaves_digits(const HcDev& h) { return hc_on_matrix_cores(h) || up_by_columns(h.up.fmt); }
 bool pyre_hc_aop_ok(const HcDev& h) { return hc_on_matrix_cores(h) && h.hc <= 4; }
+bool pyre_hc_takes_parts(const HcDev& h, int t) {
+  const int f = h.di.fmt; const DownPlan p = down_plan(h);
+  return f == FMT_IQ3_S || (t > 1 && (f == FMT_BF16 || f == FMT_F16 || f == FMT_F32) && p.nw == 8 && p.upw == 1);
+}
 bool pyre_hc_route_ok(const HcDev& h, const QMatDev& router) {
   const int f = h.up.fmt;
   return (f == FMT_IQ3_S || f == FMT_BF16 || f == FMT_F16 || f == FMT_F32) && (router.fmt == FMT_BF16 || router.fmt == FMT_F32) && router.cols == h.d && h.d / 64 <= 64 && router.U == h.d / 64;
@@ -851,7 +706,7 @@ int pyre_hc_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, cons
 int pyre_hc_mix_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const float* x_in, int in_ss, int in_ts, float* x_out, int t, const float* comb_out, const MoeOut* comb_moe, const float* comb_inj,
                        float eps, float* mixed, float* inj, const HcRoute* route, int comb_parts, const AopOut* aop) {
   if (t < 1 || t > 8) return pyre_fail(ctx, PYRE_E_ARG, "hc_mix: t = %d outside 1..8", t);
-  if (comb_parts != 1 && !(comb_parts == PYRE_GEMV_PARTS && h.di.fmt == FMT_IQ3_S && comb_out && !comb_moe)) return pyre_fail(ctx, PYRE_E_ARG, "hc_mix: %d partial vectors (1, or %d with an IQ3_S mix)", comb_parts, PYRE_GEMV_PARTS);
+  if (comb_parts != 1 && !(comb_parts == PYRE_GEMV_PARTS && pyre_hc_takes_parts(h, t) && comb_out && !comb_moe)) return pyre_fail(ctx, PYRE_E_ARG, "hc_mix: %d partial vectors (1, or %d where pyre_hc_takes_parts)", comb_parts, PYRE_GEMV_PARTS);
   if (route && !pyre_hc_route_ok(h, route->router)) return pyre_fail(ctx, PYRE_E_SHAPE, "hc_mix: this router cannot ride on the mix");
   if (x_in == x_out) return pyre_fail(ctx, PYRE_E_ARG, "hc_mix: the updated streams must go to another buffer");
   if (h.d % 64 || h.lr % 64 || h.hc * h.up.U > 16 || h.up.tiles != h.hc * (h.d / 64) || h.di.U != h.hc * (h.d / 64))

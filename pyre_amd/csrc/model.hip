@@ -808,14 +808,14 @@ struct WinRun {
     return PYRE_OK;
   }
   // whether layer il's FFN output of a window of several tokens goes to the next mix as four group sums a token: when that mix
-  // can add partial vectors (an IQ3_S mix over all of the window's tokens, no PLE layer in between); otherwise, and for a
+  // can add partial vectors (pyre_hc_takes_parts, over all of the window's tokens, no PLE layer in between); otherwise, and for a
   // single token, unreduced
   bool groups_at(int il) const {
     const pyre_model_cfg& c = m->c; const Layer& L = m->layers[il];
     bool groups = raw_moe && t > 1 && moe_groups && pyre_moe_groups_ok(L.moe);
     if (groups) {
-      if (il + 1 < c.n_layers) { const Layer& Ln = m->layers[il + 1]; groups = !Ln.ple && Ln.hca.di.fmt == FMT_IQ3_S; }
-      else groups = (o.head_tokens >= t || (s->mtp && o.keep_from < t)) && m->head.di.fmt == FMT_IQ3_S;
+      if (il + 1 < c.n_layers) { const Layer& Ln = m->layers[il + 1]; groups = !Ln.ple && pyre_hc_takes_parts(Ln.hca, t); }
+      else groups = (o.head_tokens >= t || (s->mtp && o.keep_from < t)) && pyre_hc_takes_parts(m->head, t);
     }
     return groups;
   }
