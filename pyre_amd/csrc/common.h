@@ -368,7 +368,7 @@ int pyre_ple_rows_launch(pyre_ctx* ctx, const PleCfg& c, const QMatDev& tab, con
 int pyre_ple_launch(pyre_ctx* ctx, const PleCfg& c, const PleDev& p, const PleWork& w, int d, int hc, float eps, const float* x_in, int in_ss, int in_ts, float* x_out,
                     const float* comb_out, const MoeOut* comb_moe, const float* comb_inj, int start, const int* posp, int t);
 
-// ---- hyper-connections (hc.hip) ---------------------------------------------------------------------------------------
+// ---- hyper-connections (hc.hip, hc_cols.hip, hc_m.hip) ---------------------------------------------------------------------------------------
 struct HcDev { QMatDev di; QMatDev up; const float* norm; int d, hc, lr; bool has_inject;      // di = [down ; inject] rows
                QMatDev di_m{}, up_m{}; };      // the same two matrices in the matrix-core layout (fmt == FMT_IQ3_S_M) when they are IQ3_S of whole super-blocks
 struct HcWork { float* ssq; float* o; float* smx; };    // [<=32][8] slice sums of squares of the streams, [<=32][8][tiles*64] slice sums of [down ; inject], [<=32][8] largest |x * norm weight| of each slice

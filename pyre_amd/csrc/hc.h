@@ -1,8 +1,29 @@
-// What the launches of a lane = row hyper-connection mix share (hc.hip, hc_cols.hip).
+// What the launches of a hyper-connection mix share (hc.hip, hc_cols.hip, hc_m.hip).
 #pragma once
 #include "formats.h"
 
 __device__ __forceinline__ float sigm(float x) { return 1.0f / (1.0f + expf(-x)); }
+
+// Stream element i of token ti with the pending residual update applied: x + out * w  (:1384-1387), w = 2*sigm(inj).
+// `out` is a plain [t][d] vector (comb_out) or the unreduced FFN output (mo.partial != nullptr).
+// NP > 1: `out` comes as NP partial vectors, part q of token ti at comb_out + (q*T + ti)*d, added in order from the first
+// (pyre_gemv_parts_launch); all parts are fetched before the first add.  NP = 0: never unreduced.
+template <int T, int NP, int FK = 0, int FG = 0> __device__ __forceinline__ float hc_x_new(const float* __restrict__ x_in, int in_ss, int in_ts, const float* __restrict__ comb_out, const MoeOut& mo, float w, int d, int ti, int s, int i) {
+  float v = x_in[(size_t)ti * in_ts + (size_t)s * in_ss + i];
+  if constexpr (NP > 1) {
+    float sv[NP];
+#pragma unroll
+    for (int q = 0; q < NP; ++q) sv[q] = (comb_out + ((size_t)q * T + ti) * d)[i];
+    float o = sv[0];
+#pragma unroll
+    for (int q = 1; q < NP; ++q) o += sv[q];
+    v = v + o * w;
+  } else {
+    if (NP == 1 && mo.partial) v = v + moe_out_value<FK, FG>(mo, ti, i) * w;
+    else if (comb_out) v = v + comb_out[(size_t)ti * d + i] * w;
+  }
+  return v;
+}
 
 // x / n for 0 <= x < 2^16, n <= 2^12 with r = 1 / n within two units in the last place: (x + 1/2) / n lies 1 / (2 n) or more off an
 // integer, the product's error is below x / n * 2^-21
@@ -71,3 +92,9 @@ __device__ __forceinline__ float hc_unit_sum(const float* red, int U, int stride
 // the mixes whose straight code the smaller bounds hold: up to four streams of up to sixteen slices in all
 inline bool pyre_hc_few(const HcDev& h, int ksplit) { return h.hc <= 4 && ksplit <= 16; }
 int pyre_hc_up_cols_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, int t, const float* xnew, float eps, float* mixed, float* inj);
+
+// the mixes on the matrix cores (hc_m.hip): whether a mix is one, the slices of its first launch, the two launches
+bool pyre_hc_on_matrix_cores(const HcDev& h);
+int pyre_hc_m_slices(const HcDev& h);
+int pyre_hc_norm_down_m_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const float* x_in, int in_ss, int in_ts, float* x_out, int t, const float* comb_out, int comb_parts, const MoeOut& mo, const float* comb_inj);
+int pyre_hc_up_mix_m_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, int t, const float* xnew, float eps, float* mixed, float* inj, const HcRoute* rt, const AopOut* aop);
