@@ -164,7 +164,7 @@ int pyre_gemv_n_launch(pyre_ctx* ctx, const void* nq, size_t rows, size_t cols, 
 //   co:   rows < ch are the channels of a causal depthwise conv1d (kernel kk, weights conv_w[ch][kk]); the lane that
 //         owns a row runs the window's tokens in order, o = w[kk-1]*cur + sum_j w[j]*state[j], co[t][row] = silu(o),
 //         and slides the row's state conv_in -> conv_out ([kk-1][ch], oldest first; in == out is fine).
-struct GemvEpi { uint32_t* best; const float* conv_w; const float* conv_in; float* conv_out; float* co; int ch, kk; int four_waves; int sq_heads = 0; float sq_eps = 0.0f; int nz = 0; };          // sq_*: PyreAop::sq travels to the kernel here
+struct GemvEpi { uint32_t* best; const float* conv_w; const float* conv_in; float* conv_out; float* co; int ch, kk; int four_waves; int sq_heads = 0; float sq_eps = 0.0f; };          // sq_*: PyreAop::sq travels to the kernel here
 // launchers implemented in qmat.hip, used by the block / model code
 // Matrices in the matrix-core layout (FMT_IQ3_S_M) take their activations as the f16 operand `a` when the caller has one (a
 // producer kernel wrote it); otherwise x_dev is split into the context's operand buffer by one more launch.

@@ -3,6 +3,7 @@
 #pragma once
 #include "common.h"
 #include "iq_codebooks.h"
+#include <utility>
 
 // Device formats.  The first seven keep the GGUF block's own fields; C4 and C8 are what every other supported GGUF
 // type is re-coded into at load: one f32 scale per 16 values (the exact f32 product the reference forms before its
@@ -212,6 +213,10 @@ __device__ __forceinline__ uint32_t c4_lookup(const QMatDev& m, uint32_t codes) 
   uint32_t lo = __builtin_amdgcn_perm(m.lut[1], m.lut[0], i7), hi = __builtin_amdgcn_perm(m.lut[3], m.lut[2], i7);
   return (lo & ~pick) | (hi & pick);
 }
+// The low nibbles of a word's bytes.  The mask sits in a register whose value the compiler does not know: with a literal it rewrites a byte's
+// and-then-convert into a bit-field extraction and a conversion, two instructions a value instead of one and a quarter.
+__device__ __forceinline__ uint32_t nib_mask() { uint32_t k; asm("s_mov_b32 %0, 0x0F0F0F0F" : "=s"(k)); return k; }
+__device__ __forceinline__ float ubyte_f32(uint32_t u, int k) { return (float)((u >> (8 * k)) & 0xFF); }          // v_cvt_f32_ubyte
 template <int FMT, int T> __device__ __forceinline__ void unit_fma(const QMatDev& m, const UnitRaw<FMT>& r, int ku, const uint2* lds2, int lane,
                                                                    const float* __restrict__ xs, int xstride, float (&acc)[T]) {
   if constexpr (FMT == FMT_F32) {
@@ -255,14 +260,13 @@ _Pragma("unroll")
     uint4 hb = r.hb;
     float d = h2f_bits(hb.x), mn = h2f_bits(hb.x >> 16);
     int j = ku & 3; uint32_t s1, m1, s2, m2; scale_min_k4(2 * j, hb.y, hb.z, hb.w, s1, m1); scale_min_k4(2 * j + 1, hb.y, hb.z, hb.w, s2, m2);
-    float d1 = d * (float)s1, M1 = mn * (float)m1, d2 = d * (float)s2, M2 = mn * (float)m2;
+    float d1 = d * (float)s1, M1 = mn * (float)m1, d2 = d * (float)s2, M2 = mn * (float)m2; const uint32_t nk = nib_mask();
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       uint4 v = r.v[c]; uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
-        uint32_t b = (w[k >> 2] >> (8 * (k & 3))) & 0xFF;
-        float lo = fmaf(d1, (float)(b & 0xF), -M1), hi = fmaf(d2, (float)(b >> 4), -M2);
+        float lo = fmaf(d1, ubyte_f32(w[k >> 2] & nk, k & 3), -M1), hi = fmaf(d2, ubyte_f32((w[k >> 2] >> 4) & nk, k & 3), -M2);
 #pragma unroll
         for (int t = 0; t < T; ++t) { acc[t] = fmaf(lo, xs[t * xstride + 16 * c + k], acc[t]); acc[t] = fmaf(hi, xs[t * xstride + 32 + 16 * c + k], acc[t]); }
       }
@@ -361,7 +365,7 @@ _Pragma("unroll")
     float d = h2f_bits(r.s0);
     uint32_t sc = r.s1;
     uint4 v0 = r.v[0], v1 = r.v[1];
-    uint32_t w[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+    uint32_t w[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w}; const uint32_t nk = nib_mask();
     float sx[T][2];            // sub-block sums of the activations: lane j holds x[j], folded inside each half of the wave
 #pragma unroll
     for (int t = 0; t < T; ++t) {
@@ -377,7 +381,7 @@ _Pragma("unroll")
       for (int t = 0; t < T; ++t) part[t] = 0.0f;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        uint32_t u = w[4 * sb + k], lo = u & 0x0F0F0F0Fu, hi = (u >> 4) & 0x0F0F0F0Fu;
+        uint32_t u = w[4 * sb + k], lo = u & nk, hi = (u >> 4) & nk;
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
           float fl = (float)((lo >> (8 * b)) & 0xFF), fh = (float)((hi >> (8 * b)) & 0xFF);
@@ -390,6 +394,123 @@ _Pragma("unroll")
       for (int t = 0; t < T; ++t) acc[t] = fmaf(db, fmaf(-15.0f, sx[t][sb], 2.0f * part[t]), acc[t]);
     }
   }
+}
+// ---- the same sums for several tokens on the matrix cores, bit for bit ---------------------------------------------------------------
+// v_mfma_f32_4x4x1_16b_f32 takes one column at a time: sixteen blocks of four rows of weights (lane = row, as everywhere here) times
+// four tokens, and adds a single fused product to each sum: fmaf(w, x, acc), subnormals included.  So a token's chain of
+// multiply-adds keeps its order and its bits, four tokens in the 8 cycles two multiply-adds take (ten measured, 126 TFLOP/s of f32).
+// The result has the lane's own row in four registers, one a token.  The activations need no shared memory: lane l holds columns
+// 4 (l / 4) .. + 3 of token l % 4 of its group of four (one 16-byte load a unit), and the instruction broadcasts the four lanes of
+// column c, block c / 4, to all rows.
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));          // (a caller's rows may start at any float)
+template <class F, int... I> __device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F> __device__ __forceinline__ void static_for(F&& f) { static_for_((F&&)f, std::make_integer_sequence<int, N>{}); }          // f(0) .. f(N - 1), the index a constant
+template <int NG> struct XGrp { f4u x[NG]; };
+// p[g]: the lane's token of group g, at column 4 (lane / 4)
+template <int NG> __device__ __forceinline__ void unit_x_load(const float* const (&p)[NG], int ku, XGrp<NG>& x) {
+#pragma unroll
+  for (int g = 0; g < NG; ++g) x.x[g] = *(const f4u*)(p[g] + (size_t)ku * 64);
+}
+template <int C, int NG> __device__ __forceinline__ void mma_col(float w, const XGrp<NG>& x, v4f (&a)[NG]) {
+#pragma unroll
+  for (int g = 0; g < NG; ++g) a[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(x.x[g][C & 3], w, a[g], 4, C >> 2, 0);
+}
+// eight columns, the I-th of them C0 + I * CS (PAIR: I / 2 and, for odd I, CS further): their weights are all formed before the first product
+template <int C0, int CS, bool PAIR, int NG, class F> __device__ __forceinline__ void mma_cols8(F&& w, const XGrp<NG>& x, v4f (&a)[NG]) {
+  float wv[8];
+  static_for<8>([&](auto I) { wv[I] = w(I); });
+  __builtin_amdgcn_sched_barrier(0);
+  static_for<8>([&](auto I) { constexpr int i = I; mma_col<PAIR ? C0 + (i >> 1) + (i & 1) * CS : C0 + i * CS>(wv[i], x, a); });
+  __builtin_amdgcn_sched_barrier(0);
+}
+template <int NG> __device__ __forceinline__ void mma_zero(v4f (&a)[NG]) {
+#pragma unroll
+  for (int g = 0; g < NG; ++g) a[g] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+}
+// a[g] = fmaf(s, b[g], a[g])
+template <int NG> __device__ __forceinline__ void mma_scale(float s, const v4f (&b)[NG], v4f (&a)[NG]) {
+#pragma unroll
+  for (int g = 0; g < NG; ++g)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) a[g][t] = fmaf(s, b[g][t], a[g][t]);
+}
+// the activations' sums over stretches of N = 16 or 32 columns, added in unit_fma's order: a lane has its token's sum over the stretch its columns lie in
+template <int N, int NG> __device__ __forceinline__ void x_sums(const XGrp<NG>& x, XGrp<NG>& s) {
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    f4u v = x.x[g];
+#pragma unroll
+    for (int o = N / 2; o >= 4; o >>= 1)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] += __shfl_xor(v[j], o);
+    const float t = (v[0] + v[2]) + (v[1] + v[3]);
+    s.x[g] = f4u{t, t, t, t};
+  }
+}
+// a[g] += the unit's 64 columns of the lane's row times the tokens of group g: unit_fma's operations in its order
+template <int FMT, int NG> __device__ __forceinline__ void unit_mma(const QMatDev& m, const UnitRaw<FMT>& r, int ku, const XGrp<NG>& x, v4f (&a)[NG]) {
+  constexpr int V = sizeof(r.v) / sizeof(uint4); uint32_t w[4 * V];          // (indexed by constants only: registers)
+#pragma unroll
+  for (int c = 0; c < V; ++c) { w[4 * c] = r.v[c].x; w[4 * c + 1] = r.v[c].y; w[4 * c + 2] = r.v[c].z; w[4 * c + 3] = r.v[c].w; }
+  if constexpr (FMT == FMT_F32) {
+    static_for<8>([&](auto C) { constexpr int c = C; mma_cols8<8 * c, 1, false>([&](int i) { return __uint_as_float(w[8 * c + i]); }, x, a); });
+  } else if constexpr (FMT == FMT_F16 || FMT == FMT_BF16) {
+    static_for<8>([&](auto C) { constexpr int c = C; mma_cols8<8 * c, 1, false>([&](int i) { const uint32_t v = w[4 * c + (i >> 1)]; return FMT == FMT_F16 ? h2f_bits(i & 1 ? v >> 16 : v) : __uint_as_float(i & 1 ? v & 0xFFFF0000u : v << 16); }, x, a); });
+  } else if constexpr (FMT == FMT_Q8_0 || FMT == FMT_C8) {
+    constexpr int B = FMT == FMT_Q8_0 ? 32 : 16;          // columns a scale
+    static_for<64 / B>([&](auto Bk) { constexpr int b = Bk; v4f part[NG]; mma_zero(part);
+      static_for<B / 8>([&](auto K) { constexpr int k = b * (B / 8) + K; mma_cols8<8 * k, 1, false>([&](int i) { return (float)(int)(int8_t)(w[2 * k + (i >> 2)] >> (8 * (i & 3))); }, x, part); });
+      float s;
+      if constexpr (FMT == FMT_Q8_0) s = h2f_bits(r.s0 >> (16 * b)); else s = __uint_as_float(b == 0 ? r.hb.x : b == 1 ? r.hb.y : b == 2 ? r.hb.z : r.hb.w);
+      mma_scale(s, part, a); });
+    if constexpr (FMT == FMT_C8) if (m.ty == PYRE_Q5_K) {          // the offsets leave through the groups' activation sums
+      XGrp<NG> sx; x_sums<16>(x, sx);
+      mma_col<0>(-__uint_as_float(r.hb2.x), sx, a); mma_col<16>(-__uint_as_float(r.hb2.y), sx, a); mma_col<32>(-__uint_as_float(r.hb2.z), sx, a); mma_col<48>(-__uint_as_float(r.hb2.w), sx, a);
+    }
+  } else if constexpr (FMT == FMT_Q4_K) {
+    const uint4 hb = r.hb; const float d = h2f_bits(hb.x), mn = h2f_bits(hb.x >> 16);
+    const int j = ku & 3; uint32_t s1, m1, s2, m2; scale_min_k4(2 * j, hb.y, hb.z, hb.w, s1, m1); scale_min_k4(2 * j + 1, hb.y, hb.z, hb.w, s2, m2);
+    const float d1 = d * (float)s1, M1 = mn * (float)m1, d2 = d * (float)s2, M2 = mn * (float)m2; const uint32_t nk = nib_mask();
+    static_for<8>([&](auto K) { constexpr int k = K; const uint32_t lo = w[k] & nk, hi = (w[k] >> 4) & nk;
+      mma_cols8<4 * k, 32, true>([&](int i) { return i & 1 ? fmaf(d2, ubyte_f32(hi, i >> 1), -M2) : fmaf(d1, ubyte_f32(lo, i >> 1), -M1); }, x, a); });
+  } else if constexpr (FMT == FMT_IQ2_XS) {
+    const float d = h2f_bits(r.s0);
+    XGrp<NG> sx; x_sums<16>(x, sx);
+    static_for<4>([&](auto G) { constexpr int g = G; v4f part[NG]; mma_zero(part);
+      const uint32_t S = g >> 1 ? r.hb.y : r.hb.x; uint32_t bv[4];
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) { const int k = rr + 4 * (g & 1); const uint32_t idx4 = (w[g] >> (2 * rr)) & 0x03030303u, sgn = k >= 2 ? S >> (k - 2) : S << (2 - k); bv[rr] = __builtin_amdgcn_perm(PYRE_IQ2_THI, PYRE_IQ2_TLO, (sgn & 0x04040404u) | idx4); }
+      static_for<2>([&](auto K) { constexpr int k = K; mma_cols8<16 * g + 8 * k, 1, false>([&](int i) { return ubyte_f32(bv[2 * k + (i >> 2)], i & 3); }, x, part); });
+      mma_col<16 * g>(-43.0f, sx, part);
+      mma_scale(d * (0.5f + (float)((r.s1 >> (4 * g)) & 0xF)) * 0.25f, part, a); });
+  } else if constexpr (FMT == FMT_C4) {
+    XGrp<NG> sx; x_sums<16>(x, sx); const float nbias = -(float)m.bias;
+    static_for<4>([&](auto G) { constexpr int g = G; v4f part[NG]; mma_zero(part);
+      static_for<2>([&](auto K) { constexpr int k = 2 * g + K; const uint32_t lo = c4_lookup(m, w[k] & 0x0F0F0F0Fu), hi = c4_lookup(m, (w[k] >> 4) & 0x0F0F0F0Fu);
+        mma_cols8<8 * k, 1, false>([&](int i) { return ubyte_f32(i & 1 ? hi : lo, i >> 1); }, x, part); });
+      mma_col<16 * g>(nbias, sx, part);
+      mma_scale(__uint_as_float(g == 0 ? r.hb.x : g == 1 ? r.hb.y : g == 2 ? r.hb.z : r.hb.w), part, a); });
+  } else {          // IQ3_S
+    const float d = h2f_bits(r.s0); const uint32_t nk = nib_mask();
+    XGrp<NG> sx; x_sums<32>(x, sx);
+    static_for<2>([&](auto S) { constexpr int sb = S; v4f part[NG]; mma_zero(part);
+      static_for<4>([&](auto K) { constexpr int k = 4 * sb + K; const uint32_t lo = w[k] & nk, hi = (w[k] >> 4) & nk;
+        mma_cols8<8 * k, 1, false>([&](int i) { return ubyte_f32(i & 1 ? hi : lo, i >> 1); }, x, part); });
+#pragma unroll
+      for (int g = 0; g < NG; ++g) part[g] = part[g] + part[g];
+      mma_col<32 * sb>(-15.0f, sx, part);
+      mma_scale(d * (float)(1 + 2 * ((r.s1 >> (4 * sb)) & 0xF)), part, a); });
+  }
+}
+// one of two matrices, what unit_load and unit_mma read of it, field by field: a reference chosen at run time would send the kernel's arguments through scratch memory
+__device__ __forceinline__ QMatDev pick_mat(bool first, const QMatDev& a, const QMatDev& b) {
+  QMatDev m{};
+  m.p0 = first ? a.p0 : b.p0; m.p1 = first ? a.p1 : b.p1; m.p2 = first ? a.p2 : b.p2; m.p3 = first ? a.p3 : b.p3; m.pb = first ? a.pb : b.pb;
+  m.U = first ? a.U : b.U; m.ty = first ? a.ty : b.ty; m.bias = first ? a.bias : b.bias;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) m.lut[i] = first ? a.lut[i] : b.lut[i];
+  return m;
 }
 template <int FMT, int T> __device__ __forceinline__ void unit_dot(const QMatDev& m, const uint2* lds2, int tile, int ku, int lane,
                                                                    const float* __restrict__ xs, int xstride, float (&acc)[T]) {

@@ -6,7 +6,6 @@
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 // What a wave fetches for one chunk: from the matrix (memory) its row groups' codes and super-block headers, from the
 // operand (second-level cache) the sixteen activation rows and their scale factors.

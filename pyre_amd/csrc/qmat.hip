@@ -1,6 +1,8 @@
 // Quantized matrix operator: GGUF blocks -> lane=row planes (repack), bit-exact dequant export, dequant-GEMV.
 // Drop-in for QMat / QMat::matmul of the reference (src/model/gguf_q.rs:201-247).
 #include "formats.h"
+#include <algorithm>
+#include <vector>
 #include <stdlib.h>
 PYRE_TS_DECL(qmat_ts) PYRE_TS_EXPORT(qmat_ts, pyre_debug_ts_qmat)
 
@@ -214,9 +216,12 @@ template <int FMT> __global__ __launch_bounds__(64) void k_rows(QMatDev m, const
 //                slice order (no in-kernel cross-workgroup reduction: a device-scope fence per workgroup costs about a
 //                microsecond of serialized L2 write-back per XCD on this part).
 //   best != nullptr (T == 1, ksplit == 1): best[2*tile] = bits of the tile's maximum, best[2*tile+1] = its first row.
+// A group of four tokens costs ten cycles a column on the matrix cores, a token four on the vector pipe: from four tokens on.  (Two and
+// three of a 6144 x 2048 Q4_K matrix on the matrix cores: 8.1 us, on the vector pipe 6.0 and 6.7.)
+#define PYRE_MMA_MIN 4
 template <int FMT, int T, int NW>
 __global__ __launch_bounds__(NW * 64) void k_gemv(QMatDev m, const float* __restrict__ x, float* __restrict__ y, int upw,
-                                                  GemvEpi ep, const uint2* __restrict__ g2) {
+                                                  GemvEpi ep, int tn) {
   const uint2* lds2 = nullptr;          // no format needs a codebook in shared memory any more
   PYRE_TS_VARS PYRE_TS(0);
   __shared__ float red[NW][T][64];
@@ -229,7 +234,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemv(QMatDev m, const float* __rest
 #pragma unroll
     for (int k = 0; k < 8; ++k) { cw[k] = k < ep.kk ? ep.conv_w[row * ep.kk + k] : 0.0f; chist[k] = k < ep.kk - 1 ? ep.conv_in[(size_t)k * ep.ch + row] : 0.0f; }
   }
-  if (blockIdx.z) { x += (size_t)blockIdx.z * T * m.cols; y += (size_t)blockIdx.z * T * (ksplit == 1 ? (size_t)m.rows : (size_t)ksplit * m.tiles * 64); }          // (a further group of T tokens: pyre_gemv_rows_launch)
+  const int t0 = blockIdx.z * T, nt = min(T, tn - t0); x += (size_t)t0 * m.cols;          // a window of tn tokens on several workgroups (gemv_f)
   const int k0 = (ks * NW + wave) * upw; const int k1 = min(m.U, k0 + upw);
   float acc[T];
 #pragma unroll
@@ -240,12 +245,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemv(QMatDev m, const float* __rest
     // measured slower: 4.2 against 2.3 us for a 2048-column projection -- 64 shared-memory reads per unit and vector
     // operands cost more than the units' scalar round trips save.)
     for (int ku = k0; ku < k1; ++ku) unit_dot<FMT, T>(m, lds2, tile, ku, lane, x + (size_t)ku * 64, m.cols, acc);
-  } else {
-    // Several tokens: T x 64 activations per unit do not fit the scalar registers, and scalar loads in pieces cost one
-    // memory round trip per piece.  Each wave stages the activations of two units at a time in its own slice of shared
-    // memory ([token][unit][64], vector loads issued together with the units' weights) and takes them from there; a
-    // wave's shared-memory operations execute in order, so no workgroup barrier is involved.  The arithmetic per token
-    // is the single-token sequence.
+  } else if constexpr (T < PYRE_MMA_MIN) {
     extern __shared__ __align__(16) float xsm[];
     float* xw = xsm + (size_t)wave * (2 * 64 * T);
     for (int ku = k0; ku < k1; ku += 2) {
@@ -253,7 +253,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemv(QMatDev m, const float* __rest
       UnitRaw<FMT> r0 = unit_load<FMT>(m, tile, ku, lane), r1 = unit_load<FMT>(m, tile, two ? ku + 1 : ku, lane);
       float xa[T], xb[T];
 #pragma unroll
-      for (int t = 0; t < T; ++t) { xa[t] = x[(size_t)t * m.cols + (size_t)ku * 64 + lane]; xb[t] = x[(size_t)t * m.cols + (size_t)(two ? ku + 1 : ku) * 64 + lane]; }
+      for (int t = 0; t < T; ++t) { const float* xt = x + (size_t)min(t, nt - 1) * m.cols + lane; xa[t] = xt[(size_t)ku * 64]; xb[t] = xt[(size_t)(two ? ku + 1 : ku) * 64]; }
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int t = 0; t < T; ++t) { xw[(t * 2 + 0) * 64 + lane] = xa[t]; xw[(t * 2 + 1) * 64 + lane] = xb[t]; }
@@ -262,19 +262,36 @@ __global__ __launch_bounds__(NW * 64) void k_gemv(QMatDev m, const float* __rest
       if (two) unit_fma<FMT, T>(m, r1, ku + 1, lds2, lane, xw + 64, 128, acc);
       __builtin_amdgcn_wave_barrier();
     }
+  } else {
+    // Several tokens: the same chains of multiply-adds on the matrix cores, four tokens at a time (unit_mma), two units of
+    // weights and activations fetched at once.  Five and eight tokens of 49 152 x 2048, us, multiply-adds / matrix cores: Q6_K 36.0 / 27.5 and
+    // 45.9 / 27.9, IQ4_XS 38.2 / 30.9 and 46.5 / 31.1, Q5_K 45.2 / 34.9 and 58.1 / 35.3; four of Q6_K 28.5 / 24.6 (its bytes' time), IQ4_XS 27.1 / 24.3.
+    constexpr int NG = (T + 3) / 4;
+    const float* xp[NG]; v4f a[NG]; mma_zero(a);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) xp[g] = x + (size_t)min(4 * g + (lane & 3), nt - 1) * m.cols + 4 * (lane >> 2);          // (a group's missing tokens repeat the last one; nobody reads their sums)
+    for (int ku = k0; ku < k1; ku += 2) {
+      const bool two = ku + 1 < k1; const int kv = two ? ku + 1 : ku;
+      const UnitRaw<FMT> r0 = unit_load<FMT>(m, tile, ku, lane); XGrp<NG> x0, x1; unit_x_load(xp, ku, x0);
+      const UnitRaw<FMT> r1 = unit_load<FMT>(m, tile, kv, lane); unit_x_load(xp, kv, x1);
+      unit_mma<FMT, NG>(m, r0, ku, x0, a);
+      if (two) unit_mma<FMT, NG>(m, r1, kv, x1, a);
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) acc[t] = a[t >> 2][t & 3];
   }
 #pragma unroll
   for (int t = 0; t < T; ++t) red[wave][t][lane] = acc[t];
   PYRE_TS(1);
   lds_barrier(); PYRE_TS(2);
   const size_t r64 = (size_t)m.tiles * 64;
-  for (int i = threadIdx.x; i < T * 64; i += NW * 64) {
+  for (int i = threadIdx.x; i < nt * 64; i += NW * 64) {
     int t = i >> 6, l = i & 63; float s = red[0][t][l];
 #pragma unroll
     for (int w = 1; w < NW; ++w) s += red[w][t][l];
     size_t row = (size_t)tile * 64 + l;
-    if (ksplit == 1) { if (row < (size_t)m.rows) y[(size_t)t * m.rows + row] = s; }
-    else y[((size_t)ks * T + t) * r64 + row] = s;
+    if (ksplit == 1) { if (row < (size_t)m.rows) y[(size_t)(t0 + t) * m.rows + row] = s; }
+    else y[((size_t)ks * tn + t0 + t) * r64 + row] = s;
     if (T == 1 && ep.best != nullptr) {       // threads 0..63 = wave 0: first maximum of the tile (sampler::argmax order)
       float bv = row < (size_t)m.rows ? s : -INFINITY; uint32_t bi = (uint32_t)row;
 #pragma unroll
@@ -306,6 +323,47 @@ __global__ __launch_bounds__(NW * 64) void k_gemv(QMatDev m, const float* __rest
   PYRE_TS(3); PYRE_TS_FLUSH(qmat_ts, (NW == 16 ? 0 : (gridDim.y > 1 ? 8 : 16)));
 }
 
+// ---- the same for a prompt's tokens ------------------------------------------------------------------------------------------------
+// grid (tiles, ksplit, groups of sixteen tokens): what k_gemv forms for a window, for sixteen tokens at once: a weight is decoded once
+// for them.  k_gemv's K slice is cut into SH shares of upw units, one a wave there; here a wave takes SW of them side by side (their
+// chains are independent, their loads all in flight) and the shares meet in order, so a token has a window's bits.  rows8: eight-token
+// groups in x (a multiple of eight rows readable), y [token][rows], or with ksplit > 1 [group of eight][slice][8][tiles * 64].
+// Two workgroups of eight waves a compute unit: one's products cover the other's fetches.
+template <int FMT, int SH>
+__global__ __launch_bounds__(SH == 4 ? 256 : 512, SH == 4 ? 2 : 4) void k_gemv_blk(QMatDev m, const float* __restrict__ x, float* __restrict__ y, int upw, int rows8) {
+  constexpr int SW = SH == 16 ? 2 : 1, NW = SH / SW, NG = 4;
+  __shared__ float red[SH][16][64];
+  const int tile = blockIdx.x, ks = blockIdx.y, ksplit = gridDim.y, t0 = blockIdx.z * 16, nt = min(16, rows8 * 8 - t0);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const float* xp[NG]; v4f a[SW][NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) xp[g] = x + (size_t)(t0 + min(4 * g + (lane & 3), nt - 1)) * m.cols + 4 * (lane >> 2);
+#pragma unroll
+  for (int i = 0; i < SW; ++i) mma_zero(a[i]);
+  const int s0 = ks * SH + wave * SW;
+  for (int it = 0; it < upw; ++it) {
+    UnitRaw<FMT> r[SW]; XGrp<NG> xr[SW];
+#pragma unroll
+    for (int i = 0; i < SW; ++i) { const int ku = min((s0 + i) * upw + it, m.U - 1); r[i] = unit_load<FMT>(m, tile, ku, lane); unit_x_load(xp, ku, xr[i]); }
+#pragma unroll
+    for (int i = 0; i < SW; ++i) { const int ku = (s0 + i) * upw + it; if (ku < m.U) unit_mma<FMT, NG>(m, r[i], ku, xr[i], a[i]); }
+  }
+#pragma unroll
+  for (int i = 0; i < SW; ++i)
+#pragma unroll
+    for (int t = 0; t < 16; ++t) red[wave * SW + i][t][lane] = a[i][t >> 2][t & 3];
+  lds_barrier();
+  const size_t r64 = (size_t)m.tiles * 64;
+  for (int i = threadIdx.x; i < nt * 64; i += NW * 64) {
+    const int t = i >> 6, l = i & 63; float s = red[0][t][l];
+#pragma unroll
+    for (int w = 1; w < SH; ++w) s += red[w][t][l];
+    const size_t row = (size_t)tile * 64 + l;
+    if (ksplit == 1) { if (row < (size_t)m.rows) y[(size_t)(t0 + t) * m.rows + row] = s; }
+    else y[(((size_t)((t0 + t) >> 3) * ksplit + ks) * 8 + (t & 7)) * r64 + row] = s;
+  }
+}
+
 namespace {
 int env_int(const char* n, int dflt) { const char* v = getenv(n); return v && *v ? atoi(v) : dflt; }
 
@@ -318,27 +376,36 @@ int gemv_nw(const QMatDev& m, int ksplit) {
   if (force == 4 || force == 8 || force == 16) nw = force;
   return nw;
 }
-template <int FMT, int T, int NW> int gemv_launch_nw(pyre_ctx* ctx, const QMatDev& m, const float* x, float* y, int ksplit, const GemvEpi& ep) {
+template <int FMT, int T, int NW> int gemv_launch_nw(pyre_ctx* ctx, const QMatDev& m, const float* x, int tn, float* y, int ksplit, const GemvEpi& ep) {
   int per_wg = (m.U + ksplit - 1) / ksplit, upw = (per_wg + NW - 1) / NW; if (upw < 1) upw = 1;
   static const char* fn[FMT_COUNT] = {"f32", "f16", "bf16", "q8_0", "q4_k", "iq2_xs", "iq3_s", "c4", "c8", "iq3_s", "q4_k", "iq2_xs", "q8_0"};
-  static const std::string name = std::string("gemv_") + fn[FMT] + "_t" + std::to_string(T);
-  ProfScope ps(ctx, name.c_str(), qmat_gguf_bytes(m, m.rows) + 4.0 * T * ((double)m.cols + m.rows));
-  hipLaunchKernelGGL((k_gemv<FMT, T, NW>), dim3(m.tiles, ksplit, ep.nz > 1 ? ep.nz : 1), dim3(NW * 64), T > 1 ? (size_t)NW * 2 * 64 * T * 4 : 0, ctx->stream, m, x, y, upw, ep, (const uint2*)ctx->d_iq2xs);
+  static const std::vector<std::string> names = [] { std::vector<std::string> v; for (int t = 0; t <= 8; ++t) v.push_back(std::string("gemv_") + fn[FMT] + "_t" + std::to_string(t)); return v; }();
+  ProfScope ps(ctx, names[tn].c_str(), qmat_gguf_bytes(m, m.rows) + 4.0 * tn * ((double)m.cols + m.rows));
+  hipLaunchKernelGGL((k_gemv<FMT, T, NW>), dim3(m.tiles, ksplit, (tn + T - 1) / T), dim3(NW * 64), T > 1 && T < PYRE_MMA_MIN ? (size_t)NW * 2 * 64 * T * 4 : 0, ctx->stream, m, x, y, upw, ep, tn);
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
 // Waves per workgroup: enough that a row tile's whole K range is covered by one workgroup with few units per wave,
-// fewer when there are so many tiles that the chip is full anyway.
-template <int FMT, int T> int gemv_t(pyre_ctx* ctx, const QMatDev& m, const float* x, float* y, int ksplit, const GemvEpi& ep) {
+// fewer when there are so many tiles that the chip is full anyway.  T tokens a workgroup, tn in all.
+template <int FMT, int T> int gemv_t(pyre_ctx* ctx, const QMatDev& m, const float* x, int tn, float* y, int ksplit, const GemvEpi& ep) {
   int nw = ep.four_waves ? 4 : gemv_nw(m, ksplit);
-  if (nw == 4) return gemv_launch_nw<FMT, T, 4>(ctx, m, x, y, ksplit, ep);
-  if (nw == 8) return gemv_launch_nw<FMT, T, 8>(ctx, m, x, y, ksplit, ep);
-  return gemv_launch_nw<FMT, T, 16>(ctx, m, x, y, ksplit, ep);
+  if (nw == 4) return gemv_launch_nw<FMT, T, 4>(ctx, m, x, tn, y, ksplit, ep);
+  if (nw == 8) return gemv_launch_nw<FMT, T, 8>(ctx, m, x, tn, y, ksplit, ep);
+  return gemv_launch_nw<FMT, T, 16>(ctx, m, x, tn, y, ksplit, ep);
+}
+// The tokens of a window a workgroup takes.  A launch of few row tiles leaves most compute units idle while each tile's workgroup
+// works through all of the window's tokens: there the tokens are spread over up to 256 workgroups, which read the same weights
+// out of the caches; the fewest tokens a workgroup that fit.  Eight tokens, us, one workgroup a tile / spread: 2048 x 2048 Q4_K 13.7 / 5.3, Q8_0
+// 11.4 / 4.7, IQ4_XS 14.7 / 6.3; 6144 x 2048 14.2 / 7.4, 12.2 / 8.1, 15.1 / 9.2.
+int gemv_tokens(const QMatDev& m, int t, int ksplit, const GemvEpi& ep) {
+  if (ep.best || ep.co) return t;          // (the epilogues walk a tile's tokens)
+  for (int tp = 1; tp < t && tp <= 4; tp *= 2) if (m.tiles * ksplit * ((t + tp - 1) / tp) <= 256) return tp;
+  return t;
 }
 template <int FMT> int gemv_f(pyre_ctx* ctx, const QMatDev& m, const float* x, int t, float* y, int ksplit, const GemvEpi& ep) {
-  switch (t) { case 1: return gemv_t<FMT, 1>(ctx, m, x, y, ksplit, ep); case 2: return gemv_t<FMT, 2>(ctx, m, x, y, ksplit, ep); case 3: return gemv_t<FMT, 3>(ctx, m, x, y, ksplit, ep);
-    case 4: return gemv_t<FMT, 4>(ctx, m, x, y, ksplit, ep); case 5: return gemv_t<FMT, 5>(ctx, m, x, y, ksplit, ep); case 6: return gemv_t<FMT, 6>(ctx, m, x, y, ksplit, ep);
-    case 7: return gemv_t<FMT, 7>(ctx, m, x, y, ksplit, ep); case 8: return gemv_t<FMT, 8>(ctx, m, x, y, ksplit, ep); }
-  return pyre_fail(ctx, PYRE_E_ARG, "qmatmul: t = %d outside 1..8", t);
+  if (t < 1 || t > 8) return pyre_fail(ctx, PYRE_E_ARG, "qmatmul: t = %d outside 1..8", t);
+  switch (gemv_tokens(m, t, ksplit, ep)) { case 1: return gemv_t<FMT, 1>(ctx, m, x, t, y, ksplit, ep); case 2: return gemv_t<FMT, 2>(ctx, m, x, t, y, ksplit, ep); case 3: return gemv_t<FMT, 3>(ctx, m, x, t, y, ksplit, ep);
+    case 4: return gemv_t<FMT, 4>(ctx, m, x, t, y, ksplit, ep); case 5: return gemv_t<FMT, 5>(ctx, m, x, t, y, ksplit, ep); case 6: return gemv_t<FMT, 6>(ctx, m, x, t, y, ksplit, ep);
+    case 7: return gemv_t<FMT, 7>(ctx, m, x, t, y, ksplit, ep); default: return gemv_t<FMT, 8>(ctx, m, x, t, y, ksplit, ep); }
 }
 #define FMT_DISPATCH(fmt, CALL) \
   switch (fmt) { case FMT_F32: { constexpr int F = FMT_F32; CALL; } break; case FMT_F16: { constexpr int F = FMT_F16; CALL; } break; case FMT_BF16: { constexpr int F = FMT_BF16; CALL; } break; \
@@ -372,9 +439,12 @@ int pyre_gemv_launch(pyre_ctx* ctx, const QMatDev& m, const float* x, int t, flo
 }
 int pyre_gemv_rows_launch(pyre_ctx* ctx, const QMatDev& m, const float* x, int groups, float* y, int parts) {
   if (m.fmt == FMT_IQ3_S_M || groups < 1 || groups > 65535 || !(parts == 1 || (parts == PYRE_GEMV_PARTS && pyre_gemv_parts_ok(m)))) return pyre_fail(ctx, PYRE_E_ARG, "gemv: %d groups of rows in %d parts", groups, parts);
-  GemvEpi ep{}; ep.nz = groups; ep.four_waves = parts > 1; int rc = PYRE_OK;
-  FMT_DISPATCH(m.fmt, rc = (gemv_t<F, 8>(ctx, m, x, y, parts, ep)));
-  return rc;
+  const int sh = parts > 1 ? 4 : gemv_nw(m, parts), per = (m.U + parts - 1) / parts, upw = std::max(1, (per + sh - 1) / sh);          // k_gemv's shares
+  ProfScope ps(ctx, "gemv_rows", qmat_gguf_bytes(m, m.rows) + 4.0 * groups * 8 * ((double)m.cols + m.rows));
+#define ROWS_GO(SH) hipLaunchKernelGGL((k_gemv_blk<F, SH>), dim3(m.tiles, parts, (groups + 1) / 2), dim3(SH == 4 ? 256 : 512), 0, ctx->stream, m, x, y, upw, groups)
+  FMT_DISPATCH(m.fmt, if (sh == 4) ROWS_GO(4); else if (sh == 8) ROWS_GO(8); else ROWS_GO(16));
+#undef ROWS_GO
+  PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
 int pyre_gemv_split_launch(pyre_ctx* ctx, const QMatDev& m, const float* x, int t, float* partial, int ksplit, const PyreAop* a) {
   if (m.fmt == FMT_IQ3_S_M) return gemm_m_from_f32(ctx, m, x, t, partial, ksplit, GemvEpi{}, a);
@@ -599,26 +669,38 @@ int pyre_qmat_row(pyre_ctx* ctx, const pyre_qmat* m, size_t row, float* out_host
 
 // The operator's own launch: an IQ3_S matrix goes through the matrix-core GEMM (for every t, so a token's result does not
 // depend on the window width); f32_path (or PYRE_QMATMUL_F32=1) takes the f32 lane = row GEMV the model's expert matrices use.
-static bool qmat_small_one_token(const pyre_qmat* m, int t) {
-  const int on = env_int("PYRE_QMATMUL_SMALL", 1);          // read at every call: tests switch it to reach the native-format kernel with small shapes
-  return on && t == 1 && m->dvm.fmt == FMT_IQ3_S_M && m->base != nullptr && m->dv.fmt == FMT_IQ3_S && m->dv.tiles <= 128;
+// Whether a call stays on the lane = row GEMV although the matrix has another kernel: that is one launch, without a second for the
+// activations.  One token: its fused products cost with the 64-column units of the matrix' row tiles, the native-format kernel costs some 4 us
+// more to begin with and less a unit (us, this kernel first, 2048 columns: IQ3_S 12 288 rows 5.5 / 9.7, 49 152 14.5 / 15.8, 151 936 33.3 / 33.8;
+// IQ2_XS 12 288 7.0 / 9.8, 49 152 15.0 / 15.6, 151 936 39.2 / 34.0; Q4_K 12 288 6.6 / 9.1, 49 152 14.9 / 15.6, 151 936 40.3 / 36.1; 30 000 x 4096 IQ2_XS
+// 20.0 / 18.4, Q4_K 18.6 / 19.8), and its sums are nearer the exact ones (2.1 - 3.0e-7 for 5.5 - 6.4e-7).  Windows: matrices of at most 128 row tiles
+// except IQ3_S, whatever the width, so that a token's bits do not depend on it; above, the matrix cores' sums are nearer (1.2e-7 for 3e-7).
+// PYRE_QMATMUL_SMALL=0 (read at every call: tests reach the other kernels with small shapes): never.
+static bool qmat_rows_call(const pyre_qmat* m, int t) {
+  if (m->base == nullptr) return false;
+  const int64_t units = (int64_t)m->dv.tiles * m->dv.U; bool rows;
+  switch (m->dv.fmt) {
+    case FMT_IQ3_S: rows = t == 1 && units <= 49152; break;
+    case FMT_IQ2_XS: rows = t == 1 ? units <= 24576 : m->dv.tiles <= 128; break;
+    case FMT_Q4_K: rows = t == 1 ? units <= 32768 : m->dv.tiles <= 128; break;
+    case FMT_Q8_0: rows = t == 1 || m->dv.tiles <= 128; break;
+    default: return false;
+  }
+  return rows && env_int("PYRE_QMATMUL_SMALL", 1);
 }
 static int qmatmul_launch(pyre_ctx* ctx, const pyre_qmat* m, const float* x_dev, int t, float* y_dev, bool f32_path) {
   static const int f32_only = env_int("PYRE_QMATMUL_F32", 0), native = env_int("PYRE_QMATMUL_NATIVE", 1);
-  // one token of a small IQ3_S matrix (at most 128 row tiles): the lane = row f32 GEMV -- one launch where the other two
-  // paths need a second one for the activations, and a call of this size is its launches, not its bytes
-  if (qmat_small_one_token(m, t) && !f32_path && !f32_only) return pyre_gemv_launch(ctx, m->dv, x_dev, t, y_dev);
+  if (!f32_path && !f32_only && qmat_rows_call(m, t)) return pyre_gemv_launch(ctx, m->dv, x_dev, t, y_dev);
   // one token of an IQ3_S matrix: the kernel that streams the file's 3.44 bit/weight (PYRE_QMATMUL_NATIVE=0: the matrix cores as for a window)
-  // (IQ2_XS and Q4_K have the same kernel over their own layouts, 2.5 and 4.5 bit/weight; a small matrix of them stays with the one-launch f32 GEMV likewise)
+  // (IQ2_XS and Q4_K have the same kernel over their own layouts, 2.5 and 4.5 bit/weight)
   const bool rows_only = m->dv.fmt == FMT_IQ2_XS || m->dv.fmt == FMT_Q4_K;          // (the formats without a matrix-core layout)
-  if (t == 1 && m->base_n && native && !f32_path && !f32_only && !(rows_only && m->dv.tiles <= 128 && env_int("PYRE_QMATMUL_SMALL", 1))) return pyre_gemv_n_launch(ctx, m->base_n, m->rows, m->cols, x_dev, y_dev, nullptr, rows_only ? m->dv.fmt : FMT_IQ3_S);
-  // a window of a large Q4_K matrix: the matrix cores, where eight tokens cost what two do (PYRE_QMATMUL_Q4M=0: the lane = row GEMV);
-  // small matrices stay with the one-launch GEMV, as above
-  if (t >= 2 && env_int("PYRE_QMATMUL_Q4M", 1) && m->dvm.fmt == FMT_Q4_K_M && m->dvm.mq && !f32_path && !f32_only && !(m->dv.tiles <= 128 && env_int("PYRE_QMATMUL_SMALL", 1))) return pyre_gemm_q4_launch(ctx, m->dvm, x_dev, t, y_dev);
+  if (t == 1 && m->base_n && native && !f32_path && !f32_only) return pyre_gemv_n_launch(ctx, m->base_n, m->rows, m->cols, x_dev, y_dev, nullptr, rows_only ? m->dv.fmt : FMT_IQ3_S);
+  // a window of a large Q4_K matrix: the matrix cores, where eight tokens cost what two do (PYRE_QMATMUL_Q4M=0: the lane = row GEMV)
+  if (t >= 2 && env_int("PYRE_QMATMUL_Q4M", 1) && m->dvm.fmt == FMT_Q4_K_M && m->dvm.mq && !f32_path && !f32_only) return pyre_gemm_q4_launch(ctx, m->dvm, x_dev, t, y_dev);
   // a window of a large Q8_0 matrix likewise (PYRE_QMATMUL_Q8M=0: the lane = row GEMV)
-  if (t >= 2 && env_int("PYRE_QMATMUL_Q8M", 1) && m->dvm.fmt == FMT_Q8_0_M && m->dvm.mq && !f32_path && !f32_only && !(m->dv.tiles <= 128 && env_int("PYRE_QMATMUL_SMALL", 1))) return pyre_gemm_q8_launch(ctx, m->dvm, x_dev, t, y_dev);
+  if (t >= 2 && env_int("PYRE_QMATMUL_Q8M", 1) && m->dvm.fmt == FMT_Q8_0_M && m->dvm.mq && !f32_path && !f32_only) return pyre_gemm_q8_launch(ctx, m->dvm, x_dev, t, y_dev);
   // a window of a large IQ2_XS matrix likewise (PYRE_QMATMUL_Q2M=0: the lane = row GEMV)
-  if (t >= 2 && env_int("PYRE_QMATMUL_Q2M", 1) && m->dvm.fmt == FMT_IQ2_XS_M && m->dvm.mq && !f32_path && !f32_only && !(m->dv.tiles <= 128 && env_int("PYRE_QMATMUL_SMALL", 1))) return pyre_gemm_q2_launch(ctx, m->dvm, x_dev, t, y_dev);
+  if (t >= 2 && env_int("PYRE_QMATMUL_Q2M", 1) && m->dvm.fmt == FMT_IQ2_XS_M && m->dvm.mq && !f32_path && !f32_only) return pyre_gemm_q2_launch(ctx, m->dvm, x_dev, t, y_dev);
   const bool has_m = m->dvm.fmt == FMT_IQ3_S_M && m->dvm.mq, has_rows = m->base != nullptr;
   if (has_m && (!has_rows || (!f32_path && !f32_only))) { GemvEpi ep{}; ep.four_waves = pyre_gemm_op_nw(m->dvm, true) == 4; return gemm_m_from_f32(ctx, m->dvm, x_dev, t, y_dev, 1, ep, nullptr); }
   return pyre_gemv_launch(ctx, m->dv, x_dev, t, y_dev);
@@ -646,15 +728,16 @@ int pyre_qmatmul_static_dev(pyre_ctx* ctx, const pyre_qmat* m, const float* x_de
   if (t < 1 || t > 8) return pyre_fail(ctx, PYRE_E_ARG, "pyre_qmatmul_static_dev: t = %d outside 1..8", t);
   if ((m->dv.fmt == FMT_IQ2_XS || m->dv.fmt == FMT_Q4_K) && m->base_n) {      // IQ2_XS, Q4_K: only the single token of a large matrix uses scratch (the native-format kernel's activation digits)
     if (m->cols > PYRE_QMATMUL_STATIC_MAX_COLS) return pyre_fail(ctx, PYRE_E_SHAPE, "pyre_qmatmul_static_dev: %zu columns exceed the static scratch of %d columns; use pyre_qmatmul_dev", m->cols, PYRE_QMATMUL_STATIC_MAX_COLS);
-    if (t == 1 && env_int("PYRE_QMATMUL_NATIVE", 1) && !env_int("PYRE_QMATMUL_F32", 0) && !(m->dv.tiles <= 128 && env_int("PYRE_QMATMUL_SMALL", 1))) {
+    if (qmat_rows_call(m, t)) return pyre_gemv_launch(ctx, m->dv, x_dev, t, y_dev);          // as pyre_qmatmul_dev (a launch that needs no scratch)
+    if (t == 1 && env_int("PYRE_QMATMUL_NATIVE", 1) && !env_int("PYRE_QMATMUL_F32", 0)) {
       if (!ctx->aop_static) return pyre_fail(ctx, PYRE_E_HIP, "pyre_qmatmul_static_dev: the device array was not resolved at context creation");
       return pyre_gemv_n_launch(ctx, m->base_n, m->rows, m->cols, x_dev, y_dev, ctx->aop_static, m->dv.fmt);
     }
-    if (t >= 2 && env_int("PYRE_QMATMUL_Q4M", 1) && m->dvm.fmt == FMT_Q4_K_M && m->dvm.mq && !env_int("PYRE_QMATMUL_F32", 0) && !(m->dv.tiles <= 128 && env_int("PYRE_QMATMUL_SMALL", 1))) {      // a Q4_K window on the matrix cores, as in pyre_qmatmul_dev
+    if (t >= 2 && env_int("PYRE_QMATMUL_Q4M", 1) && m->dvm.fmt == FMT_Q4_K_M && m->dvm.mq && !env_int("PYRE_QMATMUL_F32", 0)) {      // a Q4_K window on the matrix cores, as in pyre_qmatmul_dev
       if (!ctx->aop_static) return pyre_fail(ctx, PYRE_E_HIP, "pyre_qmatmul_static_dev: the device array was not resolved at context creation");
       return pyre_gemm_q4_launch(ctx, m->dvm, x_dev, t, y_dev, ctx->aop_static);
     }
-    if (t >= 2 && env_int("PYRE_QMATMUL_Q2M", 1) && m->dvm.fmt == FMT_IQ2_XS_M && m->dvm.mq && !env_int("PYRE_QMATMUL_F32", 0) && !(m->dv.tiles <= 128 && env_int("PYRE_QMATMUL_SMALL", 1))) {      // an IQ2_XS window likewise
+    if (t >= 2 && env_int("PYRE_QMATMUL_Q2M", 1) && m->dvm.fmt == FMT_IQ2_XS_M && m->dvm.mq && !env_int("PYRE_QMATMUL_F32", 0)) {      // an IQ2_XS window likewise
       if (!ctx->aop_static) return pyre_fail(ctx, PYRE_E_HIP, "pyre_qmatmul_static_dev: the device array was not resolved at context creation");
       return pyre_gemm_q2_launch(ctx, m->dvm, x_dev, t, y_dev, ctx->aop_static);
     }
@@ -662,7 +745,8 @@ int pyre_qmatmul_static_dev(pyre_ctx* ctx, const pyre_qmat* m, const float* x_de
   }
   if (m->dvm.fmt == FMT_Q8_0_M && m->dvm.mq) {      // Q8_0: only a window of a large matrix uses scratch (the matrix-core kernel's operand rows)
     if (m->cols > PYRE_QMATMUL_STATIC_MAX_COLS) return pyre_fail(ctx, PYRE_E_SHAPE, "pyre_qmatmul_static_dev: %zu columns exceed the static scratch of %d columns; use pyre_qmatmul_dev", m->cols, PYRE_QMATMUL_STATIC_MAX_COLS);
-    if (t >= 2 && env_int("PYRE_QMATMUL_Q8M", 1) && !env_int("PYRE_QMATMUL_F32", 0) && !(m->dv.tiles <= 128 && env_int("PYRE_QMATMUL_SMALL", 1))) {
+    if (qmat_rows_call(m, t)) return pyre_gemv_launch(ctx, m->dv, x_dev, t, y_dev);
+    if (t >= 2 && env_int("PYRE_QMATMUL_Q8M", 1) && !env_int("PYRE_QMATMUL_F32", 0)) {
       if (!ctx->aop_static) return pyre_fail(ctx, PYRE_E_HIP, "pyre_qmatmul_static_dev: the device array was not resolved at context creation");
       return pyre_gemm_q8_launch(ctx, m->dvm, x_dev, t, y_dev, ctx->aop_static);
     }
@@ -670,7 +754,7 @@ int pyre_qmatmul_static_dev(pyre_ctx* ctx, const pyre_qmat* m, const float* x_de
   }
   if (m->dvm.fmt != FMT_IQ3_S_M || !m->dvm.mq) return pyre_fail(ctx, PYRE_E_TYPE, "pyre_qmatmul_static_dev: IQ3_S, IQ2_XS, Q4_K and Q8_0 matrices only (the other types' GEMV uses no scratch: pyre_qmatmul_dev allocates nothing for them)");
   if (m->cols > PYRE_QMATMUL_STATIC_MAX_COLS) return pyre_fail(ctx, PYRE_E_SHAPE, "pyre_qmatmul_static_dev: %zu columns exceed the static scratch of %d columns; use pyre_qmatmul_dev", m->cols, PYRE_QMATMUL_STATIC_MAX_COLS);
-  if (qmat_small_one_token(m, t) && !env_int("PYRE_QMATMUL_F32", 0)) return pyre_gemv_launch(ctx, m->dv, x_dev, t, y_dev);      // as pyre_qmatmul_dev (a launch that happens to need no scratch; the limit above holds for every call alike)
+  if (qmat_rows_call(m, t) && !env_int("PYRE_QMATMUL_F32", 0)) return pyre_gemv_launch(ctx, m->dv, x_dev, t, y_dev);      // as pyre_qmatmul_dev (a launch that happens to need no scratch; the limit above holds for every call alike)
   if (t == 1 && m->base_n && env_int("PYRE_QMATMUL_NATIVE", 1)) {      // one token: the native-format kernel, as in pyre_qmatmul_dev, its activation digits in the static array
     if (m->cols > PYRE_QMATMUL_STATIC_MAX_COLS) return pyre_fail(ctx, PYRE_E_SHAPE, "pyre_qmatmul_static_dev: %zu columns exceed the static scratch of %d columns; use pyre_qmatmul_dev", m->cols, PYRE_QMATMUL_STATIC_MAX_COLS);
     if (!ctx->aop_static) return pyre_fail(ctx, PYRE_E_HIP, "pyre_qmatmul_static_dev: the device array was not resolved at context creation");

@@ -407,3 +407,28 @@ def test_window_launch_rules_at_their_edges(ctx, ty, rows, cols):
     assert relerr(y, m.matmul_f32(x)) <= TOL
     for t in (2, 5):          # a token's bits do not depend on the window's width
         assert np.array_equal(bits(m.matmul(x[:t])), bits(y[:t])), t
+
+
+# ---- the lane = row GEMV of a window: products on the matrix cores from four tokens on, a window's tokens on several workgroups where
+# ---- the row tiles are few (up to 256 workgroups: 1, 2, 4 tokens each).  The operation sequence of a token is the single token's, so the
+# ---- oracle is the single-token call and the comparison is of bits: subnormal, huge and zero activations among them.
+@pytest.mark.parametrize("ty", ALL)
+@pytest.mark.parametrize("rows,cols", [(1, 256), (65, 1280), (2049, 256), (4160, 512), (8193, 256), (16448, 256)])
+def test_window_of_the_lane_row_gemv_has_the_single_tokens_bits(ctx, ty, rows, cols):
+    m = lib.QMat(ctx, ty, rows, cols, raw_matrix(ty, rows, cols, 43))
+    x = synth.normal((8, cols), 44)
+    x[1] *= np.float32(1e-39); x[2] *= np.float32(1e30); x[3, ::3] = 0; x[5] = 0; x[6, :64] *= np.float32(1e-42)
+    one = np.concatenate([m.matmul_f32(x[i:i + 1]) for i in range(8)])
+    for t in range(2, 9):
+        assert np.array_equal(bits(m.matmul_f32(x[:t])), bits(one[:t])), t
+
+
+# ---- one token: the lane = row GEMV up to the units its rule names, the native-format kernel above; both within the operator's bound
+@pytest.mark.parametrize("ty,rows,cols", [(ty, r, c) for ty, units in ((lib.IQ3_S, 49152), (lib.IQ2_XS, 24576), (lib.Q4_K, 32768)) for r, c in ((units // 64 * 64, 4096), (units // 64 * 64 + 1, 4096))])
+def test_single_token_launch_rule_at_its_edge(ctx, ty, rows, cols):
+    m = lib.QMat(ctx, ty, rows, cols, raw_matrix(ty, rows, cols, 45))
+    x = synth.normal((1, cols), 46)
+    y, f = m.matmul(x), m.matmul_f32(x)
+    assert relerr(y, f) <= TOL
+    small = rows % 64 == 0
+    assert np.array_equal(bits(y), bits(f)) == small
