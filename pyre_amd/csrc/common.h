@@ -335,7 +335,7 @@ inline bool pyre_moe_groups_ok(const MoeDev& m) { return m.top_k <= PYRE_MOE_KMA
 struct MoeBlk {
   const float* x; const float* rpart; float* parts; size_t wr;
   int32_t* sel_idx; float* sel_w; float* sg; int32_t* eoff; int32_t* elist; float* g; float* u; float* partial;
-  uint16_t* xh; float* xinv; uint16_t* hh; float* hinv;
+  uint16_t* xh; float* xinv; uint16_t* hh; float* hinv; int32_t* plist;          // plist: null, or the passes of k_moe_lists
 };
 bool   pyre_moe_block_ok(const MoeDev& m);
 size_t pyre_moe_block_bytes(const MoeDev& m, int T);
@@ -343,7 +343,7 @@ void   pyre_moe_block_carve(const MoeDev& m, int T, void* base, MoeBlk* b);
 int    pyre_moe_block_zero_rows(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T);
 int    pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_router, int T_max, int nsl, int r64);
 // any number of tokens with the windows' arithmetic: moe.hip
-struct MoeRows { int32_t* sel_idx; float* sel_w; int32_t* elist; float* sg; int32_t* eoff; float* h; float* partial; uint32_t* dgx; uint32_t* dgh; };
+struct MoeRows { int32_t* sel_idx; float* sel_w; int32_t* elist; float* sg; int32_t* eoff; int32_t* plist; float* h; float* partial; uint32_t* dgx; uint32_t* dgh; };
 size_t pyre_moe_rows_bytes(const MoeDev& m, int T);
 void   pyre_moe_rows_carve(const MoeDev& m, int T, void* base, MoeRows* w);
 bool   pyre_moe_rows_ok(const MoeDev& m);

@@ -4,6 +4,7 @@
 // and top_k / soft_top / nan_clean, :3121-3139.  All experts are resident in HBM, so there is no host split.
 #include "formats.h"
 #include "digits.h"
+#include <algorithm>
 #include "gemm_m.h"
 PYRE_TS_DECL(moe_ts) PYRE_TS_EXPORT(moe_ts, pyre_debug_ts_moe)
 
@@ -649,6 +650,7 @@ __global__ __launch_bounds__(256) void k_moe_router_blk(MoeDev m, MoeBlk b, int 
     }
   }
 }
+#define MOE_PASS 8
 // the (token, choice) pairs of the block by expert: eoff[e] .. eoff[e + 1] of elist hold expert e's entries token * (k + 1) + j
 // (in no particular order: a token's sums do not depend on its neighbours).  One workgroup of 1024 threads.
 __global__ __launch_bounds__(1024) void k_moe_lists(MoeDev m, MoeBlk b, int T) {
@@ -663,6 +665,12 @@ __global__ __launch_bounds__(1024) void k_moe_lists(MoeDev m, MoeBlk b, int T) {
   cur[tid] = v - own;            // exclusive prefix
   if (tid <= m.n_exp) b.eoff[tid] = tid < m.n_exp ? v - own : np;
   __syncthreads();
+  if (b.plist) {                 // the experts' entries in passes of MOE_PASS: expert << 16 | pass of the expert
+    const int mine = (own + MOE_PASS - 1) / MOE_PASS; int c = mine;
+    for (int o = 1; o < 1024; o <<= 1) { cnt[tid] = c; __syncthreads(); const int a = tid >= o ? cnt[tid - o] : 0; __syncthreads(); c += a; }
+    if (tid == 1023) b.plist[0] = c;
+    for (int i = 0; i < mine; ++i) b.plist[1 + c - mine + i] = tid << 16 | i;
+  }
   for (int p = tid; p < np; p += 1024) { const int pos = atomicAdd(&cur[b.sel_idx[p]], 1); b.elist[pos] = (p / k) * (k + 1) + p % k; }
 }
 // What a workgroup of the two kernels below works on: blockIdx.y < n_exp: the routed expert's entries; above: eight tokens'
@@ -925,136 +933,127 @@ int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T
   return PYRE_OK;
 }
 
-// k_moe_gu<.., PRE> (both K parts in the workgroup) and k_moe_down with up to four of an expert's tokens through together: a weight is decoded once for
-// them (3.5 of a Q4_K weight's 4.5 vector instructions; 200 tokens, four an expert: 607 us an entry at a time).  grid (row tiles,
-// experts + groups of the shared expert, gate and up), NW waves, raw sums in w.h [gate, up][entry]; a wave stages the four times 64 activations of its unit in its own slice of shared
-// memory.  A token's operations are k_moe_gu's, in its order.
-// one pass of TG entries (elist + i, or i-th of the shared expert's): products of row tile `tile` of Q with x rows by token, raw sums to out [entry]
-template <int FMT, int NW, int TG>
-__device__ __forceinline__ void gu_pass(const QMatDev& Q, int tile, const float* __restrict__ x, int d, const int32_t* __restrict__ list, int first, int step, int k1, int np, float* __restrict__ out, int hstride, float* red, float* xs) {
-  const uint2* lds2 = nullptr;
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, QU = Q.U, upw = (QU + NW * np - 1) / (NW * np);
-  float* xw = xs + (size_t)wave * TG * 64;
-  int en[TG];
+// k_moe_gu<.., PRE> (both K parts in the workgroup) and k_moe_down with up to eight of an expert's tokens through together, four a matrix
+// instruction (unit_mma): a weight is decoded once for them.  grid (row tiles, groups of eight of the shared expert's tokens + passes of
+// eight of an expert's): one expert may have every token (a prompt whose tokens all take the same ten experts ran its 25 passes one
+// behind the other on eleven workgroups a row tile: 423 us), so the passes are workgroups, not a loop.
+// A K range is cut into the shares k_moe_gu / k_moe_down give their waves; here a wave walks SW of them, a unit of weights and
+// activations fetched while the one before it is consumed (straight on into the next row tile or matrix), and the shares meet in
+// k_moe_gu's order, so a token's bits are a window's.  What bounds it is the issue of decoding and f32 products: 200 tokens of A3B in Q4_K, ten
+// experts with every token, gate / up and down 423 + 195 us -> 121 + 61 (18 GFLOP at 126 TFLOP/s: 110).
+// The rows xp points at times nj row tiles: tile(j, Q) names job j's matrix and tile; the shares' sums -> red [share][4 NG][64], then done(j).
+template <int FMT, int NG, int SW, class TF, class DF>
+__device__ __forceinline__ void rows_jobs(int nj, TF tile, const float* const (&xp)[NG], int s0, int upw, int U, int lane, float* red, DF done) {
+  const int k0 = min(U, s0 * upw), k1 = min(U, (s0 + SW) * upw);
+  UnitRaw<FMT> r0, r1; XGrp<NG> x0, x1; v4f a[NG]; mma_zero(a);
+  auto store = [&](int sh) {
 #pragma unroll
-  for (int t = 0; t < TG; ++t) en[t] = __builtin_amdgcn_readfirstlane(list ? list[t] : first + t * step);
-#pragma unroll 1
-  for (int p = 0; p < np; ++p) {
-    float acc[TG];
-#pragma unroll
-    for (int t = 0; t < TG; ++t) acc[t] = 0.0f;
-    const int k0 = min(QU, (wave * np + p) * upw), kend = min(QU, k0 + upw);
-    for (int ku = k0; ku < kend; ++ku) {
-      const UnitRaw<FMT> r = unit_load<FMT>(Q, tile, ku, lane);
-      float xv[TG];
-#pragma unroll
-      for (int t = 0; t < TG; ++t) xv[t] = x[(size_t)(en[t] / k1) * d + ku * 64 + lane];
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int t = 0; t < TG; ++t) xw[t * 64 + lane] = xv[t];
-      __builtin_amdgcn_wave_barrier();
-      unit_fma<FMT, TG>(Q, r, ku, lds2, lane, xw, 64, acc);
-      __builtin_amdgcn_wave_barrier();
-    }
-#pragma unroll
-    for (int t = 0; t < TG; ++t) red[((p * NW + wave) * TG + t) * 64 + lane] = acc[t];
+    for (int t = 0; t < 4 * NG; ++t) red[(sh * 4 * NG + t) * 64 + lane] = a[t >> 2][t & 3];
+    mma_zero(a); };
+  auto fetch = [&](int j, int k, UnitRaw<FMT>& r, XGrp<NG>& x) { QMatDev Q; const int t = tile(min(j, nj - 1), Q); r = unit_load<FMT>(Q, t, k, lane); unit_x_load(xp, k, x); };
+  auto finish = [&](int j) {
+    for (int sh = s0; sh < s0 + SW; ++sh) if (sh * upw >= U) store(sh);          // (shares past the end: zero)
+    lds_barrier(); done(j); lds_barrier(); };
+  int sh = s0, left = upw;
+  auto step = [&](int j, int k, const UnitRaw<FMT>& r, const XGrp<NG>& x) {
+    QMatDev Q; tile(j, Q);
+    unit_mma<FMT, NG>(Q, r, k, x, a);
+    if (--left == 0 || k + 1 == U) { store(sh); ++sh; left = upw; }
+    if (k + 1 == k1) { finish(j); sh = s0; left = upw; } };
+  if (k0 >= k1) { for (int j = 0; j < nj; ++j) finish(j); return; }
+  auto next = [&](int& j, int& k) { if (++k == k1) { k = k0; ++j; } };
+  int j = 0, k = k0; fetch(0, k0, r0, x0);
+  while (j < nj) {
+    int j2 = j, k2 = k; next(j2, k2);
+    fetch(j2, k2, r1, x1);
+    step(j, k, r0, x0);
+    if (j2 >= nj) break;
+    j = j2; k = k2; next(j, k);
+    fetch(j, k, r0, x0);
+    step(j2, k2, r1, x1);
   }
-  __syncthreads();
-  for (int i = tid; i < TG * 64; i += NW * 64) {
-    const int t = i >> 6; float sum = 0.0f;
-    for (int p = 0; p < np; ++p) {
-      float part = red[((p * NW) * TG + t) * 64 + lane];
-#pragma unroll
-      for (int q = 1; q < NW; ++q) part += red[((p * NW + q) * TG + t) * 64 + lane];
-      sum = p == 0 ? part : sum + part;
-    }
-    int e = en[0];
-#pragma unroll
-    for (int q = 1; q < TG; ++q) if (q == t) e = en[q];
-    out[(size_t)e * hstride + blockIdx.x * 64 + lane] = sum;
-  }
-  __syncthreads();
 }
-template <int FMT, int NW>
-__global__ __launch_bounds__(NW * 64) void k_moe_gu_rows(MoeDev m, MoeRows w, const float* __restrict__ x, int hstride, int T, int np) {
-  constexpr int TG = 4;
-  __shared__ float red[2 * NW * TG * 64];
-  __shared__ __align__(16) float xs[NW * TG * 64];
-  const int ye = blockIdx.y, k1 = m.top_k + 1; const bool shared = ye >= m.n_exp;
-  if ((int)blockIdx.x * 64 >= (shared ? m.sf : m.ff)) return;
-  const int t0 = (ye - m.n_exp) * TG, e0 = shared ? 0 : w.eoff[ye], n = shared ? min(TG, T - t0) : w.eoff[ye + 1] - e0;
+// what a workgroup multiplies: n entries of `expert` (list), or those of n tokens from t0 of the shared expert (-1)
+struct RowsPass { int expert, n, t0; const int32_t* list; };
+__device__ __forceinline__ RowsPass rows_pass_of(const MoeDev& m, const MoeRows& w, int T) {
+  const int ns = (T + MOE_PASS - 1) / MOE_PASS, p = (int)blockIdx.y - ns; RowsPass r;
+  if (p < 0) { r.expert = -1; r.t0 = blockIdx.y * MOE_PASS; r.n = min(MOE_PASS, T - r.t0); r.list = nullptr; return r; }
+  if (p >= w.plist[0]) { r.expert = 0; r.t0 = 0; r.n = 0; r.list = nullptr; return r; }
+  const int e = w.plist[1 + p], i0 = (e & 0xFFFF) * MOE_PASS; r.expert = e >> 16; r.t0 = 0;
+  const int e0 = w.eoff[r.expert]; r.n = min(MOE_PASS, w.eoff[r.expert + 1] - e0 - i0); r.list = w.elist + e0 + i0; return r;
+}
+// passes of T tokens' routed entries at most
+static int moe_passes(const MoeDev& m, int T) { const int ne = T * m.top_k; return std::min(ne, m.n_exp + ne / MOE_PASS); }
+template <int FMT, int NP, int NG>
+__device__ __forceinline__ void gu_pass(const QMatDev& Qg, const QMatDev& Qu, int tile, const float* __restrict__ x, int d, const int32_t* __restrict__ list, int first, int k1, int n, float* __restrict__ h, int hstride, float* red) {
+  const int tid = threadIdx.x, t = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, upw = (Qg.U + 16 * NP - 1) / (16 * NP);
+  const float* xp[NG];
+#pragma unroll
+  for (int g = 0; g < NG; ++g) { const int i = min(4 * g + (lane & 3), n - 1), e = list ? list[i] : first + i * k1; xp[g] = x + (size_t)(e / k1) * d + 4 * (lane >> 2); }
+  float gate = 0.0f;          // the thread's row of entry t
+  rows_jobs<FMT, NG, 2 * NP>(2, [&](int j, QMatDev& Q) { Q = pick_mat(j == 0, Qg, Qu); return tile; }, xp, t * 2 * NP, upw, Qg.U, lane, red, [&](int j) {
+    if (t >= n) return;
+    float v = 0.0f;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {          // share q of part p is q * NP + p
+      float part = red[(p * 4 * NG + t) * 64 + lane];
+#pragma unroll
+      for (int q = 1; q < 16; ++q) part += red[((q * NP + p) * 4 * NG + t) * 64 + lane];
+      v = p == 0 ? part : v + part;
+    }
+    if (j == 0) { gate = v; return; }
+    const float s = 1.0f / (1.0f + expf(-gate)); const int e = list ? list[t] : first + t * k1;
+    h[(size_t)e * hstride + blockIdx.x * 64 + lane] = (gate * s) * v; });
+}
+template <int FMT, int NP>
+__global__ __launch_bounds__(512, 4) void k_moe_gu_rows(MoeDev m, MoeRows w, const float* __restrict__ x, int hstride, int T) {
+  __shared__ float red[16 * NP * 8 * 64];
+  const RowsPass P = rows_pass_of(m, w, T); const int n = P.n, t0 = P.t0, k1 = m.top_k + 1; const bool shared = P.expert < 0;
+  if (n <= 0 || (int)blockIdx.x * 64 >= (shared ? m.sf : m.ff)) return;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const QMatDev& Q = blockIdx.z ? (shared ? m.sh_up : m.up_e) : (shared ? m.sh_gate : m.gate_e);
-  float* out = w.h + (size_t)blockIdx.z * T * k1 * hstride;
-  const int tile = (shared ? 0 : ye * (m.ff >> 6)) + blockIdx.x;
-  for (int i0 = 0; i0 < n; ) {          // four entries at a time, the rest two and one
-    const int32_t* list = shared ? nullptr : w.elist + e0 + i0; const int first = (t0 + i0) * k1 + m.top_k;
-    if (n - i0 >= 4) { gu_pass<FMT, NW, 4>(Q, tile, x, m.d, list, first, k1, k1, np, out, hstride, red, xs); i0 += 4; }
-    else if (n - i0 >= 2) { gu_pass<FMT, NW, 2>(Q, tile, x, m.d, list, first, k1, k1, np, out, hstride, red, xs); i0 += 2; }
-    else { gu_pass<FMT, NW, 1>(Q, tile, x, m.d, list, first, k1, k1, np, out, hstride, red, xs); i0 += 1; }
-  }
-  if (!shared || blockIdx.x || blockIdx.z) return;
-  for (int t = 0; t < n; ++t) {          // the shared expert's gate of the group's tokens
-    const float* xt = x + (size_t)(t0 + t) * m.d; float p = 0.0f;
-    for (int ib = tid; ib < m.d; ib += NW * 64) p = fmaf(m.sh_gate_inp[ib], xt[ib], p);
+  const QMatDev Qg = pick_mat(shared, m.sh_gate, m.gate_e), Qu = pick_mat(shared, m.sh_up, m.up_e);
+  const int tile = (shared ? 0 : P.expert * (m.ff >> 6)) + blockIdx.x, first = t0 * k1 + m.top_k;
+  if (n > 4) gu_pass<FMT, NP, 2>(Qg, Qu, tile, x, m.d, P.list, first, k1, n, w.h, hstride, red); else gu_pass<FMT, NP, 1>(Qg, Qu, tile, x, m.d, P.list, first, k1, n, w.h, hstride, red);
+  if (!shared || blockIdx.x) return;
+  for (int t = 0; t < n; ++t) {          // the shared expert's gate of the group's tokens: the sums of k_moe_gu's sixteen waves
+    const float* xt = x + (size_t)(t0 + t) * m.d; float p[2] = {0.0f, 0.0f};
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) p += __shfl_xor(p, o);
-    if (lane == 0) red[wave] = p;
+    for (int i = 0; i < 2; ++i) {
+      for (int ib = tid + 512 * i; ib < m.d; ib += 1024) p[i] = fmaf(m.sh_gate_inp[ib], xt[ib], p[i]);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) p[i] += __shfl_xor(p[i], o);
+      if (lane == 0) red[wave + 8 * i] = p[i];
+    }
     __syncthreads();
-    if (tid == 0) { float tot = 0.0f; for (int q = 0; q < NW; ++q) tot += red[q]; w.sg[t0 + t] = 1.0f / (1.0f + expf(-tot)); }
+    if (tid == 0) { float tot = 0.0f; for (int q = 0; q < 16; ++q) tot += red[q]; w.sg[t0 + t] = 1.0f / (1.0f + expf(-tot)); }
     __syncthreads();
   }
 }
-// ... and k_moe_down likewise, forming silu(gate) * up of the two sums on the way
-template <int FMT, int NW, int TG>
-__device__ __forceinline__ void down_pass(const QMatDev& D, int tile, const MoeRows& w, int d, const int32_t* __restrict__ list, int first, int step, size_t up, int hstride, float* red, float* xs) {
-  const uint2* lds2 = nullptr;
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, upw = (D.U + NW - 1) / NW, k0 = wave * upw, kend = min((int)D.U, k0 + upw);
-  float* xw = xs + (size_t)wave * TG * 64;
-  int en[TG]; float acc[TG];
+// grid (row tiles / MOE_DOWN_TILES, ..): four row tiles a workgroup
+#define MOE_DOWN_TILES 4
+template <int FMT, int NG>
+__device__ __forceinline__ void down_pass(const QMatDev& D, int tile0, int row0, int nj, const float* __restrict__ h, float* __restrict__ partial, int d, const int32_t* __restrict__ list, int first, int k1, int n, int hstride, float* red) {
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, upw = (D.U + 7) / 8;
+  const float* xp[NG];
 #pragma unroll
-  for (int t = 0; t < TG; ++t) { en[t] = __builtin_amdgcn_readfirstlane(list ? list[t] : first + t * step); acc[t] = 0.0f; }
-  for (int ku = k0; ku < kend; ++ku) {
-    const UnitRaw<FMT> r = unit_load<FMT>(D, tile, ku, lane);
-    float xv[TG];
+  for (int g = 0; g < NG; ++g) { const int i = min(4 * g + (lane & 3), n - 1), e = list ? list[i] : first + i * k1; xp[g] = h + (size_t)e * hstride + 4 * (lane >> 2); }
+  rows_jobs<FMT, NG, 2>(nj, [&](int j, QMatDev& Q) { Q = D; return tile0 + j; }, xp, wave * 2, upw, D.U, lane, red, [&](int j) {
+    for (int t = wave; t < n; t += 4) {
+      float sum = red[t * 64 + lane];
 #pragma unroll
-    for (int t = 0; t < TG; ++t) { const float* h = w.h + (size_t)en[t] * hstride + ku * 64 + lane; const float g = h[0], u = h[up], s = 1.0f / (1.0f + expf(-g)); xv[t] = (g * s) * u; }
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int t = 0; t < TG; ++t) xw[t * 64 + lane] = xv[t];
-    __builtin_amdgcn_wave_barrier();
-    unit_fma<FMT, TG>(D, r, ku, lds2, lane, xw, 64, acc);
-    __builtin_amdgcn_wave_barrier();
-  }
-#pragma unroll
-  for (int t = 0; t < TG; ++t) red[(wave * TG + t) * 64 + lane] = acc[t];
-  __syncthreads();
-  for (int i = tid; i < TG * 64; i += NW * 64) {
-    const int t = i >> 6; float sum = red[t * 64 + lane];
-#pragma unroll
-    for (int q = 1; q < NW; ++q) sum += red[(q * TG + t) * 64 + lane];
-    int e = en[0];
-#pragma unroll
-    for (int q = 1; q < TG; ++q) if (q == t) e = en[q];
-    w.partial[(size_t)e * d + blockIdx.x * 64 + lane] = sum;
-  }
-  __syncthreads();
+      for (int q = 1; q < 8; ++q) sum += red[(q * 4 * NG + t) * 64 + lane];
+      const int e = list ? list[t] : first + t * k1;
+      partial[(size_t)e * d + row0 + j * 64 + lane] = sum;
+    } });
 }
-template <int FMT, int NW>
-__global__ __launch_bounds__(NW * 64) void k_moe_down_rows(MoeDev m, MoeRows w, int hstride, int T) {
-  constexpr int TG = 4;
-  __shared__ float red[NW * TG * 64];
-  __shared__ __align__(16) float xs[NW * TG * 64];
-  const int ye = blockIdx.y, k1 = m.top_k + 1; const bool shared = ye >= m.n_exp;
-  const int t0 = (ye - m.n_exp) * TG, e0 = shared ? 0 : w.eoff[ye], n = shared ? min(TG, T - t0) : w.eoff[ye + 1] - e0;
-  const QMatDev& D = shared ? m.sh_down : m.down_e;
-  const int tile = (shared ? 0 : ye * (m.d >> 6)) + blockIdx.x; const size_t up = (size_t)T * k1 * hstride;
-  for (int i0 = 0; i0 < n; ) {
-    const int32_t* list = shared ? nullptr : w.elist + e0 + i0; const int first = (t0 + i0) * k1 + m.top_k;
-    if (n - i0 >= 4) { down_pass<FMT, NW, 4>(D, tile, w, m.d, list, first, k1, up, hstride, red, xs); i0 += 4; }
-    else if (n - i0 >= 2) { down_pass<FMT, NW, 2>(D, tile, w, m.d, list, first, k1, up, hstride, red, xs); i0 += 2; }
-    else { down_pass<FMT, NW, 1>(D, tile, w, m.d, list, first, k1, up, hstride, red, xs); i0 += 1; }
-  }
+template <int FMT>
+__global__ __launch_bounds__(256, 4) void k_moe_down_rows(MoeDev m, MoeRows w, int hstride, int T) {
+  __shared__ float red[8 * 8 * 64];
+  const RowsPass P = rows_pass_of(m, w, T); const int n = P.n, k1 = m.top_k + 1; const bool shared = P.expert < 0;
+  if (n <= 0) return;
+  const QMatDev D = pick_mat(shared, m.sh_down, m.down_e);
+  const int r0 = blockIdx.x * MOE_DOWN_TILES, nj = min(MOE_DOWN_TILES, (m.d >> 6) - r0), tile = (shared ? 0 : P.expert * (m.d >> 6)) + r0, first = P.t0 * k1 + m.top_k;
+  if (n > 4) down_pass<FMT, 2>(D, tile, r0 * 64, nj, w.h, w.partial, m.d, P.list, first, k1, n, hstride, red); else down_pass<FMT, 1>(D, tile, r0 * 64, nj, w.h, w.partial, m.d, P.list, first, k1, n, hstride, red);
 }
 
 // The windows' arithmetic (k_moe_gu / k_moe_down, the digits form for IQ3_S experts) for any number of tokens in one set of launches,
@@ -1063,19 +1062,19 @@ __global__ __launch_bounds__(NW * 64) void k_moe_down_rows(MoeDev m, MoeRows w, 
 // null; y: their sum [token][d], or null; the unreduced terms stay in w (pyre_moe_rows_out).
 size_t pyre_moe_rows_bytes(const MoeDev& m, int T) {
   const size_t hs = (size_t)(m.ff > m.sf ? m.ff : m.sf), k1 = m.top_k + 1, n = T;
-  return 256 * 12 + 4 * (3 * n * m.top_k + n + 1024 + n * k1 * (2 * hs + m.d) + n * (m.d / 64) * DGX_STRIDE + n * k1 * (hs / 64) * DGX_STRIDE);
+  return 256 * 13 + 4 * (4 * n * m.top_k + 1 + n + 1024 + n * k1 * (hs + m.d) + n * (m.d / 64) * DGX_STRIDE + n * k1 * (hs / 64) * DGX_STRIDE);
 }
 void pyre_moe_rows_carve(const MoeDev& m, int T, void* base, MoeRows* w) {
   uint8_t* p = (uint8_t*)base; auto take = [&](size_t n) { void* r = p; p += (4 * n + 255) & ~(size_t)255; return r; };
   const size_t hs = (size_t)(m.ff > m.sf ? m.ff : m.sf), k1 = m.top_k + 1, n = T;
-  w->sel_idx = (int32_t*)take(n * m.top_k); w->sel_w = (float*)take(n * m.top_k); w->elist = (int32_t*)take(n * m.top_k); w->sg = (float*)take(n); w->eoff = (int32_t*)take(1024);
-  w->h = (float*)take(2 * n * k1 * hs); w->partial = (float*)take(n * k1 * m.d); w->dgx = (uint32_t*)take(n * (m.d / 64) * DGX_STRIDE); w->dgh = (uint32_t*)take(n * k1 * (hs / 64) * DGX_STRIDE);
+  w->sel_idx = (int32_t*)take(n * m.top_k); w->sel_w = (float*)take(n * m.top_k); w->elist = (int32_t*)take(n * m.top_k); w->sg = (float*)take(n); w->eoff = (int32_t*)take(1024); w->plist = (int32_t*)take(1 + n * m.top_k);
+  w->h = (float*)take(n * k1 * hs); w->partial = (float*)take(n * k1 * m.d); w->dgx = (uint32_t*)take(n * (m.d / 64) * DGX_STRIDE); w->dgh = (uint32_t*)take(n * k1 * (hs / 64) * DGX_STRIDE);
 }
 bool pyre_moe_rows_ok(const MoeDev& m) { return m.top_k <= PYRE_MOE_KMAX && m.n_exp <= 1023 && m.d % 64 == 0; }
 int pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const float* x, int T, const float* rpart, size_t wr, int nsl, int r64, float* parts, float* y) {
   if (!pyre_moe_rows_ok(m) || T < 1 || T * (m.top_k + 1) > 65535 || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe rows: unsupported shape (T = %d, %d router slices)", T, nsl);
-  MoeBlk b{}; b.rpart = rpart; b.wr = wr; b.parts = parts; b.sel_idx = w.sel_idx; b.sel_w = w.sel_w; b.eoff = w.eoff; b.elist = w.elist; b.partial = w.partial; b.sg = w.sg;
-  const int hs = m.ff > m.sf ? m.ff : m.sf, entries = T * (m.top_k + 1), P = pyre_moe_gu_parts(m);
+  MoeBlk b{}; b.rpart = rpart; b.wr = wr; b.parts = parts; b.sel_idx = w.sel_idx; b.sel_w = w.sel_w; b.eoff = w.eoff; b.elist = w.elist; b.partial = w.partial; b.sg = w.sg; b.plist = w.plist;
+  const int hs = m.ff > m.sf ? m.ff : m.sf, entries = T * (m.top_k + 1), P = pyre_moe_gu_parts(m), ns = (T + MOE_PASS - 1) / MOE_PASS;
   const uint2* g2 = (const uint2*)ctx->d_iq2xs;
   const bool idot = pyre_moe_takes_digits(m), idot_dn = idot && !moe_idot_gu_only() && m.down_e.fmt == FMT_IQ3_S && m.sh_down.fmt == FMT_IQ3_S;
   uint32_t* dgh = idot_dn ? w.dgh : nullptr;
@@ -1088,14 +1087,15 @@ int pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const
     const bool fix = m.gate_e.fmt == FMT_IQ3_S && m.down_e.fmt == FMT_IQ3_S && m.n_exp == 512 && m.top_k == 10 && m.d == 2048 && m.ff == 512 && m.sf == 512 && nsl == 32;
     if (idot && fix && P == 2) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, true, true>), ROWS_GU);
     else if (idot) { if (P == 2) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, false, true>), ROWS_GU); else hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 1, true, false, true>), ROWS_GU); }
-    else { MOE_FMT_DISPATCH(m.gate_e.fmt, hipLaunchKernelGGL((k_moe_gu_rows<F, 16>), dim3(hs / 64, m.n_exp + (T + 3) / 4, 2), dim3(16 * 64), 0, ctx->stream, m, w, x, hs, T, P)); }
+    else if (P == 2) { MOE_FMT_DISPATCH(m.gate_e.fmt, hipLaunchKernelGGL((k_moe_gu_rows<F, 2>), dim3(hs / 64, ns + moe_passes(m, T)), dim3(512), 0, ctx->stream, m, w, x, hs, T)); }
+    else { MOE_FMT_DISPATCH(m.gate_e.fmt, hipLaunchKernelGGL((k_moe_gu_rows<F, 1>), dim3(hs / 64, ns + moe_passes(m, T)), dim3(512), 0, ctx->stream, m, w, x, hs, T)); }
 #undef ROWS_GU
   } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "moe_rows_down", T * (m.top_k * qmat_gguf_bytes(m.down_e, m.d) + qmat_gguf_bytes(m.sh_down, m.d)));
 #define ROWS_DN dim3(m.d / 64, entries), dim3(8 * 64), 0, ctx->stream, m, w.sel_idx, w.h, hs, w.partial, g2, dgh, w.elist
     if (idot_dn) hipLaunchKernelGGL((k_moe_down<FMT_IQ3_S, 8, 1, false, true>), ROWS_DN);
     else if (idot) { MOE_FMT_DISPATCH(m.down_e.fmt, hipLaunchKernelGGL((k_moe_down<F, 8, 1>), ROWS_DN)); }          // (behind the digits form h is finished)
-    else { MOE_FMT_DISPATCH(m.down_e.fmt, hipLaunchKernelGGL((k_moe_down_rows<F, 8>), dim3(m.d / 64, m.n_exp + (T + 3) / 4), dim3(8 * 64), 0, ctx->stream, m, w, hs, T)); }
+    else { MOE_FMT_DISPATCH(m.down_e.fmt, hipLaunchKernelGGL((k_moe_down_rows<F>), dim3((m.d / 64 + MOE_DOWN_TILES - 1) / MOE_DOWN_TILES, ns + moe_passes(m, T)), dim3(256), 0, ctx->stream, m, w, hs, T)); }
 #undef ROWS_DN
     if (parts) hipLaunchKernelGGL(k_moe_groups_blk, dim3((m.d + 255) / 256, T), dim3(256), 0, ctx->stream, m, b, T);
     if (y) hipLaunchKernelGGL(k_moe_sum, dim3((m.d + 255) / 256, T), dim3(256), 0, ctx->stream, w.partial, w.sel_w, w.sg, m.d, m.top_k, y); } PYRE_CHECK_LAUNCH(ctx);

@@ -737,3 +737,17 @@ def test_session_chunk_grid_prefill_and_prefix_cache_give_the_state_of_a_full_pr
     off = lib.Session(gm, 400, chunk=32, cache_bytes=0)                                 # PYRE_QN_PCACHE=0
     off.prefill(A); assert off.stats()[0] == 0
     se.close(); small.close(); off.close()
+
+
+@pytest.mark.parametrize("qtype,geom", [(synth.Q4_K, {}), (synth.Q8_0, dict(d=512, ff_exp=192, ff_sh=320)), (synth.IQ2_XS, dict(d=768)), (synth.IQ4_XS, dict(d=2048, ff_exp=512, n_exp=6))])
+@pytest.mark.parametrize("n", [9, 25, 141])
+def test_prompt_rows_of_few_and_of_skewed_experts_equal_the_windows(ctx, qtype, geom, n, monkeypatch):
+    # passes of up to eight of an expert's entries: experts with none, a few, or (top_k of n_exp) nearly all of a prompt's tokens; one and two
+    # K parts, shares past the end of a row, a shared expert of another width
+    c = small_cfg(**{**dict(qtype=qtype, hc_type=synth.BF16, n_exp=8, top_k=5, n_layers=4), **geom})
+    hw = mg.build_host(c, seed=81); gm = lib.Model(ctx, c, hw.layers, hw.globals_)
+    ids = np.random.Generator(np.random.PCG64(n)).integers(0, c.vocab, n, dtype=np.uint32); out = []
+    for windows in ("1", "0"):
+        monkeypatch.setenv("PYRE_PROMPT_WINDOWS", windows)
+        out.append(gm.forward(ids, gm.new_state(n + 8)))
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
