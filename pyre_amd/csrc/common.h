@@ -440,7 +440,8 @@ struct GdnDev { const float* a; const float* dt; const float* conv_w; const floa
 // conv_done: co_scratch already holds silu(conv) of the window and the conv state has been advanced (GemvEpi).
 // gq: the launch runs on nv x 4 workgroups (a workgroup owns 32 columns of a head's state) and leaves, instead of out_dev,
 // the un-normalised gated output as f16 operand rows with the per-quarter factors and sums of squares of PyreAop::sq.
-// The state it leaves is the nv-workgroup form's, to the bit (gdn.h).
+// The state it leaves differs in rounding from the nv-workgroup form's (the column sums meet in another order): a layer
+// uses one form for every call.
 struct GdnQ { uint16_t* op; float* sq; };
 int pyre_gdn_launch(pyre_ctx* ctx, const GdnDev& g, const float* proj, int proj_stride, int t, const float* conv_in, float* conv_out,
                     const float* ssm_in, float* ssm_out, float* co_scratch, float* out_dev, bool conv_done = false, uint16_t* aop = nullptr, float aop_up = 1.0f, const GdnQ* gq = nullptr);
@@ -453,9 +454,10 @@ size_t pyre_gdn_chunk_bytes(const GdnDev& g, int T);
 void   pyre_gdn_chunk_carve(const GdnDev& g, int T, void* base, GdnChunk* b);
 int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int proj_stride, int T, const float* conv_in, float* conv_out,
                           const float* ssm_in, float* ssm_out, float* oraw);
-// the recurrence token by token instead, the bits of pyre_gdn_launch in either form (b.co and b.dec are all it needs)
+// the recurrence token by token instead, the bits of pyre_gdn_launch's per-quarter form (quarters) or of its head-a-workgroup form
+// (b.co and b.dec are all it needs)
 int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int proj_stride, int T, const float* conv_in, float* conv_out,
-                        const float* ssm_in, float* ssm_out, float* oraw);
+                        const float* ssm_in, float* ssm_out, float* oraw, bool quarters = true);
 
 // ---- gated attention over the KV cache (attn.hip) -----------------------------------------------------------------------
 struct AttnDev { const float* qn; const float* kn; const float* rope_inv; int nh, nkv, hd, n_rot, kv_bits, kv_recent; float eps; float mscale = 1.0f; };   // mscale: YaRN magnitude factor on cos and sin

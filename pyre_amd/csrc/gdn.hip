@@ -1,7 +1,6 @@
 // Gated DeltaNet recurrent step: causal depthwise conv1d + SiLU, L2-normalised q/k, gated delta rule on the fp32
 // state kept resident in HBM, gated RMSNorm.  Follows linear_core, src/model/qwen4exp_gguf.rs:1624-1673.
 #include "formats.h"
-#include "gdn.h"
 #include "workers.h"
 #include <algorithm>
 #include <condition_variable>
@@ -36,7 +35,7 @@ __global__ __launch_bounds__(256) void k_gdn_conv(const float* __restrict__ proj
 // fetches token ti's q, k, v, z and gate inputs -- eight requests a lane, all tokens in flight together -- and leaves
 // the L2-normalised q and k, v, z, the decay and beta in shared memory) and after it (wave ti: RMSNorm and gate of token
 // ti's output).  A token of the recurrence itself costs one barrier:
-//   mem = g S^T k -> barrier -> delta = (v - mem) beta; S = g S + k (x) delta; o = S^T q      (gdn.h: the order of the sums)
+//   S *= g; mem = S^T k -> barrier -> delta = (v - mem) beta; S += k (x) delta; o = S^T q      (linear_core, :1655-1668)
 // FT, FNK, FNV > 0: the window width and the head counts as compile-time constants (the launcher checks them) -- same arithmetic.
 template <int DK, int DV, int FT = 0, int FNK = 0, int FNV = 0>
 __global__ __launch_bounds__(512) void k_gdn_delta(GdnDev p, const float* __restrict__ proj, int stride, int t, const float* __restrict__ co_all,
@@ -74,18 +73,16 @@ __global__ __launch_bounds__(512) void k_gdn_delta(GdnDev p, const float* __rest
   lds_barrier(); PYRE_TS(1);
   for (int ti = 0; ti < t; ++ti) {
     const float g = gs[ti], b = bs[ti];
-    float sub[4];          // the group's 32 rows are four of the tree's sixteen leaves
+    float pmv = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sub[i] = gdn_dot8(S + 8 * i, &ks[ti][grp * R + 8 * i]);
-    pm[ti & 1][grp][j] = gdn_tree(sub);
+    for (int r = 0; r < R; ++r) { S[r] *= g; pmv += S[r] * ks[ti][grp * R + r]; }
+    pm[ti & 1][grp][j] = pmv;
     lds_barrier();
-    const float mem = ((pm[ti & 1][0][j] + pm[ti & 1][1][j]) + (pm[ti & 1][2][j] + pm[ti & 1][3][j])) * g;
+    const float mem = ((pm[ti & 1][0][j] + pm[ti & 1][1][j]) + pm[ti & 1][2][j]) + pm[ti & 1][3][j];
     const float delta = (vs[ti][j] - mem) * b;
+    float pov = 0.0f;
 #pragma unroll
-    for (int r = 0; r < R; ++r) S[r] = fmaf(ks[ti][grp * R + r], delta, S[r] * g);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sub[i] = gdn_dot8(S + 8 * i, &qs[ti][grp * R + 8 * i]);
-    const float pov = gdn_tree(sub);
+    for (int r = 0; r < R; ++r) { S[r] += ks[ti][grp * R + r] * delta; pov += S[r] * qs[ti][grp * R + r]; }
     po[ti][grp][j] = pov;
   }
   PYRE_TS(2);
@@ -93,8 +90,8 @@ __global__ __launch_bounds__(512) void k_gdn_delta(GdnDev p, const float* __rest
   for (int r = 0; r < R; ++r) sout[(size_t)(grp * R + r) * DV + j] = S[r];
   lds_barrier(); PYRE_TS(3);
   if (wave < t) {
-    const float o0 = (po[wave][0][lane] + po[wave][1][lane]) + (po[wave][2][lane] + po[wave][3][lane]);
-    const float o1 = (po[wave][0][lane + 64] + po[wave][1][lane + 64]) + (po[wave][2][lane + 64] + po[wave][3][lane + 64]);
+    const float o0 = ((po[wave][0][lane] + po[wave][1][lane]) + po[wave][2][lane]) + po[wave][3][lane];
+    const float o1 = ((po[wave][0][lane + 64] + po[wave][1][lane + 64]) + po[wave][2][lane + 64]) + po[wave][3][lane + 64];
     const float sc = 1.0f / sqrtf((wsum(o0 * o0) + wsum(o1 * o1)) / (float)DV + p.eps);
     const float r0 = (o0 * (sc * nw0)) * g_sigm(zs[wave][lane]), r1 = (o1 * (sc * nw1)) * g_sigm(zs[wave][lane + 64]);      // rms_inplace: x *= s * w  (:210)
     out[(size_t)wave * w + h * DV + lane] = r0; out[(size_t)wave * w + h * DV + lane + 64] = r1;
@@ -105,8 +102,7 @@ __global__ __launch_bounds__(512) void k_gdn_delta(GdnDev p, const float* __rest
 
 // The same recurrence on nv x 4 workgroups: workgroup (h, q) owns the 32 columns 32*q .. of head h's state (the columns of
 // the delta rule are independent), 16 KB instead of 64 KB to fetch and to store.  Thread (rg = tid/32, j = tid%32) keeps rows
-// 8*rg .. 8*rg+7 of column 32*q + j; the sixteen row groups' sums are gdn.h's tree: the two of a wave by an exchange of its halves,
-// the eight waves' through shared memory.  The head's RMS norm needs
+// 8*rg .. 8*rg+7 of column 32*q + j; the sixteen row groups' sums meet in shared memory in order.  The head's RMS norm needs
 // all 128 columns, so it is left to the consumer (the output projection, PyreAop::sq): wave ti leaves token ti's
 // un-normalised gated output u = (o * norm_w) * sigmoid(z) of its 32 columns as f16 operand rows scaled by the quarter's own
 // power of two (its largest magnitude into [2^13, 2^14)), that factor's inverse, and the quarter's sum of o^2.
@@ -117,7 +113,7 @@ __global__ __launch_bounds__(512) void k_gdn_delta_q(GdnDev p, const float* __re
   constexpr int QC = 32, G = 16, R = DK / G, MT = 8;
   args_now(p.a, p.dt, p.norm_w, p.nk, p.nv, p.eps, proj, stride, t, co_all, ssm_in, ssm_out, aop, sq);
   if constexpr (FT > 0) { t = FT; p.nk = FNK; p.nv = FNV; }
-  __shared__ float qs[MT][DK], ks[MT][DK], vs[MT][QC], zs[MT][QC], pm[2][G / 2][QC], po[MT][G / 2][QC], gs[MT], bs[MT];
+  __shared__ float qs[MT][DK], ks[MT][DK], vs[MT][QC], zs[MT][QC], pm[2][G][QC], po[MT][G][QC], gs[MT], bs[MT];
   const int h = blockIdx.x, qd = blockIdx.y, kh = h % p.nk, tid = threadIdx.x, j = tid & (QC - 1), rg = tid >> 5, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ch = 2 * p.nk * DK + p.nv * DV, w = p.nv * DV, jc = qd * QC + j;
@@ -143,26 +139,28 @@ __global__ __launch_bounds__(512) void k_gdn_delta_q(GdnDev p, const float* __re
   lds_barrier();
   for (int ti = 0; ti < t; ++ti) {
     const float g = gs[ti], b = bs[ti];
-    pm[ti & 1][wave][j] = halves_sum(gdn_dot8(S, &ks[ti][rg * R]));          // (both halves of the wave, the same value)
+    float pmv = 0.0f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) { S[r] *= g; pmv += S[r] * ks[ti][rg * R + r]; }
+    pm[ti & 1][rg][j] = pmv;
     lds_barrier();
-    float pv[G / 2];
+    float mem = pm[ti & 1][0][j];
 #pragma unroll
-    for (int k = 0; k < G / 2; ++k) pv[k] = pm[ti & 1][k][j];
-    const float mem = gdn_tree(pv) * g;
+    for (int k = 1; k < G; ++k) mem += pm[ti & 1][k][j];
     const float delta = (vs[ti][j] - mem) * b;
+    float pov = 0.0f;
 #pragma unroll
-    for (int r = 0; r < R; ++r) S[r] = fmaf(ks[ti][rg * R + r], delta, S[r] * g);
-    po[ti][wave][j] = halves_sum(gdn_dot8(S, &qs[ti][rg * R]));
+    for (int r = 0; r < R; ++r) { S[r] += ks[ti][rg * R + r] * delta; pov += S[r] * qs[ti][rg * R + r]; }
+    po[ti][rg][j] = pov;
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) sout[(size_t)(rg * R + r) * DV + jc] = S[r];
   lds_barrier();
   if (wave < t) {
     const int jl = lane & 31; const bool on = lane < QC;
-    float ov[G / 2];
+    float o = po[wave][0][jl];
 #pragma unroll
-    for (int k = 0; k < G / 2; ++k) ov[k] = po[wave][k][jl];
-    const float o = gdn_tree(ov);
+    for (int k = 1; k < G; ++k) o += po[wave][k][jl];
     const float ss = wave_sum(on ? o * o : 0.0f);
     const float u = (o * nw) * g_sigm(zs[wave][jl]);
     float am = on ? fabsf(u) : 0.0f; am = am == am ? am : INFINITY;

@@ -16,7 +16,6 @@
 // the chip idle); the scan, now the only serial part, is three small products.  fp32 throughout.
 // Tokens past T in the last chunk have beta = 0, k = q = 0 and no decay: they leave the state as it is.
 #include "formats.h"
-#include "gdn.h"
 
 typedef float v4f_ __attribute__((ext_vector_type(4)));
 
@@ -221,89 +220,144 @@ __global__ __launch_bounds__(256) void k_gdnc_scan(GdnDev p, const float* __rest
   for (int i = tid; i < DK * 16; i += 256) sout[(size_t)(i >> 4) * p.dv + (i & 15)] = St[i & 15][i >> 4];
 }
 
-// ---- the recurrence token by token, the bits of k_gdn_delta and k_gdn_delta_q -----------------------------------------------------
+// ---- the recurrence token by token, the bits of k_gdn_delta_q -------------------------------------------------------------------
 // A prompt of the model takes this one: its state and outputs are then those of decoding the tokens in windows, to the bit, so
-// that no token's expert choice tips with the path the prompt took.  The step kernels add their row groups' sums through shared
-// memory behind a barrier; here a wave keeps two columns, 32 lanes (a lane: four rows, one chain of gdn_dot8) each, and the rest of
-// gdn.h's tree is five exchanges within the 32 lanes, without a barrier: pairs, quads, half mirror, mirror, then the two rows of sixteen
-// (every lane then holds the sum).  The outputs, which nothing waits for, are added four tokens at a time.  About 30 vector
-// instructions a token and two waves a SIMD for 32 heads: a wave issues at most one instruction in four cycles, so the second fills the slots of
-// the other's shared-memory and scalar instructions.  2048 tokens of the A3B layer: groups added one after the other, sixteen lanes a column 590 us;
-// as a tree 393; this form 285.
-// grid (nv, 8), 8 waves: workgroup (h, y) columns 16 y .. of head h.  The keys, queries (normalised, co of k_gdnc_conv), values and gate
+// that no token's expert choice tips with the path the prompt took.  k_gdn_delta_q keeps 32 columns a workgroup, eight rows a
+// thread, and adds the sixteen row groups' sums through shared memory behind a barrier: 0.9 us a token.  Here a wave keeps
+// four columns, a row of sixteen lanes (a lane: eight rows) each: the sums meet in the same order by DPP row shifts
+// (x <- p + x of the lane before, fifteen times: the last lane has ((p0 + p1) + p2) + ..), without a barrier, and the
+// output's sums of one token run in the wait slots of the next token's.  About 100 vector instructions a token, one wave a SIMD
+// for 32 heads (the recurrence is a chain, so further waves would only share the SIMD).
+// grid (nv, 8), 4 waves: workgroup (h, y) columns 16 y .. of head h.  The keys, queries (normalised, co of k_gdnc_conv), values and gate
 // inputs of sixteen tokens at a time go through shared memory, the next sixteen in registers meanwhile.
-template <int CTRL> __device__ __forceinline__ float row_xor(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true)); }
-__device__ __forceinline__ float rows_sum(float x) {          // the sum of a row of sixteen lanes and its neighbour row's
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__global__ __launch_bounds__(512) void k_gdn_rec(GdnDev p, const float* __restrict__ co, const float2* __restrict__ gates, int T, const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
-  constexpr int TB = 16, R = 4;
-  __shared__ __align__(16) float4 kq[2][TB][2][32];          // [buffer][token][k, q][rows 4 i ..]
-  __shared__ float vs[2][TB][16], os[2][TB + 3][16]; __shared__ float2 gb[2][TB];
-  const int h = blockIdx.x, cb = blockIdx.y * 16, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, rl = lane & 31;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), jl = wave * 2 + (lane >> 5), col = cb + jl;
+__device__ __forceinline__ float row_shr1(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x111, 0xf, 0xf, true)); }
+__device__ __forceinline__ float row_last(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x15F, 0xf, 0xf, true)); }
+__global__ __launch_bounds__(256) void k_gdn_rec(GdnDev p, const float* __restrict__ co, const float2* __restrict__ gates, int T, const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
+  constexpr int TB = 16, R = 8;
+  __shared__ __align__(16) float4 kq[2][TB][2][2][16];          // [buffer][token][k, q][rows 0-3, 4-7 of a row group][row group]
+  __shared__ float vs[2][TB][16], os[2][TB][16]; __shared__ float2 gb[2][TB];
+  const int h = blockIdx.x, cb = blockIdx.y * 16, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, rg = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), jl = wave * 4 + (lane >> 4), col = cb + jl;
   const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv, w = p.nv * p.dv;
-  const size_t so = ((size_t)h * DK + rl * R) * p.dv + col;
+  const size_t so = ((size_t)h * DK + rg * R) * p.dv + col;
   float S[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) S[r] = ssm_in[so + (size_t)r * p.dv];
-  float4 f0, f1; float fv = 0.0f; float2 fg = make_float2(0.0f, 0.0f);
-  auto src = [&](int t0, int i) { const int e = tid + 512 * i, t = min(t0 + (e >> 6), T - 1), f = e & 63; return *(const float4*)(co + (size_t)t * ch + (f < 32 ? nqk : 0) + kh * DK + 4 * (f & 31)); };
+  float4 f0, f1, f2, f3; float fv; float2 fg = make_float2(0.0f, 0.0f);
+  auto src = [&](int t0, int i) { const int e = tid + 256 * i, t = min(t0 + (e >> 6), T - 1), f = e & 63; return *(const float4*)(co + (size_t)t * ch + (f < 32 ? nqk : 0) + kh * DK + 4 * (f & 31)); };
   auto fetch = [&](int t0) {          // token t0 + e / 64's float4 e % 64: 32 of k, 32 of q (past the end: the last token's again)
-    f0 = src(t0, 0); f1 = src(t0, 1);
-    if (tid < 256) fv = co[(size_t)min(t0 + (tid >> 4), T - 1) * ch + 2 * nqk + (size_t)h * p.dv + cb + (tid & 15)];
+    f0 = src(t0, 0); f1 = src(t0, 1); f2 = src(t0, 2); f3 = src(t0, 3);
+    fv = co[(size_t)min(t0 + (tid >> 4), T - 1) * ch + 2 * nqk + (size_t)h * p.dv + cb + (tid & 15)];
     if (tid < TB) fg = gates[(size_t)min(t0 + tid, T - 1) * p.nv + h];
   };
-  auto put = [&](int buf, int i, const float4& f) { const int e = tid + 512 * i, c = e & 63; kq[buf][e >> 6][c >> 5][c & 31] = f; };
+  auto put = [&](int buf, int i, const float4& f) { const int e = tid + 256 * i, c = e & 63; kq[buf][e >> 6][c >> 5][c & 1][(c & 31) >> 1] = f; };
   auto store = [&](int buf) {
-    put(buf, 0, f0); put(buf, 1, f1);
-    if (tid < 256) vs[buf][tid >> 4][tid & 15] = fv;
+    put(buf, 0, f0); put(buf, 1, f1); put(buf, 2, f2); put(buf, 3, f3);
+    vs[buf][tid >> 4][tid & 15] = fv;
     if (tid < TB) gb[buf][tid] = fg;
   };
-  struct Tok { float4 k, q; float2 g; float v; };
-  auto get = [&](int buf, int t) { return Tok{kq[buf][t][0][rl], kq[buf][t][1][rl], gb[buf][t], vs[buf][t][jl]}; };
-  auto dot = [&](const float4& k) { return fmaf(S[3], k.w, fmaf(S[2], k.z, fmaf(S[1], k.y, S[0] * k.x))); };
+  struct Tok { float4 k0, k1, q0, q1; float2 g; float v; };
+  auto get = [&](int buf, int t) { return Tok{kq[buf][t][0][0][rg], kq[buf][t][0][1][rg], kq[buf][t][1][0][rg], kq[buf][t][1][1][rg], gb[buf][t], vs[buf][t][jl]}; };
   fetch(0); store(0);
   lds_barrier();
   for (int t0 = 0, buf = 0; t0 < T; t0 += TB, buf ^= 1) {
     if (t0 + TB < T) fetch(t0 + TB);
     const int n = min(TB, T - t0);
-    auto step = [&](const Tok& c) {
-      float m = dot(c.k), D[R];
-      m += row_xor<0xB1>(m);
-      m += row_xor<0x4E>(m); D[0] = S[0] * c.g.x;
-      m += row_xor<0x141>(m); D[1] = S[1] * c.g.x;
-      m += row_xor<0x140>(m); D[2] = S[2] * c.g.x;
-      m = rows_sum(m); D[3] = S[3] * c.g.x;
-      const float delta = (c.v - m * c.g.x) * c.g.y;
-      S[0] = fmaf(c.k.x, delta, D[0]); S[1] = fmaf(c.k.y, delta, D[1]); S[2] = fmaf(c.k.z, delta, D[2]); S[3] = fmaf(c.k.w, delta, D[3]);
-    };
-    // The outputs of four tokens share the tree: pairs and quads of lanes keep a token each (lane bits 0, 1: the token), then two
-    // rotations add the quads -- lanes 4 .. 7 get (quad 1 + quad 0) + (quad 3 + quad 2) -- and the rows meet.
-    auto out4 = [&](float a, float b, float c, float d, int t) {
-      const bool b0 = lane & 1, b1 = lane & 2;
-      const float u = (b0 ? b : a) + row_xor<0xB1>(b0 ? a : b), v = (b0 ? d : c) + row_xor<0xB1>(b0 ? c : d);
-      float o = (b1 ? v : u) + row_xor<0x4E>(b1 ? u : v);
-      o += row_xor<0x124>(o); o += row_xor<0x128>(o); o = rows_sum(o);
-      if ((rl & 28) == 4) os[buf][t + (rl & 3)][jl] = o;
-    };
-    if (n == TB) {          // a token ahead, two sets of registers taking turns; the count known, so that no index is computed
-      Tok x[2]; x[0] = get(buf, 0);
-      float4 qp[2]; float po[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    // In the wait slots of token t's chain: the output terms of token t - 1 (its state is still there: the decayed one goes to
+    // other registers) and the output chain of token t - 2.
+    float po2 = 0.0f, po1 = 0.0f; float4 qa = make_float4(0.0f, 0.0f, 0.0f, 0.0f), qb = qa;          // chain input of token t - 2; the query of token t - 1
+    auto terms = [&]() { const float q[R] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w}; float o = S[0] * q[0];
 #pragma unroll
-      for (int t = 0; t < TB; ++t) {          // (a token's output terms run in the wait slots of the next one's chain)
-        if (t + 1 < TB) x[(t + 1) & 1] = get(buf, t + 1);
-        if (t > 0) po[(t - 1) & 3] = dot(qp[(t - 1) & 1]);
-        qp[t & 1] = x[t & 1].q;
-        step(x[t & 1]);
-        if (t > 0 && (t & 3) == 0) out4(po[0], po[1], po[2], po[3], t - 4);
+      for (int r = 1; r < R; ++r) o += S[r] * q[r];
+      return o; };
+    auto step = [&](const Tok& c, int t) {
+      const float k[R] = {c.k0.x, c.k0.y, c.k0.z, c.k0.w, c.k1.x, c.k1.y, c.k1.z, c.k1.w};
+      float D[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) D[r] = S[r] * c.g.x;
+      float pm = D[0] * k[0];
+#pragma unroll
+      for (int r = 1; r < R; ++r) pm += D[r] * k[r];
+      const float q[R] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+      float m = pm, o = po2, pt = S[0] * q[0];
+#pragma unroll
+      for (int i = 0; i < 15; ++i) {
+        m = pm + row_shr1(m); o = po2 + row_shr1(o);
+        if (i & 1) { if (i / 2 + 1 < R) pt += S[i / 2 + 1] * q[i / 2 + 1]; }
       }
-      out4(po[0], po[1], po[2], dot(qp[(TB - 1) & 1]), TB - 4);
-    } else for (int t = 0; t < n; ++t) { const Tok x = get(buf, t); step(x); const float o = dot(x.q); out4(o, o, o, o, t); }          // (rows t .. t + 3, all but the first overwritten; os has three to spare)
+      if (rg == 15) os[buf][max(t - 2, 0)][jl] = o;          // (the first two tokens' write nothing of use: the next one overwrites it)
+      const float delta = (c.v - row_last(m)) * c.g.y;
+#pragma unroll
+      for (int r = 0; r < R; ++r) S[r] = D[r] + k[r] * delta;
+      po2 = pt; qa = c.q0; qb = c.q1;
+    };
+    // a token ahead: the wave is alone on its SIMD, nothing else hides the reads; two sets of registers taking turns
+    Tok x0 = get(buf, 0), x1;
+    int t = 0;
+    for (; t + 1 < n; t += 2) { x1 = get(buf, t + 1); step(x0, t); x0 = get(buf, min(t + 2, n - 1)); step(x1, t + 1); }
+    if (t < n) step(x0, t);
+    po1 = terms();
+    { float o = po2, o1 = po1;
+#pragma unroll
+      for (int i = 0; i < 15; ++i) { o = po2 + row_shr1(o); o1 = po1 + row_shr1(o1); }
+      if (rg == 15) { if (n > 1) os[buf][n - 2][jl] = o; os[buf][n - 1][jl] = o1; } }
     if (t0 + TB < T) store(buf ^ 1);
     lds_barrier();
-    if (tid < 256 && (tid >> 4) < n) oraw[(size_t)(t0 + (tid >> 4)) * w + (size_t)h * p.dv + cb + (tid & 15)] = os[buf][tid >> 4][tid & 15];
+    if ((tid >> 4) < n) oraw[(size_t)(t0 + (tid >> 4)) * w + (size_t)h * p.dv + cb + (tid & 15)] = os[buf][tid >> 4][tid & 15];
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) ssm_out[so + (size_t)r * p.dv] = S[r];
+}
+
+// The same for layers in the head-a-workgroup form (k_gdn_delta: four groups of 32 rows a column): a quad of lanes a column, a lane its
+// group's 32 rows, the four sums by quad broadcasts in order.  grid (nv, 2), 4 waves: 64 columns a workgroup.
+template <int I> __device__ __forceinline__ float quad_lane(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), I * 0x55, 0xf, 0xf, true)); }
+__device__ __forceinline__ float quad_sum(float x) { return ((quad_lane<0>(x) + quad_lane<1>(x)) + quad_lane<2>(x)) + quad_lane<3>(x); }
+__global__ __launch_bounds__(256) void k_gdn_rec4(GdnDev p, const float* __restrict__ co, const float2* __restrict__ gates, int T, const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
+  constexpr int TB = 8, R = 32;
+  __shared__ __align__(16) float ks[2][TB][4][R + 4], qs[2][TB][4][R + 4];          // (a group's row padded: four groups, four banks)
+  __shared__ float vs[2][TB][64]; __shared__ float2 gb[2][TB];
+  const int h = blockIdx.x, cb = blockIdx.y * 64, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, g = lane & 3;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), jl = wave * 16 + (lane >> 2);
+  const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv, w = p.nv * p.dv;
+  const size_t so = ((size_t)h * DK + g * R) * p.dv + cb + jl;
+  float S[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) S[r] = ssm_in[so + (size_t)r * p.dv];
+  auto load = [&](int t0, int buf) {          // eight tokens: 128 k, 128 q, 64 v each
+    for (int i = tid; i < TB * DK; i += 256) { const int t = min(t0 + i / DK, T - 1), c = i % DK; const float* r = co + (size_t)t * ch + kh * DK + c; ks[buf][i / DK][c >> 5][c & 31] = r[nqk]; qs[buf][i / DK][c >> 5][c & 31] = r[0]; }
+    for (int i = tid; i < TB * 64; i += 256) vs[buf][i >> 6][i & 63] = co[(size_t)min(t0 + (i >> 6), T - 1) * ch + 2 * nqk + (size_t)h * p.dv + cb + (i & 63)];
+    if (tid < TB) gb[buf][tid] = gates[(size_t)min(t0 + tid, T - 1) * p.nv + h];
+  };
+  load(0, 0);
+  lds_barrier();
+  for (int t0 = 0, buf = 0; t0 < T; t0 += TB, buf ^= 1) {
+    if (t0 + TB < T) load(t0 + TB, buf ^ 1);
+    const int n = min(TB, T - t0);
+    struct Row { float4 v[8]; };
+    auto row = [&](const float* x) { Row r;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) r.v[i] = *(const float4*)(x + 4 * i);
+      return r; };
+    Row k = row(ks[buf][0][g]);
+    for (int t = 0; t < n; ++t) {          // (the query is read behind the keys' sums, the next token's keys behind the query's)
+      const float2 gt = gb[buf][t]; const float vt = vs[buf][t][jl];
+      const Row q = row(qs[buf][t][g]);
+      const float* kk = (const float*)&k; const float* qq = (const float*)&q;
+      float pm = 0.0f;
+#pragma unroll
+      for (int r = 0; r < R; ++r) { S[r] *= gt.x; pm += S[r] * kk[r]; }
+      const float delta = (vt - quad_sum(pm)) * gt.y;
+#pragma unroll
+      for (int r = 0; r < R; ++r) S[r] += kk[r] * delta;
+      k = row(ks[buf][min(t + 1, n - 1)][g]);
+      float po = 0.0f;
+#pragma unroll
+      for (int r = 0; r < R; ++r) po += S[r] * qq[r];
+      const float o = quad_sum(po);
+      if (g == 0) oraw[(size_t)(t0 + t) * w + (size_t)h * p.dv + cb + jl] = o;
+    }
+    lds_barrier();
   }
 #pragma unroll
   for (int r = 0; r < R; ++r) ssm_out[so + (size_t)r * p.dv] = S[r];
@@ -334,8 +388,8 @@ int pyre_gdn_chunk_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, con
   return PYRE_OK;
 }
 
-// the same steps with the recurrence token by token, bit for bit that of the windows' kernels (pyre_gdn_launch); ssm_in == ssm_out is fine, conv_in == conv_out is not
-int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int stride, int T, const float* conv_in, float* conv_out, const float* ssm_in, float* ssm_out, float* oraw) {
+// the same steps with the recurrence token by token, bit for bit that of the windows' kernels (pyre_gdn_launch with GdnQ); ssm_in == ssm_out is fine, conv_in == conv_out is not
+int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const float* proj, int stride, int T, const float* conv_in, float* conv_out, const float* ssm_in, float* ssm_out, float* oraw, bool quarters) {
   if (g.dk != 128 || g.dv != 128) return pyre_fail(ctx, PYRE_E_SHAPE, "gdn prompt: head dims %dx%d unsupported (128x128 only)", g.dk, g.dv);
   if (T < 1 || g.conv_k < 1 || g.conv_k > 8 || conv_in == conv_out) return pyre_fail(ctx, PYRE_E_ARG, "gdn prompt: %d tokens, %d taps%s", T, g.conv_k, conv_in == conv_out ? ", the history in place" : "");
   const int ch = 2 * g.nk * g.dk + g.nv * g.dv, Tp = (T + 15) / 16 * 16;
@@ -343,6 +397,7 @@ int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const
     if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256 + 1, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr, (float2*)b.dec);
     else hipLaunchKernelGGL(k_gdnc_conv<0>, dim3((ch + 255) / 256 + 1, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr, (float2*)b.dec); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "gdn_prompt_rec", 8.0 * g.nv * g.dk * g.dv + 4.0 * T * (ch + 2.0 * g.nv * g.dv));
-    hipLaunchKernelGGL(k_gdn_rec, dim3(g.nv, g.dv / 16), dim3(512), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
+    if (!quarters) hipLaunchKernelGGL(k_gdn_rec4, dim3(g.nv, g.dv / 64), dim3(256), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw);
+    else hipLaunchKernelGGL(k_gdn_rec, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
   return PYRE_OK;
 }

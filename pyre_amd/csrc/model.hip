@@ -525,7 +525,8 @@ static int prompt_pipe_state(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, 
 static bool fuse_aop_on() { const char* e = getenv("PYRE_AOP_SPLIT"); return !(e && *e && atoi(e) != 0); }
 static bool outp_in_parts(const Layer& L, int d) { return pyre_gemv_parts_ok(L.outp) && (int)L.outp.rows == d && L.hcf.di.fmt == FMT_IQ3_S; }
 // A Gated DeltaNet layer whose output projection is on the matrix cores runs its recurrence on nv x 4 workgroups and leaves
-// the head norm to that projection (GdnQ / PyreAop::sq).  PYRE_GDN_Q=0: nv workgroups.
+// the head norm to that projection (GdnQ / PyreAop::sq) -- in every call that touches the layer's state, the re-run of
+// pyre_spec_keep included: the two forms of the kernel round the state differently.  PYRE_GDN_Q=0: nv workgroups.
 static bool gdn_q_on(const pyre_model* m, const Layer& L) {
   const char* e = getenv("PYRE_GDN_Q");
   return !(e && *e && atoi(e) == 0) && fuse_aop_on() && !L.full && L.outp.fmt == FMT_IQ3_S_M && L.gdn.dv == 128 && L.gdn.dk == 128 && L.outp.cols == L.gdn.nv * 128 && m->gdn_sq != nullptr;
@@ -668,7 +669,7 @@ static int run_rows(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBlk
       if ((rc = mul(L.outp, B->core, B->o))) return rc;
     } else {
       const int li = L.mix_index, b = s->cur[li], nb = b ^ 1; const bool q = gdn_q_on(m, L);
-      if ((rc = pyre_gdn_rec_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], q ? B->core : (float*)B->op))) return rc;
+      if ((rc = pyre_gdn_rec_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], q ? B->core : (float*)B->op, q))) return rc;
       s->cur[li] = nb;
       if (q) {
         if ((rc = pyre_blk_gdn_out_q_launch(ctx, B->core, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, B->op, (size_t)oc * 2, B->inv, oc / 16))) return rc;
@@ -725,7 +726,7 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
       }
     } else {
       const int li = L.mix_index, b = s->cur[li], nb = b ^ 1;
-      if ((rc = pyre_gdn_rec_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], om ? B->core : (float*)B->op))) return rc;
+      if ((rc = pyre_gdn_rec_launch(ctx, L.gdn, B->gdn, B->proj, pw, T, s->conv[b][li], s->conv[nb][li], s->ssm[b][li], s->ssm[nb][li], om ? B->core : (float*)B->op, om))) return rc;
       s->cur[li] = nb;
       if (om) {
         if ((rc = pyre_blk_gdn_out_q_launch(ctx, B->core, B->proj + m->ch, pw, L.gdn.norm_w, c.eps, c.lin_nv, T, B->op, gs(oc), B->inv, oc / 16))) return rc;
