@@ -220,22 +220,48 @@ __global__ __launch_bounds__(256) void k_gdnc_scan(GdnDev p, const float* __rest
   for (int i = tid; i < DK * 16; i += 256) sout[(size_t)(i >> 4) * p.dv + (i & 15)] = St[i & 15][i >> 4];
 }
 
-// ---- the recurrence token by token, the bits of k_gdn_delta_q -------------------------------------------------------------------
+// ---- the recurrence token by token, the bits of the step and window kernels -------------------------------------------------------
 // A prompt of the model takes this one: its state and outputs are then those of decoding the tokens in windows, to the bit, so
-// that no token's expert choice tips with the path the prompt took.  k_gdn_delta_q keeps 32 columns a workgroup, eight rows a
-// thread, and adds the sixteen row groups' sums through shared memory behind a barrier: 0.9 us a token.  Here a wave keeps
-// four columns, a row of sixteen lanes (a lane: eight rows) each: the sums meet in the same order by DPP row shifts
-// (x <- p + x of the lane before, fifteen times: the last lane has ((p0 + p1) + p2) + ..), without a barrier, and the
-// output's sums of one token run in the wait slots of the next token's.  About 100 vector instructions a token, one wave a SIMD
-// for 32 heads (the recurrence is a chain, so further waves would only share the SIMD).
+// that no token's expert choice tips with the path the prompt took.  The step kernels add their row groups' sums through shared
+// memory behind a barrier: 0.9 us a token.  Here a wave keeps four columns, a row of sixteen lanes (a lane: eight rows) each, and the sums
+// meet in the step kernels' order without a barrier: one lane after the other's sum is an operand of the add, read by a row shift, so
+// that the running sum itself never passes through a shift (a value that was just written can be shifted only two instructions later:
+// x <- p + x of the lane before, fifteen times, took three slots a step).  The output's row-group sums go to the wave's own shared memory and are
+// added sixteen tokens at a time, a lane an output.  About 80 vector instructions a token, one wave a SIMD for 32 heads (the recurrence is a
+// chain, so further waves would only share the SIMD).  2048 tokens of the A3B layer: both chains by shifts of the running sum 574 us, the output's through
+// shared memory and the sum unshifted 481, moves apart from the adds 421; 200 tokens of the other form 160 -> 81.
+// QUARTERS: k_gdn_delta_q's sums, sixteen groups of eight rows; else k_gdn_delta's, four groups of 32 rows (a quad of lanes), whose
+// output is summed on the spot.
 // grid (nv, 8), 4 waves: workgroup (h, y) columns 16 y .. of head h.  The keys, queries (normalised, co of k_gdnc_conv), values and gate
 // inputs of sixteen tokens at a time go through shared memory, the next sixteen in registers meanwhile.
-__device__ __forceinline__ float row_shr1(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x111, 0xf, 0xf, true)); }
-__device__ __forceinline__ float row_last(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x15F, 0xf, 0xf, true)); }
+template <int CTRL> __device__ __forceinline__ float dpp(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true)); }
+// ... as a move of its own: folded into the add that uses it, the running sum would be an operand of a shifting instruction, two slots after its last
+template <int CTRL> __device__ __forceinline__ float dpp_mov(float x) { float v = dpp<CTRL>(x); asm("" : "+v"(v)); return v; }
+// lane 15 of a row: ((p of lane 0 + p of lane 1) + p of lane 2) + ..
+__device__ __forceinline__ float row_chain16(float p) {
+  const float v[15] = {dpp_mov<0x11F>(p), dpp_mov<0x11E>(p), dpp_mov<0x11D>(p), dpp_mov<0x11C>(p), dpp_mov<0x11B>(p), dpp_mov<0x11A>(p), dpp_mov<0x119>(p), dpp_mov<0x118>(p),
+                       dpp_mov<0x117>(p), dpp_mov<0x116>(p), dpp_mov<0x115>(p), dpp_mov<0x114>(p), dpp_mov<0x113>(p), dpp_mov<0x112>(p), dpp_mov<0x111>(p)};
+  float x = v[0];
+#pragma unroll
+  for (int i = 1; i < 15; ++i) x += v[i];
+  return x + p;
+}
+template <int L> __device__ __forceinline__ void quad_add8(const float (&p)[8], float& x) {          // x += lane L of the quad's eight, in order
+#pragma unroll
+  for (int r = 0; r < 8; ++r) { const float v = dpp_mov<L * 0x55>(p[r]); x = (L == 0 && r == 0) ? v : x + v; }
+}
+// lane 15 of a row: four quads' sums of 32 products in order, added in order
+__device__ __forceinline__ float row_chain32(const float (&p)[8]) {
+  float x = 0.0f; quad_add8<0>(p, x); quad_add8<1>(p, x); quad_add8<2>(p, x); quad_add8<3>(p, x);
+  return ((dpp_mov<0x11C>(x) + dpp_mov<0x118>(x)) + dpp_mov<0x114>(x)) + x;
+}
+template <bool QUARTERS>
 __global__ __launch_bounds__(256) void k_gdn_rec(GdnDev p, const float* __restrict__ co, const float2* __restrict__ gates, int T, const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
-  constexpr int TB = 16, R = 8;
+  constexpr int TB = 16, R = 8, OP = 20;
   __shared__ __align__(16) float4 kq[2][TB][2][2][16];          // [buffer][token][k, q][rows 0-3, 4-7 of a row group][row group]
-  __shared__ float vs[2][TB][16], os[2][TB][16]; __shared__ float2 gb[2][TB];
+  __shared__ float vs[2][TB][16]; __shared__ float2 gb[2][TB];
+  // the wave's output terms: [token][column][row group], or of four tokens [token][column][row] (in steps of 36: a row group's 32)
+  __shared__ __align__(16) float po[4][QUARTERS ? TB * 4 * OP : 4 * 4 * 4 * 36];
   const int h = blockIdx.x, cb = blockIdx.y * 16, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, rg = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), jl = wave * 4 + (lane >> 4), col = cb + jl;
   const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv, w = p.nv * p.dv;
@@ -258,105 +284,68 @@ __global__ __launch_bounds__(256) void k_gdn_rec(GdnDev p, const float* __restri
   };
   struct Tok { float4 k0, k1, q0, q1; float2 g; float v; };
   auto get = [&](int buf, int t) { return Tok{kq[buf][t][0][0][rg], kq[buf][t][0][1][rg], kq[buf][t][1][0][rg], kq[buf][t][1][1][rg], gb[buf][t], vs[buf][t][jl]}; };
+  auto step = [&](const Tok& c) {
+    const float k[R] = {c.k0.x, c.k0.y, c.k0.z, c.k0.w, c.k1.x, c.k1.y, c.k1.z, c.k1.w}; float m;
+#pragma unroll
+    for (int r = 0; r < R; ++r) S[r] *= c.g.x;
+    if constexpr (QUARTERS) {
+      float pm = S[0] * k[0];
+#pragma unroll
+      for (int r = 1; r < R; ++r) pm += S[r] * k[r];
+      m = row_chain16(pm);
+    } else {
+      float pr[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) pr[r] = S[r] * k[r];
+      m = row_chain32(pr);
+    }
+    const float delta = (c.v - dpp<0x15F>(m)) * c.g.y;          // (lane 15's)
+#pragma unroll
+    for (int r = 0; r < R; ++r) S[r] += k[r] * delta;
+  };
+  auto out = [&](const Tok& c, int t) {
+    const float q[R] = {c.q0.x, c.q0.y, c.q0.z, c.q0.w, c.q1.x, c.q1.y, c.q1.z, c.q1.w};
+    if constexpr (QUARTERS) {
+      float o = S[0] * q[0];
+#pragma unroll
+      for (int r = 1; r < R; ++r) o += S[r] * q[r];
+      po[wave][(t * 4 + (lane >> 4)) * OP + rg] = o;
+    } else {
+      float4* d = (float4*)&po[wave][(((t & 3) * 4 + (lane >> 4)) * 4 + (rg >> 2)) * 36 + (rg & 3) * 8];
+      d[0] = make_float4(S[0] * q[0], S[1] * q[1], S[2] * q[2], S[3] * q[3]); d[1] = make_float4(S[4] * q[4], S[5] * q[5], S[6] * q[6], S[7] * q[7]);
+    }
+  };
+  // four tokens' outputs from their products: lane = (token, column, row group), then the groups in order
+  auto out4 = [&](int t) {
+    __builtin_amdgcn_wave_barrier();
+    const float4* s = (const float4*)&po[wave][lane * 36]; float x = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) { const float4 v = s[i]; x = i == 0 ? v.x : x + v.x; x += v.y; x += v.z; x += v.w; }
+    const float o = ((dpp_mov<0x00>(x) + dpp_mov<0x55>(x)) + dpp_mov<0xAA>(x)) + dpp_mov<0xFF>(x);
+    const int ti = t + (lane >> 4);
+    if ((lane & 3) == 0 && ti < T) oraw[(size_t)ti * w + (size_t)h * p.dv + cb + wave * 4 + ((lane >> 2) & 3)] = o;
+    __builtin_amdgcn_wave_barrier();
+  };
   fetch(0); store(0);
   lds_barrier();
   for (int t0 = 0, buf = 0; t0 < T; t0 += TB, buf ^= 1) {
     if (t0 + TB < T) fetch(t0 + TB);
     const int n = min(TB, T - t0);
-    // In the wait slots of token t's chain: the output terms of token t - 1 (its state is still there: the decayed one goes to
-    // other registers) and the output chain of token t - 2.
-    float po2 = 0.0f, po1 = 0.0f; float4 qa = make_float4(0.0f, 0.0f, 0.0f, 0.0f), qb = qa;          // chain input of token t - 2; the query of token t - 1
-    auto terms = [&]() { const float q[R] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w}; float o = S[0] * q[0];
+    if (n == TB) {          // a token ahead: the wave is alone on its SIMD, nothing else hides the reads; two sets of registers taking turns
+      Tok x[2]; x[0] = get(buf, 0);
 #pragma unroll
-      for (int r = 1; r < R; ++r) o += S[r] * q[r];
-      return o; };
-    auto step = [&](const Tok& c, int t) {
-      const float k[R] = {c.k0.x, c.k0.y, c.k0.z, c.k0.w, c.k1.x, c.k1.y, c.k1.z, c.k1.w};
-      float D[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) D[r] = S[r] * c.g.x;
-      float pm = D[0] * k[0];
-#pragma unroll
-      for (int r = 1; r < R; ++r) pm += D[r] * k[r];
-      const float q[R] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
-      float m = pm, o = po2, pt = S[0] * q[0];
-#pragma unroll
-      for (int i = 0; i < 15; ++i) {
-        m = pm + row_shr1(m); o = po2 + row_shr1(o);
-        if (i & 1) { if (i / 2 + 1 < R) pt += S[i / 2 + 1] * q[i / 2 + 1]; }
+      for (int t = 0; t < TB; ++t) { if (t + 1 < TB) x[(t + 1) & 1] = get(buf, t + 1); step(x[t & 1]); out(x[t & 1], t); if (!QUARTERS && (t & 3) == 3) out4(t0 + t - 3); }
+    } else for (int t = 0; t < n; ++t) { const Tok x = get(buf, t); step(x); out(x, t); if (!QUARTERS && ((t & 3) == 3 || t + 1 == n)) out4(t0 + (t & ~3)); }
+    if constexpr (QUARTERS) {          // lane = (token to, column c of the wave's four)
+      __builtin_amdgcn_wave_barrier();
+      const int to = lane >> 2, c = lane & 3;
+      if (to < n) {
+        const float4* s = (const float4*)&po[wave][(to * 4 + c) * OP]; const float4 a = s[0], b = s[1], d = s[2], e = s[3];
+        oraw[(size_t)(t0 + to) * w + (size_t)h * p.dv + cb + wave * 4 + c] = ((((((((((((((a.x + a.y) + a.z) + a.w) + b.x) + b.y) + b.z) + b.w) + d.x) + d.y) + d.z) + d.w) + e.x) + e.y) + e.z) + e.w;
       }
-      if (rg == 15) os[buf][max(t - 2, 0)][jl] = o;          // (the first two tokens' write nothing of use: the next one overwrites it)
-      const float delta = (c.v - row_last(m)) * c.g.y;
-#pragma unroll
-      for (int r = 0; r < R; ++r) S[r] = D[r] + k[r] * delta;
-      po2 = pt; qa = c.q0; qb = c.q1;
-    };
-    // a token ahead: the wave is alone on its SIMD, nothing else hides the reads; two sets of registers taking turns
-    Tok x0 = get(buf, 0), x1;
-    int t = 0;
-    for (; t + 1 < n; t += 2) { x1 = get(buf, t + 1); step(x0, t); x0 = get(buf, min(t + 2, n - 1)); step(x1, t + 1); }
-    if (t < n) step(x0, t);
-    po1 = terms();
-    { float o = po2, o1 = po1;
-#pragma unroll
-      for (int i = 0; i < 15; ++i) { o = po2 + row_shr1(o); o1 = po1 + row_shr1(o1); }
-      if (rg == 15) { if (n > 1) os[buf][n - 2][jl] = o; os[buf][n - 1][jl] = o1; } }
-    if (t0 + TB < T) store(buf ^ 1);
-    lds_barrier();
-    if ((tid >> 4) < n) oraw[(size_t)(t0 + (tid >> 4)) * w + (size_t)h * p.dv + cb + (tid & 15)] = os[buf][tid >> 4][tid & 15];
-  }
-#pragma unroll
-  for (int r = 0; r < R; ++r) ssm_out[so + (size_t)r * p.dv] = S[r];
-}
-
-// The same for layers in the head-a-workgroup form (k_gdn_delta: four groups of 32 rows a column): a quad of lanes a column, a lane its
-// group's 32 rows, the four sums by quad broadcasts in order.  grid (nv, 2), 4 waves: 64 columns a workgroup.
-template <int I> __device__ __forceinline__ float quad_lane(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), I * 0x55, 0xf, 0xf, true)); }
-__device__ __forceinline__ float quad_sum(float x) { return ((quad_lane<0>(x) + quad_lane<1>(x)) + quad_lane<2>(x)) + quad_lane<3>(x); }
-__global__ __launch_bounds__(256) void k_gdn_rec4(GdnDev p, const float* __restrict__ co, const float2* __restrict__ gates, int T, const float* __restrict__ ssm_in, float* __restrict__ ssm_out, float* __restrict__ oraw) {
-  constexpr int TB = 8, R = 32;
-  __shared__ __align__(16) float ks[2][TB][4][R + 4], qs[2][TB][4][R + 4];          // (a group's row padded: four groups, four banks)
-  __shared__ float vs[2][TB][64]; __shared__ float2 gb[2][TB];
-  const int h = blockIdx.x, cb = blockIdx.y * 64, kh = h % p.nk, tid = threadIdx.x, lane = tid & 63, g = lane & 3;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), jl = wave * 16 + (lane >> 2);
-  const int nqk = p.nk * DK, ch = 2 * nqk + p.nv * p.dv, w = p.nv * p.dv;
-  const size_t so = ((size_t)h * DK + g * R) * p.dv + cb + jl;
-  float S[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) S[r] = ssm_in[so + (size_t)r * p.dv];
-  auto load = [&](int t0, int buf) {          // eight tokens: 128 k, 128 q, 64 v each
-    for (int i = tid; i < TB * DK; i += 256) { const int t = min(t0 + i / DK, T - 1), c = i % DK; const float* r = co + (size_t)t * ch + kh * DK + c; ks[buf][i / DK][c >> 5][c & 31] = r[nqk]; qs[buf][i / DK][c >> 5][c & 31] = r[0]; }
-    for (int i = tid; i < TB * 64; i += 256) vs[buf][i >> 6][i & 63] = co[(size_t)min(t0 + (i >> 6), T - 1) * ch + 2 * nqk + (size_t)h * p.dv + cb + (i & 63)];
-    if (tid < TB) gb[buf][tid] = gates[(size_t)min(t0 + tid, T - 1) * p.nv + h];
-  };
-  load(0, 0);
-  lds_barrier();
-  for (int t0 = 0, buf = 0; t0 < T; t0 += TB, buf ^= 1) {
-    if (t0 + TB < T) load(t0 + TB, buf ^ 1);
-    const int n = min(TB, T - t0);
-    struct Row { float4 v[8]; };
-    auto row = [&](const float* x) { Row r;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) r.v[i] = *(const float4*)(x + 4 * i);
-      return r; };
-    Row k = row(ks[buf][0][g]);
-    for (int t = 0; t < n; ++t) {          // (the query is read behind the keys' sums, the next token's keys behind the query's)
-      const float2 gt = gb[buf][t]; const float vt = vs[buf][t][jl];
-      const Row q = row(qs[buf][t][g]);
-      const float* kk = (const float*)&k; const float* qq = (const float*)&q;
-      float pm = 0.0f;
-#pragma unroll
-      for (int r = 0; r < R; ++r) { S[r] *= gt.x; pm += S[r] * kk[r]; }
-      const float delta = (vt - quad_sum(pm)) * gt.y;
-#pragma unroll
-      for (int r = 0; r < R; ++r) S[r] += kk[r] * delta;
-      k = row(ks[buf][min(t + 1, n - 1)][g]);
-      float po = 0.0f;
-#pragma unroll
-      for (int r = 0; r < R; ++r) po += S[r] * qq[r];
-      const float o = quad_sum(po);
-      if (g == 0) oraw[(size_t)(t0 + t) * w + (size_t)h * p.dv + cb + jl] = o;
+      __builtin_amdgcn_wave_barrier();
     }
+    if (t0 + TB < T) store(buf ^ 1);
     lds_barrier();
   }
 #pragma unroll
@@ -397,7 +386,7 @@ int pyre_gdn_rec_launch(pyre_ctx* ctx, const GdnDev& g, const GdnChunk& b, const
     if (g.conv_k == 4) hipLaunchKernelGGL(k_gdnc_conv<4>, dim3((ch + 255) / 256 + 1, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr, (float2*)b.dec);
     else hipLaunchKernelGGL(k_gdnc_conv<0>, dim3((ch + 255) / 256 + 1, Tp / 16), dim3(256), 0, ctx->stream, g, proj, stride, T, Tp, conv_in, conv_out, b.co, (float*)nullptr, (float2*)b.dec); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "gdn_prompt_rec", 8.0 * g.nv * g.dk * g.dv + 4.0 * T * (ch + 2.0 * g.nv * g.dv));
-    if (!quarters) hipLaunchKernelGGL(k_gdn_rec4, dim3(g.nv, g.dv / 64), dim3(256), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw);
-    else hipLaunchKernelGGL(k_gdn_rec, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
+    if (!quarters) hipLaunchKernelGGL(k_gdn_rec<false>, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw);
+    else hipLaunchKernelGGL(k_gdn_rec<true>, dim3(g.nv, g.dv / 16), dim3(256), 0, ctx->stream, g, b.co, (const float2*)b.dec, T, ssm_in, ssm_out, oraw); } PYRE_CHECK_LAUNCH(ctx);
   return PYRE_OK;
 }
