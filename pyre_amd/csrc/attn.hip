@@ -155,6 +155,23 @@ __device__ __forceinline__ h8v nib8_f16(uint32_t w) {
   for (int q = 0; q < 4; ++q) u.v[q] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2v, ((x >> (4 * q)) & 0x000F000Fu) | 0x64006400u) - off);
   return __builtin_bit_cast(h8v, u);
 }
+// Sums (or maxima) over the wave of N = 1, 2 or 4 values a lane, in wave_sum's order of adding: pairs and quads of lanes keep a value each
+// from the first steps on, so that four cost little more than one.  Lanes 12 + i hold value i's.
+template <int CTRL> __device__ __forceinline__ float col_dpp(float x) { return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true)); }
+template <bool MAX> __device__ __forceinline__ float col_op(float a, float b) { return MAX ? __builtin_amdgcn_fmed3f(a, b, INFINITY) : a + b; }
+template <bool MAX, int N> __device__ __forceinline__ float wave_cols(const float (&v)[N], int lane) {
+  const bool b0 = lane & 1, b1 = lane & 2; float x;
+  if constexpr (N == 4) {
+    const float u = col_op<MAX>(b0 ? v[1] : v[0], col_dpp<0xB1>(b0 ? v[0] : v[1])), w = col_op<MAX>(b0 ? v[3] : v[2], col_dpp<0xB1>(b0 ? v[2] : v[3]));
+    x = col_op<MAX>(b1 ? w : u, col_dpp<0x4E>(b1 ? u : w));
+  } else {
+    if constexpr (N == 2) x = col_op<MAX>(b0 ? v[1] : v[0], col_dpp<0xB1>(b0 ? v[0] : v[1])); else x = col_op<MAX>(v[0], col_dpp<0xB1>(v[0]));
+    x = col_op<MAX>(x, col_dpp<0x4E>(x));
+  }
+  x = col_op<MAX>(x, col_dpp<0x124>(x)); x = col_op<MAX>(x, col_dpp<0x128>(x));          // rotations by a quad and by two: the last quad has (3 + 2) + (1 + 0)
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false); x = col_op<MAX>(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false); return col_op<MAX>(__uint_as_float(h[0]), __uint_as_float(h[1]));
+}
 // One pass: chunk `chunk` of KV head kvh for tokens tk0 .. tk0 + nk - 1 of the launch.
 // NC: columns the buffers hold -- G for launches of one token a pass (tp = 1), 16 otherwise.
 template <int NC> struct AttnSm {
@@ -166,8 +183,8 @@ template <int HD, int G, int NC>
 __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, const KvDev& kv, const float* __restrict__ qbuf, const uint16_t* __restrict__ qh, const float* __restrict__ qsc, int start, float* __restrict__ part_o, float* __restrict__ part_ml, int max_chunks, int chunk, int kvh, int tk0, int nk) {
   static_assert(HD == 256, "the wave layout assumes 4 x 64 head dims");
   constexpr int NPW = PYRE_ATTN_NPW, CH = PYRE_ATTN_CHUNK, NT = 256 * NPW;
-  constexpr int RS = CH + 4;
-  static_assert(4 * RS >= NPW * HD, "the score and value partials share one buffer");
+  constexpr int RS = CH + 4, VS = HD + 8;          // (eight floats more a row of value partials: the rows a store reaches at a time then meet few banks twice)
+  static_assert(4 * RS >= NPW * VS, "the score and value partials share one buffer");
   auto& red = sm.red; auto& sc = sm.sc; auto& wmax = sm.wmax; auto& wsum = sm.wsum;
   PYRE_TS_VARS PYRE_TS(0);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -190,35 +207,38 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
   // All of it through buffer descriptors: one 32-bit offset per array and lane, the rest of an address is a constant
   // of the instruction or a scalar.
   const int pos = pw * 64 + lane;
-  constexpr int GH = (NC + 3) / 4;
+  // The columns a pass lacks (ncol .. NC - 1) go through like the others, whatever they hold: a column's sums do not depend on its neighbours,
+  // the buffers have rows for NC, and nobody reads theirs.  Behind a branch for each register and column the phases were a chain of
+  // mask instructions and of shifts waiting for their operands.  540 launches of a prompt of 8192 tokens, us each: 131; without the branches 126, four columns'
+  // maxima and sums in one tree (wave_cols) 114, rows of value partials in steps of 264 floats 110.  (Several passes a workgroup over a chunk kept in registers: a
+  // third fewer instructions a pass, 106; not kept.)
+  constexpr int GH = (NC + 3) / 4, NCQ = (NC + 3) / 4;
   // chunk-local max / exp / sum per head; called by every wave after the barrier that follows its scores
   auto softmax_phase = [&]() {
-    float sv[GH];
+    float sv[GH], ev[GH];
+    const bool any = NC % 4 == 0 || dq < NC, left = any && lane >= 12 && lane < 12 + GH; const int cl = dq + 4 * (lane - 12);          // the column whose results the lane leaves
 #pragma unroll
     for (int gi = 0; gi < GH; ++gi) {
-      const int c = dq + 4 * gi; sv[gi] = -INFINITY;
-      if (c < ncol) {
-        const bool valid = p < start + tk0 + c / G + 1;          // the column's token sees positions below its own + 1
-        float v = ((red[(0 * NC + c) * RS + pos] + red[(1 * NC + c) * RS + pos]) + red[(2 * NC + c) * RS + pos]) + red[(3 * NC + c) * RS + pos];
-        sv[gi] = valid ? v * scale : -INFINITY;
-        const float m = wave_max(sv[gi]);
-        if (lane == 0) wmax[pw][c] = m;
-      }
+      const int c = any ? dq + 4 * gi : 0;
+      const bool valid = p < start + tk0 + c / G + 1;          // the column's token sees positions below its own + 1
+      float v = ((red[(0 * NC + c) * RS + pos] + red[(1 * NC + c) * RS + pos]) + red[(2 * NC + c) * RS + pos]) + red[(3 * NC + c) * RS + pos];
+      asm volatile("" : "+v"(v));          // (read whether it counts or not: no branch around the reads)
+      sv[gi] = valid ? v * scale : -INFINITY;
     }
+    const float m = wave_cols<true, GH>(sv, lane);
+    if (left) wmax[pw][cl] = m;
     __syncthreads();
 #pragma unroll
     for (int gi = 0; gi < GH; ++gi) {
-      const int c = dq + 4 * gi;
-      if (c < ncol) {
-        const bool valid = p < start + tk0 + c / G + 1;
-        float mm = wmax[0][c];          // the chunk's maximum of the column: every thread takes it from the waves' maxima itself
+      const int c = any ? dq + 4 * gi : 0;
+      const bool valid = p < start + tk0 + c / G + 1;
+      float mm = wmax[0][c];          // the chunk's maximum of the column: every thread takes it from the waves' maxima itself
 #pragma unroll
-        for (int q = 1; q < NPW; ++q) mm = fmaxf(mm, wmax[q][c]);
-        float e = valid ? expf(sv[gi] - mm) : 0.0f; sc[c][pos] = e;
-        const float l = wave_sum(e);
-        if (lane == 0) wsum[pw][c] = l;
-      }
+      for (int q = 1; q < NPW; ++q) mm = fmaxf(mm, wmax[q][c]);
+      ev[gi] = valid ? expf(sv[gi] - mm) : 0.0f; if (any) sc[c][pos] = ev[gi];
     }
+    const float l = wave_cols<false, GH>(ev, lane);
+    if (left) wsum[pw][cl] = l;
     __syncthreads();          // weights of every position visible; the score partials in `red` are dead
   };
   // A wave is on one of two paths for the whole kernel -- packed positions or f32 ones (the branch is scalar: wbase is a
@@ -290,10 +310,11 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
           for (int r = 0; r < 4; ++r) D[pt][r] = fmaf(ksc[pt][b], d[r], D[pt][r]);
         }
       // register r of tile pt: column 4*lg + r, position 16*pt + li
+      if (lg < NCQ)
 #pragma unroll
       for (int pt = 0; pt < 4; ++pt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) if (4 * lg + r < ncol) red[(dq * NC + 4 * lg + r) * RS + pw * 64 + 16 * pt + li] = D[pt][r] * qinv[r];
+        for (int r = 0; r < 4; ++r) if (NC % 4 == 0 || 4 * lg + r < NC) red[(dq * NC + 4 * lg + r) * RS + pw * 64 + 16 * pt + li] = D[pt][r] * qinv[r];
     }
     PYRE_TS(2);
     __syncthreads(); PYRE_TS(3);
@@ -317,8 +338,8 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
       for (int g = 0; g < 2; ++g) {
         float ev[8];
         { const float4* e4 = (const float4*)&sc[li < NC ? li : 0][pw * 64 + 32 * g + 8 * lg];
-          const float4 e0 = e4[0], e1 = e4[1]; const bool on = li < ncol;
-          ev[0] = on ? e0.x : 0.0f; ev[1] = on ? e0.y : 0.0f; ev[2] = on ? e0.z : 0.0f; ev[3] = on ? e0.w : 0.0f; ev[4] = on ? e1.x : 0.0f; ev[5] = on ? e1.y : 0.0f; ev[6] = on ? e1.z : 0.0f; ev[7] = on ? e1.w : 0.0f; }
+          const float4 e0 = e4[0], e1 = e4[1];
+          ev[0] = e0.x; ev[1] = e0.y; ev[2] = e0.z; ev[3] = e0.w; ev[4] = e1.x; ev[5] = e1.y; ev[6] = e1.z; ev[7] = e1.w; }
         const int vs_bits = __float_as_int(vsl[g] * up);
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
@@ -340,12 +361,13 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
         }
       }
       // register r of (b, m): column 4*lg + r, dim dq*64 + b*32 + 8*(li & 3) + 2*(li >> 2) + m
+      if (lg < NCQ)
 #pragma unroll
       for (int b = 0; b < 2; ++b)
 #pragma unroll
         for (int m = 0; m < 2; ++m)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) if (4 * lg + r < ncol) red[((size_t)pw * NC + 4 * lg + r) * HD + dq * 64 + b * 32 + 8 * (li & 3) + 2 * (li >> 2) + m] = Dv[b][m][r] * dn;
+          for (int r = 0; r < 4; ++r) if (NC % 4 == 0 || 4 * lg + r < NC) red[((size_t)pw * NC + 4 * lg + r) * VS + dq * 64 + b * 32 + 8 * (li & 3) + 2 * (li >> 2) + m] = Dv[b][m][r] * dn;
     }
   } else {
     PYRE_TS(1);
@@ -376,11 +398,11 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
         for (int s = 0; s < 16; ++s)
 #pragma unroll
           for (int pt = 0; pt < 4; ++pt) D[pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[pt][s], B[s], D[pt], 0, 0, 0);
-        if (li < ncol) {
+        if (NC == 16 || li < NC) {
 #pragma unroll
           for (int pt = 0; pt < 4; ++pt) *(float4*)&red[(dq * NC + li) * RS + pw * 64 + 16 * pt + 4 * lg] = make_float4(D[pt][0], D[pt][1], D[pt][2], D[pt][3]);
         }
-      } else if (li < ncol) {          // a wave past the view: its positions carry no weight, their scores are read all the same
+      } else if (NC == 16 || li < NC) {          // a wave past the view: its positions carry no weight, their scores are read all the same
 #pragma unroll
         for (int pt = 0; pt < 4; ++pt) *(float4*)&red[(dq * NC + li) * RS + pw * 64 + 16 * pt + 4 * lg] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       }
@@ -407,7 +429,7 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
       if (active) {
         float B[16];
 #pragma unroll
-        for (int s = 0; s < 16; ++s) B[s] = li < ncol ? sc[li < NC ? li : 0][pw * 64 + 4 * s + lg] : 0.0f;
+        for (int s = 0; s < 16; ++s) B[s] = sc[li < NC ? li : 0][pw * 64 + 4 * s + lg];
 #pragma unroll
         for (int s = 0; s < 16; ++s) {
           const float A[4] = {vf4[s].x, vf4[s].y, vf4[s].z, vf4[s].w};
@@ -415,11 +437,9 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
           for (int dt = 0; dt < 4; ++dt) D[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[dt], B[s], D[dt], 0, 0, 0);
         }
       }
-      if (li < ncol) {
+      if (NC == 16 || li < NC) {
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) red[((size_t)pw * NC + li) * HD + dq * 64 + 4 * (4 * lg + r) + dt] = D[dt][r];
+        for (int r = 0; r < 4; ++r) *(float4*)&red[((size_t)pw * NC + li) * VS + dq * 64 + 4 * (4 * lg + r)] = make_float4(D[0][r], D[1][r], D[2][r], D[3][r]);
       }
     }
   }
@@ -427,9 +447,9 @@ __device__ __forceinline__ void attn_pass(AttnSm<NC>& sm, const AttnDev& a, cons
   __syncthreads(); PYRE_TS(6);
   for (int i = tid; i < ncol * HD; i += NT) {
     const int c = i / HD, dd = i % HD, tk = tk0 + c / G, g = c % G;
-    float o = red[((size_t)0 * NC + c) * HD + dd];
+    float o = red[((size_t)0 * NC + c) * VS + dd];
 #pragma unroll
-    for (int q = 1; q < NPW; ++q) o += red[((size_t)q * NC + c) * HD + dd];
+    for (int q = 1; q < NPW; ++q) o += red[((size_t)q * NC + c) * VS + dd];
     part_o[(((size_t)tk * a.nh + (size_t)kvh * G + g) * max_chunks + chunk) * HD + dd] = o;
   }
   if (tid < ncol) {
