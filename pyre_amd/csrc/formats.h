@@ -406,6 +406,9 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));          // (a caller's rows may start at any float)
 template <class F, int... I> __device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
 template <int N, class F> __device__ __forceinline__ void static_for(F&& f) { static_for_((F&&)f, std::make_integer_sequence<int, N>{}); }          // f(0) .. f(N - 1), the index a constant
+// A group of four tokens costs ten cycles a column on the matrix cores, a token four on the vector pipe: from four tokens on.  (Two and
+// three of a 6144 x 2048 Q4_K matrix on the matrix cores: 8.1 us, on the vector pipe 6.0 and 6.7.)
+#define PYRE_MMA_MIN 4
 template <int NG> struct XGrp { f4u x[NG]; };
 // p[g]: the lane's token of group g, at column 4 (lane / 4)
 template <int NG> __device__ __forceinline__ void unit_x_load(const float* const (&p)[NG], int ku, XGrp<NG>& x) {

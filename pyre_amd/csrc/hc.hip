@@ -12,6 +12,26 @@
 
 PYRE_TS_DECL(hc_ts) PYRE_TS_EXPORT(hc_ts, pyre_debug_ts_hc)
 
+// A unit of a matrix against T tokens in shared memory, rows of xstride floats: from PYRE_MMA_MIN tokens on by the matrix cores (the same bits), which
+// read a unit's activations with one 16-byte load a lane and four tokens where the multiply-adds read every one for every lane.  HC_PAD: the four tokens
+// a wave reads at a time meet four different sets of banks.  200 tokens of A3B's shape, bf16, groups of eight, us: first launch 47 -> 43, second 40 -> 33, with
+// the router 60 -> 42.
+#define HC_PAD 16
+template <int FMT, int T> __device__ __forceinline__ void hc_unit(const QMatDev& m, const UnitRaw<FMT>& r, int ku, int lane, const float* xs, int xstride, float (&acc)[T]) {
+  if constexpr (T < PYRE_MMA_MIN) { const uint2* lds2 = nullptr; unit_fma<FMT, T>(m, r, ku, lds2, lane, xs, xstride, acc); }
+  else {
+    constexpr int NG = (T + 3) / 4; XGrp<NG> x; v4f a[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      const float4 v = *(const float4*)(xs + min(4 * g + (lane & 3), T - 1) * xstride + 4 * (lane >> 2)); x.x[g] = f4u{v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) a[g][t] = 4 * g + t < T ? acc[4 * g + t < T ? 4 * g + t : 0] : 0.0f;
+    }
+    unit_mma<FMT, NG>(m, r, ku, x, a);
+#pragma unroll
+    for (int t = 0; t < T; ++t) acc[t] = a[t >> 2][t & 3];
+  }
+}
 // grid (row tiles of [down ; inject], K slices of a stream, streams x groups of tokens), nw waves.  A workgroup owns L = nw*upw*64 columns
 // of one stream s.
 // The RMS scale of a stream multiplies every term of a row's dot product, so it is applied after the dot (by
@@ -23,7 +43,8 @@ PYRE_TS_DECL(hc_ts) PYRE_TS_EXPORT(hc_ts, pyre_debug_ts_hc)
 // ONE: eight waves of one unit each (every width in multiples of 512 with at most 32 slices): a thread prepares one column and a wave
 // forms one unit's sums, without loops.  FG > 0: the experts a group of the unreduced FFN output (moe_out_value).  One token, bf16,
 // 2048 columns, 6.1 us with the loops and the groups at run time, 5.0 with neither; 500 tokens' groups of eight 218 and 113 us.
-template <int FMT, int T, int NP, bool ONE = false, int FG = 0> __global__ __launch_bounds__(512) void k_hc_norm_down(QMatDev m, const float* __restrict__ x_in, int in_ss, int in_ts, float* __restrict__ x_out,
+// ALLT (groups of eight of a prompt): one workgroup for all row tiles, which otherwise prepare the same columns each: 200 tokens 43 -> 26 us.
+template <int FMT, int T, int NP, bool ONE = false, int FG = 0, bool ALLT = false> __global__ __launch_bounds__(512) void k_hc_norm_down(QMatDev m, const float* __restrict__ x_in, int in_ss, int in_ts, float* __restrict__ x_out,
     const float* __restrict__ comb_out, MoeOut mo, const float* __restrict__ comb_inj, const float* __restrict__ norm, int d, int hc, float* __restrict__ ssq,
     float* __restrict__ part, int upw, const uint2* __restrict__ g2) {
   int s = blockIdx.z;
@@ -35,16 +56,15 @@ template <int FMT, int T, int NP, bool ONE = false, int FG = 0> __global__ __lau
     if (comb_out) comb_out += zt * d;
     if (comb_inj) comb_inj += zt * hc;
   }
-  const uint2* lds2 = nullptr;          // no format needs a codebook in shared memory any more
   PYRE_TS_VARS PYRE_TS(0);
   qmat_args_now(m); args_now(x_in, in_ss, in_ts, x_out, comb_out, mo.partial, mo.sel_w, mo.sg, mo.d, mo.k, comb_inj, norm, d, hc, ssq, part, upw);
   if constexpr (ONE) upw = 1;
   extern __shared__ __align__(16) float sm[];
-  const int nthr = ONE ? 512 : blockDim.x, nw = nthr >> 6, tid = threadIdx.x, L = nw * upw * 64;
-  float* xs = sm;                         // [T][L]
-  float* red = sm + (size_t)T * L;        // [nw][T][64]
-  float* wsum = red + (size_t)nw * T * 64;   // [nw][T]
-  const int tile = blockIdx.x, ks = s * gridDim.y + blockIdx.y;
+  const int nthr = ONE ? 512 : blockDim.x, nw = nthr >> 6, tid = threadIdx.x, L = nw * upw * 64, LP = L + HC_PAD;
+  float* xs = sm;                         // [T][LP]
+  float* red = sm + (size_t)T * LP;       // [nw][T][64], ALLT: twice
+  float* wsum = red + (ALLT ? 2 : 1) * (size_t)nw * T * 64;   // [nw][T]
+  const int tile = ALLT ? 0 : blockIdx.x, ks = s * gridDim.y + blockIdx.y;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int i0 = blockIdx.y * L;
   // Loads return in the order they were issued: the streams (and the pending update's terms) first, since the copy into
@@ -64,7 +84,7 @@ template <int FMT, int T, int NP, bool ONE = false, int FG = 0> __global__ __lau
     for (int t = 0; t < T; ++t) {
       const float v = v0[t];
       ss[t] += v * v;
-      xs[(size_t)t * L + tid] = v * nv0;
+      xs[(size_t)t * LP + tid] = v * nv0;
       if (tile == 0) x_out[((size_t)t * hc + s) * d + i0 + tid] = v;
     }
   }
@@ -74,7 +94,7 @@ template <int FMT, int T, int NP, bool ONE = false, int FG = 0> __global__ __lau
     for (int t = 0; t < T; ++t) {
       float v = hc_x_new<T, NP>(x_in, in_ss, in_ts, comb_out, mo, w[t], d, t, s, i0 + j);
       ss[t] += v * v;
-      xs[(size_t)t * L + j] = v * nv;
+      xs[(size_t)t * LP + j] = v * nv;
       if (tile == 0) x_out[((size_t)t * hc + s) * d + i0 + j] = v;
     }
   }
@@ -86,15 +106,34 @@ template <int FMT, int T, int NP, bool ONE = false, int FG = 0> __global__ __lau
   }
   lds_barrier(); PYRE_TS(1);
   if (tile == 0 && tid < T) { float tot = wsum[tid]; for (int q = 1; q < nw; ++q) tot += wsum[q * T + tid]; ssq[ks * T + tid] = tot; }
+  const size_t r64 = (size_t)m.tiles * 64;
   float acc[T];
+  if constexpr (ALLT) {          // every row tile, the next one's weights in flight, the waves' sums of two tiles taking turns in shared memory
+    static_assert(ONE, "a unit a wave");
+    for (int tl = 0; tl < m.tiles; ++tl) {
+      const UnitRaw<FMT> r = raw; float* rd = red + (size_t)(tl & 1) * nw * T * 64;
+      raw = unit_load<FMT>(m, min(tl + 1, m.tiles - 1), ks * nw + wave, lane);
+#pragma unroll
+      for (int t = 0; t < T; ++t) acc[t] = 0.0f;
+      hc_unit<FMT, T>(m, r, ks * nw + wave, lane, xs + wave * 64, LP, acc);
+#pragma unroll
+      for (int t = 0; t < T; ++t) rd[((size_t)wave * T + t) * 64 + lane] = acc[t];
+      lds_barrier();
+      for (int i = tid; i < T * 64; i += nthr) {
+        const int t = i >> 6, l = i & 63; float a = rd[(size_t)t * 64 + l];
+        for (int q = 1; q < nw; ++q) a += rd[((size_t)q * T + t) * 64 + l];
+        part[((size_t)ks * T + t) * r64 + (size_t)tl * 64 + l] = a;
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int t = 0; t < T; ++t) acc[t] = 0.0f;
-  for (int u = 0; u < upw; ++u) { int lu = wave * upw + u; if (u > 0) raw = unit_load<FMT>(m, tile, ks * nw * upw + lu, lane); unit_fma<FMT, T>(m, raw, ks * nw * upw + lu, lds2, lane, xs + lu * 64, L, acc); }
+  for (int u = 0; u < upw; ++u) { int lu = wave * upw + u; if (u > 0) raw = unit_load<FMT>(m, tile, ks * nw * upw + lu, lane); hc_unit<FMT, T>(m, raw, ks * nw * upw + lu, lane, xs + lu * 64, LP, acc); }
 #pragma unroll
   for (int t = 0; t < T; ++t) red[((size_t)wave * T + t) * 64 + lane] = acc[t];
   PYRE_TS(2);
   lds_barrier(); PYRE_TS(3);
-  const size_t r64 = (size_t)m.tiles * 64;
   for (int i = tid; i < T * 64; i += nthr) {
     int t = i >> 6, l = i & 63; float a = red[(size_t)t * 64 + l];
     for (int q = 1; q < nw; ++q) a += red[((size_t)q * T + t) * 64 + l];
@@ -130,8 +169,9 @@ template <int FMT, int T, int RF, int KSM, int HM, int FLR = 0> __global__ __lau
   extern __shared__ __align__(16) float sm[];
   const int tid = threadIdx.x, U = lr >> 6, nthr = hc * lr, nw = hc * U;
   const float rhc = hc_recip(hc); const int kps = __builtin_amdgcn_readfirstlane(hc_div(ksplit, rhc));
-  float* lo = sm;                         // [T][lr]
-  float* red = sm + (size_t)T * lr;       // [nw][T][64]
+  const int LP = lr + HC_PAD;
+  float* lo = sm;                         // [T][LP]
+  float* red = sm + (size_t)T * LP;       // [nw][T][64]
   float* sls = red + (size_t)nw * T * 64;   // [T][32]: the RMS scale of the stream each slice belongs to
   float* term = sls + (size_t)T * 32;     // [T*hc][64]: the streams' gated, normalized values before they are added
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -172,7 +212,7 @@ template <int FMT, int T, int RF, int KSM, int HM, int FLR = 0> __global__ __lau
   for (int i0 = 0; i0 < n_lo; i0 += nthr) {          // (a launch-uniform count of rounds)
     const int idx = i0 + tid, t = min(hc_div(idx, rlr), T - 1);
     const float v = hc_mean(hc_slice_sum<KSM>(pv, sls + t * 32, ksplit), hc);          // slices in order, each times its stream's scale
-    if (idx < n_lo) lo[idx] = v * sigm(v);
+    if (idx < n_lo) lo[idx + t * HC_PAD] = v * sigm(v);
     if (i0 + nthr < n_lo) {
       if constexpr (AHEAD) {
 #pragma unroll
@@ -191,7 +231,7 @@ template <int FMT, int T, int RF, int KSM, int HM, int FLR = 0> __global__ __lau
   float acc[T];
 #pragma unroll
   for (int t2 = 0; t2 < T; ++t2) acc[t2] = 0.0f;
-  unit_fma<FMT, T>(up, raw, ku, lds2, lane, lo + ku * 64, lr, acc);
+  hc_unit<FMT, T>(up, raw, ku, lane, lo + ku * 64, LP, acc);
 #pragma unroll
   for (int t2 = 0; t2 < T; ++t2) red[((size_t)wave * T + t2) * 64 + lane] = acc[t2];
   if (ROUTE && !R_EARLY && wave < router.tiles) rraw = unit_load<RFX>(router, wave, blockIdx.x, lane);
@@ -212,7 +252,7 @@ template <int FMT, int T, int RF, int KSM, int HM, int FLR = 0> __global__ __lau
     for (int q = 0; q < HM; ++q) if (q < hc) mx += term[(size_t)(t2 * hc + q) * 64 + l];          // streams ascending from zero (:1380)
     const float mv = hc_mean(mx, hc);
     mixed[(size_t)t2 * d + col] = mv;
-    if (ROUTE) lo[t2 * 64 + l] = mv;          // lo is free after the barrier above
+    if (ROUTE) lo[t2 * (64 + HC_PAD) + l] = mv;          // lo is free after the barrier above
   }
   PYRE_TS(5);
   if (ROUTE) {
@@ -220,12 +260,21 @@ template <int FMT, int T, int RF, int KSM, int HM, int FLR = 0> __global__ __lau
     const size_t rr64 = (size_t)router.tiles * 64;
     for (int tile = wave; tile < router.tiles; tile += nw) {
       if (tile != wave) rraw = unit_load<RFX>(router, tile, blockIdx.x, lane);
+      float ra[T];
+#pragma unroll
+      for (int t2 = 0; t2 < T; ++t2) ra[t2] = 0.0f;
+      if constexpr (T >= PYRE_MMA_MIN) hc_unit<RFX, T>(router, rraw, blockIdx.x, lane, lo, 64 + HC_PAD, ra);
+      else {
 #pragma unroll 1
-      for (int t2 = 0; t2 < T; ++t2) {          // one token at a time (same operations per token): T tokens at once would keep 64*T activations in registers
-        float ra[1] = {0.0f};
-        unit_fma<RFX, 1>(router, rraw, blockIdx.x, lds2, lane, lo + t2 * 64, 0, ra);
-        rpart[((size_t)blockIdx.x * T + t2) * rr64 + (size_t)tile * 64 + lane] = ra[0];
+        for (int t2 = 0; t2 < T; ++t2) {          // one token at a time (same operations per token): T tokens at once would keep 64*T activations in registers
+          float r1[1] = {0.0f};
+          unit_fma<RFX, 1>(router, rraw, blockIdx.x, lds2, lane, lo + t2 * (64 + HC_PAD), 0, r1);
+          rpart[((size_t)blockIdx.x * T + t2) * rr64 + (size_t)tile * 64 + lane] = r1[0];
+        }
       }
+      if constexpr (T >= PYRE_MMA_MIN)
+#pragma unroll
+        for (int t2 = 0; t2 < T; ++t2) rpart[((size_t)blockIdx.x * T + t2) * rr64 + (size_t)tile * 64 + lane] = ra[t2];
     }
   }
   PYRE_TS(7); PYRE_TS_FLUSH(hc_ts, ROUTE ? 16 : 24);
@@ -249,7 +298,7 @@ DownPlan down_plan(const HcDev& h) {
 
 template <int FMT, int T> int norm_down_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, const DownPlan& p, const float* x_in, int in_ss, int in_ts, float* x_out,
                                                const float* comb_out, int comb_parts, const MoeOut& mo, const float* comb_inj, float eps, int nz = 1) {
-  const int L = p.nw * p.upw * 64; size_t lds = 4 * ((size_t)T * L + (size_t)p.nw * T * 64 + (size_t)p.nw * T);
+  const int L = p.nw * p.upw * 64; size_t lds = 4 * ((size_t)T * (L + HC_PAD) + (size_t)p.nw * T * 64 + (size_t)p.nw * T);
   ProfScope ps(ctx, "hc_norm_down", qmat_gguf_bytes(h.di, h.di.rows) + 4.0 * T * h.hc * h.d * 4);
 #define NORM_DOWN_GO(NP) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, NP>), dim3(h.di.tiles, p.ksplit / h.hc, nz * h.hc), dim3(p.nw * 64), lds, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, \
                      w.ssq, w.o, p.upw, (const uint2*)ctx->d_iq2xs)
@@ -262,7 +311,7 @@ template <int FMT, int T> int norm_down_launch(pyre_ctx* ctx, const HcDev& h, co
   else if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {
     if (p.nw != 8 || p.upw != 1) NORM_DOWN_GO(1);
     else if (comb_parts > 1) NORM_DOWN_ONE(NPT, 0);
-    else if (T == 8 && nz > 1 && !mo.partial) NORM_DOWN_ONE(NPR, 0);
+    else if (T == 8 && nz > 1 && !mo.partial) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, NPR, true, 0, T == 8>), dim3(1, p.ksplit / h.hc, nz * h.hc), dim3(512), lds + 4 * (size_t)8 * T * 64, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, w.ssq, w.o, p.upw, (const uint2*)ctx->d_iq2xs);          // (a workgroup prepares its columns once for all row tiles)
     else if constexpr (T == 1) { switch (mo.partial ? (mo.k + 4) / 4 : 0) { case 1: NORM_DOWN_ONE(1, 1); break; case 2: NORM_DOWN_ONE(1, 2); break; case 3: NORM_DOWN_ONE(1, 3); break; case 4: NORM_DOWN_ONE(1, 4); break; case 5: NORM_DOWN_ONE(1, 5); break; default: NORM_DOWN_ONE(1, 0); } }          // (a token's gather is the launch's longest chain)
     else NORM_DOWN_ONE(1, 0);
   }
@@ -272,7 +321,7 @@ template <int FMT, int T> int norm_down_launch(pyre_ctx* ctx, const HcDev& h, co
   PYRE_CHECK_LAUNCH(ctx); return PYRE_OK;
 }
 template <int FMT, int T> int up_mix_rows_launch(pyre_ctx* ctx, const HcDev& h, const HcWork& w, int ksplit, const float* xnew, float eps, float* mixed, float* inj, const HcRoute* rt, int nz) {
-  const int nw = h.hc * h.up.U; size_t lds = 4 * ((size_t)T * h.lr + (size_t)nw * T * 64 + (size_t)T * 32 + (size_t)T * h.hc * 64);
+  const int nw = h.hc * h.up.U; size_t lds = 4 * ((size_t)T * (h.lr + HC_PAD) + (size_t)nw * T * 64 + (size_t)T * 32 + (size_t)T * h.hc * 64);
   const QMatDev rq = rt ? rt->router : QMatDev{}; float* rp = rt ? rt->part : nullptr;
   ProfScope ps(ctx, rt ? "hc_up_mix_router" : "hc_up_mix", qmat_gguf_bytes(h.up, h.up.rows) + 4.0 * T * (h.hc * h.d + h.d + (double)ksplit * (h.lr + h.hc)) +
                (rt ? qmat_gguf_bytes(rq, rq.rows) + 4.0 * T * (h.d / 64) * rq.tiles * 64 : 0.0));

@@ -216,9 +216,6 @@ template <int FMT> __global__ __launch_bounds__(64) void k_rows(QMatDev m, const
 //                slice order (no in-kernel cross-workgroup reduction: a device-scope fence per workgroup costs about a
 //                microsecond of serialized L2 write-back per XCD on this part).
 //   best != nullptr (T == 1, ksplit == 1): best[2*tile] = bits of the tile's maximum, best[2*tile+1] = its first row.
-// A group of four tokens costs ten cycles a column on the matrix cores, a token four on the vector pipe: from four tokens on.  (Two and
-// three of a 6144 x 2048 Q4_K matrix on the matrix cores: 8.1 us, on the vector pipe 6.0 and 6.7.)
-#define PYRE_MMA_MIN 4
 template <int FMT, int T, int NW>
 __global__ __launch_bounds__(NW * 64) void k_gemv(QMatDev m, const float* __restrict__ x, float* __restrict__ y, int upw,
                                                   GemvEpi ep, int tn) {
