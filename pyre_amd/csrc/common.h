@@ -327,8 +327,8 @@ struct RouteSrc { const float* p; int nsl; int r64; const uint32_t* dgx = nullpt
 // token in w.parts, group q of token ti at parts + (q*t + ti)*d, instead of the unreduced terms.
 int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const float* x_dev, int t, float* y_dev, const RouteSrc* routed = nullptr, bool in_groups = false);
 inline bool pyre_moe_groups_ok(const MoeDev& m) { return m.top_k <= PYRE_MOE_KMAX; }
-// The FFN of a prompt's block of T tokens, grouped by expert, on the matrix cores (moe.hip): x [T][d]; the router's K-slice sums of
-// group w (eight tokens; slice s of token ti at (s * 8 + ti) * r64) at rpart + w * wr; the group sums of every token in
+// The FFN of a prompt's block of T tokens, grouped by expert, on the matrix cores (moe.hip): x [T][d]; the router's logits of
+// group w (eight tokens; token ti at ti * r64) at rpart + w * wr; the group sums of every token in
 // parts [group][PYRE_MOE_GROUPS][8][d].  The rest is the block's own scratch (pyre_moe_block_carve): the routing, the (token, choice) pairs by
 // expert, x and h as f16 operand rows a token (xh [T + 1][2][d], hh [T * (k + 1) + 1][2][ff], the last row of each zero) with
 // their scale factors, the gate and up products and the unreduced down terms.
@@ -341,7 +341,7 @@ bool   pyre_moe_block_ok(const MoeDev& m);
 size_t pyre_moe_block_bytes(const MoeDev& m, int T);
 void   pyre_moe_block_carve(const MoeDev& m, int T, void* base, MoeBlk* b);
 int    pyre_moe_block_zero_rows(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T);
-int    pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_router, int T_max, int nsl, int r64);
+int    pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_router, int T_max, int r64);
 // any number of tokens with the windows' arithmetic: moe.hip
 struct MoeRows { int32_t* sel_idx; float* sel_w; int32_t* elist; float* sg; int32_t* eoff; int32_t* plist; float* h; float* partial; uint32_t* dgx; uint32_t* dgh; };
 size_t pyre_moe_rows_bytes(const MoeDev& m, int T);

@@ -583,7 +583,7 @@ static int prompt_blk_get(pyre_ctx* ctx, const pyre_model* m, int T, int n, Prom
     const MoeDev& m0 = m->layers[0].moe; const Layer* lin = nullptr; for (const Layer& L : m->layers) if (!L.full) lin = &L;
     const size_t t = T, d = c.d, nq = (size_t)c.n_head * c.hd, cmax = std::max((size_t)c.lin_nv * c.lin_dv, nq), omax = std::max(d, cmax), pmax = std::max(m->pw_lin, m->pw_attn);
     HcDev hmax = m->layers[0].hca;
-    const size_t rp = t * (d / 64) * m0.router.tiles * 64;
+    const size_t rp = (t + 7) / 8 * 8 * m0.router.tiles * 64;
     for (int pass = 0; pass < 2; ++pass) {
       uint8_t* p = (uint8_t*)B->mem; size_t sum = 0;
       auto take = [&](size_t bytes) { void* r = p; bytes = al256(bytes); if (pass) p += bytes; sum += bytes; return r; };
@@ -594,7 +594,7 @@ static int prompt_blk_get(pyre_ctx* ctx, const pyre_model* m, int T, int n, Prom
       B->q = (float*)take(4 * t * nq); B->qh = (uint16_t*)take(2 * 2 * t * nq); B->qsc = (float*)take(4 * t * c.n_head);
       if (!pass) { PYRE_HIP(ctx, hipMalloc(&B->mem, sum + 256)); continue; }
       pyre_blk_mix_carve(hmax, T, mx, &B->mix); pyre_moe_block_carve(m0, T, mo, &B->moe); pyre_moe_rows_carve(m0, PROMPT_TAIL_MAX, rw, &B->rows); if (lin) pyre_gdn_chunk_carve(lin->gdn, T, gd, &B->gdn);
-      B->moe.x = B->mixed; B->moe.rpart = rpart; B->moe.parts = parts; B->moe.wr = 8 * (d / 64) * m0.router.tiles * 64;
+      B->moe.x = B->mixed; B->moe.rpart = rpart; B->moe.parts = parts; B->moe.wr = 8 * m0.router.tiles * 64;
     }
     PYRE_HIP(ctx, hipMemsetAsync(B->mem, 0, 4096, ctx->stream));
     { int rc = pyre_moe_block_zero_rows(ctx, m0, B->moe, T); if (rc) return rc; }
@@ -737,9 +737,9 @@ static int run_block(pyre_ctx* ctx, const pyre_model* m, pyre_state* s, PromptBl
     if ((rc = pyre_blk_mix_launch(ctx, L.hcf, B->mix, xin, in_ss, in_ts, B->x, T, B->o, o_parts, B->inj_a, c.eps, B->mixed, B->inj_f, nullptr, 0, nullptr, 0))) return rc;
     const bool end = il == c.n_layers - 1;
     if (end && !head) break;          // nobody reads the last layer's FFN
-    if ((rc = pyre_moe_block_launch(ctx, L.moe, B->moe, end ? 0 : Tb, T, B->T_max, d / 64, r64))) return rc;
+    if ((rc = pyre_moe_block_launch(ctx, L.moe, B->moe, end ? 0 : Tb, T, B->T_max, r64))) return rc;
     const int i0 = end ? (T - 1) / 8 * 8 : Tb;          // (the last layer: the last group's terms, for the head)
-    if (i0 < T && (rc = pyre_moe_rows_launch(ctx, L.moe, B->rows, B->mixed + (size_t)i0 * d, T - i0, B->moe.rpart + (size_t)(i0 / 8) * B->moe.wr, B->moe.wr, d / 64, r64, end ? nullptr : B->moe.parts + (size_t)(i0 / 8) * PYRE_MOE_GROUPS * 8 * d, nullptr))) return rc;
+    if (i0 < T && (rc = pyre_moe_rows_launch(ctx, L.moe, B->rows, B->mixed + (size_t)i0 * d, T - i0, B->moe.rpart + (size_t)(i0 / 8) * B->moe.wr, B->moe.wr, 1, r64, end ? nullptr : B->moe.parts + (size_t)(i0 / 8) * PYRE_MOE_GROUPS * 8 * d, nullptr))) return rc;
     comb = B->moe.parts; np = PYRE_MOE_GROUPS; cinj = B->inj_f;
   }
   s->len = start + T;

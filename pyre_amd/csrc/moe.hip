@@ -89,7 +89,8 @@ __device__ __forceinline__ void route_select(int n_exp, int k, RouteLds& L) {
 template <int NT, int NSM = 64>
 __device__ __forceinline__ void route_topk(const float* __restrict__ logits, int nsl, int sstride, int n_exp, int k, RouteLds& L ROUTE_TS_PARAM) {
   const int e = threadIdx.x;
-  if (e < n_exp) {
+  if constexpr (NSM == 1) { if (e < n_exp) { const float v = logits[e]; L.lv[e] = isnan(v) ? -INFINITY : v; } }
+  else if (e < n_exp) {
     float sv[NSM];
 #pragma unroll
     for (int q = 0; q < NSM; ++q) sv[q] = 0.0f;
@@ -633,41 +634,49 @@ int pyre_moe_launch(pyre_ctx* ctx, const MoeDev& m, const MoeWork& w, const floa
 // the window kernels above, in the same order (k_moe_route, k_moe_gu<.., 2, true, .., ID>, k_moe_down_groups<.., ID>): its
 // bits do not depend on which path ran.  IQ3_S experts in the integer form only, gate / up rows of 32 units, expert widths
 // of at most 8 units.
-template <bool FIX>
+template <bool FIX, int NSM = 64>
 __global__ __launch_bounds__(1024) void k_moe_route_blk(MoeDev m, MoeBlk b, int nsl, int r64) {
   __shared__ RouteLds rl;
   const int ti = blockIdx.x, w = ti >> 3, tw = ti & 7;
   const int n_exp = FIX ? 512 : m.n_exp, top_k = FIX ? 10 : m.top_k;
-  if constexpr (FIX) nsl = 32;
+  if constexpr (FIX && NSM == 64) nsl = 32;
 #ifdef PYRE_PHASE_TS
   unsigned long long ts_[8];
 #endif
-  route_topk<1024>(b.rpart + (size_t)w * b.wr + (size_t)tw * r64, nsl, 8 * r64, n_exp, top_k, rl ROUTE_TS_ARG);
+  route_topk<1024, NSM>(b.rpart + (size_t)w * b.wr + (size_t)tw * r64, nsl, 8 * r64, n_exp, top_k, rl ROUTE_TS_ARG);
   route_weights(top_k, rl);
   if ((int)threadIdx.x < top_k) { b.sel_idx[ti * top_k + threadIdx.x] = rl.s_idx[threadIdx.x]; b.sel_w[ti * top_k + threadIdx.x] = rl.s_w[threadIdx.x]; }
 }
-// The router's K-slice sums of a block when they do not ride on the windows' FFN mixes: grid (d / 64, T / 8), 4 waves.  The
-// workgroup stages its window's eight tokens' 64 columns of x and forms, tile of 64 experts by tile, the partial dot products
-// the riding code of k_hc_up_mix_m forms (unit_fma over the same 64 values in the same order): the same bits, where the
-// windows' path has them.
+// A block's router logits when they do not ride on the windows' FFN mixes: grid (row tiles, groups of eight tokens), 8 waves.  The riding code of
+// k_hc_up_mix_m forms a sum for every 64 columns and the selection adds them in order; here the workgroup's waves form four of them each
+// (unit_mma: the same bits) and add them on the spot, so that the logits leave instead of d / 64 sums a logit (134 MB at 2048 tokens of 512
+// experts).  f32 products: 34 us at 126 TFLOP/s; 74 -> 53 us, and the selection, which read the sums, 19 -> 11.
 template <int RF>
-__global__ __launch_bounds__(256) void k_moe_router_blk(MoeDev m, MoeBlk b, int r64) {
-  __shared__ float xs[8][64];
-  const uint2* lds2 = nullptr;
-  const int sl = blockIdx.x, w = blockIdx.y, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const float* xw = b.x + (size_t)w * 8 * m.d;
-  for (int i = threadIdx.x; i < 8 * 64; i += 256) xs[i >> 6][i & 63] = xw[(size_t)(i >> 6) * m.d + sl * 64 + (i & 63)];
-  lds_barrier();
-  float* rp = const_cast<float*>(b.rpart) + (size_t)w * b.wr;
-  for (int tile = wave; tile < m.router.tiles; tile += 4) {
-    const UnitRaw<RF> rraw = unit_load<RF>(m.router, tile, sl, lane);
-#pragma unroll 1
-    for (int t2 = 0; t2 < 8; ++t2) {
-      float ra[1] = {0.0f};
-      unit_fma<RF, 1>(m.router, rraw, sl, lds2, lane, xs[t2], 0, ra);
-      rp[((size_t)sl * 8 + t2) * r64 + (size_t)tile * 64 + lane] = ra[0];
+__global__ __launch_bounds__(512) void k_moe_router_blk(MoeDev m, MoeBlk b, int r64) {
+  __shared__ float sl[32][8][64];
+  const int tile = blockIdx.x, w = blockIdx.y, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, U = m.router.U;
+  const float* xp[2] = {b.x + (size_t)(w * 8 + (lane & 3)) * m.d + 4 * (lane >> 2), b.x + (size_t)(w * 8 + 4 + (lane & 3)) * m.d + 4 * (lane >> 2)};
+  float v = 0.0f;          // token `wave`, row `lane`
+  for (int k0 = 0; k0 < U; k0 += 32) {
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+      const int s = wave * 4 + i, ka = min(k0 + s, U - 1), kb = min(k0 + s + 1, U - 1);
+      const UnitRaw<RF> r0 = unit_load<RF>(m.router, tile, ka, lane); XGrp<2> x0, x1; unit_x_load(xp, ka, x0);
+      const UnitRaw<RF> r1 = unit_load<RF>(m.router, tile, kb, lane); unit_x_load(xp, kb, x1);
+      v4f a0[2], a1[2]; mma_zero(a0); mma_zero(a1);
+      unit_mma<RF, 2>(m.router, r0, ka, x0, a0); unit_mma<RF, 2>(m.router, r1, kb, x1, a1);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) { sl[s][t][lane] = a0[t >> 2][t & 3]; sl[s + 1][t][lane] = a1[t >> 2][t & 3]; }
     }
+    lds_barrier();
+    const int n = min(32, U - k0);
+    if (n == 32) {
+#pragma unroll
+      for (int q = 0; q < 32; ++q) v = q == 0 && k0 == 0 ? sl[0][wave][lane] : v + sl[q][wave][lane];
+    } else for (int q = 0; q < n; ++q) v = q == 0 && k0 == 0 ? sl[0][wave][lane] : v + sl[q][wave][lane];
+    if (k0 + 32 < U) lds_barrier();
   }
+  const_cast<float*>(b.rpart)[(size_t)w * b.wr + (size_t)wave * r64 + (size_t)tile * 64 + lane] = v;
 }
 #define MOE_PASS 8
 // the (token, choice) pairs of the block by expert: eoff[e] .. eoff[e + 1] of elist hold expert e's entries token * (k + 1) + j
@@ -917,12 +926,11 @@ int pyre_moe_block_zero_rows(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, in
   PYRE_HIP(ctx, hipMemsetAsync(b.hh + 2 * ne * hs, 0, 2 * 2 * hs, ctx->stream));
   return PYRE_OK;
 }
-// The first T of T_router tokens (the router's sums are formed for all of them); T_max: the T the scratch was carved and its zero rows were set for (x readable up to the next multiple of eight rows); the router's
-// sums in nsl = d / 64 slices of r64 rows a token
-int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_router, int T_max, int nsl, int r64) {
-  if (!pyre_moe_block_ok(m) || T < 0 || T > T_router || T_router < 1 || T_router > T_max || (size_t)T_max * (m.top_k + 1) * m.ff * 4 >= (1ull << 32) || (size_t)T_max * m.d * 4 >= (1ull << 32) || nsl < 1 || nsl > 64 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe block: unsupported shape (T = %d, %d router slices)", T, nsl);
+// The first T of T_router tokens (the router's logits are formed for all of them, r64 floats a token); T_max: the T the scratch was carved and its zero rows were set for (x readable up to the next multiple of eight rows)
+int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T, int T_router, int T_max, int r64) {
+  if (!pyre_moe_block_ok(m) || T < 0 || T > T_router || T_router < 1 || T_router > T_max || (size_t)T_max * (m.top_k + 1) * m.ff * 4 >= (1ull << 32) || (size_t)T_max * m.d * 4 >= (1ull << 32) || m.d > 4096 || r64 < m.n_exp) return pyre_fail(ctx, PYRE_E_ARG, "moe block: unsupported shape (T = %d)", T);
   const int hs = m.ff, ny = m.n_exp + (T + 7) / 8, ne = T * (m.top_k + 1), ne_max = T_max * (m.top_k + 1);
-  const bool fix = m.n_exp == 512 && m.top_k == 10 && nsl == 32;
+  const bool fix = m.n_exp == 512 && m.top_k == 10;
   // Groups of eight entries that share an expert's decoding, by the mean entries an expert.  Gate / up + down, us, 512 experts top 10 of
   // width 512: 64 tokens (mean 1.2) 168 with one, 172 with two; 104 (2.0) 199, 189; 208 (4.1) 225 with two, 230 with four; 312 (6.1)
   // 262, 255; 520 (10) 320, 294; 2040 (40) 738 with four, 769 with six.  128 experts top 8: 104 (6.5) 92 with two, 101 with four; 160
@@ -931,15 +939,15 @@ int pyre_moe_block_launch(pyre_ctx* ctx, const MoeDev& m, const MoeBlk& b, int T
 #define MM_MANY(DN, TG, GX, GZ, ZR, KC) hipLaunchKernelGGL((k_moe_mm_many<DN, TG>), dim3(GX, m.n_exp + (T + 8 * TG - 1) / (8 * TG), GZ), dim3(256), (size_t)TG * 8 * (KC / 256) * 4, ctx->stream, m, b, T, ZR)
 #define MM_GO(DN, GX, GZ, ZR, KC) do { if (tg == 1) hipLaunchKernelGGL(k_moe_mm_blk<DN>, dim3(GX, ny, GZ), dim3(256), 0, ctx->stream, m, b, T, ZR); else if (tg == 2) MM_MANY(DN, 2, GX, GZ, ZR, KC); else MM_MANY(DN, 4, GX, GZ, ZR, KC); } while (0)
   {
-    if (nsl != m.d / 64 || (m.router.fmt != FMT_BF16 && m.router.fmt != FMT_F32)) return pyre_fail(ctx, PYRE_E_ARG, "moe block: the router's sums by %d slices, router format %d", nsl, m.router.fmt);
-    ProfScope ps(ctx, "moe_block_router", qmat_gguf_bytes(m.router, m.router.rows) + 4.0 * T * (m.d + (double)nsl * r64));
-    if (m.router.fmt == FMT_BF16) hipLaunchKernelGGL(k_moe_router_blk<FMT_BF16>, dim3(nsl, (T_router + 7) / 8), dim3(256), 0, ctx->stream, m, b, r64);
-    else hipLaunchKernelGGL(k_moe_router_blk<FMT_F32>, dim3(nsl, (T_router + 7) / 8), dim3(256), 0, ctx->stream, m, b, r64);
+    if (m.router.U != m.d / 64 || m.router.tiles * 64 > r64 || (m.router.fmt != FMT_BF16 && m.router.fmt != FMT_F32)) return pyre_fail(ctx, PYRE_E_ARG, "moe block: router of %d units, format %d", m.router.U, m.router.fmt);
+    ProfScope ps(ctx, "moe_block_router", qmat_gguf_bytes(m.router, m.router.rows) + 4.0 * T * (m.d + (double)r64));
+    if (m.router.fmt == FMT_BF16) hipLaunchKernelGGL(k_moe_router_blk<FMT_BF16>, dim3(m.router.tiles, (T_router + 7) / 8), dim3(512), 0, ctx->stream, m, b, r64);
+    else hipLaunchKernelGGL(k_moe_router_blk<FMT_F32>, dim3(m.router.tiles, (T_router + 7) / 8), dim3(512), 0, ctx->stream, m, b, r64);
     PYRE_CHECK_LAUNCH(ctx);
   }
   if (T == 0) return PYRE_OK;
-  { ProfScope ps(ctx, "moe_block_route", 4.0 * T * nsl * m.n_exp);
-    if (fix) hipLaunchKernelGGL(k_moe_route_blk<true>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64); else hipLaunchKernelGGL(k_moe_route_blk<false>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64);
+  { ProfScope ps(ctx, "moe_block_route", 4.0 * T * m.n_exp);
+    if (fix) hipLaunchKernelGGL((k_moe_route_blk<true, 1>), dim3(T), dim3(1024), 0, ctx->stream, m, b, 1, r64); else hipLaunchKernelGGL((k_moe_route_blk<false, 1>), dim3(T), dim3(1024), 0, ctx->stream, m, b, 1, r64);
     hipLaunchKernelGGL(k_moe_lists, dim3(1), dim3(1024), 0, ctx->stream, m, b, T);
     hipLaunchKernelGGL(k_blk_split, dim3(T), dim3(256), 0, ctx->stream, b.x, (const float*)nullptr, m.d, b.xh, b.xinv, m.sh_gate_inp, b.sg); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "moe_block_gate_up", 2.0 * m.n_exp * qmat_gguf_bytes(m.gate_e, m.ff) + 2.0 * qmat_gguf_bytes(m.sh_gate, m.sf));
@@ -1098,12 +1106,14 @@ int pyre_moe_rows_launch(pyre_ctx* ctx, const MoeDev& m, const MoeRows& w, const
   const bool idot = pyre_moe_takes_digits(m), idot_dn = idot && !moe_idot_gu_only() && m.down_e.fmt == FMT_IQ3_S && m.sh_down.fmt == FMT_IQ3_S;
   uint32_t* dgh = idot_dn ? w.dgh : nullptr;
   { ProfScope ps(ctx, "moe_rows_route", 4.0 * T * nsl * m.n_exp);
-    if (m.n_exp == 512 && m.top_k == 10 && nsl == 32) hipLaunchKernelGGL(k_moe_route_blk<true>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64); else hipLaunchKernelGGL(k_moe_route_blk<false>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64);
+    if (nsl == 1 && m.n_exp == 512 && m.top_k == 10) hipLaunchKernelGGL((k_moe_route_blk<true, 1>), dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64);
+    else if (nsl == 1) hipLaunchKernelGGL((k_moe_route_blk<false, 1>), dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64);
+    else if (m.n_exp == 512 && m.top_k == 10 && nsl == 32) hipLaunchKernelGGL(k_moe_route_blk<true>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64); else hipLaunchKernelGGL(k_moe_route_blk<false>, dim3(T), dim3(1024), 0, ctx->stream, m, b, nsl, r64);
     hipLaunchKernelGGL(k_moe_lists, dim3(1), dim3(1024), 0, ctx->stream, m, b, T);
     if (idot) hipLaunchKernelGGL(k_act_digits_eo, dim3(m.d / 64, T), dim3(64), 0, ctx->stream, x, m.d, w.dgx); } PYRE_CHECK_LAUNCH(ctx);
   { ProfScope ps(ctx, "moe_rows_gate_up", T * (2.0 * m.top_k * qmat_gguf_bytes(m.gate_e, m.ff) + 2.0 * qmat_gguf_bytes(m.sh_gate, m.sf)));
 #define ROWS_GU dim3(hs / 64, entries, 1), dim3(16 * 64), 0, ctx->stream, m, (const float*)nullptr, w.sel_idx, w.sel_w, w.sg, x, w.h, hs, g2, nsl, 0, 0, w.dgx, dgh, w.elist
-    const bool fix = m.gate_e.fmt == FMT_IQ3_S && m.down_e.fmt == FMT_IQ3_S && m.n_exp == 512 && m.top_k == 10 && m.d == 2048 && m.ff == 512 && m.sf == 512 && nsl == 32;
+    const bool fix = m.gate_e.fmt == FMT_IQ3_S && m.down_e.fmt == FMT_IQ3_S && m.n_exp == 512 && m.top_k == 10 && m.d == 2048 && m.ff == 512 && m.sf == 512;
     if (idot && fix && P == 2) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, true, true>), ROWS_GU);
     else if (idot) { if (P == 2) hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 2, true, false, true>), ROWS_GU); else hipLaunchKernelGGL((k_moe_gu<FMT_IQ3_S, 16, 1, true, false, true>), ROWS_GU); }
     else if (P == 2) { MOE_FMT_DISPATCH(m.gate_e.fmt, hipLaunchKernelGGL((k_moe_gu_rows<F, 2>), dim3(hs / 64, ns + moe_passes(m, T)), dim3(512), 0, ctx->stream, m, w, x, hs, T)); }
