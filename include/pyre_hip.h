@@ -79,11 +79,13 @@ int    pyre_qmat_row(pyre_ctx* ctx, const pyre_qmat* m, size_t row, float* out_h
 /* QMat::matmul (gguf_q.rs:216-217): y[ti*rows + r] = sum_c W[r,c] * x[ti*cols + c], t in 1..8.
  * The result for a token does not depend on t (same operations in the same order), which is what lets a
  * multi-token verify pass equal one-token decode (qwen4exp_gguf.rs:2357-2360) -- with one exception: a single token of
- * an IQ3_S matrix takes a kernel of its own (below), so t = 1 and t >= 2 agree to rounding (both within 1e-5 of the exact
- * product), not bit for bit; PYRE_QMATMUL_NATIVE=0 in the environment sends t = 1 through the window's kernel as well. */
+ * an IQ3_S matrix takes a kernel of its own (below; small matrices the lane = row GEMV, one launch), and so does one of a
+ * large IQ2_XS, Q4_K or Q8_0 matrix, so t = 1 and t >= 2 agree to rounding (both within 1e-5 of the exact product), not bit
+ * for bit; PYRE_QMATMUL_NATIVE=0 in the environment sends an IQ3_S matrix' t = 1 through the window's kernel as well where
+ * it has more than 128 row tiles. */
 int    pyre_qmatmul(pyre_ctx* ctx, const pyre_qmat* m, const float* x_host, int t, float* y_host);
 int    pyre_qmatmul_dev(pyre_ctx* ctx, const pyre_qmat* m, const float* x_dev, int t, float* y_dev);
-/* One token of an IQ3_S matrix (t = 1; the reference's GPU decode of this type, src/model/qn_cube.rs:3354-3382): the
+/* One token of a large IQ3_S matrix (t = 1; more than 128 row tiles and more than 49 152 units of 64 rows x 64 columns; the reference's GPU decode of this type, src/model/qn_cube.rs:3354-3382): the
  * matrix is streamed at the file's bits per weight -- per four weights the 9-bit codebook index and four sign bits, the
  * codebook with the signs folded in (8192 x four signed bytes) in shared memory -- and the activations are block fixed
  * point, three signed bytes per value with one power of two per 64 columns (|x - su q| <= 2^-22 of the 64 columns'

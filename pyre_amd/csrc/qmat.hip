@@ -670,17 +670,18 @@ int pyre_qmat_row(pyre_ctx* ctx, const pyre_qmat* m, size_t row, float* out_host
 // activations.  One token: its fused products cost with the 64-column units of the matrix' row tiles, the native-format kernel costs some 4 us
 // more to begin with and less a unit (us, this kernel first, 2048 columns: IQ3_S 12 288 rows 5.5 / 9.7, 49 152 14.5 / 15.8, 151 936 33.3 / 33.8;
 // IQ2_XS 12 288 7.0 / 9.8, 49 152 15.0 / 15.6, 151 936 39.2 / 34.0; Q4_K 12 288 6.6 / 9.1, 49 152 14.9 / 15.6, 151 936 40.3 / 36.1; 30 000 x 4096 IQ2_XS
-// 20.0 / 18.4, Q4_K 18.6 / 19.8), and its sums are nearer the exact ones (2.1 - 3.0e-7 for 5.5 - 6.4e-7).  Windows: matrices of at most 128 row tiles
-// except IQ3_S, whatever the width, so that a token's bits do not depend on it; above, the matrix cores' sums are nearer (1.2e-7 for 3e-7).
+// 20.0 / 18.4, Q4_K 18.6 / 19.8), and its sums are nearer the exact ones (2.1 - 3.0e-7 for 5.5 - 6.4e-7), so a matrix of at most 128 row tiles has
+// it for any count of columns.  Windows: matrices of at most 128 row tiles except IQ3_S, whatever the width, so that a token's bits do not depend
+// on it; above, the matrix cores' sums are nearer (1.2e-7 for 3e-7).  PYRE_QMATMUL_NATIVE=0 asks for an IQ3_S window's kernel above 128 row tiles.
 // PYRE_QMATMUL_SMALL=0 (read at every call: tests reach the other kernels with small shapes): never.
 static bool qmat_rows_call(const pyre_qmat* m, int t) {
   if (m->base == nullptr) return false;
-  const int64_t units = (int64_t)m->dv.tiles * m->dv.U; bool rows;
+  const int64_t units = (int64_t)m->dv.tiles * m->dv.U; bool rows = m->dv.tiles <= 128;
   switch (m->dv.fmt) {
-    case FMT_IQ3_S: rows = t == 1 && units <= 49152; break;
-    case FMT_IQ2_XS: rows = t == 1 ? units <= 24576 : m->dv.tiles <= 128; break;
-    case FMT_Q4_K: rows = t == 1 ? units <= 32768 : m->dv.tiles <= 128; break;
-    case FMT_Q8_0: rows = t == 1 || m->dv.tiles <= 128; break;
+    case FMT_IQ3_S: rows = t == 1 && (rows || (units <= 49152 && env_int("PYRE_QMATMUL_NATIVE", 1))); break;
+    case FMT_IQ2_XS: rows = rows || (t == 1 && units <= 24576); break;
+    case FMT_Q4_K: rows = rows || (t == 1 && units <= 32768); break;
+    case FMT_Q8_0: rows = rows || t == 1; break;
     default: return false;
   }
   return rows && env_int("PYRE_QMATMUL_SMALL", 1);

@@ -1,5 +1,9 @@
 """GPU parity of the quantized-matrix operator through the C ABI: dequant bit-exact with the oracle, GEMV within
 1e-5 of the f64-accumulated truth (max|dy| / max|y|, the reference's own normalisation, kquant.rs:203-206)."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -432,3 +436,19 @@ def test_single_token_launch_rule_at_its_edge(ctx, ty, rows, cols):
     assert relerr(y, f) <= TOL
     small = rows % 64 == 0
     assert np.array_equal(bits(y), bits(f)) == small
+
+
+# ---- ... and any count of columns at up to 128 row tiles; without the native-format kernel an IQ3_S matrix above them goes with its windows
+@pytest.mark.parametrize("ty,cols", [(lib.IQ3_S, 25600), (lib.IQ2_XS, 12800), (lib.Q4_K, 16896)])
+def test_wide_small_matrix_keeps_the_lane_row_gemv(ctx, ty, cols):
+    m = lib.QMat(ctx, ty, 8192, cols, raw_matrix(ty, 8192, cols, 47))
+    x = synth.normal((1, cols), 48)
+    assert np.array_equal(bits(m.matmul(x)), bits(m.matmul_f32(x)))
+
+
+def test_one_token_without_the_native_format_has_its_windows_bits():
+    code = ("import numpy as np\nfrom pyre_amd import lib, synth\nctx = lib.Context(0)\n"
+            "m = lib.QMat(ctx, lib.IQ3_S, 8256, 512, synth.matrix(lib.IQ3_S, 8256, 512, 49))\nx = synth.normal((2, 512), 50)\n"
+            "assert np.array_equal(m.matmul(x[:1]), m.matmul(x)[:1])\n")
+    r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, PYRE_QMATMUL_NATIVE="0"), cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), capture_output=True, text=True, timeout=110)
+    assert r.returncode == 0, r.stderr[-2000:]
