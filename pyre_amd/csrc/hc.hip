@@ -43,7 +43,7 @@ template <int FMT, int T> __device__ __forceinline__ void hc_unit(const QMatDev&
 // ONE: eight waves of one unit each (every width in multiples of 512 with at most 32 slices): a thread prepares one column and a wave
 // forms one unit's sums, without loops.  FG > 0: the experts a group of the unreduced FFN output (moe_out_value).  One token, bf16,
 // 2048 columns, 6.1 us with the loops and the groups at run time, 5.0 with neither; 500 tokens' groups of eight 218 and 113 us.
-// ALLT (groups of eight of a prompt): one workgroup for all row tiles, which otherwise prepare the same columns each: 200 tokens 43 -> 26 us.
+// ALLT (groups of eight of a longer prompt): one workgroup for all row tiles, which otherwise prepare the same columns each: 200 tokens 43 -> 26 us.
 template <int FMT, int T, int NP, bool ONE = false, int FG = 0, bool ALLT = false> __global__ __launch_bounds__(512) void k_hc_norm_down(QMatDev m, const float* __restrict__ x_in, int in_ss, int in_ts, float* __restrict__ x_out,
     const float* __restrict__ comb_out, MoeOut mo, const float* __restrict__ comb_inj, const float* __restrict__ norm, int d, int hc, float* __restrict__ ssq,
     float* __restrict__ part, int upw, const uint2* __restrict__ g2) {
@@ -311,6 +311,9 @@ template <int FMT, int T> int norm_down_launch(pyre_ctx* ctx, const HcDev& h, co
   else if constexpr (FMT == FMT_BF16 || FMT == FMT_F16 || FMT == FMT_F32) {
     if (p.nw != 8 || p.upw != 1) NORM_DOWN_GO(1);
     else if (comb_parts > 1) NORM_DOWN_ONE(NPT, 0);
+    // a workgroup for all row tiles prepares their columns once, one for each is the shorter chain while two of them a compute unit hold the launch
+    // (five tiles, sixteen slices, us a tile each / all in one: three groups 11.3 / 17.2, four 14.3 / 17.9, six 15.0 / 17.6, eight 21.6 / 17.9, twelve 26.9 / 18.5)
+    else if (T == 8 && nz > 1 && !mo.partial && (int64_t)h.di.tiles * p.ksplit * nz <= 512) NORM_DOWN_ONE(NPR, 0);
     else if (T == 8 && nz > 1 && !mo.partial) hipLaunchKernelGGL((k_hc_norm_down<FMT, T, NPR, true, 0, T == 8>), dim3(1, p.ksplit / h.hc, nz * h.hc), dim3(512), lds + 4 * (size_t)8 * T * 64, ctx->stream, h.di, x_in, in_ss, in_ts, x_out, comb_out, mo, comb_inj, h.norm, h.d, h.hc, w.ssq, w.o, p.upw, (const uint2*)ctx->d_iq2xs);          // (a workgroup prepares its columns once for all row tiles)
     else if constexpr (T == 1) { switch (mo.partial ? (mo.k + 4) / 4 : 0) { case 1: NORM_DOWN_ONE(1, 1); break; case 2: NORM_DOWN_ONE(1, 2); break; case 3: NORM_DOWN_ONE(1, 3); break; case 4: NORM_DOWN_ONE(1, 4); break; case 5: NORM_DOWN_ONE(1, 5); break; default: NORM_DOWN_ONE(1, 0); } }          // (a token's gather is the launch's longest chain)
     else NORM_DOWN_ONE(1, 0);
